@@ -1,62 +1,18 @@
 // kr_serve_gemm.hip -- C[M, N] (f32) = A[M, K] x W[N, K]^T for the batched serving step, single matrix or grouped (one matrix per expert, the rows
-// of a group contiguous, optional row gather for A).  Three forms:
+// of a group contiguous, optional row gather for A).  The dispatch, and the forms that take every shape; a bf16 store's aligned shapes go to kr_serve_skinny.hip (few
+// rows) and kr_serve_tile.hip (prompts).  Here:
 //   * small M (decode steps): one WAVE per output column, the K range over its lanes in 16-byte reads, up to 8 rows of A against one pass over
 //     the weight row -- bound by the weight stream;
-//   * bf16, larger M: workgroup tile 128 x 128 x 64 staged through LDS, four waves of 64 x 64 on v_mfma_f32_32x32x16_bf16, f32 accumulators, the next
-//     tile's global loads in flight during the MFMAs;
+//   * bf16, larger M: workgroup tile 128 x 128 x 64 staged through registers and LDS, four waves of 64 x 64 on v_mfma_f32_32x32x16_bf16, f32 accumulators;
 //   * f32, larger M: 64 x 64 x 16 tile, 4 x 4 outputs per thread, plain fused multiply-adds (no reduced-precision matrix mode).
 // Every shape is accepted: edges are guarded, and rows whose byte length is not a multiple of 16 take element loads.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "kr_device.h"
-#include "kr_serve_ops.h"
+#include "kr_serve_gemm_dev.h"
 
 namespace {
-typedef float gv16f __attribute__((ext_vector_type(16)));
-typedef __bf16 gb8 __attribute__((ext_vector_type(8)));
-typedef uint32_t gu4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ float gm_ld(const float* p) { return *p; }
-__device__ __forceinline__ float gm_ld(const uint16_t* p) { return kr_bf16_to_f32(*p); }
-// one element of C: f32, or the storage type when the output feeds another GEMM as it is (BF = a bf16 store)
-template <bool BF>
-__device__ __forceinline__ void gm_store(const KrSvGemm& g, int m, int n, float v) {
-    const int row = g.c_rows ? g.c_rows[m] : m;
-    const size_t i = (size_t)row * g.ldc + n;
-    if (g.bias) v += g.bias[n];
-    if (n >= g.silu_lo && n < g.silu_hi) v = v / (1.0f + expf(-v));
-    if (g.o_gate) v *= 1.0f / (1.0f + expf(-g.o_gate[(size_t)(row / g.o_gate_div) * g.o_gate_ld + (size_t)(row % g.o_gate_div) * g.N + n]));
-    if (BF && g.c_storage) ((uint16_t*)g.C)[i] = kr_f32_to_bf16(v);
-    else g.C[i] = v;
-}
-
-// columns of group `group`: all N, or what the group's own matrix has
-__device__ __forceinline__ int gm_cols(const KrSvGemm& g, int group) { return g.n_last > 0 ? (group == g.n_groups - 1 ? g.n_last : g.n_first) : g.N; }
-
-// row tile `tile` of a grouped problem: walks the segment table; returns false past the last tile
-__device__ __forceinline__ bool gm_find_tile(const int* seg, int n_groups, int tile, int BM, int& group, int& m0, int& mend) {
-    int acc = 0;
-    for (int g = 0; g < n_groups; g++) {
-        const int lo = seg[g], hi = seg[g + 1];
-        const int nt = (hi - lo + BM - 1) / BM;
-        if (tile < acc + nt) { group = g; m0 = lo + (tile - acc) * BM; mend = hi; return true; }
-        acc += nt;
-    }
-    return false;
-}
-
 // ---------------------------------------------------------------------------------------------------------------- small M
-__device__ __forceinline__ float gm_act(float g, float u, int kind, float limit, float alpha) {
-    if (kind == KR_SV_ACT_RELU2) { g = fmaxf(g, 0.0f); return g * g; }
-    if (kind == KR_SV_ACT_GELU_TANH) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
-    if (kind == KR_SV_ACT_CLAMPED_SWIGLU) { g = fminf(g, limit); u = fminf(fmaxf(u, -limit), limit); return g / (1.0f + expf(-alpha * g)) * (u + 1.0f); }
-    // silu on the hardware exponential and reciprocal (one ulp each): every wave of a decode step's down projection forms it again
-    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g)) * u;
-}
-template <typename T> __device__ __forceinline__ float gm_round(float v) { return v; }
-template <> __device__ __forceinline__ float gm_round<uint16_t>(float v) { return kr_bf16_to_f32(kr_f32_to_bf16(v)); }
-
 // ACT: the A operand is the gated activation of g.act_gu, formed as it is needed.  A wave owns CN consecutive output columns: their weight rows are
 // requested together (CN 16-byte reads in flight per k step), the input rows are read once for all of them.
 template <typename T, int MB, int CN, bool ACT>
@@ -384,15 +340,30 @@ void kr_sv_narrow_act(const KrSvGemm& g, hipStream_t st) {
         hipLaunchKernelGGL(sv_narrow_act_kernel<8>, grid, dim3(512), b, st, g); }
 }
 
-bool kr_sv_gemm_small(const KrSvGemm& g) {
-    // decode-sized problems: a pass over the weights per 8 rows; grouped problems take one row per workgroup row (each row has its own expert)
-    return g.seg ? (g.M <= (g.rowwise_upto > 64 ? g.rowwise_upto : 64) && g.row_group) : g.M <= 16;
+// the wave-per-column form: a pass over the weights per 8 rows; grouped problems take one row per workgroup row (each row has its own expert)
+static bool gm_gemv_rows(const KrSvGemm& g) { return g.seg ? (g.M <= (g.rowwise_upto > 64 ? g.rowwise_upto : 64) && g.row_group) : g.M <= 16; }
+
+bool kr_sv_gemm_takes_act(const KrSvGemm& g, bool f32, const float* gu, int ld) {
+    KrSvGemm p = g;
+    p.A = nullptr; p.act_gu = gu; p.act_ld = ld;
+    return !f32 && kr_sv_gemm_skinny_fits(p) ? kr_sv_gemm_skinny_acts(p) : gm_gemv_rows(p);
+}
+
+// Few rows, bf16: all rows of a strip of columns per workgroup.  One matrix: up to 16 rows, up to 32 where the 64 x 64 tile would have too few workgroups (2048 x 2048,
+// 30 rows: 8.0 us against 12.2; 4224 columns 15.0 against 12.7).  One matrix per expert: from 24 rows (a token's few rows go to the wave-per-column form: 6 rows
+// of 1536 x 2048 8 us against 9.6, 24 rows alike) to eight per expert (384 rows on 64 experts 85 us, tile 88; past that a strip meets experts with more than 16 rows).
+static bool gm_skinny(const KrSvGemm& g) {
+    if (!kr_sv_gemm_skinny_fits(g)) return false;
+    if (g.act_gu) return kr_sv_gemm_skinny_acts(g);
+    if (g.seg) return g.M > 24 && (g.M <= 8 * g.n_groups || g.M <= g.rowwise_upto);
+    return g.M <= 16 || (g.M <= 32 && g.N <= 2560);
 }
 
 void kr_sv_gemm(const KrSvGemm& g, bool f32, hipStream_t st) {
     if (g.M <= 0 || g.N <= 0) return;
     const bool grouped = g.seg != nullptr;
-    if (kr_sv_gemm_small(g)) {
+    if (!f32 && gm_skinny(g)) { kr_sv_gemm_skinny(g, st); return; }
+    if (gm_gemv_rows(g)) {
 #define GM_V(T_, MB_, CN_, GRID_, ARG_, MBASE_) do { if (g.act_gu) hipLaunchKernelGGL((sv_gemv_kernel<T_, MB_, CN_, true>), GRID_, dim3(256), 0, st, ARG_, MBASE_); \
                                                       else hipLaunchKernelGGL((sv_gemv_kernel<T_, MB_, CN_, false>), GRID_, dim3(256), 0, st, ARG_, MBASE_); } while (0)
         // columns per wave: 4 while that still leaves a few waves for every SIMD of the chip, else 1
@@ -418,9 +389,9 @@ void kr_sv_gemm(const KrSvGemm& g, bool f32, hipStream_t st) {
         hipLaunchKernelGGL(sv_gemm_f32_kernel, dim3((g.N + 63) / 64, tiles), dim3(256), 0, st, g);
         return;
     }
-    // grouped problems have few rows per expert: the 64-row tile wastes less of the matrix cores.  (A 256-row tile -- wave tiles of 128 x 64, six fragment
-    // reads per eight MFMAs -- was measured and did not pay: two workgroups per compute unit instead of three.)
-    // and so do narrow problems: with 128-row tiles they would leave most compute units idle
+    if (kr_sv_gemm_tile_fits(g)) { kr_sv_gemm_tile(g, st); return; }
+    // shapes whose rows are not whole 64-k slots of 16-byte pieces.  Grouped problems have few rows per expert: the 64-row tile wastes less of the matrix cores, and
+    // so do narrow problems: with 128-row tiles they would leave most compute units idle
     const bool small = grouped ? (g.M / (g.n_groups > 0 ? g.n_groups : 1) < 96) : g.M <= 64 || (long)((g.N + 127) / 128) * ((g.M + 127) / 128) < 128;
     if (small) {
         const int tiles = grouped ? (g.M + 63) / 64 + g.n_groups : (g.M + 63) / 64;

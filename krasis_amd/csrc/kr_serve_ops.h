@@ -18,7 +18,7 @@ struct KrSvGemm {
     const int* seg;                  // grouped: [n_groups + 1] row offsets on the device (rows of group g are [seg[g], seg[g + 1])); null = one matrix
     const int* row_group;            // grouped: [M] group of every row (the small-M form reads it)
     int n_groups;
-    // small-M form only (kr_sv_gemm_small): A is not read but formed on the fly as the gated activation of act_gu [M, act_ld] f32 (gate at column k, up at
+    // only where kr_sv_gemm_takes_act says so: A is not read but formed on the fly as the gated activation of act_gu [M, act_ld] f32 (gate at column k, up at
     // column K + k), rounded to the storage type -- the down projection of a feed-forward without a launch and a buffer for the activation
     const float* act_gu; int act_ld, act_kind; float act_limit, act_alpha;
     const int* c_rows;               // optional: problem row r writes C row c_rows[r] (a grouped problem whose rows return to their own order)
@@ -39,7 +39,13 @@ void kr_sv_gemm(const KrSvGemm& g, bool f32, hipStream_t st);
 // ((k / 32) * ceil(N / 16) + n / 16) * 512 + (16 * (k % 32 / 8) + n % 16) * 8 + k % 8
 bool kr_sv_narrow_act_fits(const KrSvGemm& g, bool f32);
 void kr_sv_narrow_act(const KrSvGemm& g, hipStream_t st);
-bool kr_sv_gemm_small(const KrSvGemm& g);      // true: kr_sv_gemm takes the wave-per-column form for this problem (and honours act_gu)
+bool kr_sv_gemm_takes_act(const KrSvGemm& g, bool f32, const float* gu, int ld);      // true: kr_sv_gemm forms the activation of gu [M, ld] inside its launch (act_gu) for this problem
+// the forms for a bf16 store that kr_sv_gemm chooses from; _fits: shapes and alignment
+bool kr_sv_gemm_skinny_fits(const KrSvGemm& g);
+bool kr_sv_gemm_skinny_acts(const KrSvGemm& g);
+void kr_sv_gemm_skinny(const KrSvGemm& g, hipStream_t st);
+bool kr_sv_gemm_tile_fits(const KrSvGemm& g);
+void kr_sv_gemm_tile(const KrSvGemm& g, hipStream_t st);
 
 enum { KR_SV_NORM_LAYER = 0, KR_SV_NORM_RMS = 1 };
 enum { KR_SV_ACT_GELU_TANH = 0, KR_SV_ACT_CLAMPED_SWIGLU = 1, KR_SV_ACT_SILU = 2, KR_SV_ACT_RELU2 = 3 /* un-gated: relu(x)^2 of the first F columns; no up columns */ };

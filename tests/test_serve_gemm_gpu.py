@@ -1,0 +1,51 @@
+"""The serving store's matrix products at the edges of their forms, against float64.
+
+The vocabulary projection is one product whose three sizes a caller chooses freely -- wanted rows, vocabulary, width -- so it reaches every form of a single matrix: the
+strips for few rows (one and two blocks of sixteen rows, four and eight waves), the 64-, 128- and 256-row tiles, and what takes widths that are not whole slots.
+The experts of a small mixture reach the grouped forms."""
+import numpy as np
+import pytest
+
+from tests import oracle_serve as O
+from tests.test_serve_gpu import engine, tokens
+
+pytestmark = pytest.mark.gpu
+
+
+def stream_model(width, vocab):
+    """embedding and head alone: the one layer's attention sees a single key, which stays small"""
+    return O.make_config(width=width, vocab=vocab, eps=1e-5, layers=[{"type": "attention", "mixer": O.attn(2, 1, 8, 8, 1, 0, scale=0.3), "mlp": None}])
+
+
+@pytest.mark.parametrize("want,vocab,width", [
+    (1, 33, 64), (15, 4097, 96), (16, 4095, 2048), (17, 2559, 128), (31, 47, 160), (32, 2561, 64),            # strips; 32 rows of more than 2560 columns: the small tile
+    (33, 129, 64), (63, 257, 192), (64, 255, 128), (65, 64, 96), (127, 511, 320),                            # 64-row tile, and widths of half slots
+    (257, 16385, 64), (511, 4224, 128), (2049, 7165, 64), (2304, 7168, 128), (300, 700, 72)])                  # 128- and 256-row tiles with ragged edges; a width of 16-byte pieces only
+def test_vocabulary_projection_sizes(want, vocab, width):
+    cfg = stream_model(width, vocab); W = O.random_weights(cfg, 11)
+    toks = tokens(cfg, want, 12)
+    eng = engine(cfg, W, "bfloat16", max_tokens=4096)
+    eng.store.set_capture(True)
+    logits, amax = eng.step([("a", toks, list(range(want)))])
+    x = eng.store.read_capture(want)[-1].astype(np.float64)
+    h = O.layer_norm(x, W["final.norm"].astype(np.float64), W["final.norm.b"].astype(np.float64), 1e-5)
+    head = W["head"].astype(np.float64)
+    ref = h @ head.T
+    # the row is rounded to bf16 (half a unit in the last place of eight bits, independent from element to element), the sums are f32
+    spread = np.sqrt(((np.abs(h) * 2.0 ** -9) ** 2) @ (head.T ** 2))
+    assert np.all(np.abs(logits - ref) <= 6.0 * spread + 1e-5 * np.abs(h) @ np.abs(head.T))
+    assert np.array_equal(amax, logits.argmax(-1))
+
+
+@pytest.mark.parametrize("n", [1, 2, 5, 8, 9, 16, 17, 40, 65, 130, 420])
+def test_expert_products_sizes(n):
+    # 1 - 840 rows on ten experts: row by row, strips for few rows per expert with the activation inside and outside the launch, 64-row tiles
+    cfg = O.make_config(width=128, vocab=61, eps=1e-5, layers=[{"type": "attention", "mixer": O.attn(4, 2, 32, 32, 0, 16, scale=0.2), "mlp": O.moe(10, 2, 1, 1, 192, 2.0, 64, 2.0)}])
+    W = O.random_weights(cfg, 13); toks = tokens(cfg, n, 14)
+    ref_logits, ref_streams = O.forward(cfg, W, toks)
+    eng = engine(cfg, W, "bfloat16")
+    eng.store.set_capture(True)
+    eng.step([("a", toks, [n - 1])])
+    d = eng.store.read_capture(n)[0] - ref_streams[0]
+    e = np.sqrt((d ** 2).mean(-1)) / np.sqrt((ref_streams[0] ** 2).mean())
+    assert (e < 2e-2).mean() >= 0.95          # a row whose second expert was a close call may have taken another one

@@ -752,12 +752,14 @@ __global__ void __launch_bounds__(256) sv_attn_merge_kernel(const KrSvAttn a) {
     extern __shared__ float wsp[];           // [nsplit] weight of every split, then 1 / denominator
     const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
     const size_t base = ((size_t)t * a.heads + h) * a.nsplit;
-    float M = a.sink ? a.sink[h] : -INFINITY;
+    const float sink = a.sink ? (a.prompt ? a.sink[h] * 1.44269504f : a.sink[h]) : -INFINITY;      // the 128-row form keeps its maxima in powers of two
+    auto ex = [&](float x) { return a.prompt ? exp2f(x) : expf(x); };
+    float M = sink;
     for (int s = 0; s < a.nsplit; s++) M = fmaxf(M, a.part_ml[(base + s) * 2]);
-    for (int s = tid; s < a.nsplit; s += 256) { const float ms = a.part_ml[(base + s) * 2]; wsp[s] = ms == -INFINITY ? 0.0f : expf(ms - M); }
+    for (int s = tid; s < a.nsplit; s += 256) { const float ms = a.part_ml[(base + s) * 2]; wsp[s] = ms == -INFINITY ? 0.0f : ex(ms - M); }
     __syncthreads();
     if (tid == 0) {
-        float L = a.sink ? expf(a.sink[h] - M) : 0.0f;
+        float L = a.sink ? ex(sink - M) : 0.0f;
         for (int s = 0; s < a.nsplit; s++) if (wsp[s] != 0.0f) L = __builtin_fmaf(a.part_ml[(base + s) * 2 + 1], wsp[s], L);
         wsp[a.nsplit] = 1.0f / L;
     }
@@ -1949,6 +1951,11 @@ static bool sv_attn_mfma_launch(const KrSvAttn& a, hipStream_t st) {
 
 void kr_sv_attention(const KrSvAttn& a, bool f32, hipStream_t st) {
     if (a.T <= 0) return;
+    if (a.prompt) {
+        kr_sv_attn_prompt(a, st);
+        if (a.nsplit > 1) hipLaunchKernelGGL(sv_attn_merge_kernel<uint16_t>, dim3(a.T, a.heads), dim3(256), (size_t)(a.nsplit + 1) * sizeof(float), st, a);
+        return;
+    }
     if (f32 ? sv_attn_mfma_launch<float>(a, st) : sv_attn_mfma_launch<uint16_t>(a, st)) {
         if (a.nsplit > 1) {
             if (f32) hipLaunchKernelGGL(sv_attn_merge_kernel<float>, dim3(a.T, a.heads), dim3(256), (size_t)(a.nsplit + 1) * sizeof(float), st, a);

@@ -1,0 +1,53 @@
+"""The 128-row attention of prompt portions (bf16 store) at the edges of its tiles, against the float64 restatement: head sizes and groupings it is compiled for, portions around the
+tile sizes, windows around the key tile, portions deep in a request whose keys are shared over several workgroups, unequal requests in one step."""
+import numpy as np
+import pytest
+
+from tests import oracle_serve as O
+from tests.test_serve_gpu import engine, tokens
+
+pytestmark = pytest.mark.gpu
+
+
+def model(heads, kv_heads, dim, vdim, window, rot=0):
+    return O.make_config(width=128, vocab=50, eps=1e-5, layers=[{"type": "attention", "mixer": O.attn(heads, kv_heads, dim, vdim, window, rot, scale=2.0 * dim ** -0.5), "mlp": None}])
+
+
+def row_errors(got, ref):
+    """error of every row, relative to the root mean square of the layer's own contribution over the rows"""
+    return np.sqrt(((got - ref) ** 2).mean(-1)) / np.sqrt((ref ** 2).mean())
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(4, 4, 32, 32), (2, 1, 32, 128), (8, 2, 64, 64), (16, 1, 64, 32), (32, 1, 32, 64), (8, 1, 128, 128), (4, 2, 128, 64), (2, 2, 64, 128), (16, 2, 128, 32)])
+@pytest.mark.parametrize("n,window", [(32, 0), (33, 7), (65, 64), (129, 65), (200, 1), (257, 130)])
+def test_portion_sizes(heads, kv_heads, dim, vdim, n, window):
+    cfg = model(heads, kv_heads, dim, vdim, window, rot=16); W = O.random_weights(cfg, 21)
+    toks = tokens(cfg, n, 22)
+    eng = engine(cfg, W, "bfloat16")
+    eng.store.set_capture(True)
+    eng.step([("a", toks, [n - 1])])
+    got = eng.store.read_capture(n)[0]
+    ref = O.forward(cfg, W, toks)[1][0]
+    x0 = W["embed"].astype(np.float64)[np.asarray(toks)]
+    # bf16 holds the normed input, keys, values and the mixed rows: four roundings of 2^-9 a value, averaged over the row
+    assert row_errors(got - x0, ref - x0).max() < 2e-2
+
+
+@pytest.mark.parametrize("window", [0, 700])
+def test_portions_deep_in_a_request_share_keys(window):
+    # 1500 tokens in the cache, then 40 and 33 more of two requests and one token of a third in one step: the keys of every tile go over several workgroups
+    cfg = model(8, 2, 64, 64, window); W = O.random_weights(cfg, 23)
+    a, b, c = tokens(cfg, 1540, 24), tokens(cfg, 1300, 25), tokens(cfg, 90, 26)
+    eng = engine(cfg, W, "bfloat16", max_tokens=8192)
+    for rid, t, k in (("a", a, 1500), ("b", b, 1267), ("c", c, 89)):
+        eng.step([(rid, t[:k], [])])
+    eng.store.set_capture(True)
+    eng.step([("c", c[89:], [0]), ("a", a[1500:], [39]), ("b", b[1267:], [32])])
+    got = eng.store.read_capture(74)[0]
+    lo = 0
+    for t, k in ((c, 89), (a, 1500), (b, 1267)):
+        n = len(t) - k
+        ref = O.forward(cfg, W, t)[1][0][k:]
+        x0 = W["embed"].astype(np.float64)[np.asarray(t[k:])]
+        assert row_errors(got[lo:lo + n] - x0, ref - x0).max() < 2e-2
+        lo += n

@@ -1094,15 +1094,14 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     for (SvRope& r : s->ropes) if (r.cs.ensure(Ts * (r.dims / 2) * 8)) return kr_fail(KR_ERR_HIP, "rope table");
     if (s->capture) { if (s->cap.ensure((size_t)c.n_layers * Ts * W * 4)) return kr_fail(KR_ERR_HIP, "capture buffer"); s->cap_T = T; }
     std::vector<int> nsplit(c.n_layers, 1);
-    std::vector<char> att_prompt(c.n_layers, 0);      // layers whose attention takes the 128-row form: some entry brings a prompt portion
+    std::vector<int> att_form(c.n_layers, 0);
     for (int li = 0; li < c.n_layers; li++) {
         const SvLayer& l = s->L[li]; const kr_serve_layer& d = l.d;
         if (l.recurrent() || l.no_heads()) continue;
         const int visible = d.window > 0 ? std::min(max_pos + 1, d.window + d.keep_first) : (d.chunk > 0 ? std::min(max_pos + 1, d.chunk) : max_pos + 1);
         const int ldk = l.latent() ? l.att_dim() : d.kv_heads * d.dim, ldv = l.latent() ? l.att_dim() : d.kv_heads * d.vdim;
-        att_prompt[li] = max_count >= 32 && kr_sv_attn_prompt_fits(d.heads, l.att_heads_kv(), l.att_dim(), l.att_vdim(), ldk, ldv, l.latent() ? 0 : l.n_h, s->f32);
-        if (att_prompt[li]) nsplit[li] = kr_sv_attn_prompt_splits(T, n_entries, d.heads, l.att_heads_kv(), visible);
-        else nsplit[li] = kr_sv_attention_splits(T, d.heads, l.att_heads_kv(), l.att_dim(), l.att_vdim(), ldk, ldv, s->f32, visible);
+        const int ldq = l.latent() ? d.heads * l.att_dim() : d.proj_conv ? (int)l.pconv_c() : l.n_h;
+        att_form[li] = kr_sv_attn_form(T, n_entries, max_count, d.heads, l.att_heads_kv(), l.att_dim(), l.att_vdim(), ldk, ldv, ldq, PT, s->f32, visible, &nsplit[li]);
         if (nsplit[li] > 1 && (s->part_ml.ensure(Ts * d.heads * nsplit[li] * 8) || s->part_acc.ensure(Ts * d.heads * nsplit[li] * l.att_vdim() * 4)))
             return kr_fail(KR_ERR_HIP, "attention split scratch");
     }
@@ -1199,7 +1198,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         a.sink = d.has_sink ? (const float*)l.sink.p : nullptr;
         a.kpool = kvl.kpool.p; a.page_table = d_tab; a.table_ld = s->n_pages; a.slot = d_slot; a.pos = d_pos; a.page_tokens = PT; a.T = T;
         a.out = s->att.p;
-        a.ent_off = d_eoff; a.n_entries = n_entries; a.prompt = att_prompt[li];
+        a.ent_off = d_eoff; a.n_entries = n_entries; a.form = att_form[li];
         a.nsplit = nsplit[li]; a.part_ml = (float*)s->part_ml.p; a.part_acc = (float*)s->part_acc.p;
         const void* o_in = s->att.p;
         if (l.recurrent()) {

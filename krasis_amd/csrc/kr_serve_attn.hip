@@ -1,4 +1,4 @@
-// kr_serve_attn.hip -- attention of a bf16 store's prompt portions on the bf16 matrix instruction, every operand exact.
+// kr_serve_attn.hip -- attention of a bf16 store on the bf16 matrix instruction, every operand exact: prompt portions, and decode steps further down.
 //
 // Scores and weights of this design are 32-bit numbers, the cache holds bf16.  A 32-bit float is the exact sum of three bf16 numbers (24 bits of significand = 8 + 8 + 8,
 // taken by truncation), so q K^T = (q_hi + q_mid + q_lo) K^T and P V alike are three passes of the bf16 instruction with f32 accumulators: no operand loses a bit, and
@@ -19,6 +19,7 @@
 // now (the store's bf16 roundings).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <algorithm>
 
 #include "kr_device.h"
 #include "kr_serve_ops.h"
@@ -301,6 +302,190 @@ __global__ void __launch_bounds__(256, 2) sv_attn_prompt_kernel(const KrSvAttn a
         }
 }
 
+// Decode steps: one workgroup of eight waves per (token, key / value head, 16 query heads of its group, share of the keys).  A wave takes 32 keys at a time on
+// v_mfma_f32_16x16x32_bf16 with the operands split as above, keys and values straight from the cache to registers (a row serves one token's heads only: nothing to share):
+//   S^T[key][row] = K Q^T    first operand: 16 key rows, a lane 16 bytes of a row;
+//   O^T[d][row] += V^T P^T   a lane holds the 8 keys (4 q + 0..3 of both blocks of 16) that its weights belong to, VDIM / 16 neighbouring columns each; byte permutes turn
+//                            them into the columns' fragments, column 16-row d of block j = d VDIM / 16 + j.
+// What it waits for is latency -- page table, rows, two short products, one merge through LDS -- so a wave requests keys and values together, the next 32 keys before it works on
+// these.  32 keys lie in one page (the page size is a multiple of 32).  One request, 16 / 2 heads of 128: 20.9 us on the f32 matrix instruction -> 7.3 at some 110 keys.
+template <int DIM, int VDIM>
+__global__ void __launch_bounds__(512, 2) sv_attn_step_kernel(const KrSvAttn a) {
+    constexpr int KS = DIM / 32, CPL = VDIM / 16, VW = CPL / 2, NW = 8;
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int R = a.heads / a.kv_heads, t = blockIdx.x, g = blockIdx.y, sp = blockIdx.z % a.nsplit, hb = blockIdx.z / a.nsplit;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), row = lane & 15, q = lane >> 4;
+    const int Rb = min(16, R - hb * 16), h0 = g * R + hb * 16, head = h0 + min(row, Rb - 1);
+    const int p = a.pos[t];
+    const int* table = a.page_table + (size_t)a.slot[t] * a.table_ld;
+    const int lo = a.window > 0 ? max(0, p - a.window + 1) : (a.chunk > 0 ? p - p % a.chunk : 0);
+    // kept first keys: their own leading tiles when the window has left them behind, else one contiguous range from 0
+    const int nck = a.keep > 0 && lo > a.keep ? (a.keep + 31) / 32 : 0;
+    const int first = a.keep > 0 && nck == 0 ? 0 : lo & ~31;
+    const int nch = (p - first) / 32 + 1 + nck, cps = (nch + a.nsplit - 1) / a.nsplit, c0 = sp * cps, c1 = min(nch, c0 + cps);
+    const uint16_t* kp = (const uint16_t*)a.kpool + (size_t)g * DIM + q * 8;
+    const uint16_t* vp = (const uint16_t*)a.vpool + (size_t)g * VDIM + row * CPL;
+    at_u4 kn[2][KS]; uint32_t vn[8][VW];
+    auto request = [&](int c) {
+        const int j0 = c < nck ? 32 * c : first + 32 * (c - nck), jl = (c < nck ? a.keep - 1 : p) - j0;      // keys past the last one are fetched again and masked
+        const int page = j0 / a.page_tokens;
+        const size_t base = (size_t)table[page] * a.page_tokens + (j0 - page * a.page_tokens);
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            const uint16_t* k = kp + (base + min(b * 16 + row, jl)) * a.ldk;
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) kn[b][ks] = *reinterpret_cast<const at_u4*>(k + ks * 32);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const uint16_t* v = vp + (base + min((i >> 2) * 16 + 4 * q + (i & 3), jl)) * a.ldv;
+            if constexpr (VW == 1) vn[i][0] = *reinterpret_cast<const uint32_t*>(v);
+            else if constexpr (VW == 2) { const at_u2 x = *reinterpret_cast<const at_u2*>(v); vn[i][0] = x.x; vn[i][1] = x.y; }
+            else {
+#pragma unroll
+                for (int u = 0; u < VW / 4; u++) {
+                    const at_u4 x = *reinterpret_cast<const at_u4*>(v + 8 * u);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) vn[i][4 * u + e] = x[e];
+                }
+            }
+        }
+    };
+    if (c0 + wave < c1) request(c0 + wave);
+    at_u4 qh[KS], qm[KS], ql[KS];
+    {
+        const float qscale = a.softcap > 0.0f ? a.scale : a.scale * AT_LOG2E;
+        const float* qp = a.qkv + (size_t)t * a.ldq + (size_t)head * DIM + q * 8;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            float v[8];
+            *reinterpret_cast<float4*>(&v[0]) = *reinterpret_cast<const float4*>(qp + ks * 32);
+            *reinterpret_cast<float4*>(&v[4]) = *reinterpret_cast<const float4*>(qp + ks * 32 + 4);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                uint32_t x, y, z;
+                at_split(v[2 * i] * qscale, v[2 * i + 1] * qscale, x, y, z);
+                qh[ks][i] = x; qm[ks][i] = y; ql[ks][i] = z;
+            }
+        }
+    }
+    const float slope = a.slopes ? a.slopes[head] * AT_LOG2E : 0.0f;
+    typedef float at_f4 __attribute__((ext_vector_type(4)));
+    float m = -INFINITY, l = 0.0f;
+    at_f4 acc[CPL];
+#pragma unroll
+    for (int j = 0; j < CPL; j++) acc[j] = at_f4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int c = c0 + wave; c < c1; c += NW) {
+        at_u4 kv[2][KS]; uint32_t vv[8][VW];
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) kv[b][ks] = kn[b][ks];
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+#pragma unroll
+            for (int u = 0; u < VW; u++) vv[i][u] = vn[i][u];
+        if (c + NW < c1) request(c + NW);
+        const int j0 = c < nck ? 32 * c : first + 32 * (c - nck), jl = c < nck ? a.keep - 1 : p;
+        at_f4 st[2];
+#pragma unroll
+        for (int b = 0; b < 2; b++) st[b] = at_f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+#pragma unroll
+            for (int b = 0; b < 2; b++) st[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(at_b8, kv[b][ks]), __builtin_bit_cast(at_b8, ql[ks]), st[b], 0, 0, 0);
+#pragma unroll
+            for (int b = 0; b < 2; b++) st[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(at_b8, kv[b][ks]), __builtin_bit_cast(at_b8, qm[ks]), st[b], 0, 0, 0);
+#pragma unroll
+            for (int b = 0; b < 2; b++) st[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(at_b8, kv[b][ks]), __builtin_bit_cast(at_b8, qh[ks]), st[b], 0, 0, 0);
+        }
+        float cm = -INFINITY;
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int key = j0 + b * 16 + 4 * q + i;
+                float sc = st[b][i];
+                if (a.softcap > 0.0f) sc = a.softcap * tanhf(sc / a.softcap) * AT_LOG2E;
+                if (a.slopes) sc -= slope * (float)(p - key);
+                const bool ok = (key <= jl) & ((key >= lo) | (key < a.keep));
+                st[b][i] = ok ? sc : -INFINITY;
+                cm = fmaxf(cm, st[b][i]);
+            }
+        cm = fmaxf(cm, __shfl_xor(cm, 16)); cm = fmaxf(cm, __shfl_xor(cm, 32));
+        const float mn = fmaxf(m, cm), base = mn == -INFINITY ? 0.0f : mn, alpha = __builtin_amdgcn_exp2f(m - base);
+        m = mn; l *= alpha;
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) { const float e = __builtin_amdgcn_exp2f(st[b][i] - base); st[b][i] = e; l += e; }
+        at_u4 ph, pm, pl;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            uint32_t x, y, z;
+            at_split(st[i >> 1][2 * (i & 1)], st[i >> 1][2 * (i & 1) + 1], x, y, z);
+            ph[i] = x; pm[i] = y; pl[i] = z;
+        }
+#pragma unroll
+        for (int j = 0; j < CPL; j++) {
+            at_u4 vf;
+#pragma unroll
+            for (int e = 0; e < 4; e++) vf[e] = __builtin_amdgcn_perm(vv[2 * e + 1][j >> 1], vv[2 * e][j >> 1], (j & 1) ? 0x07060302u : 0x05040100u);
+            acc[j] *= alpha;
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(at_b8, vf), __builtin_bit_cast(at_b8, pl), acc[j], 0, 0, 0);
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(at_b8, vf), __builtin_bit_cast(at_b8, pm), acc[j], 0, 0, 0);
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(at_b8, vf), __builtin_bit_cast(at_b8, ph), acc[j], 0, 0, 0);
+        }
+    }
+    // ---- the waves' states meet: [8 waves][Rb][VDIM + 4] sums | [8][16] maxima | [8][16] denominators | [8][16] factors | [16] 1 / denominator, [16] maximum
+    constexpr int VS = VDIM + 4;
+    float* ml = lds + NW * Rb * VS; float* dl = ml + NW * 16; float* fl = dl + NW * 16; float* rl = fl + NW * 16;
+    l += __shfl_xor(l, 16); l += __shfl_xor(l, 32);
+    if (q == 0) { ml[wave * 16 + row] = m; dl[wave * 16 + row] = l; }
+    if (row < Rb) {
+#pragma unroll
+        for (int j = 0; j < CPL; j++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) lds[(wave * Rb + row) * VS + (4 * q + i) * CPL + j] = acc[j][i];
+    }
+    __syncthreads();
+    const bool last = a.nsplit == 1;
+    if (tid < NW * 16) {
+        const int w = tid >> 4, r = tid & 15;
+        const float sk = last && a.sink && r < Rb ? a.sink[h0 + r] * AT_LOG2E : -INFINITY;
+        float M = sk;
+#pragma unroll
+        for (int i = 0; i < NW; i++) M = fmaxf(M, ml[i * 16 + r]);
+        fl[tid] = ml[tid] == -INFINITY ? 0.0f : exp2f(ml[tid] - M);
+        if (w == 0) {
+            float L = last && a.sink && r < Rb ? exp2f(sk - M) : 0.0f;
+            for (int i = 0; i < NW; i++) { const float mw = ml[i * 16 + r]; if (mw != -INFINITY) L += dl[i * 16 + r] * exp2f(mw - M); }
+            rl[r] = last ? 1.0f / L : L; rl[16 + r] = M;
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < Rb * VDIM; i += 64 * NW) {
+        const int r = i / VDIM, c = i - r * VDIM, h = h0 + r;
+        float v = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; w++) v = __builtin_fmaf(lds[(w * Rb + r) * VS + c], fl[w * 16 + r], v);
+        if (last) {
+            const float gt = a.out_gate ? 1.0f / (1.0f + expf(-a.out_gate[(size_t)t * a.ld_gate + (a.gate_elem ? (size_t)h * VDIM + c : (size_t)h)])) : 1.0f;
+            ((uint16_t*)a.out)[(size_t)t * (a.out_ld ? a.out_ld : a.heads * VDIM) + (size_t)h * VDIM + c] = kr_f32_to_bf16(v * rl[r] * gt * (a.out_scale != 0.0f ? a.out_scale : 1.0f));
+        } else {
+            const size_t slot = ((size_t)t * a.heads + h) * a.nsplit + sp;
+            a.part_acc[slot * VDIM + c] = v;
+            if (c == 0) { a.part_ml[slot * 2] = rl[16 + r]; a.part_ml[slot * 2 + 1] = rl[r]; }
+        }
+    }
+}
+
+template <int DIM, int VDIM> void as_launch(const KrSvAttn& a, hipStream_t st) {
+    const int R = a.heads / a.kv_heads, Rb = R < 16 ? R : 16;
+    const int lds = (8 * Rb * (VDIM + 4) + 3 * 8 * 16 + 32) * (int)sizeof(float);
+    (void)hipFuncSetAttribute((const void*)sv_attn_step_kernel<DIM, VDIM>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    hipLaunchKernelGGL((sv_attn_step_kernel<DIM, VDIM>), dim3(a.T, a.kv_heads, (R + 15) / 16 * a.nsplit), dim3(512), lds, st, a);
+}
 template <int DIM, int VDIM> void at_launch(const KrSvAttn& a, hipStream_t st) {
     const int TQ = AT_ROWS / (a.heads / a.kv_heads);
     hipLaunchKernelGGL((sv_attn_prompt_kernel<DIM, VDIM>), dim3(a.T / TQ + a.n_entries, a.kv_heads, a.nsplit), dim3(256), 0, st, a);
@@ -325,4 +510,25 @@ void kr_sv_attn_prompt(const KrSvAttn& a, hipStream_t st) {
 #define AT_D(DIM_) do { if (a.vdim == 32) at_launch<DIM_, 32>(a, st); else if (a.vdim == 64) at_launch<DIM_, 64>(a, st); else at_launch<DIM_, 128>(a, st); } while (0)
     if (a.dim == 32) AT_D(32); else if (a.dim == 64) AT_D(64); else AT_D(128);
 #undef AT_D
+}
+
+bool kr_sv_attn_step_fits(int dim, int vdim, int ldk, int ldv, int ldq, int page_tokens, bool f32) {
+    if (f32 || page_tokens % 32 != 0 || ldk % 8 != 0 || ldv % 8 != 0 || ldq % 4 != 0) return false;
+    return (dim == 32 || dim == 64 || dim == 128) && (vdim == 32 || vdim == 64 || vdim == 128);      // 256: the split operands no longer fit the registers
+}
+
+// key splits of a decode step: one workgroup up to 256 keys (one round of its waves), then shares of at least 128 up to eight, beyond that shares of 512 for about two
+// workgroups per compute unit.  (us per step of two layers, 1 / 2 / 4 / 8 / 16 shares: one request at 100 keys 248 / 248 / 253 / 252 / 253, at 1024 275 / 268 / 266 / 258 / 258;
+// twelve requests at 1024 333 / 322 / 325 / 320 / 331.)
+int kr_sv_attn_step_splits(int T, int heads, int kv_heads, int max_visible) {
+    if (max_visible <= 256) return 1;
+    const long blocks = (long)T * kv_heads * ((heads / kv_heads + 15) / 16);
+    const long near = std::min(max_visible / 128, 8), far = std::min((long)max_visible / 512, 512 / std::max(blocks, 1L));
+    return (int)std::max(near, far);
+}
+
+void kr_sv_attn_step(const KrSvAttn& a, hipStream_t st) {
+#define AS_D(DIM_) do { if (a.vdim == 32) as_launch<DIM_, 32>(a, st); else if (a.vdim == 64) as_launch<DIM_, 64>(a, st); else as_launch<DIM_, 128>(a, st); } while (0)
+    if (a.dim == 32) AS_D(32); else if (a.dim == 64) AS_D(64); else AS_D(128);
+#undef AS_D
 }

@@ -128,12 +128,19 @@ struct KrSvAttn {
     float* part_ml; float* part_acc; // [T][heads][nsplit][2] running (maximum, denominator), [T][heads][nsplit][vdim] unnormalised sums
     int tq;                          // set by the launcher of the matrix-instruction form: tokens per workgroup
     const int* ent_off; int n_entries;     // [n_entries + 1] first row of every entry of the step: rows of an entry are consecutive positions of one request
-    int prompt;                      // 1: the step's portions are prompt-sized (nsplit from kr_sv_attn_prompt_splits): the 128-row form
+    int form;                        // KR_SV_ATTN_*: the caller's choice (kr_sv_attn_form); nsplit belongs to it
 };
+enum { KR_SV_ATTN_GENERAL = 0, KR_SV_ATTN_PROMPT = 1, KR_SV_ATTN_STEP = 2 };      // the last two keep their running maxima in powers of two
+// which form a layer takes in a step whose largest portion has max_count tokens, and how many workgroups share a token's keys (at most max_visible)
+int kr_sv_attn_form(int T, int n_entries, int max_count, int heads, int kv_heads, int dim, int vdim, int ldk, int ldv, int ldq, int page_tokens, bool f32, int max_visible, int* nsplit);
 // the 128-row form of a bf16 store (kr_serve_attn.hip): sizes and strides it takes; its key splits
 bool kr_sv_attn_prompt_fits(int heads, int kv_heads, int dim, int vdim, int ldk, int ldv, int ldq, bool f32);
 int kr_sv_attn_prompt_splits(int T, int n_entries, int heads, int kv_heads, int max_visible);
 void kr_sv_attn_prompt(const KrSvAttn& a, hipStream_t st);
+// its decode form: one token per workgroup
+bool kr_sv_attn_step_fits(int dim, int vdim, int ldk, int ldv, int ldq, int page_tokens, bool f32);
+int kr_sv_attn_step_splits(int T, int heads, int kv_heads, int max_visible);
+void kr_sv_attn_step(const KrSvAttn& a, hipStream_t st);
 // how many ways to split: fills the chip when the step has few tokens; max_visible = most keys any token of the step sees in this layer
 int kr_sv_attention_splits(int T, int heads, int kv_heads, int dim, int vdim, int ldk, int ldv, bool f32, int max_visible);
 void kr_sv_qk_rms(const KrSvAttn& a, hipStream_t st);                 // unit_norm == 3: the two whole-row statistics of every token

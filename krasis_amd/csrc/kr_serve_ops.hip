@@ -752,8 +752,8 @@ __global__ void __launch_bounds__(256) sv_attn_merge_kernel(const KrSvAttn a) {
     extern __shared__ float wsp[];           // [nsplit] weight of every split, then 1 / denominator
     const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
     const size_t base = ((size_t)t * a.heads + h) * a.nsplit;
-    const float sink = a.sink ? (a.prompt ? a.sink[h] * 1.44269504f : a.sink[h]) : -INFINITY;      // the 128-row form keeps its maxima in powers of two
-    auto ex = [&](float x) { return a.prompt ? exp2f(x) : expf(x); };
+    const float sink = a.sink ? (a.form ? a.sink[h] * 1.44269504f : a.sink[h]) : -INFINITY;      // the split forms keep their maxima in powers of two
+    auto ex = [&](float x) { return a.form ? exp2f(x) : expf(x); };
     float M = sink;
     for (int s = 0; s < a.nsplit; s++) M = fmaxf(M, a.part_ml[(base + s) * 2]);
     for (int s = tid; s < a.nsplit; s += 256) { const float ms = a.part_ml[(base + s) * 2]; wsp[s] = ms == -INFINITY ? 0.0f : ex(ms - M); }
@@ -1914,6 +1914,20 @@ int kr_sv_attention_splits(int T, int heads, int kv_heads, int dim, int vdim, in
     return ns < 1 ? 1 : (int)ns;
 }
 
+// A portion of 32 tokens fills a quarter of a 128-row tile of eight heads per key head; below that the rows of single tokens go to their own workgroups.
+int kr_sv_attn_form(int T, int n_entries, int max_count, int heads, int kv_heads, int dim, int vdim, int ldk, int ldv, int ldq, int page_tokens, bool f32, int max_visible, int* nsplit) {
+    if (max_count >= 32 && kr_sv_attn_prompt_fits(heads, kv_heads, dim, vdim, ldk, ldv, ldq, f32)) {
+        *nsplit = kr_sv_attn_prompt_splits(T, n_entries, heads, kv_heads, max_visible);
+        return KR_SV_ATTN_PROMPT;
+    }
+    if (max_count < 32 && kr_sv_attn_step_fits(dim, vdim, ldk, ldv, ldq, page_tokens, f32)) {
+        *nsplit = kr_sv_attn_step_splits(T, heads, kv_heads, max_visible);
+        return KR_SV_ATTN_STEP;
+    }
+    *nsplit = kr_sv_attention_splits(T, heads, kv_heads, dim, vdim, ldk, ldv, f32, max_visible);
+    return KR_SV_ATTN_GENERAL;
+}
+
 // the matrix-instruction form takes prompt-sized steps whose head sizes fit its register tiling
 template <typename T>
 static bool sv_attn_mfma_launch(const KrSvAttn& a, hipStream_t st) {
@@ -1951,8 +1965,8 @@ static bool sv_attn_mfma_launch(const KrSvAttn& a, hipStream_t st) {
 
 void kr_sv_attention(const KrSvAttn& a, bool f32, hipStream_t st) {
     if (a.T <= 0) return;
-    if (a.prompt) {
-        kr_sv_attn_prompt(a, st);
+    if (a.form != KR_SV_ATTN_GENERAL) {
+        if (a.form == KR_SV_ATTN_PROMPT) kr_sv_attn_prompt(a, st); else kr_sv_attn_step(a, st);
         if (a.nsplit > 1) hipLaunchKernelGGL(sv_attn_merge_kernel<uint16_t>, dim3(a.T, a.heads), dim3(256), (size_t)(a.nsplit + 1) * sizeof(float), st, a);
         return;
     }

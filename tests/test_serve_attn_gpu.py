@@ -51,3 +51,20 @@ def test_portions_deep_in_a_request_share_keys(window):
         x0 = W["embed"].astype(np.float64)[np.asarray(t[k:])]
         assert row_errors(got[lo:lo + n] - x0, ref - x0).max() < 2e-2
         lo += n
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(6, 3, 32, 64), (5, 1, 64, 32), (16, 1, 64, 128), (40, 1, 32, 32), (8, 2, 128, 128)])
+@pytest.mark.parametrize("ctx,window", [(1, 0), (31, 3), (64, 33), (255, 0), (700, 0), (1300, 290)])
+def test_single_tokens(heads, kv_heads, dim, vdim, ctx, window):
+    # three requests, one token each, at positions around the 32-key tile, inside one workgroup and split over several; groups of 2 - 40 heads per key head
+    cfg = model(heads, kv_heads, dim, vdim, window, rot=8); W = O.random_weights(cfg, 27)
+    seqs = [tokens(cfg, n + 1, 28 + i) for i, n in enumerate((ctx, max(1, ctx - 5), max(1, ctx // 2)))]
+    eng = engine(cfg, W, "bfloat16", max_tokens=8192)
+    for i, s in enumerate(seqs):
+        eng.step([(i, s[:-1], [])])
+    eng.store.set_capture(True)
+    eng.step([(i, s[-1:], [0]) for i, s in enumerate(seqs)])
+    got = eng.store.read_capture(3)[0]
+    x0 = W["embed"].astype(np.float64)[[s[-1] for s in seqs]]
+    ref = np.stack([O.forward(cfg, W, s)[1][0][-1] for s in seqs])
+    assert row_errors(got - x0, ref - x0).max() < 2e-2

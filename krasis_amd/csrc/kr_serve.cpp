@@ -1017,7 +1017,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     const int* d_tab = d_tok + n_meta;
     // ---- scratch sized for this step
     const bool seq = c.block_kind == KR_SERVE_BLOCK_SEQUENTIAL;
-    size_t max_qkv = 0, max_att = 0, max_gu = 0, max_y = 0, max_rows = 0, max_pairs = 0, max_vf = 0; int max_E = 1;
+    size_t max_qkv = 0, max_att = 0, max_gu = 0, max_y = 0, max_rows = 0, max_pairs = 0, max_vf = 0, max_hist = 0; int max_E = 1;
     size_t lq_c = 0, lq_2 = 0, lq_n = 0, lq_e = 0, att2 = 0, head_i = 0, max_lin = 0, lin_tok = 0, lin_sb = 0, lin_nb = 0; bool whole_norm = false;
     size_t max_pconv = 0, max_sconv = 0, max_ga1 = 0, max_gz = 0, max_ssdz = 0;
     // prompt portions take the chunked form of the recurrent mixers (blocks of 64 tokens on the matrix instruction), decode-sized steps the token-by-token form
@@ -1068,12 +1068,13 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
             max_gu = std::max(max_gu, std::max((size_t)d.top * 2 * d.expert_ff, (size_t)2 * d.shared_ff));
             max_y = std::max(max_y, std::max((size_t)d.top * d.expert_ff, (size_t)d.shared_ff));
             max_rows = std::max(max_rows, (size_t)d.top * W); max_pairs = std::max(max_pairs, (size_t)d.top); max_E = std::max(max_E, d.experts);
+            max_hist = std::max(max_hist, kr_sv_moe_hist_ints(T * d.top, d.experts));
         }
     }
     const size_t Ts = (size_t)T;
     if (s->x.ensure(Ts * W * 4) || s->h.ensure(Ts * W * s->esz) || s->qkv.ensure(Ts * max_qkv * 4) || s->att.ensure(Ts * max_att * s->esz) || s->mix.ensure(Ts * W * 4) ||
         s->gu.ensure(Ts * max_gu * 4 + 16) || s->y.ensure(Ts * max_y * s->esz + 16) || s->rows.ensure(Ts * max_rows * 4 + 16) || s->ffout.ensure(Ts * W * 4) ||
-        s->ids.ensure(Ts * max_pairs * 4 + 16) || s->rz.ensure(Ts * (size_t)max_E * 8 + 16) || s->wts.ensure(Ts * max_pairs * 4 + 16) || s->moe_i.ensure((Ts * max_pairs * 4 + 3 * (size_t)max_E + 8) * 4) ||
+        s->ids.ensure(Ts * max_pairs * 4 + 16) || s->rz.ensure(Ts * (size_t)max_E * 8 + 16) || s->wts.ensure(Ts * max_pairs * 4 + 16) || s->moe_i.ensure((Ts * max_pairs * 4 + (size_t)max_E + 8 + max_hist) * 4) ||
         s->hw.ensure((size_t)std::max(n_want, 1) * W * s->esz) || s->logits.ensure((size_t)std::max(n_want, 1) * c.vocab * 4) || s->amax.ensure((size_t)std::max(n_want, 1) * 4))
         return kr_fail(KR_ERR_HIP, "step scratch for %d tokens", T);
     if ((max_vf && s->v_first.ensure(Ts * max_vf * 4)) ||
@@ -1397,13 +1398,12 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
             dense = (const float*)s->ffout.p;
         } else if (d.mlp_kind == KR_SERVE_MLP_MOE) {
             const int E = d.experts, top = d.top, F = d.expert_ff, P = T * top;
-            int* counts_d = mi; int* seg = mi + E; int* cursor = seg + E + 1; int* src_row = cursor + E; int* row_group = src_row + P; int* pp = row_group + P;
+            int* seg = mi; int* src_row = seg + E + 1; int* row_group = src_row + P; int* pp = row_group + P; int* hist = pp + 2 * P;
             float* row_w = d.expert_in_weight ? (float*)(pp + P) : nullptr;
             {
                 Timer tm(s, 4);
-                kr_sv_router_select(hz + l.off_router, l.n_h, s->f32 ? 1 : 2, d.router_bias ? (const float*)l.router_b.p : nullptr, d.router_bias, d.router_score, d.group_score, T, E, top,
-                                    d.groups, d.keep, d.renorm, (int*)s->ids.p, (float*)s->wts.p, st);
-                kr_sv_moe_sort((const int*)s->ids.p, T, top, E, counts_d, seg, cursor, src_row, row_group, pp, (const float*)s->wts.p, row_w, st);
+                kr_sv_router_sort(hz + l.off_router, l.n_h, s->f32 ? 1 : 2, d.router_bias ? (const float*)l.router_b.p : nullptr, d.router_bias, d.router_score, d.group_score, T, E, top, d.groups,
+                                  d.keep, d.renorm, (int*)s->ids.p, (float*)s->wts.p, hist, seg, src_row, row_group, pp, row_w, st);
             }
             g = KrSvGemm{}; g.A = s->h.p; g.lda = W; g.W = l.egu.p; g.w_stride = (size_t)2 * F * W; g.C = (float*)s->gu.p; g.ldc = 2 * F; g.M = P; g.N = 2 * F; g.K = W;
             g.a_rows = src_row; g.seg = seg; g.row_group = row_group; g.n_groups = E;

@@ -154,12 +154,11 @@ void kr_sv_attention(const KrSvAttn& a, bool f32, hipStream_t st);   // windowed
 // bias [E] or null: bias_mode 1 joins the logits before anything else; 2 joins the scores for the choice of groups and experts only (the weights are the
 // scores without it).  score_kind 0: softmax over all experts, 1: sigmoid of every logit.  group_kind 0: a group's score is its largest choice score,
 // 1: the sum of its two largest.  Experts outside the kept groups cannot be chosen, whatever their score.  renorm: weights / (their sum + 1e-20).
-void kr_sv_router_select(const float* z, int ld, int parts, const float* bias, int bias_mode, int score_kind, int group_kind, int T, int E, int top, int groups, int keep,
-                         int renorm, int* ids, float* wts, hipStream_t st);
-// rows of every expert: seg[E + 1], src_row[T * top] (token of sorted row), row_group[T * top], pair_pos[T * top] (sorted row of (token, slot)); with row_w also
-// the weight of every sorted row (wts [T * top])
-void kr_sv_moe_sort(const int* ids, int T, int top, int E, int* counts, int* seg, int* cursor, int* src_row, int* row_group, int* pair_pos, const float* wts, float* row_w,
-                    hipStream_t st);
+// The pairs then sorted by expert: seg[E + 1], src_row[T * top] (token of sorted row), row_group[T * top], pair_pos[T * top] (sorted row of (token, slot)); with row_w also
+// the weight of every sorted row.  hist: kr_sv_moe_hist_ints(T * top, E) integers of scratch.
+size_t kr_sv_moe_hist_ints(int pairs, int E);
+void kr_sv_router_sort(const float* z, int ld, int parts, const float* bias, int bias_mode, int score_kind, int group_kind, int T, int E, int top, int groups, int keep, int renorm, int* ids,
+                       float* wts, int* hist, int* seg, int* src_row, int* row_group, int* pair_pos, float* row_w, hipStream_t st);
 // gu rows `ld` floats apart (gate at [0, F), up at [F, 2F)) -> y [M, F] storage type; row_w [M] or null: multiplies a row's gate and up columns first
 // up_tab: the up factor of (row r, column c) is up_tab[up_rows[r] * up_ld + up_off + c] (storage type) instead of gu's second half
 void kr_sv_act(const float* gu, int ld, void* y, bool f32, int M, int F, int kind, float limit, float alpha, const float* row_w, hipStream_t st, const void* up_tab = nullptr,

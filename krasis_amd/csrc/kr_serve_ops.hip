@@ -850,46 +850,208 @@ __global__ void __launch_bounds__(64) sv_router_select_kernel(const float* __res
     }
 }
 
-__global__ void sv_fill_int_kernel(int* p, int n, int v) { const int i = blockIdx.x * blockDim.x + threadIdx.x; if (i < n) p[i] = v; }
-__global__ void sv_moe_count_kernel(const int* __restrict__ ids, int n, int* __restrict__ counts) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) atomicAdd(&counts[ids[i]], 1);
-}
-__global__ void sv_moe_scan_kernel(const int* __restrict__ counts, int E, int* __restrict__ seg, int* __restrict__ cursor) {
-    if (threadIdx.x == 0) {
-        int o = 0;
-        for (int e = 0; e < E; e++) { seg[e] = o; cursor[e] = 0; o += counts[e]; }
-        seg[E] = o;
+// Up to 128 experts: the scores of a token live in a wave's registers (NV per lane) and an expert's place among them is COUNTED -- every value is broadcast once and compared with
+// all -- instead of found by `top` rounds of a wave-wide maximum, each a chain of twelve LDS shuffles and two barriers.  Same order (largest first, lowest index among equals,
+// NaN and minus infinity never chosen), same sums.  SORT: a decode step's tokens are one workgroup's waves (T <= 16), which then sorts their rows by expert in the same launch.
+// 64 experts, top 6: one token 12.4 + 4.7 us as two launches -> 4.0, twelve 12.8 + 4.6 -> 7.0, 4096 (choice alone) 25 -> 12.
+template <int NV, bool SORT>
+__global__ void __launch_bounds__(SORT ? 1024 : 256) sv_router_rank_kernel(const float* __restrict__ z, int ld, int parts, const float* __restrict__ bias, int bias_mode, int score_kind,
+                                                                          int group_kind, int T, int E, int top, int groups, int keep, int renorm, int* __restrict__ ids, float* __restrict__ wts,
+                                                                          int* __restrict__ seg, int* __restrict__ src_row, int* __restrict__ row_group, int* __restrict__ pair_pos,
+                                                                          float* __restrict__ row_w) {
+    constexpr int NWAVES = SORT ? 16 : 4;
+    __shared__ float gsc[NWAVES][64];                       // choice scores by expert while groups are scored (one wave's 64 at a time), then the groups' scores
+    __shared__ float cho[NWAVES][64 * NV];
+    __shared__ int s_ids[SORT ? 16 * 64 : 1]; __shared__ float s_w[SORT ? 16 * 64 : 1];
+    __shared__ int cnt[SORT ? 128 : 1];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = blockIdx.x * NWAVES + wave;
+    if (SORT) { if (threadIdx.x < 128) cnt[threadIdx.x] = 0; }
+    if (t < T) {
+        float s[NV], c[NV];
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const int e = lane + 64 * i;
+            float v = 0.0f;
+            if (e < E) {
+                v = z[(size_t)t * ld + e];
+                for (int q = 1; q < parts; q++) v += z[(size_t)t * ld + (size_t)q * E + e];
+                if (bias && bias_mode == 1) v += bias[e];
+            }
+            s[i] = v;
+        }
+        if (score_kind == 1) {
+#pragma unroll
+            for (int i = 0; i < NV; i++) s[i] = 1.0f / (1.0f + expf(-s[i]));
+        } else {
+            float mx = -INFINITY, sum = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NV; i++) if (lane + 64 * i < E) mx = fmaxf(mx, s[i]);
+            mx = sv_wave_max(mx);
+#pragma unroll
+            for (int i = 0; i < NV; i++) if (lane + 64 * i < E) { s[i] = expf(s[i] - mx); sum += s[i]; }
+            const float inv = 1.0f / sv_wave_sum(sum);
+#pragma unroll
+            for (int i = 0; i < NV; i++) s[i] *= inv;
+        }
+        bool ok[NV];
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const int e = lane + 64 * i;
+            c[i] = e < E ? ((bias && bias_mode == 2) ? s[i] + bias[e] : s[i]) : -INFINITY;
+            ok[i] = e < E && c[i] == c[i] && c[i] != -INFINITY;
+        }
+        if (keep < groups) {                                 // only the experts of the `keep` best groups stay
+            const int per = E / groups;
+#pragma unroll
+            for (int i = 0; i < NV; i++) cho[wave][lane + 64 * i] = c[i];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            float g = -INFINITY;
+            if (lane < groups) {
+                float v = -INFINITY, v2 = -INFINITY;         // the two largest of the group
+                for (int e = lane * per; e < (lane + 1) * per; e++) { const float x = cho[wave][e]; if (x > v) { v2 = v; v = x; } else if (x > v2) v2 = x; }
+                g = (group_kind == 1 && per > 1) ? v + v2 : v;
+            }
+            int rank = 0;
+            for (int j = 0; j < groups; j++) { const float o = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(g), j)); rank += (o > g || (o == g && j < lane)) ? 1 : 0; }
+            gsc[wave][lane] = (lane < groups && g == g && g != -INFINITY && rank < keep) ? 1.0f : 0.0f;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+            for (int i = 0; i < NV; i++) { const int e = lane + 64 * i; if (e < E && gsc[wave][e / per] == 0.0f) ok[i] = false; }
+        }
+        int rank[NV];
+#pragma unroll
+        for (int i = 0; i < NV; i++) { rank[i] = 0; if (!ok[i]) c[i] = -INFINITY; }
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+#pragma unroll 16
+            for (int l = 0; l < 64; l++) {
+                const float o = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c[j]), l));
+#pragma unroll
+                for (int i = 0; i < NV; i++) rank[i] += (o > c[i] || (o == c[i] && l + 64 * j < lane + 64 * i)) ? 1 : 0;
+            }
+        }
+        int chosen = 0;
+#pragma unroll
+        for (int i = 0; i < NV; i++) { if (!ok[i]) rank[i] = 1 << 20; chosen += __popcll(__ballot(rank[i] < top)); }
+        float wsum = 0.0f;
+        for (int r = 0; r < top; r++) {                      // in order of choice
+            float w = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NV; i++) {
+                const unsigned long long m = __ballot(rank[i] == r);
+                if (m) w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s[i]), __ffsll(m) - 1));
+            }
+            wsum += w;
+        }
+        const float rinv = renorm ? 1.0f / (wsum + 1e-20f) : 1.0f;
+        auto put = [&](int r, int e, float w) {
+            ids[(size_t)t * top + r] = e; wts[(size_t)t * top + r] = w;
+            if (SORT) { s_ids[wave * top + r] = e; s_w[wave * top + r] = w; }
+        };
+#pragma unroll
+        for (int i = 0; i < NV; i++) if (rank[i] < top) put(rank[i], lane + 64 * i, renorm ? s[i] * rinv : s[i]);
+        for (int r = chosen + lane; r < top; r += 64) put(r, 0, renorm ? 0.0f * rinv : 0.0f);      // fewer allowed experts than `top` (refused on the host): zero-weight slots
+    }
+    if (!SORT) return;
+    __syncthreads();
+    const int n = T * top;
+    for (int i = threadIdx.x; i < n; i += 1024) atomicAdd(&cnt[s_ids[i]], 1);
+    __syncthreads();
+    if (wave == 0) {                                         // starts of the experts' rows: a prefix sum over two counters per lane
+        const int a = cnt[2 * lane], b = cnt[2 * lane + 1];
+        int sum = a + b;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(sum, o); if (lane >= o) sum += v; }
+        const int at = sum - a - b;
+        if (2 * lane < E) seg[2 * lane] = at;
+        if (2 * lane + 1 < E) seg[2 * lane + 1] = at + a;
+        if (lane == 63) seg[E] = sum;
+        cnt[2 * lane] = at; cnt[2 * lane + 1] = at + a;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += 1024) {
+        const int e = s_ids[i], pos = atomicAdd(&cnt[e], 1);
+        src_row[pos] = i / top; row_group[pos] = e; pair_pos[i] = pos;
+        if (row_w) row_w[pos] = s_w[i];
     }
 }
-__global__ void sv_moe_fill_kernel(const int* __restrict__ ids, int n, int top, const int* __restrict__ seg, int* __restrict__ cursor, int* __restrict__ src_row,
-                                   int* __restrict__ row_group, int* __restrict__ pair_pos, const float* __restrict__ wts, float* __restrict__ row_w) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int e = ids[i];
-    const int pos = seg[e] + atomicAdd(&cursor[e], 1);
-    src_row[pos] = i / top; row_group[pos] = e; pair_pos[i] = pos;
-    if (row_w) row_w[pos] = wts[i];
+
+// Rows of a prompt's pairs sorted by expert, without atomics on a few hot words of memory (64 counters for 24576 pairs: 39 us to count and 39 us to place): a block counts its
+// SORT_PAIRS pairs in LDS, one workgroup turns the blocks' counts into their first rows, the blocks place their pairs from LDS cursors (three launches of 5 us).
+constexpr int SORT_PAIRS = 2048;
+__global__ void __launch_bounds__(256) sv_moe_count_kernel(const int* __restrict__ ids, int n, int E, int* __restrict__ hist) {
+    extern __shared__ int cnt[];             // [E]
+    for (int e = threadIdx.x; e < E; e += 256) cnt[e] = 0;
+    __syncthreads();
+    const int i1 = min(n, (blockIdx.x + 1) * SORT_PAIRS);
+    for (int i = blockIdx.x * SORT_PAIRS + threadIdx.x; i < i1; i += 256) atomicAdd(&cnt[ids[i]], 1);
+    __syncthreads();
+    for (int e = threadIdx.x; e < E; e += 256) hist[(size_t)blockIdx.x * E + e] = cnt[e];
+}
+__global__ void __launch_bounds__(1024) sv_moe_scan_kernel(int* __restrict__ hist, int blocks, int E, int* __restrict__ seg) {
+    __shared__ int wsum[16]; __shared__ int carry;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (threadIdx.x == 0) carry = 0;
+    for (int e0 = 0; e0 < E; e0 += 1024) {
+        const int e = e0 + threadIdx.x;
+        int tot = 0;
+        if (e < E) for (int b = 0; b < blocks; b++) tot += hist[(size_t)b * E + e];
+        int sum = tot;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(sum, o); if (lane >= o) sum += v; }
+        __syncthreads();
+        if (lane == 63) wsum[wave] = sum;
+        __syncthreads();
+        int at = carry + sum - tot;
+        for (int w = 0; w < wave; w++) at += wsum[w];
+        if (e < E) {
+            seg[e] = at;
+            for (int b = 0; b < blocks; b++) { const size_t i = (size_t)b * E + e; const int c = hist[i]; hist[i] = at; at += c; }
+            if (e == E - 1) seg[E] = at;
+        }
+        __syncthreads();
+        if (threadIdx.x == 1023) { int c = carry; for (int w = 0; w < 16; w++) c += wsum[w]; carry = c; }
+        __syncthreads();
+    }
+}
+__global__ void __launch_bounds__(256) sv_moe_fill_kernel(const int* __restrict__ ids, int n, int top, int E, const int* __restrict__ hist, int* __restrict__ src_row,
+                                                          int* __restrict__ row_group, int* __restrict__ pair_pos, const float* __restrict__ wts, float* __restrict__ row_w) {
+    extern __shared__ int cnt[];             // [E] next row of this block's pairs of the expert
+    for (int e = threadIdx.x; e < E; e += 256) cnt[e] = hist[(size_t)blockIdx.x * E + e];
+    __syncthreads();
+    const int i1 = min(n, (blockIdx.x + 1) * SORT_PAIRS);
+    for (int i = blockIdx.x * SORT_PAIRS + threadIdx.x; i < i1; i += 256) {
+        const int e = ids[i];
+        const int pos = atomicAdd(&cnt[e], 1);
+        src_row[pos] = i / top; row_group[pos] = e; pair_pos[i] = pos;
+        if (row_w) row_w[pos] = wts[i];
+    }
 }
 
-// the three launches above as one workgroup, for decode-sized batches (n pairs <= 1024, E counters in LDS)
+// the same as one workgroup, for decode-sized batches (n pairs <= 1024)
 __global__ void __launch_bounds__(256) sv_moe_sort_small_kernel(const int* __restrict__ ids, int n, int top, int E, int* __restrict__ seg, int* __restrict__ src_row,
                                                                 int* __restrict__ row_group, int* __restrict__ pair_pos, const float* __restrict__ wts, float* __restrict__ row_w) {
-    extern __shared__ int cnt[];             // counts[E] | start[E]
-    int* start = cnt + E;
+    extern __shared__ int cnt[];             // [E] counts, then the next row of the expert
     for (int e = threadIdx.x; e < E; e += 256) cnt[e] = 0;
     __syncthreads();
     for (int i = threadIdx.x; i < n; i += 256) atomicAdd(&cnt[ids[i]], 1);
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 64) {                  // 64 experts at a time through a prefix sum over the lanes
         int o = 0;
-        for (int e = 0; e < E; e++) { start[e] = o; seg[e] = o; o += cnt[e]; cnt[e] = 0; }
-        seg[E] = o;
+        for (int e0 = 0; e0 < E; e0 += 64) {
+            const int e = e0 + (int)threadIdx.x, c = e < E ? cnt[e] : 0;
+            int sum = c;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) { const int v = __shfl_up(sum, d); if ((int)threadIdx.x >= d) sum += v; }
+            if (e < E) { seg[e] = o + sum - c; cnt[e] = o + sum - c; }
+            o += __shfl(sum, 63);
+        }
+        if (threadIdx.x == 0) seg[E] = o;
     }
     __syncthreads();
     for (int i = threadIdx.x; i < n; i += 256) {
         const int e = ids[i];
-        const int pos = start[e] + atomicAdd(&cnt[e], 1);
+        const int pos = atomicAdd(&cnt[e], 1);
         src_row[pos] = i / top; row_group[pos] = e; pair_pos[i] = pos;
         if (row_w) row_w[pos] = wts[i];
     }
@@ -1998,25 +2160,30 @@ void kr_sv_attention(const KrSvAttn& a, bool f32, hipStream_t st) {
 #undef SV_ATT
 }
 
-void kr_sv_router_select(const float* z, int ld, int parts, const float* bias, int bias_mode, int score_kind, int group_kind, int T, int E, int top, int groups, int keep,
-                         int renorm, int* ids, float* wts, hipStream_t st) {
-    if (T <= 0) return;
-    const size_t lds = (size_t)(2 * E + 2 * groups) * sizeof(float);
-    hipLaunchKernelGGL(sv_router_select_kernel, dim3(T), dim3(64), lds, st, z, ld, parts, bias, bias_mode, score_kind, group_kind, E, top, groups, keep, renorm, ids, wts);
-}
+size_t kr_sv_moe_hist_ints(int pairs, int E) { return pairs <= 1024 && E <= 4096 ? 0 : ((size_t)pairs + SORT_PAIRS - 1) / SORT_PAIRS * E; }
 
-void kr_sv_moe_sort(const int* ids, int T, int top, int E, int* counts, int* seg, int* cursor, int* src_row, int* row_group, int* pair_pos, const float* wts, float* row_w,
-                    hipStream_t st) {
+void kr_sv_router_sort(const float* z, int ld, int parts, const float* bias, int bias_mode, int score_kind, int group_kind, int T, int E, int top, int groups, int keep, int renorm, int* ids,
+                       float* wts, int* hist, int* seg, int* src_row, int* row_group, int* pair_pos, float* row_w, hipStream_t st) {
     const int n = T * top;
     if (n <= 0) return;
-    if (n <= 1024 && E <= 4096) {
-        hipLaunchKernelGGL(sv_moe_sort_small_kernel, dim3(1), dim3(256), (size_t)2 * E * sizeof(int), st, ids, n, top, E, seg, src_row, row_group, pair_pos, wts, row_w);
+    const bool ranked = E <= 128 && top <= 64 && groups <= 64;
+#define SV_RANK(NV_, SORT_, GRID_, NT_) hipLaunchKernelGGL((sv_router_rank_kernel<NV_, SORT_>), dim3(GRID_), dim3(NT_), 0, st, z, ld, parts, bias, bias_mode, score_kind, group_kind, T, E, top, groups, \
+                                                           keep, renorm, ids, wts, seg, src_row, row_group, pair_pos, row_w)
+    if (ranked && T <= 16) {                 // a wave per token, the sort in the same launch
+        if (E <= 64) SV_RANK(1, true, 1, 1024); else SV_RANK(2, true, 1, 1024);
         return;
     }
-    hipLaunchKernelGGL(sv_fill_int_kernel, dim3((E + 255) / 256), dim3(256), 0, st, counts, E, 0);
-    hipLaunchKernelGGL(sv_moe_count_kernel, dim3((n + 255) / 256), dim3(256), 0, st, ids, n, counts);
-    hipLaunchKernelGGL(sv_moe_scan_kernel, dim3(1), dim3(64), 0, st, counts, E, seg, cursor);
-    hipLaunchKernelGGL(sv_moe_fill_kernel, dim3((n + 255) / 256), dim3(256), 0, st, ids, n, top, seg, cursor, src_row, row_group, pair_pos, wts, row_w);
+    if (ranked) { if (E <= 64) SV_RANK(1, false, (T + 3) / 4, 256); else SV_RANK(2, false, (T + 3) / 4, 256); }
+    else hipLaunchKernelGGL(sv_router_select_kernel, dim3(T), dim3(64), (size_t)(2 * E + 2 * groups) * sizeof(float), st, z, ld, parts, bias, bias_mode, score_kind, group_kind, E, top, groups, keep, renorm, ids, wts);
+#undef SV_RANK
+    if (n <= 1024 && E <= 4096) {
+        hipLaunchKernelGGL(sv_moe_sort_small_kernel, dim3(1), dim3(256), (size_t)E * sizeof(int), st, ids, n, top, E, seg, src_row, row_group, pair_pos, wts, row_w);
+        return;
+    }
+    const int blocks = (n + SORT_PAIRS - 1) / SORT_PAIRS;
+    hipLaunchKernelGGL(sv_moe_count_kernel, dim3(blocks), dim3(256), (size_t)E * sizeof(int), st, ids, n, E, hist);
+    hipLaunchKernelGGL(sv_moe_scan_kernel, dim3(1), dim3(1024), 0, st, hist, blocks, E, seg);
+    hipLaunchKernelGGL(sv_moe_fill_kernel, dim3(blocks), dim3(256), (size_t)E * sizeof(int), st, ids, n, top, E, hist, src_row, row_group, pair_pos, wts, row_w);
 }
 
 void kr_sv_act(const float* gu, int ld, void* y, bool f32, int M, int F, int kind, float limit, float alpha, const float* row_w, hipStream_t st, const void* up_tab,

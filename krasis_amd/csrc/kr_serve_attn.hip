@@ -517,13 +517,12 @@ bool kr_sv_attn_step_fits(int dim, int vdim, int ldk, int ldv, int ldq, int page
     return (dim == 32 || dim == 64 || dim == 128) && (vdim == 32 || vdim == 64 || vdim == 128);      // 256: the split operands no longer fit the registers
 }
 
-// key splits of a decode step: one workgroup up to 256 keys (one round of its waves), then shares of at least 128 up to eight, beyond that shares of 512 for about two
-// workgroups per compute unit.  (us per step of two layers, 1 / 2 / 4 / 8 / 16 shares: one request at 100 keys 248 / 248 / 253 / 252 / 253, at 1024 275 / 268 / 266 / 258 / 258;
-// twelve requests at 1024 333 / 322 / 325 / 320 / 331.)
+// key splits of a decode step: one workgroup up to 256 keys (one round of its waves), then two, four and eight (powers of two: a new count is a new step to capture), beyond 1024
+// shares of 512 for about two workgroups per compute unit.  (us per step of two layers, 1 / 2 / 4 / 8 / 16 shares: one request at 100 keys 248 / 248 / 253 / 252 / 253, at 1024
+// 275 / 268 / 266 / 258 / 258; twelve requests at 1024 333 / 322 / 325 / 320 / 331.)
 int kr_sv_attn_step_splits(int T, int heads, int kv_heads, int max_visible) {
-    if (max_visible <= 256) return 1;
     const long blocks = (long)T * kv_heads * ((heads / kv_heads + 15) / 16);
-    const long near = std::min(max_visible / 128, 8), far = std::min((long)max_visible / 512, 512 / std::max(blocks, 1L));
+    const long near = max_visible <= 256 ? 1 : max_visible < 512 ? 2 : max_visible < 1024 ? 4 : 8, far = std::min((long)max_visible / 512, 512 / std::max(blocks, 1L));
     return (int)std::max(near, far);
 }
 

@@ -1110,10 +1110,21 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     // every launch of the step, in order; no allocation, no host copy: the same body runs eagerly or under stream capture
     auto enqueue = [&]() -> int {
     float* x = (float*)s->x.p;
-    {
+    const int NG = c.norm_groups > 1 ? c.norm_groups : 1;
+    const bool canon = c.canon_taps > 1;
+    const float escale = c.embed_scale != 0.0f ? c.embed_scale : 1.0f;
+    const void* table2 = c.pos_rows > 0 ? s->pos.p : c.bigram_buckets > 0 ? s->bigram.p : nullptr;
+    const int* rows2 = c.pos_rows > 0 ? d_pos : d_brow;
+    const SvLayer& l0 = s->L[0];
+    bool normed = false;                 // the first sublayer's input left the embedding's launch
+    if (c.pre_norm && !l0.d.pre_add && !c.embed_norm) {
         Timer tm(s, 7);
-        kr_sv_embed(s->embed.p, s->f32, d_tok, x, c.pre_norm ? nullptr : s->h.p, T, W, c.embed_scale != 0.0f ? c.embed_scale : 1.0f, c.pos_rows > 0 ? s->pos.p : c.bigram_buckets > 0 ? s->bigram.p : nullptr,
-                    c.pos_rows > 0 ? d_pos : d_brow, st);     // without input norms the first sublayer reads the embedding row itself
+        normed = kr_sv_embed_norm(s->embed.p, s->f32, d_tok, x, T, W, escale, table2, rows2, (const float*)l0.norm_w.p, c.norm_bias ? (const float*)l0.norm_b.p : nullptr, s->h.p, c.norm_eps,
+                                  c.norm_kind, NG, (canon || l0.wkv()) ? (float*)s->h32.p : nullptr, st);
+    }
+    if (!normed) {
+        Timer tm(s, 7);
+        kr_sv_embed(s->embed.p, s->f32, d_tok, x, c.pre_norm ? nullptr : s->h.p, T, W, escale, table2, rows2, st);     // without input norms the first sublayer reads the embedding row itself
     }
     if (c.embed_norm) { Timer tm(s, 0); kr_sv_stream_norm(x, nullptr, (const float*)s->enorm_w.p, nullptr, true, nullptr, s->f32, T, W, c.norm_eps, c.norm_kind, c.norm_groups > 1 ? c.norm_groups : 1, st); }
     {
@@ -1130,8 +1141,6 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     };
     // the residual sum that ends a sublayer (or, in a parallel block, the layer); `next`: the norm of the sublayer that reads the new x, null with
     // hand_on = the row as it is, or nothing when no sublayer follows
-    const int NG = c.norm_groups > 1 ? c.norm_groups : 1;
-    const bool canon = c.canon_taps > 1;
     // gate: 0 none, 1 the mixer's (logits in rg, the output projection's bias, and the input convolution's rows of this layer are kept), 2 the feed-forward's
     // (logits in the last row block of hz).  to_mixer: the handed-on row feeds a mixer (an f32 copy goes along for its input convolution)
     const SvLayer* res_layer = nullptr; const SvLayer* res_run = nullptr; int res_gate_kind = 0; bool res_to_mixer = false, res_next32 = false;
@@ -1156,7 +1165,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         r.h_out = hand_on ? s->h.p : nullptr; r.T = T; r.width = W; r.kind = c.norm_kind; r.eps = c.norm_eps;
         kr_sv_residual_norm(r, s->f32, st);
     };
-    if (c.pre_norm && !s->L[0].d.pre_add) {
+    if (c.pre_norm && !s->L[0].d.pre_add && !normed) {
         Timer tm(s, 0);
         kr_sv_norm(x, nullptr, (const float*)s->L[0].norm_w.p, c.norm_bias ? (const float*)s->L[0].norm_b.p : nullptr, s->h.p, s->f32, T, W, c.norm_eps, c.norm_kind, NG,
                    (canon || s->L[0].wkv()) ? (float*)s->h32.p : nullptr, st);

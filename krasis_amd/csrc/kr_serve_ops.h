@@ -54,6 +54,9 @@ enum { KR_SV_ACT_GELU_TANH = 0, KR_SV_ACT_CLAMPED_SWIGLU = 1, KR_SV_ACT_SILU = 2
 // scale: the row is multiplied by it (1 = as it is)
 // table2 / rows2: optional second table whose row rows2[t] is added as it is (a hashed pair-of-tokens embedding)
 void kr_sv_embed(const void* table, bool f32, const int* tokens, float* x, void* h_out, int T, int width, float scale, const void* table2, const int* rows2, hipStream_t st);
+// the same and the first sublayer's input norm in one launch (out: the normed row in the storage type, out32 optional f32 copy); false: the width is not for it, nothing was launched
+bool kr_sv_embed_norm(const void* table, bool f32, const int* tokens, float* x, int T, int width, float scale, const void* table2, const int* rows2, const float* w, const float* b, void* out,
+                      float eps, int kind, int groups, float* out32, hipStream_t st);
 // the stream itself: x[t] += add (optional [width]); then, with w, either x[t] <- norm(x[t]) * w (in_place: the normed row IS the stream) or
 // out[t] = norm(x[t]) * w in the storage type (the next sublayer's input).  One workgroup per row, the row held in LDS.
 void kr_sv_stream_norm(float* x, const float* add, const float* w, const float* b, bool in_place, void* out, bool out_f32, int T, int width, float eps, int kind, int groups,

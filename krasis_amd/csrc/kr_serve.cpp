@@ -1133,11 +1133,23 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     }
     int* mi = (int*)s->moe_i.p;
     // down projection of a gated feed-forward: decode-sized problems form the activation inside the projection's launch, larger ones write it once
-    auto down_proj = [&](KrSvGemm g, const float* gu, int ld, int rows_m, int F, int kind, float limit, float alpha, const float* row_w = nullptr) {
+    // (formed: the projection before wrote it itself, see pair_up)
+    auto down_proj = [&](KrSvGemm g, const float* gu, int ld, int rows_m, int F, int kind, float limit, float alpha, const float* row_w = nullptr, bool formed = false) {
+        if (formed) { g.A = s->y.p; g.lda = F; Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); return; }
         if (kr_sv_gemm_takes_act(g, s->f32, gu, ld)) { g.act_row_w = row_w; g.act_gu = gu; g.act_ld = ld; g.act_kind = kind; g.act_limit = limit; g.act_alpha = alpha; g.A = nullptr; Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); return; }
         { Timer tm(s, 5); kr_sv_act(gu, ld, s->y.p, s->f32, rows_m, F, kind, limit, alpha, row_w, st, g.up_tab, g.up_rows, g.up_ld, g.up_off); }
         g.A = s->y.p; g.lda = F;
         { Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); }
+    };
+    // prompt-sized: the product `up` whose columns [lo, lo + 2 F) are gate | up of the feed-forward that `down` ends hands on their activation (in y: nothing else may use
+    // it until that down projection has read it).  False: it does not, gate | up stand in C
+    auto pair_up = [&](KrSvGemm& up, const KrSvGemm& down, const float* gu, int ld, int lo, int F, int kind, float limit, float alpha, const float* row_w = nullptr) {
+        if (kind == KR_SV_ACT_RELU2 || kr_sv_gemm_takes_act(down, s->f32, gu, ld)) return false;       // no up columns; formed in the down projection
+        KrSvGemm p = up;
+        p.glu_out = s->y.p; p.glu_lo = lo; p.glu_f = F; p.glu_kind = kind; p.glu_limit = limit; p.glu_alpha = alpha; p.glu_row_w = row_w;
+        if (!kr_sv_gemm_takes_glu(p, s->f32)) return false;
+        up = p;
+        return true;
     };
     // the residual sum that ends a sublayer (or, in a parallel block, the layer); `next`: the norm of the sublayer that reads the new x, null with
     // hand_on = the row as it is, or nothing when no sublayer follows
@@ -1200,6 +1212,15 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         g.A = mixer_in; g.lda = W; g.W = l.hw.p; g.C = hz; g.ldc = l.n_h; g.M = T; g.N = seq ? l.n_qkv : l.n_h; g.K = W;
         g.bias = d.ff_bias ? (const float*)l.h_bias.p : nullptr;
         if (l.has_lt()) { g.silu_lo = l.off_lt; g.silu_hi = l.off_lt + l.lt_cols(); }
+        // the feed-forward that reads the layer's own rows (dense, or the shared expert): its down projection, and whether the product with gate | up forms the activation
+        KrSvGemm ffd{}; const int ff_f = d.mlp_kind == KR_SERVE_MLP_DENSE ? d.ff : d.mlp_kind == KR_SERVE_MLP_MOE ? d.shared_ff : 0; bool ff_formed = false;
+        const int ff_act = d.mlp_kind == KR_SERVE_MLP_DENSE ? d.dense_act : d.expert_act;
+        const float ff_limit = d.mlp_kind == KR_SERVE_MLP_DENSE ? 0.0f : d.shared_limit, ff_alpha = d.mlp_kind == KR_SERVE_MLP_DENSE ? 1.0f : d.expert_alpha;
+        if (ff_f > 0) {
+            ffd.W = d.mlp_kind == KR_SERVE_MLP_DENSE ? l.down.p : l.sdown.p; ffd.C = (float*)s->ffout.p; ffd.ldc = W; ffd.M = T; ffd.N = W; ffd.K = ff_f;
+            if (d.mlp_kind == KR_SERVE_MLP_DENSE && d.ff_bias) ffd.bias = (const float*)l.down_b.p;
+        }
+        if (!seq && ff_f > 0) ff_formed = pair_up(g, ffd, hz + l.off_gu, l.n_h, l.off_gu, ff_f, ff_act, ff_limit, ff_alpha);
         if (g.N > 0) { Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); }
         const SvLayer& kvl = d.kv_from >= 0 ? s->L[d.kv_from] : run;
         KrSvAttn a{};
@@ -1396,17 +1417,20 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
             if (has_ff && l.n_h > l.off_router) {
                 g = KrSvGemm{}; g.A = s->h.p; g.lda = W; g.W = (const char*)l.hw.p + (size_t)l.off_router * W * s->esz; g.C = hz + l.off_router; g.ldc = l.n_h; g.M = T; g.N = l.n_h - l.off_router; g.K = W;
                 g.bias = d.ff_bias ? (const float*)l.h_bias.p + l.off_router : nullptr;
+                if (ff_f > 0) ff_formed = pair_up(g, ffd, hz + l.off_gu, l.n_h, l.off_gu - l.off_router, ff_f, ff_act, ff_limit, ff_alpha);
                 Timer tm(s, 1); kr_sv_gemm(g, s->f32, st);
             }
         }
         const float *dense = nullptr, *shared = nullptr, *rows = nullptr; const int* pair_pos = nullptr;
         if (d.mlp_kind == KR_SERVE_MLP_DENSE) {
-            g = KrSvGemm{}; g.W = l.down.p; g.C = (float*)s->ffout.p; g.ldc = W; g.M = T; g.N = W; g.K = d.ff;
-            g.bias = d.ff_bias ? (const float*)l.down_b.p : nullptr;
-            down_proj(g, hz + l.off_gu, l.n_h, T, d.ff, d.dense_act, 0.0f, 1.0f);
+            down_proj(ffd, hz + l.off_gu, l.n_h, T, ff_f, ff_act, ff_limit, ff_alpha, nullptr, ff_formed);
             dense = (const float*)s->ffout.p;
         } else if (d.mlp_kind == KR_SERVE_MLP_MOE) {
             const int E = d.experts, top = d.top, F = d.expert_ff, P = T * top;
+            if (ff_f > 0) {              // before the experts: y holds its activation
+                down_proj(ffd, hz + l.off_gu, l.n_h, T, ff_f, ff_act, ff_limit, ff_alpha, nullptr, ff_formed);
+                shared = (const float*)s->ffout.p;
+            }
             int* seg = mi; int* src_row = seg + E + 1; int* row_group = src_row + P; int* pp = row_group + P; int* hist = pp + 2 * P;
             float* row_w = d.expert_in_weight ? (float*)(pp + P) : nullptr;
             {
@@ -1414,19 +1438,14 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
                 kr_sv_router_sort(hz + l.off_router, l.n_h, s->f32 ? 1 : 2, d.router_bias ? (const float*)l.router_b.p : nullptr, d.router_bias, d.router_score, d.group_score, T, E, top, d.groups,
                                   d.keep, d.renorm, (int*)s->ids.p, (float*)s->wts.p, hist, seg, src_row, row_group, pp, row_w, st);
             }
+            KrSvGemm dn{}; dn.W = l.edown.p; dn.w_stride = (size_t)W * F; dn.C = (float*)s->rows.p; dn.ldc = W; dn.M = P; dn.N = W; dn.K = F;
+            dn.seg = seg; dn.row_group = row_group; dn.n_groups = E;
             g = KrSvGemm{}; g.A = s->h.p; g.lda = W; g.W = l.egu.p; g.w_stride = (size_t)2 * F * W; g.C = (float*)s->gu.p; g.ldc = 2 * F; g.M = P; g.N = 2 * F; g.K = W;
             g.a_rows = src_row; g.seg = seg; g.row_group = row_group; g.n_groups = E;
+            const bool formed = pair_up(g, dn, g.C, 2 * F, 0, F, d.expert_act, d.expert_limit, d.expert_alpha, row_w);
             { Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); }
-            g = KrSvGemm{}; g.W = l.edown.p; g.w_stride = (size_t)W * F; g.C = (float*)s->rows.p; g.ldc = W; g.M = P; g.N = W; g.K = F;
-            g.seg = seg; g.row_group = row_group; g.n_groups = E;
-            down_proj(g, (const float*)s->gu.p, 2 * F, P, F, d.expert_act, d.expert_limit, d.expert_alpha, row_w);
+            down_proj(dn, (const float*)s->gu.p, 2 * F, P, F, d.expert_act, d.expert_limit, d.expert_alpha, row_w, formed);
             rows = (const float*)s->rows.p; pair_pos = pp;
-            if (d.shared_ff > 0) {
-                const int SF = d.shared_ff;
-                g = KrSvGemm{}; g.W = l.sdown.p; g.C = (float*)s->ffout.p; g.ldc = W; g.M = T; g.N = W; g.K = SF;
-                down_proj(g, hz + l.off_gu, l.n_h, T, SF, d.expert_act, d.shared_limit, d.expert_alpha);
-                shared = (const float*)s->ffout.p;
-            }
         }
         // x += the layer's sublayers (parallel block) or the feed-forward alone (sequential), and the next layer's input from the same launch
         res_layer = &l; res_run = &run; res_gate_kind = seq ? 2 : l.wkv() ? 1 : 0; res_to_mixer = !side;

@@ -359,6 +359,10 @@ static bool gm_skinny(const KrSvGemm& g) {
     return g.M <= 16 || (g.M <= 32 && g.N <= 2560);
 }
 
+bool kr_sv_gemm_takes_glu(const KrSvGemm& g, bool f32) {
+    return !f32 && g.M > 0 && !gm_skinny(g) && !gm_gemv_rows(g) && kr_sv_gemm_tile_fits(g) && kr_sv_gemm_tile_glu_fits(g);
+}
+
 void kr_sv_gemm(const KrSvGemm& g, bool f32, hipStream_t st) {
     if (g.M <= 0 || g.N <= 0) return;
     const bool grouped = g.seg != nullptr;

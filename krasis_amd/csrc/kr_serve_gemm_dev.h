@@ -61,6 +61,11 @@ __device__ __forceinline__ float gm_act(float g, float u, int kind, float limit,
     // silu on the hardware exponential and reciprocal (one ulp each): every wave of a decode step's down projection forms it again
     return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g)) * u;
 }
+// the same where every element is formed once
+__device__ __forceinline__ float gm_act_once(float g, float u, int kind, float limit, float alpha) {
+    if (kind == KR_SV_ACT_RELU2 || kind == KR_SV_ACT_GELU_TANH || kind == KR_SV_ACT_CLAMPED_SWIGLU) return gm_act(g, u, kind, limit, alpha);
+    return g / (1.0f + expf(-g)) * u;
+}
 template <typename T> __device__ __forceinline__ float gm_round(float v) { return v; }
 template <> __device__ __forceinline__ float gm_round<uint16_t>(float v) { return kr_bf16_to_f32(kr_f32_to_bf16(v)); }
 

@@ -33,6 +33,9 @@ struct KrSvGemm {
     int n_first;                     //   ... and the other groups' matrices have n_first
     // with act_gu: the up columns come from a table instead: element k of problem row r is up_tab[up_rows[r] * up_ld + up_off + k] (storage type)
     const void* up_tab; const int* up_rows; int up_ld, up_off;
+    // only where kr_sv_gemm_takes_glu says so: columns [glu_lo, glu_lo + glu_f) are gates and the glu_f columns behind them their up factors; they do not go to C but, as the
+    // gated activation (of both times glu_row_w[m], if given), to glu_out [M, glu_f] in the storage type, by problem row
+    void* glu_out; int glu_lo, glu_f, glu_kind; float glu_limit, glu_alpha; const float* glu_row_w;
 };
 void kr_sv_gemm(const KrSvGemm& g, bool f32, hipStream_t st);
 // prompt-sized, at most 256 columns, bf16: C (storage type) = gelu_tanh(A W^T) * rows of up_tab, in one launch; W packed by fragments: element (n, k) of [N, K] at
@@ -40,11 +43,14 @@ void kr_sv_gemm(const KrSvGemm& g, bool f32, hipStream_t st);
 bool kr_sv_narrow_act_fits(const KrSvGemm& g, bool f32);
 void kr_sv_narrow_act(const KrSvGemm& g, hipStream_t st);
 bool kr_sv_gemm_takes_act(const KrSvGemm& g, bool f32, const float* gu, int ld);      // true: kr_sv_gemm forms the activation of gu [M, ld] inside its launch (act_gu) for this problem
+// whether kr_sv_gemm forms the activation itself where g's glu fields are set (bf16, prompt-sized)
+bool kr_sv_gemm_takes_glu(const KrSvGemm& g, bool f32);
 // the forms for a bf16 store that kr_sv_gemm chooses from; _fits: shapes and alignment
 bool kr_sv_gemm_skinny_fits(const KrSvGemm& g);
 bool kr_sv_gemm_skinny_acts(const KrSvGemm& g);
 void kr_sv_gemm_skinny(const KrSvGemm& g, hipStream_t st);
 bool kr_sv_gemm_tile_fits(const KrSvGemm& g);
+bool kr_sv_gemm_tile_glu_fits(const KrSvGemm& g);
 void kr_sv_gemm_tile(const KrSvGemm& g, hipStream_t st);
 
 enum { KR_SV_NORM_LAYER = 0, KR_SV_NORM_RMS = 1 };

@@ -12,6 +12,7 @@
 #include <type_traits>
 
 #include "kr_device.h"
+#include "kr_serve_gemm_dev.h"
 #include "kr_serve_ops.h"
 
 namespace {
@@ -1179,20 +1180,9 @@ __global__ void sv_act_kernel(const float* __restrict__ gu, int ld, T* __restric
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (size_t)M * F) return;
     const size_t r = i / F; const int c = (int)(i - r * F);
-    float g = gu[r * ld + c], u = kind == KR_SV_ACT_RELU2 ? 0.0f : up_tab ? sv_ld(up_tab + (size_t)up_rows[r] * up_ld + up_off + c) : gu[r * ld + F + c], v;
+    float g = gu[r * ld + c], u = kind == KR_SV_ACT_RELU2 ? 0.0f : up_tab ? sv_ld(up_tab + (size_t)up_rows[r] * up_ld + up_off + c) : gu[r * ld + F + c];
     if (row_w) { g *= row_w[r]; u *= row_w[r]; }
-    if (kind == KR_SV_ACT_RELU2) {
-        g = fmaxf(g, 0.0f); v = g * g;
-    } else if (kind == KR_SV_ACT_GELU_TANH) {
-        const float in = 0.7978845608028654f * (g + 0.044715f * g * g * g);
-        v = 0.5f * g * (1.0f + tanhf(in)) * u;
-    } else if (kind == KR_SV_ACT_CLAMPED_SWIGLU) {
-        g = fminf(g, limit); u = fminf(fmaxf(u, -limit), limit);
-        v = g / (1.0f + expf(-alpha * g)) * (u + 1.0f);
-    } else {
-        v = g / (1.0f + expf(-g)) * u;
-    }
-    sv_st(y + i, v);
+    sv_st(y + i, gm_act_once(g, u, kind, limit, alpha));
 }
 
 // one workgroup per token: the sublayers' output row is formed in LDS, normed there when the design norms sublayer outputs, gated when the design gates

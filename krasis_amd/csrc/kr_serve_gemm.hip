@@ -1,5 +1,5 @@
 // kr_serve_gemm.hip -- C[M, N] (f32) = A[M, K] x W[N, K]^T for the batched serving step, single matrix or grouped (one matrix per expert, the rows
-// of a group contiguous, optional row gather for A).  The dispatch, and the forms that take every shape; a bf16 store's aligned shapes go to kr_serve_skinny.hip (few
+// of a group contiguous, optional row gather for A).  The dispatch, and the forms that take every shape; aligned shapes go to kr_serve_skinny.hip (bf16, few
 // rows) and kr_serve_tile.hip (prompts).  Here:
 //   * small M (decode steps): one WAVE per output column, the K range over its lanes in 16-byte reads, up to 8 rows of A against one pass over
 //     the weight row -- bound by the weight stream;
@@ -360,7 +360,7 @@ static bool gm_skinny(const KrSvGemm& g) {
 }
 
 bool kr_sv_gemm_takes_glu(const KrSvGemm& g, bool f32) {
-    return !f32 && g.M > 0 && !gm_skinny(g) && !gm_gemv_rows(g) && kr_sv_gemm_tile_fits(g) && kr_sv_gemm_tile_glu_fits(g);
+    return !f32 && g.M > 0 && !gm_skinny(g) && !gm_gemv_rows(g) && kr_sv_gemm_tile_fits(g, false) && kr_sv_gemm_tile_glu_fits(g);
 }
 
 void kr_sv_gemm(const KrSvGemm& g, bool f32, hipStream_t st) {
@@ -388,12 +388,12 @@ void kr_sv_gemm(const KrSvGemm& g, bool f32, hipStream_t st) {
 #undef GM_V
         return;
     }
+    if (kr_sv_gemm_tile_fits(g, f32)) { kr_sv_gemm_tile(g, f32, st); return; }
     if (f32) {
         const int tiles = grouped ? (g.M + 63) / 64 + g.n_groups : (g.M + 63) / 64;
         hipLaunchKernelGGL(sv_gemm_f32_kernel, dim3((g.N + 63) / 64, tiles), dim3(256), 0, st, g);
         return;
     }
-    if (kr_sv_gemm_tile_fits(g)) { kr_sv_gemm_tile(g, st); return; }
     // shapes whose rows are not whole 64-k slots of 16-byte pieces.  Grouped problems have few rows per expert: the 64-row tile wastes less of the matrix cores, and
     // so do narrow problems: with 128-row tiles they would leave most compute units idle
     const bool small = grouped ? (g.M / (g.n_groups > 0 ? g.n_groups : 1) < 96) : g.M <= 64 || (long)((g.N + 127) / 128) * ((g.M + 127) / 128) < 128;

@@ -49,9 +49,9 @@ bool kr_sv_gemm_takes_glu(const KrSvGemm& g, bool f32);
 bool kr_sv_gemm_skinny_fits(const KrSvGemm& g);
 bool kr_sv_gemm_skinny_acts(const KrSvGemm& g);
 void kr_sv_gemm_skinny(const KrSvGemm& g, hipStream_t st);
-bool kr_sv_gemm_tile_fits(const KrSvGemm& g);
+bool kr_sv_gemm_tile_fits(const KrSvGemm& g, bool f32);
 bool kr_sv_gemm_tile_glu_fits(const KrSvGemm& g);
-void kr_sv_gemm_tile(const KrSvGemm& g, hipStream_t st);
+void kr_sv_gemm_tile(const KrSvGemm& g, bool f32, hipStream_t st);
 
 enum { KR_SV_NORM_LAYER = 0, KR_SV_NORM_RMS = 1 };
 enum { KR_SV_ACT_GELU_TANH = 0, KR_SV_ACT_CLAMPED_SWIGLU = 1, KR_SV_ACT_SILU = 2, KR_SV_ACT_RELU2 = 3 /* un-gated: relu(x)^2 of the first F columns; no up columns */ };

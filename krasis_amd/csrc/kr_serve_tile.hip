@@ -1,4 +1,5 @@
-// kr_serve_tile.hip -- C[M, N] = A[M, K] x W[N, K]^T for prompt-sized problems of a bf16 store, single matrix or one matrix per expert, on v_mfma_f32_32x32x16_bf16.
+// kr_serve_tile.hip -- C[M, N] = A[M, K] x W[N, K]^T for prompt-sized problems, single matrix or one matrix per expert: a bf16 store's on v_mfma_f32_32x32x16_bf16, an f32
+// store's on v_mfma_f32_32x32x2_f32.
 //
 // Bound: the matrix cores (about 1350 TFLOP/s is what a large library product reaches here; nominal 2500).  Both operands travel from memory to LDS by
 // global_load_lds_dwordx4 into a ring of slots of 64 k (no staging registers; whole cache lines), ONE barrier per slot, the next slot requested right behind it, fragments
@@ -15,12 +16,12 @@
 #include "kr_serve_gemm_dev.h"
 
 namespace {
-constexpr int TL_BK = 64;                                      // k of a slot: 128-byte rows, whole cache lines (32 k would fetch every line twice)
+constexpr int TL_ROW = 128;                                    // bytes of a slot's row, whole cache lines (rows of 64 bytes fetch every line twice): 64 k in bf16, 32 in f32
 
 __device__ __forceinline__ uint32_t tl_lds_addr(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p; }
 // 64 lanes x 16 bytes from the lane's own address to lds_dst (wave-uniform) + 16 lane.  M0 is the compiler's register: saved and restored inside.  The compiler
 // does not count this request; the waits below do.
-__device__ __forceinline__ void tl_dma16(uint32_t lds_dst, const uint16_t* src) {
+__device__ __forceinline__ void tl_dma16(uint32_t lds_dst, const void* src) {
     unsigned keep;
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(src), "s"(lds_dst) : "memory");
 }
@@ -30,12 +31,13 @@ template <int N> __device__ __forceinline__ void tl_wait_barrier() { asm volatil
 // GLU: columns [glu_lo, glu_lo + 2 glu_f) leave as the gated activation.  Their tiles come behind those of the other columns (the column numbers of those close the gap): half a
 // tile of gates and the up columns that belong to them, laid out so that a wave holds both factors of its elements.  The f32 pair is not written and read again and
 // the activation's launch is gone: 24576 rows of 2 x 768 on 64 experts, product and activation, 242 + 55 -> 252 us; a 4096-token prompt of four layers 4.06 -> 3.80 ms.
-template <int BM, int BN, int WM, int WN, int DEPTH, int WPS, bool GLU>  // WM x WN waves; WPS: waves per SIMD the register budget is for
+template <typename T, int BM, int BN, int WM, int WN, int DEPTH, int WPS, bool GLU>  // WM x WN waves; WPS: waves per SIMD the register budget is for
 __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGemm g) {
     constexpr int MB = BM / (32 * WM), NB = BN / (32 * WN);    // 32 x 32 blocks of a wave
     constexpr int RA = BM / 8, RW = (BM + BN) / (8 * WM * WN); // requests of 8 rows per slot: A's; per wave
-    constexpr int SLOT = (BM + BN) * TL_BK;                    // elements
-    extern __shared__ __attribute__((aligned(1024))) uint16_t ring[];
+    constexpr int BK = TL_ROW / (int)sizeof(T), CH = 16 / (int)sizeof(T), SLOT = (BM + BN) * BK;     // k of a slot, elements of a chunk and of a slot
+    extern __shared__ __attribute__((aligned(1024))) uint8_t ring_[];
+    T* ring = reinterpret_cast<T*>(ring_);
     int bx = blockIdx.x, by = blockIdx.y;
     // Workgroups go round the eight XCDs, each with its own L2.  With a column count of a multiple of eight an XCD sees the same columns of W for all rows; otherwise,
     // and with one matrix per expert, it is given whole pairs of row tiles: their rows stay in its L2, the pair shares the columns of W.
@@ -52,20 +54,20 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
     const int n0 = GLU ? (pairs ? (bx - plain_tiles) * (BN / 2) : bx * BN) : bx * BN, N = GLU ? (pairs ? g.glu_f : plain) : gm_cols(g, group);
     if (n0 >= N) return;
     auto column = [&](int n) { return GLU && n >= g.glu_lo ? n + 2 * g.glu_f : n; };         // of C and row of W, of a column outside the pairs
-    const uint16_t* A = (const uint16_t*)g.A;
-    const uint16_t* W = (const uint16_t*)g.W + (size_t)group * g.w_stride;
+    const T* A = (const T*)g.A;
+    const T* W = (const T*)g.W + (size_t)group * g.w_stride;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5, wr = wave / WN, wc = wave % WN;
-    const uint16_t* src[RW];
+    const T* src[RW];
 #pragma unroll
     for (int i = 0; i < RW; i++) {
         const int q = wave * RW + i;                           // request: RA of A's rows, then W's
         const int row = (q < RA ? q : q - RA) * 8 + (lane >> 3), ch = (lane & 7) ^ ((row >> 1) & 7);
-        if (q < RA) { const int m = min(m0 + row, mend - 1); src[i] = A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda + ch * 8; }
+        if (q < RA) { const int m = min(m0 + row, mend - 1); src[i] = A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda + ch * CH; }
         else if (pairs) {                                      // a wave's columns: its gates, then their up factors
             constexpr int WC = BN / WN;
             const int j = n0 + row / WC * (WC / 2) + row % (WC / 2), up = row % WC >= WC / 2;
-            src[i] = W + (size_t)(g.glu_lo + up * g.glu_f + min(j, N - 1)) * g.K + ch * 8;
-        } else src[i] = W + (size_t)column(min(n0 + row, N - 1)) * g.K + ch * 8;
+            src[i] = W + (size_t)(g.glu_lo + up * g.glu_f + min(j, N - 1)) * g.K + ch * CH;
+        } else src[i] = W + (size_t)column(min(n0 + row, N - 1)) * g.K + ch * CH;
     }
     const uint32_t base = __builtin_amdgcn_readfirstlane(tl_lds_addr(ring)) + (uint32_t)(wave * RW) * 1024u;
     gv16f acc[MB][NB];
@@ -75,41 +77,52 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
         for (int b = 0; b < NB; b++)
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[a][b][i] = 0.0f;
-    const int steps = g.K / TL_BK;
+    const int steps = g.K / BK;
     auto request = [&](int slot) {
 #pragma unroll
-        for (int i = 0; i < RW; i++) { tl_dma16(base + (uint32_t)slot * (SLOT * 2) + i * 1024u, src[i]); src[i] += TL_BK; }
+        for (int i = 0; i < RW; i++) { tl_dma16(base + (uint32_t)slot * (uint32_t)(SLOT * sizeof(T)) + i * 1024u, src[i]); src[i] += BK; }
     };
 #pragma unroll
     for (int d = 0; d < DEPTH - 1; d++) if (d < steps) request(d);
     // fragment of rows [32 blk, +32), k step ks of the slot: chunk ks + 4 h of row r
     const int sw = (r >> 1) & 7;
-    const uint16_t* af0 = ring + (wr * (BM / WM) + r) * TL_BK;
-    const uint16_t* bf0 = ring + (BM + wc * (BN / WN) + r) * TL_BK;
+    const T* af0 = ring + (wr * (BM / WM) + r) * BK;
+    const T* bf0 = ring + (BM + wc * (BN / WN) + r) * BK;
     int slot = 0;
     for (int s = 0; s < steps; s++) {
         // slot s has landed when only the DEPTH - 2 younger ones are outstanding (none at the end)
         if (DEPTH == 2 || s + 1 >= steps) tl_wait_barrier<0>(); else tl_wait_barrier<(DEPTH - 2) * RW>();
         if (s + DEPTH - 1 < steps) request(slot == 0 ? DEPTH - 1 : slot - 1);      // the slot read in the previous step: every wave is past it
-        const uint16_t* ab = af0 + slot * SLOT;
-        const uint16_t* bb = bf0 + slot * SLOT;
-        gb8 af[2][MB], bf[2][NB];                              // fragments of two k steps: one is read while the other is multiplied
+        const T* ab = af0 + slot * SLOT;
+        const T* bb = bf0 + slot * SLOT;
+        gu4 af[2][MB], bf[2][NB];                              // fragments of two k steps: one is read while the other is multiplied
         auto read = [&](int ks) {
-            const int ch = ((ks + 4 * h) ^ sw) * 8;            // the halves of the wave take k halves of the slot (any order serves, both operands alike)
+            const int ch = ((ks + 4 * h) ^ sw) * CH;           // the halves of the wave take k halves of the slot (any order serves, both operands alike)
 #pragma unroll
-            for (int a = 0; a < MB; a++) af[ks & 1][a] = __builtin_bit_cast(gb8, *reinterpret_cast<const gu4*>(ab + a * 32 * TL_BK + ch));
+            for (int a = 0; a < MB; a++) af[ks & 1][a] = *reinterpret_cast<const gu4*>(ab + a * 32 * BK + ch);
 #pragma unroll
-            for (int b = 0; b < NB; b++) bf[ks & 1][b] = __builtin_bit_cast(gb8, *reinterpret_cast<const gu4*>(bb + b * 32 * TL_BK + ch));
+            for (int b = 0; b < NB; b++) bf[ks & 1][b] = *reinterpret_cast<const gu4*>(bb + b * 32 * BK + ch);
         };
         read(0);
 #pragma unroll
-        for (int ks = 0; ks < TL_BK / 16; ks++) {
-            if (ks + 1 < TL_BK / 16) read(ks + 1);
+        for (int ks = 0; ks < 4; ks++) {
+            if (ks + 1 < 4) read(ks + 1);
             __builtin_amdgcn_sched_barrier(0);
+            if constexpr (sizeof(T) == 2) {
 #pragma unroll
-            for (int a = 0; a < MB; a++)
+                for (int a = 0; a < MB; a++)
 #pragma unroll
-                for (int b = 0; b < NB; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks & 1][a], bf[ks & 1][b], acc[a][b], 0, 0, 0);
+                    for (int b = 0; b < NB; b++)
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(gb8, af[ks & 1][a]), __builtin_bit_cast(gb8, bf[ks & 1][b]), acc[a][b], 0, 0, 0);
+            } else {                                           // a chunk is four steps of 2 k, one per half
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int a = 0; a < MB; a++)
+#pragma unroll
+                        for (int b = 0; b < NB; b++)
+                            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(af[ks & 1][a][e]), __uint_as_float(bf[ks & 1][b][e]), acc[a][b], 0, 0, 0);
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
         slot = slot == DEPTH - 1 ? 0 : slot + 1;
@@ -118,7 +131,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
         if (pairs) {
             tl_wait_barrier<0>();
             constexpr int LD = 36;                             // floats of a staged row: 16-byte pieces
-            float* pg = reinterpret_cast<float*>(ring) + wave * (2 * 32 * LD);
+            float* pg = reinterpret_cast<float*>(ring_) + wave * (2 * 32 * LD);
             float* pu = pg + 32 * LD;
             uint16_t* out = (uint16_t*)g.glu_out;
             const bool wide = g.glu_f % 8 == 0;
@@ -190,7 +203,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
     }
     // bias, gates, row maps: one 32 x 32 block at a time through a wave's own piece of LDS, so that the element epilogue is a loop and not 16 MB NB copies of itself
     tl_wait_barrier<0>();
-    float* blk = reinterpret_cast<float*>(ring) + wave * (32 * 33);
+    float* blk = reinterpret_cast<float*>(ring_) + wave * (32 * 33);
 #pragma unroll
     for (int a = 0; a < MB; a++)
 #pragma unroll
@@ -201,26 +214,27 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
             const int n = n0 + wc * (BN / WN) + b * 32 + r, mb = m0 + wr * (BM / WM) + a * 32;
 #pragma unroll 1
             for (int i = h; i < 32; i += 2)
-                if (n < N && mb + i < mend) gm_store<true>(g, mb + i, column(n), blk[i * 33 + r]);
+                if (n < N && mb + i < mend) gm_store<sizeof(T) == 2>(g, mb + i, column(n), blk[i * 33 + r]);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
 }
 
-template <int BM, int BN, int WM, int WN, int DEPTH, int WPS, bool GLU>
+template <typename T, int BM, int BN, int WM, int WN, int DEPTH, int WPS, bool GLU>
 void tl_launch(const KrSvGemm& g, hipStream_t st) {
-    constexpr int LDS = DEPTH * (BM + BN) * TL_BK * 2;
+    constexpr int LDS = DEPTH * (BM + BN) * TL_ROW;
     static_assert(LDS <= 160 * 1024, "LDS of a compute unit");
-    static_assert(!GLU || (BN / WN % 64 == 0 && WM * WN * 2 * 32 * 36 * 4 <= LDS), "a wave holds both factors, and stages them");
+    static_assert(!GLU || (sizeof(T) == 2 && BN / WN % 64 == 0 && WM * WN * 2 * 32 * 36 * 4 <= LDS), "a wave holds both factors, and stages them");
     const int cols = GLU ? (g.N - 2 * g.glu_f + BN - 1) / BN + (g.glu_f + BN / 2 - 1) / (BN / 2) : (g.N + BN - 1) / BN;
     const dim3 grid(cols, (g.M + BM - 1) / BM + (g.seg ? g.n_groups : 0));
-    (void)hipFuncSetAttribute((const void*)sv_tile_kernel<BM, BN, WM, WN, DEPTH, WPS, GLU>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-    hipLaunchKernelGGL((sv_tile_kernel<BM, BN, WM, WN, DEPTH, WPS, GLU>), grid, dim3(64 * WM * WN), LDS, st, g);
+    (void)hipFuncSetAttribute((const void*)sv_tile_kernel<T, BM, BN, WM, WN, DEPTH, WPS, GLU>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    hipLaunchKernelGGL((sv_tile_kernel<T, BM, BN, WM, WN, DEPTH, WPS, GLU>), grid, dim3(64 * WM * WN), LDS, st, g);
 }
 }  // namespace
 
 // whole slots of 16-byte chunks
-bool kr_sv_gemm_tile_fits(const KrSvGemm& g) {
-    return g.K % TL_BK == 0 && g.lda % 8 == 0 && (((uintptr_t)g.A | (uintptr_t)g.W) % 16 == 0) && g.w_stride % 8 == 0;
+bool kr_sv_gemm_tile_fits(const KrSvGemm& g, bool f32) {
+    const int row = TL_ROW / (f32 ? 4 : 2), chunk = 16 / (f32 ? 4 : 2);
+    return g.K % row == 0 && g.lda % chunk == 0 && (((uintptr_t)g.A | (uintptr_t)g.W) % 16 == 0) && g.w_stride % chunk == 0;
 }
 
 // Which tile: the time of a slot step times how often the chip has to be filled, as measured at K = 2048 - 8192 (us per step of 64 k):
@@ -229,12 +243,12 @@ bool kr_sv_gemm_tile_fits(const KrSvGemm& g) {
 //   64 x 64, three per unit: 0.4 + 0.7 per 768 tiles: few rows, where the small tile spreads the weight stream over more units
 // (us, 256 / 128 / 64: 3300 x 4096 x 8192 267 / 315 / 391; 4096 x 2048 x 2048 61 / 42 / 57; 500 x 2048 x 2048 53 / 23 / 14.)  Tiles of a grouped problem: its rows spread
 // evenly, half a tile more per group.
+static double tl_tiles(const KrSvGemm& g, int b) {
+    const double cols = (g.N + b - 1) / b;
+    return cols * (g.seg ? g.n_groups * std::max(1.0, (double)g.M / g.n_groups / b + 0.5) : (double)((g.M + b - 1) / b));
+}
 static int tl_kind(const KrSvGemm& g) {
-    auto tiles = [&](int b) {
-        const double cols = (g.N + b - 1) / b;
-        return cols * (g.seg ? g.n_groups * std::max(1.0, (double)g.M / g.n_groups / b + 0.5) : (double)((g.M + b - 1) / b));
-    };
-    const double t256 = 2.1 * std::ceil(tiles(256) / 256), t128 = std::max(0.72, 1.5 * tiles(128) / 512), t64 = 0.4 + 0.7 * tiles(64) / 768;
+    const double t256 = 2.1 * std::ceil(tl_tiles(g, 256) / 256), t128 = std::max(0.72, 1.5 * tl_tiles(g, 128) / 512), t64 = 0.4 + 0.7 * tl_tiles(g, 64) / 768;
     return t256 <= t128 && t256 <= t64 ? 256 : t128 <= t64 ? 128 : 64;
 }
 
@@ -244,10 +258,17 @@ bool kr_sv_gemm_tile_glu_fits(const KrSvGemm& g) {
            (g.silu_hi <= g.silu_lo || g.silu_hi <= g.glu_lo || g.silu_lo >= g.glu_lo + 2 * g.glu_f) && tl_kind(g) != 64;
 }
 
-void kr_sv_gemm_tile(const KrSvGemm& g, hipStream_t st) {
+// f32 (500 tokens, 64 experts of 2 x 768 x 2048: 410 us a product on average with scalar loads and vector FMAs -> 131): the matrix instruction takes 16 times as long for the same product (32x32x2, every factor and sum in f32), so nothing but its own count matters: 128 x 128 where that fills
+// the chip without more padding than 64 x 64.
+void kr_sv_gemm_tile(const KrSvGemm& g, bool f32, hipStream_t st) {
+    if (f32) {
+        if (4.0 * std::ceil(tl_tiles(g, 128) / 256) < tl_tiles(g, 64) / 256) tl_launch<float, 128, 128, 2, 2, 2, 2, false>(g, st);
+        else tl_launch<float, 64, 64, 2, 2, 3, 3, false>(g, st);
+        return;
+    }
     switch (tl_kind(g)) {
-        case 256: if (g.glu_out) tl_launch<256, 256, 2, 4, 2, 2, true>(g, st); else tl_launch<256, 256, 2, 4, 2, 2, false>(g, st); break;
-        case 128: if (g.glu_out) tl_launch<128, 128, 2, 2, 2, 2, true>(g, st); else tl_launch<128, 128, 2, 2, 2, 2, false>(g, st); break;
-        default: tl_launch<64, 64, 2, 2, 3, 3, false>(g, st); break;
+        case 256: if (g.glu_out) tl_launch<uint16_t, 256, 256, 2, 4, 2, 2, true>(g, st); else tl_launch<uint16_t, 256, 256, 2, 4, 2, 2, false>(g, st); break;
+        case 128: if (g.glu_out) tl_launch<uint16_t, 128, 128, 2, 2, 2, 2, true>(g, st); else tl_launch<uint16_t, 128, 128, 2, 2, 2, 2, false>(g, st); break;
+        default: tl_launch<uint16_t, 64, 64, 2, 2, 3, 3, false>(g, st); break;
     }
 }

@@ -66,3 +66,29 @@ def test_activation_from_the_product(mlp, n):
     # the input row, the two factors' sums and the activation: three independent roundings of 2^-9 each, which the products pass on at their own scale; a lost factor of
     # 260 would alter its rows by 1 / sqrt(260) = 6e-2
     assert np.sqrt((d ** 2).mean(-1)).max() / np.sqrt((ref ** 2).mean()) < 2e-2
+
+
+@pytest.mark.parametrize("want,vocab,width", [(17, 129, 32), (63, 65, 96), (65, 64, 2048), (130, 257, 64), (1025, 4100, 64), (1024, 4096, 160), (70, 100, 36)])
+def test_vocabulary_projection_sizes_f32(want, vocab, width):
+    # 64- and 128-row tiles with ragged edges, one slot and many; a width of 16-byte pieces that is no whole slot
+    cfg = stream_model(width, vocab); W = O.random_weights(cfg, 17); toks = tokens(cfg, want, 18)
+    eng = engine(cfg, W, max_tokens=2048)
+    eng.store.set_capture(True)
+    logits, amax = eng.step([("a", toks, list(range(want)))])
+    h = O.layer_norm(eng.store.read_capture(want)[-1].astype(np.float64), W["final.norm"].astype(np.float64), W["final.norm.b"].astype(np.float64), 1e-5)
+    head = W["head"].astype(np.float64)
+    # sums of `width` products in f32, the row itself within a few units of its norm
+    assert np.all(np.abs(logits - h @ head.T) <= (4.0 + np.sqrt(width)) * 2.0 ** -24 * 2.0 * (np.abs(h) @ np.abs(head.T)))
+    assert np.array_equal(amax, logits.argmax(-1))
+
+
+@pytest.mark.parametrize("n", [9, 40, 130, 700])
+def test_expert_products_sizes_f32(n):
+    cfg = O.make_config(width=64, vocab=61, eps=1e-5, layers=[{"type": "attention", "mixer": O.attn(4, 2, 32, 32, 7, 16, scale=0.2), "mlp": O.moe(5, 5, 1, 1, 96, 2.0, 64, 2.0)}])
+    W = O.random_weights(cfg, 19); toks = tokens(cfg, n, 20)
+    ref = O.forward(cfg, W, toks)[1][0]
+    eng = engine(cfg, W)
+    eng.store.set_capture(True)
+    eng.step([("a", toks, [n - 1])])
+    d = eng.store.read_capture(n)[0] - ref
+    assert np.sqrt((d ** 2).mean(-1)).max() / np.sqrt((ref ** 2).mean()) < 2e-5      # f32 sums of at most 128 products, a few in a row

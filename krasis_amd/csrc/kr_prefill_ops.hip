@@ -213,110 +213,131 @@ __global__ void kr_pfm_la_conv_state_kernel(const KrPfmLaArgs a, int C) {
     for (int j = 0; j < 4; j++) cs[j] = n[j];
 }
 
-// ---- gated delta rule over the chunk (decode.rs:1293): one thread per state column, the column lives in registers ------------
-// grid nv, dv threads.  Per token: kv = chain_i fma(S[i]*e^g, k[i]); delta = (v - kv)*beta; S[i] = fma(k[i], delta, S[i]*e^g); o = chain_i fma(S[i], q[i]).
-// The two DK-long fma chains per token are inherent to the reference order, and a dependent v_fmac issues only every ~15 cycles on this part: run one after the other they
-// cost 2 x DK x 15 cycles per token (1.8 us at DK = 128: the round-5 form).  Round 6: the OUTPUT chain of token t and the kv chain of token t + 1 are independent once
-// S(t)[i] exists, so they advance together, element by element -- update S[i] with delta_t, step o_t, decay S[i] by e^g(t+1), step kv_(t+1): four instructions per element,
-// two chains in each other's latency shadow; every value is produced by the same operation in the same order as before (bit-identical).  Behind the last token runs a
-// phantom one with e^g = 1 (S * 1.0f is S) whose chain nobody reads.  The rows (k, q, v) and the two gate scalars of a token reach an LDS ring of RS slots by LDS-DMA
-// (global_load_lds_dword: lane i's word lands at M0 + 4 i), requested three tokens ahead: no staging registers, one loop body; the state slice is addressed through a
-// buffer descriptor (scalar row offsets) so that no per-row 64-bit addresses stay live across the loop.
-// (Measured earlier and slower: LDS-staged token blocks; one packed fma advancing both chains on a {S*e^g, S} register pair -- 2 x DK registers; the same interleave with
-// the rows prefetched into rotating register sets -- three copies of the loop, 328 registers.)
-__device__ __forceinline__ void pfm_dma4(uint32_t lds_dst, const void* gptr) {      // this lane's 4 bytes at gptr -> lds_dst + 4 * lane; not counted by the compiler's waits
-    unsigned keep;
-    lds_dst = __builtin_amdgcn_readfirstlane(lds_dst);
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 2\n\tglobal_load_lds_dword %2, off\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "s"(lds_dst), "v"(gptr) : "memory");
-}
+// ---- gated delta rule over the chunk (decode.rs:1293): eight lanes per state column -----------------------------------------------
+// Per token: S[i] *= e^g; kv = chain_i fma(S[i], k[i]); delta = (v - kv) * beta; S[i] = fma(k[i], delta, S[i]); o = chain_i fma(S[i], q[i]).  The order of both chains is the
+// reference's, so DK dependent steps of about four cycles are the least a token can take (0.21 us at DK = 128); everything else has to get out of their way:
+//   * a column's DK state values lie over eight neighbouring lanes (lane = 8 column + part, part p holds i in [p DK / 8, ...)): the update costs DK / 8 steps instead of DK, and
+//     a lane needs DK / 8 values of a k or q row (four 16-byte LDS reads) instead of all of them.  The chain walks through the parts: in phase p every lane adds its own
+//     products to what its left neighbour handed over (one DPP move), and part p's value is the column's.  The other lanes' sums are not used;
+//   * the output chain has its own waves: they form the same S from the deltas the state waves leave in LDS (the same operations in the same order: the same bits), one
+//     block of PFR_TB tokens behind.  A workgroup is two state waves and two output waves of eight columns each; the rows of a block come to LDS through registers, requested a
+//     block ahead, one barrier per block (blocks of 8 tokens instead of 16: 390 us).
+// 777 tokens, 32 heads of 128 x 128: 1167 -> 371 us (the form before: one thread per column, the two chains of a column interleaved; per token it issued 512 fused
+// multiply-adds and 96 broadcast reads of LDS, 13 cycles each, from the one wave that held the columns).
+#define PFR_TB 16
+#define PFR_DPP(x, ctrl) __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), (ctrl), 0xF, 0xF, true))
 template <int DK>
 __global__ void __launch_bounds__(256) kr_pfm_la_recur_kernel(float* __restrict__ state, const float* __restrict__ q, const float* __restrict__ k,
                                                              const float* __restrict__ v, const float* __restrict__ gexp, const float* __restrict__ beta,
                                                              float* __restrict__ out, int nv, int dv, int C) {
-    constexpr int RS = 5, ROW = 256;                 // ring slots; floats per row region (dv <= 256)
-    constexpr int SLOT = 3 * ROW + 128;              // floats per slot: k row, q row, v row, e^g at [3 ROW], beta at [3 ROW + 1] (wave 0's other lanes land behind them), a 64-word dump at [3 ROW + 64]
-    __shared__ __attribute__((aligned(16))) float ring[RS][SLOT];
-    const int h = blockIdx.x, j = threadIdx.x, lane = j & 63, wv = __builtin_amdgcn_readfirstlane(j >> 6), nvdk = nv * DK, nvdv = nv * dv;
-    float S[DK];
-    const __amdgpu_buffer_rsrc_t srd = __builtin_amdgcn_make_buffer_rsrc(state + (size_t)h * DK * dv, 0, DK * dv * 4, 0x00020000);
+    constexpr int U = DK / 8, PS = U + 4, ROW = 8 * PS, NV = DK * PFR_TB / 256;      // values per lane; floats from part to part (no two parts on the same banks) and per row; words of a thread per block
+    __shared__ __attribute__((aligned(16))) float ks[3][PFR_TB][ROW], qs[2][PFR_TB][ROW];
+    __shared__ float vs[3][PFR_TB][16], ds[2][PFR_TB][16], gs[3][2][PFR_TB];
+    const int h = blockIdx.x, j0 = blockIdx.y * 16, tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int part = lane & 7, cg = (wv >> 1) * 8 + (lane >> 3), j = j0 + cg;        // this lane's column, and its number in the workgroup
+    const bool live = j < dv, outs = wv & 1;
+    const int nvdk = nv * DK, nvdv = nv * dv, nb = (C + PFR_TB - 1) / PFR_TB;
+    float S[U];
+    float* sp = state + (size_t)h * DK * dv + (size_t)part * U * dv + (live ? j : 0);
 #pragma unroll
-    for (int i = 0; i < DK; i++) S[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srd, j * 4, i * dv * 4, 0));
-    const uint32_t ring0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)&ring[0][0];
-    const bool kq_wave = wv * 64 < DK;                                   // wave-uniform: this wave's columns have k / q words
-    const int jk = kq_wave ? j : lane;                                    // other waves fetch (harmless) words into the slot's spare area: every wave issues 5 DMAs per token
-    auto request = [&](int tt, int slot) {           // token tt (clamped: a phantom token behind the chunk re-reads the last one; its gates are forced below)
-        const int tc = tt < C ? tt : C - 1;
-        const uint32_t base = ring0 + (uint32_t)slot * (SLOT * 4), dump = base + (3 * ROW + 64) * 4;
-        pfm_dma4(kq_wave ? base + wv * 256 : dump, k + (size_t)tc * nvdk + (size_t)h * DK + jk);
-        pfm_dma4(kq_wave ? base + ROW * 4 + wv * 256 : dump, q + (size_t)tc * nvdk + (size_t)h * DK + jk);
-        pfm_dma4(base + 2 * ROW * 4 + wv * 256, v + (size_t)tc * nvdv + (size_t)h * dv + j);
-        pfm_dma4(wv == 0 ? base + 3 * ROW * 4 : dump, (lane == 0 ? gexp : beta) + (size_t)tc * nv + h);      // wave 0: lane 0 -> e^g, lane 1 -> beta (lanes 2 .. 63 land behind them, unread)
-        pfm_dma4(dump, beta + (size_t)tc * nv + h);                                                          // filler: every wave issues exactly 5 requests per token (the wait below counts them)
+    for (int u = 0; u < U; u++) S[u] = sp[(size_t)u * dv];
+    // words of a block on its way (tokens behind the chunk repeat the last one): k, v and the gates of block b, which its state waves read next, and q of the block before
+    float rk[NV], rq[NV], rv, rg;
+    const int et = tid / DK, ei = tid % DK, eo = ei / U * PS + ei % U;
+    auto fetch_q = [&](int b) {
+#pragma unroll
+        for (int n = 0; n < NV; n++) rq[n] = q[(size_t)min(b * PFR_TB + et + n * (256 / DK), C - 1) * nvdk + (size_t)h * DK + ei];
     };
-    request(0, 0); request(1, 1); request(2, 2);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    auto fetch = [&](int b) {
+        const int t0 = b * PFR_TB, c = j0 + (tid & 15);
+#pragma unroll
+        for (int n = 0; n < NV; n++) rk[n] = k[(size_t)min(t0 + et + n * (256 / DK), C - 1) * nvdk + (size_t)h * DK + ei];
+        rv = c < dv ? v[(size_t)min(t0 + (tid >> 4), C - 1) * nvdv + (size_t)h * dv + c] : 0.0f;
+        rg = tid < 2 * PFR_TB ? (tid < PFR_TB ? gexp : beta)[(size_t)min(t0 + tid % PFR_TB, C - 1) * nv + h] : 0.0f;
+    };
+    auto publish_q = [&](int buf) {
+#pragma unroll
+        for (int n = 0; n < NV; n++) qs[buf][et + n * (256 / DK)][eo] = rq[n];
+    };
+    auto publish = [&](int buf) {
+#pragma unroll
+        for (int n = 0; n < NV; n++) ks[buf][et + n * (256 / DK)][eo] = rk[n];
+        vs[buf][tid >> 4][tid & 15] = rv;
+        if (tid < 2 * PFR_TB) gs[buf][tid / PFR_TB][tid % PFR_TB] = rg;
+    };
+    struct Row { float x[U]; };
+    auto row = [&](const float* r) {
+        Row w;
+#pragma unroll
+        for (int u = 0; u < U / 4; u++) { const float4 f = *reinterpret_cast<const float4*>(r + part * PS + 4 * u); w.x[4 * u] = f.x; w.x[4 * u + 1] = f.y; w.x[4 * u + 2] = f.z; w.x[4 * u + 3] = f.w; }
+        return w;
+    };
+    auto chain = [&](const Row& w) {                 // part 7's lanes return the column's sum over i = 0 .. DK - 1
+        float s = 0.0f;
+#pragma unroll
+        for (int p = 0; p < 8; p++) {
+            if (p > 0) s = PFR_DPP(s, 0x111);        // row_shr:1
+#pragma unroll
+            for (int u = 0; u < U; u++) s = __builtin_fmaf(S[u], w.x[u], s);
+        }
+        return s;
+    };
+    fetch(0); publish(0);
     __syncthreads();
-    // prologue: decay + kv chain of token 0 alone
-    float delta;
-    {
-        const float4* k4 = reinterpret_cast<const float4*>(&ring[0][0]);
-        const float ge0 = ring[0][3 * ROW], bt0 = ring[0][3 * ROW + 1], vj0 = ring[0][2 * ROW + j];
-        float kv = 0.0f;
+    int buf = 0;
+    for (int b = 0; b <= nb; b++) {
+        const int nxt = buf == 2 ? 0 : buf + 1, prv = buf == 0 ? 2 : buf - 1;
+        if (b + 1 < nb) fetch(b + 1);
+        if (b < nb) fetch_q(b);
+        if (!outs && b < nb) {                       // block b: the state and the deltas
+            const int n = min(PFR_TB, C - b * PFR_TB);
+            float ge = gs[buf][0][0], bt = gs[buf][1][0], vj = vs[buf][0][cg];
+            auto token = [&](int s, const Row& kk, Row& kn) {                    // what the next token needs leaves LDS while this one's chain runs
+                const int s1 = min(s + 1, PFR_TB - 1);
+                kn = row(ks[buf][s1]);
+                const float ge1 = gs[buf][0][s1], bt1 = gs[buf][1][s1], vj1 = vs[buf][s1][cg];
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int u = 0; u < DK / 4; u++) {
-            const float4 kk = k4[u];
-            float* Sb = S + 4 * u;
-            Sb[0] = Sb[0] * ge0; kv = __builtin_fmaf(Sb[0], kk.x, kv);
-            Sb[1] = Sb[1] * ge0; kv = __builtin_fmaf(Sb[1], kk.y, kv);
-            Sb[2] = Sb[2] * ge0; kv = __builtin_fmaf(Sb[2], kk.z, kv);
-            Sb[3] = Sb[3] * ge0; kv = __builtin_fmaf(Sb[3], kk.w, kv);
+                for (int u = 0; u < U; u++) S[u] = S[u] * ge;
+                const float kv = chain(kk);
+                const float lo = PFR_DPP(PFR_DPP(kv, 0x141), 0x00), hi = PFR_DPP(kv, 0xFF);      // part 7's: mirrored into parts 0 .. 3, spread over its own four
+                const float delta = (vj - (part < 4 ? lo : hi)) * bt;
+                if (part == 0) ds[b & 1][s][cg] = delta;
+#pragma unroll
+                for (int u = 0; u < U; u++) S[u] = __builtin_fmaf(kk.x[u], delta, S[u]);
+                ge = ge1; bt = bt1; vj = vj1;
+            };
+            Row ra = row(ks[buf][0]), rb;            // rows alternate between two sets of registers
+#pragma unroll 1
+            for (int s = 0; s < n; s += 2) { token(s, ra, rb); if (s + 1 < n) token(s + 1, rb, ra); }
+        } else if (outs && b > 0) {                  // block b - 1: the same state once more, and the outputs
+            const int t0 = (b - 1) * PFR_TB, n = min(PFR_TB, C - t0);
+            const int qb2 = (b - 1) & 1;
+            float ge = gs[prv][0][0], delta = ds[qb2][0][cg];
+            auto token = [&](int s, const Row& kk, const Row& qq, Row& kn, Row& qn) {
+                const int s1 = min(s + 1, PFR_TB - 1);
+                kn = row(ks[prv][s1]); qn = row(qs[qb2][s1]);
+                const float ge1 = gs[prv][0][s1], delta1 = ds[qb2][s1][cg];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < U; u++) { S[u] = S[u] * ge; S[u] = __builtin_fmaf(kk.x[u], delta, S[u]); }
+                const float o = chain(qq);
+                if (part == 7 && live) out[(size_t)(t0 + s) * nvdv + (size_t)h * dv + j] = o;
+                ge = ge1; delta = delta1;
+            };
+            Row ra = row(ks[prv][0]), qa = row(qs[qb2][0]), rb, qb;
+#pragma unroll 1
+            for (int s = 0; s < n; s += 2) { token(s, ra, qa, rb, qb); if (s + 1 < n) token(s + 1, rb, qb, ra, qa); }
         }
-        delta = (vj0 - kv) * bt0;
-    }
-    int slot = 0;
-    for (int t = 0; t < C; t++) {
-        // token t: S update + output chain of token t, together with decay + kv chain of token t + 1; blocks of 16 elements, the next block's rows leave LDS while the
-        // current block's steps run (the scheduling fences keep the reads from sinking next to their uses)
-        const int s1 = slot + 1 >= RS ? slot + 1 - RS : slot + 1, s3 = slot + 3 >= RS ? slot + 3 - RS : slot + 3;
-        request(t + 3, s3);          // slot s3 held token t - 2: last read two barriers ago
-        const float4* k4 = reinterpret_cast<const float4*>(&ring[slot][0]); const float4* q4 = reinterpret_cast<const float4*>(&ring[slot][ROW]);
-        const float4* n4 = reinterpret_cast<const float4*>(&ring[s1][0]);
-        const bool has_next = t + 1 < C;
-        const float ge1 = has_next ? ring[s1][3 * ROW] : 1.0f, bt1 = ring[s1][3 * ROW + 1], vj1 = ring[s1][2 * ROW + j];
-        float ob = 0.0f, kv = 0.0f;
-        float4 ka[4] = {k4[0], k4[1], k4[2], k4[3]}, qa[4] = {q4[0], q4[1], q4[2], q4[3]}, na[4] = {n4[0], n4[1], n4[2], n4[3]};
-#pragma unroll
-        for (int b = 0; b < DK / 16; b++) {
-            float4 kb[4] = {ka[0], ka[1], ka[2], ka[3]}, qb[4] = {qa[0], qa[1], qa[2], qa[3]}, nb[4] = {na[0], na[1], na[2], na[3]};
-            if (b + 1 < DK / 16) {
-#pragma unroll
-                for (int u = 0; u < 4; u++) { kb[u] = k4[4 * b + 4 + u]; qb[u] = q4[4 * b + 4 + u]; nb[u] = n4[4 * b + 4 + u]; }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                float* Sb = S + 16 * b + 4 * u;
-                const float kk[4] = {ka[u].x, ka[u].y, ka[u].z, ka[u].w}, qq[4] = {qa[u].x, qa[u].y, qa[u].z, qa[u].w}, nn[4] = {na[u].x, na[u].y, na[u].z, na[u].w};
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    Sb[e] = __builtin_fmaf(kk[e], delta, Sb[e]); ob = __builtin_fmaf(Sb[e], qq[e], ob);
-                    Sb[e] = Sb[e] * ge1; kv = __builtin_fmaf(Sb[e], nn[e], kv);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < 4; u++) { ka[u] = kb[u]; qa[u] = qb[u]; na[u] = nb[u]; }
-        }
-        out[(size_t)t * nvdv + (size_t)h * dv + j] = ob;
-        delta = (vj1 - kv) * bt1;
-        // the next token reads slots t + 1 and t + 2: this wave's requests for token t + 2 (issued one token ago) are older than its 5 requests for t + 3 and the two
-        // output stores since -- at most 7 vector-memory operations may still be in flight
-        asm volatile("s_waitcnt vmcnt(7)" ::: "memory");
+        if (b < nb) publish_q(b & 1);
+        if (b + 1 < nb) publish(nxt);                // last read as block b - 2 by the output waves, a barrier ago
         __syncthreads();
-        slot = s1;
+        buf = nxt;
     }
+    if (!outs && live) {
 #pragma unroll
-    for (int i = 0; i < DK; i++) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(S[i]), srd, j * 4, i * dv * 4, 0);
+        for (int u = 0; u < U; u++) sp[(size_t)u * dv] = S[u];
+    }
 }
 
 // ---- gated RMSNorm + SiLU gate per (token, head) (decode.rs:3979) ----------------------------------------------------------------
@@ -860,8 +881,8 @@ int kr_launch_pfm_la(const KrPfmLaArgs& a, float* recur_state, float* recur_out,
     else {
         if (a.dk != 128 && a.dk != 64) return 1;
         kr_pf_wait(st, sy->wait_b);
-        if (a.dk == 128) hipLaunchKernelGGL(kr_pfm_la_recur_kernel<128>, dim3(a.nv), dim3(a.dv), 0, st, recur_state, a.q, a.k, a.v, a.gexp, a.beta, recur_out, a.nv, a.dv, C);
-        else hipLaunchKernelGGL(kr_pfm_la_recur_kernel<64>, dim3(a.nv), dim3(a.dv), 0, st, recur_state, a.q, a.k, a.v, a.gexp, a.beta, recur_out, a.nv, a.dv, C);
+        if (a.dk == 128) hipLaunchKernelGGL(kr_pfm_la_recur_kernel<128>, dim3(a.nv, (a.dv + 15) / 16), dim3(256), 0, st, recur_state, a.q, a.k, a.v, a.gexp, a.beta, recur_out, a.nv, a.dv, C);
+        else hipLaunchKernelGGL(kr_pfm_la_recur_kernel<64>, dim3(a.nv, (a.dv + 15) / 16), dim3(256), 0, st, recur_state, a.q, a.k, a.v, a.gexp, a.beta, recur_out, a.nv, a.dv, C);
     }
     kr_pf_rec(st, sy->rec_b);
     // z: the stand-alone copy [C][nv * dv] the conv launch makes (z_hr = nv: one block)
@@ -871,8 +892,8 @@ int kr_launch_pfm_la(const KrPfmLaArgs& a, float* recur_state, float* recur_out,
 // the recurrence alone (stand-alone operator linear_attention_recurrent, decode.rs:609): gexp = e^g per (token, head); non-zero = unsupported geometry
 int kr_launch_pfm_la_recur(float* state, const float* q, const float* k, const float* v, const float* gexp, const float* beta, float* out, int nv, int dk, int dv, int C, hipStream_t st) {
     if (dv > 256 || dv % 8 || dv < dk) return 1;
-    if (dk == 128) hipLaunchKernelGGL(kr_pfm_la_recur_kernel<128>, dim3(nv), dim3(dv), 0, st, state, q, k, v, gexp, beta, out, nv, dv, C);
-    else if (dk == 64) hipLaunchKernelGGL(kr_pfm_la_recur_kernel<64>, dim3(nv), dim3(dv), 0, st, state, q, k, v, gexp, beta, out, nv, dv, C);
+    if (dk == 128) hipLaunchKernelGGL(kr_pfm_la_recur_kernel<128>, dim3(nv, (dv + 15) / 16), dim3(256), 0, st, state, q, k, v, gexp, beta, out, nv, dv, C);
+    else if (dk == 64) hipLaunchKernelGGL(kr_pfm_la_recur_kernel<64>, dim3(nv, (dv + 15) / 16), dim3(256), 0, st, state, q, k, v, gexp, beta, out, nv, dv, C);
     else return 1;
     return 0;
 }

@@ -1118,16 +1118,16 @@ int kr_moe_prefill_set(kr_engine* e, int layer, const void* x_bf16, const int32_
         const int mc = M - m0 < CH ? M - m0 : CH;
         const uint16_t* xc = (const uint16_t*)x_bf16 + (size_t)m0 * H;
         const int32_t* idc = ids + (size_t)m0 * topk; const float* wc = wts + (size_t)m0 * topk;
-        const int tiles_bound = (mc * topk) / 64 + E + 1;
-        kr_launch_pf_sort(idc, mc, topk, E, so, st);
+        const int tr = kr_pf_tile_rows(L.w13.view(), L.w2.view(), (long)mc * topk, E), tiles_bound = (mc * topk) / tr + E + 1;
+        kr_launch_pf_sort(idc, mc, topk, E, so, st, tr);
         kr_launch_pf_quant_x(xc, mc, H, (int8_t*)P.xh.p, (int8_t*)P.xl.p, (float*)P.xs.p, st);
         const int var_rows = (long)mc * topk < 48L * E;     // fewer than ~48 rows per expert: most 64-row tiles have an empty second half
         kr_launch_pf_gemm(L.w13.view(), (const uint32_t*)L.w13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, &so, topk, 1,
-                          tiles_bound, 0, (float*)P.gu.p, 2 * I, st, 0, 0, var_rows);
+                          tiles_bound, 0, (float*)P.gu.p, 2 * I, st, 0, 0, var_rows, tr);
         kr_launch_pf_act((const float*)P.gu.p, mc * topk, I, 2 * I, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.hh.p, (int8_t*)P.hl.p,
                          (float*)P.hs.p, st);
         kr_launch_pf_gemm(L.w2.view(), (const uint32_t*)L.w2.wsum.p, (const int8_t*)P.hh.p, (const int8_t*)P.hl.p, (const float*)P.hs.p, &so, topk, 0,
-                          tiles_bound, 0, (float*)P.eo.p, H, st, 0, 0, var_rows);
+                          tiles_bound, 0, (float*)P.eo.p, H, st, 0, 0, var_rows, tr);
         if (use_shared) {
             kr_launch_pf_gemm(L.sw13.view(), (const uint32_t*)L.sw13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, nullptr, topk, 0,
                               0, mc, (float*)P.sgu.p, 2 * SI, st);
@@ -1173,15 +1173,15 @@ int kr_moe_prefill_rows(kr_engine* e, int layer, const void* rows_bf16, const in
     const size_t ob = out_bf16 ? 2 : 4;
     for (int m0 = 0; m0 < n; m0 += CH) {
         const int mc = n - m0 < CH ? n - m0 : CH;
-        const int tiles_bound = mc / 64 + E + 1;
-        kr_launch_pf_sort(lid + m0, mc, 1, E, so, st);
+        const int tr = kr_pf_tile_rows(L.w13.view(), L.w2.view(), mc, E), tiles_bound = mc / tr + E + 1;
+        kr_launch_pf_sort(lid + m0, mc, 1, E, so, st, tr);
         kr_launch_pf_quant_x((const uint16_t*)rows_bf16 + (size_t)m0 * H, mc, H, (int8_t*)P.xh.p, (int8_t*)P.xl.p, (float*)P.xs.p, st);
         const int var_rows = (long)mc < 48L * E;
         kr_launch_pf_gemm(L.w13.view(), (const uint32_t*)L.w13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, &so, 1, 1,
-                          tiles_bound, 0, (float*)P.gu.p, 2 * I, st, 0, 0, var_rows);
+                          tiles_bound, 0, (float*)P.gu.p, 2 * I, st, 0, 0, var_rows, tr);
         kr_launch_pf_act((const float*)P.gu.p, mc, I, 2 * I, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.hh.p, (int8_t*)P.hl.p, (float*)P.hs.p, st);
         kr_launch_pf_gemm(L.w2.view(), (const uint32_t*)L.w2.wsum.p, (const int8_t*)P.hh.p, (const int8_t*)P.hl.p, (const float*)P.hs.p, &so, 1, 0,
-                          tiles_bound, 0, (float*)((char*)out + (size_t)m0 * H * ob), H, st, 1, out_bf16, var_rows);
+                          tiles_bound, 0, (float*)((char*)out + (size_t)m0 * H * ob), H, st, 1, out_bf16, var_rows, tr);
     }
     KR_HIP(hipGetLastError());
     return KR_OK;

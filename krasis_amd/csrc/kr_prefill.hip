@@ -273,6 +273,7 @@ struct KrPfGemmArgs {
 };
 
 #include "kr_prefill_gemm2.inc"
+#include "kr_prefill_wide.inc"
 
 // ------------------------------------------------------------------------------------------
 // combine: out[t] = sum_s w[t][s] * eo[row(t,s)] in routing order (moe.rs:661-667); shared: rsf*out + shared (moe.rs:703-706)
@@ -355,14 +356,33 @@ void kr_launch_pf_wsum(const KrMatDev& m, int n_experts, uint32_t* wsum, hipStre
     if (m.bits == 8) { hipLaunchKernelGGL(kr_pf_wsum8_kernel, dim3((m.N + 7) / 8, n_experts), dim3(64), 0, st, m, wsum); return; }
     hipLaunchKernelGGL(kr_pf_wsum_kernel, dim3((m.N + 7) / 8, n_experts), dim3(64), 0, st, m, wsum);
 }
+// Which exact GEMM.  The wide kernel's workgroup is alone on its compute unit, so it needs rows and tiles: grouped, from 48 rows per expert (us per layer, 64-row tiles against wide:
+// INT8 2048 x 1408, 47 rows an expert 327 / 292, 94 rows 623 / 383, 281 rows 1498 / 940; INT4 47 rows 313 / 311, 94 rows 483 / 403; INT4 2048 x 512, 512 experts, 29 rows
+// 505 / 551, 39 rows 597 / 581, 80 rows 1107 / 904); below that most 64-row tiles have an empty half and var_rows skips it.  Dense, from 128 tiles, half the compute units
+// (a four-layer INT4 prompt, ms, 64-row tiles / wide from 128 tiles / always wide: 777 tokens 3.99 / 3.89 / 3.98, 1400 tokens 6.30 / 5.64 / 5.89).
+// It knows the fused form of the group sum only, and addresses a digit plane by 32-bit offsets.
+static bool pf_all_fma(const KrMatDev& m) { return m.n_fma >= m.N; }
+int kr_pf_tile_rows(const KrMatDev& m0, const KrMatDev& m1, long rows, int E) {
+    return pf_all_fma(m0) && pf_all_fma(m1) && rows * (long)(m0.ng > m1.ng ? m0.ng : m1.ng) * 128 < 1L << 32 && rows >= 48L * E ? PFW_TM : PF_BM;
+}
+static bool pf_dense_wide(const KrPfGemmArgs& a) {
+    int ncb = (a.m.N + PFW_TN - 1) / PFW_TN; bool all = pf_all_fma(a.m);
+    for (int i = 0; i < a.n_extra; i++) { ncb += (a.mx[i].N + PFW_TN - 1) / PFW_TN; all = all && pf_all_fma(a.mx[i]); }
+    return all && (long)a.total_rows * a.m.ng * 128 < 1L << 32 && (long)ncb * ((a.total_rows + PFW_TM - 1) / PFW_TM) >= 128;
+}
 void kr_launch_pf_gemm(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_hi, const int8_t* a_lo, const float* a_scale, const KrPfSort* sort, int topk,
-                       int gather_tokens, int max_tiles, int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows, int out_bf16, int var_rows) {
+                       int gather_tokens, int max_tiles, int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows, int out_bf16, int var_rows, int tile_rows) {
     KrPfGemmArgs a{};
     a.scatter_rows = scatter_rows; a.out_bf16 = out_bf16;
     a.var_rows = sort != nullptr && single_expert_rows <= 0 && var_rows;
     a.m = m; a.wsum = wsum; a.a_hi = a_hi; a.a_lo = a_lo; a.a_scale = a_scale; a.topk = topk; a.gather_tokens = gather_tokens;
     if (sort) { a.row_pair = sort->row_pair; a.tile_expert = sort->tile_expert; a.tile_row0 = sort->tile_row0; a.tile_rows = sort->tile_rows; a.n_tiles = sort->n_tiles; }
     a.out = out; a.out_ld = out_ld; a.single_expert = single_expert_rows > 0; a.total_rows = single_expert_rows;
+    if (single_expert_rows > 0 ? pf_dense_wide(a) : tile_rows == PFW_TM) {
+        const int wt = single_expert_rows > 0 ? (single_expert_rows + PFW_TM - 1) / PFW_TM : max_tiles;
+        if (m.bits == 8) kr_pf_wide_launch<8>(a, wt, st); else kr_pf_wide_launch<4>(a, wt, st);
+        return;
+    }
     const int mt = single_expert_rows > 0 ? (single_expert_rows + PF_BM - 1) / PF_BM : max_tiles;
     // 32 columns per wave, two quantization groups per k stage: the best of the (64|32 columns) x (1|2 groups) shapes and of a 2 x 2 row-split
     // wave grid that were measured
@@ -376,6 +396,10 @@ void kr_launch_pf_gemm_multi(const KrMatDev* mats, const uint32_t* const* wsums,
     a.m = mats[0]; a.wsum = wsums[0]; a.out = outs[0]; a.out_ld = out_lds[0]; a.a_hi = a_hi; a.a_lo = a_lo; a.a_scale = a_scale; a.topk = 1;
     a.single_expert = 1; a.total_rows = M; a.n_extra = n - 1;
     for (int i = 1; i < n; i++) { a.mx[i - 1] = mats[i]; a.wsumx[i - 1] = wsums[i]; a.outx[i - 1] = outs[i]; a.out_ldx[i - 1] = out_lds[i]; }
+    if (pf_dense_wide(a)) {
+        if (mats[0].bits == 8) kr_pf_wide_launch<8>(a, (M + PFW_TM - 1) / PFW_TM, st); else kr_pf_wide_launch<4>(a, (M + PFW_TM - 1) / PFW_TM, st);
+        return;
+    }
     const int mt = (M + PF_BM - 1) / PF_BM;
     if (mats[0].bits == 8) kr_pf_gemm2_launch<32, 2, 8>(a, mt, st);
     else kr_pf_gemm2_launch<32, 2, 4>(a, mt, st);

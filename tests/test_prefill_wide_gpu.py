@@ -1,0 +1,27 @@
+"""The exact grouped GEMM for many rows against the 64-row tiles, bit for bit: the same tokens in one call and in calls of forty rows, which take the latter.  An odd number of quantization groups,
+columns that are no whole tile, experts of 1, 63 - 65 and 127 - 129 rows, skipped slots, and a shared expert of 128 and more tiles."""
+import numpy as np
+import pytest
+
+from tests.test_prefill_gpu import _setup
+from tests.util import rand_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("H,I,bits,w2_bits,n_shared", [(640, 384, 4, 4, 1), (384, 256, 8, 8, 1), (640, 128, 4, 8, 0), (256, 640, 8, 4, 0)])
+def test_many_rows_equal_few(H, I, bits, w2_bits, n_shared):
+    E, k = 9, 2
+    eng, mgr, experts, shared, rng, torch = _setup(H, I, E, k, n_shared, 1.5 if n_shared else 1.0, bits=bits, w2_bits=w2_bits)
+    M = 7000 if n_shared else 700
+    x = torch.from_numpy(rand_bf16(rng, (M, H)).view(np.int16)).cuda().view(torch.bfloat16)
+    ids = np.full((M, k), -1, np.int32)
+    ids[:, 0] = 8
+    at = 0
+    for e, n in enumerate((1, 63, 64, 65, 127, 128, 129, 0)):
+        ids[at:at + n, 1] = e; at += n
+    ids[at] = -1                                                     # a token without experts
+    ids = torch.from_numpy(ids).cuda(); w = torch.from_numpy(rng.random((M, k)).astype(np.float32)).cuda()
+    whole = mgr.forward(0, x, ids, w).view(torch.int16).cpu().numpy()
+    few = np.concatenate([mgr.forward(0, x[i:i + 40], ids[i:i + 40], w[i:i + 40]).view(torch.int16).cpu().numpy() for i in range(0, M, 40)])
+    assert np.array_equal(whole, few)

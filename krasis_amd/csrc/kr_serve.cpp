@@ -108,7 +108,7 @@ struct kr_serve {
     DevBuf page_table;
     std::vector<int> h_table;
     // step scratch
-    DevBuf meta, x, h, qkv, att, mix, gu, y, rows, ffout, ids, wts, rz, moe_i, hw, logits, amax, part_ml, part_acc;
+    DevBuf meta, x, h, qkv, att, mix, gu, y, rows, ffout, ids, wts, moe_i, hw, logits, amax, part_ml, part_acc;
     // f32 copy of the mixer's normed input, its convolved form, residual gate logits, whole-row q / k statistics, recurrent outputs; chunked recurrence:
     // per-token gate terms, state / normaliser at every block's start, per-block gate terms
     DevBuf h32, hc, rg, qk_rms, lin_o, lin_tok, lin_sbuf, lin_nbuf, lin_cm;
@@ -1074,7 +1074,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     const size_t Ts = (size_t)T;
     if (s->x.ensure(Ts * W * 4) || s->h.ensure(Ts * W * s->esz) || s->qkv.ensure(Ts * max_qkv * 4) || s->att.ensure(Ts * max_att * s->esz) || s->mix.ensure(Ts * W * 4) ||
         s->gu.ensure(Ts * max_gu * 4 + 16) || s->y.ensure(Ts * max_y * s->esz + 16) || s->rows.ensure(Ts * max_rows * 4 + 16) || s->ffout.ensure(Ts * W * 4) ||
-        s->ids.ensure(Ts * max_pairs * 4 + 16) || s->rz.ensure(Ts * (size_t)max_E * 8 + 16) || s->wts.ensure(Ts * max_pairs * 4 + 16) || s->moe_i.ensure((Ts * max_pairs * 4 + (size_t)max_E + 8 + max_hist) * 4) ||
+        s->ids.ensure(Ts * max_pairs * 4 + 16) || s->wts.ensure(Ts * max_pairs * 4 + 16) || s->moe_i.ensure((Ts * max_pairs * 4 + (size_t)max_E + 8 + max_hist) * 4) ||
         s->hw.ensure((size_t)std::max(n_want, 1) * W * s->esz) || s->logits.ensure((size_t)std::max(n_want, 1) * c.vocab * 4) || s->amax.ensure((size_t)std::max(n_want, 1) * 4))
         return kr_fail(KR_ERR_HIP, "step scratch for %d tokens", T);
     if ((max_vf && s->v_first.ensure(Ts * max_vf * 4)) ||
@@ -1134,12 +1134,14 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     int* mi = (int*)s->moe_i.p;
     // down projection of a gated feed-forward: decode-sized problems form the activation inside the projection's launch, larger ones write it once
     // (formed: the projection before wrote it itself, see pair_up)
-    auto down_proj = [&](KrSvGemm g, const float* gu, int ld, int rows_m, int F, int kind, float limit, float alpha, const float* row_w = nullptr, bool formed = false) {
-        if (formed) { g.A = s->y.p; g.lda = F; Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); return; }
-        if (kr_sv_gemm_takes_act(g, s->f32, gu, ld)) { g.act_row_w = row_w; g.act_gu = gu; g.act_ld = ld; g.act_kind = kind; g.act_limit = limit; g.act_alpha = alpha; g.A = nullptr; Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); return; }
-        { Timer tm(s, 5); kr_sv_act(gu, ld, s->y.p, s->f32, rows_m, F, kind, limit, alpha, row_w, st, g.up_tab, g.up_rows, g.up_ld, g.up_off); }
+    auto down_ready = [&](KrSvGemm& g, const float* gu, int ld, int rows_m, int F, int kind, float limit, float alpha, const float* row_w = nullptr, bool formed = false) {
+        if (!formed && kr_sv_gemm_takes_act(g, s->f32, gu, ld)) { g.act_row_w = row_w; g.act_gu = gu; g.act_ld = ld; g.act_kind = kind; g.act_limit = limit; g.act_alpha = alpha; g.A = nullptr; return; }
+        if (!formed) { Timer tm(s, 5); kr_sv_act(gu, ld, s->y.p, s->f32, rows_m, F, kind, limit, alpha, row_w, st, g.up_tab, g.up_rows, g.up_ld, g.up_off); }
         g.A = s->y.p; g.lda = F;
-        { Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); }
+    };
+    auto down_proj = [&](KrSvGemm g, const float* gu, int ld, int rows_m, int F, int kind, float limit, float alpha, bool formed = false) {
+        down_ready(g, gu, ld, rows_m, F, kind, limit, alpha, nullptr, formed);
+        Timer tm(s, 1); kr_sv_gemm(g, s->f32, st);
     };
     // prompt-sized: the product `up` whose columns [lo, lo + 2 F) are gate | up of the feed-forward that `down` ends hands on their activation (in y: nothing else may use
     // it until that down projection has read it).  False: it does not, gate | up stand in C
@@ -1423,12 +1425,14 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         }
         const float *dense = nullptr, *shared = nullptr, *rows = nullptr; const int* pair_pos = nullptr;
         if (d.mlp_kind == KR_SERVE_MLP_DENSE) {
-            down_proj(ffd, hz + l.off_gu, l.n_h, T, ff_f, ff_act, ff_limit, ff_alpha, nullptr, ff_formed);
+            down_proj(ffd, hz + l.off_gu, l.n_h, T, ff_f, ff_act, ff_limit, ff_alpha, ff_formed);
             dense = (const float*)s->ffout.p;
         } else if (d.mlp_kind == KR_SERVE_MLP_MOE) {
             const int E = d.experts, top = d.top, F = d.expert_ff, P = T * top;
-            if (ff_f > 0) {              // before the experts: y holds its activation
-                down_proj(ffd, hz + l.off_gu, l.n_h, T, ff_f, ff_act, ff_limit, ff_alpha, nullptr, ff_formed);
+            // the shared expert: beside the experts in their launch if it forms its activation there, else before them (y holds its activation)
+            const bool beside = ff_f > 0 && !ff_formed && kr_sv_gemm_takes_act(ffd, s->f32, hz + l.off_gu, l.n_h);
+            if (ff_f > 0 && !beside) {
+                down_proj(ffd, hz + l.off_gu, l.n_h, T, ff_f, ff_act, ff_limit, ff_alpha, ff_formed);
                 shared = (const float*)s->ffout.p;
             }
             int* seg = mi; int* src_row = seg + E + 1; int* row_group = src_row + P; int* pp = row_group + P; int* hist = pp + 2 * P;
@@ -1444,7 +1448,12 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
             g.a_rows = src_row; g.seg = seg; g.row_group = row_group; g.n_groups = E;
             const bool formed = pair_up(g, dn, g.C, 2 * F, 0, F, d.expert_act, d.expert_limit, d.expert_alpha, row_w);
             { Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); }
-            down_proj(dn, (const float*)s->gu.p, 2 * F, P, F, d.expert_act, d.expert_limit, d.expert_alpha, row_w, formed);
+            down_ready(dn, (const float*)s->gu.p, 2 * F, P, F, d.expert_act, d.expert_limit, d.expert_alpha, row_w, formed);
+            if (beside) { down_ready(ffd, hz + l.off_gu, l.n_h, T, ff_f, ff_act, ff_limit, ff_alpha); shared = (const float*)s->ffout.p; }
+            {
+                Timer tm(s, 1);
+                if (!beside || !kr_sv_gemm_pair(dn, ffd, s->f32, st)) { kr_sv_gemm(dn, s->f32, st); if (beside) kr_sv_gemm(ffd, s->f32, st); }
+            }
             rows = (const float*)s->rows.p; pair_pos = pp;
         }
         // x += the layer's sublayers (parallel block) or the feed-forward alone (sequential), and the next layer's input from the same launch
@@ -1489,7 +1498,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         auto mixin = [&](uint64_t v) { key = (key ^ v) * 1099511628211ull; };
         mixin((uint64_t)T); mixin((uint64_t)n_want); mixin(want_amax);
         for (int v : nsplit) mixin((uint64_t)v);
-        for (const DevBuf* b : {&s->meta, &s->x, &s->h, &s->qkv, &s->att, &s->mix, &s->gu, &s->y, &s->rows, &s->ffout, &s->ids, &s->wts, &s->rz, &s->moe_i, &s->hw, &s->logits,
+        for (const DevBuf* b : {&s->meta, &s->x, &s->h, &s->qkv, &s->att, &s->mix, &s->gu, &s->y, &s->rows, &s->ffout, &s->ids, &s->wts, &s->moe_i, &s->hw, &s->logits,
                                 &s->amax, &s->part_ml, &s->part_acc, &s->v_first, &s->lq_c, &s->lq_2, &s->lq_n, &s->lq_e, &s->att2, &s->head_i, &s->h32, &s->hc, &s->rg, &s->qk_rms, &s->lin_o, &s->qkv2, &s->sconv, &s->ga1, &s->gz, &s->rg_ab, &s->rg_agg, &s->rg_start,
                                 &s->mixes, &s->sgate, &s->lin_tok}) mixin((uint64_t)(uintptr_t)b->p);
         for (const SvRope& r : s->ropes) mixin((uint64_t)(uintptr_t)r.cs.p);

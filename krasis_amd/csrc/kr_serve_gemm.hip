@@ -359,6 +359,13 @@ static bool gm_skinny(const KrSvGemm& g) {
     return g.M <= 16 || (g.M <= 32 && g.N <= 2560);
 }
 
+// up to 16 expert rows: with 24 of a wide layer (4096 x 1536) or 72 (2048 x 768) the experts fill the chip and the pair is no faster than the two (41.6 us against 31 + 10.3)
+bool kr_sv_gemm_pair(const KrSvGemm& e, const KrSvGemm& o, bool f32, hipStream_t st) {
+    if (f32 || e.M <= 0 || e.M > 16 || o.M <= 0 || !e.act_gu || !o.act_gu || !e.seg || o.seg || !gm_skinny(e) || !gm_skinny(o)) return false;
+    kr_sv_gemm_skinny_pair(e, o, st);
+    return true;
+}
+
 bool kr_sv_gemm_takes_glu(const KrSvGemm& g, bool f32) {
     return !f32 && g.M > 0 && !gm_skinny(g) && !gm_gemv_rows(g) && kr_sv_gemm_tile_fits(g, false) && kr_sv_gemm_tile_glu_fits(g);
 }

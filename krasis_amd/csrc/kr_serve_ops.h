@@ -45,10 +45,13 @@ void kr_sv_narrow_act(const KrSvGemm& g, hipStream_t st);
 bool kr_sv_gemm_takes_act(const KrSvGemm& g, bool f32, const float* gu, int ld);      // true: kr_sv_gemm forms the activation of gu [M, ld] inside its launch (act_gu) for this problem
 // whether kr_sv_gemm forms the activation itself where g's glu fields are set (bf16, prompt-sized)
 bool kr_sv_gemm_takes_glu(const KrSvGemm& g, bool f32);
+// a grouped problem and a single matrix that do not depend on one another, both with act_gu, in one launch where they have few rows; false: nothing was launched
+bool kr_sv_gemm_pair(const KrSvGemm& e, const KrSvGemm& o, bool f32, hipStream_t st);
 // the forms for a bf16 store that kr_sv_gemm chooses from; _fits: shapes and alignment
 bool kr_sv_gemm_skinny_fits(const KrSvGemm& g);
 bool kr_sv_gemm_skinny_acts(const KrSvGemm& g);
 void kr_sv_gemm_skinny(const KrSvGemm& g, hipStream_t st);
+void kr_sv_gemm_skinny_pair(const KrSvGemm& e, const KrSvGemm& o, hipStream_t st);
 bool kr_sv_gemm_tile_fits(const KrSvGemm& g, bool f32);
 bool kr_sv_gemm_tile_glu_fits(const KrSvGemm& g);
 void kr_sv_gemm_tile(const KrSvGemm& g, bool f32, hipStream_t st);

@@ -6,7 +6,7 @@
 // flight, LDS staging would only add a hop.  Weights are the first operand (16 columns x 32 k, lane = column + 16 (k / 8)), rows of A the second; rows past M repeat
 // the last one (same address, no traffic) and are not stored.
 // ACT: A is the gated activation of act_gu, formed once per workgroup into LDS while the first weights travel (the wave-per-column form forms it again per column).
-// Grouped problems (one matrix per expert): blockIdx.y = problem row; the first row of a group takes the group's rows, the others leave at once.
+// Grouped problems (one matrix per expert): a strip per problem row; the first row of a group takes the group's rows, the others leave at once.
 // Measured, us, before -> now (weights colder than the last cache): 12 rows: 4224 x 2048 23.9 -> 9.4, 2048 x 2048 19.2 -> 5.9, 32768 x 2048 110 -> 33.6 (4.0 TB/s); 1 row:
 // 9.3 -> 7.2, 6.6 -> 5.0, 45.6 -> 25.6 (5.2 TB/s); 64 experts of 1536 x 2048, 72 rows 54 -> 46 (5.9 TB/s), 180 rows 92 -> 68.
 #include <algorithm>
@@ -17,7 +17,7 @@ namespace {
 typedef float sk_f4 __attribute__((ext_vector_type(4)));
 
 template <int MB, int NB, int WV, bool ACT>               // row blocks of 16, column blocks of 16, waves
-__global__ void __launch_bounds__(64 * WV) sv_skinny_kernel(const KrSvGemm g) {
+__device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int by) {      // by: problem row of a grouped problem
     constexpr int U = NB * MB <= 2 ? 8 : 4;                   // k steps requested together
     constexpr int TR = MB * NB < 4 ? MB * NB : 4;             // output tiles per round of the reduction
     __shared__ __attribute__((aligned(16))) float red[WV][TR][256];
@@ -26,13 +26,13 @@ __global__ void __launch_bounds__(64 * WV) sv_skinny_kernel(const KrSvGemm g) {
     int lo = 0, hi = g.M, N = g.N;
     const uint16_t* W = (const uint16_t*)g.W;
     if (g.row_group) {
-        const int group = g.row_group[blockIdx.y];
+        const int group = g.row_group[by];
         lo = g.seg[group];
-        if (lo != (int)blockIdx.y) return;
+        if (lo != by) return;
         hi = g.seg[group + 1];
         W += (size_t)group * g.w_stride; N = gm_cols(g, group);
-        if (n0 >= N) return;
     }
+    if (n0 >= N) return;
     const int ks = g.K / 32, s0 = ks * wave / WV, s1 = ks * (wave + 1) / WV, lda = g.K + 8;
     const uint16_t* wp[NB];
 #pragma unroll
@@ -120,6 +120,16 @@ __global__ void __launch_bounds__(64 * WV) sv_skinny_kernel(const KrSvGemm g) {
     }
 }
 
+template <int MB, int NB, int WV, bool ACT>
+__global__ void __launch_bounds__(64 * WV) sv_skinny_kernel(const KrSvGemm g) { sk_strip<MB, NB, WV, ACT>(g, blockIdx.y); }
+// the experts' and the shared expert's down projection of a step in one launch, both with the activation inside: neither fills the chip, and a launch with its gap costs more
+// than the smaller of the two (six expert rows and one row, 2048 x 768: 8.1 + 6.3 -> 8.7 us)
+__global__ void __launch_bounds__(256) sv_skinny_pair_kernel(const KrSvGemm e, const KrSvGemm o) {
+    if (blockIdx.y == 0) sk_strip<1, 1, 4, true>(o, 0); else sk_strip<1, 1, 4, true>(e, blockIdx.y - 1);
+}
+
+int sk_act_lds(const KrSvGemm& g) { return (g.row_group ? 16 : std::min(16, g.M)) * (g.K + 8) * 2; }      // one block of sixteen rows
+
 template <int MB, int NB, int WV>
 void sk_launch(const KrSvGemm& g, hipStream_t st) {
     const dim3 grid((g.N + 16 * NB - 1) / (16 * NB), g.row_group ? g.M : 1);
@@ -151,4 +161,12 @@ void kr_sv_gemm_skinny(const KrSvGemm& g, hipStream_t st) {
     if (g.seg || (g.M <= 16 && g.N >= 4096)) sk_launch<1, 1, 4>(p, st);
     else if (g.M <= 16) sk_launch<1, 1, 8>(p, st);
     else sk_launch<2, 1, 8>(p, st);
+}
+
+void kr_sv_gemm_skinny_pair(const KrSvGemm& e, const KrSvGemm& o, hipStream_t st) {
+    KrSvGemm p = o;
+    p.row_group = nullptr;
+    const int lds = std::max(sk_act_lds(e), sk_act_lds(p));
+    (void)hipFuncSetAttribute((const void*)sv_skinny_pair_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    hipLaunchKernelGGL(sv_skinny_pair_kernel, dim3((std::max(e.N, o.N) + 15) / 16, e.M + 1), dim3(256), lds, st, e, p);
 }

@@ -734,6 +734,16 @@ __global__ void __launch_bounds__(1024) kr_fd_merge2_kernel(const KrFdFlashArgs 
     const int h = blockIdx.x, t = threadIdx.x, G = a.nh / a.nkv, kvh = h / G, g = h % G;
     const int seq = a.step->pos + 1, nc = min((seq + chunk - 1) / chunk, 1024);
     const float* ml = a.fd_ml + (size_t)h * n_chunks * 2;
+    // thread = (dim d, chunk phase): 1024 / HD phases walk interleaved chunks with 4 independent sums each.  Sixteen partials are on their way at a time, the first of them while
+    // the weights are formed (four at a time were ten round trips one after the other at 20000 positions: 8.0 us, now 7.3)
+    constexpr int NPH = 1024 / HD, PF = 16;
+    const int d = t % HD, ph = t / HD;
+    const float* ob = a.fd_o + ((size_t)kvh * n_chunks * G + g) * HD + d;
+    float v[PF];
+    if (ph + (PF - 1) * NPH < nc) {
+#pragma unroll
+        for (int u = 0; u < PF; u++) v[u] = ob[(size_t)(ph + u * NPH) * G * HD];
+    }
     float mx = -__builtin_inff();
     const float mv = t < nc ? ml[t * 2] : -__builtin_inff(), lv = t < nc ? ml[t * 2 + 1] : 0.0f;      // nc <= 1024 = one chunk per thread
     mx = mv;
@@ -755,12 +765,20 @@ __global__ void __launch_bounds__(1024) kr_fd_merge2_kernel(const KrFdFlashArgs 
 #pragma unroll
     for (int i = 0; i < 16; i++) lt += red[16 + i];
     const float inv = 1.0f / lt;
-    // thread = (dim d, chunk phase): 1024 / HD phases walk interleaved chunks with 4 independent sums each
-    constexpr int NPH = 1024 / HD;
-    const int d = t % HD, ph = t / HD;
-    const float* ob = a.fd_o + ((size_t)kvh * n_chunks * G + g) * HD + d;
     float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
     int c = ph;
+    while (c + (PF - 1) * NPH < nc) {
+#pragma unroll
+        for (int u = 0; u < PF; u += 4) {
+            s0 = __builtin_fmaf(wc[c + u * NPH], v[u], s0); s1 = __builtin_fmaf(wc[c + (u + 1) * NPH], v[u + 1], s1);
+            s2 = __builtin_fmaf(wc[c + (u + 2) * NPH], v[u + 2], s2); s3 = __builtin_fmaf(wc[c + (u + 3) * NPH], v[u + 3], s3);
+        }
+        c += PF * NPH;
+        if (c + (PF - 1) * NPH < nc) {
+#pragma unroll
+            for (int u = 0; u < PF; u++) v[u] = ob[(size_t)(c + u * NPH) * G * HD];
+        }
+    }
     for (; c + 3 * NPH < nc; c += 4 * NPH) {
         const float v0 = ob[(size_t)c * G * HD], v1 = ob[(size_t)(c + NPH) * G * HD], v2 = ob[(size_t)(c + 2 * NPH) * G * HD], v3 = ob[(size_t)(c + 3 * NPH) * G * HD];
         s0 = __builtin_fmaf(wc[c], v0, s0); s1 = __builtin_fmaf(wc[c + NPH], v1, s1); s2 = __builtin_fmaf(wc[c + 2 * NPH], v2, s2); s3 = __builtin_fmaf(wc[c + 3 * NPH], v3, s3);

@@ -319,8 +319,9 @@ __global__ void __launch_bounds__(512, 2) sv_attn_step_kernel(const KrSvAttn a) 
     const int p = a.pos[t];
     const int* table = a.page_table + (size_t)a.slot[t] * a.table_ld;
     const int lo = a.window > 0 ? max(0, p - a.window + 1) : (a.chunk > 0 ? p - p % a.chunk : 0);
-    // kept first keys: their own leading tiles when the window has left them behind, else one contiguous range from 0
-    const int nck = a.keep > 0 && lo > a.keep ? (a.keep + 31) / 32 : 0;
+    // kept first keys: their own leading tiles when the window's tiles, which begin at a multiple of 32, lie past the last of them (else that tile would hold kept keys too, and
+    // the mask lets them through wherever they stand), else one contiguous range from 0
+    const int nck = a.keep > 0 && (lo & ~31) >= a.keep ? (a.keep + 31) / 32 : 0;
     const int first = a.keep > 0 && nck == 0 ? 0 : lo & ~31;
     const int nch = (p - first) / 32 + 1 + nck, cps = (nch + a.nsplit - 1) / a.nsplit, c0 = sp * cps, c1 = min(nch, c0 + cps);
     const uint16_t* kp = (const uint16_t*)a.kpool + (size_t)g * DIM + q * 8;

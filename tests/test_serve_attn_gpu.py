@@ -68,3 +68,28 @@ def test_single_tokens(heads, kv_heads, dim, vdim, ctx, window):
     x0 = W["embed"].astype(np.float64)[[s[-1] for s in seqs]]
     ref = np.stack([O.forward(cfg, W, s)[1][0][-1] for s in seqs])
     assert row_errors(got - x0, ref - x0).max() < 2e-2
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,keep,window", [
+    (4, 2, 32, 32, 1, 12), (4, 1, 64, 128, 4, 64), (4, 4, 128, 64, 31, 33), (8, 2, 32, 64, 33, 31), (4, 1, 128, 128, 40, 40), (4, 2, 64, 32, 3, 12),
+    (4, 2, 64, 64, 4, 290), (4, 1, 128, 128, 33, 290), (8, 2, 32, 32, 40, 250)])                 # the last ones share their keys over several workgroups
+def test_kept_first_keys_meet_the_window(heads, kv_heads, dim, vdim, keep, window):
+    # every position from the one where the window still touches the kept keys to one where a block of 32 keys lies between them: a kept key counts once
+    from tests import oracle_gasavik as G
+    from tests.test_gasavik_gpu import engine as gasavik_engine
+    cfg = G.make_config(width=64, vocab=50, side=0, layers=[G.layer(G.parallel(heads, kv_heads, dim, vdim, window, keep, 1, 8, 8, left_scale=1.0, right_scale=0.01), None)])
+    W = {k: G.bf16_round(v) for k, v in G.random_weights(cfg, 29).items()}
+    first, n = keep + window - 1, keep + window + 62
+    toks = tokens(cfg, n, 30)
+    eng = gasavik_engine(cfg, W, "bfloat16")
+    eng.step([("a", toks[:first], [])])
+    eng.store.set_capture(True)
+    got = []
+    for i in range(first, first + 42):
+        eng.step([("a", toks[i:i + 1], [0])])
+        got.append(eng.store.read_capture(1)[0])
+    eng.step([("a", toks[first + 42:], [0])])                                                        # a portion short of the prompt form
+    got = np.concatenate(got + [eng.store.read_capture(n - first - 42)[0]])
+    x0 = G.embed(cfg, {k: np.asarray(v, np.float64) for k, v in W.items()}, toks)[first:]
+    # as above; one key of 291 twice would be off by 1 / sqrt(291) = 6e-2
+    assert row_errors(got - x0, G.forward(cfg, W, toks)[1][0][first:] - x0).max() < 2e-2

@@ -518,13 +518,13 @@ bool kr_sv_attn_step_fits(int dim, int vdim, int ldk, int ldv, int ldq, int page
     return (dim == 32 || dim == 64 || dim == 128) && (vdim == 32 || vdim == 64 || vdim == 128);      // 256: the split operands no longer fit the registers
 }
 
-// key splits of a decode step: one workgroup up to 256 keys (one round of its waves), then two, four and eight (powers of two: a new count is a new step to capture), beyond 1024
-// shares of 512 for about two workgroups per compute unit.  (us per step of two layers, 1 / 2 / 4 / 8 / 16 shares: one request at 100 keys 248 / 248 / 253 / 252 / 253, at 1024
-// 275 / 268 / 266 / 258 / 258; twelve requests at 1024 333 / 322 / 325 / 320 / 331.)
+// Key splits of a decode step: one workgroup up to 256 keys (one round of its waves), then two, four and eight (powers of two: a new count is a new step to capture), beyond 1024
+// shares of 512 keys; never more than two workgroups per compute unit in all, which bounds the partial states too.  (us per step of two layers, 1 / 2 / 4 / 8 / 16 shares: one
+// request at 100 keys 248 / 248 / 253 / 252 / 253, at 1024 275 / 268 / 266 / 258 / 258; twelve requests at 1024 333 / 322 / 325 / 320 / 331.  Many requests, shares unbounded / at most
+// 1024 / at most 512 workgroups: 64 of 8 / 8 heads at 1100 keys 388 / 298 / 279, 128 of 64 / 4 heads at 1100 627 / 507 / 476, 256 of 16 / 2 heads at 2000 960 / 840 / 844.)
 int kr_sv_attn_step_splits(int T, int heads, int kv_heads, int max_visible) {
-    const long blocks = (long)T * kv_heads * ((heads / kv_heads + 15) / 16);
-    const long near = max_visible <= 256 ? 1 : max_visible < 512 ? 2 : max_visible < 1024 ? 4 : 8, far = std::min((long)max_visible / 512, 512 / std::max(blocks, 1L));
-    return (int)std::max(near, far);
+    const long most = std::max(1L, 512 / std::max(1L, (long)T * kv_heads * ((heads / kv_heads + 15) / 16)));
+    return (int)std::min(most, (long)(max_visible <= 256 ? 1 : max_visible < 512 ? 2 : max_visible < 1024 ? 4 : std::max(8, max_visible / 512)));
 }
 
 void kr_sv_attn_step(const KrSvAttn& a, hipStream_t st) {

@@ -93,3 +93,18 @@ def test_kept_first_keys_meet_the_window(heads, kv_heads, dim, vdim, keep, windo
     x0 = G.embed(cfg, {k: np.asarray(v, np.float64) for k, v in W.items()}, toks)[first:]
     # as above; one key of 291 twice would be off by 1 / sqrt(291) = 6e-2
     assert row_errors(got - x0, G.forward(cfg, W, toks)[1][0][first:] - x0).max() < 2e-2
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,requests", [(8, 8, 32, 64, 24), (8, 2, 64, 32, 40), (16, 1, 128, 128, 33)])
+def test_many_requests_deep_in_their_caches(heads, kv_heads, dim, vdim, requests):
+    # more workgroups than the chip holds: fewer shares each.  Every request is the beginning of one sequence, so one row of the oracle each
+    cfg = model(heads, kv_heads, dim, vdim, 0, rot=8); W = O.random_weights(cfg, 31)
+    toks = tokens(cfg, 1060 + requests, 32)
+    eng = engine(cfg, W, "bfloat16", max_tokens=requests * 1152, max_slots=requests)
+    for i in range(requests):
+        eng.step([(i, toks[:1060 + i], [])])
+    eng.store.set_capture(True)
+    eng.step([(i, toks[1060 + i:1061 + i], [0]) for i in range(requests)])
+    got = eng.store.read_capture(requests)[0]
+    x0 = W["embed"].astype(np.float64)[toks[1060:1060 + requests]]
+    assert row_errors(got - x0, O.forward(cfg, W, toks)[1][0][1060:] - x0).max() < 2e-2

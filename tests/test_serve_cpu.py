@@ -144,3 +144,24 @@ def test_trace_replay_loop(tmp_path):
     assert said == ["done 0", "done 1", "done 2"] and not eng.len
     assert np.fromfile(os.path.join(tmp_path, "0.f32"), "<f4").shape == (6,) and not os.path.exists(os.path.join(tmp_path, "1.f32"))
     assert np.fromfile(os.path.join(tmp_path, "2.f32"), "<f4").shape == (3,)
+
+
+# ---------------------------------------------------------------------------------------------------------------- which launches a step takes (host rules of the native library)
+def native(name, *args, res=None):
+    import ctypes as C
+    from krasis_amd import _lib
+    f = getattr(_lib.load_library(), name)
+    f.restype = C.c_int if res is None else res
+    return f(*args)
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(8, 8), (16, 2), (64, 4), (40, 1), (128, 1)])
+def test_shares_of_keys_fill_the_chip_and_stop_there(heads, kv_heads):
+    one = {n: native("_Z22kr_sv_attn_step_splitsiiii", 1, heads, kv_heads, n) for n in (1, 256, 257, 512, 1024, 4096, 8192)}
+    assert [one[n] for n in (1, 256, 257, 512, 1024, 4096, 8192)] == [1, 1, 2, 4, 8, 8, 16]
+    for tokens in (1, 2, 12, 64, 65, 500, 2048):
+        blocks = tokens * kv_heads * -(-(heads // kv_heads) // 16)
+        for keys in (100, 600, 1100, 5000, 100000):
+            shares = native("_Z22kr_sv_attn_step_splitsiiii", tokens, heads, kv_heads, keys)
+            # a share costs a token and head 4 (vdim + 2) bytes of partial state, written and read in every layer
+            assert shares == 1 or shares * blocks <= 512

@@ -976,7 +976,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     for (int i = 0; i < n_want; i++) if (want_rows[i] < 0 || want_rows[i] >= T) return kr_fail(KR_ERR_VALUE, "wanted row %d of %d", want_rows[i], T);
     if (need_pages > (int)s->free_pages.size()) return kr_fail(KR_ERR_STATE, "cache pool exhausted: %d pages needed, %zu free", need_pages, s->free_pages.size());
     // ---- per-step arrays: tokens | slot | pos | want | page table
-    const size_t n_meta = (size_t)4 * T + n_want + 3 * (size_t)n_entries + 2;      // ... | first row of every entry and the end | slot of every entry | first 64-token block of every entry and the end
+    const size_t n_meta = (size_t)5 * T + n_want + 3 * (size_t)n_entries + 2;      // ... | first row of every entry and the end | slot of every entry | first 64-token block of every entry and the end | tokens, those of short entries first
     const size_t meta_bytes = (n_meta + s->h_table.size()) * 4;
     if (meta_bytes > s->h_meta_bytes) {
         if (s->h_meta) (void)hipHostFree(s->h_meta);
@@ -985,14 +985,15 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         s->h_meta_bytes = meta_bytes * 2;
     }
     int* hm = (int*)s->h_meta;
-    int* h_tok = hm; int* h_slot = hm + T; int* h_pos = hm + 2 * T; int* h_brow = hm + 3 * T; int* h_want = hm + 4 * T; /* h_brow: row of the pair embedding */ int* h_eoff = h_want + n_want; int* h_eslot = h_eoff + n_entries + 1; int* h_echunk = h_eslot + n_entries;
+    int* h_tok = hm; int* h_slot = hm + T; int* h_pos = hm + 2 * T; int* h_brow = hm + 3 * T; int* h_want = hm + 4 * T; /* h_brow: row of the pair embedding */ int* h_eoff = h_want + n_want; int* h_eslot = h_eoff + n_entries + 1; int* h_echunk = h_eslot + n_entries; int* h_order = h_echunk + n_entries + 1;
     int* h_tab = hm + n_meta;
     int max_pos = 0, n_chunks = 0, max_count = 0;
+    std::vector<int> last_pos(n_entries);
     {
         int t = 0;
         for (int e = 0; e < n_entries; e++) {
             SvSlot& q = s->slots[slots[e]];
-            max_pos = std::max(max_pos, q.len + counts[e] - 1);
+            last_pos[e] = q.len + counts[e] - 1; max_pos = std::max(max_pos, last_pos[e]);
             h_eoff[e] = t; h_eslot[e] = slots[e]; h_echunk[e] = n_chunks; n_chunks += (counts[e] + 63) / 64; max_count = std::max(max_count, counts[e]);
             const int np = (q.len + counts[e] + PT - 1) / PT;
             while ((int)q.pages.size() < np) { q.pages.push_back(s->free_pages.back()); s->free_pages.pop_back(); }
@@ -1006,6 +1007,11 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
             q.len += counts[e];
         }
         h_eoff[n_entries] = t; h_echunk[n_entries] = n_chunks;
+        std::vector<int> by(n_entries);
+        for (int e = 0; e < n_entries; e++) by[e] = e;
+        std::stable_sort(by.begin(), by.end(), [&](int x, int y) { return counts[x] < counts[y]; });
+        t = 0;
+        for (int e : by) for (int i = 0; i < counts[e]; i++) h_order[t++] = h_eoff[e] + i;
         for (int i = 0; i < n_want; i++) h_want[i] = want_rows[i];
         std::memcpy(h_tab, s->h_table.data(), s->h_table.size() * 4);
     }
@@ -1013,7 +1019,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     hipStream_t st = s->st;
     KR_HIP(hipMemcpyAsync(s->meta.p, hm, meta_bytes, hipMemcpyHostToDevice, st));
     const int* d_tok = (const int*)s->meta.p; const int* d_slot = d_tok + T; const int* d_pos = d_tok + 2 * T; const int* d_brow = d_tok + 3 * T; const int* d_want = d_tok + 4 * T;
-    const int* d_eoff = d_want + n_want; const int* d_eslot = d_eoff + n_entries + 1; const int* d_echunk = d_eslot + n_entries;
+    const int* d_eoff = d_want + n_want; const int* d_eslot = d_eoff + n_entries + 1; const int* d_echunk = d_eslot + n_entries; const int* d_order = d_echunk + n_entries + 1;
     const int* d_tab = d_tok + n_meta;
     // ---- scratch sized for this step
     const bool seq = c.block_kind == KR_SERVE_BLOCK_SEQUENTIAL;
@@ -1094,17 +1100,14 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     if (max_ssdz && s->ssd_z.ensure(Ts * max_ssdz * 4)) return kr_fail(KR_ERR_HIP, "state-space block scratch for %d tokens", T);
     for (SvRope& r : s->ropes) if (r.cs.ensure(Ts * (r.dims / 2) * 8)) return kr_fail(KR_ERR_HIP, "rope table");
     if (s->capture) { if (s->cap.ensure((size_t)c.n_layers * Ts * W * 4)) return kr_fail(KR_ERR_HIP, "capture buffer"); s->cap_T = T; }
-    std::vector<int> nsplit(c.n_layers, 1);
-    std::vector<int> att_form(c.n_layers, 0);
+    std::vector<KrSvAttnPlan> plan(c.n_layers, KrSvAttnPlan{KR_SV_ATTN_GENERAL, 1, 0, 0, 0, 0});
     for (int li = 0; li < c.n_layers; li++) {
         const SvLayer& l = s->L[li]; const kr_serve_layer& d = l.d;
         if (l.recurrent() || l.no_heads()) continue;
-        const int visible = d.window > 0 ? std::min(max_pos + 1, d.window + d.keep_first) : (d.chunk > 0 ? std::min(max_pos + 1, d.chunk) : max_pos + 1);
         const int ldk = l.latent() ? l.att_dim() : d.kv_heads * d.dim, ldv = l.latent() ? l.att_dim() : d.kv_heads * d.vdim;
         const int ldq = l.latent() ? d.heads * l.att_dim() : d.proj_conv ? (int)l.pconv_c() : l.n_h;
-        att_form[li] = kr_sv_attn_form(T, n_entries, max_count, d.heads, l.att_heads_kv(), l.att_dim(), l.att_vdim(), ldk, ldv, ldq, PT, s->f32, visible, &nsplit[li]);
-        if (nsplit[li] > 1 && (s->part_ml.ensure(Ts * d.heads * nsplit[li] * 8) || s->part_acc.ensure(Ts * d.heads * nsplit[li] * l.att_vdim() * 4)))
-            return kr_fail(KR_ERR_HIP, "attention split scratch");
+        plan[li] = kr_sv_attn_form(n_entries, counts, last_pos.data(), d.heads, l.att_heads_kv(), l.att_dim(), l.att_vdim(), ldk, ldv, ldq, PT, s->f32, d.window, d.keep_first, d.chunk);
+        if (plan[li].parts && (s->part_ml.ensure(plan[li].parts * 8) || s->part_acc.ensure(plan[li].parts * l.att_vdim() * 4))) return kr_fail(KR_ERR_HIP, "attention split scratch");
     }
     const bool want_amax = argmax_out != nullptr;
     // every launch of the step, in order; no allocation, no host copy: the same body runs eagerly or under stream capture
@@ -1231,8 +1234,8 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         a.sink = d.has_sink ? (const float*)l.sink.p : nullptr;
         a.kpool = kvl.kpool.p; a.page_table = d_tab; a.table_ld = s->n_pages; a.slot = d_slot; a.pos = d_pos; a.page_tokens = PT; a.T = T;
         a.out = s->att.p;
-        a.ent_off = d_eoff; a.n_entries = n_entries; a.form = att_form[li];
-        a.nsplit = nsplit[li]; a.part_ml = (float*)s->part_ml.p; a.part_acc = (float*)s->part_acc.p;
+        a.ent_off = d_eoff; a.n_entries = n_entries; a.form = plan[li].form; a.order = d_order; a.few = plan[li].few; a.n_few = plan[li].n_few; a.nsplit_few = plan[li].nsplit_few;
+        a.nsplit = plan[li].nsplit; a.part_ml = (float*)s->part_ml.p; a.part_acc = (float*)s->part_acc.p;
         const void* o_in = s->att.p;
         if (l.recurrent()) {
             KrSvLin q{};
@@ -1497,7 +1500,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         uint64_t key = 1469598103934665603ull;
         auto mixin = [&](uint64_t v) { key = (key ^ v) * 1099511628211ull; };
         mixin((uint64_t)T); mixin((uint64_t)n_want); mixin(want_amax);
-        for (int v : nsplit) mixin((uint64_t)v);
+        for (const KrSvAttnPlan& p : plan) mixin((uint64_t)p.nsplit);
         for (const DevBuf* b : {&s->meta, &s->x, &s->h, &s->qkv, &s->att, &s->mix, &s->gu, &s->y, &s->rows, &s->ffout, &s->ids, &s->wts, &s->moe_i, &s->hw, &s->logits,
                                 &s->amax, &s->part_ml, &s->part_acc, &s->v_first, &s->lq_c, &s->lq_2, &s->lq_n, &s->lq_e, &s->att2, &s->head_i, &s->h32, &s->hc, &s->rg, &s->qk_rms, &s->lin_o, &s->qkv2, &s->sconv, &s->ga1, &s->gz, &s->rg_ab, &s->rg_agg, &s->rg_start,
                                 &s->mixes, &s->sgate, &s->lin_tok}) mixin((uint64_t)(uintptr_t)b->p);

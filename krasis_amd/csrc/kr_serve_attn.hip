@@ -68,14 +68,14 @@ __global__ void __launch_bounds__(256, 2) sv_attn_prompt_kernel(const KrSvAttn a
     __shared__ __attribute__((aligned(1024))) uint16_t Vt[2 * VSLOT];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 31, h = lane >> 5;
     const int R = a.heads / a.kv_heads, TQ = AT_ROWS / R, g = blockIdx.y, sp = blockIdx.z;
-    // the tile of tokens: entries' tile counts through a prefix sum over the lanes
+    // the tile of tokens: entries' tile counts (short entries may have a launch of their own) through a prefix sum over the lanes
     int t0 = 0, cnt = 0;
     {
         int acc = 0;
         bool found = false;
         for (int e0 = 0; e0 < a.n_entries && !found; e0 += 64) {
             const int e = min(e0 + lane, a.n_entries - 1);
-            const int lo = a.ent_off[e], hi = a.ent_off[e + 1], nt = e0 + lane < a.n_entries ? (hi - lo + TQ - 1) / TQ : 0;
+            const int lo = a.ent_off[e], hi = a.ent_off[e + 1], nt = e0 + lane < a.n_entries && hi - lo > a.few ? (hi - lo + TQ - 1) / TQ : 0;
             int sum = nt;
 #pragma unroll
             for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(sum, o); if (lane >= o) sum += v; }
@@ -313,7 +313,7 @@ template <int DIM, int VDIM>
 __global__ void __launch_bounds__(512, 2) sv_attn_step_kernel(const KrSvAttn a) {
     constexpr int KS = DIM / 32, CPL = VDIM / 16, VW = CPL / 2, NW = 8;
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int R = a.heads / a.kv_heads, t = blockIdx.x, g = blockIdx.y, sp = blockIdx.z % a.nsplit, hb = blockIdx.z / a.nsplit;
+    const int R = a.heads / a.kv_heads, t = a.toks ? a.toks[blockIdx.x] : (int)blockIdx.x, g = blockIdx.y, sp = blockIdx.z % a.nsplit, hb = blockIdx.z / a.nsplit;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), row = lane & 15, q = lane >> 4;
     const int Rb = min(16, R - hb * 16), h0 = g * R + hb * 16, head = h0 + min(row, Rb - 1);
     const int p = a.pos[t];
@@ -474,7 +474,7 @@ __global__ void __launch_bounds__(512, 2) sv_attn_step_kernel(const KrSvAttn a) 
             const float gt = a.out_gate ? 1.0f / (1.0f + expf(-a.out_gate[(size_t)t * a.ld_gate + (a.gate_elem ? (size_t)h * VDIM + c : (size_t)h)])) : 1.0f;
             ((uint16_t*)a.out)[(size_t)t * (a.out_ld ? a.out_ld : a.heads * VDIM) + (size_t)h * VDIM + c] = kr_f32_to_bf16(v * rl[r] * gt * (a.out_scale != 0.0f ? a.out_scale : 1.0f));
         } else {
-            const size_t slot = ((size_t)t * a.heads + h) * a.nsplit + sp;
+            const size_t slot = ((size_t)blockIdx.x * a.heads + h) * a.nsplit + sp;
             a.part_acc[slot * VDIM + c] = v;
             if (c == 0) { a.part_ml[slot * 2] = rl[16 + r]; a.part_ml[slot * 2 + 1] = rl[r]; }
         }
@@ -489,7 +489,7 @@ template <int DIM, int VDIM> void as_launch(const KrSvAttn& a, hipStream_t st) {
 }
 template <int DIM, int VDIM> void at_launch(const KrSvAttn& a, hipStream_t st) {
     const int TQ = AT_ROWS / (a.heads / a.kv_heads);
-    hipLaunchKernelGGL((sv_attn_prompt_kernel<DIM, VDIM>), dim3(a.T / TQ + a.n_entries, a.kv_heads, a.nsplit), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((sv_attn_prompt_kernel<DIM, VDIM>), dim3((a.T - a.n_few) / TQ + a.n_entries, a.kv_heads, a.nsplit), dim3(256), 0, st, a);
 }
 }  // namespace
 

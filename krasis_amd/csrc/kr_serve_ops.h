@@ -137,14 +137,19 @@ struct KrSvAttn {
     int page_tokens, T;
     void* out;                       // [T, heads * vdim] storage type
     int nsplit;                      // >= 1: workgroups that share a token's keys (few tokens: more of the chip per token); > 1 needs the two buffers below
-    float* part_ml; float* part_acc; // [T][heads][nsplit][2] running (maximum, denominator), [T][heads][nsplit][vdim] unnormalised sums
+    float* part_ml; float* part_acc; // [T][heads][nsplit][2] running (maximum, denominator), [T][heads][nsplit][vdim] unnormalised sums (short entries: their place in `order` for T)
     int tq;                          // set by the launcher of the matrix-instruction form: tokens per workgroup
     const int* ent_off; int n_entries;     // [n_entries + 1] first row of every entry of the step: rows of an entry are consecutive positions of one request
     int form;                        // KR_SV_ATTN_*: the caller's choice (kr_sv_attn_form); nsplit belongs to it
+    // a KR_SV_ATTN_PROMPT step whose short entries (at most `few` tokens, n_few in all) take the other form, with nsplit_few shares; order [T]: the tokens, those of short entries first
+    int few, n_few, nsplit_few; const int* order;
+    const int* toks;                 // set by the launcher: the launch's tokens (null: all of them, in their order)
 };
 enum { KR_SV_ATTN_GENERAL = 0, KR_SV_ATTN_PROMPT = 1, KR_SV_ATTN_STEP = 2 };      // the last two keep their running maxima in powers of two
-// which form a layer takes in a step whose largest portion has max_count tokens, and how many workgroups share a token's keys (at most max_visible)
-int kr_sv_attn_form(int T, int n_entries, int max_count, int heads, int kv_heads, int dim, int vdim, int ldk, int ldv, int ldq, int page_tokens, bool f32, int max_visible, int* nsplit);
+// which form a layer takes in a step, and how many workgroups share a token's keys
+struct KrSvAttnPlan { int form, nsplit, few, n_few, nsplit_few; size_t parts; };  // parts: partial states [heads] that split launches leave (part_ml holds 2 floats of each, part_acc vdim)
+KrSvAttnPlan kr_sv_attn_form(int n_entries, const int* counts, const int* last_pos /* of every entry */, int heads, int kv_heads, int dim, int vdim, int ldk, int ldv, int ldq, int page_tokens, bool f32,
+                             int window, int keep, int chunk);
 // the 128-row form of a bf16 store (kr_serve_attn.hip): sizes and strides it takes; its key splits
 bool kr_sv_attn_prompt_fits(int heads, int kv_heads, int dim, int vdim, int ldk, int ldv, int ldq, bool f32);
 int kr_sv_attn_prompt_splits(int T, int n_entries, int heads, int kv_heads, int max_visible);

@@ -5,9 +5,11 @@
 // Every f32 reduction here is a lane / wave tree; sums written as a * b + c may be contracted (explicit __builtin_fmaf): the serving path states a
 // tolerance against an f32 restatement, not a bit pattern.
 #include <hip/hip_runtime.h>
+#include <limits.h>
 #include <math.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <initializer_list>
 #include <type_traits>
 
@@ -867,8 +869,8 @@ __global__ void __launch_bounds__(256) sv_attn_mfma_kernel(const KrSvAttn a) {
 template <typename T>
 __global__ void __launch_bounds__(256) sv_attn_merge_kernel(const KrSvAttn a) {
     extern __shared__ float wsp[];           // [nsplit] weight of every split, then 1 / denominator
-    const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
-    const size_t base = ((size_t)t * a.heads + h) * a.nsplit;
+    const int t = a.toks ? a.toks[blockIdx.x] : (int)blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+    const size_t base = ((size_t)(a.form == KR_SV_ATTN_STEP ? blockIdx.x : t) * a.heads + h) * a.nsplit;
     const float sink = a.sink ? (a.form ? a.sink[h] * 1.44269504f : a.sink[h]) : -INFINITY;      // the split forms keep their maxima in powers of two
     auto ex = [&](float x) { return a.form ? exp2f(x) : expf(x); };
     float M = sink;
@@ -2293,18 +2295,45 @@ int kr_sv_attention_splits(int T, int heads, int kv_heads, int dim, int vdim, in
     return ns < 1 ? 1 : (int)ns;
 }
 
-// A portion of 32 tokens fills a quarter of a 128-row tile of eight heads per key head; below that the rows of single tokens go to their own workgroups.
-int kr_sv_attn_form(int T, int n_entries, int max_count, int heads, int kv_heads, int dim, int vdim, int ldk, int ldv, int ldq, int page_tokens, bool f32, int max_visible, int* nsplit) {
-    if (max_count >= 32 && kr_sv_attn_prompt_fits(heads, kv_heads, dim, vdim, ldk, ldv, ldq, f32)) {
-        *nsplit = kr_sv_attn_prompt_splits(T, n_entries, heads, kv_heads, max_visible);
-        return KR_SV_ATTN_PROMPT;
+// Which form an entry of the step takes.  A single token goes to its own workgroups (per key head and 16 query heads), which read its keys for it alone; a portion of many tokens to
+// 128-row tiles.  Portions of 2 - 31 tokens go either way: own workgroups while all short entries together are at most 192 of them, three quarters of the chip (us per step of two layers
+// at 500 keys, own workgroups / tiles: 16 / 2 heads, one portion of 16 tokens 131 / 158, eight of 16 219 / 214, eight of 31 383 / 248; 8 / 8 heads, one of 8 143 / 158, one of 31 223 / 171;
+// at 1500 keys, 64 portions of 16, 8 / 8 heads 3847 / 828, 64 / 4 heads 2888 / 1000).
+// Short entries beside a prompt portion have rows in few waves of a tile and may see many more keys than the portion: they ride in its launch unless that makes them its tail by three
+// tiles of keys or more, else they get a launch of their own before it (one request at 20000 keys beside 512 tokens, 64 / 4 heads: 3347 riding, 453 apart; beside 2000 tokens 3783 / 1125;
+// but 15 requests at 200 keys beside 2000 tokens, 16 / 2 heads, window 1024: 522 / 563).
+KrSvAttnPlan kr_sv_attn_form(int n_entries, const int* counts, const int* last_pos, int heads, int kv_heads, int dim, int vdim, int ldk, int ldv, int ldq, int page_tokens, bool f32, int window,
+                             int keep, int chunk) {
+    KrSvAttnPlan p{};
+    const bool prompt = kr_sv_attn_prompt_fits(heads, kv_heads, dim, vdim, ldk, ldv, ldq, f32), step = kr_sv_attn_step_fits(dim, vdim, ldk, ldv, ldq, page_tokens, f32);
+    struct Part { int tokens = 0, entries = 0, keys = 0; };      // of some entries: how many, and the most keys that one of their tokens sees
+    auto part = [&](int lo, int hi) {
+        Part q;
+        for (int e = 0; e < n_entries; e++) {
+            if (counts[e] < lo || counts[e] > hi) continue;
+            const int n = last_pos[e] + 1;
+            q.tokens += counts[e]; q.entries++;
+            q.keys = std::max(q.keys, window > 0 ? std::min(n, window + keep) : chunk > 0 ? std::min(n, chunk) : n);
+        }
+        return q;
+    };
+    const Part all = part(1, INT_MAX), below = part(1, 31);
+    // (where the tiles do not fit, no form shares a token's keys with the next token)
+    const int few = !prompt || (long)below.tokens * kv_heads * ((heads / kv_heads + 15) / 16) <= 192 ? 31 : 1;
+    const Part a = part(1, few), b = part(few + 1, INT_MAX);
+    if (step && b.entries == 0) {
+        p.form = KR_SV_ATTN_STEP; p.nsplit = kr_sv_attn_step_splits(all.tokens, heads, kv_heads, all.keys);
+    } else if (prompt) {
+        p.form = KR_SV_ATTN_PROMPT; p.nsplit = kr_sv_attn_prompt_splits(all.tokens, all.entries, heads, kv_heads, all.keys);
+        if (step && a.entries > 0 && (a.keys + 63) / 64 - (b.keys + 63) / 64 >= 3 * p.nsplit) {
+            p.few = few; p.n_few = a.tokens; p.nsplit_few = kr_sv_attn_step_splits(a.tokens, heads, kv_heads, a.keys);
+            p.nsplit = kr_sv_attn_prompt_splits(b.tokens, b.entries, heads, kv_heads, b.keys);
+        }
+    } else {
+        p.form = KR_SV_ATTN_GENERAL; p.nsplit = kr_sv_attention_splits(all.tokens, heads, kv_heads, dim, vdim, ldk, ldv, f32, all.keys);
     }
-    if (max_count < 32 && kr_sv_attn_step_fits(dim, vdim, ldk, ldv, ldq, page_tokens, f32)) {
-        *nsplit = kr_sv_attn_step_splits(T, heads, kv_heads, max_visible);
-        return KR_SV_ATTN_STEP;
-    }
-    *nsplit = kr_sv_attention_splits(T, heads, kv_heads, dim, vdim, ldk, ldv, f32, max_visible);
-    return KR_SV_ATTN_GENERAL;
+    p.parts = std::max(p.nsplit > 1 ? (size_t)all.tokens * p.nsplit : 0, p.nsplit_few > 1 ? (size_t)p.n_few * p.nsplit_few : 0) * heads;
+    return p;
 }
 
 // the matrix-instruction form takes prompt-sized steps whose head sizes fit its register tiling
@@ -2345,9 +2374,16 @@ static bool sv_attn_mfma_launch(const KrSvAttn& a, hipStream_t st) {
 void kr_sv_attention(const KrSvAttn& a, bool f32, hipStream_t st) {
     if (a.T <= 0) return;
     if (a.form != KR_SV_ATTN_GENERAL) {
-        if (a.form == KR_SV_ATTN_PROMPT) kr_sv_attn_prompt(a, st); else kr_sv_attn_step(a, st);
-        if (a.nsplit > 1) hipLaunchKernelGGL(sv_attn_merge_kernel<uint16_t>, dim3(a.T, a.heads), dim3(256), (size_t)(a.nsplit + 1) * sizeof(float), st, a);
-        return;
+        // the short entries' launches come first; both kinds leave partial states in the same buffers, one after the other
+        KrSvAttn b = a;
+        if (a.form == KR_SV_ATTN_PROMPT && a.n_few > 0) { b.form = KR_SV_ATTN_STEP; b.toks = a.order; b.T = a.n_few; b.nsplit = a.nsplit_few; }
+        for (;;) {
+            if (b.form == KR_SV_ATTN_PROMPT) kr_sv_attn_prompt(b, st); else kr_sv_attn_step(b, st);
+            const int n = b.form == KR_SV_ATTN_PROMPT ? b.T - b.n_few : b.T;
+            if (b.nsplit > 1) hipLaunchKernelGGL(sv_attn_merge_kernel<uint16_t>, dim3(n, b.heads), dim3(256), (size_t)(b.nsplit + 1) * sizeof(float), st, b);
+            if (b.form == a.form) return;
+            b = a; b.toks = a.order + a.n_few;
+        }
     }
     if (f32 ? sv_attn_mfma_launch<float>(a, st) : sv_attn_mfma_launch<uint16_t>(a, st)) {
         if (a.nsplit > 1) {

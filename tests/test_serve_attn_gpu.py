@@ -108,3 +108,39 @@ def test_many_requests_deep_in_their_caches(heads, kv_heads, dim, vdim, requests
     got = eng.store.read_capture(requests)[0]
     x0 = W["embed"].astype(np.float64)[toks[1060:1060 + requests]]
     assert row_errors(got - x0, O.forward(cfg, W, toks)[1][0][1060:] - x0).max() < 2e-2
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(8, 2, 64, 64), (16, 1, 64, 128), (4, 4, 128, 32)])
+@pytest.mark.parametrize("portion", [33, 260])
+def test_short_entries_beside_a_portion(heads, kv_heads, dim, vdim, portion):
+    # a portion at the start of a request beside single tokens and a few tokens deep in others: the short entries take launches of their own, in any order of the entries
+    cfg = model(heads, kv_heads, dim, vdim, 0); W = O.random_weights(cfg, 33)
+    a, b, c = tokens(cfg, 1500, 34), tokens(cfg, portion, 35), tokens(cfg, 40, 36)
+    x0, ref = [W["embed"].astype(np.float64)[np.asarray(t)] for t in (a, b, c)], [O.forward(cfg, W, t)[1][0] for t in (a, b, c)]
+    eng = engine(cfg, W, "bfloat16", max_tokens=8192, max_slots=6)
+    for rid, n in (("a", 1495), ("b", 1300), ("d", 1409)):                 # beginnings of one sequence
+        eng.step([(rid, a[:n], [])])
+    eng.store.set_capture(True)
+    eng.step([("d", a[1409:1410], [0]), ("p", b, [portion - 1]), ("a", a[1495:], [4]), ("q", c, [39]), ("b", a[1300:1301], [0])])
+    got = eng.store.read_capture(portion + 47)[0]
+    lo = 0
+    for i, k, n in ((0, 1409, 1), (1, 0, portion), (0, 1495, 5), (2, 0, 40), (0, 1300, 1)):
+        assert row_errors(got[lo:lo + n] - x0[i][k:k + n], ref[i][k:k + n] - x0[i][k:k + n]).max() < 2e-2
+        lo += n
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(8, 8, 32, 64), (16, 2, 128, 128), (32, 1, 64, 32)])
+@pytest.mark.parametrize("n", [2, 7, 31])
+def test_many_short_portions(heads, kv_heads, dim, vdim, n):
+    cfg = model(heads, kv_heads, dim, vdim, 0, rot=8); W = O.random_weights(cfg, 37)
+    requests = 1 + 192 // (n * kv_heads * max(1, heads // kv_heads // 16))
+    toks = tokens(cfg, 70 + requests + n, 38)
+    eng = engine(cfg, W, "bfloat16", max_tokens=requests * 320, max_slots=requests)
+    for i in range(requests):
+        eng.step([(i, toks[:70 + i], [])])
+    eng.store.set_capture(True)
+    eng.step([(i, toks[70 + i:70 + i + n], [0]) for i in range(requests)])
+    got = eng.store.read_capture(requests * n)[0]
+    at = np.concatenate([np.arange(70 + i, 70 + i + n) for i in range(requests)])
+    x0 = W["embed"].astype(np.float64)[np.asarray(toks)[at]]
+    assert row_errors(got - x0, O.forward(cfg, W, toks)[1][0][at] - x0).max() < 2e-2

@@ -165,3 +165,35 @@ def test_shares_of_keys_fill_the_chip_and_stop_there(heads, kv_heads):
             shares = native("_Z22kr_sv_attn_step_splitsiiii", tokens, heads, kv_heads, keys)
             # a share costs a token and head 4 (vdim + 2) bytes of partial state, written and read in every layer
             assert shares == 1 or shares * blocks <= 512
+
+
+def attention_plan(heads, kv_heads, entries, window=0, keep=0, chunk=0, dim=128, page_tokens=64):
+    """entries: (tokens of the step, tokens in the cache before it)"""
+    import ctypes as C
+
+    class Plan(C.Structure):
+        _fields_ = [(n, C.c_int) for n in ("form", "nsplit", "few", "n_few", "nsplit_few")] + [("parts", C.c_size_t)]
+    n = len(entries)
+    counts, last = (C.c_int * n)(*[c for c, _ in entries]), (C.c_int * n)(*[c + p - 1 for c, p in entries])
+    return native("_Z15kr_sv_attn_formiPKiS0_iiiiiiiibiii", n, counts, last, heads, kv_heads, dim, dim, kv_heads * dim, kv_heads * dim, 4 * heads * dim, page_tokens, C.c_bool(False), window, keep,
+                  chunk, res=Plan)
+
+
+PROMPT, STEP = 1, 2
+
+
+def test_attention_form_follows_every_entry():
+    assert attention_plan(16, 2, [(1, 5000)] * 64).form == STEP                            # single tokens, however many
+    assert attention_plan(8, 8, [(16, 1500)] * 64).form == PROMPT                          # short portions that would be thousands of workgroups, each reading its keys again
+    assert attention_plan(64, 4, [(31, 1500)] * 64).form == PROMPT
+    assert attention_plan(16, 2, [(31, 500)]).form == STEP                                 # few enough of them stay apart
+    assert attention_plan(6, 1, [(31, 500)] * 64).form == STEP                             # (no tile takes six heads per key head)
+    # decoding requests beside a portion: apart when their keys would make them the launch's tail, and then with shares of their own
+    p = attention_plan(64, 4, [(1, 20000), (512, 0), (1, 19000)])
+    assert (p.form, p.n_few) == (PROMPT, 2) and p.few >= 1 and p.nsplit_few >= 8 and p.parts == 64 * max(2 * p.nsplit_few, 514 * p.nsplit if p.nsplit > 1 else 0)
+    p = attention_plan(16, 2, [(1, 20000)] * 15 + [(2000, 0)])
+    assert (p.form, p.n_few) == (PROMPT, 15)
+    assert attention_plan(16, 2, [(1, 200)] * 15 + [(2000, 0)]).n_few == 0                 # else they ride
+    assert attention_plan(16, 2, [(1, 20000)] * 15 + [(2000, 0)], window=1024).n_few == 0
+    assert attention_plan(16, 2, [(1, 20000), (2000, 0)], page_tokens=40).n_few == 0       # pages that the other form does not take
+    assert attention_plan(16, 2, [(1, 20000), (1, 30), (2000, 1000)], window=64, keep=4).parts == 0

@@ -22,6 +22,7 @@
 #include <algorithm>
 
 #include "kr_device.h"
+#include "kr_lds_optin.h"
 #include "kr_serve_ops.h"
 
 namespace {
@@ -484,7 +485,7 @@ __global__ void __launch_bounds__(512, 2) sv_attn_step_kernel(const KrSvAttn a) 
 template <int DIM, int VDIM> void as_launch(const KrSvAttn& a, hipStream_t st) {
     const int R = a.heads / a.kv_heads, Rb = R < 16 ? R : 16;
     const int lds = (8 * Rb * (VDIM + 4) + 3 * 8 * 16 + 32) * (int)sizeof(float);
-    (void)hipFuncSetAttribute((const void*)sv_attn_step_kernel<DIM, VDIM>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (kr_lds_optin((const void*)sv_attn_step_kernel<DIM, VDIM>, lds)) return;        // (the step ends with the runtime's error)
     hipLaunchKernelGGL((sv_attn_step_kernel<DIM, VDIM>), dim3(a.T, a.kv_heads, (R + 15) / 16 * a.nsplit), dim3(512), lds, st, a);
 }
 template <int DIM, int VDIM> void at_launch(const KrSvAttn& a, hipStream_t st) {

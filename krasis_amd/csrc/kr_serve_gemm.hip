@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "kr_lds_optin.h"
 #include "kr_serve_gemm_dev.h"
 
 namespace {
@@ -334,9 +335,9 @@ bool kr_sv_narrow_act_fits(const KrSvGemm& g, bool f32) {
 }
 void kr_sv_narrow_act(const KrSvGemm& g, hipStream_t st) {
     const dim3 grid((g.M + 31) / 32);
-    if (g.N <= 128) { const size_t b = (size_t)4 * 32 * (4 * 32 + 4) * 4; (void)hipFuncSetAttribute((const void*)sv_narrow_act_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b);
+    if (g.N <= 128) { const size_t b = (size_t)4 * 32 * (4 * 32 + 4) * 4; if (kr_lds_optin((const void*)sv_narrow_act_kernel<4>, b)) return;
         hipLaunchKernelGGL(sv_narrow_act_kernel<4>, grid, dim3(512), b, st, g); }
-    else { const size_t b = (size_t)4 * 32 * (8 * 32 + 4) * 4; (void)hipFuncSetAttribute((const void*)sv_narrow_act_kernel<8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b);
+    else { const size_t b = (size_t)4 * 32 * (8 * 32 + 4) * 4; if (kr_lds_optin((const void*)sv_narrow_act_kernel<8>, b)) return;
         hipLaunchKernelGGL(sv_narrow_act_kernel<8>, grid, dim3(512), b, st, g); }
 }
 

@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include "kr_device.h"
+#include "kr_lds_optin.h"
 #include "kr_serve_ops.h"
 
 namespace {
@@ -683,7 +684,7 @@ bool kr_sv_lin_blocks_fit(int dim, int vdim) { return dim <= 128 && vdim <= 128;
 void kr_sv_lin_chan_blocks(const KrSvLin& a, hipStream_t st) {
     if (a.T <= 0 || a.n_entries <= 0 || a.n_chunks <= 0) return;
     const dim3 g(a.n_chunks, a.heads);
-#define LN_LDS(K_, B_) do { if ((B_) > 48 * 1024) (void)hipFuncSetAttribute((const void*)K_, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(B_)); } while (0)
+#define LN_LDS(K_, B_) do { if ((B_) > 48 * 1024 && kr_lds_optin((const void*)K_, B_)) return; } while (0)
     if (a.kind == 4) {
         const size_t n = (size_t)a.T * a.heads * a.dim;
         hipLaunchKernelGGL(ln_gla_log_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, const_cast<float*>(a.gz), a.gz_bias, n, a.heads * a.dim, a.inv_tau);

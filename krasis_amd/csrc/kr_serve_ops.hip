@@ -14,6 +14,7 @@
 #include <type_traits>
 
 #include "kr_device.h"
+#include "kr_lds_optin.h"
 #include "kr_serve_gemm_dev.h"
 #include "kr_serve_ops.h"
 
@@ -2511,7 +2512,7 @@ void kr_sv_lin_scan_wide(const KrSvLin& a, hipStream_t st) {
     }
     // one workgroup per compute unit or fewer: the pipelined walk; more: the plain one (256 compute units, up to three workgroups on each)
     const bool pipe = (size_t)grid.x * grid.y * grid.z <= 384;
-#define SV_LW(K_, DP_, P_) do { if (lds > 48 * 1024) (void)hipFuncSetAttribute((const void*)sv_lin_scanw_kernel<K_, DP_, P_>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+#define SV_LW(K_, DP_, P_) do { if (lds > 48 * 1024 && kr_lds_optin((const void*)sv_lin_scanw_kernel<K_, DP_, P_>, lds)) return; \
                                 hipLaunchKernelGGL((sv_lin_scanw_kernel<K_, DP_, P_>), grid, dim3(256), lds, st, a); } while (0)
 #define SV_LW_P(K_, DP_) do { if (pipe) SV_LW(K_, DP_, true); else SV_LW(K_, DP_, false); } while (0)
 #define SV_LW_D(K_) do { if (dpr <= 4) SV_LW_P(K_, 4); else if (dpr <= 8) SV_LW_P(K_, 8); else SV_LW_P(K_, 16); } while (0)

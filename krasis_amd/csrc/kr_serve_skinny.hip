@@ -11,6 +11,7 @@
 // 9.3 -> 7.2, 6.6 -> 5.0, 45.6 -> 25.6 (5.2 TB/s); 64 experts of 1536 x 2048, 72 rows 54 -> 46 (5.9 TB/s), 180 rows 92 -> 68.
 #include <algorithm>
 
+#include "kr_lds_optin.h"
 #include "kr_serve_gemm_dev.h"
 
 namespace {
@@ -135,7 +136,7 @@ void sk_launch(const KrSvGemm& g, hipStream_t st) {
     const dim3 grid((g.N + 16 * NB - 1) / (16 * NB), g.row_group ? g.M : 1);
     if (g.act_gu) {
         const int rows = g.row_group ? 16 * MB : std::min(16 * MB, g.M), lds = rows * (g.K + 8) * 2;
-        (void)hipFuncSetAttribute((const void*)sv_skinny_kernel<MB, NB, WV, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (kr_lds_optin((const void*)sv_skinny_kernel<MB, NB, WV, true>, lds)) return;
         hipLaunchKernelGGL((sv_skinny_kernel<MB, NB, WV, true>), grid, dim3(64 * WV), lds, st, g);
     } else hipLaunchKernelGGL((sv_skinny_kernel<MB, NB, WV, false>), grid, dim3(64 * WV), 0, st, g);
 }
@@ -167,6 +168,6 @@ void kr_sv_gemm_skinny_pair(const KrSvGemm& e, const KrSvGemm& o, hipStream_t st
     KrSvGemm p = o;
     p.row_group = nullptr;
     const int lds = std::max(sk_act_lds(e), sk_act_lds(p));
-    (void)hipFuncSetAttribute((const void*)sv_skinny_pair_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (kr_lds_optin((const void*)sv_skinny_pair_kernel, lds)) return;
     hipLaunchKernelGGL(sv_skinny_pair_kernel, dim3((std::max(e.N, o.N) + 15) / 16, e.M + 1), dim3(256), lds, st, e, p);
 }

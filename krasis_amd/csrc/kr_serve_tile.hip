@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "kr_lds_optin.h"
 #include "kr_serve_gemm_dev.h"
 
 namespace {
@@ -226,7 +227,7 @@ void tl_launch(const KrSvGemm& g, hipStream_t st) {
     static_assert(!GLU || (sizeof(T) == 2 && BN / WN % 64 == 0 && WM * WN * 2 * 32 * 36 * 4 <= LDS), "a wave holds both factors, and stages them");
     const int cols = GLU ? (g.N - 2 * g.glu_f + BN - 1) / BN + (g.glu_f + BN / 2 - 1) / (BN / 2) : (g.N + BN - 1) / BN;
     const dim3 grid(cols, (g.M + BM - 1) / BM + (g.seg ? g.n_groups : 0));
-    (void)hipFuncSetAttribute((const void*)sv_tile_kernel<T, BM, BN, WM, WN, DEPTH, WPS, GLU>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    if (kr_lds_optin((const void*)sv_tile_kernel<T, BM, BN, WM, WN, DEPTH, WPS, GLU>, LDS)) return;
     hipLaunchKernelGGL((sv_tile_kernel<T, BM, BN, WM, WN, DEPTH, WPS, GLU>), grid, dim3(64 * WM * WN), LDS, st, g);
 }
 }  // namespace

@@ -197,3 +197,10 @@ def test_attention_form_follows_every_entry():
     assert attention_plan(16, 2, [(1, 20000)] * 15 + [(2000, 0)], window=1024).n_few == 0
     assert attention_plan(16, 2, [(1, 20000), (2000, 0)], page_tokens=40).n_few == 0       # pages that the other form does not take
     assert attention_plan(16, 2, [(1, 20000), (1, 30), (2000, 1000)], window=64, keep=4).parts == 0
+
+
+def test_lds_windows_are_raised_in_one_place():
+    # hipFuncSetAttribute with a call's own size would lower the window that another thread's launch of the same kernel counts on
+    src = os.path.join(os.path.dirname(R.__file__), "csrc")
+    users = [f for f in sorted(os.listdir(src)) if f.endswith((".hip", ".cpp", ".h", ".inc")) and "hipFuncSetAttribute(" in open(os.path.join(src, f)).read()]
+    assert users == ["kr_lds_optin.h"]

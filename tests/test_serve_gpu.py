@@ -431,3 +431,36 @@ def test_graph_replays_equal_eager_steps():
     ref = O.forward(cfg, W, a[:131])[0]
     e = np.sqrt(((lg[0] - ref[130]) ** 2).mean()) / np.sqrt((ref ** 2).mean())
     assert e < 4e-2
+
+
+def test_two_stores_step_in_two_threads():
+    """8 and 16 query heads per key head, expert widths of 96 and 1024: the same kernels with different amounts of LDS, from two threads at once"""
+    import threading
+    models = []
+    for heads, ff in ((8, 96), (16, 1024)):
+        cfg = O.make_config(width=128, vocab=70, eps=1e-5, layers=[{"type": "attention", "mixer": O.attn(heads, 1, 128, 128, 0, 16, scale=0.1), "mlp": O.moe(4, 2, 1, 1, ff, 2.0, ff, 2.0)}])
+        models.append((engine(cfg, O.random_weights(cfg, heads), "bfloat16"), tokens(cfg, 60, heads)))
+
+    def turn(eng, toks):
+        rows = [eng.step([("a", toks[:40], [39])])[0]]
+        for t in toks[40:]:
+            rows.append(eng.step([("a", [t], [0])])[0])
+        eng.finish("a")
+        return np.concatenate(rows)
+    alone = [turn(*m) for m in models]
+    got, errors = [[], []], []
+
+    def work(i):
+        try:
+            for _ in range(6):
+                got[i].append(turn(*models[i]))
+        except Exception as e:                                     # noqa: BLE001 -- reported below, in the test's own thread
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    for i in range(2):
+        assert len(got[i]) == 6 and all(np.array_equal(g, alone[i]) for g in got[i])

@@ -1033,7 +1033,7 @@ __global__ void __launch_bounds__(SORT ? 1024 : 256) sv_router_rank_kernel(const
             }
             int rank = 0;
             for (int j = 0; j < groups; j++) { const float o = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(g), j)); rank += (o > g || (o == g && j < lane)) ? 1 : 0; }
-            gsc[wave][lane] = (lane < groups && g == g && g != -INFINITY && rank < keep) ? 1.0f : 0.0f;
+            gsc[wave][lane] = (lane < groups && g == g && rank < keep) ? 1.0f : 0.0f;      // (a sum of two choice scores may be minus infinity with an expert left in the group)
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
             for (int i = 0; i < NV; i++) { const int e = lane + 64 * i; if (e < E && gsc[wave][e / per] == 0.0f) ok[i] = false; }

@@ -33,3 +33,24 @@ def test_rows_of_prompts(n, top):
     eng.store.set_capture(True)
     eng.step([("a", toks, [n - 1])])
     assert rel(eng.store.read_capture(n)[0], ref) < 2e-4
+
+
+@pytest.mark.parametrize("experts,groups,keep,top", [(12, 4, 3, 5), (96, 4, 3, 26), (132, 4, 3, 35)])
+@pytest.mark.parametrize("n", [3, 40])
+def test_groups_whose_score_is_minus_infinity(experts, groups, keep, top, n):
+    # a correction of minus infinity takes experts out.  The sum of a group's two largest choice scores is minus infinity when one expert is left in it: such a group still
+    # fills a free place among the kept ones (lowest index first), and its expert can be chosen
+    from tests import oracle_midisun as M
+    from tests.test_midisun_gpu import engine as midisun_engine
+    cfg = M.make_config(64, 40, [M.layer(M.retention(2, 8, 8, (0.9, 0.95)), M.moe(experts, top, 16, groups, keep))], groups=1, taps=1)
+    W = M.random_weights(cfg, 35)
+    per = experts // groups
+    for g in range(1, groups):
+        W["l0.mlp.correction"][g * per:(g + 1) * per] = -np.inf
+        W["l0.mlp.correction"][g * per + g % per] = 0.1 * g
+    toks = tokens(cfg, n, 36)
+    ref = M.forward(cfg, W, toks)[1][0]
+    eng = midisun_engine(cfg, W)
+    eng.store.set_capture(True)
+    eng.step([("a", toks, [n - 1])])
+    assert rel(eng.store.read_capture(n)[0], ref) < 2e-4

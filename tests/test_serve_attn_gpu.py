@@ -144,3 +144,28 @@ def test_many_short_portions(heads, kv_heads, dim, vdim, n):
     at = np.concatenate([np.arange(70 + i, 70 + i + n) for i in range(requests)])
     x0 = W["embed"].astype(np.float64)[np.asarray(toks)[at]]
     assert row_errors(got - x0, O.forward(cfg, W, toks)[1][0][at] - x0).max() < 2e-2
+
+
+@pytest.mark.parametrize("design,size", [("capped", 4096), ("capped", 330), ("chunked", 0), ("chunked", 300)])
+@pytest.mark.parametrize("heads,kv_heads,dim", [(8, 2, 128), (16, 4, 64)])
+def test_capped_scores_distance_bias_and_chunks(design, size, heads, kv_heads, dim):
+    # a prompt of 700 tokens as portions of 40 and 660 (one and several workgroups per token's keys), 6 tokens at once, then single ones; a soft cap near the scores' size
+    from tests import oracle_midisun as M, oracle_pamulix as P, test_midisun_gpu, test_pamulix_gpu
+    if design == "capped":
+        cfg = M.make_config(64, 50, [M.layer(M.attn(heads, kv_heads, dim, size, scale=0.2, softcap=2.5), None)], groups=1, taps=1)
+        W = {k: M.bf16_round(v) for k, v in M.random_weights(cfg, 39).items()}
+        make, forward, x0 = test_midisun_gpu.engine, M.forward, lambda t: W["embed"].astype(np.float64)[t] * cfg["embedding"]["scale"]
+    else:
+        cfg = P.make_config(width=64, vocab=50, layers=[P.layer(P.attn(heads, kv_heads, dim, dim, size, scale=0.2), None)])
+        W = P.random_weights(cfg, 39)
+        make, forward, x0 = test_pamulix_gpu.engine, P.forward, lambda t: W["embed"].astype(np.float64)[t]
+    toks = tokens(cfg, 716, 40)
+    eng = make(cfg, W, "bfloat16")
+    eng.store.set_capture(True)
+    got, at = [], 0
+    for n in [40, 660, 6] + [1] * 10:
+        eng.step([("a", toks[at:at + n], [n - 1])])
+        got.append(eng.store.read_capture(n)[0])
+        at += n
+    base = x0(np.asarray(toks))
+    assert row_errors(np.concatenate(got) - base, forward(cfg, W, toks)[1][0] - base).max() < 2e-2

@@ -735,7 +735,8 @@ __global__ void __launch_bounds__(1024) kr_fd_merge2_kernel(const KrFdFlashArgs 
     const int seq = a.step->pos + 1, nc = min((seq + chunk - 1) / chunk, 1024);
     const float* ml = a.fd_ml + (size_t)h * n_chunks * 2;
     // thread = (dim d, chunk phase): 1024 / HD phases walk interleaved chunks with 4 independent sums each.  Sixteen partials are on their way at a time, the first of them while
-    // the weights are formed (four at a time were ten round trips one after the other at 20000 positions: 8.0 us, now 7.3)
+    // the weights are formed (four at a time were ten round trips one after the other at 20000 positions: 8.1 us, now 7.4; one such launch a step of
+    // 83 us, less than its runs differ by)
     constexpr int NPH = 1024 / HD, PF = 16;
     const int d = t % HD, ph = t / HD;
     const float* ob = a.fd_o + ((size_t)kvh * n_chunks * G + g) * HD + d;

@@ -356,7 +356,7 @@ void kr_launch_pf_wsum(const KrMatDev& m, int n_experts, uint32_t* wsum, hipStre
     if (m.bits == 8) { hipLaunchKernelGGL(kr_pf_wsum8_kernel, dim3((m.N + 7) / 8, n_experts), dim3(64), 0, st, m, wsum); return; }
     hipLaunchKernelGGL(kr_pf_wsum_kernel, dim3((m.N + 7) / 8, n_experts), dim3(64), 0, st, m, wsum);
 }
-// Which exact GEMM.  The wide kernel's workgroup is alone on its compute unit, so it needs rows and tiles: grouped, from 48 rows per expert (us per layer, 64-row tiles against wide:
+// Which exact GEMM.  The wide kernel's workgroup is alone on its compute unit, so it needs rows and tiles: grouped, from 48 rows per expert (us per layer, one pass and the wait for it, 64-row tiles against wide:
 // INT8 2048 x 1408, 47 rows an expert 327 / 292, 94 rows 623 / 383, 281 rows 1498 / 940; INT4 47 rows 313 / 311, 94 rows 483 / 403; INT4 2048 x 512, 512 experts, 29 rows
 // 505 / 551, 39 rows 597 / 581, 80 rows 1107 / 904); below that most 64-row tiles have an empty half and var_rows skips it.  Dense, from 128 tiles, half the compute units
 // (a four-layer INT4 prompt, ms, 64-row tiles / wide from 128 tiles / always wide: 777 tokens 3.99 / 3.89 / 3.98, 1400 tokens 6.30 / 5.64 / 5.89).

@@ -14,7 +14,8 @@
 // LDS-DMA writes lane-linear, so the chunk order is swizzled on the source side: K chunk c of row r at c ^ (r / rows per 256 bytes), V groups of four chunks likewise, which
 // spreads the 32 rows of a fragment read, and the 4 rows x 64 bytes of a transposing read, over all banks.
 // Bound: the matrix instruction, three times 4 H D keys operations (about 50 us at the case below); exponentials, the splitting of the weights and the addresses (some 700
-// vector instructions per tile and wave beside 96 products) run beside it in the SIMD's other wave.  Per launch, us, f32 matrix instruction before -> now: 4096 tokens, 16 / 2
+// vector instructions per tile and wave beside 96 products) run beside it in the SIMD's other wave; at head size 128 the query pieces, sums and scores of two waves per SIMD are
+// 25 registers more than there are, and those spill.  Per launch, us, f32 matrix instruction before -> now: 4096 tokens, 16 / 2
 // heads of 128, window 1024: 490 -> 136; 3300 tokens of three requests, 64 / 4 heads, window 2048: 1230 -> 333.  64-bit oracle of a whole prompt: error 5.1e-3 before, 4.4e-3
 // now (the store's bf16 roundings).
 #include <hip/hip_runtime.h>

@@ -259,8 +259,8 @@ bool kr_sv_gemm_tile_glu_fits(const KrSvGemm& g) {
            (g.silu_hi <= g.silu_lo || g.silu_hi <= g.glu_lo || g.silu_lo >= g.glu_lo + 2 * g.glu_f) && tl_kind(g) != 64;
 }
 
-// f32 (500 tokens, 64 experts of 2 x 768 x 2048: 410 us a product on average with scalar loads and vector FMAs -> 131): the matrix instruction takes 16 times as long for the same product (32x32x2, every factor and sum in f32), so nothing but its own count matters: 128 x 128 where that fills
-// the chip without more padding than 64 x 64.
+// f32 (500 tokens, 64 experts of 2 x 768 x 2048: 410 us a product on average with scalar loads and vector FMAs -> 131): the matrix instruction takes 16 times as long for the
+// same product (32x32x2, every factor and sum in f32), so nothing but its own count matters: 128 x 128 where that fills the chip without more padding than 64 x 64.
 void kr_sv_gemm_tile(const KrSvGemm& g, bool f32, hipStream_t st) {
     if (f32) {
         if (4.0 * std::ceil(tl_tiles(g, 128) / 256) < tl_tiles(g, 64) / 256) tl_launch<float, 128, 128, 2, 2, 2, 2, false>(g, st);

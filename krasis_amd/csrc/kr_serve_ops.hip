@@ -2324,7 +2324,7 @@ KrSvAttnPlan kr_sv_attn_form(int n_entries, const int* counts, const int* last_p
     const Part a = part(1, few), b = part(few + 1, INT_MAX);
     if (step && b.entries == 0) {
         p.form = KR_SV_ATTN_STEP; p.nsplit = kr_sv_attn_step_splits(all.tokens, heads, kv_heads, all.keys);
-    } else if (prompt) {
+    } else if (prompt && (step || part(32, INT_MAX).entries > 0)) {      // (pages that own workgroups do not take: the general form up to 31 tokens)
         p.form = KR_SV_ATTN_PROMPT; p.nsplit = kr_sv_attn_prompt_splits(all.tokens, all.entries, heads, kv_heads, all.keys);
         if (step && a.entries > 0 && (a.keys + 63) / 64 - (b.keys + 63) / 64 >= 3 * p.nsplit) {
             p.few = few; p.n_few = a.tokens; p.nsplit_few = kr_sv_attn_step_splits(a.tokens, heads, kv_heads, a.keys);

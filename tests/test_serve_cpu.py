@@ -179,7 +179,7 @@ def attention_plan(heads, kv_heads, entries, window=0, keep=0, chunk=0, dim=128,
                   chunk, res=Plan)
 
 
-PROMPT, STEP = 1, 2
+GENERAL, PROMPT, STEP = 0, 1, 2
 
 
 def test_attention_form_follows_every_entry():
@@ -197,6 +197,10 @@ def test_attention_form_follows_every_entry():
     assert attention_plan(16, 2, [(1, 20000)] * 15 + [(2000, 0)], window=1024).n_few == 0
     assert attention_plan(16, 2, [(1, 20000), (2000, 0)], page_tokens=40).n_few == 0       # pages that the other form does not take
     assert attention_plan(16, 2, [(1, 20000), (1, 30), (2000, 1000)], window=64, keep=4).parts == 0
+    # pages that the step form does not take: steps without a portion of 32 tokens keep the general form
+    assert attention_plan(16, 2, [(1, 5000)] * 4, page_tokens=40).form == GENERAL
+    assert attention_plan(8, 8, [(31, 500)] * 64, page_tokens=40).form == GENERAL
+    assert attention_plan(8, 8, [(31, 500), (32, 0)], page_tokens=40).form == PROMPT
 
 
 def test_lds_windows_are_raised_in_one_place():

@@ -1100,13 +1100,20 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     if (max_ssdz && s->ssd_z.ensure(Ts * max_ssdz * 4)) return kr_fail(KR_ERR_HIP, "state-space block scratch for %d tokens", T);
     for (SvRope& r : s->ropes) if (r.cs.ensure(Ts * (r.dims / 2) * 8)) return kr_fail(KR_ERR_HIP, "rope table");
     if (s->capture) { if (s->cap.ensure((size_t)c.n_layers * Ts * W * 4)) return kr_fail(KR_ERR_HIP, "capture buffer"); s->cap_T = T; }
-    std::vector<KrSvAttnPlan> plan(c.n_layers, KrSvAttnPlan{KR_SV_ATTN_GENERAL, 1, 0, 0, 0, 0});
+    std::vector<KrSvAttnPlan> plan(c.n_layers, KrSvAttnPlan{KR_SV_ATTN_GENERAL, 1, 0, 0, 0, 0, 0});
+    std::vector<char> join(c.n_layers, 0);
     for (int li = 0; li < c.n_layers; li++) {
         const SvLayer& l = s->L[li]; const kr_serve_layer& d = l.d;
         if (l.recurrent() || l.no_heads()) continue;
         const int ldk = l.latent() ? l.att_dim() : d.kv_heads * d.dim, ldv = l.latent() ? l.att_dim() : d.kv_heads * d.vdim;
         const int ldq = l.latent() ? d.heads * l.att_dim() : d.proj_conv ? (int)l.pconv_c() : l.n_h;
         plan[li] = kr_sv_attn_form(n_entries, counts, last_pos.data(), d.heads, l.att_heads_kv(), l.att_dim(), l.att_vdim(), ldk, ldv, ldq, PT, s->f32, d.window, d.keep_first, d.chunk);
+        // decode steps of a parallel block with experts: the branches share launches (kr_serve_step.hip)
+        if (!s->f32 && !seq && plan[li].form == KR_SV_ATTN_STEP && !l.latent() && !l.has_side() && d.mlp_kind == KR_SERVE_MLP_MOE && d.expert_act != KR_SERVE_ACT_RELU2 &&
+            kr_sv_step_join_fits(T, W, l.o_cols(), d.experts, d.top, d.groups, d.expert_ff, d.dim)) {
+            join[li] = 1;
+            plan[li].nsplit = kr_sv_step_join_splits(T, d.heads, d.kv_heads, plan[li].keys, W, d.expert_ff, d.experts, d.top);
+        }
         if (plan[li].parts && (s->part_ml.ensure(plan[li].parts * 8) || s->part_acc.ensure(plan[li].parts * l.att_vdim() * 4))) return kr_fail(KR_ERR_HIP, "attention split scratch");
     }
     const bool want_amax = argmax_out != nullptr;
@@ -1321,8 +1328,10 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
                 a.qkv = (float*)s->qkv2.p; a.ldq = l.pconv_c(); a.q_bias = a.k_bias = a.v_bias = nullptr;
             }
             if (d.qk_unit_norm == KR_SERVE_QKNORM_WHOLE) { Timer tm(s, 2); kr_sv_qk_rms(a, st); }
-            { Timer tm(s, 2); kr_sv_qk_prep(a, s->f32, st); }
-            { Timer tm(s, 3); kr_sv_attention(a, s->f32, st); }
+            if (!join[li]) {
+                { Timer tm(s, 2); kr_sv_qk_prep(a, s->f32, st); }
+                { Timer tm(s, 3); kr_sv_attention(a, s->f32, st); }
+            }
         } else {
             // queries: norm the latent, W_uq (or as projected), turn the rotated part, fold W_uk of every head into the plain part; keys / values: the normed latent and the
             // turned shared part are the cache row, read by the attention kernels as ONE key / value head whose values are the leading kv_rank of the key row
@@ -1412,7 +1421,8 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         }
         g = KrSvGemm{};
         g.A = o_in; g.lda = l.latent() ? d.heads * d.vdim : l.o_cols(); g.W = l.o.p; g.C = (float*)s->mix.p; g.ldc = W; g.M = T; g.N = W; g.K = g.lda;
-        { Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); }
+        const KrSvGemm og = g;
+        if (!join[li]) { Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); }
         if (seq) {
             // the mixer's sublayer ends here; the new x, normed or as it is, is the feed-forward's input (or the next layer's when there is none)
             res_layer = &l; res_run = &run; res_gate_kind = 1; res_to_mixer = !has_ff && !side;
@@ -1440,22 +1450,40 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
             }
             int* seg = mi; int* src_row = seg + E + 1; int* row_group = src_row + P; int* pp = row_group + P; int* hist = pp + 2 * P;
             float* row_w = d.expert_in_weight ? (float*)(pp + P) : nullptr;
+            KrSvRoute ro{};
+            ro.z = hz + l.off_router; ro.ld = l.n_h; ro.parts = s->f32 ? 1 : 2; ro.bias = d.router_bias ? (const float*)l.router_b.p : nullptr; ro.bias_mode = d.router_bias;
+            ro.score_kind = d.router_score; ro.group_kind = d.group_score; ro.T = T; ro.E = E; ro.top = top; ro.groups = d.groups; ro.keep = d.keep; ro.renorm = d.renorm;
+            ro.ids = (int*)s->ids.p; ro.wts = (float*)s->wts.p; ro.seg = seg; ro.src_row = src_row; ro.row_group = row_group; ro.pair_pos = pp; ro.row_w = row_w;
             {
                 Timer tm(s, 4);
-                kr_sv_router_sort(hz + l.off_router, l.n_h, s->f32 ? 1 : 2, d.router_bias ? (const float*)l.router_b.p : nullptr, d.router_bias, d.router_score, d.group_score, T, E, top, d.groups,
-                                  d.keep, d.renorm, (int*)s->ids.p, (float*)s->wts.p, hist, seg, src_row, row_group, pp, row_w, st);
+                if (!join[li] || !kr_sv_prep_route(a, ro, s->f32, st)) {
+                    kr_sv_router_sort(ro, hist, st);
+                    if (join[li]) kr_sv_qk_prep(a, s->f32, st);
+                }
             }
             KrSvGemm dn{}; dn.W = l.edown.p; dn.w_stride = (size_t)W * F; dn.C = (float*)s->rows.p; dn.ldc = W; dn.M = P; dn.N = W; dn.K = F;
             dn.seg = seg; dn.row_group = row_group; dn.n_groups = E;
             g = KrSvGemm{}; g.A = s->h.p; g.lda = W; g.W = l.egu.p; g.w_stride = (size_t)2 * F * W; g.C = (float*)s->gu.p; g.ldc = 2 * F; g.M = P; g.N = 2 * F; g.K = W;
             g.a_rows = src_row; g.seg = seg; g.row_group = row_group; g.n_groups = E;
-            const bool formed = pair_up(g, dn, g.C, 2 * F, 0, F, d.expert_act, d.expert_limit, d.expert_alpha, row_w);
-            { Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); }
-            down_ready(dn, (const float*)s->gu.p, 2 * F, P, F, d.expert_act, d.expert_limit, d.expert_alpha, row_w, formed);
-            if (beside) { down_ready(ffd, hz + l.off_gu, l.n_h, T, ff_f, ff_act, ff_limit, ff_alpha); shared = (const float*)s->ffout.p; }
-            {
+            if (join[li]) {
+                g.glu_out = s->y.p; g.glu_f = F; g.glu_kind = d.expert_act; g.glu_limit = d.expert_limit; g.glu_alpha = d.expert_alpha; g.glu_row_w = row_w;
+                { Timer tm(s, 3); kr_sv_attn_up(a, g, st); if (a.nsplit > 1) kr_sv_attn_merge(a, st); }
+                down_ready(dn, nullptr, 0, P, F, d.expert_act, d.expert_limit, d.expert_alpha, row_w, true);
+                KrSvGemm sh{};
+                if (beside) { down_ready(ffd, hz + l.off_gu, l.n_h, T, ff_f, ff_act, ff_limit, ff_alpha); shared = (const float*)s->ffout.p; }
                 Timer tm(s, 1);
-                if (!beside || !kr_sv_gemm_pair(dn, ffd, s->f32, st)) { kr_sv_gemm(dn, s->f32, st); if (beside) kr_sv_gemm(ffd, s->f32, st); }
+                if (beside && kr_sv_gemm_skinny_fits(ffd)) sh = ffd;
+                else if (beside) kr_sv_gemm(ffd, s->f32, st);
+                kr_sv_downs(og, dn, sh, st);
+            } else {
+                const bool formed = pair_up(g, dn, g.C, 2 * F, 0, F, d.expert_act, d.expert_limit, d.expert_alpha, row_w);
+                { Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); }
+                down_ready(dn, (const float*)s->gu.p, 2 * F, P, F, d.expert_act, d.expert_limit, d.expert_alpha, row_w, formed);
+                if (beside) { down_ready(ffd, hz + l.off_gu, l.n_h, T, ff_f, ff_act, ff_limit, ff_alpha); shared = (const float*)s->ffout.p; }
+                {
+                    Timer tm(s, 1);
+                    if (!beside || !kr_sv_gemm_pair(dn, ffd, s->f32, st)) { kr_sv_gemm(dn, s->f32, st); if (beside) kr_sv_gemm(ffd, s->f32, st); }
+                }
             }
             rows = (const float*)s->rows.p; pair_pos = pp;
         }

@@ -147,7 +147,7 @@ struct KrSvAttn {
 };
 enum { KR_SV_ATTN_GENERAL = 0, KR_SV_ATTN_PROMPT = 1, KR_SV_ATTN_STEP = 2 };      // the last two keep their running maxima in powers of two
 // which form a layer takes in a step, and how many workgroups share a token's keys
-struct KrSvAttnPlan { int form, nsplit, few, n_few, nsplit_few; size_t parts; };  // parts: partial states [heads] that split launches leave (part_ml holds 2 floats of each, part_acc vdim)
+struct KrSvAttnPlan { int form, nsplit, few, n_few, nsplit_few, keys; size_t parts; };  // keys: the most that a token of the step sees; parts: partial states [heads] that split launches leave (part_ml holds 2 floats of each, part_acc vdim)
 KrSvAttnPlan kr_sv_attn_form(int n_entries, const int* counts, const int* last_pos /* of every entry */, int heads, int kv_heads, int dim, int vdim, int ldk, int ldv, int ldq, int page_tokens, bool f32,
                              int window, int keep, int chunk);
 // the 128-row form of a bf16 store (kr_serve_attn.hip): sizes and strides it takes; its key splits
@@ -174,8 +174,22 @@ void kr_sv_attention(const KrSvAttn& a, bool f32, hipStream_t st);   // windowed
 // The pairs then sorted by expert: seg[E + 1], src_row[T * top] (token of sorted row), row_group[T * top], pair_pos[T * top] (sorted row of (token, slot)); with row_w also
 // the weight of every sorted row.  hist: kr_sv_moe_hist_ints(T * top, E) integers of scratch.
 size_t kr_sv_moe_hist_ints(int pairs, int E);
-void kr_sv_router_sort(const float* z, int ld, int parts, const float* bias, int bias_mode, int score_kind, int group_kind, int T, int E, int top, int groups, int keep, int renorm, int* ids,
-                       float* wts, int* hist, int* seg, int* src_row, int* row_group, int* pair_pos, float* row_w, hipStream_t st);
+struct KrSvRoute {
+    const float* z; int ld, parts;                       // [T, ld] f32, `parts` column blocks of E that are added
+    const float* bias; int bias_mode, score_kind, group_kind, T, E, top, groups, keep, renorm;
+    int* ids; float* wts;                                // [T, top] the choice
+    int* seg; int* src_row; int* row_group; int* pair_pos; float* row_w;
+};
+void kr_sv_router_sort(const KrSvRoute& r, int* hist, hipStream_t st);
+// kr_sv_qk_prep and kr_sv_router_sort of a block whose attention and router read one product, in one launch (at most 16 tokens); false: nothing was launched
+bool kr_sv_prep_route(const KrSvAttn& a, const KrSvRoute& r, bool f32, hipStream_t st);
+// Decode steps of a parallel block with experts, bf16 (kr_serve_step.hip): attention beside the experts' gate and up product (up: glu fields set, columns [0, 2 glu_f)), then
+// attention's output projection, the experts' down projection (of up.glu_out) and the shared expert's in one launch.  join_fits: shapes; join_splits: attention's key splits there.
+bool kr_sv_step_join_fits(int T, int width, int o_cols, int experts, int top, int groups, int ff, int dim);
+int kr_sv_step_join_splits(int T, int heads, int kv_heads, int max_visible, int width, int ff, int experts, int top);
+void kr_sv_attn_up(const KrSvAttn& a, const KrSvGemm& up, hipStream_t st);
+void kr_sv_downs(const KrSvGemm& o, const KrSvGemm& e, const KrSvGemm& sh, hipStream_t st);
+void kr_sv_attn_merge(const KrSvAttn& a, hipStream_t st);      // the partial states of a launch with splits
 // gu rows `ld` floats apart (gate at [0, F), up at [F, 2F)) -> y [M, F] storage type; row_w [M] or null: multiplies a row's gate and up columns first
 // up_tab: the up factor of (row r, column c) is up_tab[up_rows[r] * up_ld + up_off + c] (storage type) instead of gu's second half
 void kr_sv_act(const float* gu, int ld, void* y, bool f32, int M, int F, int kind, float limit, float alpha, const float* row_w, hipStream_t st, const void* up_tab = nullptr,

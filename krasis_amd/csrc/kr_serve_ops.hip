@@ -347,10 +347,9 @@ __global__ void sv_rope_table_kernel(const int* __restrict__ pos, const double* 
 
 // one wave per (token, head): the head vector is staged in LDS, rotated and normed there; q heads are written back in place, k heads go to the
 // cache page of (slot, position), v heads are copied there
+__device__ __forceinline__ void sv_wave_sync() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront"); }
 template <typename T>
-__global__ void __launch_bounds__(64) sv_qk_prep_kernel(const KrSvAttn a) {
-    extern __shared__ float hv[];            // [dim]
-    const int t = blockIdx.x, hh = blockIdx.y, lane = threadIdx.x;
+__device__ __forceinline__ void sv_qk_prep_row(const KrSvAttn& a, const int t, const int hh, const int lane, float* hv /* [dim], the wave's own */) {
     const int H = a.heads, G = a.kv_heads;
     const int p = a.pos[t], sl = a.slot[t];
     float* row = a.qkv + (size_t)t * a.ldq;
@@ -374,13 +373,13 @@ __global__ void __launch_bounds__(64) sv_qk_prep_kernel(const KrSvAttn a) {
         }
         return;
     }
- float* v = row + (size_t)hh * a.dim;
+    float* v = row + (size_t)hh * a.dim;
     {
         const float* bias = hh < H ? a.q_bias : a.k_bias;
         if (bias) bias += (size_t)(hh < H ? hh : hh - H) * a.dim;
         for (int d = lane; d < a.dim; d += 64) hv[d] = bias ? v[d] + bias[d] : v[d];
     }
-    __syncthreads();
+    sv_wave_sync();
     if (a.v_from_k && hh >= H) {             // the value row of this key head: the key as projected
         T* dst = (T*)a.vpool + prow * a.ldv + (size_t)(hh - H) * a.dim;
         for (int d = lane; d < a.dim; d += 64) sv_st(dst + d, hv[d]);
@@ -389,7 +388,7 @@ __global__ void __launch_bounds__(64) sv_qk_prep_kernel(const KrSvAttn a) {
         const float inv3 = a.inv_rms[(size_t)t * 2 + (hh < H ? 0 : 1)];
         const float* w = hh < H ? a.q_norm_w + (size_t)hh * a.dim : a.k_norm_w + (size_t)(hh - H) * a.dim;
         for (int d = lane; d < a.dim; d += 64) hv[d] = hv[d] * inv3 * w[d];
-        __syncthreads();
+        sv_wave_sync();
     }
     if (a.unit_norm == 2) {                  // weighted, before the rotation
         const float* w = hh < H ? a.q_norm_w : a.k_norm_w;
@@ -398,7 +397,7 @@ __global__ void __launch_bounds__(64) sv_qk_prep_kernel(const KrSvAttn a) {
         s2 = sv_wave_sum(s2);
         const float inv2 = 1.0f / sqrtf(s2 / (float)a.dim + a.eps);
         for (int d = lane; d < a.dim; d += 64) hv[d] = hv[d] * inv2 * w[d];
-        __syncthreads();
+        sv_wave_sync();
     }
     const int half = a.rot_dims / 2;
     const float2* cs = a.cs + (size_t)t * half;
@@ -414,7 +413,7 @@ __global__ void __launch_bounds__(64) sv_qk_prep_kernel(const KrSvAttn a) {
     for (int d = a.rot_dims + lane; d < a.dim; d += 64) ss = __builtin_fmaf(hv[d], hv[d], ss);
     ss = sv_wave_sum(ss);
     const float inv = a.unit_norm == 1 ? 1.0f / sqrtf(ss / (float)a.dim + a.eps) : 1.0f;
-    __syncthreads();
+    sv_wave_sync();
     if (hh < H) {
         for (int d = lane; d < a.dim; d += 64) v[d] = hv[d] * inv;
     } else {
@@ -422,6 +421,11 @@ __global__ void __launch_bounds__(64) sv_qk_prep_kernel(const KrSvAttn a) {
         T* dst = (T*)a.kpool + prow * a.ldk + (size_t)g * a.dim;
         for (int d = lane; d < a.dim; d += 64) sv_st(dst + d, hv[d] * inv);
     }
+}
+template <typename T>
+__global__ void __launch_bounds__(64) sv_qk_prep_kernel(const KrSvAttn a) {
+    extern __shared__ float hv[];            // [dim]
+    sv_qk_prep_row<T>(a, blockIdx.x, blockIdx.y, threadIdx.x, hv);
 }
 
 // Windowed attention with a sink over the paged cache.  One workgroup (four waves) per (token, key / value head, batch of RM query heads of that
@@ -975,16 +979,18 @@ __global__ void __launch_bounds__(64) sv_router_select_kernel(const float* __res
 // NaN and minus infinity never chosen), same sums.  SORT: a decode step's tokens are one workgroup's waves (T <= 16), which then sorts their rows by expert in the same launch.
 // 64 experts, top 6: one token 12.4 + 4.7 us as two launches -> 4.0, twelve 12.8 + 4.6 -> 7.0, 4096 (choice alone) 25 -> 12.
 template <int NV, bool SORT>
-__global__ void __launch_bounds__(SORT ? 1024 : 256) sv_router_rank_kernel(const float* __restrict__ z, int ld, int parts, const float* __restrict__ bias, int bias_mode, int score_kind,
-                                                                          int group_kind, int T, int E, int top, int groups, int keep, int renorm, int* __restrict__ ids, float* __restrict__ wts,
-                                                                          int* __restrict__ seg, int* __restrict__ src_row, int* __restrict__ row_group, int* __restrict__ pair_pos,
-                                                                          float* __restrict__ row_w) {
+__device__ __forceinline__ void sv_router_rank(const KrSvRoute& ro, const int bx) {
+    const float* __restrict__ z = ro.z; const float* __restrict__ bias = ro.bias;
+    const int ld = ro.ld, parts = ro.parts, bias_mode = ro.bias_mode, score_kind = ro.score_kind, group_kind = ro.group_kind, T = ro.T, E = ro.E, top = ro.top, groups = ro.groups, keep = ro.keep,
+              renorm = ro.renorm;
+    int* __restrict__ ids = ro.ids; float* __restrict__ wts = ro.wts; int* __restrict__ seg = ro.seg; int* __restrict__ src_row = ro.src_row; int* __restrict__ row_group = ro.row_group;
+    int* __restrict__ pair_pos = ro.pair_pos; float* __restrict__ row_w = ro.row_w;
     constexpr int NWAVES = SORT ? 16 : 4;
     __shared__ float gsc[NWAVES][64];                       // choice scores by expert while groups are scored (one wave's 64 at a time), then the groups' scores
     __shared__ float cho[NWAVES][64 * NV];
     __shared__ int s_ids[SORT ? 16 * 64 : 1]; __shared__ float s_w[SORT ? 16 * 64 : 1];
     __shared__ int cnt[SORT ? 128 : 1];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = blockIdx.x * NWAVES + wave;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = bx * NWAVES + wave;
     if (SORT) { if (threadIdx.x < 128) cnt[threadIdx.x] = 0; }
     if (t < T) {
         float s[NV], c[NV];
@@ -1094,6 +1100,18 @@ __global__ void __launch_bounds__(SORT ? 1024 : 256) sv_router_rank_kernel(const
         src_row[pos] = i / top; row_group[pos] = e; pair_pos[i] = pos;
         if (row_w) row_w[pos] = s_w[i];
     }
+}
+template <int NV, bool SORT>
+__global__ void __launch_bounds__(SORT ? 1024 : 256) sv_router_rank_kernel(const KrSvRoute ro) { sv_router_rank<NV, SORT>(ro, blockIdx.x); }
+
+// A parallel block's router reads the same product as its queries and keys: at decode sizes one launch does both, workgroup 0 the choice and the sort, the others sixteen
+// (token, head) rows each.  A launch that depends on the one before it costs 4 - 5 us here whatever it does: one request 4.7 + 4.7 us as two launches, now 5.2.
+template <typename T, int NV>
+__global__ void __launch_bounds__(1024) sv_prep_route_kernel(const KrSvAttn a, const KrSvRoute ro, int heads_per_token) {
+    extern __shared__ float hv16[];          // [16][dim]
+    if (blockIdx.x == 0) { sv_router_rank<NV, true>(ro, 0); return; }
+    const int wave = threadIdx.x >> 6, i = (blockIdx.x - 1) * 16 + wave;
+    if (i < a.T * heads_per_token) sv_qk_prep_row<T>(a, i / heads_per_token, i % heads_per_token, threadIdx.x & 63, hv16 + wave * a.dim);
 }
 
 // Rows of a prompt's pairs sorted by expert, without atomics on a few hot words of memory (64 counters for 24576 pairs: 39 us to count and 39 us to place): a block counts its
@@ -2319,6 +2337,7 @@ KrSvAttnPlan kr_sv_attn_form(int n_entries, const int* counts, const int* last_p
         return q;
     };
     const Part all = part(1, INT_MAX), below = part(1, 31);
+    p.keys = all.keys;
     // (where the tiles do not fit, no form shares a token's keys with the next token)
     const int few = !prompt || (long)below.tokens * kv_heads * ((heads / kv_heads + 15) / 16) <= 192 ? 31 : 1;
     const Part a = part(1, few), b = part(few + 1, INT_MAX);
@@ -2372,6 +2391,10 @@ static bool sv_attn_mfma_launch(const KrSvAttn& a, hipStream_t st) {
     return false;
 }
 
+void kr_sv_attn_merge(const KrSvAttn& a, hipStream_t st) {
+    hipLaunchKernelGGL(sv_attn_merge_kernel<uint16_t>, dim3(a.T, a.heads), dim3(256), (size_t)(a.nsplit + 1) * sizeof(float), st, a);
+}
+
 void kr_sv_attention(const KrSvAttn& a, bool f32, hipStream_t st) {
     if (a.T <= 0) return;
     if (a.form != KR_SV_ATTN_GENERAL) {
@@ -2416,20 +2439,22 @@ void kr_sv_attention(const KrSvAttn& a, bool f32, hipStream_t st) {
 
 size_t kr_sv_moe_hist_ints(int pairs, int E) { return pairs <= 1024 && E <= 4096 ? 0 : ((size_t)pairs + SORT_PAIRS - 1) / SORT_PAIRS * E; }
 
-void kr_sv_router_sort(const float* z, int ld, int parts, const float* bias, int bias_mode, int score_kind, int group_kind, int T, int E, int top, int groups, int keep, int renorm, int* ids,
-                       float* wts, int* hist, int* seg, int* src_row, int* row_group, int* pair_pos, float* row_w, hipStream_t st) {
-    const int n = T * top;
+static bool sv_route_ranked(const KrSvRoute& r) { return r.E <= 128 && r.top <= 64 && r.groups <= 64; }
+
+void kr_sv_router_sort(const KrSvRoute& r, int* hist, hipStream_t st) {
+    const int T = r.T, E = r.E, top = r.top, groups = r.groups, n = T * top;
+    int *ids = r.ids, *seg = r.seg, *src_row = r.src_row, *row_group = r.row_group, *pair_pos = r.pair_pos; float *wts = r.wts, *row_w = r.row_w;
     if (n <= 0) return;
-    const bool ranked = E <= 128 && top <= 64 && groups <= 64;
-#define SV_RANK(NV_, SORT_, GRID_, NT_) hipLaunchKernelGGL((sv_router_rank_kernel<NV_, SORT_>), dim3(GRID_), dim3(NT_), 0, st, z, ld, parts, bias, bias_mode, score_kind, group_kind, T, E, top, groups, \
-                                                           keep, renorm, ids, wts, seg, src_row, row_group, pair_pos, row_w)
-    if (ranked && T <= 16) {                 // a wave per token, the sort in the same launch
-        if (E <= 64) SV_RANK(1, true, 1, 1024); else SV_RANK(2, true, 1, 1024);
+    if (sv_route_ranked(r) && T <= 16) {                 // a wave per token, the sort in the same launch
+        if (E <= 64) hipLaunchKernelGGL((sv_router_rank_kernel<1, true>), dim3(1), dim3(1024), 0, st, r);
+        else hipLaunchKernelGGL((sv_router_rank_kernel<2, true>), dim3(1), dim3(1024), 0, st, r);
         return;
     }
-    if (ranked) { if (E <= 64) SV_RANK(1, false, (T + 3) / 4, 256); else SV_RANK(2, false, (T + 3) / 4, 256); }
-    else hipLaunchKernelGGL(sv_router_select_kernel, dim3(T), dim3(64), (size_t)(2 * E + 2 * groups) * sizeof(float), st, z, ld, parts, bias, bias_mode, score_kind, group_kind, E, top, groups, keep, renorm, ids, wts);
-#undef SV_RANK
+    if (sv_route_ranked(r)) {
+        if (E <= 64) hipLaunchKernelGGL((sv_router_rank_kernel<1, false>), dim3((T + 3) / 4), dim3(256), 0, st, r);
+        else hipLaunchKernelGGL((sv_router_rank_kernel<2, false>), dim3((T + 3) / 4), dim3(256), 0, st, r);
+    } else hipLaunchKernelGGL(sv_router_select_kernel, dim3(T), dim3(64), (size_t)(2 * E + 2 * groups) * sizeof(float), st, r.z, r.ld, r.parts, r.bias, r.bias_mode, r.score_kind, r.group_kind, E, top,
+                              groups, r.keep, r.renorm, ids, wts);
     if (n <= 1024 && E <= 4096) {
         hipLaunchKernelGGL(sv_moe_sort_small_kernel, dim3(1), dim3(256), (size_t)E * sizeof(int), st, ids, n, top, E, seg, src_row, row_group, pair_pos, wts, row_w);
         return;
@@ -2438,6 +2463,18 @@ void kr_sv_router_sort(const float* z, int ld, int parts, const float* bias, int
     hipLaunchKernelGGL(sv_moe_count_kernel, dim3(blocks), dim3(256), (size_t)E * sizeof(int), st, ids, n, E, hist);
     hipLaunchKernelGGL(sv_moe_scan_kernel, dim3(1), dim3(1024), 0, st, hist, blocks, E, seg);
     hipLaunchKernelGGL(sv_moe_fill_kernel, dim3(blocks), dim3(256), (size_t)E * sizeof(int), st, ids, n, top, E, hist, src_row, row_group, pair_pos, wts, row_w);
+}
+
+bool kr_sv_prep_route(const KrSvAttn& a, const KrSvRoute& r, bool f32, hipStream_t st) {
+    const int hpt = a.heads + (a.own_kv ? (a.v_from_k ? 1 : 2) * a.kv_heads : 0);
+    const size_t lds = (size_t)16 * a.dim * sizeof(float);
+    if (a.T != r.T || a.T <= 0 || a.T > 16 || r.top <= 0 || !sv_route_ranked(r) || lds > 32 * 1024) return false;
+    const dim3 grid(1 + (a.T * hpt + 15) / 16), nt(1024);
+#define SV_PR(T_, NV_) hipLaunchKernelGGL((sv_prep_route_kernel<T_, NV_>), grid, nt, lds, st, a, r, hpt)
+    if (r.E <= 64) { if (f32) SV_PR(float, 1); else SV_PR(uint16_t, 1); }
+    else { if (f32) SV_PR(float, 2); else SV_PR(uint16_t, 2); }
+#undef SV_PR
+    return true;
 }
 
 void kr_sv_act(const float* gu, int ld, void* y, bool f32, int M, int F, int kind, float limit, float alpha, const float* row_w, hipStream_t st, const void* up_tab,

@@ -12,121 +12,21 @@
 #include <algorithm>
 
 #include "kr_lds_optin.h"
-#include "kr_serve_gemm_dev.h"
+#include "kr_serve_strip_dev.h"
 
 namespace {
-typedef float sk_f4 __attribute__((ext_vector_type(4)));
-
-template <int MB, int NB, int WV, bool ACT>               // row blocks of 16, column blocks of 16, waves
-__device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int by) {      // by: problem row of a grouped problem
-    constexpr int U = NB * MB <= 2 ? 8 : 4;                   // k steps requested together
-    constexpr int TR = MB * NB < 4 ? MB * NB : 4;             // output tiles per round of the reduction
-    __shared__ __attribute__((aligned(16))) float red[WV][TR][256];
-    extern __shared__ __attribute__((aligned(16))) uint16_t act[];      // ACT: the rows' activation [16 MB][K + 8]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4, n0 = blockIdx.x * 16 * NB;
-    int lo = 0, hi = g.M, N = g.N;
-    const uint16_t* W = (const uint16_t*)g.W;
-    if (g.row_group) {
-        const int group = g.row_group[by];
-        lo = g.seg[group];
-        if (lo != by) return;
-        hi = g.seg[group + 1];
-        W += (size_t)group * g.w_stride; N = gm_cols(g, group);
-    }
-    if (n0 >= N) return;
-    const int ks = g.K / 32, s0 = ks * wave / WV, s1 = ks * (wave + 1) / WV, lda = g.K + 8;
-    const uint16_t* wp[NB];
-#pragma unroll
-    for (int b = 0; b < NB; b++) wp[b] = W + (size_t)min(n0 + b * 16 + r, N - 1) * g.K + q * 8;
-    auto request = [&](gu4 (&wv)[U][NB], int s) {
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int k = min(s + u, s1 - 1) * 32;             // steps past the wave's last one are requested again and not multiplied
-#pragma unroll
-            for (int b = 0; b < NB; b++) wv[u][b] = *reinterpret_cast<const gu4*>(wp[b] + k);
-        }
-    };
-    for (int m0 = lo; m0 < hi; m0 += 16 * MB) {
-        const uint16_t* ap[MB];
-        gu4 wv[U][NB];
-        if constexpr (ACT) {
-            if (s0 < s1) request(wv, s0);                      // the weights' first strip travels while the activation is formed
-            const int rows = min(16 * MB, hi - m0), kv = g.K / 4;
-            const int uoff = g.act_kind == KR_SV_ACT_RELU2 || g.up_tab ? 0 : g.K;      // no up columns (un-gated, or taken from a table): the second read repeats the first
-            for (int i = tid; i < rows * kv; i += 64 * WV) {
-                const int m = i / kv, k = (i - m * kv) * 4, src = g.a_rows ? g.a_rows[m0 + m] : m0 + m;
-                const float w = g.act_row_w ? g.act_row_w[m0 + m] : 1.0f;
-                const float* gp = g.act_gu + (size_t)src * g.act_ld + k;
-                const float4 gg = *reinterpret_cast<const float4*>(gp);
-                float4 uu = *reinterpret_cast<const float4*>(gp + uoff);
-                if (g.up_tab) {
-                    const uint16_t* t = (const uint16_t*)g.up_tab + (size_t)g.up_rows[m0 + m] * g.up_ld + g.up_off + k;
-                    uu = make_float4(gm_ld(t), gm_ld(t + 1), gm_ld(t + 2), gm_ld(t + 3));
-                }
-                const uint32_t x0 = kr_f32_to_bf16(gm_act(gg.x * w, uu.x * w, g.act_kind, g.act_limit, g.act_alpha)), x1 = kr_f32_to_bf16(gm_act(gg.y * w, uu.y * w, g.act_kind, g.act_limit, g.act_alpha));
-                const uint32_t x2 = kr_f32_to_bf16(gm_act(gg.z * w, uu.z * w, g.act_kind, g.act_limit, g.act_alpha)), x3 = kr_f32_to_bf16(gm_act(gg.w * w, uu.w * w, g.act_kind, g.act_limit, g.act_alpha));
-                *reinterpret_cast<uint2*>(&act[m * lda + k]) = make_uint2(x0 | (x1 << 16), x2 | (x3 << 16));
-            }
-            __syncthreads();
-        }
-#pragma unroll
-        for (int a = 0; a < MB; a++) {
-            const int m = min(m0 + a * 16 + r, hi - 1), src = g.a_rows ? g.a_rows[m] : m;
-            ap[a] = ACT ? act + (m - m0) * lda + q * 8 : (const uint16_t*)g.A + (size_t)src * g.lda + q * 8;
-        }
-        sk_f4 acc[MB][NB];
-#pragma unroll
-        for (int a = 0; a < MB; a++)
-#pragma unroll
-            for (int b = 0; b < NB; b++) acc[a][b] = sk_f4{0.0f, 0.0f, 0.0f, 0.0f};
-        for (int s = s0; s < s1; s += U) {
-            if (!ACT || s > s0) request(wv, s);
-            gu4 av[U][MB];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int k = min(s + u, s1 - 1) * 32;
-#pragma unroll
-                for (int a = 0; a < MB; a++) av[u][a] = *reinterpret_cast<const gu4*>(ap[a] + k);
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                if (s + u < s1) {
-#pragma unroll
-                    for (int a = 0; a < MB; a++)
-#pragma unroll
-                        for (int b = 0; b < NB; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gb8, wv[u][b]), __builtin_bit_cast(gb8, av[u][a]), acc[a][b], 0, 0, 0);
-                }
-            }
-        }
-        // the waves' partial sums meet, TR tiles of 16 x 16 at a time: tile element (row r, column c) at r * 16 + c, a lane holds four columns of one row
-#pragma unroll
-        for (int t0 = 0; t0 < MB * NB; t0 += TR) {
-            if (t0 > 0) __syncthreads();
-#pragma unroll
-            for (int t = 0; t < TR; t++) {
-                const sk_f4 v = acc[(t0 + t) / NB][(t0 + t) % NB];
-                *reinterpret_cast<float4*>(&red[wave][t][r * 16 + q * 4]) = make_float4(v[0], v[1], v[2], v[3]);
-            }
-            __syncthreads();
-            for (int i = tid; i < TR * 256; i += 64 * WV) {
-                const int t = i >> 8, e = i & 255, m = m0 + ((t0 + t) / NB) * 16 + (e >> 4), n = n0 + ((t0 + t) % NB) * 16 + (e & 15);
-                if (m >= hi || n >= N) continue;
-                float v = red[0][t][e];
-#pragma unroll
-                for (int w = 1; w < WV; w++) v += red[w][t][e];
-                gm_store<true>(g, m, n, v);
-            }
-        }
-        if (m0 + 16 * MB < hi) __syncthreads();
-    }
-}
-
 template <int MB, int NB, int WV, bool ACT>
-__global__ void __launch_bounds__(64 * WV) sv_skinny_kernel(const KrSvGemm g) { sk_strip<MB, NB, WV, ACT>(g, blockIdx.y); }
+__global__ void __launch_bounds__(64 * WV) sv_skinny_kernel(const KrSvGemm g) {
+    __shared__ __attribute__((aligned(16))) float red[sk_red_floats(MB, NB, WV)];
+    extern __shared__ __attribute__((aligned(16))) uint16_t act[];
+    sk_strip<MB, NB, WV, ACT>(g, blockIdx.x, blockIdx.y, red, act);
+}
 // the experts' and the shared expert's down projection of a step in one launch, both with the activation inside: neither fills the chip, and a launch with its gap costs more
 // than the smaller of the two (six expert rows and one row, 2048 x 768: 8.1 + 6.3 -> 8.7 us)
 __global__ void __launch_bounds__(256) sv_skinny_pair_kernel(const KrSvGemm e, const KrSvGemm o) {
-    if (blockIdx.y == 0) sk_strip<1, 1, 4, true>(o, 0); else sk_strip<1, 1, 4, true>(e, blockIdx.y - 1);
+    __shared__ __attribute__((aligned(16))) float red[sk_red_floats(1, 1, 4)];
+    extern __shared__ __attribute__((aligned(16))) uint16_t act[];
+    if (blockIdx.y == 0) sk_strip<1, 1, 4, true>(o, blockIdx.x, 0, red, act); else sk_strip<1, 1, 4, true>(e, blockIdx.x, blockIdx.y - 1, red, act);
 }
 
 int sk_act_lds(const KrSvGemm& g) { return (g.row_group ? 16 : std::min(16, g.M)) * (g.K + 8) * 2; }      // one block of sixteen rows

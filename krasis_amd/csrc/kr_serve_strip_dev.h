@@ -1,0 +1,167 @@
+// kr_serve_strip_dev.h -- a workgroup's strip of columns of C[M, N] = A[M, K] x W[N, K]^T for few rows, bf16 (kr_serve_skinny.hip has the reasons), shared by the
+// launches of one product and the launches that put several products, or a product and attention, side by side (kr_serve_step.hip).
+#ifndef KR_SERVE_STRIP_DEV_H
+#define KR_SERVE_STRIP_DEV_H
+#include "kr_serve_gemm_dev.h"
+
+typedef float sk_f4 __attribute__((ext_vector_type(4)));
+
+constexpr int sk_red_floats(int MB, int NB, int WV) { return WV * (MB * NB < 4 ? MB * NB : 4) * 256; }
+
+// MB, NB: row and column blocks of 16; WV: waves.  bx: strip, by: problem row of a grouped problem; red: sk_red_floats of LDS, act (with ACT): the rows' activation [16 MB][K + 8].
+// GLU (NB = 2): the strip is 16 gate columns of g.glu_f and the 16 up columns that belong to them; their activation goes to g.glu_out, nothing to C.
+template <int MB, int NB, int WV, bool ACT, bool GLU = false>
+__device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const int by, float* red, uint16_t* act) {
+    static_assert(!GLU || (NB == 2 && MB == 1), "a gate tile and its up tile");
+    constexpr int U = NB * MB <= 2 ? 8 : 4;                   // k steps requested together
+    constexpr int TR = MB * NB < 4 ? MB * NB : 4;             // output tiles per round of the reduction
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4, n0 = bx * 16 * (GLU ? 1 : NB);
+    int lo = 0, hi = g.M, N = g.N;
+    const uint16_t* W = (const uint16_t*)g.W;
+    if (g.row_group) {
+        const int group = g.row_group[by];
+        lo = g.seg[group];
+        if (lo != by) return;
+        hi = g.seg[group + 1];
+        W += (size_t)group * g.w_stride; N = gm_cols(g, group);
+    }
+    if (n0 >= (GLU ? g.glu_f : N)) return;
+    const int ks = g.K / 32, s0 = ks * wave / WV, s1 = ks * (wave + 1) / WV, lda = g.K + 8;
+    const uint16_t* wp[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) wp[b] = W + (size_t)(GLU ? min(n0 + r, g.glu_f - 1) + b * g.glu_f : min(n0 + b * 16 + r, N - 1)) * g.K + q * 8;
+    auto request = [&](gu4 (&wv)[U][NB], int s) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = min(s + u, s1 - 1) * 32;             // steps past the wave's last one are requested again and not multiplied
+#pragma unroll
+            for (int b = 0; b < NB; b++) wv[u][b] = *reinterpret_cast<const gu4*>(wp[b] + k);
+        }
+    };
+    for (int m0 = lo; m0 < hi; m0 += 16 * MB) {
+        const uint16_t* ap[MB];
+        gu4 wv[U][NB];
+        if constexpr (ACT) {
+            if (s0 < s1) request(wv, s0);                      // the weights' first strip travels while the activation is formed
+            const int rows = min(16 * MB, hi - m0), kv = g.K / 4;
+            const int uoff = g.act_kind == KR_SV_ACT_RELU2 || g.up_tab ? 0 : g.K;      // no up columns (un-gated, or taken from a table): the second read repeats the first
+            for (int i = tid; i < rows * kv; i += 64 * WV) {
+                const int m = i / kv, k = (i - m * kv) * 4, src = g.a_rows ? g.a_rows[m0 + m] : m0 + m;
+                const float w = g.act_row_w ? g.act_row_w[m0 + m] : 1.0f;
+                const float* gp = g.act_gu + (size_t)src * g.act_ld + k;
+                const float4 gg = *reinterpret_cast<const float4*>(gp);
+                float4 uu = *reinterpret_cast<const float4*>(gp + uoff);
+                if (g.up_tab) {
+                    const uint16_t* t = (const uint16_t*)g.up_tab + (size_t)g.up_rows[m0 + m] * g.up_ld + g.up_off + k;
+                    uu = make_float4(gm_ld(t), gm_ld(t + 1), gm_ld(t + 2), gm_ld(t + 3));
+                }
+                const uint32_t x0 = kr_f32_to_bf16(gm_act(gg.x * w, uu.x * w, g.act_kind, g.act_limit, g.act_alpha)), x1 = kr_f32_to_bf16(gm_act(gg.y * w, uu.y * w, g.act_kind, g.act_limit, g.act_alpha));
+                const uint32_t x2 = kr_f32_to_bf16(gm_act(gg.z * w, uu.z * w, g.act_kind, g.act_limit, g.act_alpha)), x3 = kr_f32_to_bf16(gm_act(gg.w * w, uu.w * w, g.act_kind, g.act_limit, g.act_alpha));
+                *reinterpret_cast<uint2*>(&act[m * lda + k]) = make_uint2(x0 | (x1 << 16), x2 | (x3 << 16));
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int a = 0; a < MB; a++) {
+            const int m = min(m0 + a * 16 + r, hi - 1), src = g.a_rows ? g.a_rows[m] : m;
+            ap[a] = ACT ? act + (m - m0) * lda + q * 8 : (const uint16_t*)g.A + (size_t)src * g.lda + q * 8;
+        }
+        sk_f4 acc[MB][NB];
+#pragma unroll
+        for (int a = 0; a < MB; a++)
+#pragma unroll
+            for (int b = 0; b < NB; b++) acc[a][b] = sk_f4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int s = s0; s < s1; s += U) {
+            if (!ACT || s > s0) request(wv, s);
+            gu4 av[U][MB];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int k = min(s + u, s1 - 1) * 32;
+#pragma unroll
+                for (int a = 0; a < MB; a++) av[u][a] = *reinterpret_cast<const gu4*>(ap[a] + k);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (s + u < s1) {
+#pragma unroll
+                    for (int a = 0; a < MB; a++)
+#pragma unroll
+                        for (int b = 0; b < NB; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gb8, wv[u][b]), __builtin_bit_cast(gb8, av[u][a]), acc[a][b], 0, 0, 0);
+                }
+            }
+        }
+        // the waves' partial sums meet, TR tiles of 16 x 16 at a time: tile element (row r, column c) at r * 16 + c, a lane holds four columns of one row
+#pragma unroll
+        for (int t0 = 0; t0 < MB * NB; t0 += TR) {
+            if (t0 > 0) __syncthreads();
+#pragma unroll
+            for (int t = 0; t < TR; t++) {
+                const sk_f4 v = acc[(t0 + t) / NB][(t0 + t) % NB];
+                *reinterpret_cast<float4*>(&red[(wave * TR + t) * 256 + r * 16 + q * 4]) = make_float4(v[0], v[1], v[2], v[3]);
+            }
+            __syncthreads();
+            if constexpr (GLU) {
+                for (int e = tid; e < 256; e += 64 * WV) {
+                    const int m = m0 + (e >> 4), n = n0 + (e & 15);
+                    if (m >= hi || n >= g.glu_f) continue;
+                    float gt = red[e], up = red[256 + e];
+#pragma unroll
+                    for (int w = 1; w < WV; w++) { gt += red[w * TR * 256 + e]; up += red[(w * TR + 1) * 256 + e]; }
+                    const float wt = g.glu_row_w ? g.glu_row_w[m] : 1.0f;
+                    ((uint16_t*)g.glu_out)[(size_t)m * g.glu_f + n] = kr_f32_to_bf16(gm_act_once(gt * wt, up * wt, g.glu_kind, g.glu_limit, g.glu_alpha));
+                }
+                continue;
+            }
+            for (int i = tid; i < TR * 256; i += 64 * WV) {
+                const int t = i >> 8, e = i & 255, m = m0 + ((t0 + t) / NB) * 16 + (e >> 4), n = n0 + ((t0 + t) % NB) * 16 + (e & 15);
+                if (m >= hi || n >= N) continue;
+                float v = red[t * 256 + e];
+#pragma unroll
+                for (int w = 1; w < WV; w++) v += red[(w * TR + t) * 256 + e];
+                gm_store<true>(g, m, n, v);
+            }
+        }
+        if (m0 + 16 * MB < hi) __syncthreads();
+    }
+}
+
+// The gate and up product of problem row `by` alone, columns [WV bx, WV bx + WV) of g.glu_f, one per wave, K over its lanes: for the rows of one or
+// two tokens, which meet an expert once.  A wave reads whole rows of the matrix and waits for nothing but its row's expert.
+template <int WV>
+__device__ __forceinline__ void sk_row_glu(const KrSvGemm& g, const int bx, const int by) {
+    constexpr int U = 4;                                      // 16-byte pieces of K requested together, of both matrices
+    const int lane = threadIdx.x & 63, n = bx * WV + (threadIdx.x >> 6);
+    if (n >= g.glu_f) return;
+    const uint16_t* W = (const uint16_t*)g.W + (size_t)g.row_group[by] * g.w_stride + (size_t)n * g.K;
+    const uint16_t* A = (const uint16_t*)g.A + (size_t)(g.a_rows ? g.a_rows[by] : by) * g.lda;
+    float gt = 0.0f, up = 0.0f;
+    for (int k0 = 0; k0 < g.K; k0 += 512 * U) {
+        gu4 wg[U], wu[U], av[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = min(k0 + 512 * u + lane * 8, g.K - 8);      // lanes past the row's end read its last piece and multiply it by zero
+            wg[u] = *reinterpret_cast<const gu4*>(W + k);
+            wu[u] = *reinterpret_cast<const gu4*>(W + (size_t)g.glu_f * g.K + k);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = k0 + 512 * u + lane * 8;
+            av[u] = *reinterpret_cast<const gu4*>(A + min(k, g.K - 8));
+            if (k >= g.K) av[u] = gu4{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float a0 = __uint_as_float(av[u][i] << 16), a1 = __uint_as_float(av[u][i] & 0xFFFF0000u);
+                gt = __builtin_fmaf(a0, __uint_as_float(wg[u][i] << 16), gt); gt = __builtin_fmaf(a1, __uint_as_float(wg[u][i] & 0xFFFF0000u), gt);
+                up = __builtin_fmaf(a0, __uint_as_float(wu[u][i] << 16), up); up = __builtin_fmaf(a1, __uint_as_float(wu[u][i] & 0xFFFF0000u), up);
+            }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) { gt += __shfl_xor(gt, o); up += __shfl_xor(up, o); }
+    const float wt = g.glu_row_w ? g.glu_row_w[by] : 1.0f;
+    if (lane == 0) ((uint16_t*)g.glu_out)[(size_t)by * g.glu_f + n] = kr_f32_to_bf16(gm_act_once(gt * wt, up * wt, g.glu_kind, g.glu_limit, g.glu_alpha));
+}
+
+#endif

@@ -1,0 +1,47 @@
+"""Decode steps of a parallel block with experts in a bf16 store, where attention and the experts share launches (csrc/kr_serve_step.hip), against the float64 restatement.
+
+The sizes are the edges of those launches: rows that are each taken alone (up to 24) and the next one, strips and columns that do not fill a workgroup, up to sixteen tokens, one
+and several shares of a token's keys, one and two batches of sixteen query heads, more than 64 experts.  Tolerance: that of the store's other bf16 tests (test_serve_gpu.py)."""
+import numpy as np
+import pytest
+
+from tests import oracle_serve as O
+from tests.test_serve_gpu import engine, tokens
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("name,mixer,mlp,requests,length,steps", [
+    ("one_row_shares_of_keys", O.attn(8, 2, 32, 64, 0, 16, base=100.0, scale=0.2), O.moe(4, 1, 1, 1, 32, 1.5), 1, 600, 6),
+    ("24_rows", O.attn(8, 4, 64, 32, 0, 32, scale=0.15), O.moe(16, 3, 4, 2, 32, 1.5, 96, 2.0), 8, 30, 4),
+    ("25_rows", O.attn(8, 4, 64, 32, 19, 32, scale=0.15), O.moe(16, 5, 1, 1, 32, 1.5, 96, 2.0), 5, 30, 4),
+    ("sixteen_tokens_many_experts", O.attn(16, 1, 128, 128, 70, 64, scale=0.09), O.moe(128, 8, 1, 1, 160, 1.2, 64, 1.0), 16, 40, 3),
+    ("sixteen_tokens_few_experts", O.attn(2, 2, 128, 64, 0, 0, scale=0.09), O.moe(4, 2, 1, 1, 96, 1.2), 16, 20, 3),
+    ("two_batches_of_heads", O.attn(32, 1, 64, 64, 0, 64, scale=0.12), O.moe(8, 2, 2, 1, 64, 1.5, 64, 2.0), 3, 300, 3),
+])
+def test_steps_close_to_oracle(name, mixer, mlp, requests, length, steps):
+    cfg = O.make_config(width=160, vocab=90, eps=1e-5, layers=[{"type": "attention", "mixer": mixer, "mlp": mlp}] * 2)
+    W = O.random_weights(cfg, 11)
+    lens = [length - (3 * r) % max(1, length // 2) for r in range(requests)]
+    seqs = [tokens(cfg, n + steps, 100 + r) for r, n in enumerate(lens)]
+    eng = engine(cfg, W, "bfloat16", max_tokens=64 * requests * ((length + steps) // 64 + 1), max_slots=requests)
+    eng.step([(r, s[:n], []) for r, (s, n) in enumerate(zip(seqs, lens))])
+    got = np.stack([eng.step([(r, [s[n + i]], [0]) for r, (s, n) in enumerate(zip(seqs, lens))])[0] for i in range(steps)], 1)
+    ref = np.stack([O.forward(cfg, W, s)[0][n:] for s, n in zip(seqs, lens)])
+    e = np.sqrt(((got - ref) ** 2).mean(-1)) / np.sqrt((ref ** 2).mean())
+    assert np.median(e) < 2e-2 and (e < 4e-2).mean() >= 0.9, (name, e)
+
+
+def test_a_step_is_the_same_every_time_and_under_replay():
+    """joined launches leave the same bits eagerly and from a replayed graph, whatever ran in between"""
+    cfg = O.make_config(width=128, vocab=70, eps=1e-5, layers=[{"type": "attention", "mixer": O.attn(8, 2, 128, 128, 0, 64, scale=0.1), "mlp": O.moe(8, 3, 1, 1, 96, 1.5, 64, 2.0)}] * 2)
+    W = O.random_weights(cfg, 12)
+    a, b = tokens(cfg, 330, 13), tokens(cfg, 330, 14)
+    runs = []
+    for graph in (True, False):
+        eng = engine(cfg, W, "bfloat16")
+        eng.store.set_use_graph(graph)
+        eng.step([("a", a[:240], []), ("b", b[:9], [])])
+        runs.append([eng.step([("a", [a[240 + i]], [0]), ("b", [b[9 + i]], [0])])[0] for i in range(40)])       # past 256 keys: another share count on the way
+        assert (eng.store.graph_replays() > 0) == graph
+    assert all(np.array_equal(x, y) for x, y in zip(*runs))

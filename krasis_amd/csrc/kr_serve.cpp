@@ -119,6 +119,7 @@ struct kr_serve {
     DevBuf v_first;                                      // [T, kv_heads * vdim] f32: the values of the first value-mixing layer
     DevBuf lq_c, lq_2, lq_n, lq_e, att2, head_i;         // latent mixer: query latent, W_uq output, plain query parts, folded queries, per-head values, head row tables
     void* h_meta = nullptr; size_t h_meta_bytes = 0;     // pinned staging of the per-step arrays
+    void* h_out = nullptr; size_t h_out_bytes = 0;       // pinned: the last step's argmax [rows], then its logits
     int last_want = 0;
     // capture / profile
     bool capture = false; DevBuf cap; int cap_T = 0;
@@ -304,6 +305,22 @@ int check_layer(const kr_serve_config& c, const kr_serve_layer* all, int i) {
     return KR_OK;
 }
 
+// pinned memory for a step's results
+constexpr size_t HOST_OUT_MOST = (size_t)32 << 20;
+int host_out(kr_serve* s, size_t bytes) {
+    if (bytes <= s->h_out_bytes) return KR_OK;
+    if (s->h_out) (void)hipHostFree(s->h_out);
+    s->h_out = nullptr; s->h_out_bytes = 0;
+    KR_HIP(hipHostMalloc(&s->h_out, bytes, hipHostMallocMapped | hipHostMallocCoherent));
+    s->h_out_bytes = bytes;
+    return KR_OK;
+}
+// scratch of the step's last launch, zero before its first use (the launch leaves it so)
+int finish_scratch(kr_serve* s, int rows) {
+    const size_t n = kr_sv_finish_bytes(rows);
+    if (n <= s->amax.bytes) return 0;
+    return s->amax.ensure(n) || hipMemsetAsync(s->amax.p, 0, n, s->st) != hipSuccess;
+}
 struct Timer {       // HIP events around one kernel family when profiling is on
     kr_serve* s; int fam;
     Timer(kr_serve* s_, int f) : s(s_), fam(f) { if (s->prof) (void)hipEventRecord(s->ev0, s->st); }
@@ -482,6 +499,7 @@ void kr_serve_destroy(kr_serve* s) {
     if (s->ev0) (void)hipEventDestroy(s->ev0);
     if (s->ev1) (void)hipEventDestroy(s->ev1);
     if (s->h_meta) (void)hipHostFree(s->h_meta);
+    if (s->h_out) (void)hipHostFree(s->h_out);
     for (auto& g : s->graphs) (void)hipGraphExecDestroy(g.exec);
     delete s;
 }
@@ -909,6 +927,9 @@ int kr_serve_finalize(kr_serve* s) {
         }
         for (int r : need) if (!l.have[r]) return kr_fail(KR_ERR_STATE, "layer %d: tensor of role %d missing", i, r);
     }
+    // one row of logits per slot
+    KR_HIP(hipSetDevice(s->device));
+    { const int rc = host_out(s, std::min(HOST_OUT_MOST, (size_t)s->c.max_slots * ((size_t)s->c.vocab * 4 + 4) + 256)); if (rc) return rc; }
     s->finalized = true;
     return KR_OK;
 }
@@ -977,12 +998,12 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     if (need_pages > (int)s->free_pages.size()) return kr_fail(KR_ERR_STATE, "cache pool exhausted: %d pages needed, %zu free", need_pages, s->free_pages.size());
     // ---- per-step arrays: tokens | slot | pos | want | page table
     const size_t n_meta = (size_t)5 * T + n_want + 3 * (size_t)n_entries + 2;      // ... | first row of every entry and the end | slot of every entry | first 64-token block of every entry and the end | tokens, those of short entries first
-    const size_t meta_bytes = (n_meta + s->h_table.size()) * 4;
-    if (meta_bytes > s->h_meta_bytes) {
+    const size_t meta_bytes = (n_meta + s->h_table.size()) * 4;      // (a launch may copy up to twelve bytes more)
+    if (meta_bytes + 16 > s->h_meta_bytes) {
         if (s->h_meta) (void)hipHostFree(s->h_meta);
         s->h_meta = nullptr; s->h_meta_bytes = 0;
-        KR_HIP(hipHostMalloc(&s->h_meta, meta_bytes * 2, hipHostMallocDefault));
-        s->h_meta_bytes = meta_bytes * 2;
+        KR_HIP(hipHostMalloc(&s->h_meta, meta_bytes * 2 + 16, hipHostMallocMapped | hipHostMallocCoherent));
+        s->h_meta_bytes = meta_bytes * 2 + 16;
     }
     int* hm = (int*)s->h_meta;
     int* h_tok = hm; int* h_slot = hm + T; int* h_pos = hm + 2 * T; int* h_brow = hm + 3 * T; int* h_want = hm + 4 * T; /* h_brow: row of the pair embedding */ int* h_eoff = h_want + n_want; int* h_eslot = h_eoff + n_entries + 1; int* h_echunk = h_eslot + n_entries; int* h_order = h_echunk + n_entries + 1;
@@ -1015,9 +1036,14 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         for (int i = 0; i < n_want; i++) h_want[i] = want_rows[i];
         std::memcpy(h_tab, s->h_table.data(), s->h_table.size() * 4);
     }
-    if (s->meta.ensure(meta_bytes)) return kr_fail(KR_ERR_HIP, "step arrays");
+    if (s->meta.ensure(meta_bytes + 16)) return kr_fail(KR_ERR_HIP, "step arrays");
     hipStream_t st = s->st;
-    KR_HIP(hipMemcpyAsync(s->meta.p, hm, meta_bytes, hipMemcpyHostToDevice, st));
+    // decode-sized steps: a launch reads the arrays from the host memory they stand in and forms the rotation tables; larger arrays (whose words a launch would wait for one
+    // by one over the link) take a copy command
+    const bool begin = T <= 64 && meta_bytes <= 64 * 1024 && s->ropes.size() <= 4;
+    void* dev_hm = nullptr;
+    if (begin) KR_HIP(hipHostGetDevicePointer(&dev_hm, s->h_meta, 0));
+    else KR_HIP(hipMemcpyAsync(s->meta.p, hm, meta_bytes, hipMemcpyHostToDevice, st));
     const int* d_tok = (const int*)s->meta.p; const int* d_slot = d_tok + T; const int* d_pos = d_tok + 2 * T; const int* d_brow = d_tok + 3 * T; const int* d_want = d_tok + 4 * T;
     const int* d_eoff = d_want + n_want; const int* d_eslot = d_eoff + n_entries + 1; const int* d_echunk = d_eslot + n_entries; const int* d_order = d_echunk + n_entries + 1;
     const int* d_tab = d_tok + n_meta;
@@ -1081,7 +1107,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     if (s->x.ensure(Ts * W * 4) || s->h.ensure(Ts * W * s->esz) || s->qkv.ensure(Ts * max_qkv * 4) || s->att.ensure(Ts * max_att * s->esz) || s->mix.ensure(Ts * W * 4) ||
         s->gu.ensure(Ts * max_gu * 4 + 16) || s->y.ensure(Ts * max_y * s->esz + 16) || s->rows.ensure(Ts * max_rows * 4 + 16) || s->ffout.ensure(Ts * W * 4) ||
         s->ids.ensure(Ts * max_pairs * 4 + 16) || s->wts.ensure(Ts * max_pairs * 4 + 16) || s->moe_i.ensure((Ts * max_pairs * 4 + (size_t)max_E + 8 + max_hist) * 4) ||
-        s->hw.ensure((size_t)std::max(n_want, 1) * W * s->esz) || s->logits.ensure((size_t)std::max(n_want, 1) * c.vocab * 4) || s->amax.ensure((size_t)std::max(n_want, 1) * 4))
+        s->hw.ensure((size_t)std::max(n_want, 1) * W * s->esz) || s->logits.ensure((size_t)std::max(n_want, 1) * c.vocab * 4) || finish_scratch(s, std::max(n_want, 1)))
         return kr_fail(KR_ERR_HIP, "step scratch for %d tokens", T);
     if ((max_vf && s->v_first.ensure(Ts * max_vf * 4)) ||
         (head_i && (s->lq_c.ensure(Ts * lq_c * s->esz) || s->lq_2.ensure(Ts * lq_2 * 4) || s->lq_n.ensure(Ts * lq_n * s->esz) || s->lq_e.ensure(Ts * lq_e * 4) ||
@@ -1116,31 +1142,52 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         }
         if (plan[li].parts && (s->part_ml.ensure(plan[li].parts * 8) || s->part_acc.ensure(plan[li].parts * l.att_vdim() * 4))) return kr_fail(KR_ERR_HIP, "attention split scratch");
     }
-    const bool want_amax = argmax_out != nullptr;
-    // every launch of the step, in order; no allocation, no host copy: the same body runs eagerly or under stream capture
-    auto enqueue = [&]() -> int {
+    // results: the step's last launch stores them to pinned host memory.  (A prompt whose logits are all wanted may have more than it
+    // is given: copied from the device then)
+    const bool want_amax = n_want > 0 && argmax_out, host_logits = n_want > 0 && logits_out && (size_t)n_want * c.vocab * 4 <= HOST_OUT_MOST;
+    const size_t amax_bytes = ((size_t)n_want * 4 + 255) / 256 * 256, out_bytes = amax_bytes + (host_logits ? (size_t)n_want * c.vocab * 4 : 0);
+    void* dev_out = nullptr;
+    if (want_amax || host_logits) {
+        { const int rc = host_out(s, out_bytes); if (rc) return rc; }
+        KR_HIP(hipHostGetDevicePointer(&dev_out, s->h_out, 0));
+    }
     float* x = (float*)s->x.p;
     const int NG = c.norm_groups > 1 ? c.norm_groups : 1;
     const bool canon = c.canon_taps > 1;
+    bool normed = false;                 // the first sublayer's input left the embedding's launch
+    // the step's first launches, not part of a captured step: the host prepares its replay, some 10 us, while they run
+    auto enqueue_first = [&]() {
     const float escale = c.embed_scale != 0.0f ? c.embed_scale : 1.0f;
     const void* table2 = c.pos_rows > 0 ? s->pos.p : c.bigram_buckets > 0 ? s->bigram.p : nullptr;
     const int* rows2 = c.pos_rows > 0 ? d_pos : d_brow;
     const SvLayer& l0 = s->L[0];
-    bool normed = false;                 // the first sublayer's input left the embedding's launch
+    KrSvBegin bg{};
+    if (begin) {
+        bg.src = (const int*)dev_hm; bg.dst = (int*)s->meta.p; bg.words = (int)(meta_bytes / 4); bg.pos_at = 2 * T; bg.T = T; bg.n_rope = (int)s->ropes.size();
+        for (int r = 0; r < bg.n_rope; r++) {
+            SvRope& q = s->ropes[r];
+            bg.rope[r] = {(const double*)q.inv_freq.p, (float2*)q.cs.p, q.dims / 2, q.mult}; bg.halves += q.dims / 2;
+        }
+    }
+    auto host_side = [&](const int* d) { return begin ? bg.src + (d - d_tok) : d; };
     if (c.pre_norm && !l0.d.pre_add && !c.embed_norm) {
         Timer tm(s, 7);
-        normed = kr_sv_embed_norm(s->embed.p, s->f32, d_tok, x, T, W, escale, table2, rows2, (const float*)l0.norm_w.p, c.norm_bias ? (const float*)l0.norm_b.p : nullptr, s->h.p, c.norm_eps,
-                                  c.norm_kind, NG, (canon || l0.wkv()) ? (float*)s->h32.p : nullptr, st);
+        normed = kr_sv_embed_norm(s->embed.p, s->f32, host_side(d_tok), x, T, W, escale, table2, host_side(rows2), (const float*)l0.norm_w.p, c.norm_bias ? (const float*)l0.norm_b.p : nullptr, s->h.p, c.norm_eps,
+                                  c.norm_kind, NG, (canon || l0.wkv()) ? (float*)s->h32.p : nullptr, bg, st);
     }
     if (!normed) {
         Timer tm(s, 7);
+        if (begin) kr_sv_begin(bg, st);
         kr_sv_embed(s->embed.p, s->f32, d_tok, x, c.pre_norm ? nullptr : s->h.p, T, W, escale, table2, rows2, st);     // without input norms the first sublayer reads the embedding row itself
     }
     if (c.embed_norm) { Timer tm(s, 0); kr_sv_stream_norm(x, nullptr, (const float*)s->enorm_w.p, nullptr, true, nullptr, s->f32, T, W, c.norm_eps, c.norm_kind, c.norm_groups > 1 ? c.norm_groups : 1, st); }
-    {
+    if (!begin) {
         Timer tm(s, 2);
         for (SvRope& r : s->ropes) kr_sv_rope_table(d_pos, (const double*)r.inv_freq.p, (float2*)r.cs.p, T, r.dims / 2, r.mult, st);
     }
+    };   // enqueue_first
+    // every later launch, in order; no allocation, no host copy: the same body runs eagerly or under stream capture
+    auto enqueue = [&]() -> int {
     int* mi = (int*)s->moe_i.p;
     // down projection of a gated feed-forward: decode-sized problems form the activation inside the projection's launch, larger ones write it once
     // (formed: the projection before wrote it itself, see pair_up)
@@ -1512,22 +1559,26 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         if (s->capture) KR_HIP(hipMemcpyAsync((float*)s->cap.p + (size_t)li * Ts * W, x, Ts * W * 4, hipMemcpyDeviceToDevice, st));
     }
     if (n_want > 0) {
+        const bool scaled = c.logit_scale != 0.0f && c.logit_scale != 1.0f;
+        float* host_rows = host_logits ? (float*)((char*)dev_out + amax_bytes) : nullptr;
         { Timer tm(s, 0); kr_sv_norm(x, d_want, (const float*)s->fnorm_w.p, c.norm_bias ? (const float*)s->fnorm_b.p : nullptr, s->hw.p, s->f32, n_want, W, c.norm_eps, c.norm_kind, NG, nullptr, st); }
         KrSvGemm g{}; g.A = s->hw.p; g.lda = W; g.W = s->head.p; g.C = (float*)s->logits.p; g.ldc = c.vocab; g.M = n_want; g.N = c.vocab; g.K = W;
+        if (host_logits && !scaled && kr_sv_gemm_takes_host(g, s->f32)) { g.c_host = host_rows; host_rows = nullptr; }
         { Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); }
-        if (c.logit_scale != 0.0f && c.logit_scale != 1.0f) { Timer tm(s, 7); kr_sv_scale((float*)s->logits.p, (size_t)n_want * c.vocab, c.logit_scale, st); }
-        if (want_amax) { Timer tm(s, 7); kr_sv_argmax((const float*)s->logits.p, n_want, c.vocab, (int*)s->amax.p, st); }
+        if (scaled) { Timer tm(s, 7); kr_sv_scale((float*)s->logits.p, (size_t)n_want * c.vocab, c.logit_scale, st); }
+        { Timer tm(s, 7); kr_sv_finish((const float*)s->logits.p, n_want, c.vocab, host_rows, want_amax ? (int*)dev_out : nullptr, s->amax.p, st); }
     }
     return KR_OK;
     };   // enqueue
     bool decode_shaped = s->use_graph && !s->prof && !s->capture && T <= 64;
     for (int e = 0; e < n_entries && decode_shaped; e++) decode_shaped = counts[e] == 1;
     bool done = false;
+    enqueue_first();
     if (decode_shaped) {
         // the key: everything a launch argument depends on -- batch, wanted rows, the split of every layer, the scratch addresses
         uint64_t key = 1469598103934665603ull;
         auto mixin = [&](uint64_t v) { key = (key ^ v) * 1099511628211ull; };
-        mixin((uint64_t)T); mixin((uint64_t)n_want); mixin(want_amax);
+        mixin((uint64_t)T); mixin((uint64_t)n_want); mixin(want_amax); mixin(host_logits); mixin((uint64_t)(uintptr_t)dev_hm); mixin((uint64_t)(uintptr_t)dev_out);
         for (const KrSvAttnPlan& p : plan) mixin((uint64_t)p.nsplit);
         for (const DevBuf* b : {&s->meta, &s->x, &s->h, &s->qkv, &s->att, &s->mix, &s->gu, &s->y, &s->rows, &s->ffout, &s->ids, &s->wts, &s->moe_i, &s->hw, &s->logits,
                                 &s->amax, &s->part_ml, &s->part_acc, &s->v_first, &s->lq_c, &s->lq_2, &s->lq_n, &s->lq_e, &s->att2, &s->head_i, &s->h32, &s->hc, &s->rg, &s->qk_rms, &s->lin_o, &s->qkv2, &s->sconv, &s->ga1, &s->gz, &s->rg_ab, &s->rg_agg, &s->rg_start,
@@ -1556,12 +1607,14 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         if (exec) { KR_HIP(hipGraphLaunch(exec, st)); s->graph_replays++; done = true; }
     }
     if (!done) { const int rc = enqueue(); if (rc) return rc; }
-    if (n_want > 0) {
-        if (logits_out) KR_HIP(hipMemcpyAsync(logits_out, s->logits.p, (size_t)n_want * c.vocab * 4, hipMemcpyDeviceToHost, st));
-        if (argmax_out) KR_HIP(hipMemcpyAsync(argmax_out, s->amax.p, (size_t)n_want * 4, hipMemcpyDeviceToHost, st));
-    }
+    const size_t row_bytes = (size_t)n_want * c.vocab * 4;
+    if (n_want > 0 && logits_out && !host_logits) KR_HIP(hipMemcpyAsync(logits_out, s->logits.p, row_bytes, hipMemcpyDeviceToHost, st));
+    // the caller's pages are brought in while the launches run (fresh memory: a fault per page), not in the copy after them
+    if (host_logits) for (size_t i = 0; i < row_bytes; i += 4096) ((volatile char*)logits_out)[i] = 0;
     s->last_want = n_want;
     KR_HIP(hipStreamSynchronize(st));
+    if (want_amax) std::memcpy(argmax_out, s->h_out, (size_t)n_want * 4);
+    if (host_logits) std::memcpy(logits_out, (const char*)s->h_out + amax_bytes, row_bytes);
     KR_HIP(hipGetLastError());
     return KR_OK;
 }

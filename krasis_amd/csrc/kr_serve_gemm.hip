@@ -371,6 +371,9 @@ bool kr_sv_gemm_takes_glu(const KrSvGemm& g, bool f32) {
     return !f32 && g.M > 0 && !gm_skinny(g) && !gm_gemv_rows(g) && kr_sv_gemm_tile_fits(g, false) && kr_sv_gemm_tile_glu_fits(g);
 }
 
+// strips store 64 bytes of a row at a time (a store of one column at a time would be a transfer of its own over the host link)
+bool kr_sv_gemm_takes_host(const KrSvGemm& g, bool f32) { return !f32 && g.M > 0 && !g.seg && !g.c_rows && gm_skinny(g); }
+
 void kr_sv_gemm(const KrSvGemm& g, bool f32, hipStream_t st) {
     if (g.M <= 0 || g.N <= 0) return;
     const bool grouped = g.seg != nullptr;

@@ -23,7 +23,10 @@ __device__ __forceinline__ void gm_store(const KrSvGemm& g, int m, int n, float 
     if (n >= g.silu_lo && n < g.silu_hi) v = v / (1.0f + expf(-v));
     if (g.o_gate) v *= 1.0f / (1.0f + expf(-g.o_gate[(size_t)(row / g.o_gate_div) * g.o_gate_ld + (size_t)(row % g.o_gate_div) * g.N + n]));
     if (BF && g.c_storage) ((uint16_t*)g.C)[i] = kr_f32_to_bf16(v);
-    else g.C[i] = v;
+    else {
+        g.C[i] = v;
+        if (BF && g.c_host) g.c_host[i] = v;
+    }
 }
 
 // columns of group `group`: all N, or what the group's own matrix has

@@ -33,6 +33,7 @@ struct KrSvGemm {
     int n_first;                     //   ... and the other groups' matrices have n_first
     // with act_gu: the up columns come from a table instead: element k of problem row r is up_tab[up_rows[r] * up_ld + up_off + k] (storage type)
     const void* up_tab; const int* up_rows; int up_ld, up_off;
+    float* c_host;                   // only where kr_sv_gemm_takes_host says so: C once more, in pinned host memory
     // only where kr_sv_gemm_takes_glu says so: columns [glu_lo, glu_lo + glu_f) are gates and the glu_f columns behind them their up factors; they do not go to C but, as the
     // gated activation (of both times glu_row_w[m], if given), to glu_out [M, glu_f] in the storage type, by problem row
     void* glu_out; int glu_lo, glu_f, glu_kind; float glu_limit, glu_alpha; const float* glu_row_w;
@@ -45,6 +46,7 @@ void kr_sv_narrow_act(const KrSvGemm& g, hipStream_t st);
 bool kr_sv_gemm_takes_act(const KrSvGemm& g, bool f32, const float* gu, int ld);      // true: kr_sv_gemm forms the activation of gu [M, ld] inside its launch (act_gu) for this problem
 // whether kr_sv_gemm forms the activation itself where g's glu fields are set (bf16, prompt-sized)
 bool kr_sv_gemm_takes_glu(const KrSvGemm& g, bool f32);
+bool kr_sv_gemm_takes_host(const KrSvGemm& g, bool f32);
 // a grouped problem and a single matrix that do not depend on one another, both with act_gu, in one launch where they have few rows; false: nothing was launched
 bool kr_sv_gemm_pair(const KrSvGemm& e, const KrSvGemm& o, bool f32, hipStream_t st);
 // the forms for a bf16 store that kr_sv_gemm chooses from; _fits: shapes and alignment
@@ -59,13 +61,20 @@ void kr_sv_gemm_tile(const KrSvGemm& g, bool f32, hipStream_t st);
 enum { KR_SV_NORM_LAYER = 0, KR_SV_NORM_RMS = 1 };
 enum { KR_SV_ACT_GELU_TANH = 0, KR_SV_ACT_CLAMPED_SWIGLU = 1, KR_SV_ACT_SILU = 2, KR_SV_ACT_RELU2 = 3 /* un-gated: relu(x)^2 of the first F columns; no up columns */ };
 
+// the arrays of a step in pinned host memory: `words` of them are copied to dst, and the rotation tables of the T tokens formed (positions at src + pos_at)
+struct KrSvBegin {
+    const int* src; int* dst; int words, pos_at, T, n_rope, halves;      // halves: the sum of the tables' `half`
+    struct { const double* inv_freq; float2* cs; int half; float mult; } rope[4];
+};
+void kr_sv_begin(const KrSvBegin& b, hipStream_t st);
 // x[t] = table[tokens[t]]; with h_out also the row in the storage type (the first sublayer's input in a design without input norms)
 // scale: the row is multiplied by it (1 = as it is)
 // table2 / rows2: optional second table whose row rows2[t] is added as it is (a hashed pair-of-tokens embedding)
 void kr_sv_embed(const void* table, bool f32, const int* tokens, float* x, void* h_out, int T, int width, float scale, const void* table2, const int* rows2, hipStream_t st);
-// the same and the first sublayer's input norm in one launch (out: the normed row in the storage type, out32 optional f32 copy); false: the width is not for it, nothing was launched
+// the same and the first sublayer's input norm in one launch (out: the normed row in the storage type, out32 optional f32 copy); false: the width is not for it, nothing was launched.
+// begin (words > 0): that work in the same launch; tokens and rows2 are then host memory too
 bool kr_sv_embed_norm(const void* table, bool f32, const int* tokens, float* x, int T, int width, float scale, const void* table2, const int* rows2, const float* w, const float* b, void* out,
-                      float eps, int kind, int groups, float* out32, hipStream_t st);
+                      float eps, int kind, int groups, float* out32, const KrSvBegin& begin, hipStream_t st);
 // the stream itself: x[t] += add (optional [width]); then, with w, either x[t] <- norm(x[t]) * w (in_place: the normed row IS the stream) or
 // out[t] = norm(x[t]) * w in the storage type (the next sublayer's input).  One workgroup per row, the row held in LDS.
 void kr_sv_stream_norm(float* x, const float* add, const float* w, const float* b, bool in_place, void* out, bool out_f32, int T, int width, float eps, int kind, int groups,
@@ -365,6 +374,8 @@ struct KrSvDelta {
 void kr_sv_delta_prep(const KrSvDelta& a, hipStream_t st);
 // out[t][c] = o[t] / rms(o[t]) * w[c] * sigmoid(gate[t][c]) * scale over the whole row of n
 void kr_sv_row_out(const float* o, int n, const float* w, const float* gate, int gate_ld, float eps, float scale, void* out, int out_ld, bool f32, int T, hipStream_t st);
-void kr_sv_argmax(const float* logits, int R, int vocab, int* out, hipStream_t st);
+// rows of logits and their largest entries to pinned host memory (either may be null).  scratch: kr_sv_finish_bytes, zero before its first use and left zero
+inline size_t kr_sv_finish_bytes(int R) { return (size_t)R * 12; }
+void kr_sv_finish(const float* logits, int R, int vocab, float* host_logits, int* host_argmax, void* scratch, hipStream_t st);
 // uniform values in [-amp, amp) from a counter hash of (seed, element); amp = 0 writes zeros
 void kr_sv_fill_uniform(void* p, bool f32, size_t n, uint64_t seed, float amp, hipStream_t st);

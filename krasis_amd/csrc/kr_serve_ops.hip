@@ -194,16 +194,61 @@ __global__ void __launch_bounds__(NT) sv_norm_vec_kernel(const float* __restrict
         if (c < width) { sv_st4(out + r * width + c, v[j]); if (out32) sv_st4(out32 + r * width + c, v[j]); }
     }
 }
+// cos / sin of one (token, frequency)
+__device__ __forceinline__ float2 sv_rope_angle(int pos, double inv_freq, float mult) {
+    const double a = (double)pos * inv_freq;
+    return make_float2((float)cos(a) * mult, (float)sin(a) * mult);
+}
+__global__ void sv_rope_table_kernel(const int* __restrict__ pos, const double* __restrict__ inv_freq, float2* __restrict__ cs, int T, int half, float mult) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= T * half) return;
+    const int t = i / half, j = i - t * half;
+    cs[i] = sv_rope_angle(pos[t], inv_freq[j], mult);
+}
+
+// what a step's arrays need before its first layer, straight from the pinned host memory they were written to: the copy that later launches read, and the rotation tables.
+// A copy command, the tables and the embedding were three launches in a row of 4 - 5 us each; none needs another's result.
+// Every lane's read of host memory is a request of its own over the link (twelve requests' arrays word by word: 18 us), so the copy takes 16 bytes a lane and a position is
+// read once per workgroup.  System scope: host memory must not come from a cache line of the step before.
+__device__ __forceinline__ int sv_host_word(const int* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+__device__ __forceinline__ int sv_host_word_wave(const int* p) {      // one address per wave
+    int v = 0;
+    if ((threadIdx.x & 63) == 0) v = sv_host_word(p);
+    return __builtin_amdgcn_readfirstlane(v);
+}
+__device__ __forceinline__ void sv_begin(const KrSvBegin& b, const int block, const int blocks, const int nt) {
+    __shared__ int pos[64];
+    const int n = blocks * nt, i0 = block * nt + threadIdx.x;
+    if ((int)threadIdx.x < b.T) pos[threadIdx.x] = sv_host_word(b.src + b.pos_at + threadIdx.x);      // (T <= 64)
+    for (int i = i0; i < (b.words + 3) / 4; i += n) {
+        gu4 v;
+        asm volatile("global_load_dwordx4 %0, %1, off sc0 sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(v) : "v"(b.src + 4 * i) : "memory");
+        *reinterpret_cast<gu4*>(b.dst + 4 * i) = v;
+    }
+    __syncthreads();
+    for (int i = i0; i < b.T * b.halves; i += n) {
+        int j = i;
+        for (int r = 0; r < b.n_rope; r++) {
+            const int m = b.T * b.rope[r].half;
+            if (j < m) { b.rope[r].cs[j] = sv_rope_angle(pos[j / b.rope[r].half], b.rope[r].inv_freq[j % b.rope[r].half], b.rope[r].mult); break; }
+            j -= m;
+        }
+    }
+}
+__global__ void __launch_bounds__(256) sv_begin_kernel(const KrSvBegin b) { sv_begin(b, blockIdx.x, gridDim.x, 256); }
+static int sv_begin_blocks(const KrSvBegin& b, int nt) { return std::max(1, std::min(64, std::max((b.words + 3) / 4, b.T * b.halves) / nt + 1)); }
+
 // the token's row (scaled, a second table's row added), to the stream and, normed, to the first sublayer
 template <typename T, int KIND, int NT, int CH>
 __global__ void __launch_bounds__(NT) sv_embed_norm_kernel(const T* __restrict__ table, const int* __restrict__ tokens, float* __restrict__ x, float scale, const T* __restrict__ table2,
                                                            const int* __restrict__ rows2, const float* __restrict__ w, const float* __restrict__ b, T* __restrict__ out, int width, float eps,
-                                                           int groups, float* __restrict__ out32) {
+                                                           int groups, float* __restrict__ out32, const KrSvBegin bg, const int R) {
     __shared__ float red[NT / 64];
     extern __shared__ __attribute__((aligned(16))) float row[];
     const size_t t = blockIdx.x;
-    const T* e = table + (size_t)tokens[t] * width;
-    const T* e2 = table2 ? table2 + (size_t)rows2[t] * width : nullptr;
+    if ((int)t >= R) { sv_begin(bg, (int)t - R, gridDim.x - R, NT); return; }      // (bg.words > 0: tokens and rows2 are host memory)
+    const T* e = table + (size_t)(bg.words > 0 ? sv_host_word_wave(tokens + t) : tokens[t]) * width;
+    const T* e2 = table2 ? table2 + (size_t)(bg.words > 0 ? sv_host_word_wave(rows2 + t) : rows2[t]) * width : nullptr;
     float4 v[CH];
 #pragma unroll
     for (int j = 0; j < CH; j++) {
@@ -335,14 +380,6 @@ __global__ void __launch_bounds__(256) sv_qk_rms_kernel(const KrSvAttn a) {
     for (int c = threadIdx.x; c < n; c += 256) { const float v = b ? z[c] + b[c] : z[c]; q = __builtin_fmaf(v, v, q); }
     q = sv_block_sum<4>(q, red);
     if (threadIdx.x == 0) a.inv_rms_out[(size_t)t * 2 + part] = 1.0f / sqrtf(q / (float)n + a.eps);
-}
-
-__global__ void sv_rope_table_kernel(const int* __restrict__ pos, const double* __restrict__ inv_freq, float2* __restrict__ cs, int T, int half, float mult) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= T * half) return;
-    const int t = i / half, j = i - t * half;
-    const double a = (double)pos[t] * inv_freq[j];
-    cs[i] = make_float2((float)cos(a) * mult, (float)sin(a) * mult);
 }
 
 // one wave per (token, head): the head vector is staged in LDS, rotated and normed there; q heads are written back in place, k heads go to the
@@ -2143,33 +2180,43 @@ __global__ void __launch_bounds__(256) sv_ssd_out_kernel(const KrSvSsdOut a, T* 
     for (int c = threadIdx.x; c < inner; c += 256) sv_st(out + t * a.out_ld + c, yr[c] * gst[2 * (c / gw) + 1] * a.w[c] * a.scale);
 }
 
-__global__ void __launch_bounds__(1024) sv_argmax_kernel(const float* __restrict__ logits, int vocab, int* __restrict__ out) {
-    __shared__ float bv[16]; __shared__ int bi[16];
-    const float* row = logits + (size_t)blockIdx.x * vocab;
-    float v = -INFINITY; int idx = 0x7fffffff;
-    if (vocab % 4 == 0) {                    // rows of 16-byte pieces, eight in flight per thread: 32768 entries 12.6 -> 7.3 us
-#pragma unroll 8
-        for (int c = 4 * threadIdx.x; c < vocab; c += 4096) {
+// The end of a step, many workgroups per row: the row's largest entry (the lowest index of equals; NaN never), and the row itself, to pinned host memory.  Two copy commands and
+// the host's wait for each took 40 us after this launch, 100 with 1.5 MB of logits; the stores here cross the link beside the search.
+// best: value in order of size and index in one word, 0 = none yet; the last workgroup of a row hands the result on and leaves best and done as it found them.
+__global__ void __launch_bounds__(256) sv_finish_kernel(const float* __restrict__ logits, int vocab, int chunk, float* __restrict__ host_logits, int* __restrict__ host_argmax,
+                                                        unsigned long long* __restrict__ best, unsigned* __restrict__ done) {
+    __shared__ unsigned long long bw[4];
+    const int r = blockIdx.x, c0 = blockIdx.y * chunk, c1 = min(vocab, c0 + chunk);
+    const float* row = logits + (size_t)r * vocab;
+    float* to = host_logits ? host_logits + (size_t)r * vocab : nullptr;
+    unsigned long long b = 0;
+    auto see = [&](float x, int c) {
+        if (x != x) return;
+        const uint32_t u = __float_as_uint(x + 0.0f);          // (both zeros are equal)
+        const unsigned long long k = ((unsigned long long)((u & 0x80000000u) ? ~u : u | 0x80000000u) << 32) | (0xFFFFFFFFu - (uint32_t)c);
+        if (k > b) b = k;
+    };
+    if (vocab % 4 == 0) {
+        for (int c = c0 + 4 * threadIdx.x; c < c1; c += 1024) {
             const float4 q = *reinterpret_cast<const float4*>(row + c);
-            const float x[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-            for (int e = 0; e < 4; e++) if (x[e] > v || (x[e] == v && c + e < idx)) { v = x[e]; idx = c + e; }
+            if (to) *reinterpret_cast<float4*>(to + c) = q;
+            see(q.x, c); see(q.y, c + 1); see(q.z, c + 2); see(q.w, c + 3);
         }
     } else {
-#pragma unroll 8
-        for (int c = threadIdx.x; c < vocab; c += 1024) { const float x = row[c]; if (x > v || (x == v && c < idx)) { v = x; idx = c; } }
+        for (int c = c0 + threadIdx.x; c < c1; c += 256) { const float x = row[c]; if (to) to[c] = x; see(x, c); }
     }
+    if (!host_argmax) return;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(v, o); const int oi = __shfl_xor(idx, o);
-        if (ov > v || (ov == v && oi < idx)) { v = ov; idx = oi; }
-    }
-    if ((threadIdx.x & 63) == 0) { bv[threadIdx.x >> 6] = v; bi[threadIdx.x >> 6] = idx; }
+    for (int o = 32; o > 0; o >>= 1) { const unsigned long long v = __shfl_xor(b, o); if (v > b) b = v; }
+    if ((threadIdx.x & 63) == 0) bw[threadIdx.x >> 6] = b;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < 16; w++) if (bv[w] > v || (bv[w] == v && bi[w] < idx)) { v = bv[w]; idx = bi[w]; }
-        out[blockIdx.x] = idx == 0x7fffffff ? 0 : idx;
-    }
+    if (threadIdx.x != 0) return;
+    for (int w = 1; w < 4; w++) if (bw[w] > b) b = bw[w];
+    __hip_atomic_fetch_max(best + r, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__hip_atomic_fetch_add(done + r, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) != gridDim.y - 1) return;
+    const unsigned long long v = __hip_atomic_exchange(best + r, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(done + r, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    host_argmax[r] = v ? (int)(0xFFFFFFFFu - (uint32_t)v) : 0;
 }
 template <typename T>
 __global__ void sv_fill_uniform_kernel(T* __restrict__ p, size_t n, uint64_t seed, float amp) {
@@ -2240,19 +2287,22 @@ void kr_sv_norm(const float* x, const int* rows, const float* w, const float* b,
 
 template <typename T, int KIND>
 static bool sv_embed_norm_launch(const T* table, const int* tokens, float* x, float scale, const T* table2, const int* rows2, const float* w, const float* b, T* out, int R, int width, float eps,
-                                 int groups, float* out32, hipStream_t st) {
+                                 int groups, float* out32, const KrSvBegin& bg, hipStream_t st) {
     const size_t glds = groups > 1 ? (size_t)(width + 2 * groups) * sizeof(float) : 0;
     return sv_al16({table, x, table2, w, b, out, out32}) && sv_vec_rows(R, width, [&](auto nt, auto ch) {
-            hipLaunchKernelGGL((sv_embed_norm_kernel<T, KIND, nt(), ch()>), dim3(R), dim3(nt()), glds, st, table, tokens, x, scale, table2, rows2, w, b, out, width, eps, groups, out32); });
+            hipLaunchKernelGGL((sv_embed_norm_kernel<T, KIND, nt(), ch()>), dim3(R + (bg.words > 0 ? sv_begin_blocks(bg, nt()) : 0)), dim3(nt()), glds, st, table, tokens, x, scale, table2, rows2, w, b,
+                               out, width, eps, groups, out32, bg, R); });
 }
 bool kr_sv_embed_norm(const void* table, bool f32, const int* tokens, float* x, int T, int width, float scale, const void* table2, const int* rows2, const float* w, const float* b, void* out,
-                      float eps, int kind, int groups, float* out32, hipStream_t st) {
+                      float eps, int kind, int groups, float* out32, const KrSvBegin& bg, hipStream_t st) {
     if (T <= 0) return true;
-#define SV_ENL(T_, K_) sv_embed_norm_launch<T_, K_>((const T_*)table, tokens, x, scale, (const T_*)table2, rows2, w, b, (T_*)out, T, width, eps, groups, out32, st)
+#define SV_ENL(T_, K_) sv_embed_norm_launch<T_, K_>((const T_*)table, tokens, x, scale, (const T_*)table2, rows2, w, b, (T_*)out, T, width, eps, groups, out32, bg, st)
     if (kind == KR_SV_NORM_LAYER) return f32 ? SV_ENL(float, KR_SV_NORM_LAYER) : SV_ENL(uint16_t, KR_SV_NORM_LAYER);
     return f32 ? SV_ENL(float, KR_SV_NORM_RMS) : SV_ENL(uint16_t, KR_SV_NORM_RMS);
 #undef SV_ENL
 }
+
+void kr_sv_begin(const KrSvBegin& b, hipStream_t st) { hipLaunchKernelGGL(sv_begin_kernel, dim3(sv_begin_blocks(b, 256)), dim3(256), 0, st, b); }
 
 void kr_sv_rope_table(const int* pos, const double* inv_freq, float2* cs, int T, int half, float mult, hipStream_t st) {
     const int n = T * half;
@@ -2597,9 +2647,10 @@ void kr_sv_lin_out(const KrSvLin& a, bool f32, hipStream_t st) {
     else hipLaunchKernelGGL(sv_lin_out_kernel<uint16_t>, dim3(a.T, a.heads), dim3(64), 0, st, a, (uint16_t*)a.out);
 }
 
-void kr_sv_argmax(const float* logits, int R, int vocab, int* out, hipStream_t st) {
-    if (R <= 0) return;
-    hipLaunchKernelGGL(sv_argmax_kernel, dim3(R), dim3(1024), 0, st, logits, vocab, out);
+void kr_sv_finish(const float* logits, int R, int vocab, float* host_logits, int* host_argmax, void* scratch, hipStream_t st) {
+    if (R <= 0 || (!host_logits && !host_argmax)) return;
+    const int nb = std::min(32, (vocab + 1023) / 1024), chunk = ((vocab + nb - 1) / nb + 3) / 4 * 4;
+    hipLaunchKernelGGL(sv_finish_kernel, dim3(R, nb), dim3(256), 0, st, logits, vocab, chunk, host_logits, host_argmax, (unsigned long long*)scratch, (unsigned*)((unsigned long long*)scratch + R));
 }
 
 #ifdef KR_SV_STAMPS

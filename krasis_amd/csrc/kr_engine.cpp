@@ -1099,7 +1099,7 @@ int kr_moe_prefill_set(kr_engine* e, int layer, const void* x_bf16, const int32_
     const int CHmax = pairs / topk > 64 ? pairs / topk : 64;
     const int CH = M < CHmax ? M : CHmax;
     const size_t np = (size_t)CH * topk;
-    const int max_tiles = (int)(np / 64) + E + 1;
+    const int max_tiles = (int)(np / 16) + E + 1;      // (tiles of 16 rows are the smallest, kr_pf_tile_rows)
     const size_t n_i32 = 3 * (size_t)E + 3 * (size_t)max_tiles + 4 + 2 * np;
     if (P.i32.ensure(n_i32 * 4) || P.xh.ensure((size_t)CH * H) || P.xl.ensure((size_t)CH * H) || P.xs.ensure((size_t)CH * (H / 128) * 4) ||
         P.gu.ensure(np * 2 * I * 4) || P.hh.ensure(np * I) || P.hl.ensure(np * I) || P.hs.ensure(np * (I / 128) * 4) || P.eo.ensure(np * H * 4))
@@ -1159,7 +1159,7 @@ int kr_moe_prefill_rows(kr_engine* e, int layer, const void* rows_bf16, const in
     const int pairs = e->pf_pairs > 0 ? e->pf_pairs : KR_PF_PAIRS;
     const int CH = n < pairs ? n : pairs;
     const size_t np = (size_t)CH;
-    const int max_tiles = (int)(np / 64) + E + 1;
+    const int max_tiles = (int)(np / 16) + E + 1;      // (tiles of 16 rows are the smallest, kr_pf_tile_rows)
     const size_t n_i32 = 3 * (size_t)E + 3 * (size_t)max_tiles + 4 + 2 * np;
     if (P.i32.ensure(n_i32 * 4) || P.xh.ensure((size_t)CH * H) || P.xl.ensure((size_t)CH * H) || P.xs.ensure((size_t)CH * (H / 128) * 4) ||
         P.gu.ensure(np * 2 * I * 4) || P.hh.ensure(np * I) || P.hl.ensure(np * I) || P.hs.ensure(np * (I / 128) * 4))

@@ -274,6 +274,7 @@ struct KrPfGemmArgs {
 
 #include "kr_prefill_gemm2.inc"
 #include "kr_prefill_wide.inc"
+#include "kr_prefill_strip.inc"
 
 // ------------------------------------------------------------------------------------------
 // combine: out[t] = sum_s w[t][s] * eo[row(t,s)] in routing order (moe.rs:661-667); shared: rsf*out + shared (moe.rs:703-706)
@@ -362,8 +363,18 @@ void kr_launch_pf_wsum(const KrMatDev& m, int n_experts, uint32_t* wsum, hipStre
 // (a four-layer INT4 prompt, ms, 64-row tiles / wide from 128 tiles / always wide: 777 tokens 3.99 / 3.89 / 3.98, 1400 tokens 6.30 / 5.64 / 5.89).
 // It knows the fused form of the group sum only, and addresses a digit plane by 32-bit offsets.
 static bool pf_all_fma(const KrMatDev& m) { return m.n_fma >= m.N; }
+// Few rows per expert, INT4: strips, in tiles of 16 rows while an expert seldom has more (up to ten on average: 520 rows on 512 experts 243 us, tiles of 32 245), then of 32 while two
+// halves still cost less than the 64-row tile: to 16 rows an expert (64 experts, 160 rows 174 against 183; 240 rows 213 against 192), with many experts to 24 (512 experts, 1100 rows
+// 331 against 351, 1500 rows 393 against 400).  The rows' digits have to fit the LDS.
 int kr_pf_tile_rows(const KrMatDev& m0, const KrMatDev& m1, long rows, int E) {
-    return pf_all_fma(m0) && pf_all_fma(m1) && rows * (long)(m0.ng > m1.ng ? m0.ng : m1.ng) * 128 < 1L << 32 && rows >= 48L * E ? PFW_TM : PF_BM;
+    if (!pf_all_fma(m0) || !pf_all_fma(m1)) return PF_BM;
+    const int K = 128 * (m0.ng > m1.ng ? m0.ng : m1.ng);
+    if (rows * (long)K < 1L << 32 && rows >= 48L * E) return PFW_TM;
+    if (m0.bits == 4 && m1.bits == 4 && m0.N % 16 == 0 && m1.N % 16 == 0) {
+        if (rows <= 10L * E && pf_strip_lds(K, 16) <= PFS_LDS) return 16;
+        if (rows <= (E >= 256 ? 24L : 16L) * E && pf_strip_lds(K, 32) <= PFS_LDS) return 32;
+    }
+    return PF_BM;
 }
 static bool pf_dense_wide(const KrPfGemmArgs& a) {
     int ncb = (a.m.N + PFW_TN - 1) / PFW_TN; bool all = pf_all_fma(a.m);
@@ -381,6 +392,10 @@ void kr_launch_pf_gemm(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_
     if (single_expert_rows > 0 ? pf_dense_wide(a) : tile_rows == PFW_TM) {
         const int wt = single_expert_rows > 0 ? (single_expert_rows + PFW_TM - 1) / PFW_TM : max_tiles;
         if (m.bits == 8) kr_pf_wide_launch<8>(a, wt, st); else kr_pf_wide_launch<4>(a, wt, st);
+        return;
+    }
+    if (single_expert_rows <= 0 && tile_rows < PF_BM) {
+        if (tile_rows == 16) kr_pf_strip_launch<1, 8>(a, max_tiles, st); else kr_pf_strip_launch<2, 16>(a, max_tiles, st);
         return;
     }
     const int mt = single_expert_rows > 0 ? (single_expert_rows + PF_BM - 1) / PF_BM : max_tiles;

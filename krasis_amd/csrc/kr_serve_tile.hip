@@ -12,6 +12,7 @@
 // 64 experts 24576 x 1536 x 2048 372 -> 248 and x 2048 x 768 217 -> 149, 500 x 2048 x 2048 36.8 -> 14.1, 100 x 4224 x 2048 36.9 -> 13.2.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "kr_lds_optin.h"
 #include "kr_serve_gemm_dev.h"
@@ -79,16 +80,28 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[a][b][i] = 0.0f;
     const int steps = g.K / BK;
+    // A tile's row blocks go round the waves' rows (block a of wave row wr: rows 32 (a WM + wr)), so that the last tile of a matrix or an expert, which is seldom full, takes only the
+    // blocks it has: the k loop exists once per number of them, and rows past the last block are not requested (the waits that count requests belong to the deep ring, whose
+    // waves have one block).  24576 rows on 64 experts, about 384 each, 2 x 768 x 2048: 235 -> 222 us; 27500
+    // rows on 128, 2 x 1536 x 4096: 730 -> 702, and x 4096 x 1536 308 -> 283.
+    const int blocks = MB == 1 ? 1 : min(MB, __builtin_amdgcn_readfirstlane((mend - m0 + 32 * WM - 1) / (32 * WM)));
+    static_assert(MB == 1 || DEPTH == 2, "all waits of a tile with several blocks are for everything");
     auto request = [&](int slot) {
 #pragma unroll
-        for (int i = 0; i < RW; i++) { tl_dma16(base + (uint32_t)slot * (uint32_t)(SLOT * sizeof(T)) + i * 1024u, src[i]); src[i] += BK; }
+        for (int i = 0; i < RW; i++) {
+            const int q = wave * RW + i;
+            if (MB == 1 || q >= RA || q < blocks * 4 * WM) tl_dma16(base + (uint32_t)slot * (uint32_t)(SLOT * sizeof(T)) + i * 1024u, src[i]);
+            src[i] += BK;
+        }
     };
 #pragma unroll
     for (int d = 0; d < DEPTH - 1; d++) if (d < steps) request(d);
     // fragment of rows [32 blk, +32), k step ks of the slot: chunk ks + 4 h of row r
     const int sw = (r >> 1) & 7;
-    const T* af0 = ring + (wr * (BM / WM) + r) * BK;
+    const T* af0 = ring + (wr * 32 + r) * BK;
     const T* bf0 = ring + (BM + wc * (BN / WN) + r) * BK;
+    auto multiply = [&](auto used) {                           // used: blocks of this tile
+    constexpr int MU = used();
     int slot = 0;
     for (int s = 0; s < steps; s++) {
         // slot s has landed when only the DEPTH - 2 younger ones are outstanding (none at the end)
@@ -100,7 +113,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
         auto read = [&](int ks) {
             const int ch = ((ks + 4 * h) ^ sw) * CH;           // the halves of the wave take k halves of the slot (any order serves, both operands alike)
 #pragma unroll
-            for (int a = 0; a < MB; a++) af[ks & 1][a] = *reinterpret_cast<const gu4*>(ab + a * 32 * BK + ch);
+            for (int a = 0; a < MU; a++) af[ks & 1][a] = *reinterpret_cast<const gu4*>(ab + a * 32 * WM * BK + ch);
 #pragma unroll
             for (int b = 0; b < NB; b++) bf[ks & 1][b] = *reinterpret_cast<const gu4*>(bb + b * 32 * BK + ch);
         };
@@ -111,7 +124,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (sizeof(T) == 2) {
 #pragma unroll
-                for (int a = 0; a < MB; a++)
+                for (int a = 0; a < MU; a++)
 #pragma unroll
                     for (int b = 0; b < NB; b++)
                         acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(gb8, af[ks & 1][a]), __builtin_bit_cast(gb8, bf[ks & 1][b]), acc[a][b], 0, 0, 0);
@@ -119,7 +132,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
 #pragma unroll
                 for (int e = 0; e < 4; e++)
 #pragma unroll
-                    for (int a = 0; a < MB; a++)
+                    for (int a = 0; a < MU; a++)
 #pragma unroll
                         for (int b = 0; b < NB; b++)
                             acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(af[ks & 1][a][e]), __uint_as_float(bf[ks & 1][b][e]), acc[a][b], 0, 0, 0);
@@ -128,6 +141,12 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
         }
         slot = slot == DEPTH - 1 ? 0 : slot + 1;
     }
+    };
+    using std::integral_constant;
+    if (MB == 1 || blocks == MB) multiply(integral_constant<int, MB>{});
+    else if (MB > 2 && blocks == 3) multiply(integral_constant<int, (MB > 2 ? 3 : 1)>{});
+    else if (MB > 2 && blocks == 2) multiply(integral_constant<int, (MB > 2 ? 2 : 1)>{});
+    else multiply(integral_constant<int, 1>{});
     if constexpr (GLU) {
         if (pairs) {
             tl_wait_barrier<0>();
@@ -151,7 +170,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll 1
                     for (int it = 0; it < 2; it++) {
-                        const int o = (row + 16 * it) * LD + c8, m = m0 + wr * (BM / WM) + a * 32 + row + 16 * it;
+                        const int o = (row + 16 * it) * LD + c8, m = m0 + (a * WM + wr) * 32 + row + 16 * it;
                         if (m >= mend || n + c8 >= N) continue;
                         const float w = g.glu_row_w ? g.glu_row_w[m] : 1.0f;
                         float4 v0 = *reinterpret_cast<const float4*>(pg + o), v1 = *reinterpret_cast<const float4*>(pg + o + 4);
@@ -190,7 +209,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
         for (int a = 0; a < MB; a++)
 #pragma unroll
             for (int b = 0; b < NB; b++) {
-                const int n = n0 + wc * (BN / WN) + b * 32 + r, mb = m0 + wr * (BM / WM) + a * 32 + 4 * h;
+                const int n = n0 + wc * (BN / WN) + b * 32 + r, mb = m0 + (a * WM + wr) * 32 + 4 * h;
                 float* c = g.C + (size_t)mb * g.ldc + column(n);
                 if (n < N) {
 #pragma unroll
@@ -212,7 +231,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
 #pragma unroll
             for (int i = 0; i < 16; i++) blk[((i & 3) + 8 * (i >> 2) + 4 * h) * 33 + r] = acc[a][b][i];
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            const int n = n0 + wc * (BN / WN) + b * 32 + r, mb = m0 + wr * (BM / WM) + a * 32;
+            const int n = n0 + wc * (BN / WN) + b * 32 + r, mb = m0 + (a * WM + wr) * 32;
 #pragma unroll 1
             for (int i = h; i < 32; i += 2)
                 if (n < N && mb + i < mend) gm_store<sizeof(T) == 2>(g, mb + i, column(n), blk[i * 33 + r]);

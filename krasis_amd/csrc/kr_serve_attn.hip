@@ -14,9 +14,8 @@
 // LDS-DMA writes lane-linear, so the chunk order is swizzled on the source side: K chunk c of row r at c ^ (r / rows per 256 bytes), V groups of four chunks likewise, which
 // spreads the 32 rows of a fragment read, and the 4 rows x 64 bytes of a transposing read, over all banks.
 // Bound: the matrix instruction, three times 4 H D keys operations (about 50 us at the case below); exponentials, the splitting of the weights and the addresses (some 700
-// vector instructions per tile and wave beside 96 products) run beside it in the SIMD's other wave; at head size 128 the query pieces, sums and scores of two waves per SIMD are
-// 25 registers more than there are, and those spill.  Per launch, us, f32 matrix instruction before -> now: 4096 tokens, 16 / 2
-// heads of 128, window 1024: 490 -> 136; 3300 tokens of three requests, 64 / 4 heads, window 2048: 1230 -> 333.  64-bit oracle of a whole prompt: error 5.1e-3 before, 4.4e-3
+// vector instructions per tile and wave beside 96 products) run beside it in the SIMD's other wave.  Per launch, us, f32 matrix instruction before -> now: 4096 tokens, 16 / 2 heads
+// of 128, window 1024: 490 -> 108; 3300 tokens of three requests, 64 / 4 heads, window 2048: 1230 -> 249.  64-bit oracle of a whole prompt: error 5.1e-3 before, 4.4e-3
 // now (the store's bf16 roundings).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -55,6 +54,11 @@ __global__ void __launch_bounds__(256, 2) sv_attn_prompt_kernel(const KrSvAttn a
     constexpr int KRP = 16 / KC, VRP = 16 / VC;                // rows per 256 bytes
     __shared__ __attribute__((aligned(1024))) uint16_t Kt[2 * KSLOT];
     __shared__ __attribute__((aligned(1024))) uint16_t Vt[2 * VSLOT];
+    // The last pieces of the first LQ k steps wait in LDS, each lane's its own.  At 128 x 128 the query pieces, sums and scores of two waves per SIMD were 25 registers more than
+    // there are, and a reload of a spilled one waits, in order, for the next tile's rows requested before it: 4096 tokens 140 us a launch with the spills, 108 without, 3300 of
+    // three requests 326 / 249.
+    constexpr int LQ = DIM == 128 && VDIM == 128 ? 4 : 0;
+    __shared__ at_u4 Lq[LQ > 0 ? 4 * LQ * 64 : 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 31, h = lane >> 5;
     const int R = a.heads / a.kv_heads, TQ = AT_ROWS / R, g = blockIdx.y, sp = blockIdx.z;
     // the tile of tokens: entries' tile counts (short entries may have a launch of their own) through a prefix sum over the lanes
@@ -103,6 +107,7 @@ __global__ void __launch_bounds__(256, 2) sv_attn_prompt_kernel(const KrSvAttn a
     // exponential is then one subtraction and one hardware instruction
     const float qscale = a.softcap > 0.0f ? a.scale : a.scale * AT_LOG2E;
     at_u4 qh[KS], qm[KS], ql[KS];
+    const int lq0 = wave * LQ * 64 + lane;
     {
         const float* qp = a.qkv + (size_t)(t0 + (rv ? tq : 0)) * a.ldq + (size_t)head * DIM + (size_t)(KS * h) * 8;
 #pragma unroll
@@ -116,6 +121,7 @@ __global__ void __launch_bounds__(256, 2) sv_attn_prompt_kernel(const KrSvAttn a
                 at_split(rv ? v[2 * i] * qscale : 0.0f, rv ? v[2 * i + 1] * qscale : 0.0f, x, y, z);
                 qh[ks][i] = x; qm[ks][i] = y; ql[ks][i] = z;
             }
+            if (ks < LQ) Lq[lq0 + ks * 64] = ql[ks];
         }
     }
     const int* table = a.page_table + (size_t)sl * a.table_ld;
@@ -161,6 +167,8 @@ __global__ void __launch_bounds__(256, 2) sv_attn_prompt_kernel(const KrSvAttn a
         tile_at(c, j0, jl);
         const int je = min(j0 + AT_KEYS - 1, jl);              // last real key of the tile
         if (!w_any || j0 > wp1 || (je < wlo && j0 >= a.keep)) continue;
+        int nk = n, lv = lane;                                 // (addresses of fragments are formed per tile: hoisted, they are what spills)
+        if (LQ > 0) asm volatile("" : "+v"(nk), "+v"(lv));
         // ---- S^T: two blocks of 32 keys
         at_f16 st[2];
 #pragma unroll
@@ -170,8 +178,13 @@ __global__ void __launch_bounds__(256, 2) sv_attn_prompt_kernel(const KrSvAttn a
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             at_b8 kf[2];
+            if (ks < LQ) {
+                int at = lq0 + ks * 64;
+                asm volatile("" : "+v"(at));                   // else the read leaves the loop, for the register it was to save
+                ql[ks] = Lq[at];
+            }
 #pragma unroll
-            for (int b = 0; b < 2; b++) kf[b] = __builtin_bit_cast(at_b8, *reinterpret_cast<const at_u4*>(&Kt[slot * KSLOT + (b * 32 + n) * DIM + (((ks + KS * h) ^ (((b * 32 + n) / KRP) % KC)) * 8)]));
+            for (int b = 0; b < 2; b++) kf[b] = __builtin_bit_cast(at_b8, *reinterpret_cast<const at_u4*>(&Kt[slot * KSLOT + (b * 32 + nk) * DIM + (((ks + KS * h) ^ (((b * 32 + nk) / KRP) % KC)) * 8)]));
 #pragma unroll
             for (int b = 0; b < 2; b++) st[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[b], __builtin_bit_cast(at_b8, ql[ks]), st[b], 0, 0, 0);
 #pragma unroll
@@ -235,11 +248,11 @@ __global__ void __launch_bounds__(256, 2) sv_attn_prompt_kernel(const KrSvAttn a
                 ph[i] = x; pm[i] = y; pl[i] = z;
             }
             typedef __fp16 at_h4 __attribute__((__vector_size__(4 * sizeof(__fp16))));
-            const int r = 16 * kt + 4 * h + ((lane & 15) >> 2);          // this lane points at row r (and r + 8), four columns of its 16-lane group
+            const int r = 16 * kt + 4 * h + ((lv & 15) >> 2);          // this lane points at row r (and r + 8), four columns of its 16-lane group
             at_b8 vf[DB];
 #pragma unroll
             for (int d = 0; d < DB; d++) {
-                const int col = 32 * d + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+                const int col = 32 * d + 16 * ((lv >> 4) & 1) + 4 * (lv & 3);
                 const uint16_t* v0 = &Vt[slot * VSLOT + r * VDIM + (((col >> 3) ^ (4 * ((r / VRP) % (VC / 4)))) * 8) + (col & 7)];
                 const uint16_t* v1 = &Vt[slot * VSLOT + (r + 8) * VDIM + (((col >> 3) ^ (4 * (((r + 8) / VRP) % (VC / 4)))) * 8) + (col & 7)];
                 const at_u2 x = __builtin_bit_cast(at_u2, __builtin_amdgcn_ds_read_tr16_b64_v4f16((__attribute__((address_space(3))) at_h4*)(v0)));

@@ -114,7 +114,15 @@ __global__ void __launch_bounds__(1024) kr_pf_sort1_kernel(const int32_t* __rest
     const int t = threadIdx.x;
     s_cnt[t] = 0; s_cur[t] = 0;
     __syncthreads();
-    for (int i = t; i < n_pairs; i += 1024) { const int e = ids[i]; if (e >= 0 && e < E) atomicAdd(&s_cnt[e], 1); }
+    // Both passes over the pairs take sixteen of a thread together: a lone workgroup waits for memory once per batch instead of once per pair (18006 pairs, 64 experts: 28.1 -> 21.5 us).
+    constexpr int NB = 16;
+    for (int i0 = t; i0 < n_pairs; i0 += 1024 * NB) {
+        int e[NB];
+#pragma unroll
+        for (int u = 0; u < NB; u++) e[u] = i0 + 1024 * u < n_pairs ? ids[i0 + 1024 * u] : -1;
+#pragma unroll
+        for (int u = 0; u < NB; u++) if (e[u] >= 0 && e[u] < E) atomicAdd(&s_cnt[e[u]], 1);
+    }
     __syncthreads();
     const int c = t < E ? s_cnt[t] : 0, nt = (c + bm - 1) / bm;
     s_off[t] = c; s_til[t] = nt;
@@ -134,11 +142,19 @@ __global__ void __launch_bounds__(1024) kr_pf_sort1_kernel(const int32_t* __rest
         for (int i = 0; i < nt; i++) { tile_expert[til + i] = t; tile_row0[til + i] = off + i * bm; tile_rows[til + i] = (c - i * bm) < bm ? (c - i * bm) : bm; }
     }
     __syncthreads();
-    for (int i = t; i < n_pairs; i += 1024) {
-        const int e = ids[i];
-        if (e < 0 || e >= E) { pair_row[i] = -1; continue; }
-        const int r = s_off[e] + atomicAdd(&s_cur[e], 1);
-        row_pair[r] = i; pair_row[i] = r;
+    for (int i0 = t; i0 < n_pairs; i0 += 1024 * NB) {
+        int e[NB], r[NB];
+#pragma unroll
+        for (int u = 0; u < NB; u++) { const int i = i0 + 1024 * u; e[u] = i < n_pairs ? ids[i] : -1; if (e[u] >= E) e[u] = -1; }
+#pragma unroll
+        for (int u = 0; u < NB; u++) r[u] = e[u] >= 0 ? s_off[e[u]] + atomicAdd(&s_cur[e[u]], 1) : -1;
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            const int i = i0 + 1024 * u;
+            if (i >= n_pairs) break;
+            pair_row[i] = r[u];
+            if (r[u] >= 0) row_pair[r[u]] = i;
+        }
     }
 }
 

@@ -1264,10 +1264,8 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
             Timer tm(s, 0); kr_sv_canon(cv, s->f32, st);
             mixer_in = s->hc.p;
         }
-        if (c.res_gate) {
-            KrSvGemm gg{}; gg.A = s->h.p; gg.lda = W; gg.W = l.rg1.p; gg.C = (float*)s->rg.p; gg.ldc = W; gg.M = T; gg.N = W; gg.K = W;
-            Timer tm(s, 1); kr_sv_gemm(gg, s->f32, st);
-        }
+        KrSvGemm gg{};                                   // residual gate: beside the mixer's projections at decode sizes
+        if (c.res_gate) { gg.A = s->h.p; gg.lda = W; gg.W = l.rg1.p; gg.C = (float*)s->rg.p; gg.ldc = W; gg.M = T; gg.N = W; gg.K = W; }
         g.A = mixer_in; g.lda = W; g.W = l.hw.p; g.C = hz; g.ldc = l.n_h; g.M = T; g.N = seq ? l.n_qkv : l.n_h; g.K = W;
         g.bias = d.ff_bias ? (const float*)l.h_bias.p : nullptr;
         if (l.has_lt()) { g.silu_lo = l.off_lt; g.silu_hi = l.off_lt + l.lt_cols(); }
@@ -1280,7 +1278,12 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
             if (d.mlp_kind == KR_SERVE_MLP_DENSE && d.ff_bias) ffd.bias = (const float*)l.down_b.p;
         }
         if (!seq && ff_f > 0) ff_formed = pair_up(g, ffd, hz + l.off_gu, l.n_h, l.off_gu, ff_f, ff_act, ff_limit, ff_alpha);
-        if (g.N > 0) { Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); }
+        if (gg.M > 0 && g.N > 0 && !s->f32 && kr_sv_strips_fits(gg) && kr_sv_strips_fits(g)) { Timer tm(s, 1); kr_sv_strips(g, gg, KrSvGemm{}, st); }
+        else {
+            Timer tm(s, 1);
+            if (gg.M > 0) kr_sv_gemm(gg, s->f32, st);
+            if (g.N > 0) kr_sv_gemm(g, s->f32, st);
+        }
         const SvLayer& kvl = d.kv_from >= 0 ? s->L[d.kv_from] : run;
         KrSvAttn a{};
         a.heads = d.heads; a.kv_heads = l.att_heads_kv(); a.dim = l.att_dim(); a.vdim = l.att_vdim();
@@ -1479,8 +1482,20 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
             if (has_ff && l.n_h > l.off_router) {
                 g = KrSvGemm{}; g.A = s->h.p; g.lda = W; g.W = (const char*)l.hw.p + (size_t)l.off_router * W * s->esz; g.C = hz + l.off_router; g.ldc = l.n_h; g.M = T; g.N = l.n_h - l.off_router; g.K = W;
                 g.bias = d.ff_bias ? (const float*)l.h_bias.p + l.off_router : nullptr;
-                if (ff_f > 0) ff_formed = pair_up(g, ffd, hz + l.off_gu, l.n_h, l.off_gu - l.off_router, ff_f, ff_act, ff_limit, ff_alpha);
-                Timer tm(s, 1); kr_sv_gemm(g, s->f32, st);
+                // decode sizes, dense: the activation leaves the strips of its factors, and what stands behind them has strips of its own
+                const int lo = l.off_gu - l.off_router, behind = g.N - lo - 2 * ff_f;
+                if (!s->f32 && d.mlp_kind == KR_SERVE_MLP_DENSE && ff_f > 0 && ff_f % 32 == 0 && ff_act != KR_SERVE_ACT_RELU2 && lo == 0 && kr_sv_strips_fits(g)) {
+                    KrSvGemm rest{}, pairs = g;
+                    pairs.glu_out = s->y.p; pairs.glu_lo = 0; pairs.glu_f = ff_f; pairs.glu_kind = ff_act; pairs.glu_limit = ff_limit; pairs.glu_alpha = ff_alpha;
+                    if (behind > 0) {
+                        rest = g; rest.W = (const char*)g.W + (size_t)2 * ff_f * W * s->esz; rest.C = g.C + 2 * ff_f; rest.N = behind; rest.bias = g.bias ? g.bias + 2 * ff_f : nullptr;
+                    }
+                    ff_formed = true;
+                    Timer tm(s, 1); kr_sv_strips(rest, KrSvGemm{}, pairs, st);
+                } else {
+                    if (ff_f > 0) ff_formed = pair_up(g, ffd, hz + l.off_gu, l.n_h, l.off_gu - l.off_router, ff_f, ff_act, ff_limit, ff_alpha);
+                    Timer tm(s, 1); kr_sv_gemm(g, s->f32, st);
+                }
             }
         }
         const float *dense = nullptr, *shared = nullptr, *rows = nullptr; const int* pair_pos = nullptr;

@@ -51,6 +51,9 @@ bool kr_sv_gemm_takes_host(const KrSvGemm& g, bool f32);
 bool kr_sv_gemm_pair(const KrSvGemm& e, const KrSvGemm& o, bool f32, hipStream_t st);
 // the forms for a bf16 store that kr_sv_gemm chooses from; _fits: shapes and alignment
 bool kr_sv_gemm_skinny_fits(const KrSvGemm& g);
+// decode sizes, bf16: up to three products (M = 0: none) of at most sixteen rows in one launch; the last one may be gate | up pairs alone (its glu fields set, columns outside the pairs untouched)
+bool kr_sv_strips_fits(const KrSvGemm& g);
+void kr_sv_strips(const KrSvGemm& a, const KrSvGemm& b, const KrSvGemm& c, hipStream_t st);
 bool kr_sv_gemm_skinny_acts(const KrSvGemm& g);
 void kr_sv_gemm_skinny(const KrSvGemm& g, hipStream_t st);
 void kr_sv_gemm_skinny_pair(const KrSvGemm& e, const KrSvGemm& o, hipStream_t st);

@@ -9,7 +9,7 @@ typedef float sk_f4 __attribute__((ext_vector_type(4)));
 constexpr int sk_red_floats(int MB, int NB, int WV) { return WV * (MB * NB < 4 ? MB * NB : 4) * 256; }
 
 // MB, NB: row and column blocks of 16; WV: waves.  bx: strip, by: problem row of a grouped problem; red: sk_red_floats of LDS, act (with ACT): the rows' activation [16 MB][K + 8].
-// GLU (NB = 2): the strip is 16 gate columns of g.glu_f and the 16 up columns that belong to them; their activation goes to g.glu_out, nothing to C.
+// GLU (NB = 2): the strip is 16 gate columns, counted from g.glu_lo, and the 16 up columns that belong to them; their activation goes to g.glu_out, nothing to C.
 template <int MB, int NB, int WV, bool ACT, bool GLU = false>
 __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const int by, float* red, uint16_t* act) {
     static_assert(!GLU || (NB == 2 && MB == 1), "a gate tile and its up tile");
@@ -29,7 +29,7 @@ __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const 
     const int ks = g.K / 32, s0 = ks * wave / WV, s1 = ks * (wave + 1) / WV, lda = g.K + 8;
     const uint16_t* wp[NB];
 #pragma unroll
-    for (int b = 0; b < NB; b++) wp[b] = W + (size_t)(GLU ? min(n0 + r, g.glu_f - 1) + b * g.glu_f : min(n0 + b * 16 + r, N - 1)) * g.K + q * 8;
+    for (int b = 0; b < NB; b++) wp[b] = W + (size_t)(GLU ? g.glu_lo + min(n0 + r, g.glu_f - 1) + b * g.glu_f : min(n0 + b * 16 + r, N - 1)) * g.K + q * 8;
     auto request = [&](gu4 (&wv)[U][NB], int s) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
@@ -107,6 +107,7 @@ __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const 
                     float gt = red[e], up = red[256 + e];
 #pragma unroll
                     for (int w = 1; w < WV; w++) { gt += red[w * TR * 256 + e]; up += red[(w * TR + 1) * 256 + e]; }
+                    if (g.bias) { gt += g.bias[g.glu_lo + n]; up += g.bias[g.glu_lo + g.glu_f + n]; }
                     const float wt = g.glu_row_w ? g.glu_row_w[m] : 1.0f;
                     ((uint16_t*)g.glu_out)[(size_t)m * g.glu_f + n] = kr_f32_to_bf16(gm_act_once(gt * wt, up * wt, g.glu_kind, g.glu_limit, g.glu_alpha));
                 }

@@ -1338,15 +1338,17 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
                 q.q_scale = q.k_scale = 1.0f; q.gate = hz + l.off_ogate; q.gate_ld = l.n_h; q.gate_act = 1;
             }
             q.ent_chunk0 = d_echunk; q.n_chunks = n_chunks; q.tok = (float4*)s->lin_tok.p; q.sbuf = (float*)s->lin_sbuf.p; q.nbuf = (float*)s->lin_nbuf.p; q.cmeta = (float*)s->lin_cm.p;
+            bool stepped = false;
             {
                 Timer tm(s, 3);
-                if (lin_chunked && l.chunkable() && kr_sv_lin_chunked_fits(d.dim, d.vdim)) kr_sv_lin_chunked(q, st);
+                if (rg_step && kr_sv_lin_step(q, s->f32, st)) stepped = true;
+                else if (lin_chunked && l.chunkable() && kr_sv_lin_chunked_fits(d.dim, d.vdim)) kr_sv_lin_chunked(q, st);
                 else if (lin_chunked && (l.wkv() || l.gla()) && kr_sv_lin_blocks_fit(d.dim, d.vdim)) kr_sv_lin_chan_blocks(q, st);
                 else if (lin_chunked && l.delta() && kr_sv_lin_blocks_fit(d.dim, d.vdim)) { q.aux = (float*)s->lin_aux.p; kr_sv_delta_blocks(q, st); }
                 else if (lin_chunked && kr_sv_lin_scan_wide_fits(q.kind, d.dim)) kr_sv_lin_scan_wide(q, st);
                 else kr_sv_lin_scan(q, st);
             }
-            { Timer tm(s, 2); kr_sv_lin_out(q, s->f32, st); }
+            if (!stepped) { Timer tm(s, 2); kr_sv_lin_out(q, s->f32, st); }
         } else if (l.rglru()) {
             KrSvRglru q{};
             q.y = hz; q.x = hz + d.rg_width; q.ld = l.n_h; q.y_b = (const float*)l.rg_yb.p; q.x_b = (const float*)l.rg_xb.p; q.conv = (const float*)l.rg_conv.p;

@@ -289,6 +289,8 @@ struct KrSvLin {
 };
 // token by token, the state in registers: decode steps and short portions
 void kr_sv_lin_scan(const KrSvLin& a, hipStream_t st);
+// steps of one token per request: kr_sv_lin_scan and kr_sv_lin_out in one launch (o is not written); false: not for this shape
+bool kr_sv_lin_step(const KrSvLin& a, bool f32, hipStream_t st);
 // prompt portions in blocks of 64 tokens on the f32 matrix instruction (rotation and scales applied to q / k in place first): within a block
 // o_t = g_t S_start^T q_t + sum_(s <= t) exp(u_t + w_s) (q_t . k_s) v_s, and S_end = g_last S_start + sum_s exp(u_last + w_s) k_s v_s^T; a short serial
 // launch carries S from block to block, the outputs of all blocks are formed in parallel.  Same state layout as kr_sv_lin_scan.

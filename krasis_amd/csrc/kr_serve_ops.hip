@@ -2162,6 +2162,113 @@ __global__ void __launch_bounds__(64) sv_lin_out_kernel(const KrSvLin a, T* __re
     }
 }
 
+// A step that brings one token per request: scan and output of a head in ONE launch, a workgroup per (request, head) whose waves own 16 value columns each (lanes, registers and
+// order of operations as in sv_lin_scan_kernel and sv_lin_out_kernel, so the bits are theirs).  What such a step waits for is not the state (64 KB per head at 128 x 128) but the
+// trips to memory one after the other, and the second launch; here everything that does not hang on something read before (the state behind its slot, q, k, v, rotation, gates,
+// norm) is requested first and waited for once.  dim = 4 DP rows exactly, so that a lane's rows are whole 16-byte pieces; other sizes stay with the two launches.
+// 2 requests, 16 heads of 128 x 128: 12.2 + 4.6 -> 7.6 us.
+template <int KIND, int DP>
+__global__ void __launch_bounds__(512) sv_lin_step_kernel(const KrSvLin a, const bool f32) {
+    constexpr bool ML = KIND == 3, GLA = KIND == 4, WKV = KIND == 7, DELTA = KIND == 8, SRC = GLA || WKV || DELTA;
+    constexpr int dim = 4 * DP, PAD = DP + 4;              // the four parts of a column read LDS DP + 4 apart: no two in one bank
+    __shared__ __attribute__((aligned(16))) float qs[4 * PAD], ks[4 * PAD], as[4 * PAD], us[4 * PAD], os[128];
+    const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, cb = tid >> 6, part = lane & 3, col = cb * 16 + (lane >> 2);
+    const int vdim = a.vdim, H = a.heads, ncb = (vdim + 15) / 16, nt = blockDim.x, half = a.rot_dims / 2;
+    const bool cv = col < vdim, fresh = a.pos[t] == 0;
+    const int sl = a.ent_slot[t];
+    float* Sg = a.state + (size_t)sl * a.state_stride + ((size_t)h * vdim + (cv ? col : 0)) * dim + part * DP;
+    float* nmg = a.nm + (size_t)sl * a.nm_stride + ((size_t)h * ncb + cb) * (dim + 4);
+    float4 S4[DP / 4], n4[DP / 4];
+#pragma unroll
+    for (int r = 0; r < DP / 4; r++) { S4[r] = *reinterpret_cast<const float4*>(Sg + 4 * r); if (ML) n4[r] = *reinterpret_cast<const float4*>(nmg + part * DP + 4 * r); }
+    float m = ML ? nmg[dim] : 0.0f;
+    const float* qp = SRC ? a.qsrc + (size_t)t * a.src_ld + (size_t)(h / a.qk_group) * dim : a.z + (size_t)t * a.ld + (size_t)h * dim;
+    const float* kp = SRC ? a.ksrc + (size_t)t * a.src_ld + (size_t)(h / a.qk_group) * dim : qp + (size_t)H * dim;
+    const float* vp = SRC ? a.vsrc + (size_t)t * a.src_ld + (size_t)h * vdim : a.z + (size_t)t * a.ld + (size_t)2 * H * dim + (size_t)h * vdim;
+    const float* gp = a.gate ? a.gate + (size_t)t * a.gate_ld + (size_t)h * vdim : a.z + (size_t)t * a.ld + (size_t)2 * H * dim + (size_t)H * vdim + (size_t)h * vdim;
+    const float v = cv ? vp[col] : 0.0f;
+    const float gz = tid < vdim ? gp[tid] : 0.0f, nw = a.norm_w && tid < vdim ? a.norm_w[a.norm_shared ? (size_t)tid : (size_t)h * vdim + tid] : 1.0f;
+    float av = 1.0f, bv = 1.0f;
+    if constexpr (KIND == 2) av = a.decay[h];
+    if constexpr (DELTA) { const float4 tk = a.tok[(size_t)t * H + h]; bv = tk.w; av = expf(tk.x); }
+    if constexpr (ML) {
+        const float* zg = a.z + (size_t)t * a.ld + (size_t)2 * H * dim + (size_t)2 * H * vdim;
+        float zi = zg[h] + a.i_bias[h], zf = zg[H + h] + a.f_bias[h];
+        if (a.gate_cap > 0.0f) { zi = a.gate_cap * tanhf(zi / a.gate_cap); zf = a.gate_cap * tanhf(zf / a.gate_cap); }
+        const float fg = fminf(zf, 0.0f) - log1pf(expf(-fabsf(zf)));           // log sigmoid
+        if (fresh) m = 0.0f;
+        const float mn = fmaxf(fg + m, zi);
+        av = expf(fg + m - mn); bv = expf(zi - mn); m = mn;
+    }
+    auto at = [](int d) { return d + 4 * (d / DP); };
+    for (int i = tid; i < 2 * dim; i += nt) {              // q, then k; the thread of a rotated pair's first element turns both
+        const int d = i & (dim - 1);
+        const bool isk = i >= dim;
+        const float* src = isk ? kp : qp;
+        float* dst = isk ? ks : qs;
+        const float sc = isk ? a.k_scale : a.q_scale;
+        if (d < half) {
+            const float2 c = a.cs[(size_t)t * half + d];
+            const float u = src[d] * sc, w = src[d + half] * sc;
+            dst[at(d)] = u * c.x - w * c.y; dst[at(d + half)] = w * c.x + u * c.y;
+        } else if (d >= 2 * half) dst[at(d)] = src[d] * sc;
+        if (!isk && GLA) {
+            const float z = a.gz[(size_t)t * a.gz_ld + (size_t)h * dim + d] + a.gz_bias[(size_t)h * dim + d];
+            as[at(d)] = expf((fminf(z, 0.0f) - log1pf(expf(-fabsf(z)))) * a.inv_tau);      // sigmoid(z)^(1 / tau)
+        }
+        if (!isk && WKV) { as[at(d)] = expf(a.gz[(size_t)t * a.gz_ld + (size_t)h * dim + d]); us[at(d)] = a.bonus[(size_t)h * dim + d]; }
+    }
+    __syncthreads();
+    float bvv = bv * v, po = 0.0f, pn = 0.0f;
+    const float *qr = qs + part * PAD, *kr = ks + part * PAD, *ar = as + part * PAD, *ur = us + part * PAD;
+    float* S = reinterpret_cast<float*>(S4); float* n = reinterpret_cast<float*>(n4);
+#pragma unroll
+    for (int r = 0; r < DP; r++) { S[r] = fresh || !cv ? 0.0f : S[r]; if (ML) n[r] = fresh ? 0.0f : n[r]; }
+    if constexpr (DELTA) {                                 // the decayed state's value at k first: what is written is the rest of v
+        float pk = 0.0f;
+#pragma unroll
+        for (int r = 0; r < DP; r++) { S[r] *= av; pk = __builtin_fmaf(S[r], kr[r], pk); }
+        pk += __shfl_xor(pk, 1); pk += __shfl_xor(pk, 2);
+        bvv = bv * (v - pk);
+    }
+#pragma unroll
+    for (int r = 0; r < DP; r++) {
+        if constexpr (WKV) {                               // the read-out comes before the write
+            const float kv = kr[r] * bvv;
+            po = __builtin_fmaf(__builtin_fmaf(ur[r], kv, S[r]), qr[r], po);
+            S[r] = __builtin_fmaf(ar[r], S[r], kv);
+            continue;
+        }
+        if constexpr (GLA) S[r] = __builtin_fmaf(kr[r], bvv, ar[r] * S[r]);
+        else if constexpr (DELTA) S[r] = __builtin_fmaf(kr[r], bvv, S[r]);
+        else S[r] = __builtin_fmaf(kr[r], bvv, av * S[r]);
+        po = __builtin_fmaf(S[r], qr[r], po);
+        if constexpr (ML) { n[r] = __builtin_fmaf(bv, kr[r], av * n[r]); pn = __builtin_fmaf(n[r], qr[r], pn); }
+    }
+    po += __shfl_xor(po, 1); po += __shfl_xor(po, 2);
+    if constexpr (ML) {
+        pn += __shfl_xor(pn, 1); pn += __shfl_xor(pn, 2);
+        po = po / (fmaxf(fabsf(pn), expf(-m)) + 1e-6f);
+    }
+    if (part == 0 && cv) os[col] = po;
+#pragma unroll
+    for (int r = 0; r < DP / 4; r++) {
+        if (cv) *reinterpret_cast<float4*>(Sg + 4 * r) = S4[r];
+        if (ML && (lane >> 2) == 0) *reinterpret_cast<float4*>(nmg + part * DP + 4 * r) = n4[r];
+    }
+    if (ML && lane == 0) nmg[dim] = m;
+    __syncthreads();
+    float ss = 0.0f;
+    for (int d = lane; d < vdim; d += 64) ss = __builtin_fmaf(os[d], os[d], ss);
+    const float inv = 1.0f / sqrtf(sv_wave_sum(ss) / (float)vdim + a.eps);
+    if (tid < vdim) {
+        const float sg = 1.0f / (1.0f + expf(-gz)), o = os[tid] * inv * nw;
+        const bool sig = a.gate_act ? a.gate_act == 2 : ML;
+        const size_t at_o = ((size_t)t * H + h) * vdim + tid;
+        if (f32) ((float*)a.out)[at_o] = o * (sig ? sg : gz * sg); else sv_st((uint16_t*)a.out + at_o, o * (sig ? sg : gz * sg));
+    }
+}
+
 // the selective state-space mixer after its scan (KrSvSsdOut): one workgroup per token, the gated row in LDS
 template <typename T>
 __global__ void __launch_bounds__(256) sv_ssd_out_kernel(const KrSvSsdOut a, T* __restrict__ out) {
@@ -2581,6 +2688,19 @@ void kr_sv_lin_scan(const KrSvLin& a, hipStream_t st) {
     if (a.kind == 3) SV_LIN_D(3); else if (a.kind == 4) SV_LIN_D(4); else if (a.kind == 5) SV_LIN_D(5); else if (a.kind == 7) SV_LIN_D(7); else if (a.kind == 8) SV_LIN_D(8); else SV_LIN_D(2);
 #undef SV_LIN_D
 #undef SV_LIN
+}
+// one token per request; false: the shape is not of those (dim 32, 64 or 128 on 16-byte boundaries, at most eight waves of value columns)
+bool kr_sv_lin_step(const KrSvLin& a, bool f32, hipStream_t st) {
+    const int dp = a.dim / 4, ncb = (a.vdim + 15) / 16;
+    if (a.kind == 5 || a.T <= 0 || a.T != a.n_entries || a.dim % 4 != 0 || (dp != 8 && dp != 16 && dp != 32) || ncb > 8 || a.rot_dims > a.dim) return false;
+    if ((uintptr_t)a.state % 16 != 0 || a.state_stride % 4 != 0 || (a.kind == 3 && ((uintptr_t)a.nm % 16 != 0 || a.nm_stride % 4 != 0))) return false;
+    const dim3 grid(a.T, a.heads);
+#define SV_STEP(K_, DP_) hipLaunchKernelGGL((sv_lin_step_kernel<K_, DP_>), grid, dim3(64 * ncb), 0, st, a, f32)
+#define SV_STEP_D(K_) do { if (dp == 8) SV_STEP(K_, 8); else if (dp == 16) SV_STEP(K_, 16); else SV_STEP(K_, 32); } while (0)
+    if (a.kind == 3) SV_STEP_D(3); else if (a.kind == 4) SV_STEP_D(4); else if (a.kind == 7) SV_STEP_D(7); else if (a.kind == 8) SV_STEP_D(8); else SV_STEP_D(2);
+#undef SV_STEP_D
+#undef SV_STEP
+    return true;
 }
 // the workgroup form for prompt portions of kinds 4 and 5; false: the shape does not fit its LDS buffers (the caller takes kr_sv_lin_scan)
 static size_t sv_scanw_lds(int kind, int dim) {

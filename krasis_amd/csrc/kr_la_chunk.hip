@@ -17,8 +17,9 @@
 // Every product runs on the bf16 MFMA with its f32 operands split into two bf16 values (x = hi + lo, hi = bf16(x), lo = bf16(x - hi)) and
 // acc += hi.hi + hi.lo + lo.hi: three v_mfma_f32_32x32x16_bf16 (96 matrix-pipe cycles per 16 k) instead of eight v_mfma_f32_32x32x2_f32 (512),
 // products exact to ~2^-17 relative, f32 accumulation, f32 exponent range.  The prep kernel splits in registers (lc_blk_s); W, Q' and K^T leave it
-// already split into planes (and K transposed), so the SCAN -- the sequential part -- stages them with plain 16-byte copies (lc_blk3); only the state
-// slice and the delta rows are split inside the scan (16 values per lane and step).  Round 2 ran everything on v_mfma_f32_32x32x2_f32.
+// already split into planes (and K transposed), in the order of the scan's matrix fragments (lc_frag): the SCAN -- the sequential part -- takes them straight to registers,
+// one sub-chunk ahead (no wave shares them with another, and staging them through LDS was a quarter of its step: 32 heads, 4096 tokens 268 -> 206 us a launch);
+// only the state slice and the delta rows are split inside the scan (16 values per lane and step).  Round 2 ran everything on v_mfma_f32_32x32x2_f32.
 // (tolerance mode: tests/test_attn_fast_gpu.py states the bound.)  All exponents are differences G_t - G_j <= 0: nothing overflows, and a
 // decay that underflows gives 0, not NaN (g is clamped at -80 per token).
 #include <hip/hip_runtime.h>
@@ -64,7 +65,7 @@ __device__ __forceinline__ void lc_split(float x, uint16_t& hi, uint16_t& lo) {
 #define LC_PREP_LDS ((3 * LC_T * LC_LD + 2 * LC_T * LC_LS + 3 * LC_T + 2 * LC_T) * 4)      // K, Q, V tiles, L, B, G / b / b e^G, (fused) the 2 x 64 inverse norms
 #define LC_PA 272      // bytes per row of a [rows][128 k] bf16 plane in LDS (256 + 16: the 16-byte fragment reads of 32 consecutive rows spread over the banks)
 #define LC_PT 144      // bytes per row of a [rows][64 k] bf16 plane
-#define LC_SCAN_LDS (4 * LC_T * LC_PA + 2 * LC_D * LC_PT + 2 * 32 * LC_PA + 2 * 32 * LC_PT + LC_T * 4)
+#define LC_SCAN_LDS (2 * 32 * LC_PA + 2 * 32 * LC_PT + 2 * LC_T * 4)
 
 struct KrLacArgs {
     const float *q, *k, *v, *gexp, *beta;   // [C][nv*128] x3, [C][nv] x2   (unused when `fused`)
@@ -73,15 +74,14 @@ struct KrLacArgs {
     // 540 MB of q / k / v / z stores per 8192 tokens and the prep's re-read of them disappear from the tolerance pass
     int fused; const float* qkvz; int ld_qkvz; const float* ba; int ld_ba; const float *conv_state, *conv_w, *a_log, *dt_bias; float scale; int nk, hr;
     float *Y, *G;                           // [n_sub*nv][64][128], [n_sub*nv][64]
-    uint16_t *Wh, *Wl, *Qh, *Ql;            // bf16 planes [n_sub*nv][64][128] of W and Q' (hi, lo)
-    uint16_t *Kh, *Kl;                      // bf16 planes [n_sub*nv][128][64] of K^T
+    uint16_t *Wh, *Wl, *Qh, *Ql;            // bf16 planes [n_sub*nv] of W and Q' [64][128] (hi, lo), in fragment order (lc_frag)
+    uint16_t *Kh, *Kl;                      // bf16 planes [n_sub*nv] of K^T [128][64], in fragment order
     float *out, *state;                     // [C][nv*128]; [nv][128][128]
     int nv, C, n_sub;
 };
 
 // acc(32x32) += A(32 x K) . B(K x 32) on the bf16 MFMA with split operands (x = hi + lo in bf16: ~2^-17 relative per product, f32 accumulation, f32 range).
 //   A_ROWS: A[m][k] = A[m*lda + k] (k contiguous) else A[m][k] = A[k*lda + m];   B_ROWS: B[k][n] = B[n*ldb + k] (k contiguous) else B[k*ldb + n]
-struct LcNone { __device__ __forceinline__ void operator()(int) const {} };
 // f32 operands in LDS, split ON THE FLY (the prep kernel has no LDS left for planes): lane (r, h) takes
 // k = kb + 8 h .. + 8 of row / column r of both operands, splits the 16 values (3 VALU each) and issues hi.hi + hi.lo + lo.hi on the bf16 MFMA --
 // 96 matrix-pipe cycles + ~200 VALU cycles per 16 k against 512 cycles of f32 MFMA.
@@ -120,6 +120,9 @@ __device__ __forceinline__ void lc_blk_s(v16f& acc, const float* A, int lda, con
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, acc, 0, 0, 0);
     }
 }
+// The planes that the prep launch leaves are stored in the order in which the scan's matrix instructions take them: chunk (row, c) of 8 consecutive k goes to lane
+// (row & 31) + 32 (c & 1) of the 1-KiB fragment of row block row / 32 and k step c / 2.  COLS: k of a row.
+template <int COLS> __device__ __forceinline__ int lc_frag(int row, int c) { return ((row >> 5) * (COLS / 16) + (c >> 1)) * 64 + (c & 1) * 32 + (row & 31); }
 __device__ __forceinline__ int lc_row(int r, int lane) { return (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5); }   // accumulator register r -> block row
 
 #define LC_PTH 512     // threads of a prep workgroup: its LDS (134 KB) allows one per CU, so the workgroup itself brings the second wave per SIMD that overlaps
@@ -234,10 +237,10 @@ __global__ void __launch_bounds__(LC_PTH) kr_lac_prep_kernel(KrLacArgs a) {
             lc_split(Kt[(tb + 2 * i) * LC_LD + d], h0, l0); lc_split(Kt[(tb + 2 * i + 1) * LC_LD + d], h1, l1);
             hw[i] = (uint32_t)h0 | ((uint32_t)h1 << 16); lw[i] = (uint32_t)l0 | ((uint32_t)l1 << 16);
         }
-        lc_u4* kh = reinterpret_cast<lc_u4*>(a.Kh + (tile * LC_D + (size_t)d * LC_T + tb));      // tile * LC_D = first element of this tile's [128][64] plane
-        lc_u4* kl = reinterpret_cast<lc_u4*>(a.Kl + (tile * LC_D + (size_t)d * LC_T + tb));
+        lc_u4* kh = reinterpret_cast<lc_u4*>(a.Kh + tile * LC_D) + lc_frag<LC_T>(d, tb / 8);      // tile * LC_D = first element of this tile's plane; the second chunk is the other lane half's
+        lc_u4* kl = reinterpret_cast<lc_u4*>(a.Kl + tile * LC_D) + lc_frag<LC_T>(d, tb / 8);
 #pragma unroll
-        for (int i = 0; i < 2; i++) { kh[i] = lc_u4{hw[4 * i], hw[4 * i + 1], hw[4 * i + 2], hw[4 * i + 3]}; kl[i] = lc_u4{lw[4 * i], lw[4 * i + 1], lw[4 * i + 2], lw[4 * i + 3]}; }
+        for (int i = 0; i < 2; i++) { kh[32 * i] = lc_u4{hw[4 * i], hw[4 * i + 1], hw[4 * i + 2], hw[4 * i + 3]}; kl[32 * i] = lc_u4{lw[4 * i], lw[4 * i + 1], lw[4 * i + 2], lw[4 * i + 3]}; }
     }
     // ---- K K^T -> L (strictly lower, decayed, row-scaled by b) and Q K^T -> B (lower incl. diagonal, decayed); the (0,1) blocks are zero
     if (wave < 6) {
@@ -351,11 +354,11 @@ __global__ void __launch_bounds__(LC_PTH) kr_lac_prep_kernel(KrLacArgs a) {
         LC_STAMP(6);
     }
     __syncthreads();
-    // ---- W (K tile), Q' (Q tile) -> their bf16 planes, Y (V tile) -> f32, all with 16-byte stores: chunk u = 8 consecutive columns of row u >> 4
+    // ---- W (K tile), Q' (Q tile) -> their bf16 planes, Y (V tile) -> f32, all with 16-byte stores: planes in the scan's order (chunk u of a plane: lc_frag), Y in rows
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-        const int u = tid + LC_PTH * i, t = u >> 4, c8 = (u & 15) * 8;
-        const size_t o = (tile + t) * LC_D + c8;
+        const int u = tid + LC_PTH * i, t = (u >> 9) * 32 + (u & 31), c8 = ((u >> 5) & 15) * 8, yt = u >> 4, yc = (u & 15) * 8;
+        const size_t o = tile * LC_D + (size_t)u * 8, oy = (tile + yt) * LC_D + yc;
         auto planes = [&](const float* src, uint16_t* ph, uint16_t* pl) {
             const f4 v0 = *reinterpret_cast<const f4*>(src + t * LC_LD + c8), v1 = *reinterpret_cast<const f4*>(src + t * LC_LD + c8 + 4);
             const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
@@ -367,33 +370,30 @@ __global__ void __launch_bounds__(LC_PTH) kr_lac_prep_kernel(KrLacArgs a) {
         };
         planes(Kt, a.Wh, a.Wl);
         planes(Qt, a.Qh, a.Ql);
-        *reinterpret_cast<f4*>(a.Y + o) = *reinterpret_cast<const f4*>(Vt + t * LC_LD + c8);
-        *reinterpret_cast<f4*>(a.Y + o + 4) = *reinterpret_cast<const f4*>(Vt + t * LC_LD + c8 + 4);
+        *reinterpret_cast<f4*>(a.Y + oy) = *reinterpret_cast<const f4*>(Vt + yt * LC_LD + yc);
+        *reinterpret_cast<f4*>(a.Y + oy + 4) = *reinterpret_cast<const f4*>(Vt + yt * LC_LD + yc + 4);
     }
 }
 
-// acc(32x32) += A(32 x K) . B(K x 32) with both operands given as bf16 (hi, lo) planes whose rows hold k contiguously: A row = output row, B row =
-// output COLUMN (B is stored transposed).  Lane (r = lane & 31, h = lane >> 5) supplies k = 16 ks + 8 h .. + 8 of row r of both operands (one 16-byte
-// read per plane); three MFMAs per 16 k: hi.hi + hi.lo + lo.hi.  `between(ks)` issues the caller's global prefetch under the MFMAs of step ks.
-template <int K, typename F = LcNone>
-__device__ __forceinline__ void lc_blk3(v16f& acc, const char* Ah, const char* Al, int lda, const char* Bh, const char* Bl, int ldb, int lane, F&& between = LcNone()) {
+// acc(32x32) += A(32 x K) . B(K x 32), both operands as bf16 (hi, lo) planes.  A: this wave's fragments, in registers (a[0] hi, a[1] lo); each is requested again, for the
+// next sub-chunk (`again(plane, ks)`), as soon as the step that used it has been issued.  B: rows of LDS planes that hold k contiguously, B row = output COLUMN (stored
+// transposed): lane (r = lane & 31, h = lane >> 5) supplies k = 16 ks + 8 h .. + 8 of row r of both operands.  Three MFMAs per 16 k: hi.hi + hi.lo + lo.hi.
+template <int K, typename F>
+__device__ __forceinline__ void lc_blk3(v16f& acc, lc_u4 (&a)[2][K / 16], const char* Bh, const char* Bl, int ldb, int lane, F&& again) {
     const int r = lane & 31, h = lane >> 5;
-    const char* ah = Ah + r * lda + h * 16; const char* al = Al + r * lda + h * 16;
     const char* bh = Bh + r * ldb + h * 16; const char* bl = Bl + r * ldb + h * 16;
-    lc_b8 fa[2][2], fb[2][2];
-    auto fetch = [&](int ks, int buf) {
-        fa[buf][0] = *reinterpret_cast<const lc_b8*>(ah + ks * 32); fa[buf][1] = *reinterpret_cast<const lc_b8*>(al + ks * 32);
-        fb[buf][0] = *reinterpret_cast<const lc_b8*>(bh + ks * 32); fb[buf][1] = *reinterpret_cast<const lc_b8*>(bl + ks * 32);
-    };
+    lc_b8 fb[2][2];
+    auto fetch = [&](int ks, int buf) { fb[buf][0] = *reinterpret_cast<const lc_b8*>(bh + ks * 32); fb[buf][1] = *reinterpret_cast<const lc_b8*>(bl + ks * 32); };
     fetch(0, 0);
 #pragma unroll
     for (int ks = 0; ks < K / 16; ks++) {
         if (ks + 1 < K / 16) fetch(ks + 1, (ks + 1) & 1);
-        between(ks);
         const int b = ks & 1;
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[b][0], fb[b][0], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[b][0], fb[b][1], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[b][1], fb[b][0], acc, 0, 0, 0);
+        const lc_b8 ah = __builtin_bit_cast(lc_b8, a[0][ks]), al = __builtin_bit_cast(lc_b8, a[1][ks]);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, fb[b][0], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, fb[b][1], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, fb[b][0], acc, 0, 0, 0);
+        a[0][ks] = again(0, ks); a[1][ks] = again(1, ks);
         __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -414,11 +414,9 @@ __device__ __forceinline__ void lc_store_t(const float (&v)[16], char* Ph, char*
 
 __global__ void __launch_bounds__(256) kr_lac_scan_kernel(KrLacArgs a) {
     extern __shared__ __attribute__((aligned(16))) char lsm[];
-    char* Whs = lsm; char* Wls = Whs + LC_T * LC_PA; char* Qhs = Wls + LC_T * LC_PA; char* Qls = Qhs + LC_T * LC_PA;      // [64 t][128 k]
-    char* Khs = Qls + LC_T * LC_PA; char* Kls = Khs + LC_D * LC_PT;                                                       // K^T [128 d][64 t]
-    char* Shs = Kls + LC_D * LC_PT; char* Sls = Shs + 32 * LC_PA;                                                         // S^T slice [32 cols][128 d]
-    char* Uhs = Sls + 32 * LC_PA; char* Uls = Uhs + 32 * LC_PT;                                                           // U'^T [32 cols][64 t]
-    float* Gs = reinterpret_cast<float*>(Uls + 32 * LC_PT);
+    char* Shs = lsm; char* Sls = Shs + 32 * LC_PA;                                                         // S^T slice [32 cols][128 d]
+    char* Uhs = Sls + 32 * LC_PA; char* Uls = Uhs + 32 * LC_PT;                                            // U'^T [32 cols][64 t]
+    float* Gs2 = reinterpret_cast<float*>(Uls + 32 * LC_PT);                                               // [2][64], by parity of the sub-chunk
     const int bid = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // the 4 column slices of one head read the same W / Q' / K tiles: keep them on one XCD (workgroup id % 8) so the re-reads hit its L2
     int h, slice;
@@ -430,22 +428,23 @@ __global__ void __launch_bounds__(256) kr_lac_scan_kernel(KrLacArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; r++) S[r] = Sg[(size_t)(wave * 32 + lc_row(r, lane)) * LC_D + col];
     lc_store_t(S, Shs, Sls, LC_PA, wave * 32, lane);
-    // plane chunk u = tid + 256 i (i < 4) of 16 bytes: W / Q' planes [64][128] -> row u >> 4, chunk u & 15;  K^T planes [128][64] -> row u >> 3, chunk u & 7
-    const size_t tile_elems = (size_t)LC_T * LC_D, tile_stride = (size_t)a.nv * tile_elems;      // elements per tile / between sub-chunks
-    const lc_u4* pWh = reinterpret_cast<const lc_u4*>(a.Wh + (size_t)h * tile_elems) + tid; const lc_u4* pWl = reinterpret_cast<const lc_u4*>(a.Wl + (size_t)h * tile_elems) + tid;
-    const lc_u4* pQh = reinterpret_cast<const lc_u4*>(a.Qh + (size_t)h * tile_elems) + tid; const lc_u4* pQl = reinterpret_cast<const lc_u4*>(a.Ql + (size_t)h * tile_elems) + tid;
-    const lc_u4* pKh = reinterpret_cast<const lc_u4*>(a.Kh + (size_t)h * tile_elems) + tid; const lc_u4* pKl = reinterpret_cast<const lc_u4*>(a.Kl + (size_t)h * tile_elems) + tid;
-    lc_u4 pf[6][4]; float pg = 0.0f;
-#define LC_FETCH3(SUB, P, I) { const size_t o_ = (size_t)(SUB) * (tile_stride / 8) + 256 * (I); \
-        pf[P][I] = (P) == 0 ? pWh[o_] : (P) == 1 ? pWl[o_] : (P) == 2 ? pQh[o_] : (P) == 3 ? pQl[o_] : (P) == 4 ? pKh[o_] : pKl[o_]; }
+    // this wave's fragments of one sub-chunk: W (waves 0, 1) or Q' (2, 3), its half of the rows; K^T, its quarter of the state rows.  Nothing is shared between waves, so they come
+    // straight to registers: 24 requests of 1 KiB per wave and sub-chunk, one sub-chunk ahead
+    const size_t tile_elems = (size_t)LC_T * LC_D, tile_chunks = (size_t)a.nv * tile_elems / 8;      // elements per tile; chunks between sub-chunks
+    const int rbw = wave & 1;
+    const lc_u4* pa[2] = {reinterpret_cast<const lc_u4*>((wave < 2 ? a.Wh : a.Qh) + (size_t)h * tile_elems) + rbw * 512 + lane, reinterpret_cast<const lc_u4*>((wave < 2 ? a.Wl : a.Ql) + (size_t)h * tile_elems) + rbw * 512 + lane};
+    const lc_u4* pk[2] = {reinterpret_cast<const lc_u4*>(a.Kh + (size_t)h * tile_elems) + wave * 256 + lane, reinterpret_cast<const lc_u4*>(a.Kl + (size_t)h * tile_elems) + wave * 256 + lane};
+    lc_u4 fa[2][8], fk[2][4]; float pg = 0.0f;
 #pragma unroll
-    for (int p = 0; p < 6; p++)
+    for (int p = 0; p < 2; p++) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) LC_FETCH3(0, p, i)
-    if (tid < LC_T) pg = a.G[(size_t)h * LC_T + tid];
+        for (int i = 0; i < 8; i++) fa[p][i] = pa[p][64 * i];
+#pragma unroll
+        for (int i = 0; i < 4; i++) fk[p][i] = pk[p][64 * i];
+    }
+    if (tid < LC_T) Gs2[tid] = a.G[(size_t)h * LC_T + tid];
     // the addend of the first product (Y rows for waves 0,1; O_0 rows, written by the prep kernel, for waves 2,3) is requested ONE STEP AHEAD as well:
     // with the products at bf16 rate a step is shorter than a memory round trip
-    const int rbw = wave & 1;
     float yn[16];
     auto fetch_y = [&](int sb) {
         const size_t tl = ((size_t)sb * a.nv + h) * LC_T;
@@ -459,20 +458,12 @@ __global__ void __launch_bounds__(256) kr_lac_scan_kernel(KrLacArgs a) {
         }
     };
     fetch_y(0);
+    __syncthreads();
     for (int sub = 0; sub < a.n_sub; sub++) {
         const int c0 = sub * LC_T, n = min(LC_T, a.C - c0);
         const int nxt = min(sub + 1, a.n_sub - 1);     // the last step re-requests its own tiles: no branch in the product loop
+        const float* Gs = Gs2 + (sub & 1) * LC_T;
         if (sub == 1) LC_STAMP(10);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int u = tid + 256 * i, ro = (u >> 4) * LC_PA + (u & 15) * 16, ko = (u >> 3) * LC_PT + (u & 7) * 16;
-            *reinterpret_cast<lc_u4*>(Whs + ro) = pf[0][i]; *reinterpret_cast<lc_u4*>(Wls + ro) = pf[1][i];
-            *reinterpret_cast<lc_u4*>(Qhs + ro) = pf[2][i]; *reinterpret_cast<lc_u4*>(Qls + ro) = pf[3][i];
-            *reinterpret_cast<lc_u4*>(Khs + ko) = pf[4][i]; *reinterpret_cast<lc_u4*>(Kls + ko) = pf[5][i];
-        }
-        if (tid < LC_T) Gs[tid] = pg;
-        __syncthreads();
-        if (sub == 1) LC_STAMP(11);
         // ---- waves 0,1: U = Y - W S (row halves);  waves 2,3: O = O_0 + Q' S.  The Y / O_0 values are requested FIRST (the memory counter is in
         // order: waiting for them must not wait for the prefetch), then the next sub-chunk's planes are requested from inside the product loop
         {
@@ -486,13 +477,7 @@ __global__ void __launch_bounds__(256) kr_lac_scan_kernel(KrLacArgs a) {
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[i] = 0.0f;
             if (sub == 1) LC_STAMP(12);
-            lc_blk3<LC_D>(acc, (wave < 2 ? Whs : Qhs) + rb * 32 * LC_PA, (wave < 2 ? Wls : Qls) + rb * 32 * LC_PA, LC_PA, Shs, Sls, LC_PA, lane, [&](int ks) {
-                // 24 requests over 8 steps: plane ks >> 1 ... two planes per pair of steps, in plane order
-                if (ks < 6) {
-#pragma unroll
-                    for (int i = 0; i < 4; i++) LC_FETCH3(nxt, ks, i)
-                }
-            });
+            lc_blk3<LC_D>(acc, fa, Shs, Sls, LC_PA, lane, [&](int p, int ks) { return pa[p][(size_t)nxt * tile_chunks + 64 * ks]; });
             if (sub == 1) LC_STAMP(13);
             const float gT = Gs[LC_T - 1];
             if (wave < 2) {
@@ -514,14 +499,16 @@ __global__ void __launch_bounds__(256) kr_lac_scan_kernel(KrLacArgs a) {
             v16f sa;
 #pragma unroll
             for (int r = 0; r < 16; r++) sa[r] = S[r] * gam;
-            lc_blk3<LC_T>(sa, Khs + wave * 32 * LC_PT, Kls + wave * 32 * LC_PT, LC_PT, Uhs, Uls, LC_PT, lane);
+            lc_blk3<LC_T>(sa, fk, Uhs, Uls, LC_PT, lane, [&](int p, int ks) { return pk[p][(size_t)nxt * tile_chunks + 64 * ks]; });
 #pragma unroll
             for (int r = 0; r < 16; r++) S[r] = sa[r];
         }
         if (sub == 1) LC_STAMP(16);
-        __syncthreads();              // every wave has read S^T (first product of this step) and U'^T before they are rewritten
-        if (sub == 1) LC_STAMP(17);
+        // S^T was last read before the barrier above, U'^T and the other half of Gs2 are next written behind the one below
         lc_store_t(S, Shs, Sls, LC_PA, wave * 32, lane);
+        if (tid < LC_T) Gs2[((sub + 1) & 1) * LC_T + tid] = pg;
+        if (sub == 1) LC_STAMP(17);
+        __syncthreads();
         if (sub == 1) LC_STAMP(18);
         if (sub == 2) LC_STAMP(19);
     }

@@ -60,9 +60,9 @@ __device__ __forceinline__ void lc_split(float x, uint16_t& hi, uint16_t& lo) {
 #define LC_T 64
 #define LC_D 128
 #define LC_LD 132      // LDS row stride (floats) of the 64 x 128 tiles: rows 4 banks apart -> the float4 k-contiguous reads are conflict-free
-#define LC_LS 68       // row stride of the 64 x 64 matrices
-#define LC_SS 40       // row stride of the 32-column state / delta slices: rows k and k+4 are 32 banks apart
-#define LC_PREP_LDS ((3 * LC_T * LC_LD + 2 * LC_T * LC_LS + 3 * LC_T + 2 * LC_T) * 4)      // K, Q, V tiles, L, B, G / b / b e^G, (fused) the 2 x 64 inverse norms
+#define LC_LS 36       // row stride of the 32 x 32 blocks of L and B
+#define LC_LB (32 * LC_LS)
+#define LC_PREP_LDS ((2 * LC_T * LC_LD + 3 * LC_LB + 2 * LC_T) * 4)      // K tile, Q / V tile, three blocks of L / B, G and b
 #define LC_PA 272      // bytes per row of a [rows][128 k] bf16 plane in LDS (256 + 16: the 16-byte fragment reads of 32 consecutive rows spread over the banks)
 #define LC_PT 144      // bytes per row of a [rows][64 k] bf16 plane
 #define LC_SCAN_LDS (2 * 32 * LC_PA + 2 * 32 * LC_PT + 2 * LC_T * 4)
@@ -125,24 +125,24 @@ __device__ __forceinline__ void lc_blk_s(v16f& acc, const float* A, int lda, con
 template <int COLS> __device__ __forceinline__ int lc_frag(int row, int c) { return ((row >> 5) * (COLS / 16) + (c >> 1)) * 64 + (c & 1) * 32 + (row & 31); }
 __device__ __forceinline__ int lc_row(int r, int lane) { return (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5); }   // accumulator register r -> block row
 
-#define LC_PTH 512     // threads of a prep workgroup: its LDS (134 KB) allows one per CU, so the workgroup itself brings the second wave per SIMD that overlaps
-                       // the split arithmetic of one wave with the LDS / MFMA latency of another (256 threads: 24.7 us per workgroup, 512: see lac_timing)
-__global__ void __launch_bounds__(LC_PTH) kr_lac_prep_kernel(KrLacArgs a) {
+#define LC_PTH 512
+// What bounds the launch is the latency of its phases, each with a barrier behind it (a workgroup moves 230 KB, a tenth of its time at the memory's rate), so two workgroups share
+// a compute unit: one tile holds Q and then V (Q' needs Q again only element by element: registers), one region the three blocks of L, then T11 and T22 in their places, then
+// those of B (registers meanwhile), the rows' norms before all of them.  137 KB -> exactly half of the 160; 32 heads, 2752 tokens 175 -> 125 us a launch, 8192 487 -> 330.
+__global__ void __launch_bounds__(LC_PTH, 4) kr_lac_prep_kernel(KrLacArgs a) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    float* Kt = lds; float* Qt = Kt + LC_T * LC_LD; float* Vt = Qt + LC_T * LC_LD; float* Lm = Vt + LC_T * LC_LD; float* Bm = Lm + LC_T * LC_LS;
-    float* Gs = Bm + LC_T * LC_LS; float* bs = Gs + LC_T; float* bg = bs + LC_T;
+    float* Kt = lds; float* Qt = Kt + LC_T * LC_LD; float* Vt = Qt; float* Lm = Qt + LC_T * LC_LD;
+    float* Gs = Lm + 3 * LC_LB; float* bs = Gs + LC_T;
     const int sub = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c0 = sub * LC_T, n = min(LC_T, a.C - c0);
     const size_t ld = (size_t)a.nv * LC_D, tile = ((size_t)sub * a.nv + h) * LC_T;
     LC_STAMP(0);
-    float* nrm = bg + LC_T;       // [64][2] inverse L2 norms of the q / k rows (fused form)
-    if (a.fused) {
-        // ---- the tiles from the in-projection's output: thread = (4 consecutive tokens, 4 consecutive channels), three passes (q, k, v); the 4-tap window of the four
-        // tokens is 7 rows of 16 bytes.  Tap j of token t is X(t - 3 + j): a chunk row for >= 0, carried conv slot 4 + i for i < 0 (kr_pfm_la_conv_kernel).
-        const int kh = h / a.hr, rr = h % a.hr, gd = 2 * LC_D + 2 * LC_D * a.hr, key_dim = a.nk * LC_D;
-        const int tg = tid >> 5, c = (tid & 31) * 4;
-#pragma unroll 1
-        for (int arr = 0; arr < 3; arr++) {
+    float* nrm = Lm;              // [64][2] inverse L2 norms of the q / k rows (fused form)
+    // ---- a tile from the in-projection's output (0 q, 1 k, 2 v; v leaves scaled by the gates b): thread = (4 consecutive tokens, 4 consecutive channels); the 4-tap window of the
+    // four tokens is 7 rows of 16 bytes.  Tap j of token t is X(t - 3 + j): a chunk row for >= 0, carried conv slot 4 + i for i < 0 (kr_pfm_la_conv_kernel).
+    const int kh = a.fused ? h / a.hr : 0, rr = a.fused ? h % a.hr : 0;
+    auto conv = [&](int arr) {
+        const int gd = 2 * LC_D + 2 * LC_D * a.hr, key_dim = a.nk * LC_D, tg = tid >> 5, c = (tid & 31) * 4;
             const int ch = arr == 0 ? kh * LC_D + c : (arr == 1 ? key_dim + kh * LC_D + c : 2 * key_dim + h * LC_D + c);       // conv channel of column c
             const int off = arr == 0 ? c : (arr == 1 ? LC_D + c : 2 * LC_D + rr * LC_D + c);                                     // its column inside the key head's group
             const float* col = a.qkvz + (size_t)kh * gd + off;
@@ -157,7 +157,7 @@ __global__ void __launch_bounds__(LC_PTH) kr_lac_prep_kernel(KrLacArgs a) {
                 if (i < 0) x[j] = float4{cs[4 + i], cs[8 + i], cs[12 + i], cs[16 + i]};
                 else x[j] = i < a.C ? *reinterpret_cast<const float4*>(col + (size_t)i * a.ld_qkvz) : float4{0.0f, 0.0f, 0.0f, 0.0f};
             }
-            float* T = arr == 0 ? Qt : (arr == 1 ? Kt : Vt);
+            float* T = arr == 1 ? Kt : Qt;
 #pragma unroll
             for (int tt = 0; tt < 4; tt++) {
                 const int t = 4 * tg + tt;
@@ -169,9 +169,13 @@ __global__ void __launch_bounds__(LC_PTH) kr_lac_prep_kernel(KrLacArgs a) {
                     co.w = x[tt].w * cw[3].x + x[tt + 1].w * cw[3].y + x[tt + 2].w * cw[3].z + x[tt + 3].w * cw[3].w;
                     co.x = co.x * kr_sigmoid_poly5(co.x); co.y = co.y * kr_sigmoid_poly5(co.y); co.z = co.z * kr_sigmoid_poly5(co.z); co.w = co.w * kr_sigmoid_poly5(co.w);
                 }
+                if (arr == 2) { const float b = bs[t]; co.x *= b; co.y *= b; co.z *= b; co.w *= b; }
                 *reinterpret_cast<float4*>(T + t * LC_LD + c) = co;
             }
-        }
+    };
+    if (a.fused) {
+#pragma unroll 1
+        for (int arr = 0; arr < 2; arr++) conv(arr);
         if (wave == 0) {      // gates of the 64 tokens (decode.rs:3891-3901), then the running sum of g as below
             const int t = lane;
             float g = 0.0f, b = 0.0f;
@@ -186,7 +190,7 @@ __global__ void __launch_bounds__(LC_PTH) kr_lac_prep_kernel(KrLacArgs a) {
             }
 #pragma unroll
             for (int o = 1; o < 64; o <<= 1) { const float y = __shfl_up(g, o); if (lane >= o) g += y; }
-            Gs[t] = g; bs[t] = b; bg[t] = b * lc_exp(g);
+            Gs[t] = g; bs[t] = b;
             a.G[tile + t] = g;
         }
         __syncthreads();
@@ -208,12 +212,12 @@ __global__ void __launch_bounds__(LC_PTH) kr_lac_prep_kernel(KrLacArgs a) {
     // ---- tiles (rows past the chunk end are zero: b = 0, g = 0 make them inert)
     for (int u = tid; u < LC_T * 32; u += LC_PTH) {
         const int t = u >> 5, c4 = (u & 31) * 4;
-        float4 kk = make_float4(0, 0, 0, 0), qq = kk, vv = kk;
+        float4 kk = make_float4(0, 0, 0, 0), qq = kk;
         if (t < n) {
             const size_t o = (size_t)(c0 + t) * ld + (size_t)h * LC_D + c4;
-            kk = *reinterpret_cast<const float4*>(a.k + o); qq = *reinterpret_cast<const float4*>(a.q + o); vv = *reinterpret_cast<const float4*>(a.v + o);
+            kk = *reinterpret_cast<const float4*>(a.k + o); qq = *reinterpret_cast<const float4*>(a.q + o);
         }
-        *reinterpret_cast<float4*>(Kt + t * LC_LD + c4) = kk; *reinterpret_cast<float4*>(Qt + t * LC_LD + c4) = qq; *reinterpret_cast<float4*>(Vt + t * LC_LD + c4) = vv;
+        *reinterpret_cast<float4*>(Kt + t * LC_LD + c4) = kk; *reinterpret_cast<float4*>(Qt + t * LC_LD + c4) = qq;
     }
     if (wave == 0) {
         const int t = lane;
@@ -221,7 +225,7 @@ __global__ void __launch_bounds__(LC_PTH) kr_lac_prep_kernel(KrLacArgs a) {
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) { const float y = __shfl_up(g, o); if (lane >= o) g += y; }
         const float b = t < n ? a.beta[(size_t)(c0 + t) * a.nv + h] : 0.0f;
-        Gs[t] = g; bs[t] = b; bg[t] = b * lc_exp(g);
+        Gs[t] = g; bs[t] = b;
         a.G[tile + t] = g;
     }
     }
@@ -242,36 +246,53 @@ __global__ void __launch_bounds__(LC_PTH) kr_lac_prep_kernel(KrLacArgs a) {
 #pragma unroll
         for (int i = 0; i < 2; i++) { kh[32 * i] = lc_u4{hw[4 * i], hw[4 * i + 1], hw[4 * i + 2], hw[4 * i + 3]}; kl[32 * i] = lc_u4{lw[4 * i], lw[4 * i + 1], lw[4 * i + 2], lw[4 * i + 3]}; }
     }
-    // ---- K K^T -> L (strictly lower, decayed, row-scaled by b) and Q K^T -> B (lower incl. diagonal, decayed); the (0,1) blocks are zero
+    // ---- K K^T -> L (strictly lower, decayed, row-scaled by b), in LDS, and Q K^T -> B (lower incl. diagonal, decayed), in the accumulators of its waves; the (0,1) blocks are zero
+    v16f acc;
+    const int wb = wave % 3, rb = wb == 0 ? 0 : 1, cb = wb == 1 ? 1 : 0;       // one 32 x 32 block per wave: waves 0-2 L(0,0), L(1,1), L(1,0); waves 3-5 B(0,0), B(1,1), B(1,0)
+    float* blk = Lm + (rb + cb) * LC_LB;                                       // blocks (0,0), (1,0), (1,1)
     if (wave < 6) {
-        // one 32 x 32 block per wave: waves 0-2 L(0,0), L(1,1), L(1,0); waves 3-5 B(0,0), B(1,1), B(1,0)
         const bool isL = wave < 3;
-        const int wb = wave % 3, rb = wb == 0 ? 0 : 1, cb = wb == 1 ? 1 : 0;
-        v16f acc;
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[i] = 0.0f;
         lc_blk_s<true, true, LC_D>(acc, (isL ? Kt : Qt) + rb * 32 * LC_LD, LC_LD, Kt + cb * 32 * LC_LD, LC_LD, lane);
-        float* M = isL ? Lm : Bm;
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const int row = rb * 32 + lc_row(r, lane), col = cb * 32 + (lane & 31);
             const float d = lc_exp(Gs[row] - Gs[col]) * acc[r];
-            M[row * LC_LS + col] = isL ? (col < row ? bs[row] * d : 0.0f) : (col <= row ? d : 0.0f);
+            if (isL) blk[lc_row(r, lane) * LC_LS + (lane & 31)] = col < row ? bs[row] * d : 0.0f;
+            else acc[r] = col <= row ? d : 0.0f;
         }
-    } else {
-        for (int u = tid - 6 * 64; u < 32 * 32; u += 128) { const int row = u >> 5, col = 32 + (u & 31); Lm[row * LC_LS + col] = 0.0f; Bm[row * LC_LS + col] = 0.0f; }
+    }
+    float q0[16], q1[16];                      // waves 0-3: e^G Q of 32 columns, both row halves
+    const int wcol = (wave & 3) * 32 + (lane & 31);
+    if (wave < 4) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int r0 = lc_row(r, lane), r1 = 32 + r0;
+            q0[r] = lc_exp(Gs[r0]) * Qt[r0 * LC_LD + wcol]; q1[r] = lc_exp(Gs[r1]) * Qt[r1 * LC_LD + wcol];
+        }
     }
     __syncthreads();
     LC_STAMP(2);
+    // ---- diag(b) V over Q
+    if (a.fused) conv(2);
+    else
+        for (int u = tid; u < LC_T * 32; u += LC_PTH) {
+            const int t = u >> 5, c4 = (u & 31) * 4;
+            float4 vv = make_float4(0, 0, 0, 0);
+            if (t < n) vv = *reinterpret_cast<const float4*>(a.v + (size_t)(c0 + t) * ld + (size_t)h * LC_D + c4);
+            const float b = bs[t];
+            *reinterpret_cast<float4*>(Vt + t * LC_LD + c4) = float4{vv.x * b, vv.y * b, vv.z * b, vv.w * b};
+        }
     // ---- (I + L) X = R,  R = [diag(b e^G) K | diag(b) V]  (X = [W | Y], 64 x 256), by 32-row blocks on the matrix cores:
     //          X_top = T11 R_top,   X_bot = T22 (R_bot - L21 X_top),   T_ii = (I + L_ii)^-1
     // Wave 0 inverts the two unit-lower-triangular diagonal blocks: lane (i, c) carries column c of T_ii through a 32-step forward substitution in
     // registers (rows of L_ii are broadcast reads) -- 496 fma per lane instead of the 2016 of the 64-step column solve this replaces, whose chains
-    // were the longest phase of the kernel (8.5 of 28 us per workgroup) -- and parks T11 / T22 in the (0,1) blocks of Lm / Bm, which hold zeros nothing reads.
-    // Waves 1-3 scale the K and V rows in place meanwhile (K is not needed unscaled any more: its products and the K^T planes are done).
+    // were the longest phase of the kernel (8.5 of 28 us per workgroup) -- and leaves T11 / T22 in the places of L11 / L22, which it alone reads.
+    // The other waves scale the K rows in place meanwhile (K is not needed unscaled any more: its products and the K^T planes are done).
     if (wave == 0) {
-        const int blk = lane >> 5, c = lane & 31;
-        const float* Lb = Lm + blk * 32 * LC_LS + blk * 32;
+        const int half = lane >> 5, c = lane & 31;
+        float* Lb = Lm + 2 * half * LC_LB;
         float x[32];
 #pragma unroll
         for (int t = 0; t < 32; t++) x[t] = 0.0f;
@@ -287,14 +308,13 @@ __global__ void __launch_bounds__(LC_PTH) kr_lac_prep_kernel(KrLacArgs a) {
             }
             x[t] = t == c ? 1.0f : -((sa.x + sa.y) + (sb.x + sb.y));
         }
-        float* Td = (blk ? Bm : Lm) + 32 + c;
 #pragma unroll
-        for (int t = 0; t < 32; t++) Td[t * LC_LS] = x[t];
+        for (int t = 0; t < 32; t++) Lb[t * LC_LS + c] = x[t];
     } else {
-        for (int u = tid - 64; u < LC_T * 64; u += LC_PTH - 64) {      // 16-byte units: row u >> 6; 32 units of K, 32 of V
-            const int t = u >> 6, j = u & 63;
-            float* p = j < 32 ? Kt + t * LC_LD + 4 * j : Vt + t * LC_LD + 4 * (j - 32);
-            const float sc = j < 32 ? bg[t] : bs[t];
+        for (int u = tid - 64; u < LC_T * 32; u += LC_PTH - 64) {      // 16-byte units
+            const int t = u >> 5;
+            float* p = Kt + t * LC_LD + 4 * (u & 31);
+            const float sc = bs[t] * lc_exp(Gs[t]);
             f4 v = *reinterpret_cast<f4*>(p);
             v.x *= sc; v.y *= sc; v.z *= sc; v.w *= sc;
             *reinterpret_cast<f4*>(p) = v;
@@ -306,7 +326,7 @@ __global__ void __launch_bounds__(LC_PTH) kr_lac_prep_kernel(KrLacArgs a) {
     // products is LDS order inside one wave (a wave's LDS operations execute in issue order), not a workgroup barrier
     {
         float* X = wave < 4 ? Kt + wave * 32 : Vt + (wave - 4) * 32;
-        const float* T11 = Lm + 32; const float* T22 = Bm + 32; const float* L21 = Lm + 32 * LC_LS;
+        const float* T11 = Lm; const float* L21 = Lm + LC_LB; const float* T22 = Lm + 2 * LC_LB;
         const int n31 = lane & 31;
         v16f x0, x1;
 #pragma unroll
@@ -329,50 +349,63 @@ __global__ void __launch_bounds__(LC_PTH) kr_lac_prep_kernel(KrLacArgs a) {
     }
     __syncthreads();
     LC_STAMP(4);
+    if (wave >= 3 && wave < 6) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) blk[lc_row(r, lane) * LC_LS + (lane & 31)] = acc[r];
+    }
+    __syncthreads();
     // ---- Q' = diag(e^G) Q - B W (waves 0-3)  and  O_0 = B Y (waves 4-7): a wave takes 32 columns, both row halves (row half 0 only needs j < 32)
     {
         const bool isQ = wave < 4;
-        const int col = (wave & 3) * 32 + (lane & 31);
         const float* Rt = (isQ ? Kt : Vt) + (wave & 3) * 32;
         v16f p0, p1;
 #pragma unroll
         for (int i = 0; i < 16; i++) { p0[i] = 0.0f; p1[i] = 0.0f; }
-        lc_blk_s<true, false, 32>(p0, Bm, LC_LS, Rt, LC_LD, lane);
-        lc_blk_s<true, false, 64>(p1, Bm + 32 * LC_LS, LC_LS, Rt, LC_LD, lane);
+        lc_blk_s<true, false, 32>(p0, Lm, LC_LS, Rt, LC_LD, lane);
+        lc_blk_s<true, false, 32>(p1, Lm + LC_LB, LC_LS, Rt, LC_LD, lane);
+        lc_blk_s<true, false, 32>(p1, Lm + 2 * LC_LB, LC_LS, Rt + 32 * LC_LD, LC_LD, lane);
         LC_STAMP(5);
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const int r0 = lc_row(r, lane), r1 = 32 + r0;
-            if (isQ) {
-                Qt[r0 * LC_LD + col] = lc_exp(Gs[r0]) * Qt[r0 * LC_LD + col] - p0[r];      // Q' over Q in LDS: element (row, col) is touched by this lane only
-                Qt[r1 * LC_LD + col] = lc_exp(Gs[r1]) * Qt[r1 * LC_LD + col] - p1[r];
-            } else {
-                if (r0 < n) a.out[(size_t)(c0 + r0) * ld + (size_t)h * LC_D + col] = p0[r];
-                if (r1 < n) a.out[(size_t)(c0 + r1) * ld + (size_t)h * LC_D + col] = p1[r];
+            if (isQ) { q0[r] -= p0[r]; q1[r] -= p1[r]; }
+            else {
+                if (r0 < n) a.out[(size_t)(c0 + r0) * ld + (size_t)h * LC_D + wcol] = p0[r];
+                if (r1 < n) a.out[(size_t)(c0 + r1) * ld + (size_t)h * LC_D + wcol] = p1[r];
             }
         }
         LC_STAMP(6);
     }
-    __syncthreads();
-    // ---- W (K tile), Q' (Q tile) -> their bf16 planes, Y (V tile) -> f32, all with 16-byte stores: planes in the scan's order (chunk u of a plane: lc_frag), Y in rows
+    // ---- W (K tile), then Q' (over W) -> their bf16 planes, Y (V tile) -> f32, all with 16-byte stores: planes in the scan's order (chunk u of a plane: lc_frag), Y in rows
+    auto planes = [&](uint16_t* ph, uint16_t* pl) {
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int u = tid + LC_PTH * i, t = (u >> 9) * 32 + (u & 31), c8 = ((u >> 5) & 15) * 8, yt = u >> 4, yc = (u & 15) * 8;
-        const size_t o = tile * LC_D + (size_t)u * 8, oy = (tile + yt) * LC_D + yc;
-        auto planes = [&](const float* src, uint16_t* ph, uint16_t* pl) {
-            const f4 v0 = *reinterpret_cast<const f4*>(src + t * LC_LD + c8), v1 = *reinterpret_cast<const f4*>(src + t * LC_LD + c8 + 4);
+        for (int i = 0; i < 2; i++) {
+            const int u = tid + LC_PTH * i, t = (u >> 9) * 32 + (u & 31), c8 = ((u >> 5) & 15) * 8;
+            const size_t o = tile * LC_D + (size_t)u * 8;
+            const f4 v0 = *reinterpret_cast<const f4*>(Kt + t * LC_LD + c8), v1 = *reinterpret_cast<const f4*>(Kt + t * LC_LD + c8 + 4);
             const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
             uint16_t hh[8], ll[8];
 #pragma unroll
             for (int j = 0; j < 8; j++) lc_split(v[j], hh[j], ll[j]);
             *reinterpret_cast<lc_u4*>(ph + o) = lc_u4{(uint32_t)hh[0] | ((uint32_t)hh[1] << 16), (uint32_t)hh[2] | ((uint32_t)hh[3] << 16), (uint32_t)hh[4] | ((uint32_t)hh[5] << 16), (uint32_t)hh[6] | ((uint32_t)hh[7] << 16)};
             *reinterpret_cast<lc_u4*>(pl + o) = lc_u4{(uint32_t)ll[0] | ((uint32_t)ll[1] << 16), (uint32_t)ll[2] | ((uint32_t)ll[3] << 16), (uint32_t)ll[4] | ((uint32_t)ll[5] << 16), (uint32_t)ll[6] | ((uint32_t)ll[7] << 16)};
-        };
-        planes(Kt, a.Wh, a.Wl);
-        planes(Qt, a.Qh, a.Ql);
+        }
+    };
+    planes(a.Wh, a.Wl);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int u = tid + LC_PTH * i, yt = u >> 4, yc = (u & 15) * 8;
+        const size_t oy = (tile + yt) * LC_D + yc;
         *reinterpret_cast<f4*>(a.Y + oy) = *reinterpret_cast<const f4*>(Vt + yt * LC_LD + yc);
         *reinterpret_cast<f4*>(a.Y + oy + 4) = *reinterpret_cast<const f4*>(Vt + yt * LC_LD + yc + 4);
     }
+    __syncthreads();
+    if (wave < 4) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) { const int r0 = lc_row(r, lane); Kt[r0 * LC_LD + wcol] = q0[r]; Kt[(32 + r0) * LC_LD + wcol] = q1[r]; }
+    }
+    __syncthreads();
+    planes(a.Qh, a.Ql);
 }
 
 // acc(32x32) += A(32 x K) . B(K x 32), both operands as bf16 (hi, lo) planes.  A: this wave's fragments, in registers (a[0] hi, a[1] lo); each is requested again, for the

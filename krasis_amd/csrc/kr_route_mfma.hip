@@ -319,9 +319,10 @@ __global__ void __launch_bounds__(64 * (KS == 1 ? 2 : KS), 2) kr_route_logits_fa
 // per step); a wave's fragments are 16-byte LDS reads (rows 80 bytes apart: conflict-free).  Per logit: MFMA(hi) then MFMA(lo) per 16 k, k ascending -- the order
 // of the KS = 1 kernel.
 #define RLT_LD 80            // bytes per LDS row: 32 bf16 + 16 pad
-template <int TM>            // 64 or 128 tokens per workgroup; waves 2 x 2, each TM / 2 x 64
+// waves 2 x 2, each 32 x 64 (tiles of 128 tokens: a workgroup per compute unit instead of two, 8192 tokens 68 us against 60)
 __global__ void __launch_bounds__(256) kr_route_logits_tiled_kernel(const uint16_t* __restrict__ gate_row, const float* __restrict__ x, const float* __restrict__ bias,
                                                                    float* __restrict__ logits, int T, int E, int H) {
+    constexpr int TM = 64;                       // tokens of a workgroup
     constexpr int NRB = TM / 64;                 // 32-row blocks per wave
     constexpr int XPT = TM / 32;                 // float4 of x per thread and step
     __shared__ __attribute__((aligned(16))) char lds[2][(2 * TM + 128) * RLT_LD];
@@ -335,18 +336,22 @@ __global__ void __launch_bounds__(256) kr_route_logits_tiled_kernel(const uint16
     const uint16_t* gp[2];
 #pragma unroll
     for (int j = 0; j < 2; j++) gp[j] = gate_row + (size_t)min(e0 + (tid >> 2) + 64 * j, E - 1) * H + (tid & 3) * 8;
-    rm_f4 px[XPT]; rm_u4 pg[2];
-    auto fetch = [&](int st) {
+    // A step is 0.3 us of work and a request takes a microsecond, so PD steps are in flight in registers (8192 tokens in tiles of 128: one step ahead 77 us, four 68)
+    constexpr int PD = 4;
+    rm_f4 px[PD][XPT]; rm_u4 pg[PD][2];
+    const int nst = H / 32;
+    auto fetch = [&](int st, int q) {            // a step past the last re-reads the last
+        st = min(st, nst - 1);
 #pragma unroll
-        for (int j = 0; j < XPT; j++) px[j] = *reinterpret_cast<const rm_f4*>(xp[j] + 32 * st);
+        for (int j = 0; j < XPT; j++) px[q][j] = *reinterpret_cast<const rm_f4*>(xp[j] + 32 * st);
 #pragma unroll
-        for (int j = 0; j < 2; j++) pg[j] = *reinterpret_cast<const rm_u4*>(gp[j] + 32 * st);
+        for (int j = 0; j < 2; j++) pg[q][j] = *reinterpret_cast<const rm_u4*>(gp[j] + 32 * st);
     };
-    auto commit = [&](int buf) {
+    auto commit = [&](int buf, int q) {
         char* Xh = lds[buf]; char* Xl = Xh + TM * RLT_LD; char* G = Xl + TM * RLT_LD;
 #pragma unroll
         for (int j = 0; j < XPT; j++) {
-            const float v[4] = {px[j].x, px[j].y, px[j].z, px[j].w};
+            const float v[4] = {px[q][j].x, px[q][j].y, px[q][j].z, px[q][j].w};
             uint16_t hi[4], lo[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) { const __bf16 hb = (__bf16)v[i]; const __bf16 lb = (__bf16)(v[i] - (float)hb); hi[i] = __builtin_bit_cast(uint16_t, hb); lo[i] = __builtin_bit_cast(uint16_t, lb); }
@@ -355,7 +360,7 @@ __global__ void __launch_bounds__(256) kr_route_logits_tiled_kernel(const uint16
             *reinterpret_cast<uint2*>(Xl + off) = uint2{(uint32_t)lo[0] | ((uint32_t)lo[1] << 16), (uint32_t)lo[2] | ((uint32_t)lo[3] << 16)};
         }
 #pragma unroll
-        for (int j = 0; j < 2; j++) *reinterpret_cast<rm_u4*>(G + ((tid >> 2) + 64 * j) * RLT_LD + (tid & 3) * 16) = pg[j];
+        for (int j = 0; j < 2; j++) *reinterpret_cast<rm_u4*>(G + ((tid >> 2) + 64 * j) * RLT_LD + (tid & 3) * 16) = pg[q][j];
     };
     rm_v16f acc[NRB][2];
 #pragma unroll
@@ -364,12 +369,16 @@ __global__ void __launch_bounds__(256) kr_route_logits_tiled_kernel(const uint16
         for (int c = 0; c < 2; c++)
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[a_][c][i] = 0.0f;
-    const int nst = H / 32;
-    fetch(0); commit(0);
+#pragma unroll
+    for (int q = 0; q < PD; q++) fetch(q, q);
+    commit(0, 0);
+    fetch(PD, 0);
     __syncthreads();
-    for (int st = 0; st < nst; st++) {
-        const int buf = st & 1;
-        if (st + 1 < nst) fetch(st + 1);
+    for (int st0 = 0; st0 < nst; st0 += PD)
+#pragma unroll
+    for (int q = 0; q < PD; q++) {
+        const int st = st0 + q, buf = q & 1;
+        if (st >= nst) break;
         const char* Xh = lds[buf]; const char* Xl = Xh + TM * RLT_LD; const char* G = Xl + TM * RLT_LD;
 #pragma unroll
         for (int ks = 0; ks < 2; ks++) {
@@ -392,7 +401,10 @@ __global__ void __launch_bounds__(256) kr_route_logits_tiled_kernel(const uint16
 #pragma unroll
                 for (int c = 0; c < 2; c++) acc[a_][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[a_], b[c], acc[a_][c], 0, 0, 0);
         }
-        if (st + 1 < nst) commit(buf ^ 1);      // the other buffer: its last readers passed the barrier of the previous step
+        if (st + 1 < nst) {                     // the other buffer: its last readers passed the barrier of the previous step
+            commit(buf ^ 1, (q + 1) % PD);
+            fetch(st + 1 + PD, (q + 1) % PD);
+        }
         __syncthreads();
     }
 #pragma unroll
@@ -411,18 +423,13 @@ __global__ void __launch_bounds__(256) kr_route_logits_tiled_kernel(const uint16
 // non-zero = not covered (f32 gate, H not a multiple of 32): the caller keeps the exact kernel
 int kr_launch_route_logits_fast(const void* gate_row, int gate_bf16, const float* x, const float* bias, float* logits, int T, int E, int H, hipStream_t st) {
     if (!gate_bf16 || H % 32 || T < 1 || E < 1) return 1;
-    {   // workgroup-tiled form where its tiles still give (nearly) every CU a workgroup: 128-token tiles from ~7 k tokens x 512 experts on (8192 tokens: 74 us against 134),
-        // 64-token tiles for shorter chunks only when the k-split form below does not apply (2752 tokens: both 58 us)
-        const int n128 = (E + 127) / 128;
-        const bool ksplit_ok = H % 128 == 0 && H >= 512;
-        if ((long)((T + 127) / 128) * n128 >= 224) {
-            hipLaunchKernelGGL(kr_route_logits_tiled_kernel<128>, dim3(n128, (T + 127) / 128), dim3(256), 0, st, reinterpret_cast<const uint16_t*>(gate_row), x, bias, logits, T, E, H);
-            return 0;
-        }
-        if (T >= 256 && !ksplit_ok) {
-            hipLaunchKernelGGL(kr_route_logits_tiled_kernel<64>, dim3(n128, (T + 63) / 64), dim3(256), 0, st, reinterpret_cast<const uint16_t*>(gate_row), x, bias, logits, T, E, H);
-            return 0;
-        }
+    // workgroup-tiled form where its tiles give at least every other CU a workgroup (512 experts, 2752 tokens: 42 us against 55 of the k-split form below, 4096: 44 against 73, 8192:
+    // 60), and from 256 tokens on where that form does not apply
+    const int n128 = (E + 127) / 128;
+    const long tiles = (long)((T + 63) / 64) * n128;
+    if (tiles >= 128 || (T >= 256 && !(H % 128 == 0 && H >= 512))) {
+        hipLaunchKernelGGL(kr_route_logits_tiled_kernel, dim3(n128, (T + 63) / 64), dim3(256), 0, st, reinterpret_cast<const uint16_t*>(gate_row), x, bias, logits, T, E, H);
+        return 0;
     }
     if (H % 128 == 0 && H >= 512) {      // four k quarters per output tile: 4 x the waves (2752 tokens: 57.7 us against 70.1 stand-alone, profiles/r06_route_fast_kernel_stats.txt)
         const dim3 grid((E + 63) / 64, (T + 31) / 32);

@@ -268,15 +268,11 @@ static int prefill_impl(kr_decode_store* s, const int32_t* tokens, int n_tokens,
     hipStream_t st = kr_pick_stream(e, stream);
     const int H = s->hidden;
     if (H % 128) return kr_fail(KR_ERR_VALUE, "kr_decode_prefill needs hidden %% 128 == 0");
-    // defaults: 1024 tokens x 3 chunks in flight for the exact pass (its serial per-token kernels need the overlap); with both tolerance bits set the
-    // kernels are chunk-parallel and fatter chunks feed the expert GEMMs better (rows per expert grow with the chunk): 4096 x 2 measured best at
-    // 8192 tokens (tools/probes/prefill_sweep.py: 1024 x 3 171 ms, 2048 x 2 168, 4096 x 2 164, 8192 x 1 193)
-    // (second sweep: three chunks in flight beat two once the prompt has three chunks to give -- 8192 tokens: 2752 x 3 148.6 ms vs 4096 x 2 151.4;
-    // 20 434 tokens: 4096 x 3 407 ms vs 4096 x 2 423 -- so: a third of the prompt per chunk, between 1024 and 4096 tokens, three in flight; 3000 tokens: 1024 x 3 56.8 ms vs 2048 + 952 60.9)
-    const int third = ((n_tokens + 2) / 3 + 63) / 64 * 64;
-    const int tol_chunk = std::min(4096, std::max(KR_PFM_CHUNK, third));
-    // (round 6: the same rule with KR_ATTN_FAST alone -- its attention / delta-rule kernels are chunk-parallel too and the exact expert GEMM likes the fatter chunks:
-    // 8192 tokens 173.8 -> 162.0 ms, 20 434: 448.5 -> 428.1, 49 863: 1221.6 -> 1185.4; the exact pass keeps 1024 x 3: its per-token recurrences need the overlap)
+    // defaults: 1024 tokens x 3 chunks in flight for the exact pass (its serial per-token kernels need the overlap).  The kernels of the tolerance passes (KR_ATTN_FAST, with or
+    // without KR_GEMM_FAST) are chunk-parallel, and what a chunk costs per token falls as it grows (an expert's weights are converted once per 64 of its rows, and every launch has
+    // a last round), so the prompt is split evenly into as few chunks of at most 4096 tokens as hold it.  Against a third of the prompt per chunk, at least 1024, ms (hybrid of four
+    // layers, 512 experts): 1500 tokens 4.21 -> 3.40, 3000 6.56 -> 5.38, 4000 7.78 -> 6.71, 5000 8.87 -> 8.00, 8192 12.69 -> 11.97; 12000 in three either way.
+    const int n4k = (n_tokens + 4095) / 4096, tol_chunk = std::min(4096, ((n_tokens + n4k - 1) / n4k + 63) / 64 * 64);
     const int depth = s->pf_depth >= 1 && s->pf_depth <= KR_PF_MAX_DEPTH ? s->pf_depth : KR_PFM_DEPTH;   // chunks in flight (streams / arenas)
     // exact pass: chunks of ~1024 tokens, their COUNT a multiple of the depth when the prompt has that many -- the last round of chunks then fills every stream
     // (8192 tokens: 8 x 1024 = 3 + 3 + 2 chunks 382.9 ms, 6 x 1366 355.8; 20 434: 20 x 1024 1207.9, 18 x 1136 1180.1; 49 863: unchanged, attention-bound)

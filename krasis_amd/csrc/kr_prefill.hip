@@ -83,22 +83,28 @@ __global__ void __launch_bounds__(256) kr_pf_scatter_wg_kernel(const int32_t* __
 __global__ void __launch_bounds__(1024) kr_pf_scan_kernel(const int* __restrict__ counts, int E, int* __restrict__ offsets, int* __restrict__ cursor,
                                                          int* __restrict__ tile_expert, int* __restrict__ tile_row0, int* __restrict__ tile_rows,
                                                          int* __restrict__ n_tiles_out, int bm) {
-    __shared__ int s_off[1025], s_tile[1025];
-    const int t = threadIdx.x;
-    if (t == 0) {
-        int o = 0, tl = 0;
-        for (int e = 0; e < E; e++) { s_off[e] = o; s_tile[e] = tl; o += counts[e]; tl += (counts[e] + bm - 1) / bm; }
-        s_off[E] = o; s_tile[E] = tl; n_tiles_out[0] = tl; n_tiles_out[1] = o;   // [1]: rows in total (valid pairs)
-    }
-    __syncthreads();
-    for (int e = t; e < E; e += 1024) {
-        offsets[e] = s_off[e]; cursor[e] = 0;
-        const int c = counts[e];
-        for (int i = 0; i * bm < c; i++) {
-            const int ti = s_tile[e] + i;
-            tile_expert[ti] = e; tile_row0[ti] = s_off[e] + i * bm; tile_rows[ti] = (c - i * bm) < bm ? (c - i * bm) : bm;
+    // an expert per thread, rows and tiles before it by scans of the wave and then of the sixteen waves' sums (one thread walking 512 counts: 30 us a launch)
+    __shared__ int w_off[16], w_tile[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int o0 = 0, tl0 = 0;                             // before this band of 1024 experts
+    for (int e0 = 0; e0 < E; e0 += 1024) {
+        const int e = e0 + threadIdx.x, c = e < E ? counts[e] : 0, nt = (c + bm - 1) / bm;
+        int o = c, tl = nt;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) { const int a = __shfl_up(o, d), b = __shfl_up(tl, d); if (lane >= d) { o += a; tl += b; } }
+        if (lane == 63) { w_off[wave] = o; w_tile[wave] = tl; }
+        __syncthreads();
+        o += o0 - c; tl += tl0 - nt;
+        for (int w = 0; w < 16; w++) {
+            if (w < wave) { o += w_off[w]; tl += w_tile[w]; }
+            o0 += w_off[w]; tl0 += w_tile[w];
         }
+        __syncthreads();
+        if (e >= E) continue;
+        offsets[e] = o; cursor[e] = 0;
+        for (int i = 0; i < nt; i++) { tile_expert[tl + i] = e; tile_row0[tl + i] = o + i * bm; tile_rows[tl + i] = min(c - i * bm, bm); }
     }
+    if (threadIdx.x == 0) { n_tiles_out[0] = tl0; n_tiles_out[1] = o0; }   // [1]: rows in total (valid pairs)
 }
 
 // One workgroup sorts a chunk's (token, slot) pairs by expert: count (LDS atomics) -> exclusive scans of rows and 64-row tiles -> scatter, in ONE

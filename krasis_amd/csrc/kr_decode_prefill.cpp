@@ -90,7 +90,9 @@ static int run_layer(kr_decode_store* s, Chunk& cx, size_t li) {
     na.bias_one = s->norm_bias_one; na.eps = s->eps;
     if (s->gemm_fast) { na.xh = nullptr; na.xl = nullptr; na.xs = nullptr; }      // tolerance GEMMs take f16 rows of the normalised value instead of the digits
     if (s->gemm_fast && s->opt_norm_rows) { na.xf = B.xf; na.xfm = B.xfm; }      // ... and the norm launch writes that row image itself (round 6: one launch per norm less)
+    if (na.xf && (L.attn == ATTN_LA || L.attn == ATTN_GQA)) na.out = nullptr;      // the projections take the row image, and nothing else reads the f32 rows
     kr_launch_pfm_norm(na, Cc, st);
+    na.out = B.normed;
     if (s->gemm_fast && !s->opt_norm_rows) kr_launch_pfh_rows_f32(B.normed, Cc, H, H, B.xf, B.xfm, st);
     cx.first = false; cx.add_is_emb = false;
     if (L.attn == ATTN_LA) {
@@ -102,10 +104,12 @@ static int run_layer(kr_decode_store* s, Chunk& cx, size_t li) {
         a.a_log = (const float*)L.a_log.p; a.dt_bias = (const float*)L.dt_bias.p; a.scale = L.la_scale; a.q = B.q; a.k = B.k; a.v = B.v; a.z = B.z;
         a.gexp = B.gexp; a.beta = B.beta; a.nk = L.nk; a.nv = L.nv; a.dk = L.dk; a.dv = L.dv; a.hr = L.nv / L.nk;
         a.lac = B.lac; a.fast = s->attn_fast; a.conv_fused = s->opt_la_conv_fused;
+        if (oc != L.nv * L.dv) return kr_fail(KR_ERR_VALUE, "out_proj cols %d != nv*dv", oc);
+        const bool rows = s->gemm_fast && s->opt_norm_rows && kr_pfm_la_rows_ok(L.nv, L.dv);
+        if (rows) { a.xf = B.yf; a.xfm = B.yfm; }
         if (kr_launch_pfm_la(a, (float*)L.recur_state.p, B.recur, (const float*)L.la_norm_w.p, B.attn, Cc, s->eps, st, &cx.sy))
             return kr_fail(KR_ERR_VALUE, "unsupported linear-attention geometry");
-        if (oc != L.nv * L.dv) return kr_fail(KR_ERR_VALUE, "out_proj cols %d != nv*dv", oc);
-        pf_rows(s, B.attn, Cc, oc, oc, B, true, st);
+        if (!rows) pf_rows(s, B.attn, Cc, oc, oc, B, true, st);
         if (int rc = pf_gemm(s, L.out_wid, Y(B), Cc, B.hid, H, st)) return rc;
     } else if (L.attn == ATTN_GQA) {
         if (!L.kv_k.p) return kr_fail(KR_ERR_STATE, "set_decode_state was not called (no KV cache for layer %zu)", li);

@@ -28,6 +28,7 @@ struct KrPfmLaArgs {
     float *q, *k, *v, *z, *gexp, *beta;   // [C, nv*dk] x2, [C, nv*dv] x2, [C, nv] x2
     int nk, nv, dk, dv, hr;
     float* lac; int fast;                 // FAST mode: scratch of the 64-token closed form (kr_la_chunk.hip), kr_pfm_la_chunk_scratch_floats(C, nv) floats
+    uint16_t* xf; float* xfm;             // set: the gated norm leaves the f16 row image and its multipliers instead of f32 rows (kr_pfm_la_rows_ok)
     int conv_fused;                       // FAST mode (round 6): the conv / norms / gates inside the prep launch, z read by the gated norm where the in-projection left it (no conv launch)
 };
 struct KrPfmGqaArgs {
@@ -38,6 +39,7 @@ struct KrPfmGqaArgs {
     float *q_out, *gate, *attn_out;   // [C, nh*hd]
     int gated, nh, nkv, hd, pos0; float eps, sm_scale;
 };
+bool kr_pfm_la_rows_ok(int nv, int dv);
 void kr_launch_pfm_norm(const KrPfmNormArgs& a, int C, hipStream_t st);
 void kr_launch_pfm_nll(const float* logits, size_t ld, const int* labels, float* nll, int rows, int V, hipStream_t st);
 void kr_launch_pfm_quant_f32(const float* x, int rows, int ld, int K, int8_t* xh, int8_t* xl, float* xs, hipStream_t st);

@@ -52,7 +52,7 @@ __device__ __forceinline__ void kr_pfm_quant_chunk(const float (&v)[8], int8_t* 
 
 // ---- fused add + RMSNorm, one workgroup per token (decode.rs:1199) ------------------------------------------------------
 // value added: mode 0 = add_in[t] (attention / MLP output), mode 1 = embedding row of tokens[t]; first: residual = value.
-// outputs: residual (in place), normalised hidden f32, optional INT16 digits of the f32 value, optional bf16 copy (routed experts
+// outputs: residual (in place), normalised hidden f32 (null: nobody reads it), optional INT16 digits of the f32 value, optional bf16 copy (routed experts
 // quantise bf16(hidden), decode.rs:3307-3309).
 __global__ void __launch_bounds__(256) kr_pfm_norm_kernel(const KrPfmNormArgs a) {
     extern __shared__ __attribute__((aligned(16))) float r[];   // [H + 4]
@@ -75,8 +75,10 @@ __global__ void __launch_bounds__(256) kr_pfm_norm_kernel(const KrPfmNormArgs a)
         float v[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) { const int i = c * 8 + u; v[u] = (r[i] * rms) * (a.bias_one ? (a.w[i] + 1.0f) : a.w[i]); mx = fmaxf(mx, fabsf(v[u])); }
-        *reinterpret_cast<float4*>(out + c * 8) = make_float4(v[0], v[1], v[2], v[3]);
-        *reinterpret_cast<float4*>(out + c * 8 + 4) = make_float4(v[4], v[5], v[6], v[7]);
+        if (a.out) {
+            *reinterpret_cast<float4*>(out + c * 8) = make_float4(v[0], v[1], v[2], v[3]);
+            *reinterpret_cast<float4*>(out + c * 8 + 4) = make_float4(v[4], v[5], v[6], v[7]);
+        }
         if (a.xh) kr_pfm_quant_chunk(v, a.xh + (size_t)t * H + c * 8, a.xl + (size_t)t * H + c * 8, a.xs + (size_t)t * (H / 128) + (c >> 4), (c & 15) == 0);
         if (a.out_bf16) {
             u32x4 p;
@@ -374,6 +376,58 @@ __global__ void __launch_bounds__(256) kr_pfm_gated_norm_kernel(const float* __r
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup"); __builtin_amdgcn_wave_barrier();      // the slice is rewritten by the wave's next row
     }
+}
+
+// The same for the tolerance GEMMs, whose input is the f16 row image: a workgroup takes a token's whole row, 256 chains of eight lanes over 32 heads at once, and leaves the image itself;
+// the f32 row is not written and read again, and the row pass's launch is gone.  Memory bound (the recurrence's rows and z in, half as much out): 32 heads of 128, 4096 tokens
+// 52 + 20 -> 29 us.  NCH: 8-value pieces of a thread; heads 8 floats apart in LDS, or the chains of a wave's heads would share banks.
+template <int NCH>
+__global__ void __launch_bounds__(256) kr_pfm_gated_norm_rows_kernel(const float* __restrict__ recur, const float* __restrict__ z, size_t z_ld, int z_hr, int z_kstride, const float* __restrict__ w,
+                                                                    uint16_t* __restrict__ out, float* __restrict__ mul, int nv, int dv, float eps) {
+    extern __shared__ __attribute__((aligned(16))) float r[];       // [nv][dv + 8], then [nv]
+    __shared__ uint32_t s_max;
+    const int t = blockIdx.x, tid = threadIdx.x, per = dv / 8, K = nv * dv, ldh = dv + 8;
+    float* rms = r + (size_t)nv * ldh;
+    if (tid == 0) s_max = 0;
+    float v[NCH][8], g[NCH][8];
+#pragma unroll
+    for (int q = 0; q < NCH; q++) {
+        const int c = min(tid + 256 * q, K / 8 - 1), h = c / per, j = (c - h * per) * 8;      // a piece past the row repeats the last one
+        const float* pv = recur + (size_t)t * K + (size_t)c * 8;
+        const float* pz = z + (size_t)t * z_ld + (size_t)(h / z_hr) * z_kstride + (size_t)(h % z_hr) * dv + j;
+        const float4 v0 = *reinterpret_cast<const float4*>(pv), v1 = *reinterpret_cast<const float4*>(pv + 4), z0 = *reinterpret_cast<const float4*>(pz), z1 = *reinterpret_cast<const float4*>(pz + 4);
+        v[q][0] = v0.x; v[q][1] = v0.y; v[q][2] = v0.z; v[q][3] = v0.w; v[q][4] = v1.x; v[q][5] = v1.y; v[q][6] = v1.z; v[q][7] = v1.w;
+        g[q][0] = z0.x; g[q][1] = z0.y; g[q][2] = z0.z; g[q][3] = z0.w; g[q][4] = z1.x; g[q][5] = z1.y; g[q][6] = z1.z; g[q][7] = z1.w;
+        *reinterpret_cast<float4*>(r + h * ldh + j) = v0; *reinterpret_cast<float4*>(r + h * ldh + j + 4) = v1;
+    }
+    __syncthreads();
+    for (int u = tid; u < nv * 8; u += 256) {
+        const float ss = kr_pfm_sumsq8(r + (u >> 3) * ldh, dv, u & 7);
+        if ((u & 7) == 0) rms[u >> 3] = 1.0f / sqrtf(ss / (float)dv + eps);
+    }
+    __syncthreads();
+    float mx = 0.0f;
+#pragma unroll
+    for (int q = 0; q < NCH; q++) {
+        const int c = min(tid + 256 * q, K / 8 - 1);
+        const float s = rms[c / per];
+        const float4 w0 = *reinterpret_cast<const float4*>(w + (size_t)c * 8), w1 = *reinterpret_cast<const float4*>(w + (size_t)c * 8 + 4);
+        const float wv[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+        for (int u = 0; u < 8; u++) { v[q][u] = (g[q][u] * kr_sigmoid_poly5(g[q][u])) * ((v[q][u] * s) * wv[u]); mx = fmaxf(mx, fabsf(v[q][u])); }
+    }
+    mx = pfh_block_max(mx, &s_max);
+    float scl, inv; pfh_row_scale(mx, scl, inv);
+#pragma unroll
+    for (int q = 0; q < NCH; q++) {
+        const int c = tid + 256 * q;
+        if (c >= K / 8) break;
+        u32x4 o;
+        o.x = pfh_pack_h2(v[q][0] * scl, v[q][4] * scl); o.y = pfh_pack_h2(v[q][1] * scl, v[q][5] * scl);      // image order (0,4,1,5,2,6,3,7)
+        o.z = pfh_pack_h2(v[q][2] * scl, v[q][6] * scl); o.w = pfh_pack_h2(v[q][3] * scl, v[q][7] * scl);
+        *reinterpret_cast<u32x4*>(out + (size_t)t * K + (size_t)c * 8) = o;
+    }
+    if (tid == 0) mul[t] = inv * 0.0625f;
 }
 
 // ---- GQA: gated split, per-head RMS norm, RoPE, FP16 KV append for every token (decode.rs:2873-2966); grid (nh + nkv, C) ---------
@@ -853,6 +907,15 @@ void kr_launch_pfm_quant_f32(const float* x, int rows, int ld, int K, int8_t* xh
     const int thr = K / 8 < 1024 ? ((K / 8 + 15) / 16) * 16 : 1024;
     hipLaunchKernelGGL(kr_pfm_quant_f32_kernel, dim3(rows), dim3(thr), 0, st, x, ld, K, xh, xl, xs);
 }
+// gated norm of C tokens: the f16 row image where the caller asks for it (kr_pfm_la_rows_ok), else f32 rows
+bool kr_pfm_la_rows_ok(int nv, int dv) { return dv % 8 == 0 && nv * dv <= 8192 && (size_t)nv * (dv + 9) * 4 <= 48 * 1024; }
+static void pfm_gated_norm(const KrPfmLaArgs& a, const float* recur, const float* z, size_t z_ld, int z_hr, int z_kstride, const float* w, float* out, int C, float eps, hipStream_t st) {
+    if (a.xf) {
+        const size_t lds = (size_t)a.nv * (a.dv + 9) * 4;
+        if (a.nv * a.dv <= 4096) hipLaunchKernelGGL(kr_pfm_gated_norm_rows_kernel<2>, dim3(C), dim3(256), lds, st, recur, z, z_ld, z_hr, z_kstride, w, a.xf, a.xfm, a.nv, a.dv, eps);
+        else hipLaunchKernelGGL(kr_pfm_gated_norm_rows_kernel<4>, dim3(C), dim3(256), lds, st, recur, z, z_ld, z_hr, z_kstride, w, a.xf, a.xfm, a.nv, a.dv, eps);
+    } else hipLaunchKernelGGL(kr_pfm_gated_norm_kernel, dim3(a.nv, (C + PFG_TT - 1) / PFG_TT), dim3(256), 0, st, recur, z, z_ld, z_hr, z_kstride, w, out, a.nv, a.dv, C, eps);
+}
 static void pfm_la_conv_state(const KrPfmLaArgs& a, int C, hipStream_t st, const KrPfSync* sy) {      // advance the carried conv slots, then publish them to the next chunk
     const int conv_dim = 2 * a.nk * a.dk + a.nv * a.dv;
     hipLaunchKernelGGL(kr_pfm_la_conv_state_kernel, dim3((conv_dim + 255) / 256), dim3(256), 0, st, a, C);
@@ -870,8 +933,7 @@ int kr_launch_pfm_la(const KrPfmLaArgs& a, float* recur_state, float* recur_out,
         kr_launch_pfm_la_chunked(a, recur_state, recur_out, a.lac, C, st, sy, 1, pfm_la_conv_state) == 0) {
         kr_pf_rec(st, sy->rec_b);
         const int gd = 2 * a.dk + 2 * a.dv * a.hr;
-        hipLaunchKernelGGL(kr_pfm_gated_norm_kernel, dim3(a.nv, (C + PFG_TT - 1) / PFG_TT), dim3(256), 0, st, recur_out, a.qkvz + 2 * a.dk + a.hr * a.dv, (size_t)a.ld_qkvz, a.hr, gd, norm_w,
-                           gated_out, a.nv, a.dv, C, eps);
+        pfm_gated_norm(a, recur_out, a.qkvz + 2 * a.dk + a.hr * a.dv, (size_t)a.ld_qkvz, a.hr, gd, norm_w, gated_out, C, eps, st);
         return 0;
     }
     hipLaunchKernelGGL(kr_pfm_la_conv_kernel, dim3(a.nk, (C + PFC_WT - 1) / PFC_WT), dim3(256), (size_t)(2 * PFC_WT * a.dk + 2 * PFC_WT) * 4, st, a, C);
@@ -886,7 +948,7 @@ int kr_launch_pfm_la(const KrPfmLaArgs& a, float* recur_state, float* recur_out,
     }
     kr_pf_rec(st, sy->rec_b);
     // z: the stand-alone copy [C][nv * dv] the conv launch makes (z_hr = nv: one block)
-    hipLaunchKernelGGL(kr_pfm_gated_norm_kernel, dim3(a.nv, (C + PFG_TT - 1) / PFG_TT), dim3(256), 0, st, recur_out, (const float*)a.z, (size_t)a.nv * a.dv, a.nv, 0, norm_w, gated_out, a.nv, a.dv, C, eps);
+    pfm_gated_norm(a, recur_out, a.z, (size_t)a.nv * a.dv, a.nv, 0, norm_w, gated_out, C, eps, st);
     return 0;
 }
 // the recurrence alone (stand-alone operator linear_attention_recurrent, decode.rs:609): gexp = e^g per (token, head); non-zero = unsupported geometry

@@ -1026,7 +1026,7 @@ static int moe_prefill_fast(kr_engine* e, Layer& L, const void* x_bf16, const in
     const int CHmax = pairs / topk > 64 ? pairs / topk : 64;
     const int CH = M < CHmax ? M : CHmax;
     const size_t np = (size_t)CH * topk;
-    const int max_tiles = (int)(np / 64) + E + 1;
+    const int max_tiles = (int)(np / 16) + E + 1;      // (tiles of 16 rows are the smallest, kr_pfh_tile_rows)
     const size_t n_i32 = 3 * (size_t)E + 3 * (size_t)max_tiles + 4 + 2 * np;
     // the tolerance GEMM addresses its A rows with 32-bit byte offsets (kr_prefill_h.hip): a pass holds at most 4 GiB of f16 rows
     if ((size_t)CH * H * 2 >= (1ull << 32) || np * I * 2 >= (1ull << 32))
@@ -1047,14 +1047,14 @@ static int moe_prefill_fast(kr_engine* e, Layer& L, const void* x_bf16, const in
         const int mc = M - m0 < CH ? M - m0 : CH;
         const uint16_t* xc = (const uint16_t*)x_bf16 + (size_t)m0 * H;
         const int32_t* idc = ids + (size_t)m0 * topk; const float* wc = wts + (size_t)m0 * topk;
-        const int tiles_bound = (mc * topk) / 64 + E + 1;
+        const int tr = kr_pfh_tile_rows(L.w13.view(), L.w2.view(), (long)mc * topk, E), tiles_bound = (mc * topk) / tr + E + 1;
         int run = (int)(((long)mc * topk / E + 63) / 64);           // row tiles of an average expert: they share an XCD (one L2 fill of its weights)
         run = run < 1 ? 1 : (run > 4 ? 4 : run);
-        kr_launch_pf_sort(idc, mc, topk, E, so, st);
+        kr_launch_pf_sort(idc, mc, topk, E, so, st, tr);
         kr_launch_pfh_rows_bf16(xc, mc, H, H, (uint16_t*)P.xf.p, (float*)P.xfm.p, st);
         kr_launch_pfh_w13_act(L.w13.view(), (const uint16_t*)P.xf.p, (const float*)P.xfm.p, &so, topk, 1, tiles_bound, 0, (float*)P.gu.p, mc * topk, act_mode, e->cfg.swiglu_limit,
-                              e->cfg.activation_alpha, (uint16_t*)P.hf.p, (float*)P.hfm.p, st, run);
-        kr_launch_pfh_gemm(L.w2.view(), (const uint16_t*)P.hf.p, (const float*)P.hfm.p, &so, topk, 0, tiles_bound, 0, (float*)P.eo.p, H, st, 0, 2 /* f16 rows */, run);
+                              e->cfg.activation_alpha, (uint16_t*)P.hf.p, (float*)P.hfm.p, st, run, nullptr, nullptr, tr);
+        kr_launch_pfh_gemm(L.w2.view(), (const uint16_t*)P.hf.p, (const float*)P.hfm.p, &so, topk, 0, tiles_bound, 0, (float*)P.eo.p, H, st, 0, 2 /* f16 rows */, run, nullptr, tr);
         if (use_shared) {
             kr_launch_pfh_gemm(L.sw13.view(), (const uint16_t*)P.xf.p, (const float*)P.xfm.p, nullptr, topk, 0, 0, mc, (float*)P.sgu.p, 2 * SI, st);
             kr_launch_pfh_act((const float*)P.sgu.p, mc, SI, 2 * SI, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (uint16_t*)P.shf.p, (float*)P.shfm.p, st);

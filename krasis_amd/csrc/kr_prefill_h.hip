@@ -591,6 +591,124 @@ __global__ void __launch_bounds__(256, OCC) kr_pfh_gemm_kernel(const KrPfGemmHAr
 }
 
 
+// Few rows per expert, INT4: every weight is used once or twice and the launch is a stream of weights, which the tiles above interrupt with two barriers and a commit to LDS per 256 k.
+// Here a workgroup puts a tile's rows into LDS once, and each wave streams strips of 16 columns straight to registers, D steps of 256 k ahead, without a barrier, on
+// v_mfma_f32_16x16x32_f16: the weights are the first operand, so that a lane ends with four neighbouring columns of one row.  Same f16 values of rows and weights as the tiles, f32
+// sums over all of K.
+struct PfhStripStep { u32x4 w[2]; uint32_t sc; };      // 256 k of a strip: a lane's two records of its column, the two groups' scales
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+#define PFH_ST_ROWS 16      // rows of a tile
+#define PFH_ST_WAVES 8
+__global__ void __launch_bounds__(64 * PFH_ST_WAVES, 4) kr_pfh_strip_kernel(const KrPfGemmHArgs a, const int strips_per_wave, const int ncb) {
+    constexpr int ROWS = PFH_ST_ROWS, WAVES = PFH_ST_WAVES, D = 4;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, tq = __builtin_amdgcn_readfirstlane(slot / ncb), mt = tq * 8 + xcd, cb = slot - tq * ncb;      // a tile's column blocks on one XCD
+    if (mt >= a.n_tiles[0]) return;
+    const int expert = a.tile_expert[mt], row0 = a.tile_row0[mt], rows = a.tile_rows[mt];
+    const KrMatDev& m = a.m;
+    const int K = m.ng * 128, LD = 2 * K + 16, ng = m.ng, ngp = m.ngp;
+    float* rmul = reinterpret_cast<float*>(smem + ROWS * LD);                 // [ROWS]
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, q = lane >> 4;
+    const char* wq = reinterpret_cast<const char*>(m.q) + (size_t)expert * m.q_stride;
+    const uint32_t* wsc = reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(m.s) + (size_t)expert * m.s_stride);
+    // this wave's strips: cb * WAVES * strips_per_wave + wave + WAVES * i, each ngp steps
+    const int nstrip = m.N / 16, s0 = cb * WAVES * strips_per_wave + wave;
+    const int mine = s0 < nstrip ? min(strips_per_wave, (nstrip - s0 + WAVES - 1) / WAVES) : 0, steps = __builtin_amdgcn_readfirstlane(mine * ngp);
+    const uint32_t woff = ((uint32_t)(r >> 3) * ngp * 64 + (r & 7) * 8 + q) * 16, soff = (uint32_t)(r >> 3) * ngp * 8 + (r & 7);
+    const char* wb = wq + (size_t)2 * s0 * ngp * 1024;
+    size_t sb = (size_t)2 * s0 * ngp * 8;
+    int rs = s0, rg = 0;                                       // strip and step of the next request
+    auto request = [&](PfhStripStep& p) {
+        p.w[0] = kr_ldg_nt(reinterpret_cast<const u32x4*>(wb + woff)); p.w[1] = kr_ldg_nt(reinterpret_cast<const u32x4*>(wb + woff + 64));
+        p.sc = wsc[sb + soff];
+        wb += 1024; sb += 8;
+        if (++rg == ngp) { rg = 0; rs += WAVES; wb = wq + (size_t)2 * rs * ngp * 1024; sb = (size_t)2 * rs * ngp * 8; }
+    };
+    PfhStripStep ring[D];
+    if (mine > 0) {
+#pragma unroll
+        for (int d = 0; d < D; d++) if (d < steps) request(ring[d]);
+    }
+    // ---- the tile's rows, 16 bytes (8 k, in image order) per thread and turn; rows past the last one hold zeros
+    for (int i = tid; i < ROWS * (K / 8); i += 64 * WAVES) {
+        const int row = i / (K / 8), k8 = i - row * (K / 8);
+        u32x4 v = {0, 0, 0, 0};
+        if (row < rows) {
+            const size_t src = a.gather_tokens ? a.row_pair[row0 + row] / a.topk : row0 + row;
+            v = *reinterpret_cast<const u32x4*>(a.a + src * K + (size_t)k8 * 8);
+            if (k8 == 0) rmul[row] = a.out_bf16 == 2 ? 1.0f : a.a_mul[src];      // f16 rows carry the raw sums: the combine pass applies the row multiplier
+        }
+        *reinterpret_cast<u32x4*>(smem + row * LD + k8 * 16) = v;
+    }
+    __syncthreads();
+    if (mine == 0) return;
+    uint32_t M0 = 0x000F000Fu, M1 = 0x00F000F0u, MH = 0x03C003C0u, Kc = 0x64006400u;      // de-quantization masks, kept in registers (see pfh_dq4)
+    asm volatile("" : "+v"(M0), "+v"(M1), "+v"(MH), "+v"(Kc));
+    const char* arow = smem + r * LD + q * 32;
+    v4f acc;
+    int cs = s0, gp = 0;                                       // strip and step in it of the next step
+    auto step = [&](const PfhStripStep& p) {
+        if (gp == 0) acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int hh = 0; hh < 2; hh++) {
+            const int g = 2 * gp + hh;
+            if (g >= ng) break;
+            const _Float16 s1 = (_Float16)(__uint_as_float((hh ? p.sc >> 16 : p.sc & 0xFFFFu) << 16) * 0.25f), c1 = (_Float16)(-1536.0f * (float)s1);
+            const v2h sq = {s1, s1}, cq = {c1, c1};
+#pragma unroll
+            for (int s = 0; s < 2; s++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const v8h wf = pfh_dq4(p.w[s][2 * hh + h], sq, cq, M0, M1, MH, Kc);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf, *reinterpret_cast<const v8h*>(arow + g * 256 + s * 128 + h * 16), acc, 0, 0, 0);      // k = 128 g + 16 (q + 4 s) + 8 h
+                }
+        }
+        if (++gp < ngp) return;
+        const int n = cs * 16 + 4 * q;
+        gp = 0; cs += WAVES;
+        if (r >= rows) return;
+        const size_t o = (size_t)(row0 + r) * a.out_ld + n;
+        const float rm = rmul[r];
+        if (a.out_bf16 == 2) {
+            uint16_t h4[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) pfh_put<2>(h4, c, acc[c] * rm);
+            *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(a.out) + o) = u32x2{(uint32_t)h4[0] | ((uint32_t)h4[1] << 16), (uint32_t)h4[2] | ((uint32_t)h4[3] << 16)};
+        } else *reinterpret_cast<float4*>(a.out + o) = make_float4(acc[0] * rm, acc[1] * rm, acc[2] * rm, acc[3] * rm);
+    };
+    int i = 0;
+    for (; i + 2 * D <= steps; i += D) {       // (no branch around a request: the compiler's count of what is in flight stays exact)
+#pragma unroll
+        for (int d = 0; d < D; d++) { step(ring[d]); request(ring[d]); }
+    }
+    for (; i < steps; i += D) {
+#pragma unroll
+        for (int d = 0; d < D; d++)
+            if (i + d < steps) { step(ring[d]); if (i + d + D < steps) request(ring[d]); }
+    }
+}
+static size_t pfh_strip_lds(int K) { return (size_t)PFH_ST_ROWS * (2 * K + 16 + 4); }
+static void pfh_strip_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st) {
+    constexpr int WAVES = PFH_ST_WAVES;
+    const size_t lds = pfh_strip_lds(a.m.ng * 128);
+    if (kr_lds_optin((const void*)kr_pfh_strip_kernel, lds)) return;      // (the caller sees the runtime's error)
+    // strips per wave: as many as leave two rounds of workgroups (two a compute unit): the rows are staged once for all of them
+    const int groups = (a.m.N / 16 + WAVES - 1) / WAVES;
+    int spw = 4;
+    while (spw > 1 && (long)mt * ((groups + spw - 1) / spw) < 1024) spw /= 2;
+    const int ncb = (groups + spw - 1) / spw;
+    hipLaunchKernelGGL(kr_pfh_strip_kernel, dim3(((mt + 7) / 8) * 8 * ncb), dim3(64 * WAVES), lds, st, a, spw, ncb);
+}
+// Rows of a tile of the experts' table for `rows` rows on E experts: strips while an expert seldom has more than one tile of 16, 64-row tiles beyond.  With hundreds of experts the
+// stream is long enough to carry second tiles too.  A layer's experts, us, 64-row tiles -> strips: 512 of 2048 x 512, top 10: 32 rows 148 -> 104, 256 278 -> 206, 512 291 -> 241, 716 (14 an
+// expert) 294 -> 271; 64 of 2048 x 1408, top 6: 8 rows 82 -> 68, 80 113 -> 97, 107 (10) 115 -> 113, 130 (12) 115 -> 116, 149 (14) 114 -> 124.  Tiles of 32 rows gained nothing from 14 on.
+int kr_pfh_tile_rows(const KrMatDev& m0, const KrMatDev& m1, long rows, int E) {
+    const int K = 128 * (m0.ng > m1.ng ? m0.ng : m1.ng);
+    if (m0.bits != 4 || m1.bits != 4 || m0.qs || m1.qs || m0.N % 16 || m1.N % 16) return PFH_BM;
+    return rows <= (E >= 256 ? 14L : 10L) * E && pfh_strip_lds(K) <= 160 * 1024 ? PFH_ST_ROWS : PFH_BM;
+}
+
 template <int NC, int BITS, int SB = 0, int G = 0, int OCC = 2>
 static void pfh_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st) {
     constexpr int BN = 128 * NC, LDB = BITS == 8 ? PFH_LDB8 : PFH_LDB4;
@@ -647,13 +765,17 @@ void kr_launch_pfh_act(const float* gu, int rows, int n, int gu_ld, int act_mode
     else hipLaunchKernelGGL(kr_pfh_act_kernel<KR_ACT_SILU_MUL>, dim3(rows), dim3(256), 0, st, gu, n, gu_ld, swiglu_limit, alpha, out, mul);
 }
 void kr_launch_pfh_gemm(const KrMatDev& m, const uint16_t* a_h, const float* a_mul, const KrPfSort* sort, int topk, int gather_tokens, int max_tiles,
-                        int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows, int out_bf16, int run, const uint16_t* a_sum32) {
+                        int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows, int out_bf16, int run, const uint16_t* a_sum32, int tile_rows) {
     KrPfGemmHArgs a{};
     a.m = m; a.a = a_h; a.a_mul = a_mul; a.a_sum = a_sum32; a.topk = topk; a.gather_tokens = gather_tokens; a.scatter_rows = scatter_rows; a.out_bf16 = out_bf16;
     if (sort) { a.row_pair = sort->row_pair; a.tile_expert = sort->tile_expert; a.tile_row0 = sort->tile_row0; a.tile_rows = sort->tile_rows; a.n_tiles = sort->n_tiles; }
     a.out = out; a.out_ld = out_ld; a.single_expert = single_expert_rows > 0; a.total_rows = single_expert_rows;
     a.run = (single_expert_rows > 0 || run < 1) ? 1 : run;
     const int mt = single_expert_rows > 0 ? (single_expert_rows + PFH_BM - 1) / PFH_BM : max_tiles;
+    if (single_expert_rows <= 0 && tile_rows < PFH_BM) {
+        pfh_strip_launch(a, mt, st);
+        return;
+    }
     pfh_dispatch(a, mt, st);
 }
 // gate | up GEMM + activation -> the f16 hidden rows (+ multipliers, + per-32 sums for a Q4_K down copy).  Big problems (the 64 x 256 tile form) with
@@ -661,12 +783,12 @@ void kr_launch_pfh_gemm(const KrMatDev& m, const uint16_t* a_h, const float* a_m
 // only makes the f16 form.  Otherwise: the GEMM, then the activation pass over gate | up rows.  Same arithmetic either way.
 void kr_launch_pfh_w13_act(const KrMatDev& m, const uint16_t* a_h, const float* a_mul, const KrPfSort* sort, int topk, int gather_tokens, int max_tiles,
                            int single_expert_rows, float* gu, int rows, int act_mode, float swiglu_limit, float alpha, uint16_t* h_out, float* h_mul,
-                           hipStream_t st, int run, const uint16_t* a_sum32, uint16_t* h_sums32) {
+                           hipStream_t st, int run, const uint16_t* a_sum32, uint16_t* h_sums32, int tile_rows) {
     const int I = m.N / 2;
     const int mt = single_expert_rows > 0 ? (single_expert_rows + PFH_BM - 1) / PFH_BM : max_tiles;
-    const bool fuse = m.bits == 4 && I % 128 == 0 && I <= 2048 && (long)mt * (m.N / 128) >= 2048;
+    const bool fuse = tile_rows == PFH_BM && m.bits == 4 && I % 128 == 0 && I <= 2048 && (long)mt * (m.N / 128) >= 2048;
     if (!fuse) {
-        kr_launch_pfh_gemm(m, a_h, a_mul, sort, topk, gather_tokens, max_tiles, single_expert_rows, gu, 2 * I, st, 0, 0, run, a_sum32);
+        kr_launch_pfh_gemm(m, a_h, a_mul, sort, topk, gather_tokens, max_tiles, single_expert_rows, gu, 2 * I, st, 0, 0, run, a_sum32, tile_rows);
         kr_launch_pfh_act(gu, rows, I, 2 * I, act_mode, swiglu_limit, alpha, h_out, h_mul, st, h_sums32);
         return;
     }

@@ -1,5 +1,5 @@
 """Launches of the tolerance prompt pass that do the work of two (krasis_amd/csrc/kr_prefill_ops.hip), and the pair sort of long chunks (kr_prefill.hip), against the launches that they
-stand for: bit for bit, since the order of every sum is the same."""
+stand for: bit for bit, since the order of every sum is the same.  And the strips of the tolerance GEMM (kr_prefill_h.hip) against the exact form."""
 import numpy as np
 import pytest
 
@@ -41,3 +41,26 @@ def test_pair_sort_of_long_chunks(E, k, M):
     h = M // 2
     parts = np.concatenate([_prefill_mode(eng, torch, x[:h], ids[:h], w[:h], 0), _prefill_mode(eng, torch, x[h:], ids[h:], w[h:], 0)])
     assert np.array_equal(whole.view(np.uint32), parts.view(np.uint32)), float(np.abs(whole - parts).max())
+
+
+@pytest.mark.parametrize("H,I,E,k,M", [
+    (2048, 512, 64, 10, 64),       # ten rows an expert: tiles of up to 16 and second ones
+    (256, 128, 8, 2, 1),           # one row; one step a strip
+    (384, 128, 8, 2, 17),          # an odd group count: the last step of a strip holds one group
+    (512, 384, 300, 4, 1050),      # hundreds of experts: fourteen rows each; an odd group count in the down projection, strips that do not fill a workgroup
+])
+def test_strips_of_few_rows_per_expert(H, I, E, k, M):
+    """Rows and hidden values are rounded to f16 once each, relative error at most 2^-11 a value, in both products of an expert: the norm of the difference to the exact form (sixteen
+    times finer digits) stays under 2 * 2^-11."""
+    eng, experts, shared, rng, torch = _setup(H, I, E, k, 0, 1.0)
+    x = rand_bf16(rng, (M, H))
+    ids = np.argsort(rng.random((M, E)), axis=1)[:, :k].astype(np.int32)
+    if M > 16:
+        ids[:16, 0] = 0; ids[3, 1] = -1; ids[7, :] = -1                # an expert that fills its tile, rows left out
+        ids[:16, 1:][ids[:16, 1:] == 0] = -1
+    w = rng.random((M, k)).astype(F)
+    exact, fast = (_prefill_mode(eng, torch, x, ids, w, mode) for mode in (0, 1))
+    rel = float(np.linalg.norm((fast - exact).astype(np.float64)) / np.linalg.norm(exact.astype(np.float64)))
+    assert np.isfinite(fast).all() and 0 < rel <= 2.0 ** -10, rel
+    if M > 16:
+        assert not fast[7].any()

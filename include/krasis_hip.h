@@ -161,6 +161,8 @@ int kr_reduce_sum_bf16(kr_engine* e, const void* const* inputs, int n_inputs, vo
 /* test / tuning hook: (token, slot) pairs per pass of kr_moe_prefill (0 = default 81 920: 8192 tokens of a top-10 model, 81 920 top-1 rows
  * of the expert-parallel dispatch); larger batches are walked in passes of pairs / topk tokens */
 int kr_moe_set_prefill_pairs(kr_engine* e, int pairs);
+/* test hook: how the last pass of kr_moe_prefill cut its rows, in tiles or in strips (few rows per expert); waits for the device */
+int kr_moe_prefill_tiles(kr_engine* e, int* tiles, int* strips);
 /* numerics of the prompt-pass expert GEMMs of kr_moe_prefill: 0 (default) = the CPU engine's arithmetic (INT16 activation digits, one f32 fma per
  * 128-group: bit-identical to kr_moe_forward, moe.rs:184); 1 = tolerance form: f16 activations x weights de-quantized in registers, f32 accumulation
  * over the whole k range -- the dataflow of the reference's GPU prompt pass (gpu_prefill.py:64-239, Marlin).  Native GGUF layers stay exact.

@@ -1026,7 +1026,7 @@ static int moe_prefill_fast(kr_engine* e, Layer& L, const void* x_bf16, const in
     const int CHmax = pairs / topk > 64 ? pairs / topk : 64;
     const int CH = M < CHmax ? M : CHmax;
     const size_t np = (size_t)CH * topk;
-    const int max_tiles = (int)(np / 16) + E + 1;      // (tiles of 16 rows are the smallest, kr_pfh_tile_rows)
+    const int max_tiles = (int)(np / 16) + E + 1;      // (strips of 16 rows are the smallest, kr_pfh_tiles)
     const size_t n_i32 = 3 * (size_t)E + 3 * (size_t)max_tiles + 4 + 2 * np;
     // the tolerance GEMM addresses its A rows with 32-bit byte offsets (kr_prefill_h.hip): a pass holds at most 4 GiB of f16 rows
     if ((size_t)CH * H * 2 >= (1ull << 32) || np * I * 2 >= (1ull << 32))
@@ -1040,21 +1040,21 @@ static int moe_prefill_fast(kr_engine* e, Layer& L, const void* x_bf16, const in
     KrPfSort so{};
     so.counts = ib; so.offsets = ib + E; so.cursor = ib + 2 * E; ib += 3 * E;
     so.tile_expert = ib; so.tile_row0 = ib + max_tiles; so.tile_rows = ib + 2 * max_tiles; ib += 3 * max_tiles;
-    so.n_tiles = ib; ib += 4; so.row_pair = ib; so.pair_row = ib + np;
+    so.n_tiles = ib; P.n_tiles_at = (size_t)(ib - (int*)P.i32.p); ib += 4; so.row_pair = ib; so.pair_row = ib + np;
     const int act_mode = e->cfg.swiglu_limit > 0.0f ? KR_ACT_GPTOSS : KR_ACT_SILU_FUSED;
     const size_t ob = out_dtype == KR_OUT_BF16 ? 2 : 4;
     for (int m0 = 0; m0 < M; m0 += CH) {
         const int mc = M - m0 < CH ? M - m0 : CH;
         const uint16_t* xc = (const uint16_t*)x_bf16 + (size_t)m0 * H;
         const int32_t* idc = ids + (size_t)m0 * topk; const float* wc = wts + (size_t)m0 * topk;
-        const int tr = kr_pfh_tile_rows(L.w13.view(), L.w2.view(), (long)mc * topk, E), tiles_bound = (mc * topk) / tr + E + 1;
+        const KrPfTiles cut = kr_pfh_tiles(L.w13.view(), L.w2.view(), (long)mc * topk, E);
         int run = (int)(((long)mc * topk / E + 63) / 64);           // row tiles of an average expert: they share an XCD (one L2 fill of its weights)
         run = run < 1 ? 1 : (run > 4 ? 4 : run);
-        kr_launch_pf_sort(idc, mc, topk, E, so, st, tr);
+        kr_launch_pf_sort(idc, mc, topk, E, so, st, cut);
         kr_launch_pfh_rows_bf16(xc, mc, H, H, (uint16_t*)P.xf.p, (float*)P.xfm.p, st);
-        kr_launch_pfh_w13_act(L.w13.view(), (const uint16_t*)P.xf.p, (const float*)P.xfm.p, &so, topk, 1, tiles_bound, 0, (float*)P.gu.p, mc * topk, act_mode, e->cfg.swiglu_limit,
-                              e->cfg.activation_alpha, (uint16_t*)P.hf.p, (float*)P.hfm.p, st, run, nullptr, nullptr, tr);
-        kr_launch_pfh_gemm(L.w2.view(), (const uint16_t*)P.hf.p, (const float*)P.hfm.p, &so, topk, 0, tiles_bound, 0, (float*)P.eo.p, H, st, 0, 2 /* f16 rows */, run, nullptr, tr);
+        kr_launch_pfh_w13_act(L.w13.view(), (const uint16_t*)P.xf.p, (const float*)P.xfm.p, &so, topk, 1, cut.max_tiles, 0, (float*)P.gu.p, mc * topk, act_mode, e->cfg.swiglu_limit,
+                              e->cfg.activation_alpha, (uint16_t*)P.hf.p, (float*)P.hfm.p, st, run, nullptr, nullptr, &cut);
+        kr_launch_pfh_gemm(L.w2.view(), (const uint16_t*)P.hf.p, (const float*)P.hfm.p, &so, topk, 0, cut.max_tiles, 0, (float*)P.eo.p, H, st, 0, 2 /* f16 rows */, run, nullptr, &cut);
         if (use_shared) {
             kr_launch_pfh_gemm(L.sw13.view(), (const uint16_t*)P.xf.p, (const float*)P.xfm.p, nullptr, topk, 0, 0, mc, (float*)P.sgu.p, 2 * SI, st);
             kr_launch_pfh_act((const float*)P.sgu.p, mc, SI, 2 * SI, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (uint16_t*)P.shf.p, (float*)P.shfm.p, st);
@@ -1079,7 +1079,7 @@ int kr_moe_prefill_set(kr_engine* e, int layer, const void* x_bf16, const int32_
         return kr_fail(KR_ERR_VALUE, "kr_moe_prefill expects device pointers (hidden/topk tensors live in HBM during prefill)");
     std::lock_guard<std::mutex> lk(e->mu);
     KR_HIP(hipSetDevice(e->device));
-    const bool fast = e->gemm_fast || (set & KR_PF_SET_FAST);
+    const bool fast = e->gemm_fast || (set & KR_PF_SET_FAST), beside = (set & KR_PF_SET_BESIDE) != 0;
     set &= 0xFF;
     if (L.gguf) {      // native GGUF blocks: the exact int8-MFMA form, or (tolerance mode, Q4_K layers) f16 MFMA on the re-tiled copy
         if (fast && gg_fast_ok(L, e->cfg.hidden_size, L.gguf_shared && !routed_only)) return moe_prefill_gguf_fast(e, L, x_bf16, ids, wts, out, M, topk, out_dtype, routed_only, set, st);
@@ -1099,7 +1099,7 @@ int kr_moe_prefill_set(kr_engine* e, int layer, const void* x_bf16, const int32_
     const int CHmax = pairs / topk > 64 ? pairs / topk : 64;
     const int CH = M < CHmax ? M : CHmax;
     const size_t np = (size_t)CH * topk;
-    const int max_tiles = (int)(np / 16) + E + 1;      // (tiles of 16 rows are the smallest, kr_pf_tile_rows)
+    const int max_tiles = (int)(np / 16) + E + 1;      // (strips of 16 rows are the smallest, kr_pf_tiles)
     const size_t n_i32 = 3 * (size_t)E + 3 * (size_t)max_tiles + 4 + 2 * np;
     if (P.i32.ensure(n_i32 * 4) || P.xh.ensure((size_t)CH * H) || P.xl.ensure((size_t)CH * H) || P.xs.ensure((size_t)CH * (H / 128) * 4) ||
         P.gu.ensure(np * 2 * I * 4) || P.hh.ensure(np * I) || P.hl.ensure(np * I) || P.hs.ensure(np * (I / 128) * 4) || P.eo.ensure(np * H * 4))
@@ -1111,23 +1111,23 @@ int kr_moe_prefill_set(kr_engine* e, int layer, const void* x_bf16, const int32_
     KrPfSort so{};
     so.counts = ib; so.offsets = ib + E; so.cursor = ib + 2 * E; ib += 3 * E;
     so.tile_expert = ib; so.tile_row0 = ib + max_tiles; so.tile_rows = ib + 2 * max_tiles; ib += 3 * max_tiles;
-    so.n_tiles = ib; ib += 4; so.row_pair = ib; so.pair_row = ib + np;
+    so.n_tiles = ib; P.n_tiles_at = (size_t)(ib - (int*)P.i32.p); ib += 4; so.row_pair = ib; so.pair_row = ib + np;
     const int act_mode = e->cfg.swiglu_limit > 0.0f ? KR_ACT_GPTOSS : KR_ACT_SILU_FUSED;
     const size_t ob = out_dtype == KR_OUT_BF16 ? 2 : 4;
     for (int m0 = 0; m0 < M; m0 += CH) {
         const int mc = M - m0 < CH ? M - m0 : CH;
         const uint16_t* xc = (const uint16_t*)x_bf16 + (size_t)m0 * H;
         const int32_t* idc = ids + (size_t)m0 * topk; const float* wc = wts + (size_t)m0 * topk;
-        const int tr = kr_pf_tile_rows(L.w13.view(), L.w2.view(), (long)mc * topk, E), tiles_bound = (mc * topk) / tr + E + 1;
-        kr_launch_pf_sort(idc, mc, topk, E, so, st, tr);
+        const KrPfTiles cut = kr_pf_tiles(L.w13.view(), L.w2.view(), (long)mc * topk, E, beside);
+        kr_launch_pf_sort(idc, mc, topk, E, so, st, cut);
         kr_launch_pf_quant_x(xc, mc, H, (int8_t*)P.xh.p, (int8_t*)P.xl.p, (float*)P.xs.p, st);
         const int var_rows = (long)mc * topk < 48L * E;     // fewer than ~48 rows per expert: most 64-row tiles have an empty second half
         kr_launch_pf_gemm(L.w13.view(), (const uint32_t*)L.w13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, &so, topk, 1,
-                          tiles_bound, 0, (float*)P.gu.p, 2 * I, st, 0, 0, var_rows, tr);
+                          cut.max_tiles, 0, (float*)P.gu.p, 2 * I, st, 0, 0, var_rows, &cut);
         kr_launch_pf_act((const float*)P.gu.p, mc * topk, I, 2 * I, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.hh.p, (int8_t*)P.hl.p,
                          (float*)P.hs.p, st);
         kr_launch_pf_gemm(L.w2.view(), (const uint32_t*)L.w2.wsum.p, (const int8_t*)P.hh.p, (const int8_t*)P.hl.p, (const float*)P.hs.p, &so, topk, 0,
-                          tiles_bound, 0, (float*)P.eo.p, H, st, 0, 0, var_rows, tr);
+                          cut.max_tiles, 0, (float*)P.eo.p, H, st, 0, 0, var_rows, &cut);
         if (use_shared) {
             kr_launch_pf_gemm(L.sw13.view(), (const uint32_t*)L.sw13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, nullptr, topk, 0,
                               0, mc, (float*)P.sgu.p, 2 * SI, st);
@@ -1159,7 +1159,7 @@ int kr_moe_prefill_rows(kr_engine* e, int layer, const void* rows_bf16, const in
     const int pairs = e->pf_pairs > 0 ? e->pf_pairs : KR_PF_PAIRS;
     const int CH = n < pairs ? n : pairs;
     const size_t np = (size_t)CH;
-    const int max_tiles = (int)(np / 16) + E + 1;      // (tiles of 16 rows are the smallest, kr_pf_tile_rows)
+    const int max_tiles = (int)(np / 16) + E + 1;      // (strips of 16 rows are the smallest, kr_pf_tiles)
     const size_t n_i32 = 3 * (size_t)E + 3 * (size_t)max_tiles + 4 + 2 * np;
     if (P.i32.ensure(n_i32 * 4) || P.xh.ensure((size_t)CH * H) || P.xl.ensure((size_t)CH * H) || P.xs.ensure((size_t)CH * (H / 128) * 4) ||
         P.gu.ensure(np * 2 * I * 4) || P.hh.ensure(np * I) || P.hl.ensure(np * I) || P.hs.ensure(np * (I / 128) * 4))
@@ -1168,20 +1168,20 @@ int kr_moe_prefill_rows(kr_engine* e, int layer, const void* rows_bf16, const in
     KrPfSort so{};
     so.counts = ib; so.offsets = ib + E; so.cursor = ib + 2 * E; ib += 3 * E;
     so.tile_expert = ib; so.tile_row0 = ib + max_tiles; so.tile_rows = ib + 2 * max_tiles; ib += 3 * max_tiles;
-    so.n_tiles = ib; ib += 4; so.row_pair = ib; so.pair_row = ib + np;
+    so.n_tiles = ib; P.n_tiles_at = (size_t)(ib - (int*)P.i32.p); ib += 4; so.row_pair = ib; so.pair_row = ib + np;
     const int act_mode = e->cfg.swiglu_limit > 0.0f ? KR_ACT_GPTOSS : KR_ACT_SILU_FUSED;
     const size_t ob = out_bf16 ? 2 : 4;
     for (int m0 = 0; m0 < n; m0 += CH) {
         const int mc = n - m0 < CH ? n - m0 : CH;
-        const int tr = kr_pf_tile_rows(L.w13.view(), L.w2.view(), mc, E), tiles_bound = mc / tr + E + 1;
-        kr_launch_pf_sort(lid + m0, mc, 1, E, so, st, tr);
+        const KrPfTiles cut = kr_pf_tiles(L.w13.view(), L.w2.view(), mc, E, true);
+        kr_launch_pf_sort(lid + m0, mc, 1, E, so, st, cut);
         kr_launch_pf_quant_x((const uint16_t*)rows_bf16 + (size_t)m0 * H, mc, H, (int8_t*)P.xh.p, (int8_t*)P.xl.p, (float*)P.xs.p, st);
         const int var_rows = (long)mc < 48L * E;
         kr_launch_pf_gemm(L.w13.view(), (const uint32_t*)L.w13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, &so, 1, 1,
-                          tiles_bound, 0, (float*)P.gu.p, 2 * I, st, 0, 0, var_rows, tr);
+                          cut.max_tiles, 0, (float*)P.gu.p, 2 * I, st, 0, 0, var_rows, &cut);
         kr_launch_pf_act((const float*)P.gu.p, mc, I, 2 * I, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.hh.p, (int8_t*)P.hl.p, (float*)P.hs.p, st);
         kr_launch_pf_gemm(L.w2.view(), (const uint32_t*)L.w2.wsum.p, (const int8_t*)P.hh.p, (const int8_t*)P.hl.p, (const float*)P.hs.p, &so, 1, 0,
-                          tiles_bound, 0, (float*)((char*)out + (size_t)m0 * H * ob), H, st, 1, out_bf16, var_rows, tr);
+                          cut.max_tiles, 0, (float*)((char*)out + (size_t)m0 * H * ob), H, st, 1, out_bf16, var_rows, &cut);
     }
     KR_HIP(hipGetLastError());
     return KR_OK;
@@ -1191,6 +1191,20 @@ extern "C" int kr_moe_prefill(kr_engine* e, int layer, const void* x_bf16, const
                               int out_dtype, int routed_only, void* stream) {
     if (int rc = check_layer(e, layer)) return rc;
     return kr_moe_prefill_set(e, layer, x_bf16, ids, wts, out, M, topk, out_dtype, routed_only, 0, kr_pick_stream(e, stream));
+}
+
+// test hook: the tiles and the strips that the last pass of kr_moe_prefill (or, with expert parallelism, of its rows) was cut into; one of the two is zero
+extern "C" int kr_moe_prefill_tiles(kr_engine* e, int* tiles, int* strips) {
+    if (!e || !tiles || !strips) return kr_fail(KR_ERR_VALUE, "null argument");
+    std::lock_guard<std::mutex> lk(e->mu);
+    const kr_engine::PfSet& P = e->pf[0];
+    if (!P.n_tiles_at) return kr_fail(KR_ERR_STATE, "no prompt pass yet");
+    KR_HIP(hipSetDevice(e->device));
+    KR_HIP(hipDeviceSynchronize());
+    int n[3];
+    KR_HIP(hipMemcpy(n, (const int*)P.i32.p + P.n_tiles_at, sizeof n, hipMemcpyDeviceToHost));
+    *tiles = n[0]; *strips = n[2];
+    return KR_OK;
 }
 
 // test / tuning hook: (token, slot) pairs per pass of kr_moe_prefill (0 = default 81 920)

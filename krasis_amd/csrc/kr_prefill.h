@@ -16,20 +16,24 @@ static inline void kr_pf_super_tile(int nrt, int ncb, int* sr, int* sc, int* n_s
 struct KrPfSort {
     int* counts; int* offsets; int* cursor;        // [E]
     int* tile_expert; int* tile_row0; int* tile_rows;  // [max_tiles]
-    int* n_tiles;                                   // [1]
+    int* n_tiles;                                   // [3]: tiles, rows, strips (KrPfTiles)
     int* row_pair;                                  // [n_pairs]  GEMM row -> (token*topk + slot)
     int* pair_row;                                  // [n_pairs]  inverse (-1 for skipped ids)
 };
-void kr_launch_pf_sort(const int32_t* ids, int M, int topk, int E, KrPfSort s, hipStream_t st, int bm = 64 /* rows per tile of the tile table */);
+// How the rows of a pass are cut.  `strip` > 0: the sort, which alone knows how many rows every expert has, cuts strips of that many rows instead if those are at most strip_most
+// eighths of the tiles; each of the two forms is launched then, and the one that was not taken finds a count of zero.  max_tiles, max_strips: the most there can be of a form taken.
+struct KrPfTiles { int rows, strip, strip_most, max_tiles, max_strips; };
+KrPfTiles kr_pf_cut(int tile_rows, int strip, int strip_most, long rows, int E);
+void kr_launch_pf_sort(const int32_t* ids, int M, int topk, int E, KrPfSort s, hipStream_t st, const KrPfTiles& t = KrPfTiles{64, 0, 0, 0, 0});
 void kr_launch_pf_quant_x(const uint16_t* x, int M, int K, int8_t* xh, int8_t* xl, float* xs, hipStream_t st);
 void kr_launch_pf_act(const float* gu, int rows, int n, int gu_ld, int act_mode, float swiglu_limit, float alpha, int8_t* hh, int8_t* hl, float* hs, hipStream_t st);
 void kr_launch_pf_wsum(const KrMatDev& m, int n_experts, uint32_t* wsum, hipStream_t st);
 void kr_launch_pf_gemm(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_hi, const int8_t* a_lo, const float* a_scale, const KrPfSort* sort, int topk,
                        int gather_tokens, int max_tiles, int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows = 0, int out_bf16 = 0,
                        int var_rows = 0 /* expert tiles mostly <= 32 rows: kernel variant that skips empty 32-row blocks */,
-                       int tile_rows = 64 /* of the tile table (kr_pf_tile_rows) */);
-// rows per tile of the exact GEMMs that will run on one tile table: 128 (the wide kernel) or 64
-int kr_pf_tile_rows(const KrMatDev& m0, const KrMatDev& m1, long rows, int E);
+                       const KrPfTiles* t = nullptr /* of the tile table; null: tiles of 64 */);
+// of the exact GEMMs that will run on one tile table: tiles of 128 rows (the wide kernel) or 64, and whether strips may take their place
+KrPfTiles kr_pf_tiles(const KrMatDev& m0, const KrMatDev& m1, long rows, int E, bool beside /* launches of other chunks run at the same time */);
 void kr_launch_pf_gemm_multi(const KrMatDev* mats, const uint32_t* const* wsums, float* const* outs, const int* out_lds, int n, const int8_t* a_hi, const int8_t* a_lo,
                              const float* a_scale, int M, hipStream_t st);
 void kr_launch_pf_combine(const float* eo, const int* pair_row, const float* wts, int M, int topk, int H, const float* shared_eo, float rsf, void* out,
@@ -53,11 +57,11 @@ void kr_launch_pfh_act(const float* gu, int rows, int n, int gu_ld, int act_mode
                        uint16_t* sums32 = nullptr);     // act_mode 3 = libm SiLU of expert_forward_gguf (rows of at most 2048 values)
 void kr_launch_pfh_gemm(const KrMatDev& m, const uint16_t* a_h, const float* a_mul, const KrPfSort* sort, int topk, int gather_tokens, int max_tiles,
                         int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows = 0, int out_bf16 = 0, int run = 1,
-                        const uint16_t* a_sum32 = nullptr /* required when m.qs is set (Q4_K copy) */, int tile_rows = 64 /* of the tile table (kr_pfh_tile_rows) */);
-int kr_pfh_tile_rows(const KrMatDev& m0, const KrMatDev& m1, long rows, int E);      // of the tolerance GEMMs' tile table, at least 16
+                        const uint16_t* a_sum32 = nullptr /* required when m.qs is set (Q4_K copy) */, const KrPfTiles* t = nullptr /* of the tile table; null: tiles of 64 */);
+KrPfTiles kr_pfh_tiles(const KrMatDev& m0, const KrMatDev& m1, long rows, int E);      // of the tolerance GEMMs' tile table
 void kr_launch_pfh_w13_act(const KrMatDev& m, const uint16_t* a_h, const float* a_mul, const KrPfSort* sort, int topk, int gather_tokens, int max_tiles,
                            int single_expert_rows, float* gu, int rows, int act_mode, float swiglu_limit, float alpha, uint16_t* h_out, float* h_mul,
-                           hipStream_t st, int run = 1, const uint16_t* a_sum32 = nullptr, uint16_t* h_sums32 = nullptr, int tile_rows = 64);
+                           hipStream_t st, int run = 1, const uint16_t* a_sum32 = nullptr, uint16_t* h_sums32 = nullptr, const KrPfTiles* t = nullptr);
 void kr_launch_pfh_gemm_multi(const KrMatDev* mats, float* const* outs, const int* out_lds, int n, const uint16_t* a_h, const float* a_mul, int M, hipStream_t st);
 // the LDS-ring form of the INT4 tolerance GEMM (kr_prefill_ring.hip) is on by default; 0 keeps the register-staged kernels (process-wide A/B and test hook)
 void kr_pfr_set_enabled(int on);

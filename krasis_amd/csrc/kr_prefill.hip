@@ -115,7 +115,7 @@ __global__ void __launch_bounds__(1024) kr_pf_scan_kernel(const int* __restrict_
 #define KR_PF_SORT1_MAX 32768
 __global__ void __launch_bounds__(1024) kr_pf_sort1_kernel(const int32_t* __restrict__ ids, int n_pairs, int E, int* __restrict__ counts, int* __restrict__ offsets,
                                                           int* __restrict__ tile_expert, int* __restrict__ tile_row0, int* __restrict__ tile_rows,
-                                                          int* __restrict__ n_tiles_out, int* __restrict__ row_pair, int* __restrict__ pair_row, int bm) {
+                                                          int* __restrict__ n_tiles_out, int* __restrict__ row_pair, int* __restrict__ pair_row, int bm, int strip, int strip_most) {
     __shared__ int s_cnt[1024], s_off[1024], s_til[1024], s_cur[1024];
     const int t = threadIdx.x;
     s_cnt[t] = 0; s_cur[t] = 0;
@@ -130,8 +130,10 @@ __global__ void __launch_bounds__(1024) kr_pf_sort1_kernel(const int32_t* __rest
         for (int u = 0; u < NB; u++) if (e[u] >= 0 && e[u] < E) atomicAdd(&s_cnt[e[u]], 1);
     }
     __syncthreads();
-    const int c = t < E ? s_cnt[t] : 0, nt = (c + bm - 1) / bm;
-    s_off[t] = c; s_til[t] = nt;
+    // tiles of bm rows and, in the upper half word, of `strip` rows (at most 32768 / 16 + 1024)
+    const int c = t < E ? s_cnt[t] : 0, nts = strip ? (c + strip - 1) / strip : 0;
+    int nt = (c + bm - 1) / bm;
+    s_off[t] = c; s_til[t] = nt | (nts << 16);
     __syncthreads();
     for (int d = 1; d < 1024; d <<= 1) {             // inclusive Hillis-Steele scans of rows and tiles
         const int a = t >= d ? s_off[t - d] : 0, b = t >= d ? s_til[t - d] : 0;
@@ -139,8 +141,12 @@ __global__ void __launch_bounds__(1024) kr_pf_sort1_kernel(const int32_t* __rest
         s_off[t] += a; s_til[t] += b;
         __syncthreads();
     }
-    const int off = s_off[t] - c, til = s_til[t] - nt;   // exclusive
-    if (t == 1023) { n_tiles_out[0] = s_til[t]; n_tiles_out[1] = s_off[t]; }
+    const int off = s_off[t] - c, all = s_til[1023], n_bm = all & 0xFFFF, n_strip = all >> 16;
+    // one of the two counts is zero: its launch finds nothing to do
+    const bool strips = strip && 8 * n_strip <= strip_most * n_bm;
+    if (t == 1023) { n_tiles_out[0] = strips ? 0 : n_bm; n_tiles_out[1] = s_off[t]; n_tiles_out[2] = strips ? n_strip : 0; }
+    if (strips) { nt = nts; bm = strip; }
+    const int til = (strips ? s_til[t] >> 16 : s_til[t] & 0xFFFF) - nt;   // exclusive
     __syncthreads();
     s_off[t] = off;
     if (t < E) {
@@ -347,10 +353,20 @@ __global__ void __launch_bounds__(256) kr_pf_combine_kernel(const void* __restri
 // ------------------------------------------------------------------------------------------
 // launchers
 // ------------------------------------------------------------------------------------------
-void kr_launch_pf_sort(const int32_t* ids, int M, int topk, int E, KrPfSort s, hipStream_t st, int bm) {
-    const int n = M * topk;
+// strips <= strip_most / 8 tiles, so a pass of strips has at most (strip_most / 8) (tiles <= rows / tile_rows + E) of them; and where tiles were taken, tiles < strips / (strip_most / 8),
+// strips <= rows / strip + tiles, so that tiles < rows / strip / (strip_most / 8 - 1)
+KrPfTiles kr_pf_cut(int tile_rows, int strip, int strip_most, long rows, int E) {
+    KrPfTiles t{tile_rows, strip, strip_most, (int)(rows / tile_rows) + E + 1, 0};
+    if (strip <= 0) return t;
+    if (rows > KR_PF_SORT1_MAX || E > 1024) { t.strip = 0; return t; }      // (the sort's other form cuts tiles only)
+    t.max_strips = (int)(rows / strip) + E + 1;
+    t.max_tiles = std::min(t.max_tiles, (int)(rows * 8 / ((long)strip * (strip_most - 8))) + 1);
+    return t;
+}
+void kr_launch_pf_sort(const int32_t* ids, int M, int topk, int E, KrPfSort s, hipStream_t st, const KrPfTiles& t) {
+    const int n = M * topk, bm = t.rows;
     if (n <= KR_PF_SORT1_MAX && E <= 1024) {
-        hipLaunchKernelGGL(kr_pf_sort1_kernel, dim3(1), dim3(1024), 0, st, ids, n, E, s.counts, s.offsets, s.tile_expert, s.tile_row0, s.tile_rows, s.n_tiles, s.row_pair, s.pair_row, bm);
+        hipLaunchKernelGGL(kr_pf_sort1_kernel, dim3(1), dim3(1024), 0, st, ids, n, E, s.counts, s.offsets, s.tile_expert, s.tile_row0, s.tile_rows, s.n_tiles, s.row_pair, s.pair_row, bm, t.strip, t.strip_most);
         return;
     }
     (void)hipMemsetAsync(s.counts, 0, (size_t)E * 4, st);
@@ -385,18 +401,24 @@ void kr_launch_pf_wsum(const KrMatDev& m, int n_experts, uint32_t* wsum, hipStre
 // (a four-layer INT4 prompt, ms, 64-row tiles / wide from 128 tiles / always wide: 777 tokens 3.99 / 3.89 / 3.98, 1400 tokens 6.30 / 5.64 / 5.89).
 // It knows the fused form of the group sum only, and addresses a digit plane by 32-bit offsets.
 static bool pf_all_fma(const KrMatDev& m) { return m.n_fma >= m.N; }
-// Few rows per expert, INT4: strips, in tiles of 16 rows while an expert seldom has more (up to ten on average: 520 rows on 512 experts 243 us, tiles of 32 245), then of 32 while two
-// halves still cost less than the 64-row tile: to 16 rows an expert (64 experts, 160 rows 174 against 183; 240 rows 213 against 192), with many experts to 24 (512 experts, 1100 rows
-// 331 against 351, 1500 rows 393 against 400).  The rows' digits have to fit the LDS.
-int kr_pf_tile_rows(const KrMatDev& m0, const KrMatDev& m1, long rows, int E) {
-    if (!pf_all_fma(m0) || !pf_all_fma(m1)) return PF_BM;
+// Few rows per expert, INT4: strips may be taken, of 16 rows while an expert seldom has more (up to ten on average), then of 32 while two halves still cost less than the 64-row tile: to
+// 16 rows an expert, with many experts to 24 (us a layer, both products and what stands between them, tiles against strips: 512 experts, top 10, 160 rows 308 / 207, 400 rows 330 / 245, 700
+// rows of 32 340 / 276, 1136 rows 371 / 352; 64 experts, 60 rows 128 / 102, 150 rows of 32 131 / 124; 240 rows 192 / 213).  Beside the launches of other chunks a workgroup of 32 rows (136 KB of LDS)
+// waits for an empty compute unit, also when it has nothing to do (two chunks of 750 tokens 48 ms against 57): strips of 16 only, which pay to twelve rows an expert there (two chunks of
+// 600 tokens, four layers, 5.28 -> 5.00 ms).  The rows' digits have to fit the LDS.
+// Whether they are taken is for the experts' own rows to say.  An expert's second strip reads its weights again, and where every row goes to the same ten experts that is all there is
+// (300 tokens of 48 such layers: tiles 20.4 ms, strips 22.4, this choice 20.7).  Measured with ever fewer experts in use, strips of 16 are the faster ones up to 1.6 times as many as tiles (400
+// rows, 1.41 253 / 220 us, 1.57 215 / 210, 1.95 163 / 172), strips of 32 up to 1.35 (1136 rows, 1.28 397 / 368, 1.35 355 / 353, 1.53 291 / 306); the launch that finds nothing costs 5 us,
+// so the lines are 12 / 8 and 10 / 8.
+KrPfTiles kr_pf_tiles(const KrMatDev& m0, const KrMatDev& m1, long rows, int E, bool beside) {
+    if (!pf_all_fma(m0) || !pf_all_fma(m1)) return kr_pf_cut(PF_BM, 0, 0, rows, E);
     const int K = 128 * (m0.ng > m1.ng ? m0.ng : m1.ng);
-    if (rows * (long)K < 1L << 32 && rows >= 48L * E) return PFW_TM;
+    if (rows * (long)K < 1L << 32 && rows >= 48L * E) return kr_pf_cut(PFW_TM, 0, 0, rows, E);
     if (m0.bits == 4 && m1.bits == 4 && m0.N % 16 == 0 && m1.N % 16 == 0) {
-        if (rows <= 10L * E && pf_strip_lds(K, 16) <= PFS_LDS) return 16;
-        if (rows <= (E >= 256 ? 24L : 16L) * E && pf_strip_lds(K, 32) <= PFS_LDS) return 32;
+        if (rows <= (beside ? 12L : 10L) * E && pf_strip_lds(K, 16) <= PFS_LDS) return kr_pf_cut(PF_BM, 16, 12, rows, E);
+        if (!beside && rows <= (E >= 256 ? 24L : 16L) * E && pf_strip_lds(K, 32) <= PFS_LDS) return kr_pf_cut(PF_BM, 32, 10, rows, E);
     }
-    return PF_BM;
+    return kr_pf_cut(PF_BM, 0, 0, rows, E);
 }
 static bool pf_dense_wide(const KrPfGemmArgs& a) {
     int ncb = (a.m.N + PFW_TN - 1) / PFW_TN; bool all = pf_all_fma(a.m);
@@ -404,21 +426,22 @@ static bool pf_dense_wide(const KrPfGemmArgs& a) {
     return all && (long)a.total_rows * a.m.ng * 128 < 1L << 32 && (long)ncb * ((a.total_rows + PFW_TM - 1) / PFW_TM) >= 128;
 }
 void kr_launch_pf_gemm(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_hi, const int8_t* a_lo, const float* a_scale, const KrPfSort* sort, int topk,
-                       int gather_tokens, int max_tiles, int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows, int out_bf16, int var_rows, int tile_rows) {
+                       int gather_tokens, int max_tiles, int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows, int out_bf16, int var_rows, const KrPfTiles* t) {
     KrPfGemmArgs a{};
     a.scatter_rows = scatter_rows; a.out_bf16 = out_bf16;
     a.var_rows = sort != nullptr && single_expert_rows <= 0 && var_rows;
     a.m = m; a.wsum = wsum; a.a_hi = a_hi; a.a_lo = a_lo; a.a_scale = a_scale; a.topk = topk; a.gather_tokens = gather_tokens;
     if (sort) { a.row_pair = sort->row_pair; a.tile_expert = sort->tile_expert; a.tile_row0 = sort->tile_row0; a.tile_rows = sort->tile_rows; a.n_tiles = sort->n_tiles; }
     a.out = out; a.out_ld = out_ld; a.single_expert = single_expert_rows > 0; a.total_rows = single_expert_rows;
-    if (single_expert_rows > 0 ? pf_dense_wide(a) : tile_rows == PFW_TM) {
+    if (single_expert_rows > 0 ? pf_dense_wide(a) : t && t->rows == PFW_TM) {
         const int wt = single_expert_rows > 0 ? (single_expert_rows + PFW_TM - 1) / PFW_TM : max_tiles;
         if (m.bits == 8) kr_pf_wide_launch<8>(a, wt, st); else kr_pf_wide_launch<4>(a, wt, st);
         return;
     }
-    if (single_expert_rows <= 0 && tile_rows < PF_BM) {
-        if (tile_rows == 16) kr_pf_strip_launch<1, 8>(a, max_tiles, st); else kr_pf_strip_launch<2, 16>(a, max_tiles, st);
-        return;
+    if (single_expert_rows <= 0 && t && t->strip > 0) {
+        KrPfGemmArgs b = a;
+        b.n_tiles = a.n_tiles + 2;
+        if (t->strip == 16) kr_pf_strip_launch<1, 8>(b, t->max_strips, st); else kr_pf_strip_launch<2, 16>(b, t->max_strips, st);
     }
     const int mt = single_expert_rows > 0 ? (single_expert_rows + PF_BM - 1) / PF_BM : max_tiles;
     // 32 columns per wave, two quantization groups per k stage: the best of the (64|32 columns) x (1|2 groups) shapes and of a 2 x 2 row-split

@@ -700,13 +700,14 @@ static void pfh_strip_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st) {
     const int ncb = (groups + spw - 1) / spw;
     hipLaunchKernelGGL(kr_pfh_strip_kernel, dim3(((mt + 7) / 8) * 8 * ncb), dim3(64 * WAVES), lds, st, a, spw, ncb);
 }
-// Rows of a tile of the experts' table for `rows` rows on E experts: strips while an expert seldom has more than one tile of 16, 64-row tiles beyond.  With hundreds of experts the
-// stream is long enough to carry second tiles too.  A layer's experts, us, 64-row tiles -> strips: 512 of 2048 x 512, top 10: 32 rows 148 -> 104, 256 278 -> 206, 512 291 -> 241, 716 (14 an
-// expert) 294 -> 271; 64 of 2048 x 1408, top 6: 8 rows 82 -> 68, 80 113 -> 97, 107 (10) 115 -> 113, 130 (12) 115 -> 116, 149 (14) 114 -> 124.  Tiles of 32 rows gained nothing from 14 on.
-int kr_pfh_tile_rows(const KrMatDev& m0, const KrMatDev& m1, long rows, int E) {
+// How the rows on E experts are cut: strips of 16 may be taken while an expert seldom has more, to 14 rows on average with hundreds of experts, else to ten; 64-row tiles beyond.  A layer's
+// experts, us, tiles alone / this choice where it takes strips: 512 of 2048 x 512, top 10: 48 rows 187 / 136, 160 276 / 196, 400 289 / 239, 700 300 / 276; 64 of 2048 x 1408, top 6: 16 rows 89 / 82, 60 105 / 102,
+// 100 108 / 103.  The experts' own rows decide (see kr_pf_tiles): with fewer and fewer experts in use strips are the faster ones up to 1.4 times as many as tiles (520 rows, 1.28
+// 284 / 262 us, 1.39 262 / 262, 1.51 229 / 252), hence 11 / 8.  300 tokens on the same ten experts, 48 layers: tiles 13.7 ms, strips 15.4, this choice 13.7.
+KrPfTiles kr_pfh_tiles(const KrMatDev& m0, const KrMatDev& m1, long rows, int E) {
     const int K = 128 * (m0.ng > m1.ng ? m0.ng : m1.ng);
-    if (m0.bits != 4 || m1.bits != 4 || m0.qs || m1.qs || m0.N % 16 || m1.N % 16) return PFH_BM;
-    return rows <= (E >= 256 ? 14L : 10L) * E && pfh_strip_lds(K) <= 160 * 1024 ? PFH_ST_ROWS : PFH_BM;
+    const bool strips = m0.bits == 4 && m1.bits == 4 && !m0.qs && !m1.qs && m0.N % 16 == 0 && m1.N % 16 == 0 && rows <= (E >= 256 ? 14L : 10L) * E && pfh_strip_lds(K) <= 160 * 1024;
+    return kr_pf_cut(PFH_BM, strips ? PFH_ST_ROWS : 0, 11, rows, E);
 }
 
 template <int NC, int BITS, int SB = 0, int G = 0, int OCC = 2>
@@ -765,16 +766,17 @@ void kr_launch_pfh_act(const float* gu, int rows, int n, int gu_ld, int act_mode
     else hipLaunchKernelGGL(kr_pfh_act_kernel<KR_ACT_SILU_MUL>, dim3(rows), dim3(256), 0, st, gu, n, gu_ld, swiglu_limit, alpha, out, mul);
 }
 void kr_launch_pfh_gemm(const KrMatDev& m, const uint16_t* a_h, const float* a_mul, const KrPfSort* sort, int topk, int gather_tokens, int max_tiles,
-                        int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows, int out_bf16, int run, const uint16_t* a_sum32, int tile_rows) {
+                        int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows, int out_bf16, int run, const uint16_t* a_sum32, const KrPfTiles* t) {
     KrPfGemmHArgs a{};
     a.m = m; a.a = a_h; a.a_mul = a_mul; a.a_sum = a_sum32; a.topk = topk; a.gather_tokens = gather_tokens; a.scatter_rows = scatter_rows; a.out_bf16 = out_bf16;
     if (sort) { a.row_pair = sort->row_pair; a.tile_expert = sort->tile_expert; a.tile_row0 = sort->tile_row0; a.tile_rows = sort->tile_rows; a.n_tiles = sort->n_tiles; }
     a.out = out; a.out_ld = out_ld; a.single_expert = single_expert_rows > 0; a.total_rows = single_expert_rows;
     a.run = (single_expert_rows > 0 || run < 1) ? 1 : run;
     const int mt = single_expert_rows > 0 ? (single_expert_rows + PFH_BM - 1) / PFH_BM : max_tiles;
-    if (single_expert_rows <= 0 && tile_rows < PFH_BM) {
-        pfh_strip_launch(a, mt, st);
-        return;
+    if (single_expert_rows <= 0 && t && t->strip > 0) {
+        KrPfGemmHArgs b = a;
+        b.n_tiles = a.n_tiles + 2;
+        pfh_strip_launch(b, t->max_strips, st);
     }
     pfh_dispatch(a, mt, st);
 }
@@ -783,12 +785,12 @@ void kr_launch_pfh_gemm(const KrMatDev& m, const uint16_t* a_h, const float* a_m
 // only makes the f16 form.  Otherwise: the GEMM, then the activation pass over gate | up rows.  Same arithmetic either way.
 void kr_launch_pfh_w13_act(const KrMatDev& m, const uint16_t* a_h, const float* a_mul, const KrPfSort* sort, int topk, int gather_tokens, int max_tiles,
                            int single_expert_rows, float* gu, int rows, int act_mode, float swiglu_limit, float alpha, uint16_t* h_out, float* h_mul,
-                           hipStream_t st, int run, const uint16_t* a_sum32, uint16_t* h_sums32, int tile_rows) {
+                           hipStream_t st, int run, const uint16_t* a_sum32, uint16_t* h_sums32, const KrPfTiles* t) {
     const int I = m.N / 2;
     const int mt = single_expert_rows > 0 ? (single_expert_rows + PFH_BM - 1) / PFH_BM : max_tiles;
-    const bool fuse = tile_rows == PFH_BM && m.bits == 4 && I % 128 == 0 && I <= 2048 && (long)mt * (m.N / 128) >= 2048;
+    const bool fuse = !(t && t->strip > 0) && m.bits == 4 && I % 128 == 0 && I <= 2048 && (long)mt * (m.N / 128) >= 2048;
     if (!fuse) {
-        kr_launch_pfh_gemm(m, a_h, a_mul, sort, topk, gather_tokens, max_tiles, single_expert_rows, gu, 2 * I, st, 0, 0, run, a_sum32, tile_rows);
+        kr_launch_pfh_gemm(m, a_h, a_mul, sort, topk, gather_tokens, max_tiles, single_expert_rows, gu, 2 * I, st, 0, 0, run, a_sum32, t);
         kr_launch_pfh_act(gu, rows, I, 2 * I, act_mode, swiglu_limit, alpha, h_out, h_mul, st, h_sums32);
         return;
     }

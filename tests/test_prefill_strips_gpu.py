@@ -1,0 +1,104 @@
+"""Strips of few rows per expert (krasis_amd/csrc/kr_prefill_strip.inc, kr_prefill_h.hip): the sort takes them where the experts' own rows are few, not where the average is, and the exact
+ones give the bits of the decode kernels."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from tests.test_gemm_fast_gpu import _setup
+from tests.test_gemm_ring_gpu import _prefill_mode
+from tests.util import rand_bf16
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+
+
+def _cut(eng):
+    from krasis_amd._lib import check
+    n = (C.c_int(), C.c_int())
+    check(eng._lib.kr_moe_prefill_tiles(eng._h, C.byref(n[0]), C.byref(n[1])))
+    return n[0].value, n[1].value
+
+
+def _forward(eng, torch, x, ids, w):
+    from krasis_amd import _lib
+    from krasis_amd._lib import check
+    M, H = x.shape
+    xt = torch.from_numpy(x.view(np.int16)).cuda(); it = torch.from_numpy(ids).cuda(); wt = torch.from_numpy(w).cuda()
+    out = torch.empty((M, H), dtype=torch.float32, device="cuda")
+    check(eng._lib.kr_moe_forward(eng._h, 0, xt.data_ptr(), it.data_ptr(), wt.data_ptr(), out.data_ptr(), M, ids.shape[1], _lib.KR_OUT_F32, 0, 1))
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+def _one_each(counts, k, rng):
+    """ids [rows, k], one used slot a row: counts[e] rows of expert e in any order"""
+    e = rng.permutation(np.repeat(np.arange(len(counts)), counts)).astype(np.int32)
+    ids = np.full((len(e), k), -1, np.int32)
+    ids[np.arange(len(e)), rng.integers(0, k, len(e))] = e
+    return ids
+
+
+E = 64
+
+
+@pytest.mark.parametrize("counts,exact,fast", [
+    ([3] * E, "strips", "strips"),
+    ([17] * 32 + [1] * 32, "strips", "tiles"),            # 96 strips of 16 for 64 tiles: as many as the exact rule takes
+    ([17] * 33 + [1] * 31, "tiles", "tiles"),             # one more
+    ([17] * 24 + [1] * 40, "strips", "strips"),           # 88 for 64: as many as the tolerance rule takes
+    ([17] * 25 + [1] * 39, "strips", "tiles"),
+    ([300, 299] + [0] * 62, "tiles", "tiles"),            # every row on the same two experts
+    ([640] + [0] * 63, "tiles", "tiles"),
+])
+def test_the_cut_follows_the_experts_own_rows(counts, exact, fast):
+    """at most ten rows an expert on average, where strips of 16 may be taken"""
+    eng, experts, shared, rng, torch = _setup(256, 128, E, 1)
+    ids = _one_each(counts, 1, rng)
+    M = len(ids)
+    assert M <= 10 * E
+    x = rand_bf16(rng, (M, 256)); w = rng.random((M, 1)).astype(F)
+    ref = _forward(eng, torch, x, ids, w)
+    out = _prefill_mode(eng, torch, x, ids, w, 0)
+    tiles, strips = _cut(eng)
+    n = {"tiles": sum(-(-c // 64) for c in counts), "strips": sum(-(-c // 16) for c in counts)}
+    assert (tiles, strips) == ((n["tiles"], 0) if exact == "tiles" else (0, n["strips"]))
+    assert np.array_equal(out.view(np.uint32), ref.view(np.uint32))
+    tol = _prefill_mode(eng, torch, x, ids, w, 1)
+    assert _cut(eng) == ((n["tiles"], 0) if fast == "tiles" else (0, n["strips"]))
+    # rows and hidden values rounded to f16 once each, 2^-11 a value, in both products
+    assert float(np.linalg.norm((tol - ref).astype(np.float64)) / np.linalg.norm(ref.astype(np.float64))) <= 2.0 ** -10
+
+
+@pytest.mark.parametrize("per,strip", [(10, 16), (11, 32), (16, 32), (17, 64)])
+@pytest.mark.parametrize("H,I", [(640, 384), (256, 128)])             # odd group counts in both products (the last step of a strip holds one); one step a strip
+def test_exact_strips_are_the_decode_kernels_bits(H, I, per, strip):
+    """rows an expert around the rules' lines (10: strips of 16, then of 32 to 16 with few experts), among them an expert without rows and ones of 1, 15 - 17 and 31 - 33"""
+    eng, experts, shared, rng, torch = _setup(H, I, 20, 3)
+    M = per * 20 // 3
+    ids = np.argsort(rng.random((M, 20)), axis=1)[:, :3].astype(np.int32)
+    ids[ids == 4] = -1
+    ids[5, :] = -1
+    x = rand_bf16(rng, (M, H)); w = rng.random((M, 3)).astype(F)
+    out = _prefill_mode(eng, torch, x, ids, w, 0)
+    tiles, strips = _cut(eng)
+    counts = np.bincount(ids[ids >= 0], minlength=20)
+    assert (strips == sum(-(-c // strip) for c in counts) and tiles == 0) if strip < 64 else (strips == 0 and tiles > 0), (tiles, strips, sorted(counts))
+    assert np.array_equal(out.view(np.uint32), _forward(eng, torch, x, ids, w).view(np.uint32))
+
+
+@pytest.mark.parametrize("counts", [(1, 15, 16, 17, 0, 2, 9, 8, 7, 3), (31, 32, 33, 1, 15, 16, 17, 0, 5, 10)])
+def test_exact_strips_of_whole_and_ragged_tiles(counts):
+    eng, experts, shared, rng, torch = _setup(384, 256, 10, 1)
+    ids = _one_each(counts, 1, rng)
+    x = rand_bf16(rng, (len(ids), 384)); w = rng.random((len(ids), 1)).astype(F)
+    out = _prefill_mode(eng, torch, x, ids, w, 0)
+    assert _cut(eng)[1] > 0
+    assert np.array_equal(out.view(np.uint32), _forward(eng, torch, x, ids, w).view(np.uint32))
+
+
+@pytest.mark.parametrize("Ms,ret_bf16", [([20, 12], False), ([20, 12], True), ([3, 0], False)])
+def test_scattered_rows_of_expert_parallel_ranks(Ms, ret_bf16):
+    """nine rows a local expert, each row stored at the place that it came from, in f32 and in bf16"""
+    import tests.test_ep_gpu as ep
+    ep.test_library_expert_parallel_loopback_equals_single_engine(2, Ms, ret_bf16, False)

@@ -19,11 +19,14 @@
 namespace {
 // Eight waves of at most 128 registers (the lean form of attention), two workgroups to a compute unit, for what streams the experts beside it.
 constexpr int AU_WAVES = 8;
-// Up to this many problem rows (one to four tokens) each is taken alone, a wave per gate column and its up column: whole matrix rows per request and no wait for the group's
+// Up to this many problem rows each is taken alone, a wave per gate column and its up column: whole matrix rows per request and no wait for the group's
 // bounds.  Against strips of 16 + 16 columns: six rows of 1536 x 2048 14.8 -> 11.4 us, 24 rows of 3072 x 4096 on 128 experts 112 -> 97.
+// With more rows than experts an expert's matrix is read once per row, which costs nothing while all of them stay in the 256 MB cache (a step of two layers, us, rows alone /
+// strips: 18 rows on 16 experts of 2 x 768 x 2048 254 / 264, 24 on 8 283 / 281) and much beyond it (8 experts of 2 x 4096 x 4096, 537 MB: 12 rows 561 / 497, 24 rows 865 / 632): hence half of it.
 constexpr int AU_ROWS = 24;
+bool au_rows_alone(const KrSvGemm& up) { return up.M <= AU_ROWS && (up.M <= up.n_groups || (size_t)up.n_groups * up.w_stride * 2 <= (size_t)128 << 20); }
 template <int DIM, int VDIM>
-__global__ void __launch_bounds__(64 * AU_WAVES, 4) sv_attn_up_kernel(const KrSvAttn a, const KrSvGemm up, const int n_attn, const int strips) {
+__global__ void __launch_bounds__(64 * AU_WAVES, 4) sv_attn_up_kernel(const KrSvAttn a, const KrSvGemm up, const int n_attn, const int strips, const int alone) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     // (quotients are formed on the vector unit; without readfirstlane all that follows from them would stay there)
     if ((int)blockIdx.x < n_attn) {
@@ -31,7 +34,7 @@ __global__ void __launch_bounds__(64 * AU_WAVES, 4) sv_attn_up_kernel(const KrSv
         as_token<DIM, VDIM, AU_WAVES, true>(a, blockIdx.x - th * a.T, th - bz * a.kv_heads, bz, lds);
     } else {
         const int i = blockIdx.x - n_attn, by = __builtin_amdgcn_readfirstlane(i / strips);
-        if (up.M <= AU_ROWS) sk_row_glu<AU_WAVES>(up, i - by * strips, by);
+        if (alone) sk_row_glu<AU_WAVES>(up, i - by * strips, by);
         else sk_strip<1, 2, AU_WAVES, false, true>(up, i - by * strips, by, lds, nullptr);
     }
 }
@@ -50,9 +53,9 @@ __global__ void __launch_bounds__(256) sv_downs_kernel(const KrSvGemm o, const K
 
 template <int DIM, int VDIM> void au_launch(const KrSvAttn& a, const KrSvGemm& up, hipStream_t st) {
     const int R = a.heads / a.kv_heads, lds = std::max({as_lds_bytes(R, VDIM, AU_WAVES), as_lean_lds_bytes(DIM), sk_red_floats(1, 2, AU_WAVES) * (int)sizeof(float)});
-    const int n_attn = a.T * a.kv_heads * ((R + 15) / 16) * a.nsplit, cols = up.M <= AU_ROWS ? AU_WAVES : 16, strips = (up.glu_f + cols - 1) / cols;
+    const int n_attn = a.T * a.kv_heads * ((R + 15) / 16) * a.nsplit, alone = au_rows_alone(up), cols = alone ? AU_WAVES : 16, strips = (up.glu_f + cols - 1) / cols;
     if (kr_lds_optin((const void*)sv_attn_up_kernel<DIM, VDIM>, lds)) return;        // (the step ends with the runtime's error)
-    hipLaunchKernelGGL((sv_attn_up_kernel<DIM, VDIM>), dim3(n_attn + strips * up.M), dim3(64 * AU_WAVES), lds, st, a, up, n_attn, strips);
+    hipLaunchKernelGGL((sv_attn_up_kernel<DIM, VDIM>), dim3(n_attn + strips * up.M), dim3(64 * AU_WAVES), lds, st, a, up, n_attn, strips, alone);
 }
 }  // namespace
 

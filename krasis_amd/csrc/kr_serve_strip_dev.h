@@ -126,8 +126,8 @@ __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const 
     }
 }
 
-// The gate and up product of problem row `by` alone, columns [WV bx, WV bx + WV) of g.glu_f, one per wave, K over its lanes: for the rows of one or
-// two tokens, which meet an expert once.  A wave reads whole rows of the matrix and waits for nothing but its row's expert.
+// The gate and up product of problem row `by` alone, columns [WV bx, WV bx + WV) of g.glu_f, one per wave, K over its lanes: for few rows, which seldom meet
+// an expert twice.  A wave reads whole rows of the matrix and waits for nothing but its row's expert.
 template <int WV>
 __device__ __forceinline__ void sk_row_glu(const KrSvGemm& g, const int bx, const int by) {
     constexpr int U = 4;                                      // 16-byte pieces of K requested together, of both matrices

@@ -32,6 +32,22 @@ def test_steps_close_to_oracle(name, mixer, mlp, requests, length, steps):
     assert np.median(e) < 2e-2 and (e < 4e-2).mean() >= 0.9, (name, e)
 
 
+@pytest.mark.parametrize("ff", [1024, 4096])
+def test_more_rows_than_experts(ff):
+    """each row alone while the experts' matrices stay in the cache, strips beyond (five experts of 2 x 4096 x 2048 are 168 MB); against the f32 store, which other tests hold to the
+    float64 restatement"""
+    cfg = O.make_config(width=2048, vocab=50, eps=1e-5, layers=[{"type": "attention", "mixer": O.attn(4, 2, 64, 64, 0, 0, scale=0.12), "mlp": O.moe(5, 2, 1, 1, ff, 1.5)}])
+    W = O.random_weights(cfg, 15)
+    seqs = [tokens(cfg, 8, 60 + r) for r in range(6)]
+    got = []
+    for dtype in ("float32", "bfloat16"):
+        eng = engine(cfg, W, dtype, max_slots=6)
+        eng.step([(r, s[:5], []) for r, s in enumerate(seqs)])
+        got.append(np.stack([eng.step([(r, [s[5 + i]], [0]) for r, s in enumerate(seqs)])[0] for i in range(3)], 1).astype(np.float64))
+    e = np.sqrt(((got[1] - got[0]) ** 2).mean(-1)) / np.sqrt((got[0] ** 2).mean())
+    assert np.median(e) < 2e-2 and (e < 4e-2).mean() >= 0.9, e
+
+
 def test_a_step_is_the_same_every_time_and_under_replay():
     """joined launches leave the same bits eagerly and from a replayed graph, whatever ran in between"""
     cfg = O.make_config(width=128, vocab=70, eps=1e-5, layers=[{"type": "attention", "mixer": O.attn(8, 2, 128, 128, 0, 64, scale=0.1), "mlp": O.moe(8, 3, 1, 1, 96, 1.5, 64, 2.0)}] * 2)

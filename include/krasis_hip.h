@@ -583,7 +583,7 @@ int kr_serve_set_profiling(kr_serve* s, int enable);
 int kr_serve_get_profile(kr_serve* s, double* ms_by_family, int n);
 
 /* ---- measurement hooks (bench.py): HIP events around each kernel launch on the launch stream ----
- * kinds: 0 kr_moe_w13_kernel, 1 kr_moe_w2_kernel, 2 kr_moe_combine_kernel.  Enabling profiling serialises calls. */
+ * kinds: 0 gate and up products, 1 down projections, 2 weighted sums (none where a call of one row forms its sum in the down projection).  Enabling profiling serialises calls. */
 int kr_set_profiling(kr_engine* e, int enable);
 int kr_get_profile(kr_engine* e, int kind, double* total_ms, long* launches);
 

@@ -560,11 +560,11 @@ static int moe_forward_locked(kr_engine* e, int layer, const void* act, const in
     } else {
         for (int i = 0; i < 4; i++) if (!e->pev[i]) KR_HIP(hipEventCreate(&e->pev[i]));
         KR_HIP(hipEventRecord(e->pev[0], st)); kr_launch_moe_w13(a, st);
-        KR_HIP(hipEventRecord(e->pev[1], st)); kr_launch_moe_w2(a, st);
-        KR_HIP(hipEventRecord(e->pev[2], st)); kr_launch_moe_combine(a, st);
+        KR_HIP(hipEventRecord(e->pev[1], st)); const bool summed = kr_launch_moe_down(a, st);
+        KR_HIP(hipEventRecord(e->pev[2], st)); if (!summed) kr_launch_moe_combine(a, st);
         KR_HIP(hipEventRecord(e->pev[3], st));
         KR_HIP(hipEventSynchronize(e->pev[3]));
-        for (int i = 0; i < 3; i++) { float ms = 0; KR_HIP(hipEventElapsedTime(&ms, e->pev[i], e->pev[i + 1])); e->prof_ms[i] += ms; e->prof_n[i]++; }
+        for (int i = 0; i < (summed ? 2 : 3); i++) { float ms = 0; KR_HIP(hipEventElapsedTime(&ms, e->pev[i], e->pev[i + 1])); e->prof_ms[i] += ms; e->prof_n[i]++; }
     }
     KR_HIP(hipGetLastError());
     if (!out_dev) {
@@ -802,7 +802,7 @@ extern "C" int kr_forward_moe_routed(kr_engine* e, int layer, const void* act_bf
 }
 
 // ---- profiling hooks used by bench.py (HIP events on the launch stream, per kernel kind) ----
-// kinds: 0 = kr_moe_w13_kernel, 1 = kr_moe_w2_kernel, 2 = kr_moe_combine_kernel
+// kinds: 0 = gate and up products, 1 = down projections, 2 = weighted sums
 extern "C" int kr_set_profiling(kr_engine* e, int enable) {
     if (!e) return kr_fail(KR_ERR_VALUE, "null engine");
     e->prof = enable != 0;

@@ -73,6 +73,7 @@ struct KrMoeArgs {
 struct KrMultiMat { KrMatDev m[KR_MAX_MULTI]; float* y[KR_MAX_MULTI]; int tile_end[KR_MAX_MULTI]; int n; };
 
 void kr_launch_moe_decode(const KrMoeArgs& a, hipStream_t st);
+bool kr_launch_moe_down(const KrMoeArgs& a, hipStream_t st);      // the down projection; true: with the weighted sum (one row), else kr_launch_moe_combine follows
 void kr_launch_moe_w13(const KrMoeArgs& a, hipStream_t st);
 void kr_launch_moe_w2(const KrMoeArgs& a, hipStream_t st);
 void kr_launch_moe_combine(const KrMoeArgs& a, hipStream_t st);

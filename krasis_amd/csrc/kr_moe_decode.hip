@@ -683,18 +683,21 @@ void kr_launch_moe_combine(const KrMoeArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(kr_moe_combine_kernel, grid, dim3(KR_BLOCK), 0, st, a);
 }
 
-void kr_launch_moe_decode(const KrMoeArgs& a, hipStream_t st) {
-    kr_launch_moe_w13(a, st);
+bool kr_launch_moe_down(const KrMoeArgs& a, hipStream_t st) {
     // One row: the down projection forms the row's sum as in the decode step, two dependent launches instead of three (512 experts of 2048 x 512, top 10, INT4: 18.1 -> 15.1 us;
     // 64 of 2048 x 1408 with shared ones 27.0 -> 24.8).  From two rows on its workgroups, which each quantize the row's hidden values again, cost more than the launch saved
     // (20.7 us against 19.7 and 31.9 against 33.1 at two, 40 / 52 and 67 / 92 at eight).
     if (a.B == 1) {
         KrMoeArgs c = a;
         if (a.n_slots == a.topk) c.rsf = 1.0f;      // this operator scales the routed sum only together with a shared expert
-        if (kr_launch_moe_w2c(c, nullptr, (float*)a.out, st) == 0) return;
+        if (kr_launch_moe_w2c(c, nullptr, (float*)a.out, st) == 0) return true;
     }
     kr_launch_moe_w2(a, st);
-    kr_launch_moe_combine(a, st);
+    return false;
+}
+void kr_launch_moe_decode(const KrMoeArgs& a, hipStream_t st) {
+    kr_launch_moe_w13(a, st);
+    if (!kr_launch_moe_down(a, st)) kr_launch_moe_combine(a, st);
 }
 
 // exact decode step, linear-attention layers: in_proj_qkvz | in_proj_ba from the INT16 image with the conv / gate epilogue (kr_matvec_coop_kernel<.., LA = true>);

@@ -578,7 +578,8 @@ int kr_serve_set_capture(kr_serve* s, int enable);
 int kr_serve_read_capture(kr_serve* s, float* out_host, size_t n_floats);
 size_t kr_serve_device_bytes(const kr_serve* s);
 /* measurement hook: HIP-event time of every kernel family over the steps since the last reset (ms), families: 0 norm 1 gemm 2 qk_prep 3 attention 4 router+sort
- * 5 activation 6 residual 7 embed / head rows / argmax.  Recurrent scans and the short convolutions count as 3 and 2 */
+ * 5 activation 6 residual 7 embed / head rows / argmax.  Recurrent scans and the short convolutions count as 3 and 2; in decode steps that join launches, attention beside the
+ * experts' gate and up product counts as 1 (the merge of its shares as 3), query / key preparation beside the router as 4 */
 int kr_serve_set_profiling(kr_serve* s, int enable);
 int kr_serve_get_profile(kr_serve* s, double* ms_by_family, int n);
 

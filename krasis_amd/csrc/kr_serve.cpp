@@ -1531,7 +1531,8 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
             g.a_rows = src_row; g.seg = seg; g.row_group = row_group; g.n_groups = E;
             if (join[li]) {
                 g.glu_out = s->y.p; g.glu_f = F; g.glu_kind = d.expert_act; g.glu_limit = d.expert_limit; g.glu_alpha = d.expert_alpha; g.glu_row_w = row_w;
-                { Timer tm(s, 3); kr_sv_attn_up(a, g, st); if (a.nsplit > 1) kr_sv_attn_merge(a, st); }
+                { Timer tm(s, 1); kr_sv_attn_up(a, g, st); }      // (the product is the longer part, see kr_sv_step_join_splits)
+                if (a.nsplit > 1) { Timer tm(s, 3); kr_sv_attn_merge(a, st); }
                 down_ready(dn, nullptr, 0, P, F, d.expert_act, d.expert_limit, d.expert_alpha, row_w, true);
                 KrSvGemm sh{};
                 if (beside) { down_ready(ffd, hz + l.off_gu, l.n_h, T, ff_f, ff_act, ff_limit, ff_alpha); shared = (const float*)s->ffout.p; }

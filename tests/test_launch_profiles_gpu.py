@@ -29,3 +29,22 @@ def test_expert_operator(M, sums):
     check(eng._lib.kr_set_profiling(eng._h, 0))
     assert seen == [3, 3, sums]
     assert all(np.array_equal(t, plain) for t in timed)
+
+
+def test_joined_decode_step():
+    """attention beside the experts' gate and up product counts as the product; the merge of its shares, once there are several, as attention"""
+    from tests import oracle_serve as O
+    from tests.test_serve_gpu import engine, tokens
+    cfg = O.make_config(width=128, vocab=70, eps=1e-5, layers=[{"type": "attention", "mixer": O.attn(8, 2, 64, 64, 0, 64, scale=0.1), "mlp": O.moe(8, 3, 1, 1, 96, 1.5, 64, 2.0)}])
+    W = O.random_weights(cfg, 31)
+    eng = engine(cfg, W, "bfloat16")
+    a = tokens(cfg, 620, 32)
+    eng.step([("a", a[:100], [])])
+    seen = []
+    for i, n in ((100, 101), (101, 600), (600, 601)):
+        eng.store.set_profiling(n - i == 1)
+        eng.step([("a", a[i:n], [0])])
+        seen.append(eng.store.profile())
+    eng.store.set_profiling(False)
+    assert seen[0][1] > 0 and seen[0][3] == 0 and seen[0][4] > 0
+    assert seen[2][1] > 0 and seen[2][3] > 0 and seen[2][4] > 0

@@ -1136,7 +1136,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         plan[li] = kr_sv_attn_form(n_entries, counts, last_pos.data(), d.heads, l.att_heads_kv(), l.att_dim(), l.att_vdim(), ldk, ldv, ldq, PT, s->f32, d.window, d.keep_first, d.chunk);
         // decode steps of a parallel block with experts: the branches share launches (kr_serve_step.hip)
         if (!s->f32 && !seq && plan[li].form == KR_SV_ATTN_STEP && !l.latent() && !l.has_side() && d.mlp_kind == KR_SERVE_MLP_MOE && d.expert_act != KR_SERVE_ACT_RELU2 &&
-            kr_sv_step_join_fits(T, W, l.o_cols(), d.experts, d.top, d.groups, d.expert_ff, d.dim)) {
+            kr_sv_step_join_fits(T, W, l.o_cols(), d.experts, d.top, d.groups, d.expert_ff)) {
             join[li] = 1;
             plan[li].nsplit = kr_sv_step_join_splits(T, d.heads, d.kv_heads, plan[li].keys, W, d.expert_ff, d.experts, d.top);
         }
@@ -1520,10 +1520,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
             ro.ids = (int*)s->ids.p; ro.wts = (float*)s->wts.p; ro.seg = seg; ro.src_row = src_row; ro.row_group = row_group; ro.pair_pos = pp; ro.row_w = row_w;
             {
                 Timer tm(s, 4);
-                if (!join[li] || !kr_sv_prep_route(a, ro, s->f32, st)) {
-                    kr_sv_router_sort(ro, hist, st);
-                    if (join[li]) kr_sv_qk_prep(a, s->f32, st);
-                }
+                if (join[li]) kr_sv_prep_route(a, ro, st); else kr_sv_router_sort(ro, hist, st);
             }
             KrSvGemm dn{}; dn.W = l.edown.p; dn.w_stride = (size_t)W * F; dn.C = (float*)s->rows.p; dn.ldc = W; dn.M = P; dn.N = W; dn.K = F;
             dn.seg = seg; dn.row_group = row_group; dn.n_groups = E;
@@ -1596,7 +1593,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         // the key: everything a launch argument depends on -- batch, wanted rows, the split of every layer, the scratch addresses
         uint64_t key = 1469598103934665603ull;
         auto mixin = [&](uint64_t v) { key = (key ^ v) * 1099511628211ull; };
-        mixin((uint64_t)T); mixin((uint64_t)n_want); mixin(want_amax); mixin(host_logits); mixin((uint64_t)(uintptr_t)dev_hm); mixin((uint64_t)(uintptr_t)dev_out);
+        mixin((uint64_t)T); mixin((uint64_t)n_want); mixin(want_amax); mixin(host_logits); mixin((uint64_t)(uintptr_t)dev_out);
         for (const KrSvAttnPlan& p : plan) mixin((uint64_t)p.nsplit);
         for (const DevBuf* b : {&s->meta, &s->x, &s->h, &s->qkv, &s->att, &s->mix, &s->gu, &s->y, &s->rows, &s->ffout, &s->ids, &s->wts, &s->moe_i, &s->hw, &s->logits,
                                 &s->amax, &s->part_ml, &s->part_acc, &s->v_first, &s->lq_c, &s->lq_2, &s->lq_n, &s->lq_e, &s->att2, &s->head_i, &s->h32, &s->hc, &s->rg, &s->qk_rms, &s->lin_o, &s->qkv2, &s->sconv, &s->ga1, &s->gz, &s->rg_ab, &s->rg_agg, &s->rg_start,

@@ -51,7 +51,7 @@ bool kr_sv_gemm_takes_host(const KrSvGemm& g, bool f32);
 bool kr_sv_gemm_pair(const KrSvGemm& e, const KrSvGemm& o, bool f32, hipStream_t st);
 // the forms for a bf16 store that kr_sv_gemm chooses from; _fits: shapes and alignment
 bool kr_sv_gemm_skinny_fits(const KrSvGemm& g);
-// decode sizes, bf16: up to three products (M = 0: none) of at most sixteen rows in one launch; the last one may be gate | up pairs alone (its glu fields set, columns outside the pairs untouched)
+// decode sizes, bf16: up to three products (M = 0: none) of at most sixteen rows in one launch; the last one is gate | up pairs alone (its glu fields set, columns outside the pairs untouched)
 bool kr_sv_strips_fits(const KrSvGemm& g);
 void kr_sv_strips(const KrSvGemm& a, const KrSvGemm& b, const KrSvGemm& c, hipStream_t st);
 bool kr_sv_gemm_skinny_acts(const KrSvGemm& g);
@@ -193,11 +193,11 @@ struct KrSvRoute {
     int* seg; int* src_row; int* row_group; int* pair_pos; float* row_w;
 };
 void kr_sv_router_sort(const KrSvRoute& r, int* hist, hipStream_t st);
-// kr_sv_qk_prep and kr_sv_router_sort of a block whose attention and router read one product, in one launch (at most 16 tokens); false: nothing was launched
-bool kr_sv_prep_route(const KrSvAttn& a, const KrSvRoute& r, bool f32, hipStream_t st);
+// kr_sv_qk_prep and kr_sv_router_sort of a block whose attention and router read one product, in one launch (bf16, sizes of kr_sv_step_join_fits)
+void kr_sv_prep_route(const KrSvAttn& a, const KrSvRoute& r, hipStream_t st);
 // Decode steps of a parallel block with experts, bf16 (kr_serve_step.hip): attention beside the experts' gate and up product (up: glu fields set, columns [0, 2 glu_f)), then
 // attention's output projection, the experts' down projection (of up.glu_out) and the shared expert's in one launch.  join_fits: shapes; join_splits: attention's key splits there.
-bool kr_sv_step_join_fits(int T, int width, int o_cols, int experts, int top, int groups, int ff, int dim);
+bool kr_sv_step_join_fits(int T, int width, int o_cols, int experts, int top, int groups, int ff);
 int kr_sv_step_join_splits(int T, int heads, int kv_heads, int max_visible, int width, int ff, int experts, int top);
 void kr_sv_attn_up(const KrSvAttn& a, const KrSvGemm& up, hipStream_t st);
 void kr_sv_downs(const KrSvGemm& o, const KrSvGemm& e, const KrSvGemm& sh, hipStream_t st);

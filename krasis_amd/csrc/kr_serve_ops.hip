@@ -1143,12 +1143,12 @@ __global__ void __launch_bounds__(SORT ? 1024 : 256) sv_router_rank_kernel(const
 
 // A parallel block's router reads the same product as its queries and keys: at decode sizes one launch does both, workgroup 0 the choice and the sort, the others sixteen
 // (token, head) rows each.  A launch that depends on the one before it costs 4 - 5 us here whatever it does: one request 4.7 + 4.7 us as two launches, now 5.2.
-template <typename T, int NV>
+template <int NV>
 __global__ void __launch_bounds__(1024) sv_prep_route_kernel(const KrSvAttn a, const KrSvRoute ro, int heads_per_token) {
     extern __shared__ float hv16[];          // [16][dim]
     if (blockIdx.x == 0) { sv_router_rank<NV, true>(ro, 0); return; }
     const int wave = threadIdx.x >> 6, i = (blockIdx.x - 1) * 16 + wave;
-    if (i < a.T * heads_per_token) sv_qk_prep_row<T>(a, i / heads_per_token, i % heads_per_token, threadIdx.x & 63, hv16 + wave * a.dim);
+    if (i < a.T * heads_per_token) sv_qk_prep_row<uint16_t>(a, i / heads_per_token, i % heads_per_token, threadIdx.x & 63, hv16 + wave * a.dim);
 }
 
 // Rows of a prompt's pairs sorted by expert, without atomics on a few hot words of memory (64 counters for 24576 pairs: 39 us to count and 39 us to place): a block counts its
@@ -2622,16 +2622,12 @@ void kr_sv_router_sort(const KrSvRoute& r, int* hist, hipStream_t st) {
     hipLaunchKernelGGL(sv_moe_fill_kernel, dim3(blocks), dim3(256), (size_t)E * sizeof(int), st, ids, n, top, E, hist, src_row, row_group, pair_pos, wts, row_w);
 }
 
-bool kr_sv_prep_route(const KrSvAttn& a, const KrSvRoute& r, bool f32, hipStream_t st) {
+void kr_sv_prep_route(const KrSvAttn& a, const KrSvRoute& r, hipStream_t st) {
     const int hpt = a.heads + (a.own_kv ? (a.v_from_k ? 1 : 2) * a.kv_heads : 0);
     const size_t lds = (size_t)16 * a.dim * sizeof(float);
-    if (a.T != r.T || a.T <= 0 || a.T > 16 || r.top <= 0 || !sv_route_ranked(r) || lds > 32 * 1024) return false;
     const dim3 grid(1 + (a.T * hpt + 15) / 16), nt(1024);
-#define SV_PR(T_, NV_) hipLaunchKernelGGL((sv_prep_route_kernel<T_, NV_>), grid, nt, lds, st, a, r, hpt)
-    if (r.E <= 64) { if (f32) SV_PR(float, 1); else SV_PR(uint16_t, 1); }
-    else { if (f32) SV_PR(float, 2); else SV_PR(uint16_t, 2); }
-#undef SV_PR
-    return true;
+    if (r.E <= 64) hipLaunchKernelGGL(sv_prep_route_kernel<1>, grid, nt, lds, st, a, r, hpt);
+    else hipLaunchKernelGGL(sv_prep_route_kernel<2>, grid, nt, lds, st, a, r, hpt);
 }
 
 void kr_sv_act(const float* gu, int ld, void* y, bool f32, int M, int F, int kind, float limit, float alpha, const float* row_w, hipStream_t st, const void* up_tab,

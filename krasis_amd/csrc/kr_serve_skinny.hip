@@ -29,7 +29,7 @@ __global__ void __launch_bounds__(256) sv_skinny_pair_kernel(const KrSvGemm e, c
     if (blockIdx.y == 0) sk_strip<1, 1, 4, true>(o, blockIdx.x, 0, red, act); else sk_strip<1, 1, 4, true>(e, blockIdx.x, blockIdx.y - 1, red, act);
 }
 
-// Up to three products of the same rows in one launch, the last one optionally the gate | up pairs of a feed-forward that leave as their activation.  A launch with its gap
+// Up to three products of the same rows in one launch, the last one the gate | up pairs of a feed-forward that leave as their activation.  A launch with its gap
 // costs what 25 MB of weights cost, and the activation formed in the down projection is formed again by every one of its workgroups.  Two rows, width 2048, feed-forward 6144:
 // gate | up and the residual gate behind them, 14336 columns, 13.8 -> 13.9 us, the down projection that no longer forms the activation 15.4 -> 11.4; mixer projections and
 // residual gate 2048 x 2048 13.8 + 5.4 -> 13.9 us.
@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(256) sv_strips_kernel(const KrSvGemm a, const 
     i -= na;
     if (i < nb) { sk_strip<1, 1, 4, false>(b, i, 0, red, nullptr); return; }
     i -= nb;
-    if (c.glu_out) sk_strip<1, 2, 4, false, true>(c, i, 0, red, nullptr); else sk_strip<1, 1, 4, false>(c, i, 0, red, nullptr);
+    sk_strip<1, 2, 4, false, true>(c, i, 0, red, nullptr);
 }
 
 int sk_act_lds(const KrSvGemm& g) { return (g.row_group ? 16 : std::min(16, g.M)) * (g.K + 8) * 2; }      // one block of sixteen rows
@@ -91,6 +91,6 @@ bool kr_sv_strips_fits(const KrSvGemm& g) { return g.M > 0 && g.M <= 16 && !g.se
 void kr_sv_strips(const KrSvGemm& a, const KrSvGemm& b, const KrSvGemm& c, hipStream_t st) {
     KrSvGemm p[3] = {a, b, c};
     int n[3];
-    for (int i = 0; i < 3; i++) { p[i].row_group = nullptr; n[i] = p[i].M <= 0 ? 0 : ((p[i].glu_out ? p[i].glu_f : p[i].N) + 15) / 16; }
+    for (int i = 0; i < 3; i++) { p[i].row_group = nullptr; n[i] = p[i].M <= 0 ? 0 : ((i == 2 ? p[i].glu_f : p[i].N) + 15) / 16; }
     if (n[0] + n[1] + n[2] > 0) hipLaunchKernelGGL(sv_strips_kernel, dim3(n[0] + n[1] + n[2]), dim3(256), 0, st, p[0], p[1], p[2], n[0], n[1]);
 }

@@ -59,10 +59,10 @@ template <int DIM, int VDIM> void au_launch(const KrSvAttn& a, const KrSvGemm& u
 }
 }  // namespace
 
-// shapes: whole fragments for every product, a choice that kr_sv_prep_route makes, and experts with few enough rows that a strip per expert reads its weights about once
+// shapes: whole fragments for every product, a choice that one workgroup of kr_sv_prep_route makes, and experts with few enough rows that a strip per expert reads its weights about once
 // (the rule of the strips alone, kr_serve_gemm.hip)
-bool kr_sv_step_join_fits(int T, int width, int o_cols, int experts, int top, int groups, int ff, int dim) {
-    return T <= 16 && width % 32 == 0 && o_cols % 32 == 0 && ff % 32 == 0 && experts <= 128 && top <= 64 && groups <= 64 && dim <= 512 && T * top <= 8 * experts;
+bool kr_sv_step_join_fits(int T, int width, int o_cols, int experts, int top, int groups, int ff) {
+    return T <= 16 && width % 32 == 0 && o_cols % 32 == 0 && ff % 32 == 0 && experts <= 128 && top <= 64 && groups <= 64 && T * top <= 8 * experts;
 }
 
 // Beside the experts' product attention only has to be no longer than that: a workgroup takes 256 keys in 1.5 us past its first few us, the product min(T top, experts)

@@ -39,7 +39,7 @@ def test_rows_and_largest_entries(vocab, dtype, tol):
 
 
 def test_equal_nan_and_infinite_entries():
-    """the lowest index of equal entries (zeros of either sign), a NaN never, minus infinity only where nothing else is"""
+    """the lowest index of equal entries (zeros of either sign), a NaN never"""
     cfg, W = model(2000, 24)
     h = np.zeros_like(W["head"])
     for fill, at, want in ((0.0, {}, 0), (-0.0, {7: 0.0}, 0), (0.0, {3: np.nan}, 0), (np.nan, {}, 0), (np.nan, {1500: 0.0}, 1500)):
@@ -50,3 +50,30 @@ def test_equal_nan_and_infinite_entries():
         logits, amax = eng.step([("a", [1], [0])])
         assert amax[0] == want and np.isnan(logits[0]).sum() == np.isnan(h[:, 0]).sum()
     assert engine(cfg, W).step([("a", [1], [0])])[1][0] == O.forward(cfg, W, [1])[0][0].argmax()
+
+
+# head entries by index, the others at `fill`, and the entry that wins; a step's search is two workgroups' of a thousand entries each here
+INF = float("inf")
+INFINITE = [(-INF, {}, 0), (-INF, {1500: -2.0}, 1500), (-INF, {3: -2.0, 1999: -3.0}, 3), (np.nan, {1999: -INF}, 1999), (np.nan, {700: -INF, 1700: -INF}, 700),
+            (0.5, {1200: INF, 1700: INF}, 1200), (np.nan, {5: INF, 1400: 1.0}, 5), (-1.0, {999: -INF, 1000: INF, 1001: np.nan}, 1000)]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_infinite_entries_of_several_rows(dtype):
+    """minus infinity wins only where nothing but it and NaN is, plus infinity against everything; three rows a step, in the f32 store and from the bf16 store's strips"""
+    cfg, W = model(2000, 25)
+    h = np.zeros_like(W["head"])
+    h[:64, :64] = np.eye(64)
+    step = lambda head: engine(cfg, {**W, "head": head}, dtype).step([(r, [5 + r], [0]) for r in range(3)])
+    hidden = step(h)[0][:, :64]                                # the rows that the head multiplies
+    col = int(np.argmax(hidden.min(0)))
+    assert hidden[:, col].min() > 0.05                         # one column that is positive in all three: a row of logits is that column of the head, scaled
+    for fill, at, want in INFINITE:
+        h = np.zeros_like(W["head"])
+        h[:, col] = fill
+        for i, v in at.items():
+            h[i, col] = v
+        logits, amax = step(h)
+        assert (amax == want).all(), (fill, at, amax)
+        ref = hidden[:, col:col + 1].astype(np.float64) * h[:, col].astype(np.float64)
+        assert np.array_equal(np.isnan(logits), np.isnan(ref)) and np.array_equal(np.isinf(logits), np.isinf(ref)) and np.array_equal(np.sign(logits[np.isinf(logits)]), np.sign(ref[np.isinf(ref)]))

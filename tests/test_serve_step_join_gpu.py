@@ -61,3 +61,41 @@ def test_a_step_is_the_same_every_time_and_under_replay():
         runs.append([eng.step([("a", [a[240 + i]], [0]), ("b", [b[9 + i]], [0])])[0] for i in range(40)])       # past 256 keys: another share count on the way
         assert (eng.store.graph_replays() > 0) == graph
     assert all(np.array_equal(x, y) for x, y in zip(*runs))
+
+
+# what a joined layer may have beside the plain design; the second layer of two, where it refers to the first
+OPTIONS = {
+    "gate_per_head": dict(out_gate="OGATE_HEAD_SIGMOID"), "gate_per_element": dict(out_gate="OGATE_ELEM_SIGMOID"), "values_mixed": dict(v_mix="VMIX_BLEND"),
+    "convolution": dict(proj_conv=3), "norm_of_whole_rows": dict(qk_unit_norm="QKNORM_WHOLE"), "norm_with_weight": dict(qk_unit_norm="QKNORM_WEIGHTED"), "soft_cap": dict(softcap=1.5),
+    "distance": dict(dist_bias=1), "kept_keys": dict(window=12, keep_first=3), "kept_keys_past_a_tile": dict(window=5, keep_first=33), "chunk": dict(chunk=16), "sink": dict(has_sink="SINK_ZERO"),
+    "weights_on_inputs": dict(expert_in_weight=1), "keys_of_another_layer": dict(kv_from=0), "values_are_keys": dict(v_from_k=1), "biases": dict(proj_bias=2),
+}
+
+
+@pytest.mark.parametrize("name", OPTIONS)
+def test_every_mechanism_of_a_joined_layer(name):
+    """tokens one by one, each step joined, against the same tokens as one prompt, whose launches are not; the prompt's own distance to 64 bits is other tests' matter.  Tolerance: as above"""
+    from krasis_amd import serve_store as S
+    o = {k: getattr(S, v) if isinstance(v, str) else v for k, v in OPTIONS[name].items()}
+    base = dict(heads=4, kv_heads=2, dim=32, vdim=32, rot_dims=16, scale=0.18, mlp_kind=S.MLP_MOE, experts=6, top=2, expert_ff=64, expert_act=S.ACT_SILU, shared_ff=32)
+    first = {**base, **({"v_mix": S.VMIX_FIRST} if "v_mix" in o else {} if "kv_from" in o else o)}
+    store = S.ServeStore(80, 64, [S.LayerSpec(**first), S.LayerSpec(**{**base, **o})], max_slots=4, pool_tokens=1024)
+    store.fill_synthetic(seed=41, amp=2.5)
+    store.finalize()
+    rng = np.random.default_rng(42)
+    seqs = [rng.integers(0, 80, n) for n in (70, 61, 50)]
+    ref, slots = [], [store.admit() for _ in seqs]
+    for sl, s in zip(slots, seqs):
+        ref.append(store.step([(sl, s)], range(len(s) - 20, len(s)))[0])
+        store.release(sl)
+    slots = [store.admit() for _ in seqs]
+    for sl, s in zip(slots, seqs):
+        store.step([(sl, s[:-20])], [])
+    got = np.stack([store.step([(sl, [s[len(s) - 20 + i]]) for sl, s in zip(slots, seqs)], range(3))[0] for i in range(19)], 1).astype(np.float64)
+    store.set_profiling(True)
+    last = store.step([(sl, [s[-1]]) for sl, s in zip(slots, seqs)], range(3))[0]
+    assert store.profile()[3] == 0                              # attention had no launch of its own
+    store.set_profiling(False)
+    got, ref = np.concatenate([got, last[:, None]], 1), np.stack(ref).astype(np.float64)
+    e = np.sqrt(((got - ref) ** 2).mean(-1)) / np.sqrt((ref ** 2).mean())
+    assert np.median(e) < 2e-2 and (e < 4e-2).mean() >= 0.9, (name, e)

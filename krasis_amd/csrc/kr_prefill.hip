@@ -402,8 +402,9 @@ void kr_launch_pf_wsum(const KrMatDev& m, int n_experts, uint32_t* wsum, hipStre
 // It knows the fused form of the group sum only, and addresses a digit plane by 32-bit offsets.
 static bool pf_all_fma(const KrMatDev& m) { return m.n_fma >= m.N; }
 // Few rows per expert, INT4: strips may be taken, of 16 rows while an expert seldom has more (up to ten on average), then of 32 while two halves still cost less than the 64-row tile: to
-// 16 rows an expert, with many experts to 24 (us a layer, both products and what stands between them, tiles against strips: 512 experts, top 10, 160 rows 308 / 207, 400 rows 330 / 245, 700
-// rows of 32 340 / 276, 1136 rows 371 / 352; 64 experts, 60 rows 128 / 102, 150 rows of 32 131 / 124; 240 rows 192 / 213).  Beside the launches of other chunks a workgroup of 32 rows (136 KB of LDS)
+// 16 rows an expert, with many experts to 20 (us a layer, both products and what stands between them, tiles against this choice: 512 experts of 2048 x 512, top 10, 160 rows 308 / 207, 400 330 / 245, 700
+// in strips of 32 340 / 276; rows an expert, 256 of 2048 x 768 8 245 / 200, 16 253 / 219, 20 257 / 234, 24 270 / 279; 128 of 4096 x 1536 8 415 / 317, 16 447 / 431, 20 441 / 446; 64 of 2048 x 1408 6
+// 128 / 102, 14 131 / 124, 24 192 / 213).  Beside the launches of other chunks a workgroup of 32 rows (136 KB of LDS)
 // waits for an empty compute unit, also when it has nothing to do (two chunks of 750 tokens 48 ms against 57): strips of 16 only, which pay to twelve rows an expert there (two chunks of
 // 600 tokens, four layers, 5.28 -> 5.00 ms).  The rows' digits have to fit the LDS.
 // Whether they are taken is for the experts' own rows to say.  An expert's second strip reads its weights again, and where every row goes to the same ten experts that is all there is
@@ -416,7 +417,7 @@ KrPfTiles kr_pf_tiles(const KrMatDev& m0, const KrMatDev& m1, long rows, int E, 
     if (rows * (long)K < 1L << 32 && rows >= 48L * E) return kr_pf_cut(PFW_TM, 0, 0, rows, E);
     if (m0.bits == 4 && m1.bits == 4 && m0.N % 16 == 0 && m1.N % 16 == 0) {
         if (rows <= (beside ? 12L : 10L) * E && pf_strip_lds(K, 16) <= PFS_LDS) return kr_pf_cut(PF_BM, 16, 12, rows, E);
-        if (!beside && rows <= (E >= 256 ? 24L : 16L) * E && pf_strip_lds(K, 32) <= PFS_LDS) return kr_pf_cut(PF_BM, 32, 10, rows, E);
+        if (!beside && rows <= (E >= 256 ? 20L : 16L) * E && pf_strip_lds(K, 32) <= PFS_LDS) return kr_pf_cut(PF_BM, 32, 10, rows, E);
     }
     return kr_pf_cut(PF_BM, 0, 0, rows, E);
 }

@@ -700,13 +700,13 @@ static void pfh_strip_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st) {
     const int ncb = (groups + spw - 1) / spw;
     hipLaunchKernelGGL(kr_pfh_strip_kernel, dim3(((mt + 7) / 8) * 8 * ncb), dim3(64 * WAVES), lds, st, a, spw, ncb);
 }
-// How the rows on E experts are cut: strips of 16 may be taken while an expert seldom has more, to 14 rows on average with hundreds of experts, else to ten; 64-row tiles beyond.  A layer's
+// How the rows on E experts are cut: strips of 16 may be taken while an expert seldom has more, to 14 rows on average with more than 256 experts, else to ten; 64-row tiles beyond.  A layer's
 // experts, us, tiles alone / this choice where it takes strips: 512 of 2048 x 512, top 10: 48 rows 187 / 136, 160 276 / 196, 400 289 / 239, 700 300 / 276; 64 of 2048 x 1408, top 6: 16 rows 89 / 82, 60 105 / 102,
-// 100 108 / 103.  The experts' own rows decide (see kr_pf_tiles): with fewer and fewer experts in use strips are the faster ones up to 1.4 times as many as tiles (520 rows, 1.28
+// 100 108 / 103; rows an expert, 384 of 2048 x 512 14 231 / 224, 16 230 / 231, 256 of 2048 x 768 12 219 / 208, 14 221 / 228, 128 of 4096 x 1536 8 387 / 308, 12 394 / 393.  The experts' own rows decide (see kr_pf_tiles): with fewer and fewer experts in use strips are the faster ones up to 1.4 times as many as tiles (520 rows, 1.28
 // 284 / 262 us, 1.39 262 / 262, 1.51 229 / 252), hence 11 / 8.  300 tokens on the same ten experts, 48 layers: tiles 13.7 ms, strips 15.4, this choice 13.7.
 KrPfTiles kr_pfh_tiles(const KrMatDev& m0, const KrMatDev& m1, long rows, int E) {
     const int K = 128 * (m0.ng > m1.ng ? m0.ng : m1.ng);
-    const bool strips = m0.bits == 4 && m1.bits == 4 && !m0.qs && !m1.qs && m0.N % 16 == 0 && m1.N % 16 == 0 && rows <= (E >= 256 ? 14L : 10L) * E && pfh_strip_lds(K) <= 160 * 1024;
+    const bool strips = m0.bits == 4 && m1.bits == 4 && !m0.qs && !m1.qs && m0.N % 16 == 0 && m1.N % 16 == 0 && rows <= (E > 256 ? 14L : 10L) * E && pfh_strip_lds(K) <= 160 * 1024;
     return kr_pf_cut(PFH_BM, strips ? PFH_ST_ROWS : 0, 11, rows, E);
 }
 

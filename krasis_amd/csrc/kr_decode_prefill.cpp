@@ -275,7 +275,9 @@ static int prefill_impl(kr_decode_store* s, const int32_t* tokens, int n_tokens,
     // defaults: 1024 tokens x 3 chunks in flight for the exact pass (its serial per-token kernels need the overlap).  The kernels of the tolerance passes (KR_ATTN_FAST, with or
     // without KR_GEMM_FAST) are chunk-parallel, and what a chunk costs per token falls as it grows (an expert's weights are converted once per 64 of its rows, and every launch has
     // a last round), so the prompt is split evenly into as few chunks of at most 4096 tokens as hold it.  Against a third of the prompt per chunk, at least 1024, ms (hybrid of four
-    // layers, 512 experts): 1500 tokens 4.21 -> 3.40, 3000 6.56 -> 5.38, 4000 7.78 -> 6.71, 5000 8.87 -> 8.00, 8192 12.69 -> 11.97; 12000 in three either way.
+    // layers, 512 experts, passes over one state; a program that goes from state to state has some 10 % more on both sides): 1500 tokens 4.21 -> 3.40, 3000 6.56 -> 5.38, 4000 7.78 -> 6.71, 5000
+    // 8.87 -> 8.00, 8192 12.69 -> 11.97, 13000 22.5 -> 21.8, 17000 29.6 -> 27.5; 12000 in three either way.  Where every token takes the same ten experts there is little to convert, and one
+    // chunk has nothing beside it: 48 such layers 1500 tokens 30.6 -> 30.1, 3000 50.4 -> 52.9, 8192 129 -> 121.
     const int n4k = (n_tokens + 4095) / 4096, tol_chunk = std::min(4096, ((n_tokens + n4k - 1) / n4k + 63) / 64 * 64);
     const int depth = s->pf_depth >= 1 && s->pf_depth <= KR_PF_MAX_DEPTH ? s->pf_depth : KR_PFM_DEPTH;   // chunks in flight (streams / arenas)
     // exact pass: chunks of ~1024 tokens, their COUNT a multiple of the depth when the prompt has that many -- the last round of chunks then fills every stream

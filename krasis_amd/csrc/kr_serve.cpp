@@ -305,7 +305,8 @@ int check_layer(const kr_serve_config& c, const kr_serve_layer* all, int i) {
     return KR_OK;
 }
 
-// pinned memory for a step's results
+// pinned memory for a step's results.  The bound is one on memory that stays pinned, not on speed: stored there by the step's last launch, logits are with the caller sooner at every size
+// than by a copy command (a prompt of 260 tokens, one layer, 1 / 64 / 250 rows of 32768: 315 / 800 / 2040 us, copied 405 / 860 / 2430).
 constexpr size_t HOST_OUT_MOST = (size_t)32 << 20;
 int host_out(kr_serve* s, size_t bytes) {
     if (bytes <= s->h_out_bytes) return KR_OK;

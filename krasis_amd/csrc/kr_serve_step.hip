@@ -67,6 +67,8 @@ bool kr_sv_step_join_fits(int T, int width, int o_cols, int experts, int top, in
 
 // Beside the experts' product attention only has to be no longer than that: a workgroup takes 256 keys in 1.5 us past its first few us, the product min(T top, experts)
 // matrices at some 5 TB/s.  One workgroup per token and key head while that covers the keys (no merge of partial states then), else powers of two, never more than alone.
+// (A step of two layers without a window, us, launches of their own / joined, 64 experts of 2 x 768 x 2048: one request at 4000 keys 240 / 175, 16000 254 / 187, 40000 274 / 200; four at 8000 352 / 325;
+// twelve at 2500 506 / 446; two at 8000 with 16 / 16 heads 322 / 256; 128 experts of 2 x 1536 x 4096, one at 16000 458 / 434.)
 int kr_sv_step_join_splits(int T, int heads, int kv_heads, int max_visible, int width, int ff, int experts, int top) {
     const int alone = kr_sv_attn_step_splits(T, heads, kv_heads, max_visible);
     const double up_us = (double)std::min(T * top, experts) * 4.0 * ff * width / 5e6;

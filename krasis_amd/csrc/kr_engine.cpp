@@ -1047,7 +1047,7 @@ static int moe_prefill_fast(kr_engine* e, Layer& L, const void* x_bf16, const in
         const int mc = M - m0 < CH ? M - m0 : CH;
         const uint16_t* xc = (const uint16_t*)x_bf16 + (size_t)m0 * H;
         const int32_t* idc = ids + (size_t)m0 * topk; const float* wc = wts + (size_t)m0 * topk;
-        const KrPfTiles cut = kr_pfh_tiles(L.w13.view(), L.w2.view(), (long)mc * topk, E);
+        const KrPfTiles cut = kr_pfh_tiles(L.w13.view(), L.w2.view(), mc, (long)mc * topk, E);
         int run = (int)(((long)mc * topk / E + 63) / 64);           // row tiles of an average expert: they share an XCD (one L2 fill of its weights)
         run = run < 1 ? 1 : (run > 4 ? 4 : run);
         kr_launch_pf_sort(idc, mc, topk, E, so, st, cut);
@@ -1118,7 +1118,7 @@ int kr_moe_prefill_set(kr_engine* e, int layer, const void* x_bf16, const int32_
         const int mc = M - m0 < CH ? M - m0 : CH;
         const uint16_t* xc = (const uint16_t*)x_bf16 + (size_t)m0 * H;
         const int32_t* idc = ids + (size_t)m0 * topk; const float* wc = wts + (size_t)m0 * topk;
-        const KrPfTiles cut = kr_pf_tiles(L.w13.view(), L.w2.view(), (long)mc * topk, E, beside);
+        const KrPfTiles cut = kr_pf_tiles(L.w13.view(), L.w2.view(), mc, (long)mc * topk, E, beside);
         kr_launch_pf_sort(idc, mc, topk, E, so, st, cut);
         kr_launch_pf_quant_x(xc, mc, H, (int8_t*)P.xh.p, (int8_t*)P.xl.p, (float*)P.xs.p, st);
         const int var_rows = (long)mc * topk < 48L * E;     // fewer than ~48 rows per expert: most 64-row tiles have an empty second half
@@ -1173,7 +1173,7 @@ int kr_moe_prefill_rows(kr_engine* e, int layer, const void* rows_bf16, const in
     const size_t ob = out_bf16 ? 2 : 4;
     for (int m0 = 0; m0 < n; m0 += CH) {
         const int mc = n - m0 < CH ? n - m0 : CH;
-        const KrPfTiles cut = kr_pf_tiles(L.w13.view(), L.w2.view(), mc, E, true);
+        const KrPfTiles cut = kr_pf_tiles(L.w13.view(), L.w2.view(), mc, mc, E, true);
         kr_launch_pf_sort(lid + m0, mc, 1, E, so, st, cut);
         kr_launch_pf_quant_x((const uint16_t*)rows_bf16 + (size_t)m0 * H, mc, H, (int8_t*)P.xh.p, (int8_t*)P.xl.p, (float*)P.xs.p, st);
         const int var_rows = (long)mc < 48L * E;

@@ -21,9 +21,10 @@ struct KrPfSort {
     int* pair_row;                                  // [n_pairs]  inverse (-1 for skipped ids)
 };
 // How the rows of a pass are cut.  `strip` > 0: the sort, which alone knows how many rows every expert has, cuts strips of that many rows instead if those are at most strip_most
-// eighths of the tiles; each of the two forms is launched then, and the one that was not taken finds a count of zero.  max_tiles, max_strips: the most there can be of a form taken.
+// eighths of the tiles; each of the two forms is launched then, and the one that was not taken finds a count of zero.  max_tiles, max_strips: the most there can be of a form taken (max_tiles 0: strips
+// whatever the rows, nothing else is launched).
 struct KrPfTiles { int rows, strip, strip_most, max_tiles, max_strips; };
-KrPfTiles kr_pf_cut(int tile_rows, int strip, int strip_most, long rows, int E);
+KrPfTiles kr_pf_cut(int tile_rows, int strip, int strip_most, int tokens, long rows, int E);
 void kr_launch_pf_sort(const int32_t* ids, int M, int topk, int E, KrPfSort s, hipStream_t st, const KrPfTiles& t = KrPfTiles{64, 0, 0, 0, 0});
 void kr_launch_pf_quant_x(const uint16_t* x, int M, int K, int8_t* xh, int8_t* xl, float* xs, hipStream_t st);
 void kr_launch_pf_act(const float* gu, int rows, int n, int gu_ld, int act_mode, float swiglu_limit, float alpha, int8_t* hh, int8_t* hl, float* hs, hipStream_t st);
@@ -33,7 +34,7 @@ void kr_launch_pf_gemm(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_
                        int var_rows = 0 /* expert tiles mostly <= 32 rows: kernel variant that skips empty 32-row blocks */,
                        const KrPfTiles* t = nullptr /* of the tile table; null: tiles of 64 */);
 // of the exact GEMMs that will run on one tile table: tiles of 128 rows (the wide kernel) or 64, and whether strips may take their place
-KrPfTiles kr_pf_tiles(const KrMatDev& m0, const KrMatDev& m1, long rows, int E, bool beside /* launches of other chunks run at the same time */);
+KrPfTiles kr_pf_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows /* of all their slots */, int E, bool beside /* launches of other chunks run at the same time */);
 void kr_launch_pf_gemm_multi(const KrMatDev* mats, const uint32_t* const* wsums, float* const* outs, const int* out_lds, int n, const int8_t* a_hi, const int8_t* a_lo,
                              const float* a_scale, int M, hipStream_t st);
 void kr_launch_pf_combine(const float* eo, const int* pair_row, const float* wts, int M, int topk, int H, const float* shared_eo, float rsf, void* out,
@@ -58,7 +59,7 @@ void kr_launch_pfh_act(const float* gu, int rows, int n, int gu_ld, int act_mode
 void kr_launch_pfh_gemm(const KrMatDev& m, const uint16_t* a_h, const float* a_mul, const KrPfSort* sort, int topk, int gather_tokens, int max_tiles,
                         int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows = 0, int out_bf16 = 0, int run = 1,
                         const uint16_t* a_sum32 = nullptr /* required when m.qs is set (Q4_K copy) */, const KrPfTiles* t = nullptr /* of the tile table; null: tiles of 64 */);
-KrPfTiles kr_pfh_tiles(const KrMatDev& m0, const KrMatDev& m1, long rows, int E);      // of the tolerance GEMMs' tile table
+KrPfTiles kr_pfh_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows, int E);      // of the tolerance GEMMs' tile table
 void kr_launch_pfh_w13_act(const KrMatDev& m, const uint16_t* a_h, const float* a_mul, const KrPfSort* sort, int topk, int gather_tokens, int max_tiles,
                            int single_expert_rows, float* gu, int rows, int act_mode, float swiglu_limit, float alpha, uint16_t* h_out, float* h_mul,
                            hipStream_t st, int run = 1, const uint16_t* a_sum32 = nullptr, uint16_t* h_sums32 = nullptr, const KrPfTiles* t = nullptr);

@@ -355,11 +355,12 @@ __global__ void __launch_bounds__(256) kr_pf_combine_kernel(const void* __restri
 // ------------------------------------------------------------------------------------------
 // strips <= strip_most / 8 tiles, so a pass of strips has at most (strip_most / 8) (tiles <= rows / tile_rows + E) of them; and where tiles were taken, tiles < strips / (strip_most / 8),
 // strips <= rows / strip + tiles, so that tiles < rows / strip / (strip_most / 8 - 1)
-KrPfTiles kr_pf_cut(int tile_rows, int strip, int strip_most, long rows, int E) {
+KrPfTiles kr_pf_cut(int tile_rows, int strip, int strip_most, int tokens, long rows, int E) {
     KrPfTiles t{tile_rows, strip, strip_most, (int)(rows / tile_rows) + E + 1, 0};
     if (strip <= 0) return t;
     if (rows > KR_PF_SORT1_MAX || E > 1024) { t.strip = 0; return t; }      // (the sort's other form cuts tiles only)
     t.max_strips = (int)(rows / strip) + E + 1;
+    if (tokens <= strip) { t.strip_most = 1 << 16; t.max_tiles = 0; return t; }      // no expert has a second strip (or only of tokens that name it twice)
     t.max_tiles = std::min(t.max_tiles, (int)(rows * 8 / ((long)strip * (strip_most - 8))) + 1);
     return t;
 }
@@ -411,15 +412,15 @@ static bool pf_all_fma(const KrMatDev& m) { return m.n_fma >= m.N; }
 // (300 tokens of 48 such layers: tiles 20.4 ms, strips 22.4, this choice 20.7).  Measured with ever fewer experts in use, strips of 16 are the faster ones up to 1.6 times as many as tiles (400
 // rows, 1.41 253 / 220 us, 1.57 215 / 210, 1.95 163 / 172), strips of 32 up to 1.35 (1136 rows, 1.28 397 / 368, 1.35 355 / 353, 1.53 291 / 306); the launch that finds nothing costs 5 us,
 // so the lines are 12 / 8 and 10 / 8.
-KrPfTiles kr_pf_tiles(const KrMatDev& m0, const KrMatDev& m1, long rows, int E, bool beside) {
-    if (!pf_all_fma(m0) || !pf_all_fma(m1)) return kr_pf_cut(PF_BM, 0, 0, rows, E);
+KrPfTiles kr_pf_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows, int E, bool beside) {
+    if (!pf_all_fma(m0) || !pf_all_fma(m1)) return kr_pf_cut(PF_BM, 0, 0, tokens, rows, E);
     const int K = 128 * (m0.ng > m1.ng ? m0.ng : m1.ng);
-    if (rows * (long)K < 1L << 32 && rows >= 48L * E) return kr_pf_cut(PFW_TM, 0, 0, rows, E);
+    if (rows * (long)K < 1L << 32 && rows >= 48L * E) return kr_pf_cut(PFW_TM, 0, 0, tokens, rows, E);
     if (m0.bits == 4 && m1.bits == 4 && m0.N % 16 == 0 && m1.N % 16 == 0) {
-        if (rows <= (beside ? 12L : 10L) * E && pf_strip_lds(K, 16) <= PFS_LDS) return kr_pf_cut(PF_BM, 16, 12, rows, E);
-        if (!beside && rows <= (E >= 256 ? 20L : 16L) * E && pf_strip_lds(K, 32) <= PFS_LDS) return kr_pf_cut(PF_BM, 32, 10, rows, E);
+        if (rows <= (beside ? 12L : 10L) * E && pf_strip_lds(K, 16) <= PFS_LDS) return kr_pf_cut(PF_BM, 16, 12, tokens, rows, E);
+        if (!beside && rows <= (E >= 256 ? 20L : 16L) * E && pf_strip_lds(K, 32) <= PFS_LDS) return kr_pf_cut(PF_BM, 32, 10, tokens, rows, E);
     }
-    return kr_pf_cut(PF_BM, 0, 0, rows, E);
+    return kr_pf_cut(PF_BM, 0, 0, tokens, rows, E);
 }
 static bool pf_dense_wide(const KrPfGemmArgs& a) {
     int ncb = (a.m.N + PFW_TN - 1) / PFW_TN; bool all = pf_all_fma(a.m);
@@ -443,6 +444,7 @@ void kr_launch_pf_gemm(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_
         KrPfGemmArgs b = a;
         b.n_tiles = a.n_tiles + 2;
         if (t->strip == 16) kr_pf_strip_launch<1, 8>(b, t->max_strips, st); else kr_pf_strip_launch<2, 16>(b, t->max_strips, st);
+        if (t->max_tiles == 0) return;
     }
     const int mt = single_expert_rows > 0 ? (single_expert_rows + PF_BM - 1) / PF_BM : max_tiles;
     // 32 columns per wave, two quantization groups per k stage: the best of the (64|32 columns) x (1|2 groups) shapes and of a 2 x 2 row-split

@@ -704,10 +704,10 @@ static void pfh_strip_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st) {
 // experts, us, tiles alone / this choice where it takes strips: 512 of 2048 x 512, top 10: 48 rows 187 / 136, 160 276 / 196, 400 289 / 239, 700 300 / 276; 64 of 2048 x 1408, top 6: 16 rows 89 / 82, 60 105 / 102,
 // 100 108 / 103; rows an expert, 384 of 2048 x 512 14 231 / 224, 16 230 / 231, 256 of 2048 x 768 12 219 / 208, 14 221 / 228, 128 of 4096 x 1536 8 387 / 308, 12 394 / 393.  The experts' own rows decide (see kr_pf_tiles): with fewer and fewer experts in use strips are the faster ones up to 1.4 times as many as tiles (520 rows, 1.28
 // 284 / 262 us, 1.39 262 / 262, 1.51 229 / 252), hence 11 / 8.  300 tokens on the same ten experts, 48 layers: tiles 13.7 ms, strips 15.4, this choice 13.7.
-KrPfTiles kr_pfh_tiles(const KrMatDev& m0, const KrMatDev& m1, long rows, int E) {
+KrPfTiles kr_pfh_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows, int E) {
     const int K = 128 * (m0.ng > m1.ng ? m0.ng : m1.ng);
     const bool strips = m0.bits == 4 && m1.bits == 4 && !m0.qs && !m1.qs && m0.N % 16 == 0 && m1.N % 16 == 0 && rows <= (E > 256 ? 14L : 10L) * E && pfh_strip_lds(K) <= 160 * 1024;
-    return kr_pf_cut(PFH_BM, strips ? PFH_ST_ROWS : 0, 11, rows, E);
+    return kr_pf_cut(PFH_BM, strips ? PFH_ST_ROWS : 0, 11, tokens, rows, E);
 }
 
 template <int NC, int BITS, int SB = 0, int G = 0, int OCC = 2>
@@ -777,6 +777,7 @@ void kr_launch_pfh_gemm(const KrMatDev& m, const uint16_t* a_h, const float* a_m
         KrPfGemmHArgs b = a;
         b.n_tiles = a.n_tiles + 2;
         pfh_strip_launch(b, t->max_strips, st);
+        if (t->max_tiles == 0) return;
     }
     pfh_dispatch(a, mt, st);
 }

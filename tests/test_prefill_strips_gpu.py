@@ -102,3 +102,19 @@ def test_scattered_rows_of_expert_parallel_ranks(Ms, ret_bf16):
     """nine rows a local expert, each row stored at the place that it came from, in f32 and in bf16"""
     import tests.test_ep_gpu as ep
     ep.test_library_expert_parallel_loopback_equals_single_engine(2, Ms, ret_bf16, False)
+
+
+@pytest.mark.parametrize("M", [2, 16, 17])
+def test_up_to_sixteen_tokens(M):
+    """strips whatever the rows, also where tokens name an expert twice and it has a second strip; one token more, and the experts' own rows decide"""
+    eng, experts, shared, rng, torch = _setup(256, 128, 20, 3)
+    x = rand_bf16(rng, (M, 256)); w = rng.random((M, 3)).astype(F)
+    ids = np.full((M, 3), 7, np.int32); ids[:, 2] = 9; ids[0, 1] = -1
+    out = _prefill_mode(eng, torch, x, ids, w, 0)
+    rows = (2 * M - 1, M)
+    assert _cut(eng) == ((0, sum(-(-r // 16) for r in rows)) if M <= 16 else (2, 0))
+    ref = _forward(eng, torch, x, ids, w)
+    assert np.array_equal(out.view(np.uint32), ref.view(np.uint32))
+    tol = _prefill_mode(eng, torch, x, ids, w, 1)
+    assert (_cut(eng)[1] > 0) == (M <= 16)
+    assert float(np.linalg.norm((tol - ref).astype(np.float64)) / np.linalg.norm(ref.astype(np.float64))) <= 2.0 ** -10

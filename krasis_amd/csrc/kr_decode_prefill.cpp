@@ -259,6 +259,39 @@ static int run_final_all(kr_decode_store* s, Chunk& cx, float* vlogits, int firs
     return KR_OK;
 }
 
+static int prompt_depth(const kr_decode_store* s) { return s->pf_depth >= 1 && s->pf_depth <= KR_PF_MAX_DEPTH ? s->pf_depth : KR_PFM_DEPTH; }
+
+// tokens per chunk of a prompt.  Defaults:
+// Exact pass: chunks of ~1024 tokens, three in flight (its serial per-token kernels need the overlap), their COUNT a multiple of the depth when the prompt has that many -- the last
+// round of chunks then fills every stream (8192 tokens: 8 x 1024 = 3 + 3 + 2 chunks 382.9 ms, 6 x 1366 355.8; 20 434: 20 x 1024 1207.9, 18 x 1136 1180.1; 49 863: unchanged, attention-bound).
+// Tolerance passes (KR_ATTN_FAST, with or without KR_GEMM_FAST): their kernels are chunk-parallel, and what a chunk costs per token falls as it grows (an expert's weights are converted
+// once per 64 of its rows, and every launch has a last round), so the prompt is split evenly into as few chunks of at most 4096 tokens as hold it.  Against a third of the prompt per
+// chunk, at least 1024, ms (hybrid of four layers, 512 experts, passes over one state; a program that goes from state to state has some 10 % more on both sides): 1500 tokens
+// 4.21 -> 3.40, 3000 6.56 -> 5.38, 4000 7.78 -> 6.71, 5000 8.87 -> 8.00, 8192 12.69 -> 11.97, 13000 22.5 -> 21.8, 17000 29.6 -> 27.5; 12000 in three either way.  Where every token
+// takes the same ten experts there is little to convert, and one chunk has nothing beside it: 48 such layers 1500 tokens 30.6 -> 30.1, 3000 50.4 -> 52.9, 8192 129 -> 121.
+// MLA layers and native GGUF experts gain more from a second chunk beside the first than from its size, so there the prompt takes at least two from 1025 tokens on.  One and two chunks,
+// ms, both bits / attention bit alone: 27 MLA layers 1500 tokens 26.9, 24.7 / 30.3, 28.8; 2048 34.9, 32.3 / 38.9, 36.4; 3000 54.0, 50.9 / 58.9, 55.0; 4000 78.5, 70.1 / 81.0, 75.4;
+// 16 hybrid layers of GGUF experts 1500 tokens - / 16.0, 15.0; 2048 12.8, 12.3 / 21.0, 19.1; 3000 18.0, 16.8 / 29.2, 26.0; 4000 22.2, 21.7 / 37.0, 34.9.  MLA layers take three
+// from 4609 to 7680 tokens, two and three: 4100 tokens 76.2, 77.6 / 77.9, 82.1; 5000 103.7, 99.8 / 104.4, 104.8; 6500 157.1, 148.6 / 153.6, 152.1; 7500 182.5, 179.7 / 187.7, 184.9;
+// 8192 202.0, 205.4 / 207.0, 211.2.  The other stores, one and two, both bits: 8 layers of GQA with 128 INT4 experts 2048
+// tokens 12.8, 13.3, 4000 25.9, 25.5; 16 hybrid layers of INT8 experts 2048 tokens 16.1, 20.0, 4000 28.3, 30.0.
+static int prompt_chunk(const kr_decode_store* s, int n_tokens, int depth) {
+    if (s->pf_chunk > 0) return s->pf_chunk;
+    if (!s->attn_fast) {
+        const int q1k = (n_tokens + KR_PFM_CHUNK - 1) / KR_PFM_CHUNK, nc = q1k >= depth ? (q1k / depth) * depth : q1k;
+        return (n_tokens + nc - 1) / nc;
+    }
+    bool mla = false, gguf = false;
+    for (auto& Ly : s->layers) {
+        mla |= Ly.attn == ATTN_MLA;
+        gguf |= Ly.mlp == MLP_MOE && Ly.moe_layer < (int)s->eng->layers.size() && s->eng->layers[Ly.moe_layer].gguf;      // an index past the engine's is refused by the pass
+    }
+    int n = (n_tokens + 4095) / 4096;
+    if ((mla || gguf) && n == 1 && n_tokens > 1024) n = 2;
+    if (mla && n_tokens > 4608 && n_tokens <= 7680) n = 3;
+    return std::min(4096, ((n_tokens + n - 1) / n + 63) / 64 * 64);
+}
+
 static int prefill_impl(kr_decode_store* s, const int32_t* tokens, int n_tokens, int start_pos, float* logits_out, float* nll_out, void* stream) {
     if (!s) return kr_fail(KR_ERR_VALUE, "null decode store");
     if (!s->configured) return kr_fail(KR_ERR_STATE, "Call configure_decode first");
@@ -272,19 +305,8 @@ static int prefill_impl(kr_decode_store* s, const int32_t* tokens, int n_tokens,
     hipStream_t st = kr_pick_stream(e, stream);
     const int H = s->hidden;
     if (H % 128) return kr_fail(KR_ERR_VALUE, "kr_decode_prefill needs hidden %% 128 == 0");
-    // defaults: 1024 tokens x 3 chunks in flight for the exact pass (its serial per-token kernels need the overlap).  The kernels of the tolerance passes (KR_ATTN_FAST, with or
-    // without KR_GEMM_FAST) are chunk-parallel, and what a chunk costs per token falls as it grows (an expert's weights are converted once per 64 of its rows, and every launch has
-    // a last round), so the prompt is split evenly into as few chunks of at most 4096 tokens as hold it.  Against a third of the prompt per chunk, at least 1024, ms (hybrid of four
-    // layers, 512 experts, passes over one state; a program that goes from state to state has some 10 % more on both sides): 1500 tokens 4.21 -> 3.40, 3000 6.56 -> 5.38, 4000 7.78 -> 6.71, 5000
-    // 8.87 -> 8.00, 8192 12.69 -> 11.97, 13000 22.5 -> 21.8, 17000 29.6 -> 27.5; 12000 in three either way.  Where every token takes the same ten experts there is little to convert, and one
-    // chunk has nothing beside it: 48 such layers 1500 tokens 30.6 -> 30.1, 3000 50.4 -> 52.9, 8192 129 -> 121.
-    const int n4k = (n_tokens + 4095) / 4096, tol_chunk = std::min(4096, ((n_tokens + n4k - 1) / n4k + 63) / 64 * 64);
-    const int depth = s->pf_depth >= 1 && s->pf_depth <= KR_PF_MAX_DEPTH ? s->pf_depth : KR_PFM_DEPTH;   // chunks in flight (streams / arenas)
-    // exact pass: chunks of ~1024 tokens, their COUNT a multiple of the depth when the prompt has that many -- the last round of chunks then fills every stream
-    // (8192 tokens: 8 x 1024 = 3 + 3 + 2 chunks 382.9 ms, 6 x 1366 355.8; 20 434: 20 x 1024 1207.9, 18 x 1136 1180.1; 49 863: unchanged, attention-bound)
-    const int q1k = (n_tokens + KR_PFM_CHUNK - 1) / KR_PFM_CHUNK, nc_exact = q1k >= depth ? (q1k / depth) * depth : q1k;
-    const int exact_chunk = (n_tokens + nc_exact - 1) / nc_exact;
-    const int CH = std::min(n_tokens, s->pf_chunk > 0 ? s->pf_chunk : (s->attn_fast ? tol_chunk : exact_chunk));
+    const int depth = prompt_depth(s);   // chunks in flight (streams / arenas)
+    const int CH = std::min(n_tokens, prompt_chunk(s, n_tokens, depth));
     // expert parallelism: every rank must walk the SAME (chunk, layer) schedule -- the exchanges are collectives -- so the schedule is built from the chunk
     // count of the longest prompt shard (agreed below, before the first exchange); chunks a rank does not have run as empty shards
     int n_chunks_max = (n_tokens + CH - 1) / CH;
@@ -472,7 +494,15 @@ extern "C" int kr_decode_set_prefill_depth(kr_decode_store* s, int depth) {
     return KR_OK;
 }
 
-// test / tuning hook: tokens per chunk of the prompt pass (0 = default 1024)
+// test hook: tokens per chunk that a prompt of n_tokens takes
+extern "C" int kr_decode_prefill_chunk(const kr_decode_store* s, int n_tokens, int* chunk) {
+    if (!s || !chunk || n_tokens <= 0) return kr_fail(KR_ERR_VALUE, "null argument or empty prompt");
+    if (!s->configured || (int)s->layers.size() != s->n_layers) return kr_fail(KR_ERR_STATE, "finalize_decode was not called");
+    *chunk = std::min(n_tokens, prompt_chunk(s, n_tokens, prompt_depth(s)));
+    return KR_OK;
+}
+
+// test / tuning hook: tokens per chunk of the prompt pass (0 = the default rule)
 extern "C" int kr_decode_set_prefill_chunk(kr_decode_store* s, int chunk) {
     if (!s) return kr_fail(KR_ERR_VALUE, "null decode store");
     if (chunk < 0 || chunk > 8192) return kr_fail(KR_ERR_VALUE, "prefill chunk %d out of range [0, 8192]", chunk);

@@ -331,7 +331,7 @@ class CpuDecodeStore:
         check(self._lib.kr_decode_reset_state(self._h, kv_max_seq))
 
     def set_prefill_chunk(self, chunk: int) -> None:
-        """Tokens per chunk of the prompt pass (0 = default); chunks alternate between two streams."""
+        """Tokens per chunk of the prompt pass (0 = the default rule)."""
         self._need(); check(self._lib.kr_decode_set_prefill_chunk(self._h, chunk))
 
     def set_prefill_depth(self, depth: int) -> None:

@@ -2,14 +2,18 @@
 // store's on v_mfma_f32_32x32x2_f32.
 //
 // Bound: the matrix cores (about 1350 TFLOP/s is what a large library product reaches here; nominal 2500).  Both operands travel from memory to LDS by
-// global_load_lds_dwordx4 into a ring of slots of 64 k (no staging registers; whole cache lines), ONE barrier per slot, the next slot requested right behind it, fragments
-// of a k step read while the step before is multiplied.  What the large tile buys: 256 x 256 by eight waves of 128 x 64 reads 48 KB of fragments per 64 matrix
-// instructions and SIMD and 64 KB of operands per slot; 128 x 128 by four waves of 64 x 64 needs a third more of the first and twice the second for the same products,
-// and neither the LDS nor the L2 rate hides behind the matrix cores then (requests and reads without products 206 us, products without requests 197 us, both 315 us at
-// 3300 x 4096 x 8192).  LDS-DMA writes lane-linear (lane i at base + 16 i), so bank conflicts are avoided on the SOURCE side: the 16-byte chunk c of row r sits at
+// global_load_lds_dwordx4 into a ring of slots of 64 k (no staging registers; whole cache lines), fragments read while products run.  What the large tile buys:
+// 256 x 256 by eight waves of 128 x 64 reads 48 KB of fragments per 64 matrix instructions and SIMD and 64 KB of operands per slot; 128 x 128 by four waves of 64 x 64 needs
+// a third more of the first and twice the second for the same products, and neither the LDS nor the L2 rate hides behind the matrix cores then.
+// What the two larger tiles wait for is the operands: a slot's requests take the CU's 64 bytes a cycle of L1 path for half of the slot's matrix time, and with two whole slots
+// in turn they had one slot's time for that and for the way to L2 or memory and back (3300 x 4096 x 8192 in clocks of a CU: matrix instructions alone 287 k, with the
+// fragment reads 318 k, with the requests 466 k).  So a slot is given back by parts: the fragments of W's slot and of one row block of A's stand in registers before they
+// are multiplied, a part of the ring is free as soon as it has been read, and its next request leaves then, one and a half slots of time ahead of its use (348 k clocks).
+// LDS-DMA writes lane-linear (lane i at base + 16 i), so bank conflicts are avoided on the SOURCE side: the 16-byte chunk c of row r sits at
 // position c ^ (r / 2 % 8) of its 128-byte row and the fragment reads apply the same map (without it 1.6 - 2.1 x slower).
-// Measured, us, register-staged 128 x 128 tile before -> now: 3300 x 4096 x 8192 425 -> 238 (931 TFLOP/s), 3300 x 12544 x 4096 596 -> 376, 4096 x 4224 x 2048 144 -> 104,
-// 64 experts 24576 x 1536 x 2048 372 -> 248 and x 2048 x 768 217 -> 149, 500 x 2048 x 2048 36.8 -> 14.1, 100 x 4224 x 2048 36.9 -> 13.2.
+// Measured, us, slots whole -> by parts: 3300 x 4096 x 8192 238 -> 208 (1064 TFLOP/s), 3300 x 12416 x 4096 363 -> 344, 4096 x 4160 x 2048 101 -> 87, 2500 x 4160 x 2048 66 -> 55,
+// 3249 x 2048 x 6144 111 -> 92, 500 x 4160 x 2048 26.3 -> 20.2; 64 experts, 24576 x 1536 x 2048 237 -> 210, x 2048 x 768 133 -> 120 (201 MB of f32 results), 15000 x 1536 x 2048 188 -> 149;
+// under lasting load the clock falls and the gains are 7 - 12 %.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -36,10 +40,10 @@ template <int N> __device__ __forceinline__ void tl_wait_barrier() { asm volatil
 template <typename T, int BM, int BN, int WM, int WN, int DEPTH, int WPS, bool GLU>  // WM x WN waves; WPS: waves per SIMD the register budget is for
 __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGemm g) {
     constexpr int MB = BM / (32 * WM), NB = BN / (32 * WN);    // 32 x 32 blocks of a wave
-    constexpr int RA = BM / 8, RW = (BM + BN) / (8 * WM * WN); // requests of 8 rows per slot: A's; per wave
-    constexpr int BK = TL_ROW / (int)sizeof(T), CH = 16 / (int)sizeof(T), SLOT = (BM + BN) * BK;     // k of a slot, elements of a chunk and of a slot
+    constexpr int RA = 4 / WN, RW = 4 * NB / WM;               // requests of 8 rows that a wave makes for a row block of A's slot and for W's slot
+    constexpr int BK = TL_ROW / (int)sizeof(T), CH = 16 / (int)sizeof(T);     // k of a slot, elements of a chunk
+    constexpr uint32_t AS = BM * TL_ROW, WS = BN * TL_ROW;     // bytes of a slot of A and of W: A's slots come first
     extern __shared__ __attribute__((aligned(1024))) uint8_t ring_[];
-    T* ring = reinterpret_cast<T*>(ring_);
     int bx = blockIdx.x, by = blockIdx.y;
     // Workgroups go round the eight XCDs, each with its own L2.  With a column count of a multiple of eight an XCD sees the same columns of W for all rows; otherwise,
     // and with one matrix per expert, it is given whole pairs of row tiles: their rows stay in its L2, the pair shares the columns of W.
@@ -59,19 +63,24 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
     const T* A = (const T*)g.A;
     const T* W = (const T*)g.W + (size_t)group * g.w_stride;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5, wr = wave / WN, wc = wave % WN;
-    const T* src[RW];
+    const T* as[MB][RA]; const T* ws[RW];
+#pragma unroll
+    for (int a = 0; a < MB; a++)
+#pragma unroll
+        for (int i = 0; i < RA; i++) {
+            const int row = a * 32 * WM + (wave * RA + i) * 8 + (lane >> 3), ch = (lane & 7) ^ ((row >> 1) & 7), m = min(m0 + row, mend - 1);
+            as[a][i] = A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda + ch * CH;
+        }
 #pragma unroll
     for (int i = 0; i < RW; i++) {
-        const int q = wave * RW + i;                           // request: RA of A's rows, then W's
-        const int row = (q < RA ? q : q - RA) * 8 + (lane >> 3), ch = (lane & 7) ^ ((row >> 1) & 7);
-        if (q < RA) { const int m = min(m0 + row, mend - 1); src[i] = A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda + ch * CH; }
-        else if (pairs) {                                      // a wave's columns: its gates, then their up factors
+        const int row = (wave * RW + i) * 8 + (lane >> 3), ch = (lane & 7) ^ ((row >> 1) & 7);
+        if (pairs) {                                           // a wave's columns: its gates, then their up factors
             constexpr int WC = BN / WN;
             const int j = n0 + row / WC * (WC / 2) + row % (WC / 2), up = row % WC >= WC / 2;
-            src[i] = W + (size_t)(g.glu_lo + up * g.glu_f + min(j, N - 1)) * g.K + ch * CH;
-        } else src[i] = W + (size_t)column(min(n0 + row, N - 1)) * g.K + ch * CH;
+            ws[i] = W + (size_t)(g.glu_lo + up * g.glu_f + min(j, N - 1)) * g.K + ch * CH;
+        } else ws[i] = W + (size_t)column(min(n0 + row, N - 1)) * g.K + ch * CH;
     }
-    const uint32_t base = __builtin_amdgcn_readfirstlane(tl_lds_addr(ring)) + (uint32_t)(wave * RW) * 1024u;
+    const uint32_t ringa = __builtin_amdgcn_readfirstlane(tl_lds_addr(ring_)), basea = ringa + wave * RA * 1024u, basew = ringa + DEPTH * AS + wave * RW * 1024u;
     gv16f acc[MB][NB];
 #pragma unroll
     for (int a = 0; a < MB; a++)
@@ -81,72 +90,126 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
             for (int i = 0; i < 16; i++) acc[a][b][i] = 0.0f;
     const int steps = g.K / BK;
     // A tile's row blocks go round the waves' rows (block a of wave row wr: rows 32 (a WM + wr)), so that the last tile of a matrix or an expert, which is seldom full, takes only the
-    // blocks it has: the k loop exists once per number of them, and rows past the last block are not requested (the waits that count requests belong to the deep ring, whose
-    // waves have one block).  24576 rows on 64 experts, about 384 each, 2 x 768 x 2048: 235 -> 222 us; 27500
+    // blocks it has: the k loop exists once per number of them, and rows past the last block are not requested.  24576 rows on 64 experts, about 384 each, 2 x 768 x 2048: 235 -> 222 us; 27500
     // rows on 128, 2 x 1536 x 4096: 730 -> 702, and x 4096 x 1536 308 -> 283.
     const int blocks = MB == 1 ? 1 : min(MB, __builtin_amdgcn_readfirstlane((mend - m0 + 32 * WM - 1) / (32 * WM)));
-    static_assert(MB == 1 || DEPTH == 2, "all waits of a tile with several blocks are for everything");
-    auto request = [&](int slot) {
+    static_assert(MB == 1 || DEPTH == 2, "two slots, given back by parts");
+    auto request_a = [&](int slot, int a) {                    // row block a of A's next slot that it has not requested, into ring slot `slot`
 #pragma unroll
-        for (int i = 0; i < RW; i++) {
-            const int q = wave * RW + i;
-            if (MB == 1 || q >= RA || q < blocks * 4 * WM) tl_dma16(base + (uint32_t)slot * (uint32_t)(SLOT * sizeof(T)) + i * 1024u, src[i]);
-            src[i] += BK;
+        for (int i = 0; i < RA; i++) { tl_dma16(basea + slot * AS + a * (32 * WM * TL_ROW) + i * 1024u, as[a][i]); as[a][i] += BK; }
+    };
+    auto request_w = [&](int slot) {
+#pragma unroll
+        for (int i = 0; i < RW; i++) { tl_dma16(basew + slot * WS + i * 1024u, ws[i]); ws[i] += BK; }
+    };
+    // fragment of rows [32 blk, +32), k step ks of the slot: chunk ks + 4 h of row r (the halves of the wave take k halves of the slot; any order serves, both operands alike)
+    const int sw = (4 * h) ^ ((r >> 1) & 7);
+    const uint8_t* afp = ring_ + (wr * 32 + r) * TL_ROW;
+    const uint8_t* wfp = ring_ + DEPTH * AS + (wc * (BN / WN) + r) * TL_ROW;
+    auto multiply = [&](gv16f& c, const gu4& fa, const gu4& fb) {
+        if constexpr (sizeof(T) == 2) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(gb8, fa), __builtin_bit_cast(gb8, fb), c, 0, 0, 0);
+        else {                                                 // a chunk is four steps of 2 k, one per half
+#pragma unroll
+            for (int e = 0; e < 4; e++) c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fa[e]), __uint_as_float(fb[e]), c, 0, 0, 0);
         }
     };
-#pragma unroll
-    for (int d = 0; d < DEPTH - 1; d++) if (d < steps) request(d);
-    // fragment of rows [32 blk, +32), k step ks of the slot: chunk ks + 4 h of row r
-    const int sw = (r >> 1) & 7;
-    const T* af0 = ring + (wr * 32 + r) * BK;
-    const T* bf0 = ring + (BM + wc * (BN / WN) + r) * BK;
-    auto multiply = [&](auto used) {                           // used: blocks of this tile
-    constexpr int MU = used();
-    int slot = 0;
-    for (int s = 0; s < steps; s++) {
-        // slot s has landed when only the DEPTH - 2 younger ones are outstanding (none at the end)
-        if (DEPTH == 2 || s + 1 >= steps) tl_wait_barrier<0>(); else tl_wait_barrier<(DEPTH - 2) * RW>();
-        if (s + DEPTH - 1 < steps) request(slot == 0 ? DEPTH - 1 : slot - 1);      // the slot read in the previous step: every wave is past it
-        const T* ab = af0 + slot * SLOT;
-        const T* bb = bf0 + slot * SLOT;
-        gu4 af[2][MB], bf[2][NB];                              // fragments of two k steps: one is read while the other is multiplied
-        auto read = [&](int ks) {
-            const int ch = ((ks + 4 * h) ^ sw) * CH;           // the halves of the wave take k halves of the slot (any order serves, both operands alike)
-#pragma unroll
-            for (int a = 0; a < MU; a++) af[ks & 1][a] = *reinterpret_cast<const gu4*>(ab + a * 32 * WM * BK + ch);
-#pragma unroll
-            for (int b = 0; b < NB; b++) bf[ks & 1][b] = *reinterpret_cast<const gu4*>(bb + b * 32 * BK + ch);
+    // one block per wave, several workgroups per unit: whole slots, DEPTH deep, one barrier each; the next slot's first fragments are read during this one's last products
+    auto whole_slots = [&]() {
+        gu4 af[2], wf[2];
+        auto request = [&](int slot) { request_a(slot, 0); request_w(slot); };
+        auto read = [&](int slot, int ks) {
+            af[ks & 1] = *reinterpret_cast<const gu4*>(afp + slot * AS + ((ks ^ sw) << 4));
+            wf[ks & 1] = *reinterpret_cast<const gu4*>(wfp + slot * WS + ((ks ^ sw) << 4));
         };
-        read(0);
 #pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            if (ks + 1 < 4) read(ks + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (sizeof(T) == 2) {
+        for (int d = 0; d < DEPTH; d++) if (d < steps) request(d);
+        // a slot has landed when only the younger ones are outstanding
+        if (steps >= DEPTH) tl_wait_barrier<(DEPTH - 1) * (RA + RW)>(); else tl_wait_barrier<0>();
+        read(0, 0);
+        int slot = 0;
+        for (int s = 0; s < steps; s++) {
 #pragma unroll
-                for (int a = 0; a < MU; a++)
-#pragma unroll
-                    for (int b = 0; b < NB; b++)
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(gb8, af[ks & 1][a]), __builtin_bit_cast(gb8, bf[ks & 1][b]), acc[a][b], 0, 0, 0);
-            } else {                                           // a chunk is four steps of 2 k, one per half
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-#pragma unroll
-                    for (int a = 0; a < MU; a++)
-#pragma unroll
-                        for (int b = 0; b < NB; b++)
-                            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(af[ks & 1][a][e]), __uint_as_float(bf[ks & 1][b][e]), acc[a][b], 0, 0, 0);
+            for (int ks = 0; ks < 4; ks++) {
+                if (ks + 1 < 4) read(slot, ks + 1);
+                else if (s + 1 < steps) {
+                    // the wave's last fragments of slot s are in registers: behind the barrier every wave's are
+                    if (s + DEPTH - 1 < steps) tl_wait_barrier<(DEPTH - 2) * (RA + RW)>(); else tl_wait_barrier<0>();
+                    const int next = slot == DEPTH - 1 ? 0 : slot + 1;
+                    read(next, 0);
+                    if (s + DEPTH < steps) request(slot);
+                    slot = next;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(acc[0][0], af[ks & 1], wf[ks & 1]);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            __builtin_amdgcn_sched_barrier(0);
         }
-        slot = slot == DEPTH - 1 ? 0 : slot + 1;
-    }
+    };
+    // Slots by parts, for a tile of `used` row blocks.  Phase a multiplies block a's fragments with W's and reads block a + 1's; the last phase of a slot reads block 0 and W of
+    // the next one instead.  Two barriers a slot, before phase 0 and before phase HB, and behind each the requests for what was read since the one before:
+    //   before phase 0, slot s:    blocks HB + 1 .. of slot s + 1, block 0 and W of slot s + 2      (N1 requests of a wave)
+    //   before phase HB:           blocks 1 .. HB of slot s + 2                                     (N2)
+    // Each is needed behind the third barrier after it: that barrier waits until only the N1 + N2 requests made since then are outstanding (fewer at the end, where
+    // slots past the last are not requested).  Fragments read for a slot past the last are whatever stands in the ring and are not multiplied.
+    auto slots_by_parts = [&](auto used) {
+        constexpr int MU = used(), HB = MU / 2, N2 = HB * RA, N1 = (MU - HB) * RA + RW, NT = (MU - 1 - HB) * RA;      // NT: of N1, slot s + 1's
+        gu4 af[2][4], wf[4][NB];
+        auto read_a = [&](int buf, int slot, int a, int ks) { af[buf][ks] = *reinterpret_cast<const gu4*>(afp + slot * AS + a * (32 * WM * TL_ROW) + ((ks ^ sw) << 4)); };
+        auto read_w = [&](int slot, int ks) {
+#pragma unroll
+            for (int b = 0; b < NB; b++) wf[ks][b] = *reinterpret_cast<const gu4*>(wfp + slot * WS + b * (32 * TL_ROW) + ((ks ^ sw) << 4));
+        };
+        request_a(0, 0); request_w(0);
+#pragma unroll
+        for (int a = 1; a < MU; a++) request_a(0, a);
+        if (steps > 1) {
+            request_a(1, 0); request_w(1);
+#pragma unroll
+            for (int a = 1; a <= HB; a++) request_a(1, a);
+            tl_wait_barrier<N1 + N2>();
+        } else tl_wait_barrier<N2 + NT>();
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) { read_a(0, 0, 0, ks); read_w(0, ks); }
+        auto step = [&](auto par_, int s) {                    // par_: s % 2, the ring slot, and with an odd number of blocks the fragment buffer of block 0
+            constexpr int par = par_(), first = MU % 2 ? par : 0;
+            const bool one = s + 1 < steps, two = s + 2 < steps;
+            if (one) tl_wait_barrier<N1 + N2>(); else tl_wait_barrier<NT>();
+            auto request = [&](int i) {                        // the first barrier's requests in three portions, between products
+                if (i == 0 && one) {
+#pragma unroll
+                    for (int a = HB + 1; a < MU; a++) request_a(1 - par, a);
+                }
+                if (i == 1 && two) request_a(par, 0);
+                if (i == 2 && two) request_w(par);
+            };
+            if (HB == 0) { request(0); request(1); request(2); }
+#pragma unroll
+            for (int a = 0; a < MU; a++) {
+                const int buf = (a + first) & 1;
+                if (a == HB) { if (two) tl_wait_barrier<N1 + N2>(); else if (one) tl_wait_barrier<N2 + NT>(); else tl_wait_barrier<0>(); }
+#pragma unroll
+                for (int ks = 0; ks < 4; ks++) {
+#pragma unroll
+                    for (int b = 0; b < NB; b++) multiply(acc[a][b], af[buf][ks], wf[ks][b]);
+                    if (a + 1 < MU) read_a(buf ^ 1, par, a + 1, ks);
+                    else { read_a(buf ^ 1, 1 - par, 0, ks); read_w(1 - par, ks); }
+                    if (HB > 0 && a == 0) request(ks);
+                    if (a == HB && ks < HB && two) request_a(par, 1 + ks);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        };
+        for (int s = 0; s < steps; s += 2) {
+            step(std::integral_constant<int, 0>{}, s);
+            if (s + 1 < steps) step(std::integral_constant<int, 1>{}, s + 1);
+        }
     };
     using std::integral_constant;
-    if (MB == 1 || blocks == MB) multiply(integral_constant<int, MB>{});
-    else if (MB > 2 && blocks == 3) multiply(integral_constant<int, (MB > 2 ? 3 : 1)>{});
-    else if (MB > 2 && blocks == 2) multiply(integral_constant<int, (MB > 2 ? 2 : 1)>{});
-    else multiply(integral_constant<int, 1>{});
+    if constexpr (MB == 1) whole_slots();
+    else if (blocks == MB) slots_by_parts(integral_constant<int, MB>{});
+    else if (MB > 2 && blocks == 3) slots_by_parts(integral_constant<int, (MB > 2 ? 3 : 1)>{});
+    else if (MB > 2 && blocks == 2) slots_by_parts(integral_constant<int, (MB > 2 ? 2 : 1)>{});
+    else slots_by_parts(integral_constant<int, 1>{});
     if constexpr (GLU) {
         if (pairs) {
             tl_wait_barrier<0>();
@@ -258,6 +321,8 @@ bool kr_sv_gemm_tile_fits(const KrSvGemm& g, bool f32) {
 }
 
 // Which tile: the time of a slot step times how often the chip has to be filled, as measured at K = 2048 - 8192 (us per step of 64 k):
+// (the slots by parts take 15 - 20 % off the two larger tiles, 8 % off the small one: the choice between them is the same, within 4 % of the best of the three at 70 of 77 sizes from 40 to 1500 rows,
+// 1536 to 12416 columns and 600 to 13000 expert rows)
 //   256 x 256, eight waves, one workgroup per compute unit: 2.1 per round of 256 tiles, however empty the last round is
 //   128 x 128, two workgroups per unit: 1.5 per 512 tiles, shares of a round cost their share (the resident workgroups slow one another), at least 0.72
 //   64 x 64, three per unit: 0.4 + 0.7 per 768 tiles: few rows, where the small tile spreads the weight stream over more units

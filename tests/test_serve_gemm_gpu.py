@@ -37,6 +37,13 @@ def test_vocabulary_projection_sizes(want, vocab, width):
     assert np.array_equal(amax, logits.argmax(-1))
 
 
+# slots of the operand ring are given back by parts: 1 - 5 slots of 64 k, last tiles of one to four row blocks (256-row tile) and of one and two (128-row tile)
+@pytest.mark.parametrize("width", [64, 128, 192, 256, 320])
+@pytest.mark.parametrize("want,vocab", [(2050, 7168), (2176, 7168), (2177, 7167), (2300, 7168), (300, 8192), (383, 8191)])
+def test_row_blocks_and_slots(want, vocab, width):
+    test_vocabulary_projection_sizes(want, vocab, width)
+
+
 @pytest.mark.parametrize("n", [1, 2, 5, 8, 9, 16, 17, 40, 65, 130, 420])
 def test_expert_products_sizes(n):
     # 1 - 840 rows on ten experts: row by row, strips for few rows per expert with the activation inside and outside the launch, 64-row tiles

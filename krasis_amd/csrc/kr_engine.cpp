@@ -1048,7 +1048,7 @@ static int moe_prefill_fast(kr_engine* e, Layer& L, const void* x_bf16, const in
         const uint16_t* xc = (const uint16_t*)x_bf16 + (size_t)m0 * H;
         const int32_t* idc = ids + (size_t)m0 * topk; const float* wc = wts + (size_t)m0 * topk;
         const KrPfTiles cut = kr_pfh_tiles(L.w13.view(), L.w2.view(), mc, (long)mc * topk, E);
-        int run = (int)(((long)mc * topk / E + 63) / 64);           // row tiles of an average expert: they share an XCD (one L2 fill of its weights)
+        int run = (int)(((long)mc * topk / E + cut.rows - 1) / cut.rows);           // row tiles of an average expert: they share an XCD (one L2 fill of its weights)
         run = run < 1 ? 1 : (run > 4 ? 4 : run);
         kr_launch_pf_sort(idc, mc, topk, E, so, st, cut);
         kr_launch_pfh_rows_bf16(xc, mc, H, H, (uint16_t*)P.xf.p, (float*)P.xfm.p, st);

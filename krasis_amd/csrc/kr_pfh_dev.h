@@ -144,5 +144,10 @@ __device__ __forceinline__ void pfh_store_tile(const ACC& acc, int nsb, int rows
     }
 }
 
+// kr_prefill_w.hip: tiles of KR_PFW_ROWS rows, whose weights travel wave by wave; mt: tiles of that many rows
+#define KR_PFW_ROWS 96
+bool kr_pfw_dense(const KrPfGemmHArgs& a);      // a dense problem that it takes
+void kr_pfw_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st);
+bool kr_pfr_default();                          // neither of the other two forms is asked for by name (kr_pfr_set_enabled)
 // kr_prefill_ring.hip: the LDS-ring form of the INT4 GEMM; 0 = launched, 1 = this shape stays on the register-staged kernel.  mt64 = 64-row tiles of the experts' tile table
 int kr_pfr_try_launch(const KrPfGemmHArgs& a, int mt64, hipStream_t st);

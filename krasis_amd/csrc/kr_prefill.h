@@ -23,7 +23,7 @@ struct KrPfSort {
 // How the rows of a pass are cut.  `strip` > 0: the sort, which alone knows how many rows every expert has, cuts strips of that many rows instead if those are at most strip_most
 // eighths of the tiles; each of the two forms is launched then, and the one that was not taken finds a count of zero.  max_tiles, max_strips: the most there can be of a form taken (max_tiles 0: strips
 // whatever the rows, nothing else is launched).
-struct KrPfTiles { int rows, strip, strip_most, max_tiles, max_strips; };
+struct KrPfTiles { int rows, strip, strip_most, max_tiles, max_strips; bool wave = false; };      // wave: the tiles are kr_prefill_w.hip's (at most KR_PFW_ROWS rows)
 KrPfTiles kr_pf_cut(int tile_rows, int strip, int strip_most, int tokens, long rows, int E);
 void kr_launch_pf_sort(const int32_t* ids, int M, int topk, int E, KrPfSort s, hipStream_t st, const KrPfTiles& t = KrPfTiles{64, 0, 0, 0, 0});
 void kr_launch_pf_quant_x(const uint16_t* x, int M, int K, int8_t* xh, int8_t* xl, float* xs, hipStream_t st);

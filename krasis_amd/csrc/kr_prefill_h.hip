@@ -700,14 +700,18 @@ static void pfh_strip_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st) {
     const int ncb = (groups + spw - 1) / spw;
     hipLaunchKernelGGL(kr_pfh_strip_kernel, dim3(((mt + 7) / 8) * 8 * ncb), dim3(64 * WAVES), lds, st, a, spw, ncb);
 }
-// How the rows on E experts are cut: strips of 16 may be taken while an expert seldom has more, to 14 rows on average with more than 256 experts, else to ten; 64-row tiles beyond.  A layer's
-// experts, us, tiles alone / this choice where it takes strips: 512 of 2048 x 512, top 10: 48 rows 187 / 136, 160 276 / 196, 400 289 / 239, 700 300 / 276; 64 of 2048 x 1408, top 6: 16 rows 89 / 82, 60 105 / 102,
-// 100 108 / 103; rows an expert, 384 of 2048 x 512 14 231 / 224, 16 230 / 231, 256 of 2048 x 768 12 219 / 208, 14 221 / 228, 128 of 4096 x 1536 8 387 / 308, 12 394 / 393.  The experts' own rows decide (see kr_pf_tiles): with fewer and fewer experts in use strips are the faster ones up to 1.4 times as many as tiles (520 rows, 1.28
-// 284 / 262 us, 1.39 262 / 262, 1.51 229 / 252), hence 11 / 8.  300 tokens on the same ten experts, 48 layers: tiles 13.7 ms, strips 15.4, this choice 13.7.
+// How the rows on E experts are cut.  Evenly spread INT4 rows: strips of 16 up to nine rows an expert with more than 256 experts, seven with fewer, where every expert's weights are met once either way
+// and a strip waits for less; tiles (kr_prefill_w.hip) beyond.  Both products of a layer, us, strips / tiles: 512 experts of 2048 x 512, top 10: 200 tokens 175 / 201, 400 190 / 208,
+// 500 218 / 210, 700 245 / 214; 64 of 2048 x 1408, top 6: 40 tokens 79 / 78, 80 78 / 76, 110 94 / 78; 128 of 4096 x 1536, top 8: 60 tokens 279 / 277, 100 281 / 279, 150 343 / 282.
+// The experts' own rows decide (see kr_pf_tiles), at up to 11 / 8 strips a tile of 64; tiles of 96 where few experts have fewer rows than that.  Under 512 rows in all the tiles, which
+// are taken there only where a handful of experts has them, are kr_pfh_gemm_kernel's of 128 columns, twice as many (48 tokens on 28 experts 49.7 us, 57.8 with half as many; 160 tokens on 38 72 and 69).
 KrPfTiles kr_pfh_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows, int E) {
     const int K = 128 * (m0.ng > m1.ng ? m0.ng : m1.ng);
-    const bool strips = m0.bits == 4 && m1.bits == 4 && !m0.qs && !m1.qs && m0.N % 16 == 0 && m1.N % 16 == 0 && rows <= (E > 256 ? 14L : 10L) * E && pfh_strip_lds(K) <= 160 * 1024;
-    return kr_pf_cut(PFH_BM, strips ? PFH_ST_ROWS : 0, 11, tokens, rows, E);
+    const bool int4 = m0.bits == 4 && m1.bits == 4 && !m0.qs && !m1.qs, wave = int4 && rows >= 512 && kr_pfr_default();
+    const bool strips = int4 && m0.N % 16 == 0 && m1.N % 16 == 0 && rows <= (E > 256 ? 9L : 7L) * E && pfh_strip_lds(K) <= 160 * 1024;
+    KrPfTiles t = kr_pf_cut(wave && rows > (E > 256 ? 14L : 10L) * E ? KR_PFW_ROWS : PFH_BM, strips ? PFH_ST_ROWS : 0, 11, tokens, rows, E);
+    t.wave = wave;
+    return t;
 }
 
 template <int NC, int BITS, int SB = 0, int G = 0, int OCC = 2>
@@ -724,7 +728,8 @@ static void pfh_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st) {
     hipLaunchKernelGGL((kr_pfh_gemm_kernel<NC, BITS, SB, G, OCC>), grid, dim3(256), lds, st, b);
 }
 static void pfh_dispatch(const KrPfGemmHArgs& a, int mt, hipStream_t st) {
-    if (kr_pfr_try_launch(a, mt, st) == 0) return;       // big INT4 problems: the LDS-ring form (bit-identical results)
+    if (kr_pfr_try_launch(a, mt, st) == 0) return;       // the LDS-ring form, where it is asked for (bit-identical results)
+    if (kr_pfw_dense(a)) { kr_pfw_launch(a, (a.total_rows + KR_PFW_ROWS - 1) / KR_PFW_ROWS, st); return; }
     if (a.m.bits == 8) { if (a.m.qs) pfh_launch<1, 8, 0, 1>(a, mt, st); else pfh_launch<1, 8>(a, mt, st); return; }
     // 256-column tiles when they still fill the chip (>= 2 workgroups per CU), else 128-column tiles
     long n128 = (a.m.N + 127) / 128;
@@ -779,6 +784,7 @@ void kr_launch_pfh_gemm(const KrMatDev& m, const uint16_t* a_h, const float* a_m
         pfh_strip_launch(b, t->max_strips, st);
         if (t->max_tiles == 0) return;
     }
+    if (single_expert_rows <= 0 && t && t->wave) { kr_pfw_launch(a, mt, st); return; }
     pfh_dispatch(a, mt, st);
 }
 // gate | up GEMM + activation -> the f16 hidden rows (+ multipliers, + per-32 sums for a Q4_K down copy).  Big problems (the 64 x 256 tile form) with
@@ -789,7 +795,8 @@ void kr_launch_pfh_w13_act(const KrMatDev& m, const uint16_t* a_h, const float* 
                            hipStream_t st, int run, const uint16_t* a_sum32, uint16_t* h_sums32, const KrPfTiles* t) {
     const int I = m.N / 2;
     const int mt = single_expert_rows > 0 ? (single_expert_rows + PFH_BM - 1) / PFH_BM : max_tiles;
-    const bool fuse = !(t && t->strip > 0) && m.bits == 4 && I % 128 == 0 && I <= 2048 && (long)mt * (m.N / 128) >= 2048;
+    const bool wave = t && t->wave;
+    const bool fuse = !(t && t->strip > 0) && m.bits == 4 && I % 128 == 0 && I <= 2048 && (wave || (long)mt * (m.N / 128) >= 2048);
     if (!fuse) {
         kr_launch_pfh_gemm(m, a_h, a_mul, sort, topk, gather_tokens, max_tiles, single_expert_rows, gu, 2 * I, st, 0, 0, run, a_sum32, t);
         kr_launch_pfh_act(gu, rows, I, 2 * I, act_mode, swiglu_limit, alpha, h_out, h_mul, st, h_sums32);
@@ -801,7 +808,7 @@ void kr_launch_pfh_w13_act(const KrMatDev& m, const uint16_t* a_h, const float* 
     a.out = gu; a.out_ld = I; a.single_expert = single_expert_rows > 0; a.total_rows = single_expert_rows;
     a.run = (single_expert_rows > 0 || run < 1) ? 1 : run;
     a.act_fused = act_mode == KR_ACT_GPTOSS ? 2 : (act_mode == KR_ACT_SILU_LIBM ? 3 : 1); a.act_limit = swiglu_limit; a.act_alpha = alpha;
-    if (m.qs) pfh_launch<2, 4, 1, 1>(a, mt, st); else if (kr_pfr_try_launch(a, mt, st) != 0) pfh_launch<2, 4, 1>(a, mt, st);
+    if (wave) kr_pfw_launch(a, mt, st); else if (m.qs) pfh_launch<2, 4, 1, 1>(a, mt, st); else if (kr_pfr_try_launch(a, mt, st) != 0) pfh_launch<2, 4, 1>(a, mt, st);
     const int cpl = I <= 512 ? 1 : (I <= 1024 ? 2 : 4);
 #define KR_ROWW(C_) hipLaunchKernelGGL((kr_pfh_act_wave_kernel<KR_ACT_NONE, C_>), dim3((rows + 3) / 4), dim3(256), 0, st, (const float*)gu, rows, I, I, 0.0f, 0.0f, h_out, h_mul, h_sums32)
     if (rows > 0) { if (cpl == 1) KR_ROWW(1); else if (cpl == 2) KR_ROWW(2); else KR_ROWW(4); }

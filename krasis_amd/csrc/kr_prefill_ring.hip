@@ -426,6 +426,7 @@ static int pfr_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st) {
 // on the experts: both are bound by the 7.8 vector instructions per MFMA of the INT4 -> f16 conversion, profiles/r06_gemm_ring_experiments.txt), 2 = every shape the kernel takes
 static std::atomic<int> g_pfr_on{1};
 void kr_pfr_set_enabled(int on) { g_pfr_on.store(on < 0 ? 0 : (on > 2 ? 2 : on)); }
+bool kr_pfr_default() { return g_pfr_on.load(std::memory_order_relaxed) == 1; }
 int kr_pfr_try_launch(const KrPfGemmHArgs& a, int mt64, hipStream_t st) {
     const int on = g_pfr_on.load(std::memory_order_relaxed);
     const long min_wg = 1;

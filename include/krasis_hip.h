@@ -568,6 +568,10 @@ int kr_serve_free_pages(kr_serve* s, int* n_out);
  * argmax_out: host i32 [n_want] or NULL.  KR_ERR_STATE when the pool has too few free pages (nothing is changed then). */
 int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* counts, const int* tokens, int n_want, const int* want_rows, float* logits_out,
                   int* argmax_out);
+/* Pinned memory that callers hold results in: a step whose logits_out lies in it (16-byte aligned) has its logits stored there by the device, without a copy.  It may outlive the
+ * store; free it when no step writes to it any more, from any thread. */
+int kr_serve_rows_alloc(kr_serve* s, size_t bytes, void** rows_out);
+int kr_serve_rows_free(void* rows);
 /* Steps whose entries all bring one token (decode) replay a hipGraph captured at the second visit of their shape (batch, wanted rows, attention splits,
  * scratch addresses); enable = 0 runs every step eagerly (same kernels, same results).  kr_serve_graph_replays counts the replayed steps. */
 int kr_serve_set_use_graph(kr_serve* s, int enable);

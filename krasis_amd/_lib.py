@@ -30,6 +30,7 @@ SYMBOLS = [
     "kr_serve_create", "kr_serve_destroy", "kr_serve_set_tensor", "kr_serve_fill_synthetic", "kr_serve_finalize", "kr_serve_admit", "kr_serve_release",
     "kr_serve_slot_len", "kr_serve_free_pages", "kr_serve_step", "kr_serve_sample", "kr_serve_set_capture", "kr_serve_read_capture", "kr_serve_device_bytes",
     "kr_serve_set_profiling", "kr_serve_get_profile", "kr_serve_set_use_graph", "kr_serve_graph_replays", "kr_serve_abi",
+    "kr_serve_rows_alloc", "kr_serve_rows_free",
 ]
 TOKEN_CB = C.CFUNCTYPE(C.c_int, C.c_int, C.c_int, C.c_void_p)      # kr_token_cb(token, finish_reason, user) -> continue?
 
@@ -105,6 +106,8 @@ def _bind_serve(lib: C.CDLL) -> None:
     lib.kr_serve_set_use_graph.argtypes = [vp, ci]
     lib.kr_serve_graph_replays.argtypes = [vp]; lib.kr_serve_graph_replays.restype = C.c_long
     lib.kr_serve_abi.argtypes = []
+    lib.kr_serve_rows_alloc.argtypes = [vp, C.c_size_t, C.POINTER(vp)]
+    lib.kr_serve_rows_free.argtypes = [vp]
 
 
 def load_serve_library(build: bool = False) -> C.CDLL:

@@ -9,6 +9,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -315,6 +317,19 @@ int host_out(kr_serve* s, size_t bytes) {
     KR_HIP(hipHostMalloc(&s->h_out, bytes, hipHostMallocMapped | hipHostMallocCoherent));
     s->h_out_bytes = bytes;
     return KR_OK;
+}
+// Memory that callers hold results in (kr_serve_rows_alloc): a step stores logits there itself.  It may outlive its store, and be given back from another thread.
+struct RowsBlock { size_t bytes; int device; char* dev; };
+std::mutex rows_mu;
+std::map<char*, RowsBlock> rows_blocks;
+// the device's address of `bytes` at p in such memory of this device, or null
+char* rows_device_ptr(const void* p, size_t bytes, int device) {
+    std::lock_guard<std::mutex> g(rows_mu);
+    auto it = rows_blocks.upper_bound((char*)p);
+    if (it == rows_blocks.begin()) return nullptr;
+    --it;
+    const size_t at = (size_t)((char*)p - it->first);
+    return it->second.device == device && at + bytes <= it->second.bytes && ((uintptr_t)p & 15) == 0 ? it->second.dev + at : nullptr;
 }
 // scratch of the step's last launch, zero before its first use (the launch leaves it so)
 int finish_scratch(kr_serve* s, int rows) {
@@ -937,6 +952,30 @@ int kr_serve_finalize(kr_serve* s) {
 
 int kr_serve_abi(void) { return KR_SERVE_ABI; }
 
+int kr_serve_rows_alloc(kr_serve* s, size_t bytes, void** rows_out) {
+    if (!s || !rows_out || !bytes) return kr_fail(KR_ERR_VALUE, "bad argument");
+    *rows_out = nullptr;
+    KR_HIP(hipSetDevice(s->device));
+    void *p = nullptr, *d = nullptr;
+    KR_HIP(hipHostMalloc(&p, bytes, hipHostMallocMapped | hipHostMallocCoherent));
+    if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess) { (void)hipHostFree(p); return kr_fail(KR_ERR_HIP, "no device address of %zu pinned bytes", bytes); }
+    try {
+        std::lock_guard<std::mutex> g(rows_mu);
+        rows_blocks[(char*)p] = {bytes, s->device, (char*)d};
+    } catch (...) { (void)hipHostFree(p); return kr_fail(KR_ERR_STATE, "out of host memory"); }
+    *rows_out = p;
+    return KR_OK;
+}
+int kr_serve_rows_free(void* rows) {
+    if (!rows) return KR_OK;
+    {
+        std::lock_guard<std::mutex> g(rows_mu);
+        if (!rows_blocks.erase((char*)rows)) return kr_fail(KR_ERR_VALUE, "not from kr_serve_rows_alloc");
+    }
+    KR_HIP(hipHostFree(rows));
+    return KR_OK;
+}
+
 int kr_serve_admit(kr_serve* s, int* slot_out) {
     if (!s || !slot_out) return kr_fail(KR_ERR_VALUE, "null argument");
     for (size_t i = 0; i < s->slots.size(); i++) if (!s->slots[i].live) { s->slots[i].live = true; s->slots[i].len = 0; s->slots[i].last_token = -1; *slot_out = (int)i; return KR_OK; }
@@ -998,7 +1037,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     for (int i = 0; i < n_want; i++) if (want_rows[i] < 0 || want_rows[i] >= T) return kr_fail(KR_ERR_VALUE, "wanted row %d of %d", want_rows[i], T);
     if (need_pages > (int)s->free_pages.size()) return kr_fail(KR_ERR_STATE, "cache pool exhausted: %d pages needed, %zu free", need_pages, s->free_pages.size());
     // ---- per-step arrays: tokens | slot | pos | want | page table
-    const size_t n_meta = (size_t)5 * T + n_want + 3 * (size_t)n_entries + 2;      // ... | first row of every entry and the end | slot of every entry | first 64-token block of every entry and the end | tokens, those of short entries first
+    const size_t n_own = ((size_t)5 * T + n_want + 3 * (size_t)n_entries + 2 + 1) / 2 * 2, n_meta = n_own + 2;      // behind them, in two words, where the logits go; ... | first row of every entry and the end | slot of every entry | first 64-token block of every entry and the end | tokens, those of short entries first
     const size_t meta_bytes = (n_meta + s->h_table.size()) * 4;      // (a launch may copy up to twelve bytes more)
     if (meta_bytes + 16 > s->h_meta_bytes) {
         if (s->h_meta) (void)hipHostFree(s->h_meta);
@@ -1038,6 +1077,18 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         std::memcpy(h_tab, s->h_table.data(), s->h_table.size() * 4);
     }
     if (s->meta.ensure(meta_bytes + 16)) return kr_fail(KR_ERR_HIP, "step arrays");
+    // results: the step's last launch stores them to pinned host memory, the logits to the caller's where that is the kind (kr_serve_rows_alloc), else to the store's, from where they are
+    // copied.  (A prompt whose logits are all wanted may have more than the store keeps: copied from the device then)
+    const size_t row_bytes = (size_t)n_want * c.vocab * 4;
+    char* const direct = n_want > 0 && logits_out ? rows_device_ptr(logits_out, row_bytes, s->device) : nullptr;
+    const bool want_amax = n_want > 0 && argmax_out, host_logits = n_want > 0 && logits_out && (direct || row_bytes <= HOST_OUT_MOST);
+    const size_t amax_bytes = ((size_t)n_want * 4 + 255) / 256 * 256;
+    void* dev_out = nullptr;
+    if (want_amax || host_logits) {
+        { const int rc = host_out(s, amax_bytes + (host_logits && !direct ? row_bytes : 0)); if (rc) return rc; }
+        KR_HIP(hipHostGetDevicePointer(&dev_out, s->h_out, 0));
+    }
+    { const uint64_t to = (uint64_t)(uintptr_t)(direct ? direct : host_logits ? (char*)dev_out + amax_bytes : nullptr); std::memcpy(hm + n_own, &to, 8); }
     hipStream_t st = s->st;
     // decode-sized steps: a launch reads the arrays from the host memory they stand in and forms the rotation tables; larger arrays (whose words a launch would wait for one
     // by one over the link) take a copy command
@@ -1142,15 +1193,6 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
             plan[li].nsplit = kr_sv_step_join_splits(T, d.heads, d.kv_heads, plan[li].keys, W, d.expert_ff, d.experts, d.top);
         }
         if (plan[li].parts && (s->part_ml.ensure(plan[li].parts * 8) || s->part_acc.ensure(plan[li].parts * l.att_vdim() * 4))) return kr_fail(KR_ERR_HIP, "attention split scratch");
-    }
-    // results: the step's last launch stores them to pinned host memory.  (A prompt whose logits are all wanted may have more than it
-    // is given: copied from the device then)
-    const bool want_amax = n_want > 0 && argmax_out, host_logits = n_want > 0 && logits_out && (size_t)n_want * c.vocab * 4 <= HOST_OUT_MOST;
-    const size_t amax_bytes = ((size_t)n_want * 4 + 255) / 256 * 256, out_bytes = amax_bytes + (host_logits ? (size_t)n_want * c.vocab * 4 : 0);
-    void* dev_out = nullptr;
-    if (want_amax || host_logits) {
-        { const int rc = host_out(s, out_bytes); if (rc) return rc; }
-        KR_HIP(hipHostGetDevicePointer(&dev_out, s->h_out, 0));
     }
     float* x = (float*)s->x.p;
     const int NG = c.norm_groups > 1 ? c.norm_groups : 1;
@@ -1576,7 +1618,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     }
     if (n_want > 0) {
         const bool scaled = c.logit_scale != 0.0f && c.logit_scale != 1.0f;
-        float* host_rows = host_logits ? (float*)((char*)dev_out + amax_bytes) : nullptr;
+        float* const* host_rows = host_logits ? (float* const*)(d_tok + n_own) : nullptr;
         { Timer tm(s, 0); kr_sv_norm(x, d_want, (const float*)s->fnorm_w.p, c.norm_bias ? (const float*)s->fnorm_b.p : nullptr, s->hw.p, s->f32, n_want, W, c.norm_eps, c.norm_kind, NG, nullptr, st); }
         KrSvGemm g{}; g.A = s->hw.p; g.lda = W; g.W = s->head.p; g.C = (float*)s->logits.p; g.ldc = c.vocab; g.M = n_want; g.N = c.vocab; g.K = W;
         if (host_logits && !scaled && kr_sv_gemm_takes_host(g, s->f32)) { g.c_host = host_rows; host_rows = nullptr; }
@@ -1623,14 +1665,13 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         if (exec) { KR_HIP(hipGraphLaunch(exec, st)); s->graph_replays++; done = true; }
     }
     if (!done) { const int rc = enqueue(); if (rc) return rc; }
-    const size_t row_bytes = (size_t)n_want * c.vocab * 4;
     if (n_want > 0 && logits_out && !host_logits) KR_HIP(hipMemcpyAsync(logits_out, s->logits.p, row_bytes, hipMemcpyDeviceToHost, st));
     // the caller's pages are brought in while the launches run (fresh memory: a fault per page), not in the copy after them
-    if (host_logits) for (size_t i = 0; i < row_bytes; i += 4096) ((volatile char*)logits_out)[i] = 0;
+    if (host_logits && !direct) for (size_t i = 0; i < row_bytes; i += 4096) ((volatile char*)logits_out)[i] = 0;
     s->last_want = n_want;
     KR_HIP(hipStreamSynchronize(st));
     if (want_amax) std::memcpy(argmax_out, s->h_out, (size_t)n_want * 4);
-    if (host_logits) std::memcpy(logits_out, (const char*)s->h_out + amax_bytes, row_bytes);
+    if (host_logits && !direct) std::memcpy(logits_out, (const char*)s->h_out + amax_bytes, row_bytes);
     KR_HIP(hipGetLastError());
     return KR_OK;
 }

@@ -16,7 +16,7 @@ __device__ __forceinline__ float gm_ld(const float* p) { return *p; }
 __device__ __forceinline__ float gm_ld(const uint16_t* p) { return kr_bf16_to_f32(*p); }
 // one element of C: f32, or the storage type when the output feeds another GEMM as it is (BF = a bf16 store)
 template <bool BF>
-__device__ __forceinline__ void gm_store(const KrSvGemm& g, int m, int n, float v) {
+__device__ __forceinline__ void gm_store(const KrSvGemm& g, int m, int n, float v, float* host = nullptr) {
     const int row = g.c_rows ? g.c_rows[m] : m;
     const size_t i = (size_t)row * g.ldc + n;
     if (g.bias) v += g.bias[n];
@@ -25,10 +25,12 @@ __device__ __forceinline__ void gm_store(const KrSvGemm& g, int m, int n, float 
     if (BF && g.c_storage) ((uint16_t*)g.C)[i] = kr_f32_to_bf16(v);
     else {
         g.C[i] = v;
-        if (BF && g.c_host) g.c_host[i] = v;
+        if (BF && host) host[i] = v;
     }
 }
 
+// where a step's arrays say that its results go (KrSvGemm::c_host, sv_finish); a scalar load: the word does not change while a launch runs
+__device__ __forceinline__ float* gm_host(float* const* at) { return at ? (float*)*(const __attribute__((address_space(4))) uint64_t*)(uintptr_t)at : nullptr; }
 // columns of group `group`: all N, or what the group's own matrix has
 __device__ __forceinline__ int gm_cols(const KrSvGemm& g, int group) { return g.n_last > 0 ? (group == g.n_groups - 1 ? g.n_last : g.n_first) : g.N; }
 

@@ -33,7 +33,7 @@ struct KrSvGemm {
     int n_first;                     //   ... and the other groups' matrices have n_first
     // with act_gu: the up columns come from a table instead: element k of problem row r is up_tab[up_rows[r] * up_ld + up_off + k] (storage type)
     const void* up_tab; const int* up_rows; int up_ld, up_off;
-    float* c_host;                   // only where kr_sv_gemm_takes_host says so: C once more, in pinned host memory
+    float* const* c_host;            // only where kr_sv_gemm_takes_host says so: C once more, in the pinned host memory whose address stands at this device address
     // only where kr_sv_gemm_takes_glu says so: columns [glu_lo, glu_lo + glu_f) are gates and the glu_f columns behind them their up factors; they do not go to C but, as the
     // gated activation (of both times glu_row_w[m], if given), to glu_out [M, glu_f] in the storage type, by problem row
     void* glu_out; int glu_lo, glu_f, glu_kind; float glu_limit, glu_alpha; const float* glu_row_w;
@@ -381,6 +381,6 @@ void kr_sv_delta_prep(const KrSvDelta& a, hipStream_t st);
 void kr_sv_row_out(const float* o, int n, const float* w, const float* gate, int gate_ld, float eps, float scale, void* out, int out_ld, bool f32, int T, hipStream_t st);
 // rows of logits and their largest entries to pinned host memory (either may be null).  scratch: kr_sv_finish_bytes, zero before its first use and left zero
 inline size_t kr_sv_finish_bytes(int R) { return (size_t)R * 12; }
-void kr_sv_finish(const float* logits, int R, int vocab, float* host_logits, int* host_argmax, void* scratch, hipStream_t st);
+void kr_sv_finish(const float* logits, int R, int vocab, float* const* host_logits /* as KrSvGemm::c_host */, int* host_argmax, void* scratch, hipStream_t st);
 // uniform values in [-amp, amp) from a counter hash of (seed, element); amp = 0 writes zeros
 void kr_sv_fill_uniform(void* p, bool f32, size_t n, uint64_t seed, float amp, hipStream_t st);

@@ -2290,12 +2290,13 @@ __global__ void __launch_bounds__(256) sv_ssd_out_kernel(const KrSvSsdOut a, T* 
 // The end of a step, many workgroups per row: the row's largest entry (the lowest index of equals; NaN never), and the row itself, to pinned host memory.  Two copy commands and
 // the host's wait for each took 40 us after this launch, 100 with 1.5 MB of logits; the stores here cross the link beside the search.
 // best: value in order of size and index in one word, 0 = none yet; the last workgroup of a row hands the result on and leaves best and done as it found them.
-__global__ void __launch_bounds__(256) sv_finish_kernel(const float* __restrict__ logits, int vocab, int chunk, float* __restrict__ host_logits, int* __restrict__ host_argmax,
+__global__ void __launch_bounds__(256) sv_finish_kernel(const float* __restrict__ logits, int vocab, int chunk, float* const* host_logits, int* __restrict__ host_argmax,
                                                         unsigned long long* __restrict__ best, unsigned* __restrict__ done) {
     __shared__ unsigned long long bw[4];
     const int r = blockIdx.x, c0 = blockIdx.y * chunk, c1 = min(vocab, c0 + chunk);
     const float* row = logits + (size_t)r * vocab;
-    float* to = host_logits ? host_logits + (size_t)r * vocab : nullptr;
+    float* to = gm_host(host_logits);
+    if (to) to += (size_t)r * vocab;
     unsigned long long b = 0;
     auto see = [&](float x, int c) {
         if (x != x) return;
@@ -2763,7 +2764,7 @@ void kr_sv_lin_out(const KrSvLin& a, bool f32, hipStream_t st) {
     else hipLaunchKernelGGL(sv_lin_out_kernel<uint16_t>, dim3(a.T, a.heads), dim3(64), 0, st, a, (uint16_t*)a.out);
 }
 
-void kr_sv_finish(const float* logits, int R, int vocab, float* host_logits, int* host_argmax, void* scratch, hipStream_t st) {
+void kr_sv_finish(const float* logits, int R, int vocab, float* const* host_logits, int* host_argmax, void* scratch, hipStream_t st) {
     if (R <= 0 || (!host_logits && !host_argmax)) return;
     const int nb = std::min(32, (vocab + 1023) / 1024), chunk = ((vocab + nb - 1) / nb + 3) / 4 * 4;
     hipLaunchKernelGGL(sv_finish_kernel, dim3(R, nb), dim3(256), 0, st, logits, vocab, chunk, host_logits, host_argmax, (unsigned long long*)scratch, (unsigned*)((unsigned long long*)scratch + R));

@@ -26,6 +26,7 @@ __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const 
         W += (size_t)group * g.w_stride; N = gm_cols(g, group);
     }
     if (n0 >= (GLU ? g.glu_f : N)) return;
+    float* host = gm_host(g.c_host);
     const int ks = g.K / 32, s0 = ks * wave / WV, s1 = ks * (wave + 1) / WV, lda = g.K + 8;
     const uint16_t* wp[NB];
 #pragma unroll
@@ -119,7 +120,7 @@ __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const 
                 float v = red[t * 256 + e];
 #pragma unroll
                 for (int w = 1; w < WV; w++) v += red[(w * TR + t) * 256 + e];
-                gm_store<true>(g, m, n, v);
+                gm_store<true>(g, m, n, v, host);
             }
         }
         if (m0 + 16 * MB < hi) __syncthreads();

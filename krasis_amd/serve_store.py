@@ -5,6 +5,8 @@ Slots and pages are managed by the library (`admit` / `release`); nothing here c
 from __future__ import annotations
 
 import ctypes as C
+import sys
+from collections import deque
 from dataclasses import dataclass, fields
 from typing import List, Optional, Sequence, Tuple
 
@@ -117,6 +119,57 @@ class LayerSpec:
     lt_vdim: int = 0
 
 
+class _Slab:
+    """Pinned memory of the library, given back with its last reference."""
+    def __init__(self, lib, handle, nbytes: int):
+        self._lib, self.ptr = lib, C.c_void_p()
+        check_serve(lib.kr_serve_rows_alloc(handle, nbytes, C.byref(self.ptr)))
+
+    def __del__(self):
+        if getattr(self, "ptr", None) and not sys.is_finalizing():
+            self._lib.kr_serve_rows_free(self.ptr)
+
+
+class _Lease:
+    """A block of a slab under one returned array: back to the pool's free blocks when the array and all its views are gone."""
+    def __init__(self, free: deque, slab: _Slab, at: int):
+        self.free, self.slab, self.at = free, slab, at
+
+    def __del__(self):
+        if self.slab.ptr:
+            self.free.append((self.slab, self.at))
+
+
+class _RowPool:
+    """Arrays for logits in memory that the device stores to itself: the copy out of the store's own results was 50 us for twelve rows of 32768, and fresh pages for it a fault each.
+    Blocks are powers of two; MOST bytes per store at a time, then None (the caller takes ordinary memory and the copy).  Blocks change hands by deque operations alone, so arrays may
+    be dropped on any thread; a slab lives as long as the pool or one of its arrays."""
+    MOST, LEAST, LARGEST = 128 << 20, 64 << 10, 32 << 20
+
+    def __init__(self, lib):
+        self._lib, self._free, self._bytes = lib, {}, 0
+
+    def take(self, handle, rows: int, cols: int) -> Optional[np.ndarray]:
+        size = self.LEAST
+        while size < rows * cols * 4:
+            size *= 2
+        if size > self.LARGEST:
+            return None
+        free = self._free.setdefault(size, deque())
+        try:
+            slab, at = free.popleft()
+        except IndexError:
+            nbytes = max(size, min(16 * size, self.LARGEST))
+            if self._bytes + nbytes > self.MOST:
+                return None
+            slab, at = _Slab(self._lib, handle, nbytes), 0
+            self._bytes += nbytes
+            free.extend((slab, o) for o in range(size, nbytes, size))
+        block = (C.c_float * (rows * cols)).from_address(slab.ptr.value + at)
+        block.lease = _Lease(free, slab, at)
+        return np.frombuffer(block, np.float32).reshape(rows, cols)
+
+
 class ServeStore:
     def __init__(self, vocab: int, width: int, layers: Sequence[LayerSpec], dtype: int = BF16, norm_kind: int = NORM_LAYER, norm_eps: float = 1e-5,
                  max_slots: int = 4, pool_tokens: int = 4096, page_tokens: int = PAGE_TOKENS, device: int = 0, build: bool = False,
@@ -138,12 +191,14 @@ class ServeStore:
             for f in fields(LayerSpec):
                 setattr(arr[i], f.name, getattr(l, f.name))
         self._h = C.c_void_p()
+        self._rows = _RowPool(self._lib)
         check_serve(self._lib.kr_serve_create(device, C.byref(cfg), arr, C.byref(self._h)))
 
     def close(self) -> None:
         if getattr(self, "_h", None):
             self._lib.kr_serve_destroy(self._h)
             self._h = None
+            self._rows = None                       # (arrays that are still held keep their slabs)
 
     def __del__(self):
         try:
@@ -196,7 +251,9 @@ class ServeStore:
         counts = np.asarray([len(e[1]) for e in entries], np.int32)
         toks = np.ascontiguousarray(np.concatenate([np.asarray(e[1], np.int32).reshape(-1) for e in entries]) if entries else np.zeros(0, np.int32))
         want = np.asarray(list(want_rows), np.int32)
-        out = np.empty((len(want), self.vocab), np.float32) if logits else None
+        out = self._rows.take(self._h, len(want), self.vocab) if logits and len(want) and self._h else None
+        if logits and out is None:
+            out = np.empty((len(want), self.vocab), np.float32)
         amax = np.empty(len(want), np.int32)
         check_serve(self._lib.kr_serve_step(self._h, len(entries), slots.ctypes.data, counts.ctypes.data, toks.ctypes.data, len(want), want.ctypes.data if len(want) else None,
                                             out.ctypes.data if (logits and len(want)) else None, amax.ctypes.data if len(want) else None))

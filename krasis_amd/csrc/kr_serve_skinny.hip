@@ -15,18 +15,19 @@
 #include "kr_serve_strip_dev.h"
 
 namespace {
-template <int MB, int NB, int WV, bool ACT>
+template <int MB, int NB, int WV, bool ACT, int U>
 __global__ void __launch_bounds__(64 * WV) sv_skinny_kernel(const KrSvGemm g) {
     __shared__ __attribute__((aligned(16))) float red[sk_red_floats(MB, NB, WV)];
     extern __shared__ __attribute__((aligned(16))) uint16_t act[];
-    sk_strip<MB, NB, WV, ACT>(g, blockIdx.x, blockIdx.y, red, act);
+    sk_strip<MB, NB, WV, ACT, false, U>(g, blockIdx.x, blockIdx.y, red, act);
 }
 // the experts' and the shared expert's down projection of a step in one launch, both with the activation inside: neither fills the chip, and a launch with its gap costs more
 // than the smaller of the two (six expert rows and one row, 2048 x 768: 8.1 + 6.3 -> 8.7 us)
+template <int U>
 __global__ void __launch_bounds__(256) sv_skinny_pair_kernel(const KrSvGemm e, const KrSvGemm o) {
     __shared__ __attribute__((aligned(16))) float red[sk_red_floats(1, 1, 4)];
     extern __shared__ __attribute__((aligned(16))) uint16_t act[];
-    if (blockIdx.y == 0) sk_strip<1, 1, 4, true>(o, blockIdx.x, 0, red, act); else sk_strip<1, 1, 4, true>(e, blockIdx.x, blockIdx.y - 1, red, act);
+    if (blockIdx.y == 0) sk_strip<1, 1, 4, true, false, U>(o, blockIdx.x, 0, red, act); else sk_strip<1, 1, 4, true, false, U>(e, blockIdx.x, blockIdx.y - 1, red, act);
 }
 
 // Up to three products of the same rows in one launch, the last one the gate | up pairs of a feed-forward that leave as their activation.  A launch with its gap
@@ -45,14 +46,26 @@ __global__ void __launch_bounds__(256) sv_strips_kernel(const KrSvGemm a, const 
 
 int sk_act_lds(const KrSvGemm& g) { return (g.row_group ? 16 : std::min(16, g.M)) * (g.K + 8) * 2; }      // one block of sixteen rows
 
-template <int MB, int NB, int WV>
-void sk_launch(const KrSvGemm& g, hipStream_t st) {
+template <int MB, int NB, int WV, int U>
+void sk_launch_u(const KrSvGemm& g, hipStream_t st) {
     const dim3 grid((g.N + 16 * NB - 1) / (16 * NB), g.row_group ? g.M : 1);
     if (g.act_gu) {
         const int rows = g.row_group ? 16 * MB : std::min(16 * MB, g.M), lds = rows * (g.K + 8) * 2;
-        if (kr_lds_optin((const void*)sv_skinny_kernel<MB, NB, WV, true>, lds)) return;
-        hipLaunchKernelGGL((sv_skinny_kernel<MB, NB, WV, true>), grid, dim3(64 * WV), lds, st, g);
-    } else hipLaunchKernelGGL((sv_skinny_kernel<MB, NB, WV, false>), grid, dim3(64 * WV), 0, st, g);
+        if (kr_lds_optin((const void*)sv_skinny_kernel<MB, NB, WV, true, U>, lds)) return;
+        hipLaunchKernelGGL((sv_skinny_kernel<MB, NB, WV, true, U>), grid, dim3(64 * WV), lds, st, g);
+    } else hipLaunchKernelGGL((sv_skinny_kernel<MB, NB, WV, false, U>), grid, dim3(64 * WV), 0, st, g);
+}
+template <int MB, int NB, int WV>
+void sk_launch(const KrSvGemm& g, hipStream_t st) {
+    switch (sk_steps(g.K, WV)) {
+        case 4: sk_launch_u<MB, NB, WV, 4>(g, st); break;
+        case 6: sk_launch_u<MB, NB, WV, 6>(g, st); break;
+        default: sk_launch_u<MB, NB, WV, 8>(g, st); break;
+    }
+}
+template <int U> void sk_pair_launch(const KrSvGemm& e, const KrSvGemm& o, int lds, hipStream_t st) {
+    if (kr_lds_optin((const void*)sv_skinny_pair_kernel<U>, lds)) return;
+    hipLaunchKernelGGL(sv_skinny_pair_kernel<U>, dim3((std::max(e.N, o.N) + 15) / 16, e.M + 1), dim3(256), lds, st, e, o);
 }
 }  // namespace
 
@@ -82,8 +95,11 @@ void kr_sv_gemm_skinny_pair(const KrSvGemm& e, const KrSvGemm& o, hipStream_t st
     KrSvGemm p = o;
     p.row_group = nullptr;
     const int lds = std::max(sk_act_lds(e), sk_act_lds(p));
-    if (kr_lds_optin((const void*)sv_skinny_pair_kernel, lds)) return;
-    hipLaunchKernelGGL(sv_skinny_pair_kernel, dim3((std::max(e.N, o.N) + 15) / 16, e.M + 1), dim3(256), lds, st, e, p);
+    switch (sk_steps(e.K, 4)) {
+        case 4: sk_pair_launch<4>(e, p, lds, st); break;
+        case 6: sk_pair_launch<6>(e, p, lds, st); break;
+        default: sk_pair_launch<8>(e, p, lds, st); break;
+    }
 }
 
 bool kr_sv_strips_fits(const KrSvGemm& g) { return g.M > 0 && g.M <= 16 && !g.seg && !g.act_gu && !g.c_rows && !g.c_host && kr_sv_gemm_skinny_fits(g); }

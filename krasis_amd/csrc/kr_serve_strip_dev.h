@@ -8,12 +8,19 @@ typedef float sk_f4 __attribute__((ext_vector_type(4)));
 
 constexpr int sk_red_floats(int MB, int NB, int WV) { return WV * (MB * NB < 4 ? MB * NB : 4) * 256; }
 
+// k steps requested together: the count that leaves the fewest requests of no use behind a wave's last step (they are made all the same, for the last step's bytes again).  Eight where
+// six do, with 12 rows on 64 experts of 768 x 2048, 36.5 us where 27.7 do; 24 on 128 of 1536 x 4096 61 and 52.
+constexpr int sk_steps(int K, int WV) {
+    const int steps = (K / 32 + WV - 1) / WV;
+    int best = 8;
+    for (int u : {6, 4}) if ((steps + u - 1) / u * u < (steps + best - 1) / best * best) best = u;
+    return best;
+}
 // MB, NB: row and column blocks of 16; WV: waves.  bx: strip, by: problem row of a grouped problem; red: sk_red_floats of LDS, act (with ACT): the rows' activation [16 MB][K + 8].
 // GLU (NB = 2): the strip is 16 gate columns, counted from g.glu_lo, and the 16 up columns that belong to them; their activation goes to g.glu_out, nothing to C.
-template <int MB, int NB, int WV, bool ACT, bool GLU = false>
+template <int MB, int NB, int WV, bool ACT, bool GLU = false, int U = NB * MB <= 2 ? 8 : 4>      // U: k steps requested together
 __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const int by, float* red, uint16_t* act) {
     static_assert(!GLU || (NB == 2 && MB == 1), "a gate tile and its up tile");
-    constexpr int U = NB * MB <= 2 ? 8 : 4;                   // k steps requested together
     constexpr int TR = MB * NB < 4 ? MB * NB : 4;             // output tiles per round of the reduction
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4, n0 = bx * 16 * (GLU ? 1 : NB);
     int lo = 0, hi = g.M, N = g.N;

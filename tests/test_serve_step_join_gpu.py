@@ -99,3 +99,19 @@ def test_every_mechanism_of_a_joined_layer(name):
     got, ref = np.concatenate([got, last[:, None]], 1), np.stack(ref).astype(np.float64)
     e = np.sqrt(((got - ref) ** 2).mean(-1)) / np.sqrt((ref ** 2).mean())
     assert np.median(e) < 2e-2 and (e < 4e-2).mean() >= 0.9, (name, e)
+
+
+@pytest.mark.parametrize("requests", [2, 12])
+@pytest.mark.parametrize("ff", [96, 384, 640, 768, 1024, 1408])
+def test_steps_of_k_requested_together(ff, requests):
+    """a wave's share of the down projections is 1, 3, 5, 6, 8 and 11 steps of 32 k, requested four, six or eight at a time, beside attention's projection six or eight at a time (few and
+    many expert rows); the prompts' fifteen and sixty rows meet the same strips in launches of their own"""
+    cfg = O.make_config(width=256, vocab=50, eps=1e-5, layers=[{"type": "attention", "mixer": O.attn(4, 2, 64, 64, 0, 0, scale=0.12), "mlp": O.moe(10, 2, 1, 1, ff, 1.5, ff, 1.5)}])
+    W = O.random_weights(cfg, 21)
+    seqs = [tokens(cfg, 8, 70 + r) for r in range(requests)]
+    eng = engine(cfg, W, "bfloat16", max_slots=requests)
+    first = eng.step([(r, s[:5], [4]) for r, s in enumerate(seqs)])[0]
+    got = np.stack([first] + [eng.step([(r, [s[5 + i]], [0]) for r, s in enumerate(seqs)])[0] for i in range(3)], 1)
+    ref = np.stack([O.forward(cfg, W, s)[0][4:] for s in seqs])
+    e = np.sqrt(((got - ref) ** 2).mean(-1)) / np.sqrt((ref ** 2).mean())
+    assert np.median(e) < 2e-2 and (e < 4e-2).mean() >= 0.9, (ff, requests, e)

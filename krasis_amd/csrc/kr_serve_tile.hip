@@ -1,5 +1,5 @@
-// kr_serve_tile.hip -- C[M, N] = A[M, K] x W[N, K]^T for prompt-sized problems, single matrix or one matrix per expert: a bf16 store's on v_mfma_f32_32x32x16_bf16, an f32
-// store's on v_mfma_f32_32x32x2_f32.
+// kr_serve_tile.hip -- C[M, N] = A[M, K] x W[N, K]^T for prompt-sized problems, single matrix or one matrix per expert, of a bf16 store (an f32 store's:
+// kr_serve_tile_f32.hip).
 //
 // Bound: the matrix cores (about 1350 TFLOP/s is what a large library product reaches here; nominal 2500).  Both operands travel from memory to LDS by
 // global_load_lds_dwordx4 into a ring of slots of 64 k (no staging registers; whole cache lines), fragments read while products run.  What the large tile buys:
@@ -19,29 +19,17 @@
 #include <type_traits>
 
 #include "kr_lds_optin.h"
-#include "kr_serve_gemm_dev.h"
+#include "kr_serve_tile_dev.h"
 
 namespace {
-constexpr int TL_ROW = 128;                                    // bytes of a slot's row, whole cache lines (rows of 64 bytes fetch every line twice): 64 k in bf16, 32 in f32
-
-__device__ __forceinline__ uint32_t tl_lds_addr(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p; }
-// 64 lanes x 16 bytes from the lane's own address to lds_dst (wave-uniform) + 16 lane.  M0 is the compiler's register: saved and restored inside.  The compiler
-// does not count this request; the waits below do.
-__device__ __forceinline__ void tl_dma16(uint32_t lds_dst, const void* src) {
-    unsigned keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(src), "s"(lds_dst) : "memory");
-}
-// at most N of this wave's requests are outstanding and its LDS reads have returned, then the workgroup barrier
-template <int N> __device__ __forceinline__ void tl_wait_barrier() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory"); }
-
 // GLU: columns [glu_lo, glu_lo + 2 glu_f) leave as the gated activation.  Their tiles come behind those of the other columns (the column numbers of those close the gap): half a
 // tile of gates and the up columns that belong to them, laid out so that a wave holds both factors of its elements.  The f32 pair is not written and read again and
 // the activation's launch is gone: 24576 rows of 2 x 768 on 64 experts, product and activation, 242 + 55 -> 252 us; a 4096-token prompt of four layers 4.06 -> 3.80 ms.
-template <typename T, int BM, int BN, int WM, int WN, int DEPTH, int WPS, bool GLU>  // WM x WN waves; WPS: waves per SIMD the register budget is for
+template <int BM, int BN, int WM, int WN, int DEPTH, int WPS, bool GLU>  // WM x WN waves; WPS: waves per SIMD the register budget is for
 __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGemm g) {
     constexpr int MB = BM / (32 * WM), NB = BN / (32 * WN);    // 32 x 32 blocks of a wave
     constexpr int RA = 4 / WN, RW = 4 * NB / WM;               // requests of 8 rows that a wave makes for a row block of A's slot and for W's slot
-    constexpr int BK = TL_ROW / (int)sizeof(T), CH = 16 / (int)sizeof(T);     // k of a slot, elements of a chunk
+    constexpr int BK = TL_ROW / 2, CH = 8;                     // k of a slot, elements of a chunk
     constexpr uint32_t AS = BM * TL_ROW, WS = BN * TL_ROW;     // bytes of a slot of A and of W: A's slots come first
     extern __shared__ __attribute__((aligned(1024))) uint8_t ring_[];
     int bx = blockIdx.x, by = blockIdx.y;
@@ -60,10 +48,10 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
     const int n0 = GLU ? (pairs ? (bx - plain_tiles) * (BN / 2) : bx * BN) : bx * BN, N = GLU ? (pairs ? g.glu_f : plain) : gm_cols(g, group);
     if (n0 >= N) return;
     auto column = [&](int n) { return GLU && n >= g.glu_lo ? n + 2 * g.glu_f : n; };         // of C and row of W, of a column outside the pairs
-    const T* A = (const T*)g.A;
-    const T* W = (const T*)g.W + (size_t)group * g.w_stride;
+    const uint16_t* A = (const uint16_t*)g.A;
+    const uint16_t* W = (const uint16_t*)g.W + (size_t)group * g.w_stride;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5, wr = wave / WN, wc = wave % WN;
-    const T* as[MB][RA]; const T* ws[RW];
+    const uint16_t* as[MB][RA]; const uint16_t* ws[RW];
 #pragma unroll
     for (int a = 0; a < MB; a++)
 #pragma unroll
@@ -107,11 +95,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
     const uint8_t* afp = ring_ + (wr * 32 + r) * TL_ROW;
     const uint8_t* wfp = ring_ + DEPTH * AS + (wc * (BN / WN) + r) * TL_ROW;
     auto multiply = [&](gv16f& c, const gu4& fa, const gu4& fb) {
-        if constexpr (sizeof(T) == 2) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(gb8, fa), __builtin_bit_cast(gb8, fb), c, 0, 0, 0);
-        else {                                                 // a chunk is four steps of 2 k, one per half
-#pragma unroll
-            for (int e = 0; e < 4; e++) c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fa[e]), __uint_as_float(fb[e]), c, 0, 0, 0);
-        }
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(gb8, fa), __builtin_bit_cast(gb8, fb), c, 0, 0, 0);
     };
     // one block per wave, several workgroups per unit: whole slots, DEPTH deep, one barrier each; the next slot's first fragments are read during this one's last products
     auto whole_slots = [&]() {
@@ -297,27 +281,27 @@ __global__ void __launch_bounds__(64 * WM * WN, WPS) sv_tile_kernel(const KrSvGe
             const int n = n0 + wc * (BN / WN) + b * 32 + r, mb = m0 + (a * WM + wr) * 32;
 #pragma unroll 1
             for (int i = h; i < 32; i += 2)
-                if (n < N && mb + i < mend) gm_store<sizeof(T) == 2>(g, mb + i, column(n), blk[i * 33 + r]);
+                if (n < N && mb + i < mend) gm_store<true>(g, mb + i, column(n), blk[i * 33 + r]);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
 }
 
-template <typename T, int BM, int BN, int WM, int WN, int DEPTH, int WPS, bool GLU>
+template <int BM, int BN, int WM, int WN, int DEPTH, int WPS, bool GLU>
 void tl_launch(const KrSvGemm& g, hipStream_t st) {
     constexpr int LDS = DEPTH * (BM + BN) * TL_ROW;
     static_assert(LDS <= 160 * 1024, "LDS of a compute unit");
-    static_assert(!GLU || (sizeof(T) == 2 && BN / WN % 64 == 0 && WM * WN * 2 * 32 * 36 * 4 <= LDS), "a wave holds both factors, and stages them");
+    static_assert(!GLU || (BN / WN % 64 == 0 && WM * WN * 2 * 32 * 36 * 4 <= LDS), "a wave holds both factors, and stages them");
     const int cols = GLU ? (g.N - 2 * g.glu_f + BN - 1) / BN + (g.glu_f + BN / 2 - 1) / (BN / 2) : (g.N + BN - 1) / BN;
     const dim3 grid(cols, (g.M + BM - 1) / BM + (g.seg ? g.n_groups : 0));
-    if (kr_lds_optin((const void*)sv_tile_kernel<T, BM, BN, WM, WN, DEPTH, WPS, GLU>, LDS)) return;
-    hipLaunchKernelGGL((sv_tile_kernel<T, BM, BN, WM, WN, DEPTH, WPS, GLU>), grid, dim3(64 * WM * WN), LDS, st, g);
+    if (kr_lds_optin((const void*)sv_tile_kernel<BM, BN, WM, WN, DEPTH, WPS, GLU>, LDS)) return;
+    hipLaunchKernelGGL((sv_tile_kernel<BM, BN, WM, WN, DEPTH, WPS, GLU>), grid, dim3(64 * WM * WN), LDS, st, g);
 }
 }  // namespace
 
 // whole slots of 16-byte chunks
 bool kr_sv_gemm_tile_fits(const KrSvGemm& g, bool f32) {
     const int row = TL_ROW / (f32 ? 4 : 2), chunk = 16 / (f32 ? 4 : 2);
-    return g.K % row == 0 && g.lda % chunk == 0 && (((uintptr_t)g.A | (uintptr_t)g.W) % 16 == 0) && g.w_stride % chunk == 0;
+    return g.K % row == 0 && (!f32 || g.K < 1 << 24) && g.lda % chunk == 0 && (((uintptr_t)g.A | (uintptr_t)g.W) % 16 == 0) && g.w_stride % chunk == 0;
 }
 
 // Which tile: the time of a slot step times how often the chip has to be filled, as measured at K = 2048 - 8192 (us per step of 64 k):
@@ -343,17 +327,11 @@ bool kr_sv_gemm_tile_glu_fits(const KrSvGemm& g) {
            (g.silu_hi <= g.silu_lo || g.silu_hi <= g.glu_lo || g.silu_lo >= g.glu_lo + 2 * g.glu_f) && tl_kind(g) != 64;
 }
 
-// f32 (500 tokens, 64 experts of 2 x 768 x 2048: 410 us a product on average with scalar loads and vector FMAs -> 131): the matrix instruction takes 16 times as long for the
-// same product (32x32x2, every factor and sum in f32), so nothing but its own count matters: 128 x 128 where that fills the chip without more padding than 64 x 64.
 void kr_sv_gemm_tile(const KrSvGemm& g, bool f32, hipStream_t st) {
-    if (f32) {
-        if (4.0 * std::ceil(tl_tiles(g, 128) / 256) < tl_tiles(g, 64) / 256) tl_launch<float, 128, 128, 2, 2, 2, 2, false>(g, st);
-        else tl_launch<float, 64, 64, 2, 2, 3, 3, false>(g, st);
-        return;
-    }
+    if (f32) { kr_sv_gemm_tile_f32(g, st); return; }
     switch (tl_kind(g)) {
-        case 256: if (g.glu_out) tl_launch<uint16_t, 256, 256, 2, 4, 2, 2, true>(g, st); else tl_launch<uint16_t, 256, 256, 2, 4, 2, 2, false>(g, st); break;
-        case 128: if (g.glu_out) tl_launch<uint16_t, 128, 128, 2, 2, 2, 2, true>(g, st); else tl_launch<uint16_t, 128, 128, 2, 2, 2, 2, false>(g, st); break;
-        default: tl_launch<uint16_t, 64, 64, 2, 2, 3, 3, false>(g, st); break;
+        case 256: if (g.glu_out) tl_launch<256, 256, 2, 4, 2, 2, true>(g, st); else tl_launch<256, 256, 2, 4, 2, 2, false>(g, st); break;
+        case 128: if (g.glu_out) tl_launch<128, 128, 2, 2, 2, 2, true>(g, st); else tl_launch<128, 128, 2, 2, 2, 2, false>(g, st); break;
+        default: tl_launch<64, 64, 2, 2, 3, 3, false>(g, st); break;
     }
 }

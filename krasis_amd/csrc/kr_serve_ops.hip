@@ -2453,9 +2453,11 @@ static bool sv_mfma_fits(int heads, int kv_heads, int dim, int vdim, int ldk, in
     return sv_mfma_tiling(dim / 4, vdim / 16);
 }
 // keys a wave takes at a time in a split launch: long rows on the matrix path go 16 at a time (a wave's loads of one 64-key block are ~40 dependent
-// batches at one wave per SIMD: a decode step is over sooner with four times the waves), everything else 64
-static int sv_split_key_block(int heads, int kv_heads, int dim, int vdim, int ldk, int ldv, bool f32) {
-    return (dim >= 192 && sv_mfma_fits(heads, kv_heads, dim, vdim, ldk, ldv, f32)) ? 16 : 64;
+// batches at one wave per SIMD: a decode step is over sooner with four times the waves), everything else 64.  f32 rows of 128 elements are as long, up to 256 workgroups: a step of one
+// layer, us, 64 -> 16 keys: one request at 250 / 500 / 2500 keys 207 / 207 / 212 -> 196 / 196 / 199, twelve at 300 608 -> 598, forty at 200 665 -> 635; but a portion of 250 tokens 564 -> 578.
+static int sv_split_key_block(int T, int heads, int kv_heads, int dim, int vdim, int ldk, int ldv, bool f32) {
+    const bool few = f32 && dim >= 128 && (long)T * kv_heads * ((heads / kv_heads + 15) / 16) <= 256;
+    return (dim >= 192 || few) && sv_mfma_fits(heads, kv_heads, dim, vdim, ldk, ldv, f32) ? 16 : 64;
 }
 
 int kr_sv_attention_splits(int T, int heads, int kv_heads, int dim, int vdim, int ldk, int ldv, bool f32, int max_visible) {
@@ -2465,7 +2467,7 @@ int kr_sv_attention_splits(int T, int heads, int kv_heads, int dim, int vdim, in
     int rm = 2;
     while (rm < R && rm < rmax) rm *= 2;
     const long blocks = (long)T * kv_heads * ((R + rm - 1) / rm);
-    const int kblk = sv_split_key_block(heads, kv_heads, dim, vdim, ldk, ldv, f32);
+    const int kblk = sv_split_key_block(T, heads, kv_heads, dim, vdim, ldk, ldv, f32);
     const int nch = (max_visible + kblk - 1) / kblk;
     long ns = 1024 / (blocks > 0 ? blocks : 1);              // about four workgroups per compute unit
     if (ns > (nch + 3) / 4) ns = (nch + 3) / 4;              // a workgroup keeps at least one block of keys per wave
@@ -2527,17 +2529,19 @@ static bool sv_attn_mfma_launch(const KrSvAttn& a, hipStream_t st) {
 #define SV_MF(DQ_, DB_) do { hipLaunchKernelGGL((sv_attn_mfma_kernel<T, DQ_, DB_>), grid, dim3(256), lds, st, b); return true; } while (0)
 #define SV_MF1(DQ_, DB_) do { if (a.nsplit > 1) hipLaunchKernelGGL((sv_attn_mfma_kernel<T, DQ_, DB_, 1>), grid, dim3(256), lds, st, b); \
                               else hipLaunchKernelGGL((sv_attn_mfma_kernel<T, DQ_, DB_>), grid, dim3(256), lds, st, b); return true; } while (0)
+    const bool short_blocks = sv_split_key_block(a.T, a.heads, a.kv_heads, a.dim, a.vdim, a.ldk, a.ldv, sizeof(T) == 4) == 16;
+#define SV_MF4(DQ_, DB_) do { if constexpr (sizeof(T) == 4) { if (short_blocks) SV_MF1(DQ_, DB_); } SV_MF(DQ_, DB_); } while (0)
     const int dq = a.dim / 4, db = a.vdim / 16;
     if (dq == 16 && db == 4) SV_MF(16, 4);
-    if (dq == 32 && db == 8) SV_MF(32, 8);
+    if (dq == 32 && db == 8) SV_MF4(32, 8);
     if (dq == 16 && db == 8) SV_MF(16, 8);
-    if (dq == 32 && db == 4) SV_MF(32, 4);
+    if (dq == 32 && db == 4) SV_MF4(32, 4);
     if (dq == 8 && db == 2) SV_MF(8, 2);
     if (dq == 8 && db == 4) SV_MF(8, 4);
     if (dq == 16 && db == 2) SV_MF(16, 2);
     if (dq == 64 && db == 16) SV_MF(64, 16);
     if (dq == 64 && db == 8) SV_MF(64, 8);
-    if (dq == 32 && db == 16) SV_MF(32, 16);
+    if (dq == 32 && db == 16) SV_MF4(32, 16);
     if (dq == 8 && db == 16) SV_MF(8, 16);
     if (dq == 8 && db == 1) SV_MF(8, 1);
     if (dq == 16 && db == 1) SV_MF(16, 1);
@@ -2546,6 +2550,7 @@ static bool sv_attn_mfma_launch(const KrSvAttn& a, hipStream_t st) {
     if (dq == 48 && db == 8) SV_MF1(48, 8);
 #undef SV_MF
 #undef SV_MF1
+#undef SV_MF4
     return false;
 }
 

@@ -169,3 +169,22 @@ def test_capped_scores_distance_bias_and_chunks(design, size, heads, kv_heads, d
         at += n
     base = x0(np.asarray(toks))
     assert row_errors(np.concatenate(got) - base, forward(cfg, W, toks)[1][0] - base).max() < 2e-2
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(16, 2, 128, 128), (4, 4, 128, 64), (32, 1, 128, 256)])
+@pytest.mark.parametrize("ctx,window", [(15, 0), (16, 7), (63, 0), (64, 17), (65, 0), (300, 130), (700, 0)])
+def test_single_tokens_f32(heads, kv_heads, dim, vdim, ctx, window):
+    # blocks of 16 keys a wave, one workgroup and several; a step of 130 single tokens, past the line, takes 64 again
+    cfg = model(heads, kv_heads, dim, vdim, window, rot=8); W = O.random_weights(cfg, 61)
+    for requests in (2, 130 if ctx == 65 else 1):
+        seqs = [tokens(cfg, max(1, ctx - i % 3) + 1, 62 + i % 3) for i in range(requests)]
+        eng = engine(cfg, W, max_tokens=2048 + 128 * requests, max_slots=requests)
+        for i, s in enumerate(seqs):
+            eng.step([(i, s[:-1], [])])
+        eng.store.set_capture(True)
+        eng.step([(i, s[-1:], [0]) for i, s in enumerate(seqs)])
+        got = eng.store.read_capture(requests)[0]
+        x0 = W["embed"].astype(np.float64)[[s[-1] for s in seqs]]
+        kinds = [O.forward(cfg, W, s)[1][0][-1] for s in seqs[:3]]
+        ref = np.stack([kinds[i % 3] for i in range(requests)])
+        assert row_errors(got - x0, ref - x0).max() < 2e-5      # f32 throughout: sums of some hundred products and exponentials, each within 2^-23

@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "kr_lds_optin.h"
 #include "kr_serve_gemm_dev.h"
 
@@ -51,49 +53,65 @@ __global__ void __launch_bounds__(256) sv_gemv_kernel(const KrSvGemm g, int mbas
     const bool vec = ACT ? (g.K % VEC == 0) && (g.act_ld % 4 == 0) && (g.K % 4 == 0) && ((uintptr_t)g.act_gu % 16 == 0) && ((uintptr_t)g.W % 16 == 0) && (g.w_stride % VEC == 0)
                          : (g.K % VEC == 0) && (g.lda % VEC == 0) && (((uintptr_t)g.A | (uintptr_t)g.W) % 16 == 0) && (g.w_stride % VEC == 0);
     if (vec) {
-        for (int k = lane * VEC; k < g.K; k += 64 * VEC) {
-            gu4 wv[CN];
+        auto steps = [&](auto u_, int k) {                       // u_ k steps from the lane's k on, requested together, added in their order
+            constexpr int U = u_();
+            gu4 wv[U][CN];
 #pragma unroll
-            for (int c = 0; c < CN; c++) wv[c] = *reinterpret_cast<const gu4*>(wr[c] + k);
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int c = 0; c < CN; c++) wv[u][c] = *reinterpret_cast<const gu4*>(wr[c] + k + u * 64 * VEC);
 #pragma unroll
             for (int m = 0; m < MB; m++) {
                 if (m < mcnt) {
-                    float af[VEC];
-                    if constexpr (ACT) {
+                    float af[U][VEC];
 #pragma unroll
-                        for (int q = 0; q < VEC / 4; q++) {
-                            const float4 gg = *reinterpret_cast<const float4*>(gr[m] + k + 4 * q);
-                            float4 uu = *reinterpret_cast<const float4*>(gr[m] + uoff + k + 4 * q);
-                            if (ur[m]) uu = make_float4(gm_ld(ur[m] + k + 4 * q), gm_ld(ur[m] + k + 4 * q + 1), gm_ld(ur[m] + k + 4 * q + 2), gm_ld(ur[m] + k + 4 * q + 3));
-                            af[4 * q] = gm_round<T>(gm_act(gg.x * gw[m], uu.x * gw[m], g.act_kind, g.act_limit, g.act_alpha)); af[4 * q + 1] = gm_round<T>(gm_act(gg.y * gw[m], uu.y * gw[m], g.act_kind, g.act_limit, g.act_alpha));
-                            af[4 * q + 2] = gm_round<T>(gm_act(gg.z * gw[m], uu.z * gw[m], g.act_kind, g.act_limit, g.act_alpha)); af[4 * q + 3] = gm_round<T>(gm_act(gg.w * gw[m], uu.w * gw[m], g.act_kind, g.act_limit, g.act_alpha));
-                        }
-                    } else {
-                        const gu4 av = *reinterpret_cast<const gu4*>(ar[m] + k);
-                        if constexpr (sizeof(T) == 2) {
+                    for (int u = 0; u < U; u++) {
+                        const int ku = k + u * 64 * VEC;
+                        if constexpr (ACT) {
 #pragma unroll
-                            for (int i = 0; i < 4; i++) { af[2 * i] = __uint_as_float(av[i] << 16); af[2 * i + 1] = __uint_as_float(av[i] & 0xFFFF0000u); }
-                        } else {
+                            for (int q = 0; q < VEC / 4; q++) {
+                                const float4 gg = *reinterpret_cast<const float4*>(gr[m] + ku + 4 * q);
+                                float4 uu = *reinterpret_cast<const float4*>(gr[m] + uoff + ku + 4 * q);
+                                if (ur[m]) uu = make_float4(gm_ld(ur[m] + ku + 4 * q), gm_ld(ur[m] + ku + 4 * q + 1), gm_ld(ur[m] + ku + 4 * q + 2), gm_ld(ur[m] + ku + 4 * q + 3));
+                                const float gv[4] = {gg.x, gg.y, gg.z, gg.w}, uv[4] = {uu.x, uu.y, uu.z, uu.w};
 #pragma unroll
-                            for (int i = 0; i < 4; i++) af[i] = __uint_as_float(av[i]);
-                        }
-                    }
-#pragma unroll
-                    for (int c = 0; c < CN; c++) {
-                        if constexpr (sizeof(T) == 2) {
-#pragma unroll
-                            for (int i = 0; i < 4; i++) {
-                                acc[m][c] = __builtin_fmaf(af[2 * i], __uint_as_float(wv[c][i] << 16), acc[m][c]);
-                                acc[m][c] = __builtin_fmaf(af[2 * i + 1], __uint_as_float(wv[c][i] & 0xFFFF0000u), acc[m][c]);
+                                for (int i = 0; i < 4; i++) af[u][4 * q + i] = gm_round<T>(gm_act(gv[i] * gw[m], uv[i] * gw[m], g.act_kind, g.act_limit, g.act_alpha));
                             }
                         } else {
+                            const gu4 av = *reinterpret_cast<const gu4*>(ar[m] + ku);
+                            if constexpr (sizeof(T) == 2) {
 #pragma unroll
-                            for (int i = 0; i < 4; i++) acc[m][c] = __builtin_fmaf(af[i], __uint_as_float(wv[c][i]), acc[m][c]);
+                                for (int i = 0; i < 4; i++) { af[u][2 * i] = __uint_as_float(av[i] << 16); af[u][2 * i + 1] = __uint_as_float(av[i] & 0xFFFF0000u); }
+                            } else {
+#pragma unroll
+                                for (int i = 0; i < 4; i++) af[u][i] = __uint_as_float(av[i]);
+                            }
                         }
                     }
+#pragma unroll
+                    for (int u = 0; u < U; u++)
+#pragma unroll
+                        for (int c = 0; c < CN; c++) {
+                            if constexpr (sizeof(T) == 2) {
+#pragma unroll
+                                for (int i = 0; i < 4; i++) {
+                                    acc[m][c] = __builtin_fmaf(af[u][2 * i], __uint_as_float(wv[u][c][i] << 16), acc[m][c]);
+                                    acc[m][c] = __builtin_fmaf(af[u][2 * i + 1], __uint_as_float(wv[u][c][i] & 0xFFFF0000u), acc[m][c]);
+                                }
+                            } else {
+#pragma unroll
+                                for (int i = 0; i < 4; i++) acc[m][c] = __builtin_fmaf(af[u][i], __uint_as_float(wv[u][c][i]), acc[m][c]);
+                            }
+                        }
                 }
             }
-        }
+        };
+        // one weight row a wave: a step at a time has 1 KB of it on its way.  (us, f32, 1 -> 4 steps, with four rows 2: 12 rows of a step 598 -> 568, one 196 -> 193; 8 and 4: 195)
+        constexpr int UM = !ACT && CN == 1 ? 4 : 2;
+        int done = 0;
+        for (; done + UM * 64 * VEC <= g.K; done += UM * 64 * VEC) steps(std::integral_constant<int, UM>{}, done + lane * VEC);
+        if (UM > 2) for (; done + 2 * 64 * VEC <= g.K; done += 2 * 64 * VEC) steps(std::integral_constant<int, 2>{}, done + lane * VEC);
+        for (; done + lane * VEC < g.K; done += 64 * VEC) steps(std::integral_constant<int, 1>{}, done + lane * VEC);
     } else {
         for (int k = lane; k < g.K; k += 64) {
             float w[CN];

@@ -1122,20 +1122,23 @@ int kr_moe_prefill_set(kr_engine* e, int layer, const void* x_bf16, const int32_
         kr_launch_pf_sort(idc, mc, topk, E, so, st, cut);
         kr_launch_pf_quant_x(xc, mc, H, (int8_t*)P.xh.p, (int8_t*)P.xl.p, (float*)P.xs.p, st);
         const int var_rows = (long)mc * topk < 48L * E;     // fewer than ~48 rows per expert: most 64-row tiles have an empty second half
+        KrPfDense d13{}, d2{};
+        if (use_shared) {
+            d13 = KrPfDense{L.sw13.view(), (const uint32_t*)L.sw13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, mc, (float*)P.sgu.p, 2 * SI};
+            d2 = KrPfDense{L.sw2.view(), (const uint32_t*)L.sw2.wsum.p, (const int8_t*)P.shh.p, (const int8_t*)P.shl.p, (const float*)P.shs.p, mc, (float*)P.seo.p, H};
+        }
+        const bool join = use_shared && kr_pf_joins(cut, L.w13.view(), d13.m, mc) && kr_pf_joins(cut, L.w2.view(), d2.m, mc);
+        auto shared_gemm = [&](const KrPfDense& d) { kr_launch_pf_gemm(d.m, d.wsum, d.a_hi, d.a_lo, d.a_scale, nullptr, topk, 0, 0, d.rows, d.out, d.out_ld, st); };
+        auto shared_act = [&] { kr_launch_pf_act((const float*)P.sgu.p, mc, SI, 2 * SI, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.shh.p, (int8_t*)P.shl.p,
+                                                 (float*)P.shs.p, st); };
         kr_launch_pf_gemm(L.w13.view(), (const uint32_t*)L.w13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, &so, topk, 1,
-                          cut.max_tiles, 0, (float*)P.gu.p, 2 * I, st, 0, 0, var_rows, &cut);
+                          cut.max_tiles, 0, (float*)P.gu.p, 2 * I, st, 0, 0, var_rows, &cut, join ? &d13 : nullptr);
         kr_launch_pf_act((const float*)P.gu.p, mc * topk, I, 2 * I, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.hh.p, (int8_t*)P.hl.p,
                          (float*)P.hs.p, st);
+        if (join) shared_act();
         kr_launch_pf_gemm(L.w2.view(), (const uint32_t*)L.w2.wsum.p, (const int8_t*)P.hh.p, (const int8_t*)P.hl.p, (const float*)P.hs.p, &so, topk, 0,
-                          cut.max_tiles, 0, (float*)P.eo.p, H, st, 0, 0, var_rows, &cut);
-        if (use_shared) {
-            kr_launch_pf_gemm(L.sw13.view(), (const uint32_t*)L.sw13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, nullptr, topk, 0,
-                              0, mc, (float*)P.sgu.p, 2 * SI, st);
-            kr_launch_pf_act((const float*)P.sgu.p, mc, SI, 2 * SI, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.shh.p, (int8_t*)P.shl.p,
-                             (float*)P.shs.p, st);
-            kr_launch_pf_gemm(L.sw2.view(), (const uint32_t*)L.sw2.wsum.p, (const int8_t*)P.shh.p, (const int8_t*)P.shl.p, (const float*)P.shs.p, nullptr, topk, 0,
-                              0, mc, (float*)P.seo.p, H, st);
-        }
+                          cut.max_tiles, 0, (float*)P.eo.p, H, st, 0, 0, var_rows, &cut, join ? &d2 : nullptr);
+        if (use_shared && !join) { shared_gemm(d13); shared_act(); shared_gemm(d2); }
         kr_launch_pf_combine((const float*)P.eo.p, so.pair_row, wc, mc, topk, H, use_shared ? (const float*)P.seo.p : nullptr, e->cfg.routed_scaling_factor,
                              (char*)out + (size_t)m0 * H * ob, out_dtype == KR_OUT_BF16, st);
     }

@@ -29,10 +29,13 @@ void kr_launch_pf_sort(const int32_t* ids, int M, int topk, int E, KrPfSort s, h
 void kr_launch_pf_quant_x(const uint16_t* x, int M, int K, int8_t* xh, int8_t* xl, float* xs, hipStream_t st);
 void kr_launch_pf_act(const float* gu, int rows, int n, int gu_ld, int act_mode, float swiglu_limit, float alpha, int8_t* hh, int8_t* hl, float* hs, hipStream_t st);
 void kr_launch_pf_wsum(const KrMatDev& m, int n_experts, uint32_t* wsum, hipStream_t st);
+// a single matrix over rows 0 .. rows - 1
+struct KrPfDense { KrMatDev m; const uint32_t* wsum; const int8_t* a_hi; const int8_t* a_lo; const float* a_scale; int rows; float* out; int out_ld; };
 void kr_launch_pf_gemm(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_hi, const int8_t* a_lo, const float* a_scale, const KrPfSort* sort, int topk,
                        int gather_tokens, int max_tiles, int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows = 0, int out_bf16 = 0,
                        int var_rows = 0 /* expert tiles mostly <= 32 rows: kernel variant that skips empty 32-row blocks */,
-                       const KrPfTiles* t = nullptr /* of the tile table; null: tiles of 64 */);
+                       const KrPfTiles* t = nullptr /* of the tile table; null: tiles of 64 */, const KrPfDense* beside = nullptr /* for the same launch, where kr_pf_joins */);
+bool kr_pf_joins(const KrPfTiles& t, const KrMatDev& experts, const KrMatDev& dense, int rows);
 // of the exact GEMMs that will run on one tile table: tiles of 128 rows (the wide kernel) or 64, and whether strips may take their place
 KrPfTiles kr_pf_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows /* of all their slots */, int E, bool beside /* launches of other chunks run at the same time */);
 void kr_launch_pf_gemm_multi(const KrMatDev* mats, const uint32_t* const* wsums, float* const* outs, const int* out_lds, int n, const int8_t* a_hi, const int8_t* a_lo,

@@ -427,8 +427,15 @@ static bool pf_dense_wide(const KrPfGemmArgs& a) {
     for (int i = 0; i < a.n_extra; i++) { ncb += (a.mx[i].N + PFW_TN - 1) / PFW_TN; all = all && pf_all_fma(a.mx[i]); }
     return all && (long)a.total_rows * a.m.ng * 128 < 1L << 32 && (long)ncb * ((a.total_rows + PFW_TM - 1) / PFW_TM) >= 128;
 }
+// A shared expert's products ride in the launches of the routed experts' where those take the wide kernel: each of its own launches ends in a round of workgroups that is seldom full
+// (3001 rows of 2 x 2816 x 2048 are 528 tiles, three rounds of 256 for the time of two).  (3001 rows, 64 INT8 experts of 2 x 1408 x 2048, top 6, two shared: us of the layer, apart / joined: 836 / 783;
+// 540 rows 291 / 246, 1500 546 / 479, 4096 1039 / 1032; INT4 279 / 241, 531 / 522, 1037 / 1033, 3001 842 / 801.)
+bool kr_pf_joins(const KrPfTiles& t, const KrMatDev& experts, const KrMatDev& dense, int rows) {
+    return t.rows == PFW_TM && dense.bits == experts.bits && pf_all_fma(dense) && (long)rows * dense.ng * 128 < 1L << 32;
+}
 void kr_launch_pf_gemm(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_hi, const int8_t* a_lo, const float* a_scale, const KrPfSort* sort, int topk,
-                       int gather_tokens, int max_tiles, int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows, int out_bf16, int var_rows, const KrPfTiles* t) {
+                       int gather_tokens, int max_tiles, int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows, int out_bf16, int var_rows, const KrPfTiles* t,
+                       const KrPfDense* beside) {
     KrPfGemmArgs a{};
     a.scatter_rows = scatter_rows; a.out_bf16 = out_bf16;
     a.var_rows = sort != nullptr && single_expert_rows <= 0 && var_rows;
@@ -437,7 +444,12 @@ void kr_launch_pf_gemm(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_
     a.out = out; a.out_ld = out_ld; a.single_expert = single_expert_rows > 0; a.total_rows = single_expert_rows;
     if (single_expert_rows > 0 ? pf_dense_wide(a) : t && t->rows == PFW_TM) {
         const int wt = single_expert_rows > 0 ? (single_expert_rows + PFW_TM - 1) / PFW_TM : max_tiles;
-        if (m.bits == 8) kr_pf_wide_launch<8>(a, wt, st); else kr_pf_wide_launch<4>(a, wt, st);
+        KrPfGemmArgs b{};
+        if (beside) {
+            b.m = beside->m; b.wsum = beside->wsum; b.a_hi = beside->a_hi; b.a_lo = beside->a_lo; b.a_scale = beside->a_scale; b.topk = topk;
+            b.out = beside->out; b.out_ld = beside->out_ld; b.single_expert = 1; b.total_rows = beside->rows;
+        }
+        if (m.bits == 8) kr_pf_wide_launch<8>(a, wt, st, beside ? &b : nullptr); else kr_pf_wide_launch<4>(a, wt, st, beside ? &b : nullptr);
         return;
     }
     if (single_expert_rows <= 0 && t && t->strip > 0) {

@@ -25,3 +25,17 @@ def test_many_rows_equal_few(H, I, bits, w2_bits, n_shared):
     whole = mgr.forward(0, x, ids, w).view(torch.int16).cpu().numpy()
     few = np.concatenate([mgr.forward(0, x[i:i + 40], ids[i:i + 40], w[i:i + 40]).view(torch.int16).cpu().numpy() for i in range(0, M, 40)])
     assert np.array_equal(whole, few)
+
+
+@pytest.mark.parametrize("M", [216, 256, 257, 601])
+@pytest.mark.parametrize("H,I,bits,w2_bits,n_shared", [(640, 384, 4, 4, 1), (384, 256, 8, 8, 2), (256, 640, 8, 4, 1), (256, 128, 4, 8, 2)])
+def test_shared_expert_in_the_experts_launches(M, H, I, bits, w2_bits, n_shared):
+    # fewer shared tiles than a launch of its own would take, whole and ragged row tiles, matrices of either type; forty rows at a time take neither the wide kernel nor the join
+    E, k = 9, 2
+    eng, mgr, experts, shared, rng, torch = _setup(H, I, E, k, n_shared, 1.5, bits=bits, w2_bits=w2_bits)
+    x = torch.from_numpy(rand_bf16(rng, (M, H)).view(np.int16)).cuda().view(torch.bfloat16)
+    ids = np.stack([rng.permutation(E)[:k] for _ in range(M)]).astype(np.int32); ids[5] = -1
+    ids = torch.from_numpy(ids).cuda(); w = torch.from_numpy(rng.random((M, k)).astype(np.float32)).cuda()
+    whole = mgr.forward(0, x, ids, w).view(torch.int16).cpu().numpy()
+    few = np.concatenate([mgr.forward(0, x[i:i + 40], ids[i:i + 40], w[i:i + 40]).view(torch.int16).cpu().numpy() for i in range(0, M, 40)])
+    assert np.array_equal(whole, few)

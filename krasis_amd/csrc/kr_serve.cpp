@@ -1081,6 +1081,8 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     // copied.  (A prompt whose logits are all wanted may have more than the store keeps: copied from the device then)
     const size_t row_bytes = (size_t)n_want * c.vocab * 4;
     char* const direct = n_want > 0 && logits_out ? rows_device_ptr(logits_out, row_bytes, s->device) : nullptr;
+    bool all_rows = n_want == T;                             // every row, in its place
+    for (int i = 0; i < n_want && all_rows; i++) all_rows = want_rows[i] == i;
     const bool want_amax = n_want > 0 && argmax_out, host_logits = n_want > 0 && logits_out && (direct || row_bytes <= HOST_OUT_MOST);
     const size_t amax_bytes = ((size_t)n_want * 4 + 255) / 256 * 256;
     void* dev_out = nullptr;
@@ -1258,6 +1260,9 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     // gate: 0 none, 1 the mixer's (logits in rg, the output projection's bias, and the input convolution's rows of this layer are kept), 2 the feed-forward's
     // (logits in the last row block of hz).  to_mixer: the handed-on row feeds a mixer (an f32 copy goes along for its input convolution)
     const SvLayer* res_layer = nullptr; const SvLayer* res_run = nullptr; int res_gate_kind = 0; bool res_to_mixer = false, res_next32 = false;
+    // Where every row is wanted in its place, as a decode step's are, the sum that ends the last layer hands on the final norm's rows: the same statements on the same numbers, and
+    // a launch of 3 - 5 us less (24 tokens of four layers after their prompts, ms, one request 6.31 -> 6.28, twelve 15.9 -> 15.7).
+    bool res_final = false, final_normed = false;
     auto residual = [&](const float* mixp, const float* dense, const float* shared, const float* rows, const int* pair_pos, int top, const DevBuf* post_w, const DevBuf* post_b,
                         bool hand_on, const DevBuf* next_w, const DevBuf* next_b) {
         Timer tm(s, 6);
@@ -1277,6 +1282,11 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         r.post_w = post_w ? (const float*)post_w->p : nullptr; r.post_b = (post_w && c.norm_bias && post_b) ? (const float*)post_b->p : nullptr; r.mult = c.residual_mult;
         r.norm_w = (hand_on && next_w) ? (const float*)next_w->p : nullptr; r.norm_b = (hand_on && next_w && c.norm_bias && next_b) ? (const float*)next_b->p : nullptr;
         r.h_out = hand_on ? s->h.p : nullptr; r.T = T; r.width = W; r.kind = c.norm_kind; r.eps = c.norm_eps;
+        if (res_final && all_rows) {
+            KrSvResidual f = r;
+            f.norm_w = (const float*)s->fnorm_w.p; f.norm_b = c.norm_bias ? (const float*)s->fnorm_b.p : nullptr; f.h_out = s->hw.p; f.h32_out = nullptr;
+            if (kr_sv_residual_vec(f)) { r = f; final_normed = true; }
+        }
         kr_sv_residual_norm(r, s->f32, st);
     };
     if (c.pre_norm && !s->L[0].d.pre_add && !normed) {
@@ -1593,7 +1603,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
             rows = (const float*)s->rows.p; pair_pos = pp;
         }
         // x += the layer's sublayers (parallel block) or the feed-forward alone (sequential), and the next layer's input from the same launch
-        res_layer = &l; res_run = &run; res_gate_kind = seq ? 2 : l.wkv() ? 1 : 0; res_to_mixer = !side;
+        res_layer = &l; res_run = &run; res_gate_kind = seq ? 2 : l.wkv() ? 1 : 0; res_to_mixer = !side; res_final = li + 1 == c.n_layers && !side;
         if (!seq) residual((const float*)s->mix.p, dense, shared, rows, pair_pos, d.top, nullptr, nullptr, hand || side, (nx && c.pre_norm && !side) ? &nx->norm_w : nullptr, nx ? &nx->norm_b : nullptr);
         else if (has_ff) residual(nullptr, dense, shared, rows, pair_pos, d.top, c.post_norm ? &l.post2_w : nullptr, &l.post2_b, hand || side, (nx && c.pre_norm && !side) ? &nx->norm_w : nullptr,
                                   nx ? &nx->norm_b : nullptr);
@@ -1611,7 +1621,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
                 { Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); }
                 down_proj(gp, (const float*)s->sgate.p, ns, T, ns, KR_SV_ACT_GELU_TANH, 0.0f, 1.0f);
             }
-            res_layer = nullptr; res_run = nullptr; res_gate_kind = 0; res_to_mixer = true;
+            res_layer = nullptr; res_run = nullptr; res_gate_kind = 0; res_to_mixer = true; res_final = li + 1 == c.n_layers;
             residual((const float*)s->mix.p, nullptr, nullptr, nullptr, nullptr, 0, &l.side_norm, nullptr, hand, (nx && c.pre_norm) ? &nx->norm_w : nullptr, nx ? &nx->norm_b : nullptr);
         }
         if (s->capture) KR_HIP(hipMemcpyAsync((float*)s->cap.p + (size_t)li * Ts * W, x, Ts * W * 4, hipMemcpyDeviceToDevice, st));
@@ -1619,7 +1629,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
     if (n_want > 0) {
         const bool scaled = c.logit_scale != 0.0f && c.logit_scale != 1.0f;
         float* const* host_rows = host_logits ? (float* const*)(d_tok + n_own) : nullptr;
-        { Timer tm(s, 0); kr_sv_norm(x, d_want, (const float*)s->fnorm_w.p, c.norm_bias ? (const float*)s->fnorm_b.p : nullptr, s->hw.p, s->f32, n_want, W, c.norm_eps, c.norm_kind, NG, nullptr, st); }
+        if (!final_normed) { Timer tm(s, 0); kr_sv_norm(x, d_want, (const float*)s->fnorm_w.p, c.norm_bias ? (const float*)s->fnorm_b.p : nullptr, s->hw.p, s->f32, n_want, W, c.norm_eps, c.norm_kind, NG, nullptr, st); }
         KrSvGemm g{}; g.A = s->hw.p; g.lda = W; g.W = s->head.p; g.C = (float*)s->logits.p; g.ldc = c.vocab; g.M = n_want; g.N = c.vocab; g.K = W;
         if (host_logits && !scaled && kr_sv_gemm_takes_host(g, s->f32)) { g.c_host = host_rows; host_rows = nullptr; }
         { Timer tm(s, 1); kr_sv_gemm(g, s->f32, st); }
@@ -1636,7 +1646,7 @@ int kr_serve_step(kr_serve* s, int n_entries, const int* slots, const int* count
         // the key: everything a launch argument depends on -- batch, wanted rows, the split of every layer, the scratch addresses
         uint64_t key = 1469598103934665603ull;
         auto mixin = [&](uint64_t v) { key = (key ^ v) * 1099511628211ull; };
-        mixin((uint64_t)T); mixin((uint64_t)n_want); mixin(want_amax); mixin(host_logits); mixin((uint64_t)(uintptr_t)dev_out);
+        mixin((uint64_t)T); mixin((uint64_t)n_want); mixin(want_amax); mixin(host_logits); mixin(all_rows); mixin((uint64_t)(uintptr_t)dev_out);
         for (const KrSvAttnPlan& p : plan) mixin((uint64_t)p.nsplit);
         for (const DevBuf* b : {&s->meta, &s->x, &s->h, &s->qkv, &s->att, &s->mix, &s->gu, &s->y, &s->rows, &s->ffout, &s->ids, &s->wts, &s->moe_i, &s->hw, &s->logits,
                                 &s->amax, &s->part_ml, &s->part_acc, &s->v_first, &s->lq_c, &s->lq_2, &s->lq_n, &s->lq_e, &s->att2, &s->head_i, &s->h32, &s->hc, &s->rg, &s->qk_rms, &s->lin_o, &s->qkv2, &s->sconv, &s->ga1, &s->gz, &s->rg_ab, &s->rg_agg, &s->rg_start,

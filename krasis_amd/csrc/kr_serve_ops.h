@@ -222,6 +222,7 @@ struct KrSvResidual {
     const float* h32_in; float* canon_state; int canon_keep; const int* slot; const int* pos;
 };
 void kr_sv_residual_norm(const KrSvResidual& r, bool out_f32, hipStream_t st);
+bool kr_sv_residual_vec(const KrSvResidual& r);              // takes the form whose norm is kr_sv_norm's, bit for bit
 
 // ---- latent mixer (keys / values, and with q_rank > 0 the queries, through low-rank latents; the cache row is [latent | rotated shared key part])
 struct KrSvLatent {

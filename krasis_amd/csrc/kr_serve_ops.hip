@@ -2645,9 +2645,13 @@ void kr_sv_act(const float* gu, int ld, void* y, bool f32, int M, int F, int kin
     else hipLaunchKernelGGL(sv_act_kernel<uint16_t>, grid, dim3(256), 0, st, gu, ld, (uint16_t*)y, M, F, kind, limit, alpha, row_w, (const uint16_t*)up_tab, up_rows, up_ld, up_off);
 }
 
+static bool sv_residual_al16(const KrSvResidual& r) {
+    return sv_al16({r.x, r.mix, r.mix_bias, r.rows, r.shared, r.dense, r.post_w, r.post_b, r.norm_w, r.norm_b, r.h_out, r.h32_in, r.h32_out, r.canon_state});
+}
+bool kr_sv_residual_vec(const KrSvResidual& r) { return sv_residual_al16(r) && sv_vec_rows(r.T, r.width, [](auto, auto) {}); }
 template <typename T, int KIND> static void sv_residual_launch(const KrSvResidual& r, hipStream_t st) {
     const size_t lds = (size_t)(r.width + 2 * (r.groups > 1 ? r.groups : 0)) * sizeof(float), glds = r.groups > 1 ? lds : 0;
-    if (sv_al16({r.x, r.mix, r.mix_bias, r.rows, r.shared, r.dense, r.post_w, r.post_b, r.norm_w, r.norm_b, r.h_out, r.h32_in, r.h32_out, r.canon_state}) &&
+    if (sv_residual_al16(r) &&
         sv_vec_rows(r.T, r.width, [&](auto nt, auto ch) { hipLaunchKernelGGL((sv_residual_vec_kernel<T, KIND, nt(), ch()>), dim3(r.T), dim3(nt()), glds, st, r, (T*)r.h_out); })) return;
     if (r.T <= 64) hipLaunchKernelGGL((sv_residual_norm_kernel<T, KIND, 1024>), dim3(r.T), dim3(1024), lds, st, r, (T*)r.h_out);
     else hipLaunchKernelGGL((sv_residual_norm_kernel<T, KIND, 256>), dim3(r.T), dim3(256), lds, st, r, (T*)r.h_out);

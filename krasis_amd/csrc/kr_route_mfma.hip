@@ -28,25 +28,35 @@ typedef uint32_t rm_u4 __attribute__((ext_vector_type(4)));
 // Batched form (blockIdx.z): the same 16-chain dot + fold tree is the reference's w_vc projection of MLA (mla_project_wvc_avx2, decode.rs:4555: two
 // 8-lane accumulators over alternating 8-blocks = chains j = 8 a + l over elements 16 m + j, then acc0 + acc1 and the hsum tree) -- head h reads
 // x + h * x_bs with row stride ldx, gate + h * g_bs, and writes logits + h * o_bs with row stride ldo.
-// SPLIT: the problem has too few 64 x 64 tiles to fill the chip (the router of a 1024-token chunk: 128 workgroups of 256-register waves on 256 CUs).
+// S == 2: the problem has too few 64 x 64 tiles to fill the chip (the router of a 1024-token chunk: 128 workgroups of 256-register waves on 256 CUs).
 // A workgroup then takes 32 tokens x 64 experts and its four waves are (expert block, CHAIN HALF): wave half c owns the 8 chains
 // j = {0,1,4,5,8,9,12,13} + 2 c, i.e. the sub-trees (c0 + c1) or (c2 + c3) of the fold; the halves meet through LDS and the last add is the
 // tree's root -- the same 15 adds in the same order.  Twice the workgroups, half the accumulators (two waves per SIMD).
-template <bool GATE_BF16, bool SPLIT>
-__global__ void __launch_bounds__(256, SPLIT ? 2 : 1) kr_route_logits_mfma_kernel(const void* __restrict__ gate_row_, const float* __restrict__ x_, const float* __restrict__ bias,
+// S == 4: with fewer tokens still a launch is one wave's chain of products, 30 us at K = 2048 however few there are.  32 x 32 tiles, a wave takes chains j = q mod 4, one of the
+// sub-trees c0 .. c3: a quarter of the chain.
+template <bool GATE_BF16, int S>
+__global__ void __launch_bounds__(256, S > 1 ? 2 : 1) kr_route_logits_mfma_kernel(const void* __restrict__ gate_row_, const float* __restrict__ x_, const float* __restrict__ bias,
                                                                    float* __restrict__ logits_, int T, int E, int H, int ldx, int ldo, size_t x_bs, size_t g_bs, size_t o_bs) {
     const float* x = x_ + (size_t)blockIdx.z * x_bs; float* logits = logits_ + (size_t)blockIdx.z * o_bs;
     const void* gate_row = GATE_BF16 ? (const void*)(reinterpret_cast<const uint16_t*>(gate_row_) + (size_t)blockIdx.z * g_bs)
                                      : (const void*)(reinterpret_cast<const float*>(gate_row_) + (size_t)blockIdx.z * g_bs);
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    constexpr int TT = SPLIT ? 32 : 64, NJ = SPLIT ? 8 : 16, NA = TT / 8;
-    constexpr int A_BYTES = TT * RM_LDA * 4, B_BYTES = GATE_BF16 ? 64 * RM_LDB16 * 2 : 64 * RM_LDB32 * 4;
+    constexpr bool SPLIT = S > 1;
+    constexpr int TT = SPLIT ? 32 : 64, TE = S == 4 ? 32 : 64, NJ = 16 / S, NA = TT / 8, NBG = TE / (GATE_BF16 ? 16 : 8);
+    // Rows of LDS: 16-byte reads want them four banks apart, the 8-byte reads of SPLIT two (at four, four lanes met in every bank and the reads took 0.9 of the products' time)
+    constexpr int LDA = SPLIT ? RM_KS + 2 : RM_LDA, LDB32 = SPLIT ? RM_KS + 2 : RM_LDB32, LDB16 = SPLIT ? RM_KS + 4 : RM_LDB16;
+    constexpr int A_BYTES = TT * LDA * 4, B_BYTES = GATE_BF16 ? TE * LDB16 * 2 : TE * LDB32 * 4;
+    typedef float rm_f2 __attribute__((ext_vector_type(2)));
+    auto put = [](void* dst, rm_f4 v) {
+        if constexpr (SPLIT) { reinterpret_cast<rm_f2*>(dst)[0] = rm_f2{v.x, v.y}; reinterpret_cast<rm_f2*>(dst)[1] = rm_f2{v.z, v.w}; }
+        else *reinterpret_cast<rm_f4*>(dst) = v;
+    };
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, h = lane >> 5;
-    const int t0 = blockIdx.y * TT, e0 = blockIdx.x * 64;
-    const int tb = SPLIT ? 0 : (wave >> 1) * 32, eb = (wave & 1) * 32;         // this wave's block inside the tile
-    const int ch = SPLIT ? (wave >> 1) : 0;                                       // its chain half
+    const int t0 = blockIdx.y * TT, e0 = blockIdx.x * TE;
+    const int tb = SPLIT ? 0 : (wave >> 1) * 32, eb = S == 4 ? 0 : (wave & 1) * 32;         // this wave's block inside the tile
+    const int ch = S == 4 ? wave : S == 2 ? wave >> 1 : 0;                     // its quarter or half of the chains
     // ---- global -> register staging: x tile TT rows x 128 floats, gate tile 64 rows x 128 values
-    rm_f4 pa[NA]; rm_u4 pb[GATE_BF16 ? 4 : 8];
+    rm_f4 pa[NA]; rm_u4 pb[NBG];
     auto load_stage = [&](int st) {
         const int k0 = st * RM_KS;
 #pragma unroll
@@ -57,14 +67,14 @@ __global__ void __launch_bounds__(256, SPLIT ? 2 : 1) kr_route_logits_mfma_kerne
         }
         if (GATE_BF16) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
+            for (int i = 0; i < NBG; i++) {
                 const int u = tid + 256 * i, row = u >> 4, c8 = (u & 15) * 8;
                 const int er = min(e0 + row, E - 1);
                 pb[i] = *reinterpret_cast<const rm_u4*>(reinterpret_cast<const uint16_t*>(gate_row) + (size_t)er * H + k0 + c8);
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
+            for (int i = 0; i < NBG; i++) {
                 const int u = tid + 256 * i, row = u >> 5, c4 = (u & 31) * 4;
                 const int er = min(e0 + row, E - 1);
                 pb[i] = *reinterpret_cast<const rm_u4*>(reinterpret_cast<const float*>(gate_row) + (size_t)er * H + k0 + c4);
@@ -75,13 +85,13 @@ __global__ void __launch_bounds__(256, SPLIT ? 2 : 1) kr_route_logits_mfma_kerne
         float* As = reinterpret_cast<float*>(smem + buf * (A_BYTES + B_BYTES));
         char* Bs = smem + buf * (A_BYTES + B_BYTES) + A_BYTES;
 #pragma unroll
-        for (int i = 0; i < NA; i++) { const int u = tid + 256 * i, row = u >> 5, c4 = (u & 31) * 4; *reinterpret_cast<rm_f4*>(As + row * RM_LDA + c4) = pa[i]; }
+        for (int i = 0; i < NA; i++) { const int u = tid + 256 * i, row = u >> 5, c4 = (u & 31) * 4; put(As + row * LDA + c4, pa[i]); }
         if (GATE_BF16) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) { const int u = tid + 256 * i, row = u >> 4, c8 = (u & 15) * 8; *reinterpret_cast<rm_u4*>(Bs + (row * RM_LDB16 + c8) * 2) = pb[i]; }
+            for (int i = 0; i < NBG; i++) { const int u = tid + 256 * i, row = u >> 4, c8 = (u & 15) * 8; put(Bs + (row * LDB16 + c8) * 2, __builtin_bit_cast(rm_f4, pb[i])); }
         } else {
 #pragma unroll
-            for (int i = 0; i < 8; i++) { const int u = tid + 256 * i, row = u >> 5, c4 = (u & 31) * 4; *reinterpret_cast<rm_u4*>(Bs + (row * RM_LDB32 + c4) * 4) = pb[i]; }
+            for (int i = 0; i < NBG; i++) { const int u = tid + 256 * i, row = u >> 5, c4 = (u & 31) * 4; put(Bs + (row * LDB32 + c4) * 4, __builtin_bit_cast(rm_f4, pb[i])); }
         }
     };
     rm_v16f acc[NJ];
@@ -99,21 +109,28 @@ __global__ void __launch_bounds__(256, SPLIT ? 2 : 1) kr_route_logits_mfma_kerne
     for (int st = 0; st < nst; st++) {
         const int buf = st & 1;
         if (st + 1 < nst) load_stage(st + 1);
-        const float* As = reinterpret_cast<const float*>(smem + buf * (A_BYTES + B_BYTES)) + (tb + r) * RM_LDA + 16 * h;
+        const float* As = reinterpret_cast<const float*>(smem + buf * (A_BYTES + B_BYTES)) + (tb + r) * LDA + 16 * h;
         const char* Bs = smem + buf * (A_BYTES + B_BYTES) + A_BYTES;
 #pragma unroll
         for (int m = 0; m < RM_KS / 32; m++) {            // 32 consecutive k: the (s, s+1) pair of every chain
             float a[NJ], b[NJ];
-            if (SPLIT) {      // local chain 2 q + i = chain 4 q + 2 ch + i: two consecutive values per group of four
-                typedef float rm_f2 __attribute__((ext_vector_type(2)));
+            if constexpr (S == 4) {      // local chain q = chain 4 q + ch
+#pragma unroll
+                for (int q = 0; q < 4; q++) a[q] = As[32 * m + 4 * q + ch];
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    if (GATE_BF16) b[q] = __uint_as_float((uint32_t)reinterpret_cast<const uint16_t*>(Bs)[(eb + r) * LDB16 + 32 * m + 16 * h + 4 * q + ch] << 16);
+                    else b[q] = reinterpret_cast<const float*>(Bs)[(eb + r) * LDB32 + 32 * m + 16 * h + 4 * q + ch];
+                }
+            } else if constexpr (SPLIT) {      // local chain 2 q + i = chain 4 q + 2 ch + i: two consecutive values per group of four
 #pragma unroll
                 for (int q = 0; q < 4; q++) { const rm_f2 v = *reinterpret_cast<const rm_f2*>(As + 32 * m + 4 * q + 2 * ch); a[2 * q] = v.x; a[2 * q + 1] = v.y; }
                 if (GATE_BF16) {
-                    const uint16_t* bp = reinterpret_cast<const uint16_t*>(Bs) + (eb + r) * RM_LDB16 + 32 * m + 16 * h + 2 * ch;
+                    const uint16_t* bp = reinterpret_cast<const uint16_t*>(Bs) + (eb + r) * LDB16 + 32 * m + 16 * h + 2 * ch;
 #pragma unroll
                     for (int q = 0; q < 4; q++) { const uint32_t w = *reinterpret_cast<const uint32_t*>(bp + 4 * q); b[2 * q] = __uint_as_float(w << 16); b[2 * q + 1] = __uint_as_float(w & 0xFFFF0000u); }
                 } else {
-                    const float* bp = reinterpret_cast<const float*>(Bs) + (eb + r) * RM_LDB32 + 32 * m + 16 * h + 2 * ch;
+                    const float* bp = reinterpret_cast<const float*>(Bs) + (eb + r) * LDB32 + 32 * m + 16 * h + 2 * ch;
 #pragma unroll
                     for (int q = 0; q < 4; q++) { const rm_f2 v = *reinterpret_cast<const rm_f2*>(bp + 4 * q); b[2 * q] = v.x; b[2 * q + 1] = v.y; }
                 }
@@ -121,7 +138,7 @@ __global__ void __launch_bounds__(256, SPLIT ? 2 : 1) kr_route_logits_mfma_kerne
 #pragma unroll
                 for (int q = 0; q < 4; q++) { const rm_f4 v = *reinterpret_cast<const rm_f4*>(As + 32 * m + 4 * q); a[4 * q] = v.x; a[4 * q + 1] = v.y; a[4 * q + 2] = v.z; a[4 * q + 3] = v.w; }
                 if (GATE_BF16) {
-                    const uint16_t* bp = reinterpret_cast<const uint16_t*>(Bs) + (eb + r) * RM_LDB16 + 32 * m + 16 * h;
+                    const uint16_t* bp = reinterpret_cast<const uint16_t*>(Bs) + (eb + r) * LDB16 + 32 * m + 16 * h;
 #pragma unroll
                     for (int q = 0; q < 2; q++) {
                         const rm_u4 v = *reinterpret_cast<const rm_u4*>(bp + 8 * q);
@@ -130,7 +147,7 @@ __global__ void __launch_bounds__(256, SPLIT ? 2 : 1) kr_route_logits_mfma_kerne
                         for (int p = 0; p < 4; p++) { b[8 * q + 2 * p] = __uint_as_float(w4[p] << 16); b[8 * q + 2 * p + 1] = __uint_as_float(w4[p] & 0xFFFF0000u); }
                     }
                 } else {
-                    const float* bp = reinterpret_cast<const float*>(Bs) + (eb + r) * RM_LDB32 + 32 * m + 16 * h;
+                    const float* bp = reinterpret_cast<const float*>(Bs) + (eb + r) * LDB32 + 32 * m + 16 * h;
 #pragma unroll
                     for (int q = 0; q < 4; q++) { const rm_f4 v = *reinterpret_cast<const rm_f4*>(bp + 4 * q); b[4 * q] = v.x; b[4 * q + 1] = v.y; b[4 * q + 2] = v.z; b[4 * q + 3] = v.w; }
                 }
@@ -142,7 +159,27 @@ __global__ void __launch_bounds__(256, SPLIT ? 2 : 1) kr_route_logits_mfma_kerne
         __syncthreads();
     }
     // ---- the reference's tree over the 16 chains (decode.rs:1419-1427), then + bias (decode.rs:3292)
-    if (SPLIT) {
+    if constexpr (S == 4) {
+        // quarter q's chains q, q + 4, q + 8, q + 12: (a_q + a_q+8) + (a_q+4 + a_q+12); the quarters meet as (c0 + c1) + (c2 + c3)
+        float* xch = reinterpret_cast<float*>(smem) + lane;               // [3 quarters][16][64 lanes]: the stage buffers are free after the last barrier
+        float c[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            c[i] = (acc[0][i] + acc[2][i]) + (acc[1][i] + acc[3][i]);
+            if (ch > 0) xch[((ch - 1) * 16 + i) * 64] = c[i];
+        }
+        __syncthreads();
+        if (ch > 0) return;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            float v = (c[i] + xch[i * 64]) + (xch[(16 + i) * 64] + xch[(32 + i) * 64]);
+            if (bias) v += bv;
+            const int t = t0 + (i & 3) + 8 * (i >> 2) + 4 * h;
+            if (t < T && e < E) logits[(size_t)t * ldo + e] = v;
+        }
+        return;
+    }
+    if constexpr (S == 2) {
         // local chains l = 2 q + i <-> chain 4 q + 2 ch + i: (l0 + l4) + (l2 + l6) is (a0 + a8) + (a4 + a12) for half 0 and (a2 + a10) + (a6 + a14) for half 1
         float* xch = reinterpret_cast<float*>(smem) + ((wave & 1) * 64 + lane) * 16;      // the stage buffers are free after the last barrier
         float half[16];
@@ -174,16 +211,18 @@ __global__ void __launch_bounds__(256, SPLIT ? 2 : 1) kr_route_logits_mfma_kerne
         }
         return;
     }
+    if constexpr (S == 1) {
 #pragma unroll
     for (int i = 0; i < 16; i++) {
-        const float c0 = (acc[0][i] + acc[SPLIT ? 0 : 8][i]) + (acc[4][i] + acc[SPLIT ? 0 : 12][i]);
-        const float c1 = (acc[1][i] + acc[SPLIT ? 0 : 9][i]) + (acc[5][i] + acc[SPLIT ? 0 : 13][i]);
-        const float c2 = (acc[2][i] + acc[SPLIT ? 0 : 10][i]) + (acc[6][i] + acc[SPLIT ? 0 : 14][i]);
-        const float c3 = (acc[3][i] + acc[SPLIT ? 0 : 11][i]) + (acc[7][i] + acc[SPLIT ? 0 : 15][i]);
+        const float c0 = (acc[0][i] + acc[8][i]) + (acc[4][i] + acc[12][i]);
+        const float c1 = (acc[1][i] + acc[9][i]) + (acc[5][i] + acc[13][i]);
+        const float c2 = (acc[2][i] + acc[10][i]) + (acc[6][i] + acc[14][i]);
+        const float c3 = (acc[3][i] + acc[11][i]) + (acc[7][i] + acc[15][i]);
         float v = (c0 + c1) + (c2 + c3);
         if (bias) v += bv;
         const int t = t0 + tb + (i & 3) + 8 * (i >> 2) + 4 * h;
         if (t < T && e < E) logits[(size_t)t * ldo + e] = v;
+    }
     }
 }
 
@@ -191,15 +230,17 @@ __global__ void __launch_bounds__(256, SPLIT ? 2 : 1) kr_route_logits_mfma_kerne
 static int rm_launch(const void* gate_row, int gate_bf16, const float* x, const float* bias, float* out, int T, int E, int H, int ldx, int ldo, int batch, size_t x_bs,
                      size_t g_bs, size_t o_bs, hipStream_t st) {
     if (H % RM_KS || T < 1 || E < 1 || batch < 1) return 1;
-    // too few 64 x 64 tiles for the chip: 32-token tiles with the chains split over wave pairs (bit-identical, see the kernel)
-    const bool split = (long)((E + 63) / 64) * ((T + 63) / 64) * batch < 256;
-    const int tt = split ? 32 : 64;
-    const dim3 grid((E + 63) / 64, (T + tt - 1) / tt, batch);
-    const size_t lds = 2 * ((size_t)tt * RM_LDA * 4 + (gate_bf16 ? (size_t)64 * RM_LDB16 * 2 : (size_t)64 * RM_LDB32 * 4));
+    // too few 64 x 64 tiles for the chip: 32-token tiles with the chains split over the waves (bit-identical, see the kernel), over all four while a unit has at most two of their tiles
+    // (an exact prompt of four layers, 512 experts, halves / quarters, us: 33 tokens 1444 / 1386, 200 2135 / 2079, 512 2960 / 2913, 777 3765 / 3752, 1000 4339 / 4331)
+    const long rows = (T + 31) / 32;
+    const bool split = (long)((E + 63) / 64) * ((T + 63) / 64) * batch < 256, quarters = split && (E + 31) / 32 * rows * batch <= 512;
+    const int tt = split ? 32 : 64, te = quarters ? 32 : 64;
+    const dim3 grid((E + te - 1) / te, (T + tt - 1) / tt, batch);
+    const size_t lds = 2 * ((size_t)tt * RM_LDA * 4 + (gate_bf16 ? (size_t)te * RM_LDB16 * 2 : (size_t)te * RM_LDB32 * 4));
 #define KR_RM(B_, S_) do { if (kr_lds_optin(reinterpret_cast<const void*>(kr_route_logits_mfma_kernel<B_, S_>), lds)) return 1; \
         hipLaunchKernelGGL((kr_route_logits_mfma_kernel<B_, S_>), grid, dim3(256), lds, st, gate_row, x, bias, out, T, E, H, ldx, ldo, x_bs, g_bs, o_bs); } while (0)
-    if (gate_bf16) { if (split) KR_RM(true, true); else KR_RM(true, false); }
-    else { if (split) KR_RM(false, true); else KR_RM(false, false); }
+    if (gate_bf16) { if (quarters) KR_RM(true, 4); else if (split) KR_RM(true, 2); else KR_RM(true, 1); }
+    else { if (quarters) KR_RM(false, 4); else if (split) KR_RM(false, 2); else KR_RM(false, 1); }
 #undef KR_RM
     return 0;
 }

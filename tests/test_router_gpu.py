@@ -128,3 +128,21 @@ def test_decode_rule_batch_logits_tolerance_form(E, H, m, use_bias):
     b = eng.route(0, x, m, RULE_DECODE, want_logits=True)[2]
     check(eng._lib.kr_moe_set_gemm_mode(eng._h, 0))
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.parametrize("bf16_gate", [True, False])
+@pytest.mark.parametrize("E,H", [(512, 2048), (100, 256), (36, 128)])
+def test_matrix_form_of_few_tokens_equals_the_chains(E, H, bf16_gate):
+    # 32 x 32 tiles with the chains in quarters, 32 x 64 with halves, 64 x 64 whole: ragged tokens and experts; sixteen tokens at a time take the vector form
+    rng = np.random.default_rng(E + H + bf16_gate)
+    gate = ((rng.random((E, H), dtype=np.float32) - 0.5) * 0.04).astype(np.float32)
+    if bf16_gate:
+        gate = O.bf16_to_f32(O.f32_to_bf16(gate)).reshape(E, H)
+    eng = _engine(E, H, 4)
+    eng.set_route_weight_f32(0, gate, None, None)
+    most = 2100 if E == 512 else 200
+    x = (rng.random((most, H), dtype=np.float32) - 0.5).astype(np.float32)
+    want = np.concatenate([eng.route(0, x[i:i + 16], len(x[i:i + 16]), RULE_DECODE, want_logits=True)[2] for i in range(0, most, 16)])
+    for m in (32, 33, 65, 200) + ((1024, 1025, 2100) if most > 200 else ()):
+        got = eng.route(0, x[:m], m, RULE_DECODE, want_logits=True)[2]
+        assert np.array_equal(got.view(np.uint32), want[:m].view(np.uint32)), m

@@ -54,17 +54,28 @@ __device__ __forceinline__ void kr_pfm_quant_chunk(const float (&v)[8], int8_t* 
 // value added: mode 0 = add_in[t] (attention / MLP output), mode 1 = embedding row of tokens[t]; first: residual = value.
 // outputs: residual (in place), normalised hidden f32 (null: nobody reads it), optional INT16 digits of the f32 value, optional bf16 copy (routed experts
 // quantise bf16(hidden), decode.rs:3307-3309).
-__global__ void __launch_bounds__(256) kr_pfm_norm_kernel(const KrPfmNormArgs a) {
-    extern __shared__ __attribute__((aligned(16))) float r[];   // [H + 4]
+__global__ void __launch_bounds__(256) kr_pfm_norm_kernel(const KrPfmNormArgs a, const int ld /* of the chains' copy; 0: too long a row for it */) {
+    extern __shared__ __attribute__((aligned(16))) float r[];   // [H + 4], then [8][ld]: the same numbers as the eight chains of the sum of squares take them (16 bytes a read; one
+                                                                // number at a time: 777 rows of 2048 11.0 us against 8.6, a tolerance prompt of 8192 tokens 10.48 ms against 10.33)
     __shared__ uint32_t s_max;
     const int t = blockIdx.x, H = a.H, tid = threadIdx.x;
+    float* rt = r + (H + 7) / 4 * 4;
     if (tid == 0) s_max = 0;
     const float* add = a.mode == 1 ? a.emb + (size_t)a.tokens[t] * H : a.add_in + (size_t)t * H;
     float* res = a.res + (size_t)t * H;
-    for (int i = tid; i < H; i += 256) { const float v = a.first ? add[i] : (add[i] + res[i]); r[i] = v; res[i] = v; }
+    if (H % 4 == 0 && (((uintptr_t)add | (uintptr_t)res) & 15) == 0) {
+        for (int c = tid; c < H / 4; c += 256) {
+            float4 v = reinterpret_cast<const float4*>(add)[c];
+            if (!a.first) { const float4 o = reinterpret_cast<const float4*>(res)[c]; v = make_float4(v.x + o.x, v.y + o.y, v.z + o.z, v.w + o.w); }
+            reinterpret_cast<float4*>(r)[c] = v; reinterpret_cast<float4*>(res)[c] = v;
+            float* q = rt + (c & 1) * 4 * ld + (c >> 1);
+            if (ld) { q[0] = v.x; q[ld] = v.y; q[2 * ld] = v.z; q[3 * ld] = v.w; }
+        }
+    } else
+        for (int i = tid; i < H; i += 256) { const float v = a.first ? add[i] : (add[i] + res[i]); r[i] = v; res[i] = v; if (ld) rt[(i & 7) * ld + (i >> 3)] = v; }
     __syncthreads();
     if (tid < 8) {
-        float ss = kr_pfm_sumsq8(r, H, tid);
+        float ss = ld ? kr_pfm_hsum8(kr_sumsq_lane_t(rt, ld, H, tid)) : kr_pfm_sumsq8(r, H, tid);
         if (tid == 0) { for (int q = (H / 8) * 8; q < H; q++) ss += r[q] * r[q]; r[H] = 1.0f / sqrtf(ss / (float)H + a.eps); }
     }
     __syncthreads();
@@ -901,7 +912,9 @@ __global__ void __launch_bounds__(256) kr_pfm_moe_epilogue_kernel(const float* _
 // launchers
 // ------------------------------------------------------------------------------------------
 void kr_launch_pfm_norm(const KrPfmNormArgs& a, int C, hipStream_t st) {
-    hipLaunchKernelGGL(kr_pfm_norm_kernel, dim3(C), dim3(256), (size_t)(a.H + 4) * 4, st, a);
+    const int row = (a.H + 7) / 4 * 4, ld = (a.H / 8 + 4) / 4 * 4 + 4;
+    const bool copy = (size_t)(row + 8 * ld) * 4 <= 64 * 1024 - 16;
+    hipLaunchKernelGGL(kr_pfm_norm_kernel, dim3(C), dim3(256), (size_t)(row + (copy ? 8 * ld : 0)) * 4, st, a, copy ? ld : 0);
 }
 void kr_launch_pfm_quant_f32(const float* x, int rows, int ld, int K, int8_t* xh, int8_t* xl, float* xs, hipStream_t st) {
     const int thr = K / 8 < 1024 ? ((K / 8 + 15) / 16) * 16 : 1024;

@@ -173,3 +173,17 @@ def test_prefill_argument_errors():
         st.prefill([1, 2, 3], d["kv_max"] - 1)            # does not fit kv_max_seq
     with pytest.raises(ValueError):
         st.prefill([d["V"] + 5], 0)                       # token id out of range
+
+
+@pytest.mark.parametrize("H", [384, 8064, 8192])
+def test_norm_rows_with_and_without_the_chains_copy(H):
+    # the copy of a row that the norm's eight chains read fits the LDS up to 8064 columns
+    st, eng, orc, keep, d = build(seed=29, dims=(H, 512, 8, 2, 128, 128), kinds=["la", "gqa"])
+    toks = [int(x) for x in np.random.default_rng(3).integers(0, d["V"], 6)]
+    ref = np.empty(d["V"], F); got = np.empty(d["V"], F)
+    for i, t in enumerate(toks):
+        st.decode_step(t, 2 + i, ref.ctypes.data)
+    tok = st.last_token()
+    d["reset"]()
+    assert st.prefill(toks, 2, got.ctypes.data) == tok
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))

@@ -25,8 +25,8 @@
 // kernel; experts only, 8192 tokens: 1.07 against 1.03 ms per layer.  Timing-only ablations of the same loop: without the conversion 1050 - 1080 TFLOP/s,
 // without requests, reads and conversion 1290, the 16 MFMAs of a unit alone 1024 matrix-pipe cycles per SIMD against 1890 measured -- the two waves of a SIMD
 // issue 2 x (16 MFMA + ~125 VALU) x 4 cycles = 1130 cycles through one vector port per unit: the conversion (7.8 vector instructions per MFMA at a 64 x 64
-// wave tile), not the operand staging, is what bounds BOTH forms.  So the dispatch keeps the register-staged kernel (two workgroups per CU also hide each
-// other's prologue and store phase, ~10 k cycles per tile here); this form stays selectable (kr_moe_set_gemm_mode 5, option "gemm_ring" 2) and tested.
+// wave tile), not the operand staging, is what bounds BOTH forms.  So the dispatch never takes it by itself (INT4 products of 512 rows and more go to kr_prefill_w.hip, the others to the register-staged kernel, whose two
+// workgroups per CU hide each other's prologue and store phase, ~10 k cycles per tile here); this form stays selectable (kr_moe_set_gemm_mode 5, option "gemm_ring" 2) and tested.
 //
 // Tiles: 8 waves as WM x WN, wave tile 64 x 64 (2 x 2 accumulators of 32 x 32, as the register-staged kernel): 64 x 512 for the experts (the 64-row tile table
 // of kr_launch_pf_sort; B ring of 2 stages = 128 KiB, A ring of 3) and 128 x 256 for the dense projections (B ring of 2 = 64 KiB, A ring of 4).

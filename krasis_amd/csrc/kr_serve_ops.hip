@@ -2031,12 +2031,17 @@ __global__ void __launch_bounds__(256) sv_lin_cscan_kernel(const KrSvLin a) {
 // products are formed transposed: S^T[s][t] = K Q^T (queries of the wave's tokens stay in registers: lane (t = lane % 16, quarter = lane / 16) keeps
 // the quarter-th part of q_t), O^T[c][t] += V^T P^T with the weights where the first product left them; the state's share S_start^T q_t goes into the
 // same accumulators first.  DQ >= ceil(dim / 4), DB >= ceil(vdim / 16).
-template <bool ML, int DB>
-__global__ void __launch_bounds__(256) sv_lin_cout_kernel(const KrSvLin a) {
+// DIM > 0: that dim, vdim = 16 DB, key rows of whole 16-byte pieces; the queries in registers, so that four workgroups share a unit and not three.  A vector instruction between two f32 matrix instructions costs about 20 clocks (kr_serve_tile_f32.hip), and the
+// guards put one beside every product: here products come in runs of 16 on operands read before them, from addresses that stand still.  Same products, same order.
+// 3249 tokens of two requests, 16 heads of 128 x 128: 108 -> 55 us (three workgroups a unit 61; without the registers 91).
+template <bool ML, int DB, int DIM>
+__global__ void __launch_bounds__(256, DIM > 0 ? 4 : 1) sv_lin_cout_kernel(const KrSvLin a) {
+    constexpr bool FULL = DIM > 0;
+    constexpr int UNROLL = FULL ? DIM / 64 : 1;
     extern __shared__ __attribute__((aligned(16))) float sl[];      // [32][lds] rows of the block's start state | [4 waves][dq][64] the waves' queries
     const int gc = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, kq = lane >> 4;
-    const int H = a.heads, dim = a.dim, vdim = a.vdim, dq = 4 * ((dim + 15) / 16);
-    const int lds = ((vdim + 31) / 32) * 32 + 16;                   // rows 16 banks apart: the lanes of two neighbouring rows fall into distinct banks
+    const int H = a.heads, dim = FULL ? DIM : a.dim, vdim = FULL ? 16 * DB : a.vdim, dq = 4 * ((dim + 15) / 16);
+    const int lds = FULL ? 16 * DB + 16 : ((vdim + 31) / 32) * 32 + 16;      // rows 16 banks apart: the lanes of two neighbouring rows fall into distinct banks
     float* qs = sl + 32 * lds + (size_t)wave * dq * 64;             // this wave's queries, one word per (step, lane): a register file that loops can index
     int e = 0;
     while (e + 1 < a.n_entries && a.ent_chunk0[e + 1] <= gc) e++;
@@ -2051,13 +2056,59 @@ __global__ void __launch_bounds__(256) sv_lin_cout_kernel(const KrSvLin a) {
     // d = 16 (i / 4) + 4 kq + i % 4, so that four steps of a lane are 16 contiguous bytes of a key row
     auto dof = [&](int i) { return 16 * (i >> 2) + 4 * kq + (i & 3); };
     const bool kvec = (a.ld & 3) == 0 && (dim & 15) == 0;          // key rows start 16-byte aligned and hold whole pieces
-    for (int i = 0; i < dq; i++) { const int d = dof(i); qs[i * 64 + lane] = (active && d < dim) ? zq[tg * a.ld + d] : 0.0f; }
+    float qr[FULL ? DIM / 4 : 1];
+    if constexpr (FULL) {
+#pragma unroll
+        for (int j = 0; j < DIM / 16; j++) {
+            const float4 q4 = *reinterpret_cast<const float4*>(zq + tg * a.ld + 16 * j + 4 * kq);
+            qr[4 * j] = q4.x; qr[4 * j + 1] = q4.y; qr[4 * j + 2] = q4.z; qr[4 * j + 3] = q4.w;
+        }
+    } else
+        for (int i = 0; i < dq; i++) { const int d = dof(i); qs[i * 64 + lane] = (active && d < dim) ? zq[tg * a.ld + d] : 0.0f; }
     sv_f4 acc[DB];
 #pragma unroll
     for (int c = 0; c < DB; c++) acc[c] = sv_f4{0.0f, 0.0f, 0.0f, 0.0f};
     const float* Sc = a.sbuf + ((size_t)gc * H + h) * dim * vdim;
     const float* nc = a.nbuf + ((size_t)gc * H + h) * dim;
     float den = 0.0f;
+    if constexpr (FULL) {
+        constexpr int V4 = 4 * DB, NP = 32 * V4 / 256, G = 2;      // 16-byte pieces of a row; of a pass, per thread; steps whose rows are read together (four: 132 registers)
+        sv_f4 pre[NP];
+#pragma unroll
+        for (int j = 0; j < NP; j++) pre[j] = reinterpret_cast<const sv_f4*>(Sc)[tid + 256 * j];
+#pragma unroll
+        for (int p0 = 0; p0 < DIM; p0 += 32) {
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < NP; j++) { const int idx = tid + 256 * j; *reinterpret_cast<sv_f4*>(sl + idx / V4 * lds + 4 * (idx % V4)) = pre[j]; }
+            if (p0 + 32 < DIM) {
+#pragma unroll
+                for (int j = 0; j < NP; j++) pre[j] = reinterpret_cast<const sv_f4*>(Sc + (size_t)(p0 + 32) * vdim)[tid + 256 * j];
+            }
+            __syncthreads();
+            if (active) {
+            const float* srow = sl + 4 * kq * lds + r;
+#pragma unroll
+            for (int i4 = 0; i4 < 8; i4 += G) {
+                float sv[G][DB];
+#pragma unroll
+                for (int i = 0; i < G; i++)
+#pragma unroll
+                    for (int c = 0; c < DB; c++) sv[i][c] = srow[(16 * ((i4 + i) >> 2) + ((i4 + i) & 3)) * lds + c * 16];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < G; i++)
+#pragma unroll
+                    for (int c = 0; c < DB; c++) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(sv[i][c], qr[p0 / 4 + i4 + i], acc[c], 0, 0, 0);
+                if constexpr (ML) {
+#pragma unroll
+                    for (int i = 0; i < G; i++) den = __builtin_fmaf(qr[p0 / 4 + i4 + i], nc[p0 + dof(i4 + i)], den);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            }
+        }
+    } else
     for (int p0 = 0; p0 < dim; p0 += 32) {                          // passes over 32 rows of the state
         const int rows = min(32, dim - p0);
         __syncthreads();
@@ -2091,11 +2142,19 @@ __global__ void __launch_bounds__(256) sv_lin_cout_kernel(const KrSvLin a) {
     for (int stile = 0; stile <= wave; stile++) {
         const float* krow = zk + ((size_t)tb + min(stile * 16 + r, nt - 1)) * a.ld;
         sv_f4 st = sv_f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll UNROLL
         for (int i0 = 0; i0 < dq; i0 += 16) {                    // sixteen key coordinates and queries requested at a time, then their products
             float kf[16], qf[16];
 #pragma unroll
-            for (int i = 0; i < 16; i++) qf[i] = i0 + i < dq ? qs[(i0 + i) * 64 + lane] : 0.0f;
-            if (kvec) {
+            for (int i = 0; i < 16; i++) qf[i] = FULL ? qr[FULL ? i0 + i : 0] : i0 + i < dq ? qs[(i0 + i) * 64 + lane] : 0.0f;
+            if (FULL) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float4 k4 = *reinterpret_cast<const float4*>(krow + 16 * (i0 / 4 + j) + 4 * kq);
+                    kf[4 * j] = k4.x; kf[4 * j + 1] = k4.y; kf[4 * j + 2] = k4.z; kf[4 * j + 3] = k4.w;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            } else if (kvec) {
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     const float4 k4 = i0 + 4 * j < dq ? *reinterpret_cast<const float4*>(krow + 16 * (i0 / 4 + j) + 4 * kq) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -2124,11 +2183,13 @@ __global__ void __launch_bounds__(256) sv_lin_cout_kernel(const KrSvLin a) {
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int c = 0; c < DB; c++) { const int cc = c * 16 + r; vf[i][c] = cc < vdim ? zv[srow[i] * a.ld + cc] : 0.0f; }
+            for (int c = 0; c < DB; c++) { const int cc = c * 16 + r; vf[i][c] = FULL || cc < vdim ? zv[srow[i] * a.ld + cc] : 0.0f; }
+        if (FULL) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
             for (int c = 0; c < DB; c++) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][c], st[i], acc[c], 0, 0, 0);
+        if (FULL) __builtin_amdgcn_sched_barrier(0);
     }
     const float inv = ML ? 1.0f / (fmaxf(fabsf(den), me.w) + 1e-6f) : 1.0f;
     if (!tv) return;
@@ -2762,8 +2823,13 @@ void kr_sv_lin_block_out(const KrSvLin& a, hipStream_t st) {
     const dim3 go(a.n_chunks, a.heads);
     const bool small = a.dim <= 64 && a.vdim <= 64;
     const size_t lds = ((size_t)32 * (((a.vdim + 31) / 32) * 32 + 16) + (size_t)4 * (4 * ((a.dim + 15) / 16)) * 64) * sizeof(float);
-#define SV_CO(ML_) do { if (small) hipLaunchKernelGGL((sv_lin_cout_kernel<ML_, 4>), go, dim3(256), lds, st, a); \
-                        else hipLaunchKernelGGL((sv_lin_cout_kernel<ML_, 8>), go, dim3(256), lds, st, a); } while (0)
+    const bool whole = a.ld % 4 == 0 && (uintptr_t)a.z % 16 == 0;
+    const size_t lds_whole = (size_t)32 * (a.vdim + 16) * sizeof(float);
+#define SV_CO(ML_) do { if (whole && a.dim == 64 && a.vdim == 64) hipLaunchKernelGGL((sv_lin_cout_kernel<ML_, 4, 64>), go, dim3(256), lds_whole, st, a); \
+                        else if (whole && a.dim == 64 && a.vdim == 128) hipLaunchKernelGGL((sv_lin_cout_kernel<ML_, 8, 64>), go, dim3(256), lds_whole, st, a); \
+                        else if (whole && a.dim == 128 && a.vdim == 128) hipLaunchKernelGGL((sv_lin_cout_kernel<ML_, 8, 128>), go, dim3(256), lds_whole, st, a); \
+                        else if (small) hipLaunchKernelGGL((sv_lin_cout_kernel<ML_, 4, 0>), go, dim3(256), lds, st, a); \
+                        else hipLaunchKernelGGL((sv_lin_cout_kernel<ML_, 8, 0>), go, dim3(256), lds, st, a); } while (0)
     if (ml) SV_CO(true); else SV_CO(false);
 #undef SV_CO
 }

@@ -131,7 +131,27 @@ def test_decode_rule_batch_logits_tolerance_form(E, H, m, use_bias):
 
 
 @pytest.mark.parametrize("bf16_gate", [True, False])
-@pytest.mark.parametrize("E,H", [(512, 2048), (100, 256), (36, 128)])
+@pytest.mark.parametrize("E", [1, 3, 16, 17, 33, 50, 130])       # a workgroup has four blocks of four experts: nothing but a part of a block, whole workgroups, one to three experts past them
+def test_vector_form_counts_every_expert(E, bf16_gate):
+    H, m, k = 256, 5, min(E, 4)
+    rng = np.random.default_rng(E + bf16_gate)
+    gate = ((rng.random((E, H), dtype=np.float32) - 0.5) * 0.04).astype(np.float32)
+    if bf16_gate:
+        gate = O.bf16_to_f32(O.f32_to_bf16(gate)).reshape(E, H)
+    bias = ((rng.random(E, dtype=np.float32) - 0.5) * 0.1).astype(np.float32)
+    eng = _engine(E, H, k)
+    x = (rng.random((2 * m, H), dtype=np.float32) - 0.5).astype(np.float32)
+    for use_bias, xs in ((bias, x[:m]), (None, x[m:])):          # the second pass would find the first one's logits where it leaves any out
+        eng.set_route_weight_f32(0, gate, use_bias, None)
+        ids, w, lg = eng.route(0, xs, m, RULE_DECODE, want_logits=True)
+        for t in range(m):
+            r_ids, r_w, r_lg = O.route_decode(gate, xs[t], k, 1, True, use_bias, None)
+            assert np.array_equal(lg[t].view(np.uint32), r_lg.view(np.uint32)), ("logits", t)
+            assert np.array_equal(ids[t], r_ids) and np.array_equal(w[t].view(np.uint32), r_w.view(np.uint32)), t
+
+
+@pytest.mark.parametrize("bf16_gate", [True, False])
+@pytest.mark.parametrize("E,H", [(512, 2048), (100, 256), (36, 128), (33, 128)])
 def test_matrix_form_of_few_tokens_equals_the_chains(E, H, bf16_gate):
     # 32 x 32 tiles with the chains in quarters, 32 x 64 with halves, 64 x 64 whole: ragged tokens and experts; sixteen tokens at a time take the vector form
     rng = np.random.default_rng(E + H + bf16_gate)

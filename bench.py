@@ -1183,7 +1183,7 @@ def prefill_experts(eng, dims, L, M, torch, gemm_fast=False, gemm_mode=None):
     ids = torch.rand((M, E), device="cuda", generator=g).topk(k, dim=1).indices.to(torch.int32)
     w = torch.softmax(torch.randn((M, k), device="cuda", generator=g), dim=1)
     mgr = GpuPrefillManager(eng, k)
-    # gemm_mode 3: tolerance form on the register-staged kernels only (A/B against the default LDS-ring form, same bits)
+    # gemm_mode 3: tolerance form on the register-staged kernels only (A/B against the default dispatch, same bits)
     _lib.check(eng._lib.kr_moe_set_gemm_mode(eng._h, gemm_mode if gemm_mode is not None else (1 if gemm_fast else 0)))
     try:
         for l in range(L):      # every layer builds its derived tables on first use (per-weight nibble sums; the tolerance copy of GGUF layers) -- outside the timed region
@@ -1197,8 +1197,6 @@ def prefill_experts(eng, dims, L, M, torch, gemm_fast=False, gemm_mode=None):
         ev1.record(); torch.cuda.synchronize()
         allocs = alloc_count() - a0
     finally:
-        if gemm_mode is not None:
-            _lib.check(eng._lib.kr_moe_set_gemm_mode(eng._h, 1))       # the ring kernel back to its default dispatch
         _lib.check(eng._lib.kr_moe_set_gemm_mode(eng._h, 0))
     ms = ev0.elapsed_time(ev1)
     if allocs:

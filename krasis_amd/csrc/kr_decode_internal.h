@@ -58,6 +58,7 @@ struct kr_decode_store {
     int* gen_ring = nullptr; int gen_ring_n = 0; hipEvent_t gen_ev[2] = {nullptr, nullptr};   // pinned token ring + events of the look-ahead loop
     int decode_fast = 0; DevBuf f_qk;         // KR_DECODE_FAST: decode steps on the tolerance-mode kernels (kr_decode_fast.hip); f_qk = conv outputs [nk][q(dk) | k(dk)]
     int gemm_fast = 0;                        // KR_GEMM_FAST: prompt-pass GEMMs in the tolerance form (kr_prefill_h.hip)
+    KrPfhForm gemm_form = KR_PFH_AUTO;        // ... and on which kernels (option "gemm_ring")
     int attn_fast = 0; DevBuf fd_o, fd_ml;   // KR_ATTN_FAST: split-KV softmax + p.v with a log-sum-exp merge for long caches (tolerance mode)
     DevBuf gqa_scores; int gqa_split_min = 1024, mla_split_min = 512;   // caches longer than this split decode attention into a scores launch + softmax / p.v launch
     bool fuse_la = true;       // conv + recurrence + gated norm of a linear-attention layer in one launch (kr_la_step_kernel)

@@ -44,7 +44,7 @@ size_t al(size_t n) { return (n + 255) & ~(size_t)255; }
 
 static int pf_gemm(kr_decode_store* s, int wid, const Act& A, int C, float* out, int ld, hipStream_t st) {
     DWeight& W = *s->weights[wid];
-    if (s->gemm_fast) { kr_launch_pfh_gemm(W.ms.view(), A.f, A.fm, nullptr, 1, 0, 0, C, out, ld, st); return KR_OK; }
+    if (s->gemm_fast) { kr_launch_pfh_gemm(W.ms.view(), A.f, A.fm, nullptr, 1, 0, 0, C, out, ld, st, 0, 0, 1, nullptr, nullptr, s->gemm_form); return KR_OK; }
     if (!W.ms.wsum.p) return kr_fail(KR_ERR_STATE, "internal: nibble sums of weight %d were not prepared", wid);
     kr_launch_pf_gemm(W.ms.view(), (const uint32_t*)W.ms.wsum.p, A.h, A.l, A.s, nullptr, 1, 0, 0, C, out, ld, st);
     return KR_OK;
@@ -60,7 +60,7 @@ static int pf_gemm_multi(kr_decode_store* s, const int* wids, float* const* outs
         if (i < 3) { mats[i] = W.ms.view(); ws[i] = (const uint32_t*)W.ms.wsum.p; same = same && mats[i].bits == mats[0].bits && mats[i].ng == mats[0].ng; }
     }
     if (same && n > 1) {
-        if (s->gemm_fast) kr_launch_pfh_gemm_multi(mats, outs, lds, n, A.f, A.fm, C, st);
+        if (s->gemm_fast) kr_launch_pfh_gemm_multi(mats, outs, lds, n, A.f, A.fm, C, st, s->gemm_form);
         else kr_launch_pf_gemm_multi(mats, ws, outs, lds, n, A.h, A.l, A.s, C, st);
         return KR_OK;
     }
@@ -195,7 +195,7 @@ static int run_layer(kr_decode_store* s, Chunk& cx, size_t li) {
         // prefill_impl pads ranks that have fewer chunks with empty-shard calls.  Every chunk in flight has its own exchange-buffer set (cx.set) and stream; the
         // collectives of all chunks are ISSUED in one host order that is the same on every rank (the loop structure below depends only on the agreed chunk count).
         if (e->ep) { if (int rc = kr_moe_prefill_ep_set(e, L.moe_layer, B.xb, B.ids, B.w, B.moe, Cc, k, KR_OUT_F32, 1, cx.set, st ? (void*)st : (void*)1)) return rc; }
-        else if (int rc = kr_moe_prefill_set(e, L.moe_layer, B.xb, B.ids, B.w, B.moe, Cc, k, KR_OUT_F32, 1, cx.set | (s->gemm_fast ? KR_PF_SET_FAST : 0) | (cx.sy.rec_a ? KR_PF_SET_BESIDE : 0), st)) return rc;
+        else if (int rc = kr_moe_prefill_set(e, L.moe_layer, B.xb, B.ids, B.w, B.moe, Cc, k, KR_OUT_F32, 1, cx.set | (s->gemm_fast ? KR_PF_SET_FAST | KR_PF_SET_FORM(s->gemm_form) : 0) | (cx.sy.rec_a ? KR_PF_SET_BESIDE : 0), st)) return rc;
         const bool has_shared = L.sgu_wid >= 0, has_gate = has_shared && L.sg_wid >= 0;
         if (has_shared) {   // decode-store numerics: f32 input digits, fast_silu_mul + f32::round digits (decode.rs:3356-3378)
             const int si2 = s->weights[L.sgu_wid]->rows, SI = si2 / 2;

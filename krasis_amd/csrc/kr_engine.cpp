@@ -1017,7 +1017,7 @@ static int moe_prefill_gguf(kr_engine* e, Layer& L, int layer, const void* x_bf1
 // kr_moe_prefill in the tolerance form (kr_moe_set_gemm_mode(e, 1)): same launches, the activations travel as f16 rows and the GEMMs run on the
 // f16 matrix cores with f32 accumulation over the whole k range (kr_prefill_h.hip).  Sort, combine, routing weights and skip rules are the exact path's.
 static int moe_prefill_fast(kr_engine* e, Layer& L, const void* x_bf16, const int32_t* ids, const float* wts, void* out, int M, int topk,
-                            int out_dtype, int routed_only, int set, hipStream_t st) {
+                            int out_dtype, int routed_only, int set, KrPfhForm form, hipStream_t st) {
     kr_engine::PfSet& P = e->pf[set % KR_PF_MAX_DEPTH];
     const int H = e->cfg.hidden_size, I = L.inter, E = e->cfg.n_routed_experts;
     const bool use_shared = L.shared_present && !routed_only;
@@ -1047,18 +1047,20 @@ static int moe_prefill_fast(kr_engine* e, Layer& L, const void* x_bf16, const in
         const int mc = M - m0 < CH ? M - m0 : CH;
         const uint16_t* xc = (const uint16_t*)x_bf16 + (size_t)m0 * H;
         const int32_t* idc = ids + (size_t)m0 * topk; const float* wc = wts + (size_t)m0 * topk;
-        const KrPfTiles cut = kr_pfh_tiles(L.w13.view(), L.w2.view(), mc, (long)mc * topk, E);
+        const KrPfTiles cut = kr_pfh_tiles(L.w13.view(), L.w2.view(), mc, (long)mc * topk, E, form);
         int run = (int)(((long)mc * topk / E + cut.rows - 1) / cut.rows);           // row tiles of an average expert: they share an XCD (one L2 fill of its weights)
         run = run < 1 ? 1 : (run > 4 ? 4 : run);
         kr_launch_pf_sort(idc, mc, topk, E, so, st, cut);
         kr_launch_pfh_rows_bf16(xc, mc, H, H, (uint16_t*)P.xf.p, (float*)P.xfm.p, st);
         kr_launch_pfh_w13_act(L.w13.view(), (const uint16_t*)P.xf.p, (const float*)P.xfm.p, &so, topk, 1, cut.max_tiles, 0, (float*)P.gu.p, mc * topk, act_mode, e->cfg.swiglu_limit,
-                              e->cfg.activation_alpha, (uint16_t*)P.hf.p, (float*)P.hfm.p, st, run, nullptr, nullptr, &cut);
-        kr_launch_pfh_gemm(L.w2.view(), (const uint16_t*)P.hf.p, (const float*)P.hfm.p, &so, topk, 0, cut.max_tiles, 0, (float*)P.eo.p, H, st, 0, 2 /* f16 rows */, run, nullptr, &cut);
+                              e->cfg.activation_alpha, (uint16_t*)P.hf.p, (float*)P.hfm.p, st, run, nullptr, nullptr, &cut, form);
+        kr_launch_pfh_gemm(L.w2.view(), (const uint16_t*)P.hf.p, (const float*)P.hfm.p, &so, topk, 0, cut.max_tiles, 0, (float*)P.eo.p, H, st, 0, 2 /* f16 rows */, run, nullptr, &cut, form);
         if (use_shared) {
-            kr_launch_pfh_gemm(L.sw13.view(), (const uint16_t*)P.xf.p, (const float*)P.xfm.p, nullptr, topk, 0, 0, mc, (float*)P.sgu.p, 2 * SI, st);
+            kr_launch_pfh_gemm(L.sw13.view(), (const uint16_t*)P.xf.p, (const float*)P.xfm.p, nullptr, topk, 0, 0, mc, (float*)P.sgu.p, 2 * SI, st, 0, 0, 1, nullptr, nullptr,
+                               form);
             kr_launch_pfh_act((const float*)P.sgu.p, mc, SI, 2 * SI, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (uint16_t*)P.shf.p, (float*)P.shfm.p, st);
-            kr_launch_pfh_gemm(L.sw2.view(), (const uint16_t*)P.shf.p, (const float*)P.shfm.p, nullptr, topk, 0, 0, mc, (float*)P.seo.p, H, st);
+            kr_launch_pfh_gemm(L.sw2.view(), (const uint16_t*)P.shf.p, (const float*)P.shfm.p, nullptr, topk, 0, 0, mc, (float*)P.seo.p, H, st, 0, 0, 1, nullptr, nullptr,
+                               form);
         }
         kr_launch_pf_combine_f16rows((const uint16_t*)P.eo.p, (const float*)P.hfm.p, so.pair_row, wc, mc, topk, H, use_shared ? (const float*)P.seo.p : nullptr, e->cfg.routed_scaling_factor,
                                      (char*)out + (size_t)m0 * H * ob, out_dtype == KR_OUT_BF16, st);
@@ -1080,6 +1082,7 @@ int kr_moe_prefill_set(kr_engine* e, int layer, const void* x_bf16, const int32_
     std::lock_guard<std::mutex> lk(e->mu);
     KR_HIP(hipSetDevice(e->device));
     const bool fast = e->gemm_fast || (set & KR_PF_SET_FAST), beside = (set & KR_PF_SET_BESIDE) != 0;
+    const KrPfhForm form = set & KR_PF_SET_FORM(0) ? (KrPfhForm)(set >> 10 & 3) : e->gemm_form;
     set &= 0xFF;
     if (L.gguf) {      // native GGUF blocks: the exact int8-MFMA form, or (tolerance mode, Q4_K layers) f16 MFMA on the re-tiled copy
         if (fast && gg_fast_ok(L, e->cfg.hidden_size, L.gguf_shared && !routed_only)) return moe_prefill_gguf_fast(e, L, x_bf16, ids, wts, out, M, topk, out_dtype, routed_only, set, st);
@@ -1087,7 +1090,7 @@ int kr_moe_prefill_set(kr_engine* e, int layer, const void* x_bf16, const int32_
     }
     if (e->cfg.hidden_size % 128 || L.inter % 128) return kr_fail(KR_ERR_VALUE, "prefill path needs dims divisible by 128");
     if (fast && (!L.shared_present || routed_only || L.shared_inter % 128 == 0))
-        return moe_prefill_fast(e, L, x_bf16, ids, wts, out, M, topk, out_dtype, routed_only, set, st);
+        return moe_prefill_fast(e, L, x_bf16, ids, wts, out, M, topk, out_dtype, routed_only, set, form, st);
     kr_engine::PfSet& P = e->pf[set % KR_PF_MAX_DEPTH];
     const int H = e->cfg.hidden_size, I = L.inter, E = e->cfg.n_routed_experts;
     const bool use_shared = L.shared_present && !routed_only;
@@ -1225,7 +1228,7 @@ extern "C" int kr_moe_set_gemm_mode(kr_engine* e, int fast) {
     if (fast != 0 && fast != 1 && fast != 3 && fast != 5) return kr_fail(KR_ERR_VALUE, "gemm mode %d unknown (0 = exact, 1 = fast, 3 = fast on the register-staged kernels only, 5 = fast with the ring kernel for every shape it takes)", fast);
     std::lock_guard<std::mutex> lk(e->mu);
     e->gemm_fast = fast & 1;
-    if (fast) kr_pfr_set_enabled(fast == 1 ? 1 : (fast == 5 ? 2 : 0));      // 3: A/B and test hook, process-wide -- the LDS-ring GEMM (kr_prefill_ring.hip) off; results are bit-identical either way
+    e->gemm_form = fast == 3 ? KR_PFH_STAGED : fast == 5 ? KR_PFH_RING : KR_PFH_AUTO;
     return KR_OK;
 }
 

@@ -4,7 +4,10 @@
 #include <stddef.h>
 #include <stdint.h>
 
-// One quantized [K -> N] matrix in the lane-tiled HBM layout (DESIGN.md §3):
+// Which kernels take the INT4 problems of the tolerance GEMMs; the same bits from all.  A choice of the engine's (kr_moe_set_gemm_mode) or the decode store's (option "gemm_ring"), never the process's.
+enum KrPfhForm { KR_PFH_STAGED = 0 /* kr_prefill_h.hip's only */, KR_PFH_AUTO = 1 /* by size: kr_prefill_w.hip for problems that fill the chip */, KR_PFH_RING = 2 /* kr_prefill_ring.hip wherever it can */ };
+
+// One quantized [K -> N] matrix in the lane-tiled HBM layout:
 //   INT4-g128: q = [N/8 tiles][ngp group-pairs][64 lanes] x 16 B, lane = col*8 + l holds packed words
 //              {W(g0,2l), W(g0,2l+1), W(g1,2l), W(g1,2l+1)}, W(g,i) = nibbles k = g*128+8i..+8 of the column
 //   INT8-g128: q = [N/8 tiles][ng groups][64 lanes] x 16 B, lane holds k = g*128+16l..+16 of the column

@@ -48,6 +48,7 @@ struct KrPfGemmHArgs {
     int run;                                 // experts: consecutive row tiles given to one XCD (> 1: the tiles of one expert share an L2)
     int sr, sc;                              // dense: super-tile of sr row tiles x sc column blocks per XCD (kr_pf_super_tile)
     int n_extra; KrMatDev mx[2]; float* outx[2]; int out_ldx[2];
+    KrPfhForm form;
 };
 
 // one packed INT4 word (nibbles k .. k + 7 of a column) -> 8 f16 in the order (0,4,1,5,2,6,3,7); sq = s / 4 (both halves), cq = -1536 * sq.
@@ -148,6 +149,5 @@ __device__ __forceinline__ void pfh_store_tile(const ACC& acc, int nsb, int rows
 #define KR_PFW_ROWS 96
 bool kr_pfw_dense(const KrPfGemmHArgs& a);      // a dense problem that it takes
 void kr_pfw_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st);
-bool kr_pfr_default();                          // neither of the other two forms is asked for by name (kr_pfr_set_enabled)
 // kr_prefill_ring.hip: the LDS-ring form of the INT4 GEMM; 0 = launched, 1 = this shape stays on the register-staged kernel.  mt64 = 64-row tiles of the experts' tile table
 int kr_pfr_try_launch(const KrPfGemmHArgs& a, int mt64, hipStream_t st);

@@ -61,11 +61,11 @@ void kr_launch_pfh_act(const float* gu, int rows, int n, int gu_ld, int act_mode
                        uint16_t* sums32 = nullptr);     // act_mode 3 = libm SiLU of expert_forward_gguf (rows of at most 2048 values)
 void kr_launch_pfh_gemm(const KrMatDev& m, const uint16_t* a_h, const float* a_mul, const KrPfSort* sort, int topk, int gather_tokens, int max_tiles,
                         int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows = 0, int out_bf16 = 0, int run = 1,
-                        const uint16_t* a_sum32 = nullptr /* required when m.qs is set (Q4_K copy) */, const KrPfTiles* t = nullptr /* of the tile table; null: tiles of 64 */);
-KrPfTiles kr_pfh_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows, int E);      // of the tolerance GEMMs' tile table
+                        const uint16_t* a_sum32 = nullptr /* required when m.qs is set (Q4_K copy) */, const KrPfTiles* t = nullptr /* of the tile table; null: tiles of 64 */,
+                        KrPfhForm form = KR_PFH_AUTO);
+KrPfTiles kr_pfh_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows, int E, KrPfhForm form);      // of the tolerance GEMMs' tile table
 void kr_launch_pfh_w13_act(const KrMatDev& m, const uint16_t* a_h, const float* a_mul, const KrPfSort* sort, int topk, int gather_tokens, int max_tiles,
                            int single_expert_rows, float* gu, int rows, int act_mode, float swiglu_limit, float alpha, uint16_t* h_out, float* h_mul,
-                           hipStream_t st, int run = 1, const uint16_t* a_sum32 = nullptr, uint16_t* h_sums32 = nullptr, const KrPfTiles* t = nullptr);
-void kr_launch_pfh_gemm_multi(const KrMatDev* mats, float* const* outs, const int* out_lds, int n, const uint16_t* a_h, const float* a_mul, int M, hipStream_t st);
-// the LDS-ring form of the INT4 tolerance GEMM (kr_prefill_ring.hip) is on by default; 0 keeps the register-staged kernels (process-wide A/B and test hook)
-void kr_pfr_set_enabled(int on);
+                           hipStream_t st, int run = 1, const uint16_t* a_sum32 = nullptr, uint16_t* h_sums32 = nullptr, const KrPfTiles* t = nullptr, KrPfhForm form = KR_PFH_AUTO);
+void kr_launch_pfh_gemm_multi(const KrMatDev* mats, float* const* outs, const int* out_lds, int n, const uint16_t* a_h, const float* a_mul, int M, hipStream_t st,
+                              KrPfhForm form);

@@ -705,9 +705,9 @@ static void pfh_strip_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st) {
 // 500 218 / 210, 700 245 / 214; 64 of 2048 x 1408, top 6: 40 tokens 79 / 78, 80 78 / 76, 110 94 / 78; 128 of 4096 x 1536, top 8: 60 tokens 279 / 277, 100 281 / 279, 150 343 / 282.
 // The experts' own rows decide (see kr_pf_tiles), at up to 11 / 8 strips a tile of 64; tiles of 96 where few experts have fewer rows than that.  Under 512 rows in all the tiles, which
 // are taken there only where a handful of experts has them, are kr_pfh_gemm_kernel's of 128 columns, twice as many (48 tokens on 28 experts 49.7 us, 57.8 with half as many; 160 tokens on 38 72 and 69).
-KrPfTiles kr_pfh_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows, int E) {
+KrPfTiles kr_pfh_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows, int E, KrPfhForm form) {
     const int K = 128 * (m0.ng > m1.ng ? m0.ng : m1.ng);
-    const bool int4 = m0.bits == 4 && m1.bits == 4 && !m0.qs && !m1.qs, wave = int4 && rows >= 512 && kr_pfr_default();
+    const bool int4 = m0.bits == 4 && m1.bits == 4 && !m0.qs && !m1.qs, wave = int4 && rows >= 512 && form == KR_PFH_AUTO;
     const bool strips = int4 && m0.N % 16 == 0 && m1.N % 16 == 0 && rows <= (E > 256 ? 9L : 7L) * E && pfh_strip_lds(K) <= 160 * 1024;
     KrPfTiles t = kr_pf_cut(wave && rows > (E > 256 ? 14L : 10L) * E ? KR_PFW_ROWS : PFH_BM, strips ? PFH_ST_ROWS : 0, 11, tokens, rows, E);
     t.wave = wave;
@@ -771,8 +771,10 @@ void kr_launch_pfh_act(const float* gu, int rows, int n, int gu_ld, int act_mode
     else hipLaunchKernelGGL(kr_pfh_act_kernel<KR_ACT_SILU_MUL>, dim3(rows), dim3(256), 0, st, gu, n, gu_ld, swiglu_limit, alpha, out, mul);
 }
 void kr_launch_pfh_gemm(const KrMatDev& m, const uint16_t* a_h, const float* a_mul, const KrPfSort* sort, int topk, int gather_tokens, int max_tiles,
-                        int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows, int out_bf16, int run, const uint16_t* a_sum32, const KrPfTiles* t) {
+                        int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows, int out_bf16, int run, const uint16_t* a_sum32, const KrPfTiles* t,
+                        KrPfhForm form) {
     KrPfGemmHArgs a{};
+    a.form = form;
     a.m = m; a.a = a_h; a.a_mul = a_mul; a.a_sum = a_sum32; a.topk = topk; a.gather_tokens = gather_tokens; a.scatter_rows = scatter_rows; a.out_bf16 = out_bf16;
     if (sort) { a.row_pair = sort->row_pair; a.tile_expert = sort->tile_expert; a.tile_row0 = sort->tile_row0; a.tile_rows = sort->tile_rows; a.n_tiles = sort->n_tiles; }
     a.out = out; a.out_ld = out_ld; a.single_expert = single_expert_rows > 0; a.total_rows = single_expert_rows;
@@ -792,17 +794,18 @@ void kr_launch_pfh_gemm(const KrMatDev& m, const uint16_t* a_h, const float* a_m
 // only makes the f16 form.  Otherwise: the GEMM, then the activation pass over gate | up rows.  Same arithmetic either way.
 void kr_launch_pfh_w13_act(const KrMatDev& m, const uint16_t* a_h, const float* a_mul, const KrPfSort* sort, int topk, int gather_tokens, int max_tiles,
                            int single_expert_rows, float* gu, int rows, int act_mode, float swiglu_limit, float alpha, uint16_t* h_out, float* h_mul,
-                           hipStream_t st, int run, const uint16_t* a_sum32, uint16_t* h_sums32, const KrPfTiles* t) {
+                           hipStream_t st, int run, const uint16_t* a_sum32, uint16_t* h_sums32, const KrPfTiles* t, KrPfhForm form) {
     const int I = m.N / 2;
     const int mt = single_expert_rows > 0 ? (single_expert_rows + PFH_BM - 1) / PFH_BM : max_tiles;
     const bool wave = t && t->wave;
     const bool fuse = !(t && t->strip > 0) && m.bits == 4 && I % 128 == 0 && I <= 2048 && (wave || (long)mt * (m.N / 128) >= 2048);
     if (!fuse) {
-        kr_launch_pfh_gemm(m, a_h, a_mul, sort, topk, gather_tokens, max_tiles, single_expert_rows, gu, 2 * I, st, 0, 0, run, a_sum32, t);
+        kr_launch_pfh_gemm(m, a_h, a_mul, sort, topk, gather_tokens, max_tiles, single_expert_rows, gu, 2 * I, st, 0, 0, run, a_sum32, t, form);
         kr_launch_pfh_act(gu, rows, I, 2 * I, act_mode, swiglu_limit, alpha, h_out, h_mul, st, h_sums32);
         return;
     }
     KrPfGemmHArgs a{};
+    a.form = form;
     a.m = m; a.a = a_h; a.a_mul = a_mul; a.a_sum = a_sum32; a.topk = topk; a.gather_tokens = gather_tokens;
     if (sort) { a.row_pair = sort->row_pair; a.tile_expert = sort->tile_expert; a.tile_row0 = sort->tile_row0; a.tile_rows = sort->tile_rows; a.n_tiles = sort->n_tiles; }
     a.out = gu; a.out_ld = I; a.single_expert = single_expert_rows > 0; a.total_rows = single_expert_rows;
@@ -814,8 +817,10 @@ void kr_launch_pfh_w13_act(const KrMatDev& m, const uint16_t* a_h, const float* 
     if (rows > 0) { if (cpl == 1) KR_ROWW(1); else if (cpl == 2) KR_ROWW(2); else KR_ROWW(4); }
 #undef KR_ROWW
 }
-void kr_launch_pfh_gemm_multi(const KrMatDev* mats, float* const* outs, const int* out_lds, int n, const uint16_t* a_h, const float* a_mul, int M, hipStream_t st) {
+void kr_launch_pfh_gemm_multi(const KrMatDev* mats, float* const* outs, const int* out_lds, int n, const uint16_t* a_h, const float* a_mul, int M, hipStream_t st,
+                              KrPfhForm form) {
     KrPfGemmHArgs a{};
+    a.form = form;
     a.m = mats[0]; a.out = outs[0]; a.out_ld = out_lds[0]; a.a = a_h; a.a_mul = a_mul; a.topk = 1; a.single_expert = 1; a.total_rows = M; a.n_extra = n - 1; a.run = 1;
     for (int i = 1; i < n; i++) { a.mx[i - 1] = mats[i]; a.outx[i - 1] = outs[i]; a.out_ldx[i - 1] = out_lds[i]; }
     pfh_dispatch(a, (M + PFH_BM - 1) / PFH_BM, st);

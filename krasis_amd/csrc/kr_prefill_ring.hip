@@ -32,7 +32,6 @@
 // of kr_launch_pf_sort; B ring of 2 stages = 128 KiB, A ring of 3) and 128 x 256 for the dense projections (B ring of 2 = 64 KiB, A ring of 4).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-#include <atomic>
 #include <cstdlib>
 #include <type_traits>
 
@@ -419,18 +418,12 @@ static int pfr_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st) {
     return 0;
 }
 
-// 0 = launched.  mt64 = row tiles of 64 rows (the experts' tile table); dense problems carry their row count in a.total_rows.  kr_pfr_set_enabled(0) keeps the
-// register-staged kernel (process-wide A/B and test hook: kr_moe_set_gemm_mode(e, 3), kr_decode_set_option(s, "gemm_ring", 0)); the caller falls back to it for
-// every shape this form does not take.
-// 0 off, 1 = the measured policy (today: never -- on one MI355X the ring form ties the register-staged kernel on dense problems, 780 - 810 TFLOP/s, and is 4 - 12 % behind it
-// on the experts: both are bound by the 7.8 vector instructions per MFMA of the INT4 -> f16 conversion, profiles/r06_gemm_ring_experiments.txt), 2 = every shape the kernel takes
-static std::atomic<int> g_pfr_on{1};
-void kr_pfr_set_enabled(int on) { g_pfr_on.store(on < 0 ? 0 : (on > 2 ? 2 : on)); }
-bool kr_pfr_default() { return g_pfr_on.load(std::memory_order_relaxed) == 1; }
+// 0 = launched.  mt64 = row tiles of 64 rows (the experts' tile table); dense problems carry their row count in a.total_rows.  Only where it is asked for (KR_PFH_RING: kr_moe_set_gemm_mode(e, 5),
+// kr_decode_set_option(s, "gemm_ring", 2)): on one MI355X the ring form ties the register-staged kernel on dense problems, 780 - 810 TFLOP/s, and is 4 - 12 % behind it on the experts (both are bound by
+// the 7.8 vector instructions per MFMA of the INT4 -> f16 conversion, profiles/r06_gemm_ring_experiments.txt), and kr_prefill_w.hip is ahead of both.  The caller falls back for every shape this form does not take.
 int kr_pfr_try_launch(const KrPfGemmHArgs& a, int mt64, hipStream_t st) {
-    const int on = g_pfr_on.load(std::memory_order_relaxed);
     const long min_wg = 1;
-    if (on != 2 || a.m.bits != 4 || a.m.qs) return 1;
+    if (a.form != KR_PFH_RING || a.m.bits != 4 || a.m.qs) return 1;
     if (a.m.ng < 2) return 1;
     for (int i = 0; i < a.n_extra; i++) if (a.mx[i].bits != 4 || a.mx[i].qs || a.mx[i].ng != a.m.ng) return 1;
     if (a.single_expert) {

@@ -293,7 +293,7 @@ static int pfw_columns(const KrPfGemmHArgs& a) {
 // dense problems: where the tiles come near one a compute unit; below that kr_pfh_gemm_kernel's of 64 x 128 spread wider (us, there / here: 2752 x 2048 x 4096, 232 tiles 75 / 63, 400 x 12352 x 2048, 245
 // tiles 40 / 35, but 2048 x 2048 x 4096, 176 tiles 51 / 60 and 4096 x 1024 x 2048, 172 tiles 29 / 34)
 bool kr_pfw_dense(const KrPfGemmHArgs& a) {
-    if (!a.single_expert || a.m.bits != 4 || a.m.qs || !kr_pfr_default()) return false;
+    if (!a.single_expert || a.m.bits != 4 || a.m.qs || a.form != KR_PFH_AUTO) return false;
     for (int i = 0; i < a.n_extra; i++) if (a.mx[i].bits != 4 || a.mx[i].qs || a.mx[i].ng != a.m.ng) return false;
     return (long)((a.total_rows + BM - 1) / BM) * pfw_columns(a) >= 220;
 }

@@ -1,8 +1,8 @@
 """The LDS-ring form of the tolerance GEMM (krasis_amd/csrc/kr_prefill_ring.hip: operands by LDS-DMA into rings, 8-wave workgroups, one barrier per 64-k
 unit) against the register-staged kernel it replaces for big INT4 problems (kr_prefill_h.hip).  Both feed v_mfma_f32_32x32x16_f16 the same fragments in
 the same order per accumulator, so the check is BIT IDENTITY of the f32 / f16 outputs, not a tolerance; the tolerance of either form against the exact
-(oracle-identical) kernel is stated in tests/test_gemm_fast_gpu.py, whose QCN-shaped cases run the ring kernel by default.
-kr_moe_set_gemm_mode: 1 = default (ring for problems that fill the chip), 3 = register-staged kernels only, 5 = ring for every shape it takes."""
+(oracle-identical) kernel is stated in tests/test_gemm_fast_gpu.py.  kr_moe_set_gemm_mode: 1 = default (kr_prefill_w.hip for INT4 problems that fill the chip, never the
+rings), 3 = register-staged kernels only, 5 = ring for every shape it takes."""
 import numpy as np
 import pytest
 
@@ -22,7 +22,7 @@ def _prefill_mode(eng, torch, x, ids, w, mode, routed_only=False):
     check(eng._lib.kr_moe_set_gemm_mode(eng._h, mode))
     check(eng._lib.kr_moe_prefill(eng._h, 0, xt.data_ptr(), it.data_ptr(), wt.data_ptr(), out.data_ptr(), M, ids.shape[1], _lib.KR_OUT_F32, int(routed_only), 1))
     torch.cuda.synchronize()
-    check(eng._lib.kr_moe_set_gemm_mode(eng._h, 1)); check(eng._lib.kr_moe_set_gemm_mode(eng._h, 0))      # ring back to its default, exact mode
+    check(eng._lib.kr_moe_set_gemm_mode(eng._h, 0))
     return out.cpu().numpy()
 
 
@@ -50,6 +50,34 @@ def test_ring_gemm_bit_identical_to_register_staged(H, I, E, k, M, n_shared):
     r_staged = _prefill_mode(eng, torch, x[:70], ids[:70], w[:70], 3, routed_only=True)
     r_ring = _prefill_mode(eng, torch, x[:70], ids[:70], w[:70], 5, routed_only=True)
     assert np.array_equal(r_staged.view(np.uint32), r_ring.view(np.uint32))
+
+
+def test_the_form_is_the_engines_own():
+    """an engine's mode and a store's option choose the kernels of their own calls only: the tiles that a pass was cut into (of 96 rows, or of 64) tell which"""
+    import ctypes as C
+    from krasis_amd import CpuDecodeStore
+    from krasis_amd._lib import check
+    E, M, k = 4, 600, 2                                              # 300 rows an expert: 4 tiles of 96, 5 of 64
+    a, _, _, rng, torch = _setup(256, 256, E, k, 0, 1.0)
+    b = _setup(256, 256, E, k, 0, 1.0)[0]
+    x = rand_bf16(rng, (M, 256)); w = rng.random((M, k)).astype(F)
+    ids = np.stack([np.arange(M) % E, (np.arange(M) + 1) % E], 1).astype(np.int32)
+
+    def tiles(eng, mode):
+        _prefill_mode(eng, torch, x, ids, w, mode)
+        t, s = C.c_int(), C.c_int()
+        check(eng._lib.kr_moe_prefill_tiles(eng._h, C.byref(t), C.byref(s)))
+        return t.value
+    assert tiles(b, 1) == 4 * E
+    for mode in (3, 5):
+        assert tiles(a, mode) == 5 * E                               # leaves engine a in mode 0
+        check(a._lib.kr_moe_set_gemm_mode(a._h, mode))
+        assert tiles(b, 1) == 4 * E
+        assert tiles(a, 1) == 4 * E
+    st = CpuDecodeStore(128, True, True); st.set_moe_store(a)
+    for value in (0, 2):
+        st.set_option("gemm_ring", value)
+        assert tiles(a, 1) == 4 * E and tiles(b, 1) == 4 * E
 
 
 def test_ring_gemm_repeatable():
@@ -81,7 +109,6 @@ def test_ring_gemm_prompt_pass_bit_identical(kinds):
         lg = np.empty(d["V"], F)
         st.prefill(toks, 0, lg.ctypes.data)
         res.append(lg.copy())
-        st.set_option("gemm_ring", 1)
     assert np.isfinite(res[1]).all()
     assert np.array_equal(res[0].view(np.uint32), res[1].view(np.uint32)), float(np.abs(res[0] - res[1]).max())
 

@@ -5,6 +5,8 @@
 #define KR_TIMING 1
 #include "../../krasis_amd/csrc/kr_prefill_h.hip"
 #include "../../krasis_amd/csrc/kr_prefill_ring.hip"
+#include "../../krasis_amd/csrc/kr_prefill_w.hip"
+#include "../../krasis_amd/csrc/kr_prefill.hip"
 #include "mx_gemm_experiment.hip"
 #include <cstdio>
 #include <cstdlib>
@@ -31,7 +33,6 @@ int main(int argc, char** argv) {
     hipEvent_t e0, e1; CK(hipEventCreate(&e0)); CK(hipEventCreate(&e1));
     kr_launch_pfx_wimage(m, 1, img, ib, st); CK(hipStreamSynchronize(st)); CK(hipGetLastError());
     const double flop = 2.0 * M * (double)K * N;
-    kr_pfr_set_enabled(0);
     for (int form = 0; form < 2; form++)
         for (int rep = 0; rep < 4; rep++) {
             float ms_rows, ms;
@@ -39,7 +40,7 @@ int main(int argc, char** argv) {
             if (form == 0) kr_launch_pfh_rows_f32(x, M, K, K, ah, mulh, st); else if (kr_launch_pfx_rows_f32(x, M, K, K, amx, mulx, st)) { printf("rows: shape not covered\n"); return 1; }
             CK(hipEventRecord(e1, st)); CK(hipStreamSynchronize(st)); CK(hipGetLastError()); CK(hipEventElapsedTime(&ms_rows, e0, e1));
             CK(hipEventRecord(e0, st));
-            if (form == 0) kr_launch_pfh_gemm(m, ah, mulh, nullptr, 1, 0, 0, M, out0, N, st);
+            if (form == 0) kr_launch_pfh_gemm(m, ah, mulh, nullptr, 1, 0, 0, M, out0, N, st, 0, 0, 1, nullptr, nullptr, KR_PFH_STAGED);
             else if (kr_launch_pfx_gemm(m, img, ib, amx, mulx, nullptr, 1, 0, 0, M, out1, N, st)) { printf("gemm: shape not covered\n"); return 1; }
             CK(hipEventRecord(e1, st)); CK(hipStreamSynchronize(st)); CK(hipGetLastError()); CK(hipEventElapsedTime(&ms, e0, e1));
             printf("%s rep %d: rows %.1f us, GEMM %.1f us = %.0f TFLOP/s\n", form ? "MX " : "f16", rep, ms_rows * 1e3, ms * 1e3, flop / (ms * 1e-3) / 1e12);

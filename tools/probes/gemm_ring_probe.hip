@@ -5,6 +5,8 @@
 #define KR_TIMING 1
 #include "../../krasis_amd/csrc/kr_prefill_h.hip"
 #include "../../krasis_amd/csrc/kr_prefill_ring.hip"
+#include "../../krasis_amd/csrc/kr_prefill_w.hip"
+#include "../../krasis_amd/csrc/kr_prefill.hip"
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -35,8 +37,7 @@ int main(int argc, char** argv) {
             std::fill(ha.begin(), ha.end(), 0); for (int r = 0; r < M; r++) ha[(size_t)r * K + p] = 0x3C00;
             CK(hipMemcpy(a, ha.data(), ha.size() * 2, hipMemcpyHostToDevice));
             for (int form = 0; form < 2; form++) {
-                kr_pfr_set_enabled(form ? 2 : 0);
-                kr_launch_pfh_gemm(m, a, mul, nullptr, 1, 0, 0, M, out0, N, st); CK(hipStreamSynchronize(st));
+                kr_launch_pfh_gemm(m, a, mul, nullptr, 1, 0, 0, M, out0, N, st, 0, 0, 1, nullptr, nullptr, form ? KR_PFH_RING : KR_PFH_STAGED); CK(hipStreamSynchronize(st));
                 CK(hipMemcpy((form ? R : S)[p].data(), out0 + (size_t)5 * N, N * 4, hipMemcpyDeviceToHost));      // row 5
             }
         }
@@ -50,12 +51,11 @@ int main(int argc, char** argv) {
         return 0;
     }
     for (int form = 0; form < 2; form++) {
-        kr_pfr_set_enabled(form ? 2 : 0);
         float* out = form ? out1 : out0;
         CK(hipMemset(out, 0xFF, (size_t)M * N * 4));
         for (int rep = 0; rep < 4; rep++) {
             CK(hipEventRecord(e0, st));
-            kr_launch_pfh_gemm(m, a, mul, nullptr, 1, 0, 0, M, out, N, st);
+            kr_launch_pfh_gemm(m, a, mul, nullptr, 1, 0, 0, M, out, N, st, 0, 0, 1, nullptr, nullptr, form ? KR_PFH_RING : KR_PFH_STAGED);
             CK(hipEventRecord(e1, st)); CK(hipStreamSynchronize(st)); CK(hipGetLastError());
             float ms; CK(hipEventElapsedTime(&ms, e0, e1));
             printf("%s rep %d: %.1f us, %.0f TFLOP/s\n", form ? "ring  " : "staged", rep, ms * 1e3, flop / (ms * 1e-3) / 1e12);

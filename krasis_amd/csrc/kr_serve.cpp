@@ -957,8 +957,8 @@ int kr_serve_rows_alloc(kr_serve* s, size_t bytes, void** rows_out) {
     *rows_out = nullptr;
     KR_HIP(hipSetDevice(s->device));
     void *p = nullptr, *d = nullptr;
-    KR_HIP(hipHostMalloc(&p, bytes, hipHostMallocMapped | hipHostMallocCoherent));
-    if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess) { (void)hipHostFree(p); return kr_fail(KR_ERR_HIP, "no device address of %zu pinned bytes", bytes); }
+    if (hipHostMalloc(&p, bytes, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) { (void)hipGetLastError(); return kr_fail(KR_ERR_HIP, "no %zu bytes of pinned memory", bytes); }      // not the next step's error
+    if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess) { (void)hipGetLastError(); (void)hipHostFree(p); return kr_fail(KR_ERR_HIP, "no device address of %zu pinned bytes", bytes); }
     try {
         std::lock_guard<std::mutex> g(rows_mu);
         rows_blocks[(char*)p] = {bytes, s->device, (char*)d};

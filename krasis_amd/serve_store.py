@@ -123,7 +123,8 @@ class _Slab:
     """Pinned memory of the library, given back with its last reference."""
     def __init__(self, lib, handle, nbytes: int):
         self._lib, self.ptr = lib, C.c_void_p()
-        check_serve(lib.kr_serve_rows_alloc(handle, nbytes, C.byref(self.ptr)))
+        if lib.kr_serve_rows_alloc(handle, nbytes, C.byref(self.ptr)):
+            raise MemoryError(f"{nbytes} bytes of pinned memory")
 
     def __del__(self):
         if getattr(self, "ptr", None) and not sys.is_finalizing():
@@ -142,12 +143,13 @@ class _Lease:
 
 class _RowPool:
     """Arrays for logits in memory that the device stores to itself: the copy out of the store's own results was 50 us for twelve rows of 32768, and fresh pages for it a fault each.
-    Blocks are powers of two; MOST bytes per store at a time, then None (the caller takes ordinary memory and the copy).  Blocks change hands by deque operations alone, so arrays may
+    Blocks are powers of two; MOST bytes per store at a time, or what the system pins, then None (the caller takes ordinary memory and the copy).  Blocks change hands by deque operations alone, so arrays may
     be dropped on any thread; a slab lives as long as the pool or one of its arrays."""
     MOST, LEAST, LARGEST = 128 << 20, 64 << 10, 32 << 20
+    RETRY = 16                                      # arrays that take the copy before refused memory is asked for again
 
     def __init__(self, lib):
-        self._lib, self._free, self._bytes = lib, {}, 0
+        self._lib, self._free, self._bytes, self._wait = lib, {}, 0, 0
 
     def take(self, handle, rows: int, cols: int) -> Optional[np.ndarray]:
         size = self.LEAST
@@ -162,7 +164,14 @@ class _RowPool:
             nbytes = max(size, min(16 * size, self.LARGEST))
             if self._bytes + nbytes > self.MOST:
                 return None
-            slab, at = _Slab(self._lib, handle, nbytes), 0
+            if self._wait > 0:
+                self._wait -= 1
+                return None
+            try:
+                slab, at = _Slab(self._lib, handle, nbytes), 0
+            except MemoryError:
+                self._wait = self.RETRY
+                return None
             self._bytes += nbytes
             free.extend((slab, o) for o in range(size, nbytes, size))
         block = (C.c_float * (rows * cols)).from_address(slab.ptr.value + at)

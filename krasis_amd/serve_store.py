@@ -122,7 +122,7 @@ class LayerSpec:
 class _Slab:
     """Pinned memory of the library, given back with its last reference."""
     def __init__(self, lib, handle, nbytes: int):
-        self._lib, self.ptr = lib, C.c_void_p()
+        self._lib, self.ptr, self.nbytes = lib, C.c_void_p(), nbytes
         if lib.kr_serve_rows_alloc(handle, nbytes, C.byref(self.ptr)):
             raise MemoryError(f"{nbytes} bytes of pinned memory")
 
@@ -149,7 +149,8 @@ class _RowPool:
     RETRY = 16                                      # arrays that take the copy before refused memory is asked for again
 
     def __init__(self, lib):
-        self._lib, self._free, self._bytes, self._wait = lib, {}, 0, 0
+        self._lib, self._free, self._bytes = lib, {}, 0
+        self._wait, self._full = 0, {}              # arrays until refused memory is asked for again; until the pool makes room for a size of block
 
     def take(self, handle, rows: int, cols: int) -> Optional[np.ndarray]:
         size = self.LEAST
@@ -161,22 +162,53 @@ class _RowPool:
         try:
             slab, at = free.popleft()
         except IndexError:
-            nbytes = max(size, min(16 * size, self.LARGEST))
-            if self._bytes + nbytes > self.MOST:
+            slab, at = self._grow(handle, size), 0
+            if slab is None:
                 return None
-            if self._wait > 0:
-                self._wait -= 1
-                return None
-            try:
-                slab, at = _Slab(self._lib, handle, nbytes), 0
-            except MemoryError:
-                self._wait = self.RETRY
-                return None
-            self._bytes += nbytes
-            free.extend((slab, o) for o in range(size, nbytes, size))
+            free.extend((slab, o) for o in range(size, slab.nbytes, size))
         block = (C.c_float * (rows * cols)).from_address(slab.ptr.value + at)
         block.lease = _Lease(free, slab, at)
         return np.frombuffer(block, np.float32).reshape(rows, cols)
+
+    def _grow(self, handle, size: int) -> Optional[_Slab]:
+        if self._wait > 0:
+            self._wait -= 1
+            return None
+        nbytes = max(size, min(16 * size, self.LARGEST))
+        if self._bytes + nbytes > self.MOST:
+            # Full.  Slabs of other sizes that nobody holds a block of make room, but not at once: where batches of many sizes come in turn, a slab given back and another one pinned
+            # cost more than the copies of sixteen steps.
+            left = self._full.get(size, self.RETRY)
+            if left > 0:
+                self._full[size] = left - 1
+                return None
+            self._full.pop(size)
+            self._drop_idle(self._bytes + nbytes - self.MOST)
+            if self._bytes + nbytes > self.MOST:
+                return None
+        try:
+            slab = _Slab(self._lib, handle, nbytes)
+        except MemoryError:
+            self._wait = self.RETRY
+            return None
+        self._bytes += nbytes
+        return slab
+
+    def _drop_idle(self, wanted: int) -> None:
+        """gives back slabs that are whole among the free blocks, until `wanted` bytes are"""
+        for size, free in self._free.items():
+            if wanted <= 0:
+                return
+            blocks = {}
+            while free:                             # (blocks that come back meanwhile stay)
+                slab, at = free.popleft()
+                blocks.setdefault(slab, []).append(at)
+            for slab, ats in blocks.items():
+                if wanted > 0 and len(ats) * size == slab.nbytes:
+                    wanted -= slab.nbytes
+                    self._bytes -= slab.nbytes      # its last reference goes with `blocks`
+                else:
+                    free.extend((slab, at) for at in ats)
 
 
 class ServeStore:

@@ -42,3 +42,30 @@ def test_refused_memory_means_the_copy():
     lib.refuse = False
     got = [pool.take(None, 1, 20000) for _ in range(pool.RETRY + 1)]
     assert got[-1] is not None and got[-1].shape == (1, 20000)
+
+
+def test_growing_batches_are_not_shut_out():
+    """one row of 151936 logits to sixteen, every size for a while: blocks of sizes that are no longer used make room"""
+    lib = Lib(); pool = S._RowPool(lib); V = 151936
+    for rows in (1, 2, 5, 13, 16, 27, 1):
+        for _ in range(pool.RETRY + 2):
+            last = pool.take(None, rows, V)
+            if last is not None:
+                last[0, 0] = last[-1, -1] = rows
+        assert last is not None and last.shape == (rows, V), rows
+        assert pool._bytes == lib.pinned() <= pool.MOST
+
+
+def test_room_is_not_made_of_what_is_held_and_not_at_every_step():
+    lib = Lib(); pool = S._RowPool(lib); V = 151936
+    held = [pool.take(None, 5, V) for _ in range(32)]            # 32 blocks of 4 MB
+    for i, h in enumerate(held):
+        h[:] = i
+    asked = lib.asked
+    assert all(pool.take(None, 13, V) is None for _ in range(3 * pool.RETRY)) and lib.asked == asked
+    assert all((h == i).all() for i, h in enumerate(held))
+    held = held[:1]                                              # the first slab keeps one block
+    for _ in range(2 * pool.RETRY + 2):                          # sizes in turn
+        a, b = pool.take(None, 13, V), pool.take(None, 5, V)
+    assert a is not None and b is not None and lib.asked - asked <= 4
+    assert (held[0] == 0).all()

@@ -126,8 +126,8 @@ class _Slab:
         if lib.kr_serve_rows_alloc(handle, nbytes, C.byref(self.ptr)):
             raise MemoryError(f"{nbytes} bytes of pinned memory")
 
-    def __del__(self):
-        if getattr(self, "ptr", None) and not sys.is_finalizing():
+    def __del__(self, ending=sys.is_finalizing):    # (an argument: a module's names may be gone when the interpreter ends)
+        if getattr(self, "ptr", None) and not ending():
             self._lib.kr_serve_rows_free(self.ptr)
 
 

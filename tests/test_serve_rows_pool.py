@@ -1,5 +1,7 @@
 """The pool of memory that a step's logits stand on (krasis_amd.serve_store._RowPool), on the CPU: a stand-in for the library hands out ordinary pages."""
 import mmap
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -69,3 +71,13 @@ def test_room_is_not_made_of_what_is_held_and_not_at_every_step():
         a, b = pool.take(None, 13, V), pool.take(None, 5, V)
     assert a is not None and b is not None and lib.asked - asked <= 4
     assert (held[0] == 0).all()
+
+
+def test_the_interpreter_ends_quietly():
+    """a store, its pool and arrays that nobody closed: nothing is said at the end, and nothing is called into a library that may be down"""
+    code = ("import sys; sys.path.insert(0, '.')\n"
+            "from tests.test_serve_rows_pool import Lib, S\n"
+            "lib = Lib(); pool = S._RowPool(lib); keep = pool.take(None, 3, 20000)\n"
+            "sys.modules['anchor'] = S; S.anchor = (pool, keep)\n")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stderr == "", r.stderr

@@ -5,7 +5,11 @@ Slots and pages are managed by the library (`admit` / `release`); nothing here c
 from __future__ import annotations
 
 import ctypes as C
+import mmap
+import os
 import sys
+import threading
+import weakref
 from collections import deque
 from dataclasses import dataclass, fields
 from typing import List, Optional, Sequence, Tuple
@@ -121,10 +125,14 @@ class LayerSpec:
 
 class _Slab:
     """Pinned memory of the library, given back with its last reference."""
+    every = weakref.WeakSet()
+
     def __init__(self, lib, handle, nbytes: int):
         self._lib, self.ptr, self.nbytes = lib, C.c_void_p(), nbytes
+        self.held = {}                              # offset -> bytes of the blocks under arrays
         if lib.kr_serve_rows_alloc(handle, nbytes, C.byref(self.ptr)):
             raise MemoryError(f"{nbytes} bytes of pinned memory")
+        _Slab.every.add(self)
 
     def __del__(self, ending=sys.is_finalizing):    # (an argument: a module's names may be gone when the interpreter ends)
         if getattr(self, "ptr", None) and not ending():
@@ -137,8 +145,37 @@ class _Lease:
         self.free, self.slab, self.at = free, slab, at
 
     def __del__(self):
+        self.slab.held.pop(self.at, None)
         if self.slab.ptr:
             self.free.append((self.slab, self.at))
+
+
+# Pinned memory of a device is not handed on to a forked child (its pages are not even mapped there), and the arrays that stand on it are anyone's: what they hold at the fork is put under them
+# again in the child, as ordinary memory.  The child gives nothing back and takes no blocks: the device is its parent's.
+_at_fork = threading.local()
+_map = C.CDLL(None).mmap
+_map.restype, _map.argtypes = C.c_void_p, [C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_int, C.c_long]
+_MAP_FIXED = 0x10
+
+
+def _before_fork() -> None:
+    _at_fork.held = [(slab.ptr.value + at, C.string_at(slab.ptr.value + at, n)) for slab in list(_Slab.every) if slab.ptr for at, n in slab.held.copy().items()]
+
+
+def _after_fork_in_parent() -> None:
+    _at_fork.held = None
+
+
+def _after_fork_in_child() -> None:
+    for at, data in _at_fork.held:
+        if _map(at, len(data), mmap.PROT_READ | mmap.PROT_WRITE, mmap.MAP_PRIVATE | mmap.MAP_ANONYMOUS | _MAP_FIXED, -1, 0) == at:
+            C.memmove(at, data, len(data))
+    _at_fork.held = None
+    for slab in list(_Slab.every):
+        slab.ptr = C.c_void_p()
+
+
+os.register_at_fork(before=_before_fork, after_in_parent=_after_fork_in_parent, after_in_child=_after_fork_in_child)
 
 
 class _RowPool:
@@ -161,11 +198,14 @@ class _RowPool:
         free = self._free.setdefault(size, deque())
         try:
             slab, at = free.popleft()
+            while not slab.ptr:
+                slab, at = free.popleft()
         except IndexError:
             slab, at = self._grow(handle, size), 0
             if slab is None:
                 return None
             free.extend((slab, o) for o in range(size, slab.nbytes, size))
+        slab.held[at] = rows * cols * 4
         block = (C.c_float * (rows * cols)).from_address(slab.ptr.value + at)
         block.lease = _Lease(free, slab, at)
         return np.frombuffer(block, np.float32).reshape(rows, cols)
@@ -287,7 +327,9 @@ class ServeStore:
 
     # ---- the step
     def step(self, entries: Sequence[Tuple[int, Sequence[int]]], want_rows: Sequence[int], logits: bool = True) -> Tuple[Optional[np.ndarray], np.ndarray]:
-        """entries: (slot, tokens); want_rows: indices into the entries' tokens laid end to end.  Returns (logits [n_want, vocab] f32 or None, argmax [n_want])."""
+        """entries: (slot, tokens); want_rows: indices into the entries' tokens laid end to end.  Returns (logits [n_want, vocab] f32 or None, argmax [n_want]).
+        The logits are the caller's for as long as any reference or view of them is left, also past `close` and in a forked child.  They stand on memory that the device writes, which
+        the array does not own (`flags.owndata`): to resize them in place, or to free the store's memory while they are kept for long, take a copy."""
         slots = np.asarray([e[0] for e in entries], np.int32)
         counts = np.asarray([len(e[1]) for e in entries], np.int32)
         toks = np.ascontiguousarray(np.concatenate([np.asarray(e[1], np.int32).reshape(-1) for e in entries]) if entries else np.zeros(0, np.int32))

@@ -1,5 +1,7 @@
 """The pool of memory that a step's logits stand on (krasis_amd.serve_store._RowPool), on the CPU: a stand-in for the library hands out ordinary pages."""
+import gc
 import mmap
+import os
 import subprocess
 import sys
 
@@ -10,7 +12,7 @@ from krasis_amd import serve_store as S
 
 
 class Lib:
-    """kr_serve_rows_alloc / kr_serve_rows_free over anonymous pages; `refuse`: allocations fail"""
+    """kr_serve_rows_alloc / kr_serve_rows_free over anonymous pages that, as a device's, a forked child does not get; `refuse`: allocations fail"""
     def __init__(self):
         self.live, self.asked, self.refuse = {}, 0, False
 
@@ -19,6 +21,7 @@ class Lib:
         if self.refuse:
             return -3
         m = mmap.mmap(-1, nbytes)
+        m.madvise(mmap.MADV_DONTFORK)
         at = np.frombuffer(m, np.uint8).ctypes.data
         self.live[at] = m
         out._obj.value = at
@@ -81,3 +84,25 @@ def test_the_interpreter_ends_quietly():
             "sys.modules['anchor'] = S; S.anchor = (pool, keep)\n")
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stderr == "", r.stderr
+
+
+def test_arrays_live_on_in_a_forked_child():
+    lib = Lib(); pool = S._RowPool(lib)
+    a, b, gone = pool.take(None, 3, 20001), pool.take(None, 3, 20001), pool.take(None, 3, 20001)
+    a[:] = np.arange(a.size).reshape(a.shape); b[:] = -1
+    view = b[2, 5:]
+    del gone, b
+    want = a.copy()
+    pid = os.fork()
+    if pid == 0:
+        ok = np.array_equal(a, want) and bool((view == -1).all())
+        a[:] = 5; view[:] = 6                                    # the child's own from here on
+        del a, view; gc.collect()
+        os._exit(0 if ok and len(lib.live) == 1 and pool.take(None, 3, 20001) is not None else 1)      # (a stand-in's new slab; the parent's blocks are not the child's)
+    assert os.waitpid(pid, 0)[1] == 0
+    assert np.array_equal(a, want) and (view == -1).all()
+    del a, view; gc.collect()
+    assert pool._bytes == lib.pinned()
+    for _ in range(40):
+        assert pool.take(None, 3, 20001) is not None             # the parent's blocks still come round
+    assert pool._bytes == lib.pinned()

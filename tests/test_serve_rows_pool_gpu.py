@@ -2,6 +2,7 @@
 than the pool holds, rows past its largest block, memory of the caller's -- takes the copy."""
 import ctypes as C
 import gc
+import os
 import threading
 
 import numpy as np
@@ -102,6 +103,18 @@ def test_rows_of_the_c_interface():
         check_serve(lib.kr_serve_rows_free(p))
     with pytest.raises(ValueError):
         check_serve(lib.kr_serve_rows_alloc(st._h, 0, C.byref(p)))
+
+
+def test_a_forked_child_reads_the_arrays():
+    cfg = model(); W = O.random_weights(cfg, 11); toks = tokens(cfg, 28, 12)
+    eng = engine(cfg, W, "bfloat16", max_tokens=512)
+    held = run(eng, "a", toks)
+    want = [h.copy() for h in held]
+    pid = os.fork()
+    if pid == 0:                                         # nothing of the device in here
+        os._exit(0 if all(np.array_equal(h, w) for h, w in zip(held, want)) else 1)
+    assert os.waitpid(pid, 0)[1] == 0
+    assert all(np.array_equal(h, w) for h, w in zip(run(eng, "b", toks), want)) and all(np.array_equal(h, w) for h, w in zip(held, want))
 
 
 def test_two_stores_on_two_threads():

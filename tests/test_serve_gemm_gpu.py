@@ -61,9 +61,9 @@ def test_expert_products_sizes(n):
 @pytest.mark.parametrize("mlp,n", [
     (O.dense(481), 1501), (O.dense(1000), 1200), (O.dense(2884), 2305),                                     # behind the layer's other columns: 128-, 128- and 256-column tiles
     (O.moe(3, 3, 1, 1, 264, 1.5), 1700), (O.moe(8, 8, 1, 1, 260, 1.5, 520, 0.8), 2100)])                     # one matrix per expert, and both
-def test_activation_from_the_product(mlp, n):
+def test_activation_from_the_product(mlp, n, width=64):
     # factors that are no whole tiles, with and without whole 16-byte pieces; every expert is chosen, so that no close call hides an error
-    cfg = O.make_config(width=64, vocab=61, eps=1e-5, layers=[{"type": "attention", "mixer": O.attn(2, 1, 8, 8, 1, 0, scale=0.3), "mlp": mlp}])
+    cfg = O.make_config(width=width, vocab=61, eps=1e-5, layers=[{"type": "attention", "mixer": O.attn(2, 1, 8, 8, 1, 0, scale=0.3), "mlp": mlp}])
     W = O.random_weights(cfg, 15, router_gain=1.0); toks = tokens(cfg, n, 16)
     ref = O.forward(cfg, W, toks)[1][0]
     eng = engine(cfg, W, "bfloat16", max_tokens=4096)
@@ -73,6 +73,12 @@ def test_activation_from_the_product(mlp, n):
     # the input row, the two factors' sums and the activation: three independent roundings of 2^-9 each, which the products pass on at their own scale; a lost factor of
     # 260 would alter its rows by 1 / sqrt(260) = 6e-2
     assert np.sqrt((d ** 2).mean(-1)).max() / np.sqrt((ref ** 2).mean()) < 2e-2
+
+
+@pytest.mark.parametrize("width", [128, 192, 320])                                                             # two, three and five slots of k: the rings by parts behind the pairs
+@pytest.mark.parametrize("mlp,n", [(O.dense(1000), 1200), (O.dense(2884), 2305), (O.moe(3, 3, 1, 1, 264, 1.5), 1700)])
+def test_activation_from_the_product_of_several_slots(mlp, n, width):
+    test_activation_from_the_product(mlp, n, width)
 
 
 def _clamped_experts(ff, limit=1.5):

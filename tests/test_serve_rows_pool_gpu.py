@@ -121,13 +121,17 @@ def test_two_stores_on_two_threads():
     cfg = model(); W = O.random_weights(cfg, 9); toks = tokens(cfg, 28, 10)
     engs = [engine(cfg, W, "bfloat16", max_tokens=512) for _ in range(2)]
     ref = [a.copy() for a in run(engs[0], "r", toks)]
-    bad = []
+    bad, done = [], []
 
     def work(e):
-        for i in range(30):
-            if not all(np.array_equal(a, b) for a, b in zip(run(e, i, toks), ref)):
-                bad.append(i)
+        try:
+            for i in range(30):
+                if not all(np.array_equal(a, b) for a, b in zip(run(e, i, toks), ref)):
+                    bad.append(i)
+                done.append(e)
+        except BaseException as err:                     # an exception would end its thread alone
+            bad.append(err)
     ts = [threading.Thread(target=work, args=(e,)) for e in engs]
     for t in ts: t.start()
     for t in ts: t.join()
-    assert not bad
+    assert not bad and [sum(d is e for d in done) for e in engs] == [30, 30], bad

@@ -147,10 +147,13 @@ __global__ void __launch_bounds__(256) kr_pfm_gqa_pv_mfma_kernel(const KrPfmGqaA
     static_assert(VCH >= 1 && (PPT == 4 || PPT == 8), "stage shape");
     __shared__ __attribute__((aligned(16))) float Ps[32 * PLD];
     __shared__ __attribute__((aligned(16))) char Vs[PS * VROW];
-    const int group = a.nh / a.nkv, lg = __builtin_ctz(group), gm = group - 1, kvh = blockIdx.y, TT = 32 >> lg, kvs = a.nkv * HD;      // group: a power of two
-    // A tile's work grows with its position.  Workgroups go round the compute units, so the tiles of every other key head go backwards: a unit's second tile is short where its first is
-    // long (777 tokens, 16 / 2 heads of 256: 83 -> 66 us)
-    const int t0 = (int)(kvh & 1 ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * TT;
+    const int group = a.nh / a.nkv, lg = __builtin_ctz(group), gm = group - 1, TT = 32 >> lg, kvs = a.nkv * HD;      // group: a power of two
+    // A tile's work grows with its position, and up to three workgroups share a compute unit: those whose numbers are 256 apart.  So the tiles of all key heads are dealt by falling work, 256 at a
+    // time, every other time backwards: a unit's second tile is long where its first is short.  (us, tiles in the order of their numbers / dealt: 777 rows of 16 / 2 heads of 256 82 / 64, 32 / 8 of 128
+    // 52 / 41, 64 / 8 83 / 67, 32 / 32 of 64 42 / 35; 1024 rows of 32 / 8 90 / 55; the same up to 256 tiles.  The tiles of every other head backwards: 65, 43, 73, 45 and 92.)
+    const int id = blockIdx.y * gridDim.x + blockIdx.x, round = id & ~255, at = id - round, last = min(255, (int)(gridDim.x * gridDim.y) - 1 - round);
+    const int rank = round + (id & 256 ? at : last - at);
+    const int kvh = rank % a.nkv, t0 = ((int)gridDim.x - 1 - rank / a.nkv) * TT;
     const int tn = min(TT, C - t0), R = group * tn, p_max = a.pos0 + t0 + tn - 1;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r31 = lane & 31, kh = lane >> 5;
     xm_v16f acc[NB];

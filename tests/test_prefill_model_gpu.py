@@ -187,3 +187,18 @@ def test_norm_rows_with_and_without_the_chains_copy(H):
     d["reset"]()
     assert st.prefill(toks, 2, got.ctypes.data) == tok
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("nh,n_tok", [(64, 150), (64, 300), (32, 259)])      # one query head of each key head a row: a tile is one token (or two); 300, 600 and 260 tiles, dealt in two and three rounds, the last one short
+def test_exact_attention_tiles_of_several_rounds(nh, n_tok):
+    st, eng, orc, keep, d = build(seed=31, kv_max=330, hd=64, nh=nh, kinds=["gqa", "gqa"])
+    toks = [int(x) for x in np.random.default_rng(nh + n_tok).integers(0, d["V"], n_tok)]
+    ref = np.empty(d["V"], F); got = np.empty(d["V"], F)
+    for i, t in enumerate(toks):
+        st.decode_step(t, 9 + i, ref.ctypes.data)
+    tok = st.last_token(); kv = _snapshot(st, d)
+    d["reset"]()
+    assert st.prefill(toks, 9, got.ctypes.data) == tok
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+    for a, b in zip(_snapshot(st, d), kv):
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])

@@ -12,6 +12,7 @@
 #include "kr_pfh_dev.h"
 #include <hip/hip_fp16.h>
 #include <stdlib.h>
+#include <algorithm>
 
 __device__ __forceinline__ float kr_pfm_hsum8(float v) { v = v + __shfl_xor(v, 4); v = v + __shfl_xor(v, 1); v = v + __shfl_xor(v, 2); return v; }
 
@@ -913,7 +914,11 @@ __global__ void __launch_bounds__(256) kr_pfm_moe_epilogue_kernel(const float* _
 // ------------------------------------------------------------------------------------------
 void kr_launch_pfm_norm(const KrPfmNormArgs& a, int C, hipStream_t st) {
     const int row = (a.H + 7) / 4 * 4, ld = (a.H / 8 + 4) / 4 * 4 + 4;
-    const bool copy = (size_t)(row + 8 * ld) * 4 <= 64 * 1024 - 16;
+    // The copy doubles a workgroup's LDS: it is made where the rows take no more rounds of the chip for it, eight workgroups a compute unit being the most without it.  (us, without / with, in as many
+    // rounds: 1024 rows of 4096 16.0 / 13.7, 768 of 5120 16.7 / 14.1, 400 of 7168 17.4 / 13.8; in one more: 1536 of 4096 19.6 / 20.7, 900 of 5120 18.7 / 20.4, 640 of 7168 21.4 / 24.1, 4096 of 7168 113 / 127)
+    const size_t both = (size_t)(row + 8 * ld) * 4;
+    const int most = 256 * 8, with = 256 * std::min(8, (int)(160 * 1024 / (both + 16)));
+    const bool copy = both <= 64 * 1024 - 16 && (C + with - 1) / with == (C + most - 1) / most;
     hipLaunchKernelGGL(kr_pfm_norm_kernel, dim3(C), dim3(256), (size_t)(row + (copy ? 8 * ld : 0)) * 4, st, a, copy ? ld : 0);
 }
 void kr_launch_pfm_quant_f32(const float* x, int rows, int ld, int K, int8_t* xh, int8_t* xl, float* xs, hipStream_t st) {

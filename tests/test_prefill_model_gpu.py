@@ -202,3 +202,16 @@ def test_exact_attention_tiles_of_several_rounds(nh, n_tok):
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
     for a, b in zip(_snapshot(st, d), kv):
         assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
+def test_norm_rows_in_one_round_and_in_more():
+    # 1100 rows of 4096: a round more with the chains' copy, so without it; chunks of 500 with it
+    st, eng, orc, keep, d = build(seed=37, dims=(4096, 512, 8, 2, 128, 128), kinds=["la", "gqa"], kv_max=1120)
+    toks = [int(x) for x in np.random.default_rng(4).integers(0, d["V"], 1100)]
+    res = []
+    for chunk in (1100, 500):
+        d["reset"](); st.set_prefill_chunk(chunk)
+        lg = np.empty(d["V"], F)
+        tok = st.prefill(toks, 2, lg.ctypes.data)
+        res.append((tok, lg.view(np.uint32)))
+    assert res[0][0] == res[1][0] and np.array_equal(res[0][1], res[1][1])

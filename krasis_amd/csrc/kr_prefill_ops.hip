@@ -57,7 +57,7 @@ __device__ __forceinline__ void kr_pfm_quant_chunk(const float (&v)[8], int8_t* 
 // quantise bf16(hidden), decode.rs:3307-3309).
 __global__ void __launch_bounds__(256) kr_pfm_norm_kernel(const KrPfmNormArgs a, const int ld /* of the chains' copy; 0: too long a row for it */) {
     extern __shared__ __attribute__((aligned(16))) float r[];   // [H + 4], then [8][ld]: the same numbers as the eight chains of the sum of squares take them (16 bytes a read; one
-                                                                // number at a time: 777 rows of 2048 11.0 us against 8.6, a tolerance prompt of 8192 tokens 10.48 ms against 10.33)
+                                                                // number at a time: 777 rows of 2048 8.3 us against 7.2, a tolerance prompt of 8192 tokens 10.48 ms against 10.33)
     __shared__ uint32_t s_max;
     const int t = blockIdx.x, H = a.H, tid = threadIdx.x;
     float* rt = r + (H + 7) / 4 * 4;

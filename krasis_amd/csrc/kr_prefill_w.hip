@@ -1,7 +1,7 @@
 // kr_prefill_w.hip -- the tolerance GEMM of the prompt pass (KR_GEMM_FAST), INT4 weights, for problems that fill the chip: f16 rows x weights de-quantized in registers on
 // v_mfma_f32_32x32x16_f16, f32 accumulation over the whole k range.  Same products and the same order of sums per output as kr_pfh_gemm_kernel (kr_prefill_h.hip): the same bits.
 //
-// Bound: the matrix cores and, beside them, the vector port, which turns every weight into f16 once per tile: 24 instructions per 32 columns and 16 k, whatever the tile's rows.  So a
+// Bound: the matrix cores and, beside them, the vector port, which turns every weight into f16 once per tile: 12 instructions per 32 columns and 16 k, 24 for a wave's two column blocks, whatever the tile's rows.  So a
 // wave multiplies them by three row blocks (4 - 5 vector instructions per matrix instruction; two blocks: 7.8, with the rows' way through registers), and a tile takes the
 // 80 rows that an expert of 512 has of 4096 tokens as three blocks of 32 where two tiles of 64 were four blocks and formed the weights twice.
 // What travels, and how:
@@ -291,7 +291,8 @@ static int pfw_columns(const KrPfGemmHArgs& a) {
     return ncb;
 }
 // dense problems: where the tiles come near one a compute unit; below that kr_pfh_gemm_kernel's of 64 x 128 spread wider (us, there / here: 2752 x 2048 x 4096, 232 tiles 75 / 63, 400 x 12352 x 2048, 245
-// tiles 40 / 35, but 2048 x 2048 x 4096, 176 tiles 51 / 60 and 4096 x 1024 x 2048, 172 tiles 29 / 34)
+// tiles 40 / 35, but 2048 x 2048 x 4096, 176 tiles 51 / 60 and 4096 x 1024 x 2048, 172 tiles 29 / 34).  Those are launches alone.  Beside another chunk's launches the smaller problems are as well off here: whole
+// prompts of 700 - 8192 tokens, the line at 170 / at 220 / never: 700 2.19 / 2.20 / 2.24 ms, 2300 3.97 / 4.03, 4096 5.92 / 5.97 / 6.2, 7000 9.01 / 9.22, 8192 10.24 / 10.38 / 11.0; at 120 as at 170.
 bool kr_pfw_dense(const KrPfGemmHArgs& a) {
     if (!a.single_expert || a.m.bits != 4 || a.m.qs || a.form != KR_PFH_AUTO) return false;
     for (int i = 0; i < a.n_extra; i++) if (a.mx[i].bits != 4 || a.mx[i].qs || a.mx[i].ng != a.m.ng) return false;

@@ -2031,7 +2031,7 @@ __global__ void __launch_bounds__(256) sv_lin_cscan_kernel(const KrSvLin a) {
 // products are formed transposed: S^T[s][t] = K Q^T (queries of the wave's tokens stay in registers: lane (t = lane % 16, quarter = lane / 16) keeps
 // the quarter-th part of q_t), O^T[c][t] += V^T P^T with the weights where the first product left them; the state's share S_start^T q_t goes into the
 // same accumulators first.  DQ >= ceil(dim / 4), DB >= ceil(vdim / 16).
-// DIM > 0: that dim, vdim = 16 DB, key rows of whole 16-byte pieces; the queries in registers, so that four workgroups share a unit and not three.  A vector instruction between two f32 matrix instructions costs about 20 clocks (kr_serve_tile_f32.hip), and the
+// DIM > 0: that dim, vdim = 16 DB, key rows of whole 16-byte pieces (instances: 64 x 64, 64 x 128 and 128 x 128; other sizes, 128 x 64 among them, keep the guards); the queries in registers, so that four workgroups share a unit and not three.  A vector instruction between two f32 matrix instructions costs about 20 clocks (kr_serve_tile_f32.hip), and the
 // guards put one beside every product: here products come in runs of 16 on operands read before them, from addresses that stand still.  Same products, same order.
 // 3249 tokens of two requests, 16 heads of 128 x 128: 108 -> 55 us (three workgroups a unit 61; without the registers 91).
 template <bool ML, int DB, int DIM>

@@ -55,7 +55,7 @@ def test_ring_gemm_bit_identical_to_register_staged(H, I, E, k, M, n_shared):
 def test_the_form_is_the_engines_own():
     """an engine's mode and a store's option choose the kernels of their own calls only: the tiles that a pass was cut into (of 96 rows, or of 64) tell which"""
     import ctypes as C
-    from krasis_amd import CpuDecodeStore
+    from krasis_amd import CpuDecodeStore, _lib
     from krasis_amd._lib import check
     E, M, k = 4, 600, 2                                              # 300 rows an expert: 4 tiles of 96, 5 of 64
     a, _, _, rng, torch = _setup(256, 256, E, k, 0, 1.0)
@@ -63,21 +63,30 @@ def test_the_form_is_the_engines_own():
     x = rand_bf16(rng, (M, 256)); w = rng.random((M, k)).astype(F)
     ids = np.stack([np.arange(M) % E, (np.arange(M) + 1) % E], 1).astype(np.int32)
 
-    def tiles(eng, mode):
-        _prefill_mode(eng, torch, x, ids, w, mode)
+    xt = torch.from_numpy(x.view(np.int16)).cuda(); it = torch.from_numpy(ids).cuda(); wt = torch.from_numpy(w).cuda()
+    out = torch.empty((M, 256), dtype=torch.float32, device="cuda")
+
+    def mode(eng, m):
+        check(eng._lib.kr_moe_set_gemm_mode(eng._h, m))
+
+    def tiles(eng):                                                  # in the mode that the engine was given
+        check(eng._lib.kr_moe_prefill(eng._h, 0, xt.data_ptr(), it.data_ptr(), wt.data_ptr(), out.data_ptr(), M, k, _lib.KR_OUT_F32, 0, 1))
         t, s = C.c_int(), C.c_int()
         check(eng._lib.kr_moe_prefill_tiles(eng._h, C.byref(t), C.byref(s)))
         return t.value
-    assert tiles(b, 1) == 4 * E
-    for mode in (3, 5):
-        assert tiles(a, mode) == 5 * E                               # leaves engine a in mode 0
-        check(a._lib.kr_moe_set_gemm_mode(a._h, mode))
-        assert tiles(b, 1) == 4 * E
-        assert tiles(a, 1) == 4 * E
+    mode(b, 1)
+    assert tiles(b) == 4 * E
+    for m in (3, 5):
+        mode(a, m)
+        assert tiles(b) == 4 * E and tiles(a) == 5 * E
+        mode(a, 0)
+        assert tiles(b) == 4 * E
+        mode(a, 1)
+        assert tiles(a) == 4 * E
     st = CpuDecodeStore(128, True, True); st.set_moe_store(a)
     for value in (0, 2):
         st.set_option("gemm_ring", value)
-        assert tiles(a, 1) == 4 * E and tiles(b, 1) == 4 * E
+        assert tiles(a) == 4 * E and tiles(b) == 4 * E
 
 
 def test_ring_gemm_repeatable():

@@ -429,7 +429,7 @@ static bool pf_dense_wide(const KrPfGemmArgs& a) {
 }
 // A shared expert's products ride in the launches of the routed experts' where those take the wide kernel: each of its own launches ends in a round of workgroups that is seldom full
 // (3001 rows of 2 x 2816 x 2048 are 528 tiles, three rounds of 256 for the time of two).  (3001 rows, 64 INT8 experts of 2 x 1408 x 2048, top 6, two shared: us of the layer, apart / joined: 836 / 783;
-// 540 rows 291 / 246, 1500 546 / 479, 4096 1039 / 1032; INT4 279 / 241, 531 / 522, 1037 / 1033, 3001 842 / 801.)
+// 540 rows 291 / 246, 1500 546 / 479, 4096 1039 / 1032, 6000 1384 / 1361, 8192 1815 / 1818, 13653 2994 / 2992; INT4 279 / 241, 531 / 522, 1037 / 1033, 1440 / 1406, 1877 / 1879, 3127 / 3103, 3001 842 / 801.)
 bool kr_pf_joins(const KrPfTiles& t, const KrMatDev& experts, const KrMatDev& dense, int rows) {
     return t.rows == PFW_TM && dense.bits == experts.bits && pf_all_fma(dense) && (long)rows * dense.ng * 128 < 1L << 32;
 }

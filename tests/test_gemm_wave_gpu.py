@@ -35,6 +35,7 @@ def test_wave_gemm_bit_identical_to_register_staged(H, I, E, k, M, n_shared):
 @pytest.mark.parametrize("kinds,kw,n_tok", [
     (["la", "gqa"], dict(la_heads=(14, 28), la_dkdv=(128, 128), nh=8), 500),      # 10752 + 56 columns: six panels of eight column blocks, the sixth over the border; a second matrix that is no whole wave; 258 tiles, 6 row tiles of which the last has 20 rows
     (["la", "gqa"], dict(la_heads=(16, 32), la_dkdv=(128, 128), nh=8), 450),      # 12288 + 64
+    (["la", "gqa"], dict(la_heads=(9, 27), la_dkdv=(128, 128), nh=8), 600),        # 9216 + 54: rows of the second result that are no whole 16-byte pieces; 259 tiles, a last row tile of 24 rows
     (["gqa", "la"], dict(nh=32), 700),                                             # q with its gate, k and v: 8192 + 256 + 256 columns, two borders inside the fifth panel; 272 tiles, a last row tile of 28 rows
 ])
 def test_several_matrices_of_a_launch(kinds, kw, n_tok):

@@ -167,7 +167,7 @@ def _after_fork_in_parent() -> None:
 
 
 def _after_fork_in_child() -> None:
-    for at, data in _at_fork.held:
+    for at, data in getattr(_at_fork, "held", None) or ():
         if _map(at, len(data), mmap.PROT_READ | mmap.PROT_WRITE, mmap.MAP_PRIVATE | mmap.MAP_ANONYMOUS | _MAP_FIXED, -1, 0) == at:
             C.memmove(at, data, len(data))
     _at_fork.held = None

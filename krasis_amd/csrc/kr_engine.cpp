@@ -1134,11 +1134,10 @@ int kr_moe_prefill_set(kr_engine* e, int layer, const void* x_bf16, const int32_
         auto shared_gemm = [&](const KrPfDense& d) { kr_launch_pf_gemm(d.m, d.wsum, d.a_hi, d.a_lo, d.a_scale, nullptr, topk, 0, 0, d.rows, d.out, d.out_ld, st); };
         auto shared_act = [&] { kr_launch_pf_act((const float*)P.sgu.p, mc, SI, 2 * SI, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.shh.p, (int8_t*)P.shl.p,
                                                  (float*)P.shs.p, st); };
-        kr_launch_pf_gemm(L.w13.view(), (const uint32_t*)L.w13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, &so, topk, 1,
-                          cut.max_tiles, 0, (float*)P.gu.p, 2 * I, st, 0, 0, var_rows, &cut, join ? &d13 : nullptr);
-        kr_launch_pf_act((const float*)P.gu.p, mc * topk, I, 2 * I, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.hh.p, (int8_t*)P.hl.p,
-                         (float*)P.hs.p, st);
-        if (join) shared_act();
+        const KrPfAct f13{act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.hh.p, (int8_t*)P.hl.p, (float*)P.hs.p};
+        const KrPfAct fs13{act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.shh.p, (int8_t*)P.shl.p, (float*)P.shs.p};
+        kr_launch_pf_w13_act(L.w13.view(), (const uint32_t*)L.w13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, &so, topk, (float*)P.gu.p, mc * topk, f13, st,
+                             var_rows, cut, join ? &d13 : nullptr, &fs13);
         kr_launch_pf_gemm(L.w2.view(), (const uint32_t*)L.w2.wsum.p, (const int8_t*)P.hh.p, (const int8_t*)P.hl.p, (const float*)P.hs.p, &so, topk, 0,
                           cut.max_tiles, 0, (float*)P.eo.p, H, st, 0, 0, var_rows, &cut, join ? &d2 : nullptr);
         if (use_shared && !join) { shared_gemm(d13); shared_act(); shared_gemm(d2); }
@@ -1183,9 +1182,8 @@ int kr_moe_prefill_rows(kr_engine* e, int layer, const void* rows_bf16, const in
         kr_launch_pf_sort(lid + m0, mc, 1, E, so, st, cut);
         kr_launch_pf_quant_x((const uint16_t*)rows_bf16 + (size_t)m0 * H, mc, H, (int8_t*)P.xh.p, (int8_t*)P.xl.p, (float*)P.xs.p, st);
         const int var_rows = (long)mc < 48L * E;
-        kr_launch_pf_gemm(L.w13.view(), (const uint32_t*)L.w13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, &so, 1, 1,
-                          cut.max_tiles, 0, (float*)P.gu.p, 2 * I, st, 0, 0, var_rows, &cut);
-        kr_launch_pf_act((const float*)P.gu.p, mc, I, 2 * I, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.hh.p, (int8_t*)P.hl.p, (float*)P.hs.p, st);
+        const KrPfAct f13{act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.hh.p, (int8_t*)P.hl.p, (float*)P.hs.p};
+        kr_launch_pf_w13_act(L.w13.view(), (const uint32_t*)L.w13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, &so, 1, (float*)P.gu.p, mc, f13, st, var_rows, cut);
         kr_launch_pf_gemm(L.w2.view(), (const uint32_t*)L.w2.wsum.p, (const int8_t*)P.hh.p, (const int8_t*)P.hl.p, (const float*)P.hs.p, &so, 1, 0,
                           cut.max_tiles, 0, (float*)((char*)out + (size_t)m0 * H * ob), H, st, 1, out_bf16, var_rows, &cut);
     }

@@ -35,6 +35,10 @@ void kr_launch_pf_gemm(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_
                        int gather_tokens, int max_tiles, int single_expert_rows, float* out, int out_ld, hipStream_t st, int scatter_rows = 0, int out_bf16 = 0,
                        int var_rows = 0 /* expert tiles mostly <= 32 rows: kernel variant that skips empty 32-row blocks */,
                        const KrPfTiles* t = nullptr /* of the tile table; null: tiles of 64 */, const KrPfDense* beside = nullptr /* for the same launch, where kr_pf_joins */);
+// activation of gate | up and where the hidden rows' digits go ([rows][n] twice, scales [rows][n / 128])
+struct KrPfAct { int mode; float limit, alpha; int8_t* hh; int8_t* hl; float* hs; };
+void kr_launch_pf_w13_act(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_hi, const int8_t* a_lo, const float* a_scale, const KrPfSort* sort, int topk, float* gu, int rows,
+                          const KrPfAct& act, hipStream_t st, int var_rows, const KrPfTiles& t, const KrPfDense* beside = nullptr, const KrPfAct* beside_act = nullptr);
 bool kr_pf_joins(const KrPfTiles& t, const KrMatDev& experts, const KrMatDev& dense, int rows);
 // of the exact GEMMs that will run on one tile table: tiles of 128 rows (the wide kernel) or 64, and whether strips may take their place
 KrPfTiles kr_pf_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows /* of all their slots */, int E, bool beside /* launches of other chunks run at the same time */);

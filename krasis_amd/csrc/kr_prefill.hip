@@ -211,6 +211,28 @@ __global__ void kr_pf_quant_x_kernel(const uint16_t* __restrict__ x, int K, int8
     }
 }
 
+// one value of the hidden row, and the digits of eight of them by one of the sixteen lanes that hold a group (all sixteen call it; `hs`: where the group's scale goes, one lane's)
+__device__ __forceinline__ float pf_act_value(int act, float gate, float up, float swiglu_limit, float alpha) {
+    if (act == KR_ACT_GPTOSS) {
+        if (gate > swiglu_limit) gate = swiglu_limit;
+        if (up > swiglu_limit) up = swiglu_limit;
+        if (up < -swiglu_limit) up = -swiglu_limit;
+        return (up + 1.0f) * (gate * kr_sigmoid_poly5_scalar(gate * alpha));
+    }
+    return (gate * kr_sigmoid_poly5(gate)) * up;
+}
+__device__ __forceinline__ void pf_act_digits(int act, const float (&h)[8], bool store, int8_t* hh, int8_t* hl, float* hs) {
+    float mx = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) mx = fmaxf(mx, fabsf(h[i]));
+    mx = kr_red16_max_f32(mx);
+    const float scale = mx > 0.0f ? mx / 32767.0f : 1.0f, inv = mx > 0.0f ? 32767.0f / mx : 0.0f;
+    int q[8];
+    if (act == KR_ACT_SILU_FUSED) kr_quant8<true>(h, inv, q); else kr_quant8<false>(h, inv, q);
+    if (!store) return;
+    kr_store_digits(hh, hl, q);
+    if (hs) *hs = scale;
+}
 // hidden digits from gu rows: silu_quantize_int16_avx2 (avx2.rs:2310) or the GPT-OSS activation (moe.rs:268-287). grid (rows), block I/8
 template <int ACT>
 __global__ void kr_pf_act_kernel(const float* __restrict__ gu, int n, int gu_ld, float swiglu_limit, float alpha, int8_t* __restrict__ hh,
@@ -221,24 +243,10 @@ __global__ void kr_pf_act_kernel(const float* __restrict__ gu, int n, int gu_ld,
         const float4 g0 = *reinterpret_cast<const float4*>(g + c * 8), g1 = *reinterpret_cast<const float4*>(g + c * 8 + 4);
         const float4 u0 = *reinterpret_cast<const float4*>(g + n + c * 8), u1 = *reinterpret_cast<const float4*>(g + n + c * 8 + 4);
         const float gg[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w}, uu[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-        float h[8], mx = 0.0f;
+        float h[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            if (ACT == KR_ACT_GPTOSS) {
-                float gate = gg[i], up = uu[i];
-                if (gate > swiglu_limit) gate = swiglu_limit;
-                if (up > swiglu_limit) up = swiglu_limit;
-                if (up < -swiglu_limit) up = -swiglu_limit;
-                h[i] = (up + 1.0f) * (gate * kr_sigmoid_poly5_scalar(gate * alpha));
-            } else h[i] = (gg[i] * kr_sigmoid_poly5(gg[i])) * uu[i];
-            mx = fmaxf(mx, fabsf(h[i]));
-        }
-        mx = kr_red16_max_f32(mx);
-        const float scale = mx > 0.0f ? mx / 32767.0f : 1.0f, inv = mx > 0.0f ? 32767.0f / mx : 0.0f;
-        int q[8];
-        if (ACT == KR_ACT_SILU_FUSED) kr_quant8<true>(h, inv, q); else kr_quant8<false>(h, inv, q);
-        kr_store_digits(hh + (size_t)row * n + c * 8, hl + (size_t)row * n + c * 8, q);
-        if ((c & 15) == 0) hs[(size_t)row * (n / 128) + (c >> 4)] = scale;
+        for (int i = 0; i < 8; i++) h[i] = pf_act_value(ACT, gg[i], uu[i], swiglu_limit, alpha);
+        pf_act_digits(ACT, h, true, hh + (size_t)row * n + c * 8, hl + (size_t)row * n + c * 8, (c & 15) == 0 ? hs + (size_t)row * (n / 128) + (c >> 4) : nullptr);
     }
 }
 
@@ -298,6 +306,7 @@ struct KrPfGemmArgs {
     // (q | k | v, qkvz | ba, shared gate_up | shared gate: a 64- or 1-column GEMM of its own is one latency-bound launch per chunk and layer)
     int n_extra; KrMatDev mx[2]; const uint32_t* wsumx[2]; float* outx[2]; int out_ldx[2];
     int sr, sc;                             // dense launches: super-tile shape per XCD (kr_pf_super_tile), set by the launcher
+    int act_mode; float act_limit, act_alpha; int8_t* act_hh; int8_t* act_hl; float* act_hs;      // the wide kernel's activation form: where the digits of the hidden rows [row][N / 2] go
 };
 
 #include "kr_prefill_gemm2.inc"
@@ -463,6 +472,29 @@ void kr_launch_pf_gemm(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_
     // wave grid that were measured
     if (m.bits == 8) kr_pf_gemm2_launch<32, 2, 8>(a, mt, st);
     else kr_pf_gemm2_launch<32, 2, 4>(a, mt, st);
+}
+// Gate and up products of a pass's experts and the digits of the hidden rows.  The wide kernel forms the digits itself where a group of them is a workgroup's column block, N a multiple of 256
+// (its products never pass through memory: 3001 rows on 64 INT8 experts, us a layer, 799 -> 749); the other kernels leave gate and up in `gu`, for a launch of the activation.
+void kr_launch_pf_w13_act(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_hi, const int8_t* a_lo, const float* a_scale, const KrPfSort* sort, int topk, float* gu, int rows,
+                          const KrPfAct& act, hipStream_t st, int var_rows, const KrPfTiles& t, const KrPfDense* beside, const KrPfAct* beside_act) {
+    if (t.rows == PFW_TM && m.N % 256 == 0 && (!beside || beside->m.N % 256 == 0)) {
+        auto args = [](KrPfGemmArgs& a, const KrPfAct& f) {
+            a.act_mode = f.mode; a.act_limit = f.limit; a.act_alpha = f.alpha; a.act_hh = f.hh; a.act_hl = f.hl; a.act_hs = f.hs;
+        };
+        KrPfGemmArgs a{}, b{};
+        a.m = m; a.wsum = wsum; a.a_hi = a_hi; a.a_lo = a_lo; a.a_scale = a_scale; a.topk = topk; a.gather_tokens = 1;
+        a.row_pair = sort->row_pair; a.tile_expert = sort->tile_expert; a.tile_row0 = sort->tile_row0; a.tile_rows = sort->tile_rows; a.n_tiles = sort->n_tiles;
+        args(a, act);
+        if (beside) {
+            b.m = beside->m; b.wsum = beside->wsum; b.a_hi = beside->a_hi; b.a_lo = beside->a_lo; b.a_scale = beside->a_scale; b.topk = topk; b.single_expert = 1; b.total_rows = beside->rows;
+            args(b, *beside_act);
+        }
+        if (m.bits == 8) kr_pf_wide_launch<8, true>(a, t.max_tiles, st, beside ? &b : nullptr); else kr_pf_wide_launch<4, true>(a, t.max_tiles, st, beside ? &b : nullptr);
+        return;
+    }
+    kr_launch_pf_gemm(m, wsum, a_hi, a_lo, a_scale, sort, topk, 1, t.max_tiles, 0, gu, m.N, st, 0, 0, var_rows, &t, beside);
+    kr_launch_pf_act(gu, rows, m.N / 2, m.N, act.mode, act.limit, act.alpha, act.hh, act.hl, act.hs, st);
+    if (beside) kr_launch_pf_act(beside->out, beside->rows, beside->m.N / 2, beside->m.N, beside_act->mode, beside_act->limit, beside_act->alpha, beside_act->hh, beside_act->hl, beside_act->hs, st);
 }
 // dense GEMMs of up to three matrices over the same A rows (rows 0..M-1 in order), one launch; all matrices share K and the weight width
 void kr_launch_pf_gemm_multi(const KrMatDev* mats, const uint32_t* const* wsums, float* const* outs, const int* out_lds, int n, const int8_t* a_hi, const int8_t* a_lo,

@@ -39,3 +39,25 @@ def test_shared_expert_in_the_experts_launches(M, H, I, bits, w2_bits, n_shared)
     whole = mgr.forward(0, x, ids, w).view(torch.int16).cpu().numpy()
     few = np.concatenate([mgr.forward(0, x[i:i + 40], ids[i:i + 40], w[i:i + 40]).view(torch.int16).cpu().numpy() for i in range(0, M, 40)])
     assert np.array_equal(whole, few)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("limit", [0.0, 0.75])
+def test_hidden_digits_of_the_gate_and_up_launch(bits, limit):
+    # the wide kernel's own digits against the activation's launch (forty rows at a time), both activations: rows of exact zeros (a scale of one), a row far past the clamp, ragged tiles
+    import torch
+    from krasis_amd import GpuPrefillManager, KrasisEngine, ModelConfig
+    from tests.util import make_experts, upload
+    H, I, E, k, M = 384, 384, 5, 2, 301
+    rng = np.random.default_rng(7)
+    experts, shared = make_experts(rng, E, H, I, bits), make_experts(rng, 1, H, I, bits)[0]
+    eng = KrasisEngine(); eng.configure(ModelConfig(H, I, E, k, 1, 1, 1.0, swiglu_limit=limit, activation_alpha=1.702))
+    upload(eng, 0, experts, shared)
+    mgr = GpuPrefillManager(eng, k)
+    x = rand_bf16(rng, (M, H)); x[3] = 0; x[200] = 0
+    x = torch.from_numpy(x.view(np.int16)).cuda().view(torch.bfloat16)
+    x[17] *= 64
+    ids = torch.from_numpy(np.stack([rng.permutation(E)[:k] for _ in range(M)]).astype(np.int32)).cuda(); w = torch.from_numpy(rng.random((M, k)).astype(np.float32)).cuda()
+    whole = mgr.forward(0, x, ids, w).view(torch.int16).cpu().numpy()
+    few = np.concatenate([mgr.forward(0, x[i:i + 40], ids[i:i + 40], w[i:i + 40]).view(torch.int16).cpu().numpy() for i in range(0, M, 40)])
+    assert np.array_equal(whole, few) and np.any(whole[17]) and not np.any(whole[3] & 0x7FFF)

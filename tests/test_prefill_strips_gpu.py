@@ -97,6 +97,24 @@ def test_exact_strips_of_whole_and_ragged_tiles(counts):
     assert np.array_equal(out.view(np.uint32), _forward(eng, torch, x, ids, w).view(np.uint32))
 
 
+@pytest.mark.parametrize("E,per,strip", [(250, 12, 32), (257, 12, 32), (300, 12, 32), (520, 6, 16), (640, 6, 16)])
+def test_exact_strips_whose_last_round_is_cut(E, per, strip):
+    """tiles around what the chip holds (256 workgroups of 32 rows, 512 of 16): whole rounds with several strips a wave, and the tiles that are left, among them none, in smaller pieces"""
+    import torch
+    from krasis_amd import KrasisEngine, ModelConfig
+    from tests.util import make_experts, upload
+    rng = np.random.default_rng(E)
+    few = make_experts(rng, 7, 512, 512, 4)
+    eng = KrasisEngine(); eng.configure(ModelConfig(512, 512, E, 1, 1, 0, 1.0))
+    upload(eng, 0, [few[e % 7] for e in range(E)], None)
+    counts = np.full(E, per); counts[3], counts[8] = 0, strip + 1
+    ids = _one_each(counts, 1, rng)
+    x = rand_bf16(rng, (len(ids), 512)); w = rng.random((len(ids), 1)).astype(F)
+    out = _prefill_mode(eng, torch, x, ids, w, 0)
+    assert _cut(eng) == (0, E)                               # one tile an expert, one expert without, one with two
+    assert np.array_equal(out.view(np.uint32), _forward(eng, torch, x, ids, w).view(np.uint32))
+
+
 @pytest.mark.parametrize("Ms,ret_bf16", [([20, 12], False), ([20, 12], True), ([3, 0], False)])
 def test_scattered_rows_of_expert_parallel_ranks(Ms, ret_bf16):
     """nine rows a local expert, each row stored at the place that it came from, in f32 and in bf16"""

@@ -615,21 +615,20 @@ __global__ void __launch_bounds__(64 * PFH_ST_WAVES, 4) kr_pfh_strip_kernel(cons
     // this wave's strips: cb * WAVES * strips_per_wave + wave + WAVES * i, each ngp steps
     const int nstrip = m.N / 16, s0 = cb * WAVES * strips_per_wave + wave;
     const int mine = s0 < nstrip ? min(strips_per_wave, (nstrip - s0 + WAVES - 1) / WAVES) : 0, steps = __builtin_amdgcn_readfirstlane(mine * ngp);
-    const uint32_t woff = ((uint32_t)(r >> 3) * ngp * 64 + (r & 7) * 8 + q) * 16, soff = (uint32_t)(r >> 3) * ngp * 8 + (r & 7);
-    const char* wb = wq + (size_t)2 * s0 * ngp * 1024;
-    size_t sb = (size_t)2 * s0 * ngp * 8;
-    int rs = s0, rg = 0;                                       // strip and step of the next request
-    auto request = [&](PfhStripStep& p) {
-        p.w[0] = kr_ldg_nt(reinterpret_cast<const u32x4*>(wb + woff)); p.w[1] = kr_ldg_nt(reinterpret_cast<const u32x4*>(wb + woff + 64));
+    const uint32_t woff = ((r & 7) * 8 + (r >> 3) * 4 + q) * 16, woff1 = woff + (uint32_t)ngp * 1024, soff = (uint32_t)(r >> 3) * ngp * 8 + (r & 7);
+    int rs = min(s0, nstrip - 1), rg = 0, rn = 1;              // strip and step of the next request, and its number
+    const char* wb = wq + (size_t)2 * rs * ngp * 1024;
+    size_t sb = (size_t)2 * rs * ngp * 8;
+    auto request = [&](PfhStripStep& p) {                      // whole lines; past the last step: that one's bytes again, so that no request hangs on a condition
+        p.w[0] = kr_ldg_nt(reinterpret_cast<const u32x4*>(wb + woff)); p.w[1] = kr_ldg_nt(reinterpret_cast<const u32x4*>(wb + woff1));
         p.sc = wsc[sb + soff];
+        if (rn++ >= steps) return;
         wb += 1024; sb += 8;
         if (++rg == ngp) { rg = 0; rs += WAVES; wb = wq + (size_t)2 * rs * ngp * 1024; sb = (size_t)2 * rs * ngp * 8; }
     };
     PfhStripStep ring[D];
-    if (mine > 0) {
 #pragma unroll
-        for (int d = 0; d < D; d++) if (d < steps) request(ring[d]);
-    }
+    for (int d = 0; d < D; d++) request(ring[d]);
     // ---- the tile's rows, 16 bytes (8 k, in image order) per thread and turn; rows past the last one hold zeros
     for (int i = tid; i < ROWS * (K / 8); i += 64 * WAVES) {
         const int row = i / (K / 8), k8 = i - row * (K / 8);
@@ -650,6 +649,13 @@ __global__ void __launch_bounds__(64 * PFH_ST_WAVES, 4) kr_pfh_strip_kernel(cons
     int cs = s0, gp = 0;                                       // strip and step in it of the next step
     auto step = [&](const PfhStripStep& p) {
         if (gp == 0) acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        // w[0] came from columns 0 - 7 and w[1] from 8 - 15: lanes r < 8 hold the first 64 k of both groups, the others the second.  Lanes r and r ^ 8 trade
+        u32x4 w[2];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            w[0][e] = __builtin_amdgcn_update_dpp(p.w[0][e], p.w[1][e], 0x128, 0xF, 0xC, false);      // row_ror:8
+            w[1][e] = __builtin_amdgcn_update_dpp(p.w[1][e], p.w[0][e], 0x128, 0xF, 0x3, false);
+        }
 #pragma unroll
         for (int hh = 0; hh < 2; hh++) {
             const int g = 2 * gp + hh;
@@ -660,7 +666,7 @@ __global__ void __launch_bounds__(64 * PFH_ST_WAVES, 4) kr_pfh_strip_kernel(cons
             for (int s = 0; s < 2; s++)
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
-                    const v8h wf = pfh_dq4(p.w[s][2 * hh + h], sq, cq, M0, M1, MH, Kc);
+                    const v8h wf = pfh_dq4(w[s][2 * hh + h], sq, cq, M0, M1, MH, Kc);
                     acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf, *reinterpret_cast<const v8h*>(arow + g * 256 + s * 128 + h * 16), acc, 0, 0, 0);      // k = 128 g + 16 (q + 4 s) + 8 h
                 }
         }
@@ -678,15 +684,13 @@ __global__ void __launch_bounds__(64 * PFH_ST_WAVES, 4) kr_pfh_strip_kernel(cons
         } else *reinterpret_cast<float4*>(a.out + o) = make_float4(acc[0] * rm, acc[1] * rm, acc[2] * rm, acc[3] * rm);
     };
     int i = 0;
-    for (; i + 2 * D <= steps; i += D) {       // (no branch around a request: the compiler's count of what is in flight stays exact)
+    for (; i + D < steps; i += D) {            // (no branch around a request: the compiler's count of what is in flight stays exact)
 #pragma unroll
         for (int d = 0; d < D; d++) { step(ring[d]); request(ring[d]); }
     }
-    for (; i < steps; i += D) {
 #pragma unroll
-        for (int d = 0; d < D; d++)
-            if (i + d < steps) { step(ring[d]); if (i + d + D < steps) request(ring[d]); }
-    }
+    for (int d = 0; d < D; d++)
+        if (i + d < steps) step(ring[d]);
 }
 static size_t pfh_strip_lds(int K) { return (size_t)PFH_ST_ROWS * (2 * K + 16 + 4); }
 static void pfh_strip_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st) {

@@ -18,11 +18,12 @@ constexpr int sk_steps(int K, int WV) {
 }
 // MB, NB: row and column blocks of 16; WV: waves.  bx: strip, by: problem row of a grouped problem; red: sk_red_floats of LDS, act (with ACT): the rows' activation [16 MB][K + 8].
 // GLU (NB = 2): the strip is 16 gate columns, counted from g.glu_lo, and the 16 up columns that belong to them; their activation goes to g.glu_out, nothing to C.
-template <int MB, int NB, int WV, bool ACT, bool GLU = false, int U = NB * MB <= 2 ? 8 : 4>      // U: k steps requested together
+template <int MB, int NB, int WV, bool ACT, bool GLU = false, int U = NB * MB <= 2 ? 8 : 4, int LD = 0>      // U: k steps requested together; LD: how (below)
 __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const int by, float* red, uint16_t* act) {
     static_assert(!GLU || (NB == 2 && MB == 1), "a gate tile and its up tile");
     constexpr int TR = MB * NB < 4 ? MB * NB : 4;             // output tiles per round of the reduction
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4, n0 = bx * 16 * (GLU ? 1 : NB);
+    // (the wave's number is scalar, and so are its k steps: a matrix instruction does not heed the execution mask, it has to stand behind a real branch)
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, q = lane >> 4, n0 = bx * 16 * (GLU ? 1 : NB);
     int lo = 0, hi = g.M, N = g.N;
     const uint16_t* W = (const uint16_t*)g.W;
     if (g.row_group) {
@@ -35,15 +36,38 @@ __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const 
     if (n0 >= (GLU ? g.glu_f : N)) return;
     float* host = gm_host(g.c_host);
     const int ks = g.K / 32, s0 = ks * wave / WV, s1 = ks * (wave + 1) / WV, lda = g.K + 8;
-    const uint16_t* wp[NB];
+    // How the weights are read.  0: half a line from each of the sixteen columns per request.  2: whole 128-byte lines, two k steps of eight columns (lanes r < 8 the first step, the others the second; the
+    // even one of a pair of requests takes columns 0 - 7 of the block, the odd one 8 - 15), which lanes r and r ^ 8 then trade, and past the caches.  For matrices that a step meets once
+    // and whose strips are in flight together (us, 0 / 2: two rows of 14336 x 2048 15.7 / 13.7, 2048 x 6144 10.9 / 10.0, 12 rows of 4224 x 2048 10.1 / 9.6).  Not for experts whose workgroups
+    // come in many rounds (72 rows on 64 experts of 768 x 2048 30.9 / 31.7), nor for more than two rows that go to host memory (32768 columns, 12 rows: 48 / 63; three alike; one and two
+    // gain, not there but in the launches of the next step, whose matrices the vocabulary's 134 MB then leave in the last cache: a chat turn 5890 / 5750, two requests of a recurrent model 5670 / 5600).
+    // All matrices, with the k steps scalar (112 -> 74 registers, 12 words of scratch -> 0 beside attention): 72 rows on 64 experts of 2 x 768 x 2048 beside attention 60.1 -> 52.6.
+    constexpr bool LINES = LD == 2;
+    const uint16_t* wp[NB][LINES ? 2 : 1];
 #pragma unroll
-    for (int b = 0; b < NB; b++) wp[b] = W + (size_t)(GLU ? g.glu_lo + min(n0 + r, g.glu_f - 1) + b * g.glu_f : min(n0 + b * 16 + r, N - 1)) * g.K + q * 8;
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int t = 0; t < (LINES ? 2 : 1); t++) {
+            const int c = LINES ? 8 * t + (r & 7) : r;
+            wp[b][t] = W + (size_t)(GLU ? g.glu_lo + min(n0 + c, g.glu_f - 1) + b * g.glu_f : min(n0 + b * 16 + c, N - 1)) * g.K + q * 8;
+        }
     auto request = [&](gu4 (&wv)[U][NB], int s) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int k = min(s + u, s1 - 1) * 32;             // steps past the wave's last one are requested again and not multiplied
+            const int k = min(LINES ? s + (u & ~1) + (r >> 3) : s + u, s1 - 1) * 32;      // steps past the wave's last one are requested again and not multiplied
 #pragma unroll
-            for (int b = 0; b < NB; b++) wv[u][b] = *reinterpret_cast<const gu4*>(wp[b] + k);
+            for (int b = 0; b < NB; b++) {
+                const gu4* p = reinterpret_cast<const gu4*>(wp[b][LINES ? u & 1 : 0] + k);
+                wv[u][b] = LINES ? __builtin_nontemporal_load(p) : *p;
+            }
+        }
+    };
+    [[maybe_unused]] auto trade = [&](gu4 (&wv)[U][NB], int u, int b) {         // lanes r and r ^ 8: step u + t of column r in wv[u + t]
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const uint32_t x = wv[u][b][e], y = wv[u + 1][b][e];
+            wv[u][b][e] = __builtin_amdgcn_update_dpp(x, y, 0x128, 0xF, 0xC, false);        // row_ror:8
+            wv[u + 1][b][e] = __builtin_amdgcn_update_dpp(y, x, 0x128, 0xF, 0x3, false);
         }
     };
     for (int m0 = lo; m0 < hi; m0 += 16 * MB) {
@@ -90,6 +114,10 @@ __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const 
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
+                if (LINES && u % 2 == 0) {
+#pragma unroll
+                    for (int b = 0; b < NB; b++) trade(wv, u, b);
+                }
                 if (s + u < s1) {
 #pragma unroll
                     for (int a = 0; a < MB; a++)
@@ -139,7 +167,7 @@ __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const 
 template <int WV>
 __device__ __forceinline__ void sk_row_glu(const KrSvGemm& g, const int bx, const int by) {
     constexpr int U = 4;                                      // 16-byte pieces of K requested together, of both matrices
-    const int lane = threadIdx.x & 63, n = bx * WV + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, n = bx * WV + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (n >= g.glu_f) return;
     const uint16_t* W = (const uint16_t*)g.W + (size_t)g.row_group[by] * g.w_stride + (size_t)n * g.K;
     const uint16_t* A = (const uint16_t*)g.A + (size_t)(g.a_rows ? g.a_rows[by] : by) * g.lda;
@@ -149,8 +177,8 @@ __device__ __forceinline__ void sk_row_glu(const KrSvGemm& g, const int bx, cons
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int k = min(k0 + 512 * u + lane * 8, g.K - 8);      // lanes past the row's end read its last piece and multiply it by zero
-            wg[u] = *reinterpret_cast<const gu4*>(W + k);
-            wu[u] = *reinterpret_cast<const gu4*>(W + (size_t)g.glu_f * g.K + k);
+            wg[u] = __builtin_nontemporal_load(reinterpret_cast<const gu4*>(W + k));      // (used once, and not in the way of what the next step meets again)
+            wu[u] = __builtin_nontemporal_load(reinterpret_cast<const gu4*>(W + (size_t)g.glu_f * g.K + k));
         }
 #pragma unroll
         for (int u = 0; u < U; u++) {

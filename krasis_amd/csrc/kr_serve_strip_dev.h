@@ -162,14 +162,12 @@ __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const 
     }
 }
 
-// The gate and up product of problem row `by` alone, columns [WV bx, WV bx + WV) of g.glu_f, one per wave, K over its lanes: for few rows, which seldom meet
-// an expert twice.  A wave reads whole rows of the matrix and waits for nothing but its row's expert.
-template <int WV>
-__device__ __forceinline__ void sk_row_glu(const KrSvGemm& g, const int bx, const int by) {
+// Column n of the gate and up product of problem row `by`, K over a wave's lanes.  PAST: past the caches.
+template <bool PAST>
+__device__ __forceinline__ void sk_row_glu_column(const KrSvGemm& g, const int n, const int by, const int group) {
     constexpr int U = 4;                                      // 16-byte pieces of K requested together, of both matrices
-    const int lane = threadIdx.x & 63, n = bx * WV + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (n >= g.glu_f) return;
-    const uint16_t* W = (const uint16_t*)g.W + (size_t)g.row_group[by] * g.w_stride + (size_t)n * g.K;
+    const int lane = threadIdx.x & 63;
+    const uint16_t* W = (const uint16_t*)g.W + (size_t)group * g.w_stride + (size_t)n * g.K;
     const uint16_t* A = (const uint16_t*)g.A + (size_t)(g.a_rows ? g.a_rows[by] : by) * g.lda;
     float gt = 0.0f, up = 0.0f;
     for (int k0 = 0; k0 < g.K; k0 += 512 * U) {
@@ -177,8 +175,9 @@ __device__ __forceinline__ void sk_row_glu(const KrSvGemm& g, const int bx, cons
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int k = min(k0 + 512 * u + lane * 8, g.K - 8);      // lanes past the row's end read its last piece and multiply it by zero
-            wg[u] = __builtin_nontemporal_load(reinterpret_cast<const gu4*>(W + k));      // (used once, and not in the way of what the next step meets again)
-            wu[u] = __builtin_nontemporal_load(reinterpret_cast<const gu4*>(W + (size_t)g.glu_f * g.K + k));
+            const gu4 *pg = reinterpret_cast<const gu4*>(W + k), *pu = reinterpret_cast<const gu4*>(W + (size_t)g.glu_f * g.K + k);
+            wg[u] = PAST ? __builtin_nontemporal_load(pg) : *pg;
+            wu[u] = PAST ? __builtin_nontemporal_load(pu) : *pu;
         }
 #pragma unroll
         for (int u = 0; u < U; u++) {
@@ -199,6 +198,18 @@ __device__ __forceinline__ void sk_row_glu(const KrSvGemm& g, const int bx, cons
     for (int o = 32; o > 0; o >>= 1) { gt += __shfl_xor(gt, o); up += __shfl_xor(up, o); }
     const float wt = g.glu_row_w ? g.glu_row_w[by] : 1.0f;
     if (lane == 0) ((uint16_t*)g.glu_out)[(size_t)by * g.glu_f + n] = kr_f32_to_bf16(gm_act_once(gt * wt, up * wt, g.glu_kind, g.glu_limit, g.glu_alpha));
+}
+// The gate and up product of problem row `by` alone, columns [WV bx, WV bx + WV) of g.glu_f, one per wave: for few rows, which seldom meet an expert twice.  A wave reads whole
+// rows of the matrix and waits for nothing but its row's expert and its neighbours' (rows of one expert stand together).  A row that has its expert to itself reads past the caches;
+// where a neighbour reads the matrix too it has to stay (us a step: 24 rows on 8 of 128 experts of
+// 2 x 1536 x 4096, one layer, all past the caches / none / this rule 261 / 238 / 239, on 22 of them 301 / 304 / 298; one request, six rows, two layers of 64 of 2 x 768 x 2048 132 / 139 / 131).
+template <int WV>
+__device__ __forceinline__ void sk_row_glu(const KrSvGemm& g, const int bx, const int by) {
+    const int n = bx * WV + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (n >= g.glu_f) return;
+    const int group = g.row_group[by], before = g.row_group[max(by - 1, 0)], behind = g.row_group[min(by + 1, g.M - 1)];
+    if ((before != group || by == 0) && (behind != group || by == g.M - 1)) sk_row_glu_column<true>(g, n, by, group);
+    else sk_row_glu_column<false>(g, n, by, group);
 }
 
 #endif

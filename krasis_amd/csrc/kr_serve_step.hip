@@ -39,29 +39,28 @@ __global__ void __launch_bounds__(64 * AU_WAVES, 4) sv_attn_up_kernel(const KrSv
     }
 }
 
-// U: k steps together of the down projections, by their K (sk_steps).  UO: of attention's projection; where many rows' experts fill the chip, six at a time (us, six / eight,
-// before the k steps were scalar: 72 rows of 768 x 2048 on 64 experts 30.2 / 32.7, 24 of 1536 x 4096 on 128 74.6 / 76.8; six rows 9.9 / 9.0)
-// LD: how the weights are read (sk_strip), whole lines up to sixteen rows
-template <int UO, int U, int LD>
-__global__ void __launch_bounds__(256) sv_downs_kernel(const KrSvGemm o, const KrSvGemm e, const KrSvGemm sh, const int so, const int ss, const int se) {
+// U: k steps together of the down projections, by their K (sk_steps); attention's projection takes eight.  128 registers: with more waves to a SIMD asked for, or none, the compiler
+// orders the requests worse (72 rows on 43 of 64 experts of 2048 x 768 27.0 us, 29.1 without the bound).
+// LD: how the weights are read (sk_strip), whole lines up to sixteen expert rows (us, halves / lines: 16 rows on 16 of 128 experts of 4096 x 1536 44.1 / 38.9, 12 on 11 of 64 of 2048 x 768
+// 10.9 / 10.2, of 2048 x 704 11.1 / 10.9).  Beyond it depends: 24 rows of 4096 x 1536 59.7 / 53.5, 96 161 / 154, but 72 of 2048 x 768 27.0 / 27.8, of 2048 x 704 27.5 / 30.1.
+template <int U, int LD>
+__global__ void __launch_bounds__(256, 4) sv_downs_kernel(const KrSvGemm o, const KrSvGemm e, const KrSvGemm sh, const int so, const int ss, const int se) {
     __shared__ __attribute__((aligned(16))) float red[sk_red_floats(1, 1, 4)];
     extern __shared__ __attribute__((aligned(16))) uint16_t act[];
     int i = blockIdx.x;
-    if (i < so) { sk_strip<1, 1, 4, false, false, UO, LD>(o, i, 0, red, act); return; }
+    if (i < so) { sk_strip<1, 1, 4, false, false, 8, LD>(o, i, 0, red, act); return; }
     i -= so;
     if (i < ss) { sk_strip<1, 1, 4, true, false, U, LD>(sh, i, 0, red, act); return; }
     i -= ss;
     const int by = __builtin_amdgcn_readfirstlane(i / se);
     sk_strip<1, 1, 4, false, false, U, LD>(e, i - by * se, by, red, act);
 }
-template <int UO, int U, int LD> void downs_launch_u(const KrSvGemm& o, const KrSvGemm& e, const KrSvGemm& sh, int so, int ss, int se, int lds, hipStream_t st) {
-    if (kr_lds_optin((const void*)sv_downs_kernel<UO, U, LD>, lds)) return;
-    hipLaunchKernelGGL((sv_downs_kernel<UO, U, LD>), dim3(so + ss + se * e.M), dim3(256), lds, st, o, e, sh, so, ss, se);
+template <int U, int LD> void downs_launch_u(const KrSvGemm& o, const KrSvGemm& e, const KrSvGemm& sh, int so, int ss, int se, int lds, hipStream_t st) {
+    if (kr_lds_optin((const void*)sv_downs_kernel<U, LD>, lds)) return;
+    hipLaunchKernelGGL((sv_downs_kernel<U, LD>), dim3(so + ss + se * e.M), dim3(256), lds, st, o, e, sh, so, ss, se);
 }
 template <int U> void downs_launch(const KrSvGemm& o, const KrSvGemm& e, const KrSvGemm& sh, int so, int ss, int se, int lds, hipStream_t st) {
-    if (e.M <= 16) downs_launch_u<8, U, 2>(o, e, sh, so, ss, se, lds, st);
-    else if (U < 8) downs_launch_u<6, U, 0>(o, e, sh, so, ss, se, lds, st);
-    else downs_launch_u<8, U, 0>(o, e, sh, so, ss, se, lds, st);
+    if (e.M <= 16) downs_launch_u<U, 2>(o, e, sh, so, ss, se, lds, st); else downs_launch_u<U, 0>(o, e, sh, so, ss, se, lds, st);
 }
 
 template <int DIM, int VDIM> void au_launch(const KrSvAttn& a, const KrSvGemm& up, hipStream_t st) {

@@ -2,6 +2,8 @@
 // launches of one product and the launches that put several products, or a product and attention, side by side (kr_serve_step.hip).
 #ifndef KR_SERVE_STRIP_DEV_H
 #define KR_SERVE_STRIP_DEV_H
+#include <type_traits>
+
 #include "kr_serve_gemm_dev.h"
 
 typedef float sk_f4 __attribute__((ext_vector_type(4)));
@@ -22,7 +24,7 @@ template <int MB, int NB, int WV, bool ACT, bool GLU = false, int U = NB * MB <=
 __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const int by, float* red, uint16_t* act) {
     static_assert(!GLU || (NB == 2 && MB == 1), "a gate tile and its up tile");
     constexpr int TR = MB * NB < 4 ? MB * NB : 4;             // output tiles per round of the reduction
-    // (the wave's number is scalar, and so are its k steps: a matrix instruction does not heed the execution mask, it has to stand behind a real branch)
+    // (the wave's number is scalar, and so are its k steps: 112 -> 74 registers)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, q = lane >> 4, n0 = bx * 16 * (GLU ? 1 : NB);
     int lo = 0, hi = g.M, N = g.N;
     const uint16_t* W = (const uint16_t*)g.W;
@@ -103,8 +105,10 @@ __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const 
         for (int a = 0; a < MB; a++)
 #pragma unroll
             for (int b = 0; b < NB; b++) acc[a][b] = sk_f4{0.0f, 0.0f, 0.0f, 0.0f};
-        for (int s = s0; s < s1; s += U) {
-            if (!ACT || s > s0) request(wv, s);
+        // U steps of k; part: fewer are left, the others' operands are zeros.  No branch stands around a product: a matrix instruction does not heed the execution mask, and the compiler
+        // puts a request that only the product behind a branch needs behind that branch too, a round trip of its own (us, branches / none: 72 rows on 43 of 64 experts of 2048 x 768 31.1 / 27.0,
+        // 96 on 71 of 128 of 4096 x 1536 189 / 162, 20 rows of 2048 x 768 5.44 / 4.90).
+        auto products = [&](int s, auto part) {
             gu4 av[U][MB];
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -112,19 +116,33 @@ __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const 
 #pragma unroll
                 for (int a = 0; a < MB; a++) av[u][a] = *reinterpret_cast<const gu4*>(ap[a] + k);
             }
+            // every request before the first product (us, without / with: 24 rows on 22 of 64 experts of 2048 x 768 19.1 / 16.4).  Not where registers are short (pairs beside attention: 20 bytes of
+            // scratch, twelve requests' step 333 / 338), nor where the rows come from LDS (experts' and shared expert's strips of twelve requests alike 12.9 / 13.5)
+            if (!LINES && !ACT && MB * NB == 1 && U > 4) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 if (LINES && u % 2 == 0) {
 #pragma unroll
                     for (int b = 0; b < NB; b++) trade(wv, u, b);
                 }
-                if (s + u < s1) {
+                const bool none = decltype(part)::value && s + u >= s1;
 #pragma unroll
-                    for (int a = 0; a < MB; a++)
+                for (int a = 0; a < MB; a++)
 #pragma unroll
-                        for (int b = 0; b < NB; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gb8, wv[u][b]), __builtin_bit_cast(gb8, av[u][a]), acc[a][b], 0, 0, 0);
-                }
+                    for (int b = 0; b < NB; b++) {
+                        const gu4 zero = {0, 0, 0, 0}, x = none ? zero : wv[u][b], y = none ? zero : av[u][a];
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gb8, x), __builtin_bit_cast(gb8, y), acc[a][b], 0, 0, 0);
+                    }
             }
+        };
+        int s = s0;
+        for (; s + U <= s1; s += U) {
+            if (!ACT || s > s0) request(wv, s);
+            products(s, std::false_type{});
+        }
+        if (s < s1) {
+            if (!ACT || s > s0) request(wv, s);
+            products(s, std::true_type{});
         }
         // the waves' partial sums meet, TR tiles of 16 x 16 at a time: tile element (row r, column c) at r * 16 + c, a lane holds four columns of one row
 #pragma unroll

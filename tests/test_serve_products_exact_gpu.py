@@ -88,7 +88,7 @@ def streams(eng, vocab):
 
 # a wave's steps of 32 k: none, one, odd and even numbers of them, several rounds of eight.  Rows of the experts: each alone (up to 24, among them rows that share an expert) and in strips,
 # down projections of up to sixteen and of more rows, one to sixteen rows an expert
-@pytest.mark.parametrize("width,heads,ff,shared_ff", [(96, 1, 32, 32), (352, 2, 160, 96), (1088, 3, 544, 224), (2080, 9, 704, 768)])
+@pytest.mark.parametrize("width,heads,ff,shared_ff", [(96, 1, 32, 32), (352, 2, 160, 96), (1088, 3, 544, 224), (2080, 9, 992, 768)])
 @pytest.mark.parametrize("T,top,experts", [(1, 1, 4), (2, 2, 8), (3, 2, 4), (12, 2, 16), (13, 2, 8), (16, 1, 2), (16, 2, 8), (16, 2, 64)])
 def test_joined_decode_step(T, top, experts, width, heads, ff, shared_ff):
     cfg = O.make_config(width=width, vocab=T, eps=1e-30, layers=[{"type": "attention", "mixer": O.attn(heads, 1, 32, 32, 0, 0, scale=0.3), "mlp": O.moe(experts, top, 1, 1, ff, 4096.0, shared_ff, 4096.0)}])

@@ -163,6 +163,9 @@ int kr_reduce_sum_bf16(kr_engine* e, const void* const* inputs, int n_inputs, vo
 int kr_moe_set_prefill_pairs(kr_engine* e, int pairs);
 /* test hook: how the last pass of kr_moe_prefill cut its rows, in tiles or in strips (few rows per expert); waits for the device */
 int kr_moe_prefill_tiles(kr_engine* e, int* tiles, int* strips);
+/* test hook, without a GPU: what the strips' launch (16 or 32 rows a tile) for a [N, K] matrix and up to max_tiles tiles does when there are `tiles`: its grid; cut[3]: the first cut[2]
+ * tiles with 2^cut[0] strips a wave, the others with 2^cut[1]; for every workgroup below n_places its tile (-1: none), column block and strips, 2^places[3 b + 2] a wave */
+int kr_moe_strip_plan(int strip, int N, int K, int max_tiles, int tiles, int* cut, int* places, int n_places, int* grid);
 /* numerics of the prompt-pass expert GEMMs of kr_moe_prefill: 0 (default) = the CPU engine's arithmetic (INT16 activation digits, one f32 fma per
  * 128-group: bit-identical to kr_moe_forward, moe.rs:184); 1 = tolerance form: f16 activations x weights de-quantized in registers, f32 accumulation
  * over the whole k range -- the dataflow of the reference's GPU prompt pass (gpu_prefill.py:64-239, Marlin).  Native GGUF layers stay exact.

@@ -1211,6 +1211,13 @@ extern "C" int kr_moe_prefill_tiles(kr_engine* e, int* tiles, int* strips) {
     return KR_OK;
 }
 
+extern "C" int kr_moe_strip_plan(int strip, int N, int K, int max_tiles, int tiles, int* cut, int* places, int n_places, int* grid) {
+    if ((strip != 16 && strip != 32) || N < 16 || N % 16 || K < 128 || K % 128 || max_tiles < 1 || tiles < 0 || tiles > max_tiles || !cut || !grid || n_places < 0 || (n_places && !places))
+        return kr_fail(KR_ERR_VALUE, "kr_moe_strip_plan: strips of 16 or 32 rows, N by 16, K by 128, 0 <= tiles <= max_tiles");
+    kr_pf_strip_plan(strip, N, K, max_tiles, tiles, cut, places, n_places, grid);
+    return KR_OK;
+}
+
 // test / tuning hook: (token, slot) pairs per pass of kr_moe_prefill (0 = default 81 920)
 extern "C" int kr_moe_set_prefill_pairs(kr_engine* e, int pairs) {
     if (!e) return kr_fail(KR_ERR_VALUE, "null engine");

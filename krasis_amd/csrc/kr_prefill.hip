@@ -419,7 +419,7 @@ static bool pf_all_fma(const KrMatDev& m) { return m.n_fma >= m.N; }
 // 600 tokens, four layers, 5.28 -> 5.00 ms).  The rows' digits have to fit the LDS.
 // Whether they are taken is for the experts' own rows to say.  An expert's second strip reads its weights again, and where every row goes to the same ten experts that is all there is
 // (300 tokens of 48 such layers: tiles 20.4 ms, strips 22.4, this choice 20.7).  Measured with ever fewer experts in use, strips of 16 are the faster ones up to 1.6 times as many as tiles (400
-// rows, 1.41 253 / 220 us, 1.57 215 / 210, 1.95 163 / 172), strips of 32 up to 1.35 (1136 rows, 1.28 397 / 368, 1.35 355 / 353, 1.53 291 / 306); the launch that finds nothing costs 5 us,
+// rows, 1.41 253 / 220 us, 1.57 215 / 210, 1.95 163 / 172), strips of 32 up to 1.35 (1136 rows, 1.28 397 / 368, 1.35 355 / 353, 1.53 291 / 306); the launch that finds nothing costs some 5 us,
 // so the lines are 12 / 8 and 10 / 8.
 KrPfTiles kr_pf_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows, int E, bool beside) {
     if (!pf_all_fma(m0) || !pf_all_fma(m1)) return kr_pf_cut(PF_BM, 0, 0, tokens, rows, E);

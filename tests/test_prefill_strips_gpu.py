@@ -7,6 +7,7 @@ import pytest
 
 from tests.test_gemm_fast_gpu import _setup
 from tests.test_gemm_ring_gpu import _prefill_mode
+from tests.test_prefill_strips_cpu import plan
 from tests.util import rand_bf16
 
 pytestmark = pytest.mark.gpu
@@ -97,8 +98,10 @@ def test_exact_strips_of_whole_and_ragged_tiles(counts):
     assert np.array_equal(out.view(np.uint32), _forward(eng, torch, x, ids, w).view(np.uint32))
 
 
-@pytest.mark.parametrize("E,per,strip", [(250, 12, 32), (257, 12, 32), (300, 12, 32), (520, 6, 16), (640, 6, 16)])
-def test_exact_strips_whose_last_round_is_cut(E, per, strip):
+# (strips a wave of the whole rounds, of the rest, tiles in whole rounds; none where all are alike) of the two products
+@pytest.mark.parametrize("E,per,strip,cuts", [(250, 12, 32, (None, None)), (257, 12, 32, ((4, 1, 256), (2, 1, 256))), (300, 12, 32, ((4, 1, 256), (2, 1, 256))),
+                                              (520, 6, 16, ((4, 1, 512), (2, 1, 512))), (576, 6, 16, ((4, 1, 512), (2, 1, 512))), (640, 6, 16, (None, (2, 1, 512)))])
+def test_exact_strips_whose_last_round_is_cut(E, per, strip, cuts):
     """tiles around what the chip holds (256 workgroups of 32 rows, 512 of 16): whole rounds with several strips a wave, and the tiles that are left, among them none, in smaller pieces"""
     import torch
     from krasis_amd import KrasisEngine, ModelConfig
@@ -112,6 +115,10 @@ def test_exact_strips_whose_last_round_is_cut(E, per, strip):
     x = rand_bf16(rng, (len(ids), 512)); w = rng.random((len(ids), 1)).astype(F)
     out = _prefill_mode(eng, torch, x, ids, w, 0)
     assert _cut(eng) == (0, E)                               # one tile an expert, one expert without, one with two
+    most = len(ids) // strip + E + 1
+    for N, want in ((1024, cuts[0]), (512, cuts[1])):
+        (first, others, whole), places = plan(strip, N, 512, most, E)
+        assert ((first, others, whole) == want) if want else (first == others or whole == E), (N, first, others, whole)
     assert np.array_equal(out.view(np.uint32), _forward(eng, torch, x, ids, w).view(np.uint32))
 
 

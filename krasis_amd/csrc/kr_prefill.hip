@@ -473,28 +473,28 @@ void kr_launch_pf_gemm(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_
     if (m.bits == 8) kr_pf_gemm2_launch<32, 2, 8>(a, mt, st);
     else kr_pf_gemm2_launch<32, 2, 4>(a, mt, st);
 }
-// Gate and up products of a pass's experts and the digits of the hidden rows.  The wide kernel forms the digits itself where a group of them is a workgroup's column block, N a multiple of 256
-// (its products never pass through memory: 3001 rows on 64 INT8 experts, us a layer, 799 -> 749); the other kernels leave gate and up in `gu`, for a launch of the activation.
+// Gate and up products of a pass's experts and the digits of the hidden rows.  The wide kernel forms the digits itself: a group of them is a workgroup's column block (N, twice a multiple of 128, is one of
+// 256), and its products never pass through memory (3001 rows on 64 INT8 experts, us a layer, 799 -> 749).  The other kernels leave gate and up in `gu`, for a launch of the activation.
+// `beside`: where kr_pf_joins, that is beside the wide kernel only.
 void kr_launch_pf_w13_act(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_hi, const int8_t* a_lo, const float* a_scale, const KrPfSort* sort, int topk, float* gu, int rows,
                           const KrPfAct& act, hipStream_t st, int var_rows, const KrPfTiles& t, const KrPfDense* beside, const KrPfAct* beside_act) {
-    if (t.rows == PFW_TM && m.N % 256 == 0 && (!beside || beside->m.N % 256 == 0)) {
-        auto args = [](KrPfGemmArgs& a, const KrPfAct& f) {
-            a.act_mode = f.mode; a.act_limit = f.limit; a.act_alpha = f.alpha; a.act_hh = f.hh; a.act_hl = f.hl; a.act_hs = f.hs;
-        };
-        KrPfGemmArgs a{}, b{};
-        a.m = m; a.wsum = wsum; a.a_hi = a_hi; a.a_lo = a_lo; a.a_scale = a_scale; a.topk = topk; a.gather_tokens = 1;
-        a.row_pair = sort->row_pair; a.tile_expert = sort->tile_expert; a.tile_row0 = sort->tile_row0; a.tile_rows = sort->tile_rows; a.n_tiles = sort->n_tiles;
-        args(a, act);
-        if (beside) {
-            b.m = beside->m; b.wsum = beside->wsum; b.a_hi = beside->a_hi; b.a_lo = beside->a_lo; b.a_scale = beside->a_scale; b.topk = topk; b.single_expert = 1; b.total_rows = beside->rows;
-            args(b, *beside_act);
-        }
-        if (m.bits == 8) kr_pf_wide_launch<8, true>(a, t.max_tiles, st, beside ? &b : nullptr); else kr_pf_wide_launch<4, true>(a, t.max_tiles, st, beside ? &b : nullptr);
+    if (t.rows != PFW_TM) {
+        kr_launch_pf_gemm(m, wsum, a_hi, a_lo, a_scale, sort, topk, 1, t.max_tiles, 0, gu, m.N, st, 0, 0, var_rows, &t);
+        kr_launch_pf_act(gu, rows, m.N / 2, m.N, act.mode, act.limit, act.alpha, act.hh, act.hl, act.hs, st);
         return;
     }
-    kr_launch_pf_gemm(m, wsum, a_hi, a_lo, a_scale, sort, topk, 1, t.max_tiles, 0, gu, m.N, st, 0, 0, var_rows, &t, beside);
-    kr_launch_pf_act(gu, rows, m.N / 2, m.N, act.mode, act.limit, act.alpha, act.hh, act.hl, act.hs, st);
-    if (beside) kr_launch_pf_act(beside->out, beside->rows, beside->m.N / 2, beside->m.N, beside_act->mode, beside_act->limit, beside_act->alpha, beside_act->hh, beside_act->hl, beside_act->hs, st);
+    auto args = [](KrPfGemmArgs& a, const KrPfAct& f) {
+        a.act_mode = f.mode; a.act_limit = f.limit; a.act_alpha = f.alpha; a.act_hh = f.hh; a.act_hl = f.hl; a.act_hs = f.hs;
+    };
+    KrPfGemmArgs a{}, b{};
+    a.m = m; a.wsum = wsum; a.a_hi = a_hi; a.a_lo = a_lo; a.a_scale = a_scale; a.topk = topk; a.gather_tokens = 1;
+    a.row_pair = sort->row_pair; a.tile_expert = sort->tile_expert; a.tile_row0 = sort->tile_row0; a.tile_rows = sort->tile_rows; a.n_tiles = sort->n_tiles;
+    args(a, act);
+    if (beside) {
+        b.m = beside->m; b.wsum = beside->wsum; b.a_hi = beside->a_hi; b.a_lo = beside->a_lo; b.a_scale = beside->a_scale; b.topk = topk; b.single_expert = 1; b.total_rows = beside->rows;
+        args(b, *beside_act);
+    }
+    if (m.bits == 8) kr_pf_wide_launch<8, true>(a, t.max_tiles, st, beside ? &b : nullptr); else kr_pf_wide_launch<4, true>(a, t.max_tiles, st, beside ? &b : nullptr);
 }
 // dense GEMMs of up to three matrices over the same A rows (rows 0..M-1 in order), one launch; all matrices share K and the weight width
 void kr_launch_pf_gemm_multi(const KrMatDev* mats, const uint32_t* const* wsums, float* const* outs, const int* out_lds, int n, const int8_t* a_hi, const int8_t* a_lo,

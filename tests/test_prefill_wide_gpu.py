@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from tests.test_prefill_gpu import _setup
+from tests.test_prefill_strips_gpu import _cut
 from tests.util import rand_bf16
 
 pytestmark = pytest.mark.gpu
@@ -58,6 +59,13 @@ def test_hidden_digits_of_the_gate_and_up_launch(bits, limit):
     x = torch.from_numpy(x.view(np.int16)).cuda().view(torch.bfloat16)
     x[17] *= 64
     ids = torch.from_numpy(np.stack([rng.permutation(E)[:k] for _ in range(M)]).astype(np.int32)).cuda(); w = torch.from_numpy(rng.random((M, k)).astype(np.float32)).cuda()
+    counts = np.bincount(ids.flatten().cpu().numpy(), minlength=E)
     whole = mgr.forward(0, x, ids, w).view(torch.int16).cpu().numpy()
-    few = np.concatenate([mgr.forward(0, x[i:i + 40], ids[i:i + 40], w[i:i + 40]).view(torch.int16).cpu().numpy() for i in range(0, M, 40)])
-    assert np.array_equal(whole, few) and np.any(whole[17]) and not np.any(whole[3] & 0x7FFF)
+    assert _cut(eng) == (sum(-(-c // 128) for c in counts), 0) and _cut(eng)[0] < sum(-(-c // 64) for c in counts)      # the wide kernel's tiles
+    few = []
+    for i in range(0, M, 40):
+        few.append(mgr.forward(0, x[i:i + 40], ids[i:i + 40], w[i:i + 40]).view(torch.int16).cpu().numpy())
+        counts = np.bincount(ids[i:i + 40].flatten().cpu().numpy(), minlength=E)
+        assert _cut(eng) in ((sum(-(-c // 64) for c in counts), 0), (0, sum(-(-c // 32) for c in counts)), (0, sum(-(-c // 16) for c in counts)))
+    assert np.array_equal(whole, np.concatenate(few)) and np.any(whole[17]) and not np.any(whole[3] & 0x7FFF)
+

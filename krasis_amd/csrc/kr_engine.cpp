@@ -6,6 +6,7 @@
 // the reference's CPU/GPU split, expert DMA, LRU/HCS caches (python/krasis/gpu_prefill.py) do not exist here.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -1103,11 +1104,15 @@ int kr_moe_prefill_set(kr_engine* e, int layer, const void* x_bf16, const int32_
     const int CH = M < CHmax ? M : CHmax;
     const size_t np = (size_t)CH * topk;
     const int max_tiles = (int)(np / 16) + E + 1;      // (strips of 16 rows are the smallest, kr_pf_tiles)
+    auto joins = [&](const KrPfTiles& t, int mc) { return use_shared && kr_pf_joins(t, L.w13.view(), L.sw13.view(), mc) && kr_pf_joins(t, L.w2.view(), L.sw2.view(), mc); };
+    // gate and up in memory: of this pass, or of the smaller ones that leave them there
+    const KrPfTiles most = kr_pf_tiles(L.w13.view(), L.w2.view(), CH, (long)np, E, beside);
+    const size_t gu_rows = kr_pf_gu_rows(most, np, E), sgu_rows = joins(most, CH) ? std::min((size_t)CH, gu_rows / topk) : CH;
     const size_t n_i32 = 3 * (size_t)E + 3 * (size_t)max_tiles + 4 + 2 * np;
     if (P.i32.ensure(n_i32 * 4) || P.xh.ensure((size_t)CH * H) || P.xl.ensure((size_t)CH * H) || P.xs.ensure((size_t)CH * (H / 128) * 4) ||
-        P.gu.ensure(np * 2 * I * 4) || P.hh.ensure(np * I) || P.hl.ensure(np * I) || P.hs.ensure(np * (I / 128) * 4) || P.eo.ensure(np * H * 4))
+        P.gu.ensure(gu_rows * 2 * I * 4) || P.hh.ensure(np * I) || P.hl.ensure(np * I) || P.hs.ensure(np * (I / 128) * 4) || P.eo.ensure(np * H * 4))
         return kr_fail(KR_ERR_HIP, "hipMalloc of prefill scratch failed");
-    if (use_shared && (P.sgu.ensure((size_t)CH * 2 * SI * 4) || P.shh.ensure((size_t)CH * SI) || P.shl.ensure((size_t)CH * SI) ||
+    if (use_shared && (P.sgu.ensure(sgu_rows * 2 * SI * 4) || P.shh.ensure((size_t)CH * SI) || P.shl.ensure((size_t)CH * SI) ||
                        P.shs.ensure((size_t)CH * (SI / 128) * 4) || P.seo.ensure((size_t)CH * H * 4)))
         return kr_fail(KR_ERR_HIP, "hipMalloc of prefill scratch failed");
     int* ib = (int*)P.i32.p;
@@ -1130,7 +1135,7 @@ int kr_moe_prefill_set(kr_engine* e, int layer, const void* x_bf16, const int32_
             d13 = KrPfDense{L.sw13.view(), (const uint32_t*)L.sw13.wsum.p, (const int8_t*)P.xh.p, (const int8_t*)P.xl.p, (const float*)P.xs.p, mc, (float*)P.sgu.p, 2 * SI};
             d2 = KrPfDense{L.sw2.view(), (const uint32_t*)L.sw2.wsum.p, (const int8_t*)P.shh.p, (const int8_t*)P.shl.p, (const float*)P.shs.p, mc, (float*)P.seo.p, H};
         }
-        const bool join = use_shared && kr_pf_joins(cut, L.w13.view(), d13.m, mc) && kr_pf_joins(cut, L.w2.view(), d2.m, mc);
+        const bool join = joins(cut, mc);
         auto shared_gemm = [&](const KrPfDense& d) { kr_launch_pf_gemm(d.m, d.wsum, d.a_hi, d.a_lo, d.a_scale, nullptr, topk, 0, 0, d.rows, d.out, d.out_ld, st); };
         auto shared_act = [&] { kr_launch_pf_act((const float*)P.sgu.p, mc, SI, 2 * SI, act_mode, e->cfg.swiglu_limit, e->cfg.activation_alpha, (int8_t*)P.shh.p, (int8_t*)P.shl.p,
                                                  (float*)P.shs.p, st); };
@@ -1165,9 +1170,10 @@ int kr_moe_prefill_rows(kr_engine* e, int layer, const void* rows_bf16, const in
     const int CH = n < pairs ? n : pairs;
     const size_t np = (size_t)CH;
     const int max_tiles = (int)(np / 16) + E + 1;      // (strips of 16 rows are the smallest, kr_pf_tiles)
+    const size_t gu_rows = kr_pf_gu_rows(kr_pf_tiles(L.w13.view(), L.w2.view(), CH, (long)np, E, true), np, E);      // (see kr_moe_prefill_set)
     const size_t n_i32 = 3 * (size_t)E + 3 * (size_t)max_tiles + 4 + 2 * np;
     if (P.i32.ensure(n_i32 * 4) || P.xh.ensure((size_t)CH * H) || P.xl.ensure((size_t)CH * H) || P.xs.ensure((size_t)CH * (H / 128) * 4) ||
-        P.gu.ensure(np * 2 * I * 4) || P.hh.ensure(np * I) || P.hl.ensure(np * I) || P.hs.ensure(np * (I / 128) * 4))
+        P.gu.ensure(gu_rows * 2 * I * 4) || P.hh.ensure(np * I) || P.hl.ensure(np * I) || P.hs.ensure(np * (I / 128) * 4))
         return kr_fail(KR_ERR_HIP, "hipMalloc of prefill scratch failed");
     int* ib = (int*)P.i32.p;
     KrPfSort so{};

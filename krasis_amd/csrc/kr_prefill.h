@@ -39,6 +39,7 @@ void kr_launch_pf_gemm(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_
 struct KrPfAct { int mode; float limit, alpha; int8_t* hh; int8_t* hl; float* hs; };
 void kr_launch_pf_w13_act(const KrMatDev& m, const uint32_t* wsum, const int8_t* a_hi, const int8_t* a_lo, const float* a_scale, const KrPfSort* sort, int topk, float* gu, int rows,
                           const KrPfAct& act, hipStream_t st, int var_rows, const KrPfTiles& t, const KrPfDense* beside = nullptr, const KrPfAct* beside_act = nullptr);
+size_t kr_pf_gu_rows(const KrPfTiles& t, size_t rows, int E);      // rows of gate and up that kr_launch_pf_w13_act may leave in memory, in a pass of `rows` that is cut as t or in a smaller one
 void kr_pf_strip_plan(int strip, int N, int K, int max_tiles, int tiles, int* cut, int* places, int n_places, int* grid);
 bool kr_pf_joins(const KrPfTiles& t, const KrMatDev& experts, const KrMatDev& dense, int rows);
 // of the exact GEMMs that will run on one tile table: tiles of 128 rows (the wide kernel) or 64, and whether strips may take their place

@@ -12,6 +12,8 @@
 // one-fma-per-group f32 chain as the reference: out = fma(f32(isum), bf16(w_scale) * a_scale, out).
 //
 // Tile: 64 rows (tokens routed to one expert) x 128 columns per workgroup of 4 waves; one group PAIR (256 k) per LDS stage.
+#include <algorithm>
+
 #include "kr_lds_optin.h"
 #include "kr_device.h"
 #include "kr_kernels.h"
@@ -431,6 +433,7 @@ KrPfTiles kr_pf_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long r
     }
     return kr_pf_cut(PF_BM, 0, 0, tokens, rows, E);
 }
+size_t kr_pf_gu_rows(const KrPfTiles& t, size_t rows, int E) { return t.rows == PFW_TM ? std::min(rows, 48 * (size_t)E - 1) : rows; }
 static bool pf_dense_wide(const KrPfGemmArgs& a) {
     int ncb = (a.m.N + PFW_TN - 1) / PFW_TN; bool all = pf_all_fma(a.m);
     for (int i = 0; i < a.n_extra; i++) { ncb += (a.mx[i].N + PFW_TN - 1) / PFW_TN; all = all && pf_all_fma(a.mx[i]); }

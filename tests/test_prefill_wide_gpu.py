@@ -69,3 +69,18 @@ def test_hidden_digits_of_the_gate_and_up_launch(bits, limit):
         assert _cut(eng) in ((sum(-(-c // 64) for c in counts), 0), (0, sum(-(-c // 32) for c in counts)), (0, sum(-(-c // 16) for c in counts)))
     assert np.array_equal(whole, np.concatenate(few)) and np.any(whole[17]) and not np.any(whole[3] & 0x7FFF)
 
+
+def test_gate_and_up_take_no_memory():
+    """2400 rows whose hidden digits leave the first launch: 39 MB of gate and up in f32 are not kept, only what a pass of fewer rows may leave"""
+    E, k, M, H, I = 9, 2, 1200, 256, 2048
+    eng, mgr, experts, shared, rng, torch = _setup(H, I, E, k, 1, 1.0)
+    x = torch.from_numpy(rand_bf16(rng, (M, H)).view(np.int16)).cuda().view(torch.bfloat16)
+    ids = torch.from_numpy(np.stack([rng.permutation(E)[:k] for _ in range(M)]).astype(np.int32)).cuda(); w = torch.from_numpy(rng.random((M, k)).astype(np.float32)).cuda()
+    mgr.forward(0, x[:40], ids[:40], w[:40])
+    torch.empty((M, H), device="cuda")                               # (torch's own, for the result)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    mgr.forward(0, x, ids, w)
+    torch.cuda.synchronize()
+    need = (M * k + M) * (2 * I + 4 * H) + 431 * 2 * I * 4 + 215 * 2 * I * 4      # digits and results; gate and up of up to 431 rows on nine experts, and of the shared one's 215
+    assert before - torch.cuda.mem_get_info()[0] <= need + (12 << 20)       # each buffer in whole pages of 2 MB

@@ -7,19 +7,19 @@
 // the last one (same address, no traffic) and are not stored.
 // ACT: A is the gated activation of act_gu, formed once per workgroup into LDS while the first weights travel (the wave-per-column form forms it again per column).
 // Grouped problems (one matrix per expert): a strip per problem row; the first row of a group takes the group's rows, the others leave at once.
-// Measured, us, before -> now (weights colder than the last cache): 12 rows: 4224 x 2048 23.9 -> 9.4, 2048 x 2048 19.2 -> 5.9, 32768 x 2048 110 -> 33.6 (4.0 TB/s); 1 row:
-// 9.3 -> 7.2, 6.6 -> 5.0, 45.6 -> 25.6 (5.2 TB/s); 64 experts of 1536 x 2048, 72 rows 54 -> 46 (5.9 TB/s), 180 rows 92 -> 68.
+// Measured, us, before -> now (weights colder than the last cache): 12 rows: 4224 x 2048 23.9 -> 9.3, 2048 x 2048 19.2 -> 5.7, 32768 x 2048 110 -> 33.6 (4.0 TB/s); 1 row:
+// 9.3 -> 7.3, 6.6 -> 4.9, 45.6 -> 25.6 (5.2 TB/s); 64 experts of 1536 x 2048, 72 rows 54 -> 46 (5.9 TB/s), 180 rows 92 -> 68.
 #include <algorithm>
 
 #include "kr_lds_optin.h"
 #include "kr_serve_strip_dev.h"
 
 namespace {
-template <int MB, int NB, int WV, bool ACT, int U, int LD>
+template <int MB, int NB, int WV, bool ACT, int U, bool LINES>
 __global__ void __launch_bounds__(64 * WV) sv_skinny_kernel(const KrSvGemm g) {
     __shared__ __attribute__((aligned(16))) float red[sk_red_floats(MB, NB, WV)];
     extern __shared__ __attribute__((aligned(16))) uint16_t act[];
-    sk_strip<MB, NB, WV, ACT, false, U, LD>(g, blockIdx.x, blockIdx.y, red, act);
+    sk_strip<MB, NB, WV, ACT, false, U, LINES>(g, blockIdx.x, blockIdx.y, red, act);
 }
 // the experts' and the shared expert's down projection of a step in one launch, both with the activation inside: neither fills the chip, and a launch with its gap costs more
 // than the smaller of the two (six expert rows and one row, 2048 x 768: 8.1 + 6.3 -> 8.7 us)
@@ -37,31 +37,31 @@ __global__ void __launch_bounds__(256) sv_skinny_pair_kernel(const KrSvGemm e, c
 __global__ void __launch_bounds__(256) sv_strips_kernel(const KrSvGemm a, const KrSvGemm b, const KrSvGemm c, const int na, const int nb) {
     __shared__ __attribute__((aligned(16))) float red[sk_red_floats(1, 2, 4)];
     int i = blockIdx.x;
-    if (i < na) { sk_strip<1, 1, 4, false, false, 8, 2>(a, i, 0, red, nullptr); return; }
+    if (i < na) { sk_strip<1, 1, 4, false, false, 8, true>(a, i, 0, red, nullptr); return; }
     i -= na;
-    if (i < nb) { sk_strip<1, 1, 4, false, false, 8, 2>(b, i, 0, red, nullptr); return; }
+    if (i < nb) { sk_strip<1, 1, 4, false, false, 8, true>(b, i, 0, red, nullptr); return; }
     i -= nb;
-    sk_strip<1, 2, 4, false, true, 8, 2>(c, i, 0, red, nullptr);
+    sk_strip<1, 2, 4, false, true, 8, true>(c, i, 0, red, nullptr);
 }
 
 int sk_act_lds(const KrSvGemm& g) { return (g.row_group ? 16 : std::min(16, g.M)) * (g.K + 8) * 2; }      // one block of sixteen rows
 
-template <int MB, int NB, int WV, int U, int LD>
+template <int MB, int NB, int WV, int U, bool LINES>
 void sk_launch_u(const KrSvGemm& g, hipStream_t st) {
     const dim3 grid((g.N + 16 * NB - 1) / (16 * NB), g.row_group ? g.M : 1);
     if (g.act_gu) {
         const int rows = g.row_group ? 16 * MB : std::min(16 * MB, g.M), lds = rows * (g.K + 8) * 2;
-        if (kr_lds_optin((const void*)sv_skinny_kernel<MB, NB, WV, true, U, LD>, lds)) return;
-        hipLaunchKernelGGL((sv_skinny_kernel<MB, NB, WV, true, U, LD>), grid, dim3(64 * WV), lds, st, g);
-    } else if (g.c_host && g.M > 2) hipLaunchKernelGGL((sv_skinny_kernel<MB, NB, WV, false, U, 0>), grid, dim3(64 * WV), 0, st, g);
-    else hipLaunchKernelGGL((sv_skinny_kernel<MB, NB, WV, false, U, LD>), grid, dim3(64 * WV), 0, st, g);
+        if (kr_lds_optin((const void*)sv_skinny_kernel<MB, NB, WV, true, U, LINES>, lds)) return;
+        hipLaunchKernelGGL((sv_skinny_kernel<MB, NB, WV, true, U, LINES>), grid, dim3(64 * WV), lds, st, g);
+    } else if (g.c_host && g.M > 2) hipLaunchKernelGGL((sv_skinny_kernel<MB, NB, WV, false, U, false>), grid, dim3(64 * WV), 0, st, g);
+    else hipLaunchKernelGGL((sv_skinny_kernel<MB, NB, WV, false, U, LINES>), grid, dim3(64 * WV), 0, st, g);
 }
-template <int MB, int NB, int WV, int LD>
+template <int MB, int NB, int WV, bool LINES>
 void sk_launch(const KrSvGemm& g, hipStream_t st) {
     switch (sk_steps(g.K, WV)) {
-        case 4: sk_launch_u<MB, NB, WV, 4, LD>(g, st); break;
-        case 6: sk_launch_u<MB, NB, WV, 6, LD>(g, st); break;
-        default: sk_launch_u<MB, NB, WV, 8, LD>(g, st); break;
+        case 4: sk_launch_u<MB, NB, WV, 4, LINES>(g, st); break;
+        case 6: sk_launch_u<MB, NB, WV, 6, LINES>(g, st); break;
+        default: sk_launch_u<MB, NB, WV, 8, LINES>(g, st); break;
     }
 }
 template <int U> void sk_pair_launch(const KrSvGemm& e, const KrSvGemm& o, int lds, hipStream_t st) {
@@ -87,10 +87,10 @@ void kr_sv_gemm_skinny(const KrSvGemm& g, hipStream_t st) {
     if (!g.seg) p.row_group = nullptr;
     // waves: four where the columns alone give every compute unit a workgroup (32768 x 2048, 12 rows: 33.6 us, eight waves 36.4), else eight, which halve a wave's
     // chain of requests (2048 x 768 with the activation, 12 rows: 8.2 us, four waves 9.7)
-    if (g.seg) sk_launch<1, 1, 4, 0>(p, st);
-    else if (g.M <= 16 && g.N >= 4096) sk_launch<1, 1, 4, 2>(p, st);
-    else if (g.M <= 16) sk_launch<1, 1, 8, 2>(p, st);
-    else sk_launch<2, 1, 8, 0>(p, st);
+    if (g.seg) sk_launch<1, 1, 4, false>(p, st);
+    else if (g.M <= 16 && g.N >= 4096) sk_launch<1, 1, 4, true>(p, st);
+    else if (g.M <= 16) sk_launch<1, 1, 8, true>(p, st);
+    else sk_launch<2, 1, 8, false>(p, st);
 }
 
 void kr_sv_gemm_skinny_pair(const KrSvGemm& e, const KrSvGemm& o, hipStream_t st) {

@@ -20,9 +20,9 @@ namespace {
 // Eight waves of at most 128 registers (the lean form of attention), two workgroups to a compute unit, for what streams the experts beside it.
 constexpr int AU_WAVES = 8;
 // Up to this many problem rows each is taken alone, a wave per gate column and its up column: whole matrix rows per request and no wait for the group's
-// bounds.  Against strips of 16 + 16 columns: six rows of 1536 x 2048 14.8 -> 11.4 us, 24 rows of 3072 x 4096 on 128 experts 112 -> 97.
-// With more rows than experts an expert's matrix is read once per row, which costs nothing while all of them stay in the 256 MB cache (a step of two layers, us, rows alone /
-// strips: 18 rows on 16 experts of 2 x 768 x 2048 254 / 264, 24 on 8 283 / 281) and much beyond it (8 experts of 2 x 4096 x 4096, 537 MB: 12 rows 561 / 497, 24 rows 865 / 632): hence half of it.
+// bounds.  A step, us, rows alone / strips of 16 + 16 columns: 24 rows on 64 experts of 2 x 768 x 2048, two layers, 192 / 206, on 128 of 2 x 1536 x 4096, one layer, 291 / 311.
+// With more rows than experts an expert's matrix is read by several rows, which costs little while all of them stay in the 256 MB cache (two layers: 18 rows on 16 experts of 2 x 768 x 2048 167 / 178,
+// 24 on 8 168 / 164) and much beyond it (one layer of 8 of 2 x 4096 x 4096, 537 MB: 12 rows 289 / 268, 24 rows 414 / 300): hence half of it.
 constexpr int AU_ROWS = 24;
 bool au_rows_alone(const KrSvGemm& up) { return up.M <= AU_ROWS && (up.M <= up.n_groups || (size_t)up.n_groups * up.w_stride * 2 <= (size_t)128 << 20); }
 template <int DIM, int VDIM>
@@ -41,26 +41,26 @@ __global__ void __launch_bounds__(64 * AU_WAVES, 4) sv_attn_up_kernel(const KrSv
 
 // U: k steps together of the down projections, by their K (sk_steps); attention's projection takes eight.  128 registers: with more waves to a SIMD asked for, or none, the compiler
 // orders the requests worse (72 rows on 43 of 64 experts of 2048 x 768 27.0 us, 29.1 without the bound).
-// LD: how the weights are read (sk_strip), whole lines up to sixteen expert rows (us, halves / lines: 16 rows on 16 of 128 experts of 4096 x 1536 44.1 / 38.9, 12 on 11 of 64 of 2048 x 768
+// LINES: how the weights are read (sk_strip), whole lines up to sixteen expert rows (us, halves / lines: 16 rows on 16 of 128 experts of 4096 x 1536 44.1 / 38.9, 12 on 11 of 64 of 2048 x 768
 // 10.9 / 10.2, of 2048 x 704 11.1 / 10.9).  Beyond it depends: 24 rows of 4096 x 1536 59.7 / 53.5, 96 161 / 154, but 72 of 2048 x 768 27.0 / 27.8, of 2048 x 704 27.5 / 30.1.
-template <int U, int LD>
+template <int U, bool LINES>
 __global__ void __launch_bounds__(256, 4) sv_downs_kernel(const KrSvGemm o, const KrSvGemm e, const KrSvGemm sh, const int so, const int ss, const int se) {
     __shared__ __attribute__((aligned(16))) float red[sk_red_floats(1, 1, 4)];
     extern __shared__ __attribute__((aligned(16))) uint16_t act[];
     int i = blockIdx.x;
-    if (i < so) { sk_strip<1, 1, 4, false, false, 8, LD>(o, i, 0, red, act); return; }
+    if (i < so) { sk_strip<1, 1, 4, false, false, 8, LINES>(o, i, 0, red, act); return; }
     i -= so;
-    if (i < ss) { sk_strip<1, 1, 4, true, false, U, LD>(sh, i, 0, red, act); return; }
+    if (i < ss) { sk_strip<1, 1, 4, true, false, U, LINES>(sh, i, 0, red, act); return; }
     i -= ss;
     const int by = __builtin_amdgcn_readfirstlane(i / se);
-    sk_strip<1, 1, 4, false, false, U, LD>(e, i - by * se, by, red, act);
+    sk_strip<1, 1, 4, false, false, U, LINES>(e, i - by * se, by, red, act);
 }
-template <int U, int LD> void downs_launch_u(const KrSvGemm& o, const KrSvGemm& e, const KrSvGemm& sh, int so, int ss, int se, int lds, hipStream_t st) {
-    if (kr_lds_optin((const void*)sv_downs_kernel<U, LD>, lds)) return;
-    hipLaunchKernelGGL((sv_downs_kernel<U, LD>), dim3(so + ss + se * e.M), dim3(256), lds, st, o, e, sh, so, ss, se);
+template <int U, bool LINES> void downs_launch_u(const KrSvGemm& o, const KrSvGemm& e, const KrSvGemm& sh, int so, int ss, int se, int lds, hipStream_t st) {
+    if (kr_lds_optin((const void*)sv_downs_kernel<U, LINES>, lds)) return;
+    hipLaunchKernelGGL((sv_downs_kernel<U, LINES>), dim3(so + ss + se * e.M), dim3(256), lds, st, o, e, sh, so, ss, se);
 }
 template <int U> void downs_launch(const KrSvGemm& o, const KrSvGemm& e, const KrSvGemm& sh, int so, int ss, int se, int lds, hipStream_t st) {
-    if (e.M <= 16) downs_launch_u<U, 2>(o, e, sh, so, ss, se, lds, st); else downs_launch_u<U, 0>(o, e, sh, so, ss, se, lds, st);
+    if (e.M <= 16) downs_launch_u<U, true>(o, e, sh, so, ss, se, lds, st); else downs_launch_u<U, false>(o, e, sh, so, ss, se, lds, st);
 }
 
 template <int DIM, int VDIM> void au_launch(const KrSvAttn& a, const KrSvGemm& up, hipStream_t st) {

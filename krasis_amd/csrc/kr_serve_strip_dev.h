@@ -11,7 +11,7 @@ typedef float sk_f4 __attribute__((ext_vector_type(4)));
 constexpr int sk_red_floats(int MB, int NB, int WV) { return WV * (MB * NB < 4 ? MB * NB : 4) * 256; }
 
 // k steps requested together: the count that leaves the fewest requests of no use behind a wave's last step (they are made all the same, for the last step's bytes again).  Eight where
-// six do, with 12 rows on 64 experts of 768 x 2048, 36.5 us where 27.7 do; 24 on 128 of 1536 x 4096 61 and 52.
+// six do, with 72 rows on 43 of 64 experts of 2048 x 768, 33.3 us where 26.8 do; 24 on 24 of 128 of 4096 x 1536 65.7 and 59.5.
 constexpr int sk_steps(int K, int WV) {
     const int steps = (K / 32 + WV - 1) / WV;
     int best = 8;
@@ -20,9 +20,10 @@ constexpr int sk_steps(int K, int WV) {
 }
 // MB, NB: row and column blocks of 16; WV: waves.  bx: strip, by: problem row of a grouped problem; red: sk_red_floats of LDS, act (with ACT): the rows' activation [16 MB][K + 8].
 // GLU (NB = 2): the strip is 16 gate columns, counted from g.glu_lo, and the 16 up columns that belong to them; their activation goes to g.glu_out, nothing to C.
-template <int MB, int NB, int WV, bool ACT, bool GLU = false, int U = NB * MB <= 2 ? 8 : 4, int LD = 0>      // U: k steps requested together; LD: how (below)
+template <int MB, int NB, int WV, bool ACT, bool GLU = false, int U = NB * MB <= 2 ? 8 : 4, bool LINES = false>      // U: k steps requested together; LINES: how (below)
 __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const int by, float* red, uint16_t* act) {
     static_assert(!GLU || (NB == 2 && MB == 1), "a gate tile and its up tile");
+    static_assert(!LINES || U % 2 == 0, "lines are taken by pairs of steps");
     constexpr int TR = MB * NB < 4 ? MB * NB : 4;             // output tiles per round of the reduction
     // (the wave's number is scalar, and so are its k steps: 112 -> 74 registers)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, q = lane >> 4, n0 = bx * 16 * (GLU ? 1 : NB);
@@ -38,13 +39,12 @@ __device__ __forceinline__ void sk_strip(const KrSvGemm& g, const int bx, const 
     if (n0 >= (GLU ? g.glu_f : N)) return;
     float* host = gm_host(g.c_host);
     const int ks = g.K / 32, s0 = ks * wave / WV, s1 = ks * (wave + 1) / WV, lda = g.K + 8;
-    // How the weights are read.  0: half a line from each of the sixteen columns per request.  2: whole 128-byte lines, two k steps of eight columns (lanes r < 8 the first step, the others the second; the
-    // even one of a pair of requests takes columns 0 - 7 of the block, the odd one 8 - 15), which lanes r and r ^ 8 then trade, and past the caches.  For matrices that a step meets once
-    // and whose strips are in flight together (us, 0 / 2: two rows of 14336 x 2048 15.7 / 13.7, 2048 x 6144 10.9 / 10.0, 12 rows of 4224 x 2048 10.1 / 9.6).  Not for experts whose workgroups
-    // come in many rounds (72 rows on 64 experts of 768 x 2048 30.9 / 31.7), nor for more than two rows that go to host memory (32768 columns, 12 rows: 48 / 63; three alike; one and two
-    // gain, not there but in the launches of the next step, whose matrices the vocabulary's 134 MB then leave in the last cache: a chat turn 5890 / 5750, two requests of a recurrent model 5670 / 5600).
-    // All matrices, with the k steps scalar (112 -> 74 registers, 12 words of scratch -> 0 beside attention): 72 rows on 64 experts of 2 x 768 x 2048 beside attention 60.1 -> 52.6.
-    constexpr bool LINES = LD == 2;
+    // How the weights are read: half a line from each of the sixteen columns per request, or (LINES) whole 128-byte lines, two k steps of eight columns (lanes r < 8 the first step, the others the second;
+    // the even one of a pair of requests takes columns 0 - 7 of the block, the odd one 8 - 15), which lanes r and r ^ 8 then trade, and past the caches.  Where a wave's part of K begins at an odd step,
+    // or K is an odd number of them, a pair holds halves of two lines (12 rows of 2048 x 704, us, halves / lines 4.31 / 3.95, of 3072 x 1056 4.70 / 4.68).  For matrices that a step meets once
+    // and whose strips are in flight together (two rows of 2048 x 6144 11.2 / 10.3, 2048 x 2048 5.48 / 4.95, 12 rows of 4224 x 2048 10.5 / 9.4); a matrix that is still in the caches is up to 15 % slower
+    // so.  Not for experts whose workgroups come in many rounds (sv_downs_kernel), nor for more than two rows that go to host memory (32768 columns, a step of twelve requests 314 / 333, of three 156 / 160;
+    // one and two gain, not there but in the launches of the next step, whose matrices the vocabulary's 134 MB then leave in the last cache).
     const uint16_t* wp[NB][LINES ? 2 : 1];
 #pragma unroll
     for (int b = 0; b < NB; b++)

@@ -413,16 +413,16 @@ void kr_launch_pf_wsum(const KrMatDev& m, int n_experts, uint32_t* wsum, hipStre
 // (a four-layer INT4 prompt, ms, 64-row tiles / wide from 128 tiles / always wide: 777 tokens 3.99 / 3.89 / 3.98, 1400 tokens 6.30 / 5.64 / 5.89).
 // It knows the fused form of the group sum only, and addresses a digit plane by 32-bit offsets.
 static bool pf_all_fma(const KrMatDev& m) { return m.n_fma >= m.N; }
-// Few rows per expert, INT4: strips may be taken, of 16 rows while an expert seldom has more (up to ten on average), then of 32 while two halves still cost less than the 64-row tile: to
-// 16 rows an expert, with many experts to 20 (us a layer, both products and what stands between them, tiles against this choice: 512 experts of 2048 x 512, top 10, 160 rows 308 / 207, 400 330 / 245, 700
-// in strips of 32 340 / 276; rows an expert, 256 of 2048 x 768 8 245 / 200, 16 253 / 219, 20 257 / 234, 24 270 / 279; 128 of 4096 x 1536 8 415 / 317, 16 447 / 431, 20 441 / 446; 64 of 2048 x 1408 6
-// 128 / 102, 14 131 / 124, 24 192 / 213).  Beside the launches of other chunks a workgroup of 32 rows (136 KB of LDS)
-// waits for an empty compute unit, also when it has nothing to do (two chunks of 750 tokens 48 ms against 57): strips of 16 only, which pay to twelve rows an expert there (two chunks of
-// 600 tokens, four layers, 5.28 -> 5.00 ms).  The rows' digits have to fit the LDS.
+// Few rows per expert, INT4: strips may be taken, of 16 rows while an expert seldom has more (up to ten on average), then of 32 to 16 rows an expert, with many experts to 20.  Beside the launches of other
+// chunks a workgroup of 32 rows (136 KB of LDS) waits for an empty compute unit, also when it has nothing to do (two chunks of 750 tokens 48 ms against 57): strips of 16 only, which pay to twelve rows an
+// expert there (two chunks of 600 tokens, four layers, 5.28 -> 5.00 ms).  The rows' digits have to fit the LDS.
+// us a layer, both products and what stands between them, tiles / strips of 16 / of 32, by rows an expert, each form alone: 512 experts of 2048 x 512 8 331 / 201 / 213, 12 340 / 234 / 232,
+// 20 357 / 367 / 283, 28 398 / 447 / 359; 256 of 2048 x 768 8 251 / 165 / 161, 16 268 / 230 / 184, 24 285 / 295 / 234; 64 of 2048 x 1408 6 130 / 91 / 94, 14 137 / 109 / 105, 20 139 / 149 / 124,
+// 28 155 / 177 / 130, 32 163 / 191 / 177; 128 of 4096 x 1536 8 431 / 277, 14 439 / 348, 18 453 / 447, 20 453 / 508 (no room for 32 rows).
 // Whether they are taken is for the experts' own rows to say.  An expert's second strip reads its weights again, and where every row goes to the same ten experts that is all there is
-// (300 tokens of 48 such layers: tiles 20.4 ms, strips 22.4, this choice 20.7).  Measured with ever fewer experts in use, strips of 16 are the faster ones up to 1.6 times as many as tiles (400
-// rows, 1.41 253 / 220 us, 1.57 215 / 210, 1.95 163 / 172), strips of 32 up to 1.35 (1136 rows, 1.28 397 / 368, 1.35 355 / 353, 1.53 291 / 306); the launch that finds nothing costs some 5 us,
-// so the lines are 12 / 8 and 10 / 8.
+// (300 tokens of 48 such layers: tiles 20.4 ms, strips 22.4, this choice 20.7).  At most 12 / 8 as many strips of 16 as tiles, 10 / 8 of 32 (ever fewer of 512 experts in use, tiles / strips of 16 at
+// 1.61 times as many 147 / 129, 1.81 196 / 197, 2.30 164 / 181; strips of 32 at 1.31 164 / 136, 1.85 145 / 137, 1.93 193 / 219); a launch that finds nothing costs 2.5 - 5 us.
+// The lines are where strips that took 10 - 17 % longer met the tiles: they lie on the safe side of these figures.
 KrPfTiles kr_pf_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows, int E, bool beside) {
     if (!pf_all_fma(m0) || !pf_all_fma(m1)) return kr_pf_cut(PF_BM, 0, 0, tokens, rows, E);
     const int K = 128 * (m0.ng > m1.ng ? m0.ng : m1.ng);

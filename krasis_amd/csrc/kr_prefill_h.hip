@@ -705,8 +705,9 @@ static void pfh_strip_launch(const KrPfGemmHArgs& a, int mt, hipStream_t st) {
     hipLaunchKernelGGL(kr_pfh_strip_kernel, dim3(((mt + 7) / 8) * 8 * ncb), dim3(64 * WAVES), lds, st, a, spw, ncb);
 }
 // How the rows on E experts are cut.  Evenly spread INT4 rows: strips of 16 up to nine rows an expert with more than 256 experts, seven with fewer, where every expert's weights are met once either way
-// and a strip waits for less; tiles (kr_prefill_w.hip) beyond.  Both products of a layer, us, strips / tiles: 512 experts of 2048 x 512, top 10: 200 tokens 175 / 201, 400 190 / 208,
-// 500 218 / 210, 700 245 / 214; 64 of 2048 x 1408, top 6: 40 tokens 79 / 78, 80 78 / 76, 110 94 / 78; 128 of 4096 x 1536, top 8: 60 tokens 279 / 277, 100 281 / 279, 150 343 / 282.
+// and a strip waits for less; tiles (kr_prefill_w.hip) beyond.  Both products of a layer and what stands between them, us, tiles / strips, by rows an expert: 512 experts of 2048 x 512 6 234 / 184,
+// 9 239 / 208, 12 242 / 225, 14 247 / 242, 16 248 / 280; 256 of 2048 x 768 7 180 / 143, 11 182 / 174, 14 185 / 189; 64 of 2048 x 1408 6 114 / 92, 9 101 / 99, 11 103 / 104; 128 of 4096 x 1536
+// 6 309 / 257, 8 309 / 304, 10 312 / 315.  The lines are where strips that took 6 - 8 % longer met the tiles.
 // The experts' own rows decide (see kr_pf_tiles), at up to 11 / 8 strips a tile of 64; tiles of 96 where few experts have fewer rows than that.  Under 512 rows in all the tiles, which
 // are taken there only where a handful of experts has them, are kr_pfh_gemm_kernel's of 128 columns, twice as many (48 tokens on 28 experts 49.7 us, 57.8 with half as many; 160 tokens on 38 72 and 69).
 KrPfTiles kr_pfh_tiles(const KrMatDev& m0, const KrMatDev& m1, int tokens, long rows, int E, KrPfhForm form) {

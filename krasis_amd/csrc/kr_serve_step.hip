@@ -34,17 +34,17 @@ __global__ void __launch_bounds__(64 * AU_WAVES, 4) sv_attn_up_kernel(const KrSv
         as_token<DIM, VDIM, AU_WAVES, true>(a, blockIdx.x - th * a.T, th - bz * a.kv_heads, bz, lds);
     } else {
         const int i = blockIdx.x - n_attn, by = __builtin_amdgcn_readfirstlane(i / strips);
-        if (alone) sk_row_glu<AU_WAVES>(up, i - by * strips, by);
+        if (alone) sk_row_glu<AU_WAVES>(up, i - by * strips, by, a.T == 1);
         else sk_strip<1, 2, AU_WAVES, false, true>(up, i - by * strips, by, lds, nullptr);
     }
 }
 
-// U: k steps together of the down projections, by their K (sk_steps); attention's projection takes eight.  128 registers: with more waves to a SIMD asked for, or none, the compiler
-// orders the requests worse (72 rows on 43 of 64 experts of 2048 x 768 27.0 us, 29.1 without the bound).
+// U: k steps together of the down projections, by their K (sk_steps); attention's projection takes eight.  128 registers for the requests of half lines: without the bound, or with one for more waves
+// to a SIMD, the compiler orders them worse (72 rows on 43 of 64 experts of 2048 x 768 27.0 us, 29.1 without); whole lines are as quick without it.
 // LINES: how the weights are read (sk_strip), whole lines up to sixteen expert rows (us, halves / lines: 16 rows on 16 of 128 experts of 4096 x 1536 44.1 / 38.9, 12 on 11 of 64 of 2048 x 768
 // 10.9 / 10.2, of 2048 x 704 11.1 / 10.9).  Beyond it depends: 24 rows of 4096 x 1536 59.7 / 53.5, 96 161 / 154, but 72 of 2048 x 768 27.0 / 27.8, of 2048 x 704 27.5 / 30.1.
 template <int U, bool LINES>
-__global__ void __launch_bounds__(256, 4) sv_downs_kernel(const KrSvGemm o, const KrSvGemm e, const KrSvGemm sh, const int so, const int ss, const int se) {
+__global__ void __launch_bounds__(256, LINES ? 1 : 4) sv_downs_kernel(const KrSvGemm o, const KrSvGemm e, const KrSvGemm sh, const int so, const int ss, const int se) {
     __shared__ __attribute__((aligned(16))) float red[sk_red_floats(1, 1, 4)];
     extern __shared__ __attribute__((aligned(16))) uint16_t act[];
     int i = blockIdx.x;

@@ -221,10 +221,12 @@ __device__ __forceinline__ void sk_row_glu_column(const KrSvGemm& g, const int n
 // rows of the matrix and waits for nothing but its row's expert and its neighbours' (rows of one expert stand together).  A row that has its expert to itself reads past the caches;
 // where a neighbour reads the matrix too it has to stay (us a step: 24 rows on 8 of 128 experts of
 // 2 x 1536 x 4096, one layer, all past the caches / none / this rule 261 / 238 / 239, on 22 of them 301 / 304 / 298; one request, six rows, two layers of 64 of 2 x 768 x 2048 132 / 139 / 131).
+// one: the rows of one token, whose experts differ; they do not wait for neighbours (a chat turn 5806 -> 5763).
 template <int WV>
-__device__ __forceinline__ void sk_row_glu(const KrSvGemm& g, const int bx, const int by) {
+__device__ __forceinline__ void sk_row_glu(const KrSvGemm& g, const int bx, const int by, const bool one) {
     const int n = bx * WV + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (n >= g.glu_f) return;
+    if (one) { sk_row_glu_column<true>(g, n, by, g.row_group[by]); return; }
     const int group = g.row_group[by], before = g.row_group[max(by - 1, 0)], behind = g.row_group[min(by + 1, g.M - 1)];
     if ((before != group || by == 0) && (behind != group || by == g.M - 1)) sk_row_glu_column<true>(g, n, by, group);
     else sk_row_glu_column<false>(g, n, by, group);
